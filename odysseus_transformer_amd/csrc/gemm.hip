@@ -14,7 +14,7 @@
 // fp32 (its 1e-4 tolerance rules out bf16 inputs): v_mfma_f32_32x32x2_f32 on
 // 64 x 64 or 128 x 128 workgroup tiles, any shape and alignment.
 #include <type_traits>
-#include "ody_common.h"
+#include "gemm_epi.h"
 
 namespace {
 
@@ -95,26 +95,9 @@ __device__ __forceinline__ void store_out16(bf16* dst, bf16x8 w) {
   __builtin_nontemporal_store(__builtin_bit_cast(raw_t, w), reinterpret_cast<raw_t*>(dst));
 }
 
-// What the fast kernel's epilogue does besides rounding and storing the tile.
-//   EPI_RESIDUAL    C = A B + R                      (R = aux, row pitch ld_aux; one rounding, after the add)
-//   EPI_SWIGLU_FWD  NT only.  B is the packed (2 I, K) gate_up weight.  A 256-column tile holds 128 gate columns
-//                   and the 128 matching up columns, interleaved in blocks of 32 (block c of the tile: gate if c is
-//                   even, up if odd, columns j0 + 32 (c / 2) ...), so that a lane owns gate and up of the same
-//                   (token, j).  Writes gate_up to C in its usual [gate | up] layout and h = silu(gate) * up to out2,
-//                   computed from the rounded gate / up values exactly as the stand-alone SwiGLU kernel would.
-//   EPI_ROPE        NT only, head_dim 128.  A wavefront's 128 columns are one head; columns below I (a multiple of 128)
-//                   are rotated before the one rounding: with the cos / sin table of ody_rope_table in aux (row pitch
-//                   ld_aux), column j < 64 of a head pairs with column j + 64, both in the same lane
-//   EPI_SWIGLU_BWD  the tile is dh = dy Wd (N = I); with gate_up = aux the epilogue writes d_gate_up to C (pitch
-//                   ldc, 2 I columns) as the stand-alone SwiGLU backward would from the rounded dh.
-enum { EPI_NONE = 0, EPI_RESIDUAL = 1, EPI_SWIGLU_FWD = 2, EPI_SWIGLU_BWD = 3, EPI_ROPE = 4 };
-struct GemmEpi {
-  const bf16* aux;
-  bf16* out2;
-  int64_t ld_aux, ld_out2;
-  int I;
-};
-
+// Epilogues (gemm_epi.h) of the 256 x 256 kernel.  EPI_SWIGLU_FWD: a 256-column tile holds 128 gate columns and the 128 matching
+// up columns, interleaved in blocks of 32 (block c of the tile: gate if c is even, up if odd, columns j0 + 32 (c / 2) ...), so that
+// a lane owns gate and up of the same (token, j).  EPI_ROPE: a wavefront's 128 columns are one head, j and j + 64 in the same lane.
 //
 // SPLITK: blockIdx.y selects one of gridDim.y ranges of K slabs; the block writes its fp32 partial tile to
 // part[blockIdx.y][M][N] and gemm_splitk_sum_kernel adds the ranges up (bias, C += and the rounding happen
@@ -858,6 +841,8 @@ int launch_fused(const char* name, const bf16* A, const bf16* B, bf16* C, int M,
 // kernel, and an edge strip on the right and at the bottom for the general kernel.
 int gemm_bf16(int op, const bf16* a, const bf16* b, bf16* c, const bf16* bias, int M, int N, int K, int64_t lda,
               int64_t ldb, int64_t ldc, int accumulate, void* workspace, size_t workspace_bytes, hipStream_t st) {
+  if (op == ODY_GEMM_NT && ody_gemm_skinny_ok(EPI_NONE, M, N, K, lda, ldb))
+    return ody_launch_gemm_skinny(EPI_NONE, a, b, c, bias, M, N, K, lda, ldb, ldc, accumulate, GemmEpi{}, st);
   const int64_t big_tiles = (int64_t)((M + 255) / 256) * ((N + 255) / 256);
   const int tile = big_tiles >= 192 ? 256 : 128;
   const int M0 = M / tile * tile, N0 = N / tile * tile;
@@ -1133,8 +1118,11 @@ extern "C" int ody_linear_rope(const void* x, const void* w, const void* table, 
   ODY_REQUIRE(vec16(table, ld_table) && vec16(y, ldy), ODY_ERR_MISALIGNED,
               "ody_linear_rope: table and y need 16-byte aligned rows");
   hipStream_t st = static_cast<hipStream_t>(stream);
+  const GemmEpi ep{static_cast<const bf16*>(table), nullptr, ld_table, 0, n_rot * D};
+  if (ody_gemm_skinny_ok(EPI_ROPE, M, N, K, ldx, ldw) && vec16(x, ldx) && vec16(w, ldw) && K % 8 == 0)
+    return ody_launch_gemm_skinny(EPI_ROPE, static_cast<const bf16*>(x), static_cast<const bf16*>(w), static_cast<bf16*>(y), nullptr,
+                                  M, N, K, ldx, ldw, ldy, 0, ep, st);
   if (fused_shape_ok(M, N, K, ldx, ldw) && vec16(x, ldx) && vec16(w, ldw)) {
-    GemmEpi ep{static_cast<const bf16*>(table), nullptr, ld_table, 0, n_rot * D};
     return launch_fused<true, EPI_ROPE>("gemm_bf16_nt_rope", static_cast<const bf16*>(x), static_cast<const bf16*>(w),
                                         static_cast<bf16*>(y), M, N, K, ldx, ldw, ldy, ep, st);
   }
@@ -1152,6 +1140,12 @@ extern "C" int ody_linear_residual(const void* x, const void* w, const void* res
   ODY_REQUIRE(ldx >= K && ldw >= K && ld_res >= N && ldy >= N, ODY_ERR_BAD_SHAPE,
               "ody_linear_residual: leading dimension smaller than the row length");
   hipStream_t st = static_cast<hipStream_t>(stream);
+  if (dtype == ODY_BF16 && ody_gemm_skinny_ok(EPI_RESIDUAL, M, N, K, ldx, ldw) && vec16(x, ldx) && vec16(w, ldw) &&
+      vec16(residual, ld_res) && vec16(y, ldy) && K % 8 == 0 && N % 8 == 0) {
+    const GemmEpi ep{static_cast<const bf16*>(residual), nullptr, ld_res, 0, 0};
+    return ody_launch_gemm_skinny(EPI_RESIDUAL, static_cast<const bf16*>(x), static_cast<const bf16*>(w), static_cast<bf16*>(y),
+                                  nullptr, M, N, K, ldx, ldw, ldy, 0, ep, st);
+  }
   if (dtype == ODY_BF16 && fused_shape_ok(M, N, K, ldx, ldw) && vec16(x, ldx) && vec16(w, ldw) && vec16(residual, ld_res) &&
       vec16(y, ldy) && (int64_t)((M + 255) / 256) * ((N + 255) / 256) >= 128) {
     GemmEpi ep{static_cast<const bf16*>(residual), nullptr, ld_res, 0, 0};
@@ -1181,6 +1175,12 @@ extern "C" int ody_linear_swiglu(const void* x, const void* w_gate_up, void* gat
   ODY_REQUIRE(ldx >= K && ldw >= K && ld_gu >= 2 * (int64_t)I && ld_h >= I, ODY_ERR_BAD_SHAPE,
               "ody_linear_swiglu: leading dimension smaller than the row length");
   hipStream_t st = static_cast<hipStream_t>(stream);
+  if (dtype == ODY_BF16 && ody_gemm_skinny_ok(EPI_SWIGLU_FWD, T, 2 * I, K, ldx, ldw) && vec16(x, ldx) && vec16(w_gate_up, ldw) &&
+      vec16(gate_up, ld_gu) && vec16(h, ld_h) && K % 8 == 0) {
+    const GemmEpi ep{nullptr, static_cast<bf16*>(h), 0, ld_h, I};
+    return ody_launch_gemm_skinny(EPI_SWIGLU_FWD, static_cast<const bf16*>(x), static_cast<const bf16*>(w_gate_up),
+                                  static_cast<bf16*>(gate_up), nullptr, T, 2 * I, K, ldx, ldw, ld_gu, 0, ep, st);
+  }
   if (dtype == ODY_BF16 && I % 128 == 0 && fused_shape_ok(T, 2 * I, K, ldx, ldw) && (int64_t)I * ldw < (1ll << 40) &&
       vec16(x, ldx) && vec16(w_gate_up, ldw) && vec16(gate_up, ld_gu) && vec16(h, ld_h)) {
     GemmEpi ep{nullptr, static_cast<bf16*>(h), 0, ld_h, I};

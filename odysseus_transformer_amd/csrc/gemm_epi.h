@@ -1,0 +1,25 @@
+// What the epilogue of a bf16 product does besides rounding and storing.
+//   EPI_RESIDUAL    C = A B + R                      (R = aux, row pitch ld_aux; one rounding, after the add)
+//   EPI_SWIGLU_FWD  NT only.  B is the packed (2 I, K) gate_up weight.  Writes gate_up to C in its usual [gate | up] layout and
+//                   h = silu(gate) * up to out2, computed from the rounded gate / up values exactly as the stand-alone SwiGLU
+//                   kernel would.
+//   EPI_ROPE        NT only, head_dim 128.  Columns below I (a multiple of 128) are rotated before the one rounding: with the
+//                   cos / sin table of ody_rope_table in aux (row pitch ld_aux), column j < 64 of a head pairs with column j + 64
+//   EPI_SWIGLU_BWD  the result is dh = dy Wd (N = I); with gate_up = aux the epilogue writes d_gate_up to C (pitch ldc, 2 I
+//                   columns) as the stand-alone SwiGLU backward would from the rounded dh.
+#pragma once
+#include "ody_common.h"
+
+enum { EPI_NONE = 0, EPI_RESIDUAL = 1, EPI_SWIGLU_FWD = 2, EPI_SWIGLU_BWD = 3, EPI_ROPE = 4 };
+struct GemmEpi {
+  const bf16* aux;
+  bf16* out2;
+  int64_t ld_aux, ld_out2;
+  int I;
+};
+
+// C (M, N) = A (M, K) . W (N, K)^T for few rows of A (gemm_skinny.hip); EPI_NONE also takes a bias and accumulation into C.
+constexpr int ODY_SKINNY_MAX_M = 64;
+bool ody_gemm_skinny_ok(int epi, int M, int N, int K, int64_t lda, int64_t ldw);
+int ody_launch_gemm_skinny(int epi, const bf16* A, const bf16* W, bf16* C, const bf16* bias, int M, int N, int K, int64_t lda,
+                           int64_t ldw, int64_t ldc, int accumulate, const GemmEpi& ep, hipStream_t st);

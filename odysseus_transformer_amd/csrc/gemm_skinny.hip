@@ -1,0 +1,201 @@
+// Products with few rows, C (M, N) = A (M, K) . W (N, K)^T with M <= 64: a decoding step, or a handful of tokens.
+//
+// Bound by reading W once (an element of it serves M <= 64 multiply-adds), so the work is split for bytes in flight and
+// not for operand reuse: a block owns NT groups of 16 rows of W, its wavefronts each take a share of K, and every wavefront
+// loads its W fragments straight from global memory in the operand order of v_mfma_f32_16x16x32_bf16 -- no LDS, no barrier
+// until the wavefronts' partial results are summed through LDS at the end.  The rows of A (all blocks read the same ones)
+// come from cache; rows beyond M repeat row M - 1 and fall away with their unused result columns.
+//
+// Measured, weights cold, M = 1 (before: 128 x 128 tiles, one block per 128 columns): 4096 x 4096 68 -> 9.4 us (3.6 TB/s),
+// 4096 x 11008 176 -> 22 us (4.1 TB/s), 22016 x 4096 76 -> 40 us (4.5 TB/s), 32000 x 4096 82 -> 54 us (4.9 TB/s; a copy of
+// 1 GiB reaches 5.2).
+#include "gemm_epi.h"
+
+namespace {
+
+constexpr int SK_WAVES = 8;
+
+template <int MT, int NT, int U, int EPI>
+__global__ __launch_bounds__(64 * SK_WAVES) void gemm_skinny_kernel(const bf16* __restrict__ A, const bf16* __restrict__ W,
+                                                                    bf16* __restrict__ C, const bf16* __restrict__ bias, int M,
+                                                                    int N, int K, int64_t lda, int64_t ldw, int64_t ldc,
+                                                                    int accumulate, GemmEpi ep) {
+  __shared__ f32x4 red[SK_WAVES][MT][NT][64];
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, c = lane & 15, q = lane >> 4;
+  // first W row of group t of this block
+  int row0[NT];
+#pragma unroll
+  for (int t = 0; t < NT; t++) {
+    if (EPI == EPI_SWIGLU_FWD) row0[t] = 16 * blockIdx.x + t * ep.I;                                   // gate, up
+    else if (EPI == EPI_ROPE) row0[t] = 128 * (blockIdx.x >> 2) + 16 * (blockIdx.x & 3) + 64 * t;      // j, j + 64 of a head
+    else row0[t] = 16 * (NT * blockIdx.x + t);
+  }
+  const bf16* wp[NT];
+  const bf16* ap[MT];
+#pragma unroll
+  for (int t = 0; t < NT; t++) wp[t] = W + (int64_t)min(row0[t] + c, N - 1) * ldw + 8 * q;
+#pragma unroll
+  for (int m = 0; m < MT; m++) ap[m] = A + (int64_t)min(16 * m + c, M - 1) * lda + 8 * q;
+
+  f32x4 acc[MT][NT];
+#pragma unroll
+  for (int m = 0; m < MT; m++)
+#pragma unroll
+    for (int t = 0; t < NT; t++) acc[m][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  const int steps = (K + 31) / 32, per = (steps + SK_WAVES - 1) / SK_WAVES;
+  const int s0 = wave * per, s1 = min(s0 + per, steps);
+  bf16x8 wf[U][NT], af[U][MT];
+  auto multiply = [&]() {
+#pragma unroll
+    for (int u = 0; u < U; u++)
+#pragma unroll
+      for (int m = 0; m < MT; m++)
+#pragma unroll
+        for (int t = 0; t < NT; t++)
+          acc[m][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[u][t], af[u][m], acc[m][t], 0, 0, 0);   // rows = n, columns = m
+  };
+  int s = s0;
+  const int whole = K / 32;   // steps that lie inside K for every lane
+  for (; s + U <= min(s1, whole); s += U) {
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+#pragma unroll
+      for (int t = 0; t < NT; t++) wf[u][t] = *reinterpret_cast<const bf16x8*>(wp[t] + (int64_t)(s + u) * 32);
+#pragma unroll
+      for (int m = 0; m < MT; m++) af[u][m] = *reinterpret_cast<const bf16x8*>(ap[m] + (int64_t)(s + u) * 32);
+    }
+    multiply();
+  }
+  if (s < s1) {   // the remainder, all of it in flight at once
+    const bf16x8 zero = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const bool in = s + u < s1 && (s + u) * 32 + 8 * q < K;   // K is a multiple of 8: a chunk is all in or out
+#pragma unroll
+      for (int t = 0; t < NT; t++) wf[u][t] = in ? *reinterpret_cast<const bf16x8*>(wp[t] + (int64_t)(s + u) * 32) : zero;
+#pragma unroll
+      for (int m = 0; m < MT; m++) af[u][m] = in ? *reinterpret_cast<const bf16x8*>(ap[m] + (int64_t)(s + u) * 32) : zero;
+    }
+    multiply();
+  }
+
+#pragma unroll
+  for (int m = 0; m < MT; m++)
+#pragma unroll
+    for (int t = 0; t < NT; t++) red[wave][m][t][lane] = acc[m][t];
+  __syncthreads();
+  // thread (m-group, lane) owns row 16 mg + c of A and columns 4 q .. 4 q + 3 of every group of W rows
+  if (tid >= 64 * MT) return;
+  const int mg = tid >> 6, row = 16 * mg + c;
+  if (row >= M) return;
+  f32x4 v[NT];
+#pragma unroll
+  for (int t = 0; t < NT; t++) {
+    v[t] = red[0][mg][t][lane];
+#pragma unroll
+    for (int w = 1; w < SK_WAVES; w++) v[t] += red[w][mg][t][lane];
+  }
+  auto rounded = [](f32x4 x) {
+    bf16x4 w;
+#pragma unroll
+    for (int e = 0; e < 4; e++) w[e] = (bf16)x[e];
+    return w;
+  };
+  bf16* cp = C + (int64_t)row * ldc;
+  if constexpr (EPI == EPI_SWIGLU_FWD) {
+    const int n = row0[0] + 4 * q;
+    if (n >= ep.I) return;
+    const bf16x4 g4 = rounded(v[0]), u4 = rounded(v[1]);
+    bf16x4 h4;
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+      const float a1 = (float)g4[e], a3 = (float)u4[e];
+      h4[e] = (bf16)(a1 / (1.f + __expf(-a1)) * a3);
+    }
+    *reinterpret_cast<bf16x4*>(cp + n) = g4;
+    *reinterpret_cast<bf16x4*>(cp + ep.I + n) = u4;
+    *reinterpret_cast<bf16x4*>(ep.out2 + (int64_t)row * ep.ld_out2 + n) = h4;
+  } else if constexpr (EPI == EPI_ROPE) {
+    const int n = row0[0] + 4 * q, j = n & 127;
+    f32x4 o1 = v[0], o2 = v[1];
+    if (n < ep.I) {
+      const bf16x8 cs = *reinterpret_cast<const bf16x8*>(ep.aux + (int64_t)row * ep.ld_aux + 2 * j);
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        const float co = (float)cs[2 * e], sn = (float)cs[2 * e + 1];
+        o1[e] = v[0][e] * co - v[1][e] * sn;
+        o2[e] = v[1][e] * co + v[0][e] * sn;
+      }
+    }
+    *reinterpret_cast<bf16x4*>(cp + n) = rounded(o1);
+    *reinterpret_cast<bf16x4*>(cp + n + 64) = rounded(o2);
+  } else {
+#pragma unroll
+    for (int t = 0; t < NT; t++) {
+      const int n = row0[t] + 4 * q;
+      if (n >= N) continue;   // N % 8 == 0: four columns are all in or out
+      if constexpr (EPI == EPI_RESIDUAL) {
+        const bf16x4 r = *reinterpret_cast<const bf16x4*>(ep.aux + (int64_t)row * ep.ld_aux + n);
+#pragma unroll
+        for (int e = 0; e < 4; e++) v[t][e] += (float)r[e];
+      } else {
+        if (bias) {
+          const bf16x4 b = *reinterpret_cast<const bf16x4*>(bias + n);
+#pragma unroll
+          for (int e = 0; e < 4; e++) v[t][e] += (float)b[e];
+        }
+        if (accumulate) {
+          const bf16x4 o = *reinterpret_cast<const bf16x4*>(cp + n);
+#pragma unroll
+          for (int e = 0; e < 4; e++) v[t][e] += (float)o[e];
+        }
+      }
+      *reinterpret_cast<bf16x4*>(cp + n) = rounded(v[t]);
+    }
+  }
+}
+
+template <int MT, int NT, int U, int EPI>
+int launch(const char* name, int blocks, const bf16* A, const bf16* W, bf16* C, const bf16* bias, int M, int N, int K, int64_t lda,
+           int64_t ldw, int64_t ldc, int accumulate, const GemmEpi& ep, hipStream_t st) {
+  ODY_LAUNCH(name, st, (gemm_skinny_kernel<MT, NT, U, EPI>), dim3(blocks), dim3(64 * SK_WAVES), 0, A, W, C, bias, M, N, K, lda, ldw,
+             ldc, accumulate, ep);
+  return ody_check_launch(name);
+}
+
+template <int NT, int EPI>
+int by_rows(const char* name, int blocks, const bf16* A, const bf16* W, bf16* C, const bf16* bias, int M, int N, int K, int64_t lda,
+            int64_t ldw, int64_t ldc, int accumulate, const GemmEpi& ep, hipStream_t st) {
+  if (M <= 16) return launch<1, NT, 8, EPI>(name, blocks, A, W, C, bias, M, N, K, lda, ldw, ldc, accumulate, ep, st);
+  if (M <= 32) return launch<2, NT, 4, EPI>(name, blocks, A, W, C, bias, M, N, K, lda, ldw, ldc, accumulate, ep, st);
+  return launch<4, NT, 4, EPI>(name, blocks, A, W, C, bias, M, N, K, lda, ldw, ldc, accumulate, ep, st);
+}
+
+}  // namespace
+
+bool ody_gemm_skinny_ok(int epi, int M, int N, int K, int64_t lda, int64_t ldw) {
+  // beyond 16 rows the loads of A weigh as much as those of W, and with many columns the 128 x 128 tiles, which share both
+  // through LDS, fill the chip: 22016 x 4096, M = 32 / 64: 62 / 83 us here, 76 / 77 us there; 4096 x 4096, M = 64: 24 against 71
+  (void)K; (void)lda; (void)ldw;
+  if (M > ODY_SKINNY_MAX_M || (M > 32 && N >= 16384)) return false;
+  if (epi == EPI_SWIGLU_FWD) return N % 32 == 0;   // whole groups of 16 gate rows and of 16 up rows
+  if (epi == EPI_ROPE) return N % 128 == 0;
+  return epi == EPI_NONE || epi == EPI_RESIDUAL;
+}
+
+int ody_launch_gemm_skinny(int epi, const bf16* A, const bf16* W, bf16* C, const bf16* bias, int M, int N, int K, int64_t lda,
+                           int64_t ldw, int64_t ldc, int accumulate, const GemmEpi& ep, hipStream_t st) {
+  const int groups = (N + 15) / 16;
+  if (epi == EPI_SWIGLU_FWD)
+    return by_rows<2, EPI_SWIGLU_FWD>("gemm_skinny_swiglu", groups / 2, A, W, C, bias, M, N, K, lda, ldw, ldc, accumulate, ep, st);
+  if (epi == EPI_ROPE)
+    return by_rows<2, EPI_ROPE>("gemm_skinny_rope", groups / 2, A, W, C, bias, M, N, K, lda, ldw, ldc, accumulate, ep, st);
+  const bool wide = groups >= 1024;
+  if (epi == EPI_RESIDUAL) {
+    if (wide) return by_rows<2, EPI_RESIDUAL>("gemm_skinny_residual", (groups + 1) / 2, A, W, C, bias, M, N, K, lda, ldw, ldc, accumulate, ep, st);
+    return by_rows<1, EPI_RESIDUAL>("gemm_skinny_residual", groups, A, W, C, bias, M, N, K, lda, ldw, ldc, accumulate, ep, st);
+  }
+  if (wide) return by_rows<2, EPI_NONE>("gemm_skinny", (groups + 1) / 2, A, W, C, bias, M, N, K, lda, ldw, ldc, accumulate, ep, st);
+  return by_rows<1, EPI_NONE>("gemm_skinny", groups, A, W, C, bias, M, N, K, lda, ldw, ldc, accumulate, ep, st);
+}

@@ -244,3 +244,28 @@ def test_rope_table_is_reused_for_the_same_position_tensor_only(dev):
     pos.add_(7)                                                        # modified in place: built again
     t4 = ops.rope_table(pos, 64, 128, 10000.0)
     assert ops.rope_table(pos, 64, 128, 10000.0) is t4 and not torch.equal(t4, t3)
+
+
+@pytest.mark.parametrize("M", [1, 16, 17, 40, 64])
+def test_fused_epilogues_with_few_rows(M, dev):
+    """Residual, SwiGLU and rotary epilogues of the kernel for few rows, against fp32 products."""
+    from odysseus_transformer_amd import ops
+    K, D, H, I = 264, 128, 3, 176
+    x = randn((M, K), 9600, dtype=BF)
+    r, w, wgu = randn((M, H * D), 9601, dtype=BF), randn((H * D, K), 9602, std=0.05, dtype=BF), randn((2 * I, K), 9603, std=0.05, dtype=BF)
+    pos = torch.randint(0, 9000, (1, M), generator=torch.Generator().manual_seed(9604)).to(dev)
+    y, names = _kernels_of(lambda: ops.linear_residual(x.to(dev), w.to(dev), r.to(dev)))
+    assert any("skinny" in n for n in names), names
+    plain = x.float() @ w.float().t()
+    assert rel_err(y, plain + r.float()) <= TOL_BF16, "residual"
+    gu, h = ops.linear_swiglu(x.to(dev), wgu.to(dev))
+    ref = x.float() @ wgu.float().t()
+    assert rel_err(gu, ref) <= TOL_BF16, "gate_up"
+    g, u = gu.float().cpu()[:, :I], gu.float().cpu()[:, I:]
+    assert rel_err(h, torch.nn.functional.silu(g) * u) <= TOL_BF16, "h"
+    table = ops.rope_table(pos, M, D)
+    got = ops.linear_rope(x.to(dev), w.to(dev), table, 2, D).float().cpu().view(M, H, D)
+    c, s = table.float().cpu()[:, 0::2][:, None], table.float().cpu()[:, 1::2][:, None]
+    a, b = plain.view(M, H, D)[:, :2].split(64, dim=-1)
+    want = torch.cat([torch.cat([a * c - b * s, b * c + a * s], -1), plain.view(M, H, D)[:, 2:]], 1)
+    assert rel_err(got, want) <= TOL_BF16, "rope"

@@ -134,3 +134,21 @@ def test_gemm_errors(dev):
         ops.gemm(ops.GEMM_NT, a, a)
     with pytest.raises(ValueError):
         ops.gemm(ops.GEMM_NT, a, torch.zeros(16, 24, dtype=torch.bfloat16, device=dev))
+
+
+@pytest.mark.parametrize("M", [1, 15, 16, 17, 32, 33, 64, 65])
+@pytest.mark.parametrize("N,K", [(264, 136), (128, 4096), (512, 2056), (16512, 64)], ids=lambda v: str(v))
+def test_products_with_few_rows(M, N, K, dev):
+    """The kernel for few rows of A: edges of its 16-row groups on both sides, K that is no multiple of 32 or of the
+    wavefronts' shares, bias, accumulation and padded leading dimensions."""
+    from odysseus_transformer_amd import ops
+    print(f"few rows M={M} N={N} K={K}", flush=True)
+    x = randn((M, K + 8), 31, dtype=torch.bfloat16)[:, :K]
+    w = randn((N, K), 32, std=0.05, dtype=torch.bfloat16)
+    bias = randn((N,), 33, dtype=torch.bfloat16)
+    ref = x.float() @ w.float().t()
+    xd, wd = x.to(dev), w.to(dev)
+    assert rel_err(ops.gemm(ops.GEMM_NT, xd, wd), ref) <= TOL_BF16, "y"
+    out = torch.ones((M, N), dtype=torch.bfloat16, device=dev)
+    ops.gemm(ops.GEMM_NT, xd, wd, bias=bias.to(dev), out=out, accumulate=True)
+    assert rel_err(out, ref + bias.float() + 1.0) <= TOL_BF16, "y + bias + C"
