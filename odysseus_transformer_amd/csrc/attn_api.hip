@@ -74,6 +74,11 @@ int attn_fwd_impl(const char* who, const void* q, const void* k, const void* v, 
   ODY_REQUIRE(lse != nullptr, ODY_ERR_NULL, "%s: lse is NULL", who);
   ODY_REQUIRE(scale > 0.f && std::isfinite(scale), ODY_ERR_BAD_SHAPE, "%s: scale must be positive", who);
   hipStream_t st = static_cast<hipStream_t>(stream);
+  // few rows: no image of V to write, no 256-query block to fill
+  if (dtype == ODY_BF16 && p.drop_thresh == 0 && ody_attn_decode_ok(Lq, Hq, Hkv, D)) {
+    ODY_REQUIRE((reinterpret_cast<uintptr_t>(workspace) & 15u) == 0, ODY_ERR_MISALIGNED, "%s: workspace must be 16-byte aligned", who);
+    return ody_launch_attn_decode(p, D, workspace, workspace_bytes, st);
+  }
   if (dtype == ODY_BF16 && D == 128 && p.drop_thresh == 0) {
     // the least that will do: without room for the parts of a key-split call the call runs unsplit
     const size_t need = (ody_attn_fwd_w8_workspace(B, Lq, Lk, Hq, Hkv, false) + 255) & ~(size_t)255;
@@ -149,7 +154,10 @@ extern "C" int ody_attn_fwd_noalloc(const void* q, const void* k, const void* v,
   // the fixed scratch holds the flags and the V images, and the parts of a call that cuts its key ranges if they fit
   // as well (then the result is that of ody_attn_fwd bit for bit); otherwise such a call runs unsplit here
   size_t need = 0;
-  if (dtype == ODY_BF16 && D == 128) {
+  if (dtype == ODY_BF16 && ody_attn_decode_ok(Lq, Hq, Hkv, D)) {
+    need = (ody_attn_decode_workspace(B, Lq, Lk, Hq, Hkv, D) + 255) & ~(size_t)255;
+    if (need > (size_t)ODY_ATTN_FWD_NOALLOC_SCRATCH_BYTES) need = 0;
+  } else if (dtype == ODY_BF16 && D == 128) {
     need = (ody_attn_fwd_w8_workspace(B, Lq, Lk, Hq, Hkv, true) + 255) & ~(size_t)255;
     if (need > (size_t)ODY_ATTN_FWD_NOALLOC_SCRATCH_BYTES)
       need = (ody_attn_fwd_w8_workspace(B, Lq, Lk, Hq, Hkv, false) + 255) & ~(size_t)255;
@@ -166,6 +174,10 @@ extern "C" int ody_attn_fwd_noalloc(const void* q, const void* k, const void* v,
 
 extern "C" size_t ody_attn_fwd_workspace_bytes(int B, int Lq, int Lk, int Hq, int Hkv, int D, int dtype) {
   if (B <= 0 || Lq <= 0 || Lk <= 0 || Hq <= 0 || Hkv <= 0) return 0;
+  if (dtype == ODY_BF16 && ody_attn_decode_ok(Lq, Hq, Hkv, D)) {
+    // a caller with dropout on these sizes (other kernels, no workspace) merely holds bytes it does not use
+    return (ody_attn_decode_workspace(B, Lq, Lk, Hq, Hkv, D) + 255) & ~(size_t)255;
+  }
   if (dtype == ODY_BF16 && D == 128) return (ody_attn_fwd_w8_workspace(B, Lq, Lk, Hq, Hkv, true) + 255) & ~(size_t)255;
   return 0;
 }

@@ -86,6 +86,11 @@ int ody_launch_attn_bwd_prepass(const AttnParams& p, void* qimg, void* doimg, vo
 // blocks against many keys); a workspace without that room makes such a call run unsplit.
 int ody_launch_attn_fwd_w8(const AttnParams& p, void* workspace, size_t workspace_bytes, hipStream_t st);
 size_t ody_attn_fwd_w8_workspace(int B, int Lq, int Lk, int Hq, int Hkv, bool with_split);
+// forward for at most 64 rows per kv head (rows = queries x query heads of its group), key ranges cut over blocks; a workspace
+// without room for the parts makes the call run on one block per kv head
+bool ody_attn_decode_ok(int Lq, int Hq, int Hkv, int D);
+size_t ody_attn_decode_workspace(int B, int Lq, int Lk, int Hq, int Hkv, int D);
+int ody_launch_attn_decode(const AttnParams& p, int D, void* workspace, size_t workspace_bytes, hipStream_t st);
 // the online-rescaling forward kernel restricted to query blocks of `block` rows whose flag is set
 int ody_launch_attn_fwd_mfma_flagged(const AttnParams& p, const int* flags, int block, hipStream_t st);
 // head_dim 128 only; workspace of ody_attn_bwd_pipe_workspace(...) bytes (p.delta is set separately)

@@ -522,3 +522,24 @@ def test_attention_dropout_errors(dev):
     o0, lse0 = ops.attn_fwd(q, k, v, dropout_p=0.0)
     o1, lse1 = ops.attn_fwd(q, k, v)
     assert torch.equal(o0, o1) and torch.equal(lse0, lse1)
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("case", [(1, 1, 1, 4, 1, True), (1, 1, 127, 8, 2, True), (1, 1, 8192, 32, 8, True), (2, 3, 129, 4, 4, True),
+                                  (1, 16, 1000, 8, 2, True), (1, 32, 33, 2, 1, True), (1, 17, 5000, 2, 2, False), (2, 20, 8, 3, 1, True),
+                                  (1, 31, 300, 4, 2, False)],
+                         ids=lambda c: "B%d_Lq%d_Lk%d_H%d_%d_c%d" % c)
+def test_attention_fwd_few_queries(case, D, dev):
+    """The kernel for few rows per kv head: 16-, 32- and 64-row instances, keys on both sides of its 32-key tiles, one and many
+    key ranges, queries that see no key, strided keys as a cache hands them over."""
+    from odysseus_transformer_amd import ops
+    B, Lq, Lk, Hq, Hkv, causal = case
+    print(f"few queries case={case} D={D}", flush=True)
+    q, k, v, _ = _inputs(B, Lq, Lk, Hq, Hkv, D, torch.bfloat16, seed=29)
+    o_ref, lse_ref = oracle.attention_fwd(q.float(), k.float(), v.float(), causal=causal)
+    cache = torch.full((2, B, Hkv, Lk + 5, D), float("nan"), dtype=torch.bfloat16, device=dev)   # what lies behind the keys is not read
+    cache[0, :, :, :Lk], cache[1, :, :, :Lk] = k.transpose(1, 2).to(dev), v.transpose(1, 2).to(dev)
+    o, lse = ops.attn_fwd(q.to(dev), cache[0, :, :, :Lk].transpose(1, 2), cache[1, :, :, :Lk].transpose(1, 2), causal=causal)
+    torch.cuda.synchronize()
+    assert_parity(o, o_ref, TOL_BF16, "o")
+    assert torch.allclose(lse.cpu(), lse_ref, atol=TOL_LSE, rtol=TOL_LSE)
