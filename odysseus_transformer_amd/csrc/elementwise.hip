@@ -48,7 +48,7 @@ __device__ __forceinline__ float wave_sum(float x) {
 template <typename T> __device__ __forceinline__ float rnd(float x) { return (float)(T)x; }
 
 // ---------------------------------------------------------------------------
-// RMSNorm forward: one wavefront per row; the row is cached in registers when it
+// RMSNorm forward, many narrow rows: one wavefront per row; the row is cached in registers when it
 // fits (d <= 64 * N * CACHE), otherwise re-read.
 // ---------------------------------------------------------------------------
 template <typename T>
@@ -93,6 +93,67 @@ __global__ __launch_bounds__(256) void rmsnorm_fwd_kernel(const T* __restrict__ 
     }
   }
   for (int vi = lane + 64 * CACHE; vi < nvec; vi += 64) {
+    float f[N], wf[N], o[N];
+    VecIO<T>::load(xr + vi * N, f);
+    VecIO<T>::load(w + vi * N, wf);
+#pragma unroll
+    for (int e = 0; e < N; e++) o[e] = wf[e] * rnd<T>(f[e] * rstd);
+    VecIO<T>::store_streaming(yr + vi * N, o);
+  }
+}
+
+// The same with one block per row: a row's chain of load, reduction and store is four times shorter than a wavefront's, and the
+// weight is fetched beside the row instead of behind its reduction.  CACHE vectors per thread stay in registers, anything beyond
+// is read again.  Measured against a wavefront per row, d = 4096 bf16: 1 row 4.0 -> 2.3 us, 1000 rows 8.6 -> 4.8, 4096 rows
+// 15.2 -> 14.3, 16384 rows 55 -> 47 us (5.8 TB/s); d = 512 fp32, where half of the block has no vector: 2048 rows 3.7 -> 3.5,
+// 4096 rows 4.8 -> 6.3.
+template <typename T>
+__global__ __launch_bounds__(256) void rmsnorm_fwd_row_kernel(const T* __restrict__ x, const T* __restrict__ w, T* __restrict__ y,
+                                                              float* __restrict__ rstd_out, int d, float eps) {
+  constexpr int N = VecIO<T>::N, CACHE = 2;
+  typedef typename VecIO<T>::vec_t vec_t;
+  __shared__ float red[4];
+  const int tid = threadIdx.x, row = blockIdx.x, nvec = d / N;
+  const T* xr = x + (int64_t)row * d;
+  T* yr = y + (int64_t)row * d;
+  vec_t cache[CACHE], wv[CACHE];
+  float ss = 0.f;
+#pragma unroll
+  for (int c = 0; c < CACHE; c++) {
+    const int vi = tid + 256 * c;
+    if (vi < nvec) {
+      cache[c] = *reinterpret_cast<const vec_t*>(xr + vi * N);
+      wv[c] = *reinterpret_cast<const vec_t*>(w + vi * N);
+    }
+  }
+#pragma unroll
+  for (int c = 0; c < CACHE; c++)
+    if (tid + 256 * c < nvec) {
+#pragma unroll
+      for (int e = 0; e < N; e++) ss = fmaf((float)cache[c][e], (float)cache[c][e], ss);
+    }
+  for (int vi = tid + 256 * CACHE; vi < nvec; vi += 256) {
+    float f[N];
+    VecIO<T>::load(xr + vi * N, f);
+#pragma unroll
+    for (int e = 0; e < N; e++) ss = fmaf(f[e], f[e], ss);
+  }
+  ss = wave_sum(ss);
+  if ((tid & 63) == 0) red[tid >> 6] = ss;
+  __syncthreads();
+  const float rstd = rsqrtf((red[0] + red[1] + red[2] + red[3]) / (float)d + eps);
+  if (tid == 0 && rstd_out) rstd_out[row] = rstd;
+#pragma unroll
+  for (int c = 0; c < CACHE; c++) {
+    const int vi = tid + 256 * c;
+    if (vi < nvec) {
+      float o[N];
+#pragma unroll
+      for (int e = 0; e < N; e++) o[e] = (float)wv[c][e] * rnd<T>((float)cache[c][e] * rstd);
+      VecIO<T>::store_streaming(yr + vi * N, o);
+    }
+  }
+  for (int vi = tid + 256 * CACHE; vi < nvec; vi += 256) {
     float f[N], wf[N], o[N];
     VecIO<T>::load(xr + vi * N, f);
     VecIO<T>::load(w + vi * N, wf);
@@ -473,6 +534,15 @@ extern "C" int ody_rmsnorm_fwd(const void* x, const void* w, void* y, float* rst
   ODY_REQUIRE(ody_aligned16(x) && ody_aligned16(w) && ody_aligned16(y), ODY_ERR_MISALIGNED,
               "ody_rmsnorm_fwd: pointers must be 16-byte aligned");
   hipStream_t st = static_cast<hipStream_t>(stream);
+  // a wavefront per row only where a row is too narrow for a block and there are many (see rmsnorm_fwd_row_kernel)
+  if (T <= 2048 || d / n >= 256) {
+    ODY_BY_DTYPE(dtype,
+                 ODY_LAUNCH("rmsnorm_fwd", st, rmsnorm_fwd_row_kernel<bf16>, dim3(T), dim3(256), 0, (const bf16*)x, (const bf16*)w,
+                            (bf16*)y, rstd, d, eps),
+                 ODY_LAUNCH("rmsnorm_fwd", st, rmsnorm_fwd_row_kernel<float>, dim3(T), dim3(256), 0, (const float*)x,
+                            (const float*)w, (float*)y, rstd, d, eps));
+    return ody_check_launch("rmsnorm_fwd");
+  }
   dim3 grid((T + 3) / 4);
   ODY_BY_DTYPE(dtype,
                ODY_LAUNCH("rmsnorm_fwd", st, rmsnorm_fwd_kernel<bf16>, grid, dim3(256), 0, (const bf16*)x, (const bf16*)w,

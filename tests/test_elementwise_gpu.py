@@ -214,3 +214,15 @@ def test_ring_blocks_autograd_function(dtype, dev):
     for b in range(NB):
         assert_parity(kg[b].grad, dk_ref[b], tol, f"dk block {b}")
         assert_parity(vg[b].grad, dv_ref[b], tol, f"dv block {b}")
+
+
+@DTYPES
+@pytest.mark.parametrize("T,d", [(1, 24), (2048, 512), (2049, 512), (2049, 4096), (3, 8200), (2, 16392)])
+def test_rmsnorm_fwd_block_and_wavefront_rows(T, d, dtype, dev):
+    """Both splits of the forward on each side of their line, rows that do not fill a block and rows beyond its registers."""
+    from odysseus_transformer_amd import ops
+    x = randn((1, T, d), 11, dtype=dtype)
+    w = (1.0 + randn((d,), 12, std=0.02)).to(dtype)
+    y, rstd = ops.rmsnorm_fwd(x.to(dev), w.to(dev), 1e-6)
+    assert rel_err(y, oracle.rmsnorm(x.float(), w.float())) <= _tol(dtype)
+    assert rel_err(rstd, torch.rsqrt(x.float().pow(2).mean(-1) + 1e-6).view(-1)) <= 1e-5
