@@ -168,7 +168,7 @@ class LlamaFlashAttention2TPSP(nn.Module):
             elif self._can_fuse_rope(hidden_states):
                 # projection, rotary embedding and attention as one autograd node: the rotation rides in the
                 # projection's epilogue, its backward in the epilogues of the attention backward
-                qkv3, attn_output, _ = ops.QKVRoPEAttnFunc.apply(hidden_states, self.qkv_proj.weight, nh, nkv, D,
+                qkv3, attn_output, _ = ops.run_function(ops.QKVRoPEAttnFunc, hidden_states, self.qkv_proj.weight, nh, nkv, D,
                                                                  position_ids, self.rope_theta, scale)
             else:
                 qkv3, attn_output, _ = PackedRoPEAttnFunc.apply(self.qkv_proj(hidden_states), nh, nkv, D, position_ids,
@@ -195,7 +195,7 @@ class LlamaFlashAttention2TPSP(nn.Module):
         residual = kwargs.get("residual")
         if residual is not None and self._can_fuse_residual(residual, attn_output):
             # the caller's skip connection rides in the output projection's epilogue
-            attn_output = ops.LinearResidualFunc.apply(attn_output, self.o_proj.weight, residual)
+            attn_output = ops.run_function(ops.LinearResidualFunc, attn_output, self.o_proj.weight, residual)
         else:
             attn_output = self.o_proj(attn_output)
             if residual is not None:
@@ -289,7 +289,7 @@ class LlamaMLPZeRO(nn.Module):
                    and not _has_hooks(self.gate_up_proj, self.down_proj)
                    and not torch.is_autocast_enabled("cuda"))
         if fusable and self.fuse_elementwise:
-            return ops.SwiGLUMLPResidualFunc.apply(x, w1, w2, residual)
+            return ops.run_function(ops.SwiGLUMLPResidualFunc, x, w1, w2, residual)
         y = self.down_proj(ops.swiglu(self.gate_up_proj(x)))
         return y if residual is None else residual + y
 

@@ -33,7 +33,36 @@ def _need_gpu(*ts: torch.Tensor) -> None:
 
 
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    # torch.cuda.current_stream() builds a Stream object and re-checks the driver on every call: 9 us against 0.4
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
+
+
+class _NoContext:
+    """Stands in for autograd's context where nothing is recorded: keeps nothing."""
+    __slots__ = ()
+
+    def __setattr__(self, name, value):
+        pass
+
+    def save_for_backward(self, *tensors):
+        pass
+
+    def mark_non_differentiable(self, *tensors):
+        pass
+
+    def set_materialize_grads(self, value):
+        pass
+
+
+_NO_CONTEXT = _NoContext()
+
+
+def run_function(fn, *args):
+    """fn.apply(*args), or fn's forward alone under no_grad / inference mode: an inference step is a handful of small launches,
+    and the autograd machinery around each costs more host time (8-10 us) than the launch itself."""
+    if torch.is_grad_enabled():
+        return fn.apply(*args)
+    return fn.forward(_NO_CONTEXT, *args)
 
 
 def scratch(nbytes: int, name: str, device) -> torch.Tensor:
@@ -799,7 +828,7 @@ def flash_attn_func(q, k, v, dropout_p: float = 0.0, softmax_scale: Optional[flo
     a host value: a captured graph replays the mask it was captured with -- pass `seed` per step there."""
     if dropout_p != 0.0 and seed is None:
         seed = int(torch.randint(0, 1 << 62, (1,)).item())
-    out, lse = FlashAttnFunc.apply(q, k, v, softmax_scale, causal, float(dropout_p), seed)
+    out, lse = run_function(FlashAttnFunc, q, k, v, softmax_scale, causal, float(dropout_p), seed)
     return (out, lse) if return_lse else out
 
 
@@ -960,17 +989,17 @@ class SwiGLUMLPResidualFunc(torch.autograd.Function):
 
 
 def rmsnorm(x, weight, eps: float = 1e-6):
-    return RMSNormFunc.apply(x, weight, eps)
+    return run_function(RMSNormFunc, x, weight, eps)
 
 
 def rmsnorm_fork(x, weight, eps: float = 1e-6):
     """-> (rmsnorm(x), x) with the two returning gradients summed inside the norm's backward kernel."""
-    return RMSNormForkFunc.apply(x, weight, eps)
+    return run_function(RMSNormForkFunc, x, weight, eps)
 
 
 def swiglu(gate_up):
-    return SwiGLUFunc.apply(gate_up)
+    return run_function(SwiGLUFunc, gate_up)
 
 
 def apply_rope_packed(qkv, n_rot: int, position_ids=None, base: float = 10000.0):
-    return RoPEFunc.apply(qkv, n_rot, position_ids, base)
+    return run_function(RoPEFunc, qkv, n_rot, position_ids, base)

@@ -179,8 +179,8 @@ def linear_with_grad_accumulation_and_async_allreduce(
             warnings.warn(f"When using {what} it is recommended to set the environment variable "
                           "CUDA_DEVICE_MAX_CONNECTIONS to 1 for maximum speedup")
             fn.warned = True
-    return LinearWithGradAccumulationAndAsyncCommunication.apply(
-        input, weight, bias, gradient_accumulation_fusion, async_grad_allreduce, sequence_parallel,
+    return ops.run_function(
+        LinearWithGradAccumulationAndAsyncCommunication, input, weight, bias, gradient_accumulation_fusion, async_grad_allreduce, sequence_parallel,
         grad_output_buffer)
 
 
@@ -312,6 +312,6 @@ class RowParallelLinearRS(torch.nn.Module):
     def forward(self, input_: torch.Tensor) -> torch.Tensor:
         if not self.input_is_parallel:
             require_single_rank("scatter of the input over the model-parallel group")
-        output_parallel = _PlainLinearFunc.apply(input_, self.weight)
+        output_parallel = ops.run_function(_PlainLinearFunc, input_, self.weight)
         output_ = reducescatter_from_model_parallel_region(output_parallel)
         return output_ if self.bias is None else output_ + self.bias

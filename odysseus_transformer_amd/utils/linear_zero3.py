@@ -10,6 +10,7 @@ from typing import Optional
 import torch
 from torch import nn
 
+from .. import ops
 from ..parallel_state import (get_model_parallel_group, get_model_parallel_world_size, require_single_rank)
 from .comm import prepare_input_tensors_for_wgrad_compute
 from .linear_tpsp import linear_dgrad, linear_forward, linear_wgrad
@@ -50,7 +51,7 @@ class LinearZeROFunc(torch.autograd.Function):
 
 
 def linear_with_zero(input: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor]) -> torch.Tensor:
-    return LinearZeROFunc.apply(input, weight, bias)
+    return ops.run_function(LinearZeROFunc, input, weight, bias)
 
 
 class LinearZeRO3(nn.Module):
