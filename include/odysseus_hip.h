@@ -209,8 +209,7 @@ int ody_gemm(int op, const void* A, const void* B, void* C, const void* bias,
  * ody_linear_residual     y (M, N) = x (M, K) W (N, K)^T + residual (M, N): the output projection and the
  *                         down projection together with the decoder layer's residual add
  *                         (utils/linear_tpsp.py:588 / utils/linear_zero3.py:44, then decoder/ring.py:80,86).
- *                         The sum is formed in fp32 and rounded once.  y may be the residual buffer itself only
- *                         when the shape takes the unfused path; pass distinct buffers.
+ *                         The sum is formed in fp32 and rounded once.  y may be the residual buffer itself.
  * ody_linear_swiglu       gate_up (T, 2 I) = x (T, K) Wgu (2 I, K)^T and h (T, I) = silu(gate) * up
  *                         (decoder/odysseus.py:293-295); gate_up is kept because the backward needs it.
  * ody_linear_dgrad_swiglu d_gate_up (T, 2 I) = SwiGLU backward of (gate_up, dh) with dh = dy (T, K) Wd (K, I):
@@ -224,6 +223,11 @@ int ody_gemm(int op, const void* A, const void* B, void* C, const void* bias,
  */
 int ody_linear_residual(const void* x, const void* w, const void* residual, void* y, int M, int N, int K,
                         int64_t ldx, int64_t ldw, int64_t ld_res, int64_t ldy, int dtype, void* stream);
+/* the same with a caller workspace (ody_gemm_workspace_bytes(ODY_GEMM_NT, M, N, K, dtype) bytes, 16-byte aligned; NULL and 0 do
+ * too): a product with few output tiles for its K then cuts K into ranges */
+int ody_linear_residual_ws(const void* x, const void* w, const void* residual, void* y, int M, int N, int K,
+                           int64_t ldx, int64_t ldw, int64_t ld_res, int64_t ldy, int dtype, void* workspace,
+                           size_t workspace_bytes, void* stream);
 int ody_linear_swiglu(const void* x, const void* w_gate_up, void* gate_up, void* h, int T, int I, int K,
                       int64_t ldx, int64_t ldw, int64_t ld_gu, int64_t ld_h, int dtype, void* stream);
 size_t ody_linear_dgrad_swiglu_workspace_bytes(int T, int I, int K, int dtype);
@@ -294,6 +298,10 @@ int ody_rope_table(const int64_t* position_ids, const float* inv_freq, int64_t r
                    void* table, void* stream);
 int ody_linear_rope(const void* x, const void* w, const void* table, void* y, int M, int N, int K, int n_rot,
                     int D, int64_t ldx, int64_t ldw, int64_t ld_table, int64_t ldy, int dtype, void* stream);
+/* with a caller workspace, as ody_linear_residual_ws */
+int ody_linear_rope_ws(const void* x, const void* w, const void* table, void* y, int M, int N, int K, int n_rot,
+                       int D, int64_t ldx, int64_t ldw, int64_t ld_table, int64_t ldy, int dtype, void* workspace,
+                       size_t workspace_bytes, void* stream);
 int ody_attn_bwd_rope(const void* q, const void* k, const void* v, const void* out, const float* lse,
                       const void* dout, void* dq, void* dk, void* dv,
                       int B, int Lq, int Lk, int Hq, int Hkv, int D,

@@ -19,7 +19,7 @@ struct GemmEpi {
 };
 
 // C (M, N) = A (M, K) . W (N, K)^T for few rows of A (gemm_skinny.hip); EPI_NONE also takes a bias and accumulation into C.
-constexpr int ODY_SKINNY_MAX_M = 64;
-bool ody_gemm_skinny_ok(int epi, int M, int N, int K, int64_t lda, int64_t ldw);
+constexpr int ODY_SKINNY_MAX_M = 16;
+bool ody_gemm_skinny_ok(int epi, int M, int N);
 int ody_launch_gemm_skinny(int epi, const bf16* A, const bf16* W, bf16* C, const bf16* bias, int M, int N, int K, int64_t lda,
                            int64_t ldw, int64_t ldc, int accumulate, const GemmEpi& ep, hipStream_t st);

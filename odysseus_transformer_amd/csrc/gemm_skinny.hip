@@ -1,6 +1,6 @@
-// Products with few rows, C (M, N) = A (M, K) . W (N, K)^T with M <= 64: a decoding step, or a handful of tokens.
+// Products with few rows, C (M, N) = A (M, K) . W (N, K)^T with M <= 16: a decoding step, or a handful of tokens.
 //
-// Bound by reading W once (an element of it serves M <= 64 multiply-adds), so the work is split for bytes in flight and
+// Bound by reading W once (an element of it serves M <= 16 multiply-adds), so the work is split for bytes in flight and
 // not for operand reuse: a block owns NT groups of 16 rows of W, its wavefronts each take a share of K, and every wavefront
 // loads its W fragments straight from global memory in the operand order of v_mfma_f32_16x16x32_bf16 -- no LDS, no barrier
 // until the wavefronts' partial results are summed through LDS at the end.  The rows of A (all blocks read the same ones)
@@ -15,12 +15,12 @@ namespace {
 
 constexpr int SK_WAVES = 8;
 
-template <int MT, int NT, int U, int EPI>
+template <int NT, int U, int EPI>
 __global__ __launch_bounds__(64 * SK_WAVES) void gemm_skinny_kernel(const bf16* __restrict__ A, const bf16* __restrict__ W,
                                                                     bf16* __restrict__ C, const bf16* __restrict__ bias, int M,
                                                                     int N, int K, int64_t lda, int64_t ldw, int64_t ldc,
                                                                     int accumulate, GemmEpi ep) {
-  __shared__ f32x4 red[SK_WAVES][MT][NT][64];
+  __shared__ f32x4 red[SK_WAVES][NT][64];
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, c = lane & 15, q = lane >> 4;
   // first W row of group t of this block
   int row0[NT];
@@ -31,29 +31,23 @@ __global__ __launch_bounds__(64 * SK_WAVES) void gemm_skinny_kernel(const bf16* 
     else row0[t] = 16 * (NT * blockIdx.x + t);
   }
   const bf16* wp[NT];
-  const bf16* ap[MT];
 #pragma unroll
   for (int t = 0; t < NT; t++) wp[t] = W + (int64_t)min(row0[t] + c, N - 1) * ldw + 8 * q;
-#pragma unroll
-  for (int m = 0; m < MT; m++) ap[m] = A + (int64_t)min(16 * m + c, M - 1) * lda + 8 * q;
+  const bf16* ap = A + (int64_t)min(c, M - 1) * lda + 8 * q;
 
-  f32x4 acc[MT][NT];
+  f32x4 acc[NT];
 #pragma unroll
-  for (int m = 0; m < MT; m++)
-#pragma unroll
-    for (int t = 0; t < NT; t++) acc[m][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int t = 0; t < NT; t++) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
 
   const int steps = (K + 31) / 32, per = (steps + SK_WAVES - 1) / SK_WAVES;
   const int s0 = wave * per, s1 = min(s0 + per, steps);
-  bf16x8 wf[U][NT], af[U][MT];
+  bf16x8 wf[U][NT], af[U];
   auto multiply = [&]() {
 #pragma unroll
     for (int u = 0; u < U; u++)
 #pragma unroll
-      for (int m = 0; m < MT; m++)
-#pragma unroll
-        for (int t = 0; t < NT; t++)
-          acc[m][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[u][t], af[u][m], acc[m][t], 0, 0, 0);   // rows = n, columns = m
+      for (int t = 0; t < NT; t++)
+        acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[u][t], af[u], acc[t], 0, 0, 0);   // rows = n, columns = m
   };
   int s = s0;
   const int whole = K / 32;   // steps that lie inside K for every lane
@@ -62,8 +56,7 @@ __global__ __launch_bounds__(64 * SK_WAVES) void gemm_skinny_kernel(const bf16* 
     for (int u = 0; u < U; u++) {
 #pragma unroll
       for (int t = 0; t < NT; t++) wf[u][t] = *reinterpret_cast<const bf16x8*>(wp[t] + (int64_t)(s + u) * 32);
-#pragma unroll
-      for (int m = 0; m < MT; m++) af[u][m] = *reinterpret_cast<const bf16x8*>(ap[m] + (int64_t)(s + u) * 32);
+      af[u] = *reinterpret_cast<const bf16x8*>(ap + (int64_t)(s + u) * 32);
     }
     multiply();
   }
@@ -74,27 +67,23 @@ __global__ __launch_bounds__(64 * SK_WAVES) void gemm_skinny_kernel(const bf16* 
       const bool in = s + u < s1 && (s + u) * 32 + 8 * q < K;   // K is a multiple of 8: a chunk is all in or out
 #pragma unroll
       for (int t = 0; t < NT; t++) wf[u][t] = in ? *reinterpret_cast<const bf16x8*>(wp[t] + (int64_t)(s + u) * 32) : zero;
-#pragma unroll
-      for (int m = 0; m < MT; m++) af[u][m] = in ? *reinterpret_cast<const bf16x8*>(ap[m] + (int64_t)(s + u) * 32) : zero;
+      af[u] = in ? *reinterpret_cast<const bf16x8*>(ap + (int64_t)(s + u) * 32) : zero;
     }
     multiply();
   }
 
 #pragma unroll
-  for (int m = 0; m < MT; m++)
-#pragma unroll
-    for (int t = 0; t < NT; t++) red[wave][m][t][lane] = acc[m][t];
+  for (int t = 0; t < NT; t++) red[wave][t][lane] = acc[t];
   __syncthreads();
-  // thread (m-group, lane) owns row 16 mg + c of A and columns 4 q .. 4 q + 3 of every group of W rows
-  if (tid >= 64 * MT) return;
-  const int mg = tid >> 6, row = 16 * mg + c;
-  if (row >= M) return;
+  // lane 16 q + c of the first wavefront owns row c of A and columns 4 q .. 4 q + 3 of every group of W rows
+  const int row = c;
+  if (tid >= 64 || row >= M) return;
   f32x4 v[NT];
 #pragma unroll
   for (int t = 0; t < NT; t++) {
-    v[t] = red[0][mg][t][lane];
+    v[t] = red[0][t][lane];
 #pragma unroll
-    for (int w = 1; w < SK_WAVES; w++) v[t] += red[w][mg][t][lane];
+    for (int w = 1; w < SK_WAVES; w++) v[t] += red[w][t][lane];
   }
   auto rounded = [](f32x4 x) {
     bf16x4 w;
@@ -156,29 +145,21 @@ __global__ __launch_bounds__(64 * SK_WAVES) void gemm_skinny_kernel(const bf16* 
   }
 }
 
-template <int MT, int NT, int U, int EPI>
+template <int NT, int U, int EPI>
 int launch(const char* name, int blocks, const bf16* A, const bf16* W, bf16* C, const bf16* bias, int M, int N, int K, int64_t lda,
            int64_t ldw, int64_t ldc, int accumulate, const GemmEpi& ep, hipStream_t st) {
-  ODY_LAUNCH(name, st, (gemm_skinny_kernel<MT, NT, U, EPI>), dim3(blocks), dim3(64 * SK_WAVES), 0, A, W, C, bias, M, N, K, lda, ldw,
+  ODY_LAUNCH(name, st, (gemm_skinny_kernel<NT, U, EPI>), dim3(blocks), dim3(64 * SK_WAVES), 0, A, W, C, bias, M, N, K, lda, ldw,
              ldc, accumulate, ep);
   return ody_check_launch(name);
 }
 
-template <int NT, int EPI>
-int by_rows(const char* name, int blocks, const bf16* A, const bf16* W, bf16* C, const bf16* bias, int M, int N, int K, int64_t lda,
-            int64_t ldw, int64_t ldc, int accumulate, const GemmEpi& ep, hipStream_t st) {
-  if (M <= 16) return launch<1, NT, 8, EPI>(name, blocks, A, W, C, bias, M, N, K, lda, ldw, ldc, accumulate, ep, st);
-  if (M <= 32) return launch<2, NT, 4, EPI>(name, blocks, A, W, C, bias, M, N, K, lda, ldw, ldc, accumulate, ep, st);
-  return launch<4, NT, 4, EPI>(name, blocks, A, W, C, bias, M, N, K, lda, ldw, ldc, accumulate, ep, st);
-}
-
 }  // namespace
 
-bool ody_gemm_skinny_ok(int epi, int M, int N, int K, int64_t lda, int64_t ldw) {
-  // beyond 16 rows the loads of A weigh as much as those of W, and with many columns the 128 x 128 tiles, which share both
-  // through LDS, fill the chip: 22016 x 4096, M = 32 / 64: 62 / 83 us here, 76 / 77 us there; 4096 x 4096, M = 64: 24 against 71
-  (void)K; (void)lda; (void)ldw;
-  if (M > ODY_SKINNY_MAX_M || (M > 32 && N >= 16384)) return false;
+bool ody_gemm_skinny_ok(int epi, int M, int N) {
+  // one 16-row operand: with a second one the loads of A weigh as much as those of W, and the tile kernel, which shares both
+  // through LDS and cuts K over blocks, is ahead (weights cold, us here / there: 6144 x 4096, M = 8: 17.8 / 17.6, 16: 20.8 / 17.8,
+  // 32: 27.5 / 18.7; 4096 x 4096, M = 8: 10.7 / 14.0, 16: 12.2 / 13.9, 32: 15.5 / 14.2; 2048 x 2048, M = 16: 6.7 / 9.3)
+  if (M > ODY_SKINNY_MAX_M) return false;
   if (epi == EPI_SWIGLU_FWD) return N % 32 == 0;   // whole groups of 16 gate rows and of 16 up rows
   if (epi == EPI_ROPE) return N % 128 == 0;
   return epi == EPI_NONE || epi == EPI_RESIDUAL;
@@ -188,14 +169,14 @@ int ody_launch_gemm_skinny(int epi, const bf16* A, const bf16* W, bf16* C, const
                            int64_t ldw, int64_t ldc, int accumulate, const GemmEpi& ep, hipStream_t st) {
   const int groups = (N + 15) / 16;
   if (epi == EPI_SWIGLU_FWD)
-    return by_rows<2, EPI_SWIGLU_FWD>("gemm_skinny_swiglu", groups / 2, A, W, C, bias, M, N, K, lda, ldw, ldc, accumulate, ep, st);
+    return launch<2, 8, EPI_SWIGLU_FWD>("gemm_skinny_swiglu", groups / 2, A, W, C, bias, M, N, K, lda, ldw, ldc, accumulate, ep, st);
   if (epi == EPI_ROPE)
-    return by_rows<2, EPI_ROPE>("gemm_skinny_rope", groups / 2, A, W, C, bias, M, N, K, lda, ldw, ldc, accumulate, ep, st);
+    return launch<2, 8, EPI_ROPE>("gemm_skinny_rope", groups / 2, A, W, C, bias, M, N, K, lda, ldw, ldc, accumulate, ep, st);
   const bool wide = groups >= 1024;
   if (epi == EPI_RESIDUAL) {
-    if (wide) return by_rows<2, EPI_RESIDUAL>("gemm_skinny_residual", (groups + 1) / 2, A, W, C, bias, M, N, K, lda, ldw, ldc, accumulate, ep, st);
-    return by_rows<1, EPI_RESIDUAL>("gemm_skinny_residual", groups, A, W, C, bias, M, N, K, lda, ldw, ldc, accumulate, ep, st);
+    if (wide) return launch<2, 8, EPI_RESIDUAL>("gemm_skinny_residual", (groups + 1) / 2, A, W, C, bias, M, N, K, lda, ldw, ldc, accumulate, ep, st);
+    return launch<1, 8, EPI_RESIDUAL>("gemm_skinny_residual", groups, A, W, C, bias, M, N, K, lda, ldw, ldc, accumulate, ep, st);
   }
-  if (wide) return by_rows<2, EPI_NONE>("gemm_skinny", (groups + 1) / 2, A, W, C, bias, M, N, K, lda, ldw, ldc, accumulate, ep, st);
-  return by_rows<1, EPI_NONE>("gemm_skinny", groups, A, W, C, bias, M, N, K, lda, ldw, ldc, accumulate, ep, st);
+  if (wide) return launch<2, 8, EPI_NONE>("gemm_skinny", (groups + 1) / 2, A, W, C, bias, M, N, K, lda, ldw, ldc, accumulate, ep, st);
+  return launch<1, 8, EPI_NONE>("gemm_skinny", groups, A, W, C, bias, M, N, K, lda, ldw, ldc, accumulate, ep, st);
 }

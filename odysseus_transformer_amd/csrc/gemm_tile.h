@@ -1,0 +1,477 @@
+// The bf16 tile kernel of the dense products (gemm_nt.hip, gemm_nn.hip, gemm_tn.hip instantiate it per operand orientation).
+//
+// C (M, N) = op(A) . op(B), computed as C^T = op(B)^T . op(A)^T so that a lane ends up with 4 consecutive n of one row.
+//
+// A block of 8 wavefronts owns BM x BN results and walks K in slabs of 64; two wavefronts share each SIMD.  They form two
+// groups (upper and lower half of the rows) that run in anti-phase: while one group multiplies a slab from registers, the
+// other reads its fragments of the next one from LDS and issues the global loads of later ones, and a barrier swaps the roles.
+// The matrix pipe then always has a wavefront that does nothing but MFMAs.  Operands travel from global memory straight to
+// LDS (buffer loads with the LDS bit): no staging registers, no LDS writes, and the loads have a whole slab to land.
+//
+//   A: two stages; each group loads and reads its own half of the rows, so a stage is free as soon as the group is done with it.
+//   B: three stages, loaded by all wavefronts and read by both groups.
+//
+// LDS layout of an operand tile of W rows (or columns) x 64 k, by its layout in memory:
+//   contiguous along K:  [W][64], the eight 16-byte chunks of a row permuted (chunk kc of row r at position kc ^ (r & 7)), read
+//                        with 16-byte reads;
+//   contiguous along W:  [64][W], the 32-byte column groups of a k row permuted (group x of row k at x ^ g(k)), read with the
+//                        transposing read.
+// Both are conflict-free for the 16-row fragments of v_mfma_f32_16x16x32_bf16 and are produced by permuting the SOURCE chunk
+// of each lane, as a direct load writes its 64 lanes to consecutive LDS addresses.
+//
+// Rows and columns past the edge re-read the last valid ones and are not stored.  A last slab that K does not fill reads zeros:
+// those lanes get an offset beyond the buffer descriptor's range.
+//
+// Bound: the package power limit.  With constant operands the NT instance sustains 2170 TFLOP/s (4096 x 4096 x 11008, 87 % of
+// the matrix peak), with random ones 1500.  Measured against the kernel it replaced (4 wavefronts, operands staged through
+// registers), TFLOP/s, 8192^3 / 4096 x 4096 x 11008: NT 1305 -> 1450 / 1347 -> 1520, NN 1283 -> 1443 / 1343 -> 1500, TN
+// 1266 -> 1376 / 1265 -> 1398.
+#pragma once
+#include "gemm_epi.h"
+
+namespace gemm_tile {
+
+constexpr int BK = 64, THREADS = 512;
+constexpr int A_STAGES = 2, B_STAGES = 3;
+
+struct Args {
+  const bf16* A;
+  const bf16* B;
+  bf16* C;
+  const bf16* bias;   // EPI_NONE only, may be NULL
+  const bf16* add;    // EPI_NONE only, may be NULL: C = add + A B (+ bias), added before the one rounding
+  float* part;        // fp32 partial tiles of a call that cuts K, [splits][M][N]
+  int M, N, K;
+  int64_t lda, ldb, ldc, ld_add;
+  int tiles_m, tiles_n;
+  int vec16;          // C (and add) have 16-byte aligned rows
+  GemmEpi ep;
+};
+
+typedef __attribute__((address_space(3))) void* lds_ptr;
+#define ODY_FENCE() __builtin_amdgcn_sched_barrier(0)
+
+constexpr unsigned PAST_END = 0x80000000u;   // beyond every descriptor's range: reads as zero
+
+// column group permutation of a [64][W] tile: the 8 k rows that half a wavefront's transposing read touches (8 q + t, q < 2,
+// t < 4) must fall on different 32-byte groups of the 256 bytes that the banks span
+template <int W> __device__ __forceinline__ int group_perm(int k) {
+  if (W >= 128) return (k & 3) | (((k >> 3) & 1) << 2);
+  return ((k >> 1) & 1) | (((k >> 3) & 1) << 1);   // W = 64: two k rows per 256 bytes
+}
+
+// One operand's share of the direct loads: W rows (columns) x 64 k per stage, brought by NW wavefronts.
+template <bool KC, int W, int NW>
+struct Mover {
+  static constexpr int NINS = W / 8 / NW;           // 1 KB instructions per wavefront and stage
+  static constexpr int LPR = KC ? 8 : W / 8;        // lanes (16-byte chunks) per tile row
+  static constexpr int RPI = 64 / LPR;              // tile rows per instruction
+  // a [64][W] tile's permutation takes two values over a wavefront's instructions, by bit SEL of the instruction
+  static constexpr int SEL = W == 128 && NW == 4 ? 1 : 0;
+  static constexpr int NV = KC ? NINS : (W == 128 && NW == 8 ? 1 : 2);
+  unsigned v[NV];                                    // byte offset of this lane's chunk from the slab's base
+  unsigned step;                                     // bytes between the tile rows of consecutive instructions (k rows, if not KC)
+
+  // row_of(r): operand row of tile row r (KC), or first column of the tile's columns r .. r + 7 (else), clamped to the matrix
+  template <typename F>
+  __device__ __forceinline__ void init(int wv, int lane, int64_t ld, F row_of) {
+    step = (unsigned)(2 * RPI * ld);
+#pragma unroll
+    for (int i = 0; i < NV; i++) {
+      const int j = KC ? i : (SEL ? 2 * i : i), r = (wv * NINS + j) * RPI + lane / LPR, p = lane % LPR;
+      if (KC) v[i] = (unsigned)(2 * ((int64_t)row_of(r) * ld + 8 * (p ^ (r & 7))));
+      else v[i] = (unsigned)(2 * ((int64_t)r * ld + row_of(8 * (p ^ (2 * group_perm<W>(r))))));
+    }
+  }
+  // slab: first element of the operand's slab; krem: k values left from there (>= 64 except in a last, partial slab)
+  __device__ __forceinline__ void load(const bf16* slab, bf16* stage, int wv, int lane, int krem) const {
+    auto rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16*>(slab), (short)0, 0x7fffffff, 0x00020000);
+#pragma unroll
+    for (int j = 0; j < NINS; j++) {
+      const int i = KC ? j : (NV == 1 ? 0 : (j >> SEL) & 1), from = KC ? j : (NV == 1 ? 0 : (SEL ? 2 * i : i));
+      const int k = KC ? 8 * ((lane & 7) ^ (lane >> 3)) : (wv * NINS + j) * RPI + lane / LPR;   // k of the chunk inside the slab
+      const unsigned off = k < krem ? v[i] : PAST_END;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_ptr)(stage + (wv * NINS + j) * 512), 16, (int)off, (int)((j - from) * step), 0, 0);
+    }
+  }
+};
+
+// The fragments of NB 16-row blocks of an operand for both k-steps of a slab: lane 16 q + c holds row c, k = 32 ks + 8 q .. + 7.
+// Transposing reads are inline assembly: the compiler takes the intrinsic for a possible alias of the direct loads in flight and
+// waits for all of them in front of it.  wait() below is what makes their results safe to use.
+template <bool KC, int NB>
+struct Frags {
+  bf16x8 f[2][NB];
+};
+template <int NB>
+struct Frags<false, NB> {
+  s16x4 lo[2][NB], hi[2][NB];
+};
+
+template <int NB>
+__device__ __forceinline__ bf16x8 frag(const Frags<true, NB>& f, int ks, int b) { return f.f[ks][b]; }
+template <int NB>
+__device__ __forceinline__ bf16x8 frag(const Frags<false, NB>& f, int ks, int b) {
+  return concat4(__builtin_bit_cast(bf16x4, f.lo[ks][b]), __builtin_bit_cast(bf16x4, f.hi[ks][b]));
+}
+// ties the fragments to a point behind the wait for them
+template <int NB>
+__device__ __forceinline__ void tie(Frags<true, NB>&) {}
+template <int NB>
+__device__ __forceinline__ void tie(Frags<false, NB>& f) {
+#pragma unroll
+  for (int ks = 0; ks < 2; ks++)
+#pragma unroll
+    for (int b = 0; b < NB; b++) asm volatile("" : "+v"(f.lo[ks][b]), "+v"(f.hi[ks][b]));
+}
+
+template <int OFF0, int OFF1>
+__device__ __forceinline__ void read_tr(unsigned addr, s16x4& lo, s16x4& hi) {
+  asm volatile("ds_read_b64_tr_b16 %0, %2 offset:%3\n\tds_read_b64_tr_b16 %1, %2 offset:%4"
+               : "=&v"(lo), "=&v"(hi)
+               : "v"(addr), "n"(OFF0), "n"(OFF1));
+}
+
+template <bool A_KC, bool B_KC, int BM, int BN, bool SPLITK, int EPI>
+__global__ __launch_bounds__(THREADS, BM * BN <= 128 * 128 ? 4 : 2) void gemm_tile_kernel(const Args p) {
+  constexpr int WM = BM / 32, WN = BN / 64;      // 16-row blocks per wavefront: rows BM / 2, columns BN / 4
+  constexpr int HALF = BM / 2, NH = WN / 2;
+  static_assert(EPI == EPI_NONE || !SPLITK, "fused epilogues: one pass over K");
+  static_assert((EPI != EPI_SWIGLU_FWD && EPI != EPI_ROPE) || (A_KC && B_KC), "these epilogues belong to the NT product");
+  extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
+  bf16* As = reinterpret_cast<bf16*>(smem);      // [A_STAGES][2 halves][HALF x 64]
+  bf16* Bs = As + A_STAGES * BM * BK;            // [B_STAGES][BN x 64]
+
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, c = lane & 15, q = lane >> 4;
+  const int wm = wave >> 2, wn = wave & 3;
+
+  // Block -> tile.  Consecutive ids go round-robin over the 8 XCDs, each with its own L2: give every XCD a contiguous range of
+  // tiles, and inside it walk down M in groups of 8 so that the tiles in flight share panels of both operands.
+  int pid = blockIdx.x;
+  const int nblk = p.tiles_m * p.tiles_n;
+  {
+    const int x = pid & 7, whole = nblk >> 3, extra = nblk & 7;
+    pid = x * whole + min(x, extra) + (pid >> 3);
+  }
+  constexpr int GROUP = 8;
+  const int per_group = GROUP * p.tiles_n, gid = pid / per_group, first_m = gid * GROUP, gsz = min(p.tiles_m - first_m, GROUP);
+  const int tm = first_m + (pid % per_group) % gsz, tn = (pid % per_group) / gsz;
+  const int m0 = tm * BM, n0 = tn * BN;
+
+  // slabs [s0, s0 + nk) of the K range
+  const int slabs = (p.K + BK - 1) / BK;
+  int s0 = 0, nk = slabs;
+  if (SPLITK) {
+    const int per = (slabs + (int)gridDim.y - 1) / (int)gridDim.y;
+    s0 = blockIdx.y * per;
+    nk = max(0, min(slabs - s0, per));
+  }
+
+  Mover<A_KC, HALF, 4> ma;
+  Mover<B_KC, BN, 8> mb;
+  const int j0 = EPI == EPI_SWIGLU_FWD ? tn * (BN / 2) : 0;   // first column of h
+  if (A_KC) ma.init(wn, lane, p.lda, [&](int r) { return min(m0 + wm * HALF + r, p.M - 1) - m0; });
+  else ma.init(wn, lane, p.lda, [&](int col) { return min(m0 + wm * HALF + col, p.M - 8) - m0; });
+  if (EPI == EPI_SWIGLU_FWD)
+    mb.init(wave, lane, p.ldb, [&](int r) { return min(j0 + (r & (BN / 2 - 1)), p.ep.I - 1) + (r < BN / 2 ? 0 : p.ep.I); });
+  else if (B_KC) mb.init(wave, lane, p.ldb, [&](int r) { return min(n0 + r, p.N - 1) - n0; });
+  else mb.init(wave, lane, p.ldb, [&](int col) { return min(n0 + col, p.N - 8) - n0; });
+  const bf16* a_base = A_KC ? p.A + (int64_t)m0 * p.lda : p.A + m0;
+  const bf16* b_base = EPI == EPI_SWIGLU_FWD ? p.B : (B_KC ? p.B + (int64_t)n0 * p.ldb : p.B + n0);
+  const int64_t a_slab = A_KC ? BK : BK * p.lda, b_slab = B_KC ? BK : BK * p.ldb;
+  // loads past the range repeat its last slab: in bounds, and nobody reads them
+  auto load_a = [&](int kt) {
+    const int s = s0 + min(kt, nk - 1);
+    ma.load(a_base + s * a_slab, As + (kt & 1) * BM * BK + wm * HALF * BK, wn, lane, p.K - s * BK);
+  };
+  auto load_b = [&](int kt, int slot) {
+    const int s = s0 + min(kt, nk - 1);
+    mb.load(b_base + s * b_slab, Bs + slot * BN * BK, wave, lane, p.K - s * BK);
+  };
+
+  // tile row (column) of this wavefront's n block b
+  auto nblock = [&](int b) {
+    if (EPI == EPI_SWIGLU_FWD) return (b / NH) * (BN / 2) + wn * 16 * NH + 16 * (b % NH);      // gate blocks, then their up blocks
+    if (EPI == EPI_ROPE) {                                                                      // j blocks of a head, then j + 64
+      constexpr int WPH = 4 / (BN / 128);
+      return (wn / WPH) * 128 + (b / NH) * 64 + (wn % WPH) * 16 * NH + 16 * (b % NH);
+    }
+    return wn * 16 * WN + 16 * b;
+  };
+  const unsigned lds0 = (unsigned)(uintptr_t)(lds_ptr)smem;
+  const int kc_off = c * BK + 8 * (q ^ (c & 7));                                               // + 64 * row block, ^ 32 for ks = 1
+  const int a_tr = A_KC ? 0 : (8 * q + (c >> 2)) * HALF + 16 * group_perm<HALF>(8 * q + (c >> 2)) + 4 * (c & 3);
+  const int b_tr = B_KC ? 0 : (8 * q + (c >> 2)) * BN + 16 * ((wn * WN) ^ group_perm<BN>(8 * q + (c >> 2))) + 4 * (c & 3);
+
+  f32x4 acc[WM][WN];
+#pragma unroll
+  for (int a = 0; a < WM; a++)
+#pragma unroll
+    for (int b = 0; b < WN; b++) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  if (nk > 0) {
+    constexpr int NA = Mover<A_KC, HALF, 4>::NINS, NB = Mover<B_KC, BN, 8>::NINS;
+    load_b(0, 0);
+    load_a(0);
+    load_b(1, 1);
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NB) : "memory");
+    __builtin_amdgcn_s_barrier();
+    if (wm == 1) __builtin_amdgcn_s_barrier();   // the second group runs one phase behind
+    int slot = 0;
+    for (int kt = 0; kt < nk; kt++) {
+      const bf16* At = As + (kt & 1) * BM * BK + wm * HALF * BK;
+      const bf16* Bt = Bs + slot * BN * BK;
+      Frags<A_KC, WM> fa;
+      Frags<B_KC, WN> fb;
+      // ---- memory phase: this slab's fragments; A of the next slab, B of the one after (its stage was read last two phases ago)
+      ODY_FENCE();
+#pragma unroll
+      for (int ks = 0; ks < 2; ks++) {
+        if constexpr (B_KC) {
+#pragma unroll
+          for (int b = 0; b < WN; b++) fb.f[ks][b] = *reinterpret_cast<const bf16x8*>(Bt + (kc_off ^ (32 * ks)) + nblock(b) * BK);
+        } else {
+#pragma unroll
+          for (int b = 0; b < WN; b++) {
+            const unsigned at = lds0 + 2 * ((int)(Bt - As) + (b_tr ^ (16 * b)));
+            if (ks == 0) read_tr<0, 8 * BN>(at, fb.lo[0][b], fb.hi[0][b]);
+            else read_tr<64 * BN, 72 * BN>(at, fb.lo[1][b], fb.hi[1][b]);
+          }
+        }
+        if constexpr (A_KC) {
+#pragma unroll
+          for (int a = 0; a < WM; a++) fa.f[ks][a] = *reinterpret_cast<const bf16x8*>(At + (kc_off ^ (32 * ks)) + 16 * a * BK);
+        } else {
+#pragma unroll
+          for (int a = 0; a < WM; a++) {
+            const unsigned at = lds0 + 2 * ((int)(At - As) + (a_tr ^ (16 * a)));
+            if (ks == 0) read_tr<0, 8 * HALF>(at, fa.lo[0][a], fa.hi[0][a]);
+            else read_tr<64 * HALF, 72 * HALF>(at, fa.lo[1][a], fa.hi[1][a]);
+          }
+        }
+        ODY_FENCE();
+        if (ks == 0) load_a(kt + 1);
+        else load_b(kt + 2, slot == 0 ? 2 : slot - 1);
+        ODY_FENCE();
+      }
+      // this wavefront's part of B's next slab has landed (the other group may read it two barriers from here)
+      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(NA + NB) : "memory");
+      tie(fa);
+      tie(fb);
+      __builtin_amdgcn_s_barrier();
+      ODY_FENCE();
+      // ---- compute phase
+#pragma unroll
+      for (int ks = 0; ks < 2; ks++)
+#pragma unroll
+        for (int a = 0; a < WM; a++)
+#pragma unroll
+          for (int b = 0; b < WN; b++)
+            acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(frag(fb, ks, b), frag(fa, ks, a), acc[a][b], 0, 0, 0);   // rows = n, columns = m
+      ODY_FENCE();
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NB) : "memory");   // A of the next slab has landed
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+      slot = slot == 2 ? 0 : slot + 1;
+    }
+    if (wm == 0) __builtin_amdgcn_s_barrier();
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  }
+  __syncthreads();   // the epilogue reuses the operand stages
+
+  // ---- epilogue.  Lane 16 q + c holds row m = c and columns n = 4 q .. 4 q + 3 of each 16 x 16 block; the blocks leave through a
+  // patch of LDS that belongs to the wavefront (its LDS operations complete in order), 32 rows at a time, as 16-byte pieces of
+  // rows, by streaming stores: this kernel does not read them again.
+  constexpr int COLS = 16 * WN;
+  const int mw = m0 + wm * HALF;
+  auto store16 = [](bf16* dst, bf16x8 w) {
+    typedef unsigned raw_t __attribute__((ext_vector_type(4)));
+    __builtin_nontemporal_store(__builtin_bit_cast(raw_t, w), reinterpret_cast<raw_t*>(dst));
+  };
+  auto rounded = [](f32x4 x) {
+    bf16x4 w;
+#pragma unroll
+    for (int e = 0; e < 4; e++) w[e] = (bf16)x[e];
+    return w;
+  };
+  auto biased = [&](f32x4 x, int b) {
+    if (EPI == EPI_NONE && !SPLITK && p.bias) {
+      const bf16x4 bv = *reinterpret_cast<const bf16x4*>(p.bias + min(n0 + wn * COLS + 16 * b + 4 * q, p.N - 4));
+#pragma unroll
+      for (int e = 0; e < 4; e++) x[e] += (float)bv[e];
+    }
+    return x;
+  };
+  if constexpr (SPLITK) {
+    constexpr int EP = COLS + 4, CPR = COLS / 4, RPP = 64 / CPR;
+    float* band = reinterpret_cast<float*>(smem) + wave * 32 * EP;
+    float* dst = p.part + (int64_t)blockIdx.y * p.M * p.N;
+#pragma unroll
+    for (int a2 = 0; a2 < WM / 2; a2++) {
+      ODY_FENCE();
+#pragma unroll
+      for (int t = 0; t < 2; t++)
+#pragma unroll
+        for (int b = 0; b < WN; b++) *reinterpret_cast<f32x4*>(band + (16 * t + c) * EP + 16 * b + 4 * q) = acc[2 * a2 + t][b];
+#pragma unroll
+      for (int pass = 0; pass < 32 / RPP; pass++) {
+        const int row = pass * RPP + lane / CPR, ch = lane % CPR, m = mw + 32 * a2 + row, n = n0 + wn * COLS + 4 * ch;
+        const f32x4 v = *reinterpret_cast<const f32x4*>(band + row * EP + 4 * ch);
+        if (m < p.M && n < p.N) *reinterpret_cast<f32x4*>(dst + (int64_t)m * p.N + n) = v;
+      }
+    }
+    return;
+  }
+  if constexpr (EPI == EPI_NONE) {
+    if (!p.vec16) {   // rows of C that 16-byte pieces cannot address
+#pragma unroll
+      for (int a = 0; a < WM; a++) {
+        ODY_FENCE();
+        int m = mw + 16 * a + c;
+        asm volatile("" : "+v"(m));   // addresses are made here, not all at once in front
+#pragma unroll
+        for (int b = 0; b < WN; b++) {
+          const int n = n0 + wn * COLS + 16 * b + 4 * q;
+          if (m >= p.M || n >= p.N) continue;
+          f32x4 v = biased(acc[a][b], b);
+          if (p.add) {
+            const bf16x4 o = *reinterpret_cast<const bf16x4*>(p.add + (int64_t)m * p.ld_add + n);
+#pragma unroll
+            for (int e = 0; e < 4; e++) v[e] += (float)o[e];
+          }
+          *reinterpret_cast<bf16x4*>(p.C + (int64_t)m * p.ldc + n) = rounded(v);
+        }
+      }
+      return;
+    }
+    if (p.add) {   // fp32 bands, so that the sum is rounded once
+      constexpr int EP = COLS + 4, CPR = COLS / 8, RPP = 64 / CPR;
+      float* band = reinterpret_cast<float*>(smem) + wave * 32 * EP;
+#pragma unroll
+      for (int a2 = 0; a2 < WM / 2; a2++) {
+        ODY_FENCE();
+#pragma unroll
+        for (int t = 0; t < 2; t++)
+#pragma unroll
+          for (int b = 0; b < WN; b++) *reinterpret_cast<f32x4*>(band + (16 * t + c) * EP + 16 * b + 4 * q) = biased(acc[2 * a2 + t][b], b);
+#pragma unroll
+        for (int pass = 0; pass < 32 / RPP; pass++) {
+          const int row = pass * RPP + lane / CPR, ch = lane % CPR, m = mw + 32 * a2 + row, n = n0 + wn * COLS + 8 * ch;
+          const f32x4 v0 = *reinterpret_cast<const f32x4*>(band + row * EP + 8 * ch);
+          const f32x4 v1 = *reinterpret_cast<const f32x4*>(band + row * EP + 8 * ch + 4);
+          if (m < p.M && n < p.N) {
+            const bf16x8 r = *reinterpret_cast<const bf16x8*>(p.add + (int64_t)m * p.ld_add + n);
+            bf16x8 w;
+#pragma unroll
+            for (int e = 0; e < 4; e++) w[e] = (bf16)(v0[e] + (float)r[e]), w[4 + e] = (bf16)(v1[e] + (float)r[4 + e]);
+            store16(p.C + (int64_t)m * p.ldc + n, w);
+          }
+        }
+      }
+      return;
+    }
+  }
+  // bf16 bands
+  constexpr int EP = COLS + 8, CPR = COLS / 8, RPP = 64 / CPR;
+  bf16* band = reinterpret_cast<bf16*>(smem) + wave * 32 * EP;
+#pragma unroll
+  for (int a2 = 0; a2 < WM / 2; a2++) {
+    ODY_FENCE();
+    bf16x4 w[2][WN];
+#pragma unroll
+    for (int t = 0; t < 2; t++) {
+      const int m = min(mw + 32 * a2 + 16 * t + c, p.M - 1);
+      if (EPI == EPI_ROPE && n0 + nblock(0) < p.ep.I) {   // this wavefront's head is a query or key head
+#pragma unroll
+        for (int b = 0; b < NH; b++) {
+          const int j = (nblock(b) & 127) + 4 * q;         // (cos, sin) of frequencies j .. j + 3: 16 bytes of the token's table row
+          const bf16x8 cs = *reinterpret_cast<const bf16x8*>(p.ep.aux + (int64_t)m * p.ep.ld_aux + 2 * j);
+          f32x4 o1, o2;
+#pragma unroll
+          for (int e = 0; e < 4; e++) {
+            const float co = (float)cs[2 * e], sn = (float)cs[2 * e + 1], x1 = acc[2 * a2 + t][b][e], x2 = acc[2 * a2 + t][b + NH][e];
+            o1[e] = x1 * co - x2 * sn;
+            o2[e] = x2 * co + x1 * sn;
+          }
+          w[t][b] = rounded(o1), w[t][b + NH] = rounded(o2);
+        }
+      } else {
+#pragma unroll
+        for (int b = 0; b < WN; b++) w[t][b] = rounded(biased(acc[2 * a2 + t][b], b));
+      }
+#pragma unroll
+      for (int b = 0; b < WN; b++) *reinterpret_cast<bf16x4*>(band + (16 * t + c) * EP + 16 * b + 4 * q) = w[t][b];
+    }
+#pragma unroll
+    for (int pass = 0; pass < 32 / RPP; pass++) {
+      const int row = pass * RPP + lane / CPR, ch = lane % CPR, m = mw + 32 * a2 + row;
+      const bf16x8 v = *reinterpret_cast<const bf16x8*>(band + row * EP + 8 * ch);
+      const int b = ch >> 1;
+      if constexpr (EPI == EPI_SWIGLU_FWD) {
+        const int j = j0 + wn * 16 * NH + 16 * (b % NH) + 8 * (ch & 1);
+        if (m < p.M && j < p.ep.I) store16(p.C + (int64_t)m * p.ldc + (b / NH) * p.ep.I + j, v);
+      } else if constexpr (EPI == EPI_SWIGLU_BWD) {
+        const int j = n0 + wn * COLS + 8 * ch;
+        if (m < p.M && j < p.N) {
+          const bf16* gu = p.ep.aux + (int64_t)m * p.ep.ld_aux + j;
+          const bf16x8 gt = *reinterpret_cast<const bf16x8*>(gu), up = *reinterpret_cast<const bf16x8*>(gu + p.ep.I);
+          bf16x8 d1, d3;
+#pragma unroll
+          for (int e = 0; e < 8; e++) {
+            const float a1 = (float)gt[e], a3 = (float)up[e], gg = (float)v[e];
+            const float sig = 1.f / (1.f + __expf(-a1));
+            d1[e] = (bf16)(gg * a3 * sig * (1.f + a1 * (1.f - sig)));
+            d3[e] = (bf16)(gg * a1 * sig);
+          }
+          store16(p.C + (int64_t)m * p.ldc + j, d1);
+          store16(p.C + (int64_t)m * p.ldc + p.ep.I + j, d3);
+        }
+      } else {
+        const int n = n0 + nblock(b) + 8 * (ch & 1);
+        if (m < p.M && n < p.N) store16(p.C + (int64_t)m * p.ldc + n, v);
+      }
+    }
+    if constexpr (EPI == EPI_SWIGLU_FWD) {
+      // h from the rounded values: block b of the first half is the gate of block b of the second
+      constexpr int EPH = COLS / 2 + 8, CPH = COLS / 16, RPH = 64 / CPH;
+#pragma unroll
+      for (int t = 0; t < 2; t++)
+#pragma unroll
+        for (int b = 0; b < NH; b++) {
+          bf16x4 hv;
+#pragma unroll
+          for (int e = 0; e < 4; e++) {
+            const float a1 = (float)w[t][b][e], a3 = (float)w[t][b + NH][e];
+            hv[e] = (bf16)(a1 / (1.f + __expf(-a1)) * a3);
+          }
+          *reinterpret_cast<bf16x4*>(band + (16 * t + c) * EPH + 16 * b + 4 * q) = hv;
+        }
+#pragma unroll
+      for (int pass = 0; pass < (32 + RPH - 1) / RPH; pass++) {
+        const int row = pass * RPH + lane / CPH, ch = lane % CPH, m = mw + 32 * a2 + row, j = j0 + wn * 16 * NH + 8 * ch;
+        const bf16x8 v = *reinterpret_cast<const bf16x8*>(band + row * EPH + 8 * ch);
+        if (m < p.M && j < p.ep.I) store16(p.ep.out2 + (int64_t)m * p.ep.ld_out2 + j, v);
+      }
+    }
+  }
+}
+#undef ODY_FENCE
+
+template <bool A_KC, bool B_KC, int BM, int BN, bool SPLITK, int EPI>
+int launch(const char* name, Args a, int splits, hipStream_t st) {
+  constexpr size_t smem = sizeof(bf16) * BK * (A_STAGES * BM + B_STAGES * BN);
+  static_assert(smem >= 8 * 32 * (BN / 4 + 4) * sizeof(float), "the fp32 bands fit in the operand stages");
+  auto kern = &gemm_tile_kernel<A_KC, B_KC, BM, BN, SPLITK, EPI>;
+  if (int rc = ody_allow_dynamic_lds(reinterpret_cast<const void*>(kern), smem, name)) return rc;
+  a.tiles_m = (a.M + BM - 1) / BM, a.tiles_n = (a.N + BN - 1) / BN;
+  if (EPI == EPI_SWIGLU_FWD) a.tiles_n = (a.ep.I + BN / 2 - 1) / (BN / 2);
+  ODY_LAUNCH(name, st, kern, dim3(a.tiles_m * a.tiles_n, splits), dim3(THREADS), smem, a);
+  return ody_check_launch(name);
+}
+
+}  // namespace gemm_tile
+
+// one per orientation: tile BM x BN, K cut into `splits` ranges (EPI_NONE only, partials to a.part)
+int ody_launch_gemm_nt(int epi, int BM, int BN, int splits, const gemm_tile::Args& a, hipStream_t st);
+int ody_launch_gemm_nn(int epi, int BM, int BN, int splits, const gemm_tile::Args& a, hipStream_t st);
+int ody_launch_gemm_tn(int BM, int BN, int splits, const gemm_tile::Args& a, hipStream_t st);

@@ -155,14 +155,12 @@ class LlamaFlashAttention2TPSP(nn.Module):
             if not self.sequence_parallel:
                 hidden_states = allgather_bsz1(hidden_states)
             if general:
-                if self._can_fuse_rope(hidden_states) and not torch.is_grad_enabled():
-                    # inference: the rotation rides in the projection's epilogue
-                    table = ops.rope_table(position_ids, q_len, D, self.rope_theta, device=hidden_states.device)
-                    qkv = ops.linear_rope(hidden_states.reshape(q_len, -1), self.qkv_proj.weight, table, nh + nkv, D)
+                if self._can_fuse_rope(hidden_states):   # the rotation rides in the projection's epilogue
+                    qkv = ops.run_function(ops.LinearRoPEFunc, hidden_states, self.qkv_proj.weight, nh + nkv, D, position_ids,
+                                           self.rope_theta)
                 else:
                     qkv = self.qkv_proj(hidden_states).view(bsz, q_len, nh + 2 * nkv, D)
                     qkv = ops.apply_rope_packed(qkv, nh + nkv, position_ids, self.rope_theta)
-                qkv = qkv.view(bsz, q_len, nh + 2 * nkv, D)
                 attn_output = self._attend_general(qkv[:, :, :nh], qkv[:, :, nh:nh + nkv], qkv[:, :, nh + nkv:],
                                                    attention_mask, past_key_value, cache_position, scale, dropout)
             elif self._can_fuse_rope(hidden_states):

@@ -374,6 +374,12 @@ def _rowmajor2d(t: torch.Tensor, name: str) -> int:
     return t.stride(0) if t.shape[0] > 1 else max(t.stride(0), t.shape[1])
 
 
+def _gemm_scratch(op: int, M: int, N: int, K: int, like):
+    """(bytes, scratch or None) for a product that cuts K into ranges."""
+    n = _lib.load().ody_gemm_workspace_bytes(op, M, N, K, _dt(like))
+    return n, (scratch(n, "gemm_workspace", like.device) if n else None)
+
+
 def gemm(op: int, a, b, bias=None, out=None, accumulate: bool = False):
     """op NT: a (M,K) b (N,K); NN: a (M,K) b (K,N); TN: a (K,M) b (K,N) -> (M,N)."""
     _need_gpu(a, b, bias, out)
@@ -397,8 +403,7 @@ def gemm(op: int, a, b, bias=None, out=None, accumulate: bool = False):
         raise ValueError(f"out must be ({M}, {N}) {a.dtype}, got {tuple(out.shape)} {out.dtype}")
     if bias is not None and (tuple(bias.shape) != (N,) or bias.dtype != a.dtype or not bias.is_contiguous()):
         raise ValueError(f"bias must be a contiguous ({N},) {a.dtype} tensor, got {tuple(bias.shape)} {bias.dtype}")
-    ws_bytes = _lib.load().ody_gemm_workspace_bytes(op, M, N, K, _dt(a))
-    ws = scratch(ws_bytes, "gemm_workspace", a.device) if ws_bytes else None
+    ws_bytes, ws = _gemm_scratch(op, M, N, K, a)
     _lib.call("ody_gemm", op, a.data_ptr(), b.data_ptr(), out.data_ptr(), 0 if bias is None else bias.data_ptr(),
               M, N, K, _rowmajor2d(a, "a"), _rowmajor2d(b, "b"), _rowmajor2d(out, "out"),
               int(accumulate), _dt(a), ws.data_ptr() if ws is not None else 0, ws_bytes, _stream())
@@ -422,9 +427,10 @@ def linear_residual(x, weight, residual):
         raise ValueError(f"linear_residual: x {tuple(x.shape)}, weight {tuple(weight.shape)}, residual "
                          f"{tuple(residual.shape)} {residual.dtype} do not fit")
     y = torch.empty((M, N), dtype=x.dtype, device=x.device)
-    _lib.call("ody_linear_residual", x.data_ptr(), weight.data_ptr(), residual.data_ptr(), y.data_ptr(), M, N, K,
+    ws_bytes, ws = _gemm_scratch(GEMM_NT, M, N, K, x)
+    _lib.call("ody_linear_residual_ws", x.data_ptr(), weight.data_ptr(), residual.data_ptr(), y.data_ptr(), M, N, K,
               _rowmajor2d(x, "x"), _rowmajor2d(weight, "weight"), _rowmajor2d(residual, "residual"), y.stride(0),
-              _dt(x), _stream())
+              _dt(x), 0 if ws is None else ws.data_ptr(), ws_bytes, _stream())
     return y
 
 
@@ -493,8 +499,10 @@ def linear_rope(x, weight, table, n_rot: int, head_dim: int):
     if table.dtype != torch.bfloat16 or tuple(table.shape) != (M, head_dim) or not table.is_contiguous():
         raise ValueError(f"linear_rope: table must be a contiguous bfloat16 ({M}, {head_dim}) tensor")
     y = torch.empty((M, N), dtype=x.dtype, device=x.device)
-    _lib.call("ody_linear_rope", x.data_ptr(), weight.data_ptr(), table.data_ptr(), y.data_ptr(), M, N, K, n_rot, head_dim,
-              _rowmajor2d(x, "x"), _rowmajor2d(weight, "weight"), table.stride(0), y.stride(0), _dt(x), _stream())
+    ws_bytes, ws = _gemm_scratch(GEMM_NT, M, N, K, x)
+    _lib.call("ody_linear_rope_ws", x.data_ptr(), weight.data_ptr(), table.data_ptr(), y.data_ptr(), M, N, K, n_rot, head_dim,
+              _rowmajor2d(x, "x"), _rowmajor2d(weight, "weight"), table.stride(0), y.stride(0), _dt(x),
+              0 if ws is None else ws.data_ptr(), ws_bytes, _stream())
     return y
 
 
@@ -955,6 +963,30 @@ class QKVRoPEAttnFunc(torch.autograd.Function):
         dx = gemm(GEMM_NN, d2, weight).view(x_shape)
         dw = gemm(GEMM_TN, d2, x2)
         return dx, dw, None, None, None, None, None, None
+
+
+class LinearRoPEFunc(torch.autograd.Function):
+    """Packed projection x W^T (bf16, head_dim 128) with its first n_rot heads rotated in the product's epilogue; the backward
+    un-rotates the gradient and runs the two products.  Returns (B, L, H, D)."""
+
+    @staticmethod
+    def forward(ctx, x, weight, n_rot, head_dim, position_ids, rope_base):
+        B, L, K = x.shape
+        x2 = x.reshape(B * L, K)
+        x2 = x2 if x2.stride(1) == 1 else x2.contiguous()
+        table = rope_table(position_ids, B * L, head_dim, rope_base, device=x.device)
+        ctx.save_for_backward(x2, weight, position_ids)
+        ctx.dims = (n_rot, rope_base, x.shape)
+        return linear_rope(x2, weight, table, n_rot, head_dim).view(B, L, -1, head_dim)
+
+    @staticmethod
+    def backward(ctx, dy):
+        x2, weight, position_ids = ctx.saved_tensors
+        n_rot, rope_base, x_shape = ctx.dims
+        d = dy.clone(memory_format=torch.contiguous_format)
+        rope_(d, n_rot, position_ids, rope_base, inverse=True)
+        d2 = d.view(x2.shape[0], -1)
+        return gemm(GEMM_NN, d2, weight).view(x_shape), gemm(GEMM_TN, d2, x2), None, None, None, None
 
 
 class SwiGLUMLPResidualFunc(torch.autograd.Function):

@@ -248,14 +248,14 @@ def test_rope_table_is_reused_for_the_same_position_tensor_only(dev):
 
 @pytest.mark.parametrize("M", [1, 16, 17, 40, 64])
 def test_fused_epilogues_with_few_rows(M, dev):
-    """Residual, SwiGLU and rotary epilogues of the kernel for few rows, against fp32 products."""
+    """Residual, SwiGLU and rotary epilogues of the kernel for few rows (and of the next one beyond its 16), against fp32 products."""
     from odysseus_transformer_amd import ops
     K, D, H, I = 264, 128, 3, 176
     x = randn((M, K), 9600, dtype=BF)
     r, w, wgu = randn((M, H * D), 9601, dtype=BF), randn((H * D, K), 9602, std=0.05, dtype=BF), randn((2 * I, K), 9603, std=0.05, dtype=BF)
     pos = torch.randint(0, 9000, (1, M), generator=torch.Generator().manual_seed(9604)).to(dev)
     y, names = _kernels_of(lambda: ops.linear_residual(x.to(dev), w.to(dev), r.to(dev)))
-    assert any("skinny" in n for n in names), names
+    assert any("skinny" in n for n in names) == (M <= 16), names
     plain = x.float() @ w.float().t()
     assert rel_err(y, plain + r.float()) <= TOL_BF16, "residual"
     gu, h = ops.linear_swiglu(x.to(dev), wgu.to(dev))
@@ -269,3 +269,29 @@ def test_fused_epilogues_with_few_rows(M, dev):
     a, b = plain.view(M, H, D)[:, :2].split(64, dim=-1)
     want = torch.cat([torch.cat([a * c - b * s, b * c + a * s], -1), plain.view(M, H, D)[:, 2:]], 1)
     assert rel_err(got, want) <= TOL_BF16, "rope"
+
+
+@pytest.mark.parametrize("T,I,K", [(65, 128, 72), (200, 384, 4096), (1000, 640, 520), (3001, 1408, 264)])
+def test_fused_epilogues_on_ragged_rows(T, I, K, dev):
+    """Rows and K that fill no tile, with and without K cut into ranges: SwiGLU both ways bit for bit against the two-kernel
+    path, residual and rotary epilogues against fp32 products."""
+    from odysseus_transformer_amd import ops
+    x, wgu = randn((T, K), 9700, dtype=BF).to(dev), randn((2 * I, K), 9701, std=0.05, dtype=BF).to(dev)
+    (gu, h), names = _kernels_of(lambda: ops.linear_swiglu(x, wgu))
+    assert "gemm_bf16_nt_swiglu" in names, names
+    assert rel_err(gu, x.float() @ wgu.float().t()) <= TOL_BF16
+    assert torch.equal(h, ops.swiglu_fwd(gu)), "h differs from the stand-alone SwiGLU kernel"
+    dy, wd = randn((T, K), 9702, dtype=BF).to(dev), randn((K, I), 9703, std=0.05, dtype=BF).to(dev)
+    dgu, names = _kernels_of(lambda: ops.linear_dgrad_swiglu(dy, wd, gu))
+    assert "gemm_bf16_nn_swiglu_bwd" in names, names
+    ref = oracle.swiglu_bwd(gu.float().cpu(), (dy.float() @ wd.float()).cpu())
+    assert_parity(dgu, ref, TOL_BF16, "d_gate_up")
+    w, r = randn((I, K), 9704, std=0.05, dtype=BF).to(dev), randn((T, I), 9705, dtype=BF).to(dev)
+    plain = x.float() @ w.float().t()
+    assert rel_err(ops.linear_residual(x, w, r), plain + r.float()) <= 4e-3
+    table = ops.rope_table(torch.arange(T, device=dev)[None] * 3, T, 128)
+    got = ops.linear_rope(x, w, table, I // 128 - 1, 128).float().view(T, I // 128, 128)
+    c, s = table.float()[:, None, 0::2], table.float()[:, None, 1::2]
+    p = plain.view(T, I // 128, 128)
+    a, b = p[:, :-1].split(64, dim=-1)
+    assert rel_err(got, torch.cat([torch.cat([a * c - b * s, b * c + a * s], -1), p[:, -1:]], 1)) <= 1e-2

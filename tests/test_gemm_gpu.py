@@ -152,3 +152,41 @@ def test_products_with_few_rows(M, N, K, dev):
     out = torch.ones((M, N), dtype=torch.bfloat16, device=dev)
     ops.gemm(ops.GEMM_NT, xd, wd, bias=bias.to(dev), out=out, accumulate=True)
     assert rel_err(out, ref + bias.float() + 1.0) <= TOL_BF16, "y + bias + C"
+
+
+@pytest.mark.parametrize("op", ["nt", "nn", "tn"])
+@pytest.mark.parametrize("M,N,K", [(72, 8, 8), (128, 264, 72), (136, 248, 64), (248, 256, 1000), (264, 520, 200), (1000, 1096, 2056),
+                                   (2056, 4104, 136), (4104, 5128, 72)], ids=lambda v: str(v))
+def test_tile_edges(op, M, N, K, dev):
+    """The tile kernel around its edges in all three extents: rows and columns on both sides of 64, 128 and 256, a partial last
+    slab of K, K cut into ranges, padded pitches whose padding is not a number, bias and accumulation."""
+    from odysseus_transformer_amd import ops
+    print(f"tile edges {op} M={M} N={N} K={K}", flush=True)
+    nan = float("nan")
+
+    def padded(r, c, seed, std=1.0):
+        t = torch.full((r, c + 8), nan, dtype=torch.bfloat16, device=dev)
+        t[:, :c] = randn((r, c), seed, std=std, dtype=torch.bfloat16).to(dev)
+        return t[:, :c]
+    a = padded(*((K, M) if op == "tn" else (M, K)), 41)
+    b = padded(*((N, K) if op == "nt" else (K, N)), 42, 0.05)
+    code = {"nt": ops.GEMM_NT, "nn": ops.GEMM_NN, "tn": ops.GEMM_TN}[op]
+    ref = (a.float().t() if op == "tn" else a.float()) @ (b.float().t() if op == "nt" else b.float())
+    assert rel_err(ops.gemm(code, a, b), ref) <= TOL_BF16
+    bias = randn((N,), 43, dtype=torch.bfloat16).to(dev)
+    for pad in (8, 4):                                  # rows of C with and without 16-byte alignment
+        out = torch.ones((M, N + pad), dtype=torch.bfloat16, device=dev)
+        ops.gemm(code, a, b, bias=bias, out=out[:, :N], accumulate=True)
+        assert rel_err(out[:, :N], ref + bias.float() + 1.0) <= TOL_BF16
+        assert bool((out[:, N:] == 1).all()), "columns beyond N were written"
+
+
+def test_row_pitch_beyond_the_tile_kernels_offsets(dev):
+    """A pitch of more than 2^22 elements takes the kernel with 64-bit offsets."""
+    from odysseus_transformer_amd import ops
+    M, N, K, pitch = 72, 136, 64, (1 << 22) + 8
+    flat = torch.zeros(M * pitch, dtype=torch.bfloat16, device=dev)
+    a = flat.as_strided((M, K), (pitch, 1))
+    a.copy_(randn((M, K), 44, dtype=torch.bfloat16))
+    w = randn((N, K), 45, std=0.05, dtype=torch.bfloat16).to(dev)
+    assert rel_err(ops.gemm(ops.GEMM_NT, a, w), a.float() @ w.float().t()) <= TOL_BF16
