@@ -14,6 +14,13 @@
 // cross-lane traffic beyond one swap of the wavefront halves, and the result registers
 // are directly the B operand of the next product.
 //
+// SPLIT instances serve calls with few rows, whose 128-row workgroups would leave compute units idle (and, under a causal
+// mask, wait for the longest): the wavefronts (eight at head_dim 64) own the SAME 32 rows and take the streamed tiles in turn, each through
+// LDS of its own (no barrier in the loop), and add their results up through LDS at the end.  8 heads x 64, L = 2048,
+// causal: forward 162 -> 63 us, dQ 237 -> 81, dK / dV 304 -> 109; 8 x 64, L = 8192 (one 128-row workgroup per half compute
+// unit): 840 -> 688, 1238 -> 913, 1610 -> 1275; the line lies at the
+// widest launches tried.
+//
 // Two index permutations keep every LDS read conflict-free and 16 bytes wide where it
 // can be:
 //  * contraction over head_dim: k-step 4 j + t multiplies element 8 j + 4 g + t, so the
@@ -40,16 +47,16 @@ __device__ __forceinline__ f32x16 mfma_f32(float a, float b, f32x16 c) {
 // row of a 32-row tile that result register r of a lane in half g holds
 __device__ __forceinline__ int acc_row(int r, int g) { return 8 * (r >> 2) + 4 * g + (r & 3); }
 
-// One 32-row tile of a (rows, D) fp32 matrix on its way from global memory to LDS:
-// D / 32 16-byte pieces per thread, rows past `nvalid` read as zero.
-template <int D>
+// One 32-row tile of a (rows, D) fp32 matrix on its way from global memory to LDS, brought by NT threads: 8 D / NT
+// 16-byte pieces per thread, rows past `nvalid` read as zero.
+template <int D, int NT>
 struct TileRegs {
-  static constexpr int N = D / 32, LD = D + 4;
+  static constexpr int N = 8 * D / NT, LD = D + 4;
   f32x4 v[N];
   __device__ __forceinline__ void fetch(const float* src, int64_t stride, int row0, int nvalid, int tid) {
 #pragma unroll
     for (int c = 0; c < N; c++) {
-      const int e = tid + c * F_THREADS, r = e / (D / 4), x = e % (D / 4);
+      const int e = tid + c * NT, r = e / (D / 4), x = e % (D / 4);
       v[c] = (r < nvalid) ? *reinterpret_cast<const f32x4*>(src + (int64_t)(row0 + r) * stride + 4 * x)
                           : f32x4{0.f, 0.f, 0.f, 0.f};
     }
@@ -57,11 +64,54 @@ struct TileRegs {
   __device__ __forceinline__ void put(float* dst, int tid) const {
 #pragma unroll
     for (int c = 0; c < N; c++) {
-      const int e = tid + c * F_THREADS, r = e / (D / 4), x = e % (D / 4);
+      const int e = tid + c * NT, r = e / (D / 4), x = e % (D / 4);
       *reinterpret_cast<f32x4*>(dst + r * LD + 4 * x) = v[c];
     }
   }
 };
+
+// Geometry of an instance: who owns which rows, who streams which tiles, through which LDS.
+template <int D, bool SPLIT>
+struct Shape {
+  static constexpr int LD = D + 4;
+  // as many as the tiles in LDS allow: two per SIMD at head_dim 64, one at 128
+  static constexpr int WAVES = SPLIT && D == 64 ? 8 : F_WAVES, THREADS = 64 * WAVES;
+  static constexpr int ROWS = SPLIT ? 32 : F_ROWS;                 // rows owned by a workgroup
+  static constexpr int LOADERS = SPLIT ? 64 : F_THREADS;           // threads that bring one tile
+  static constexpr int STEP = SPLIT ? WAVES * F_TILE : F_TILE;   // streamed rows between two turns of a wavefront
+  static constexpr int TILES = SPLIT ? WAVES : 1;                // tiles of each kind in LDS
+  __device__ static __forceinline__ void sync() {
+    if (!SPLIT) __syncthreads();   // a wavefront's own LDS operations complete in order
+  }
+};
+
+// SPLIT: the wavefronts' 32 x D results (result-register order, already on a common scale) through `lds` ([WAVES][32][LD],
+// the streamed tiles' room), summed, times mul(row), to dst(row); `add`: onto what is there.
+template <int D, int WAVES, typename Dst, typename Mul>
+__device__ __forceinline__ void sum_wavefronts(float* lds, const f32x16 (&acc)[D / 32], int wave, int i, int g, int tid, int nrows, bool add,
+                                               Dst dst, Mul mul) {
+  constexpr int LD = D + 4;
+  __syncthreads();
+#pragma unroll
+  for (int db = 0; db < D / 32; db++)
+#pragma unroll
+    for (int a = 0; a < 4; a++)
+      *reinterpret_cast<f32x4*>(lds + (wave * 32 + i) * LD + 32 * db + 8 * a + 4 * g) =
+          f32x4{acc[db][4 * a], acc[db][4 * a + 1], acc[db][4 * a + 2], acc[db][4 * a + 3]};
+  __syncthreads();
+#pragma unroll
+  for (int c = 0; c < 8 * D / (64 * WAVES); c++) {
+    const int e = tid + c * 64 * WAVES, r = e / (D / 4), x = e % (D / 4);
+    if (r >= nrows) continue;
+    f32x4 v = *reinterpret_cast<const f32x4*>(lds + r * LD + 4 * x);
+#pragma unroll
+    for (int w = 1; w < WAVES; w++) v += *reinterpret_cast<const f32x4*>(lds + (w * 32 + r) * LD + 4 * x);
+    v *= mul(r);
+    f32x4* out = reinterpret_cast<f32x4*>(dst(r) + 4 * x);
+    if (add) v += *out;
+    *out = v;
+  }
+}
 
 // The resident operand of a head_dim contraction: row `row` of a (rows, D) matrix in
 // k-step order (element 4 j + t = column 8 j + 4 g + t), times `mul`.
@@ -145,17 +195,20 @@ __device__ __forceinline__ void store_rows(float* dst, const f32x16 (&acc)[D / 3
 // ---------------------------------------------------------------------------------------
 // DROP (all three kernels): attention dropout (AttnParams::drop_*, ody_dropout_hash): row sums and lse are those of the
 // full P; the entries that enter P V are the kept ones scaled by 1 / (1 - p), and dP counts only where an entry was kept.
-template <int D, bool DROP>
-__global__ __launch_bounds__(F_THREADS, D == 64 ? 3 : 1) void attn_fwd_f32_kernel(const AttnParams p) {
-  constexpr int LD = D + 4, NDB = D / 32;
-  __shared__ __attribute__((aligned(16))) float Ks[F_TILE * LD];
-  __shared__ __attribute__((aligned(16))) float Vs[F_TILE * LD];
+template <int D, bool DROP, bool SPLIT>
+__global__ __launch_bounds__((Shape<D, SPLIT>::THREADS), D == 64 ? (SPLIT ? 2 : 3) : 1) void attn_fwd_f32_kernel(const AttnParams p) {
+  using S = Shape<D, SPLIT>;
+  constexpr int LD = S::LD, NDB = D / 32;
+  extern __shared__ __attribute__((aligned(16))) float smem[];   // [TILES][K tile, V tile]
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, i = lane & 31, g = lane >> 5;
   const BlockCoord bc = ody_block_coord(p.Hq, p.B);
   const int nqb = gridDim.x / (p.Hq * p.B);
   const int qblk = p.causal ? (nqb - 1 - bc.rank) : bc.rank;  // heaviest blocks first
   const int h = bc.h, b = bc.b, hk = h / p.group;
-  const int q0 = qblk * F_ROWS, wq0 = q0 + wave * 32, qi = wq0 + i;
+  const int q0 = qblk * S::ROWS, wq0 = SPLIT ? q0 : q0 + wave * 32, qi = wq0 + i;
+  const int ltid = SPLIT ? lane : tid;
+  float* Ks = smem + (SPLIT ? wave : 0) * 2 * F_TILE * LD;
+  float* Vs = Ks + F_TILE * LD;
   const float* qp = static_cast<const float*>(p.q) + b * p.sq.b + h * p.sq.h;
   const float* kp = static_cast<const float*>(p.k) + b * p.sk.b + hk * p.sk.h;
   const float* vp = static_cast<const float*>(p.v) + b * p.sv.b + hk * p.sv.h;
@@ -174,23 +227,24 @@ __global__ __launch_bounds__(F_THREADS, D == 64 ? 3 : 1) void attn_fwd_f32_kerne
   // key ranges the workgroup and the wavefront have to walk
   const int lim = p.causal ? min(p.Lk - 1, qi + p.off) : p.Lk - 1;
   const int lim_first = p.causal ? min(p.Lk - 1, wq0 + p.off) : p.Lk - 1;
-  const int blk_hi = min(q0 + F_ROWS, p.Lq) - 1, wav_hi = min(wq0 + 32, p.Lq) - 1;
+  const int blk_hi = min(q0 + S::ROWS, p.Lq) - 1, wav_hi = min(wq0 + 32, p.Lq) - 1;
   const int n_end = max(0, p.causal ? min(p.Lk, blk_hi + p.off + 1) : p.Lk);
   const int w_end = (wq0 < p.Lq) ? max(0, p.causal ? min(p.Lk, wav_hi + p.off + 1) : p.Lk) : 0;
 
-  TileRegs<D> kr, vr;
-  if (n_end > 0) {
-    kr.fetch(kp, p.sk.l, 0, min(F_TILE, p.Lk), tid);
-    vr.fetch(vp, p.sv.l, 0, min(F_TILE, p.Lk), tid);
+  TileRegs<D, S::LOADERS> kr, vr;
+  const int n_first = SPLIT ? wave * F_TILE : 0;
+  if (n_first < n_end) {
+    kr.fetch(kp, p.sk.l, n_first, min(F_TILE, p.Lk - n_first), ltid);
+    vr.fetch(vp, p.sv.l, n_first, min(F_TILE, p.Lk - n_first), ltid);
   }
-  for (int n0 = 0; n0 < n_end; n0 += F_TILE) {
-    __syncthreads();
-    kr.put(Ks, tid);
-    vr.put(Vs, tid);
-    __syncthreads();
-    if (n0 + F_TILE < n_end) {
-      kr.fetch(kp, p.sk.l, n0 + F_TILE, min(F_TILE, p.Lk - n0 - F_TILE), tid);
-      vr.fetch(vp, p.sv.l, n0 + F_TILE, min(F_TILE, p.Lk - n0 - F_TILE), tid);
+  for (int n0 = n_first; n0 < n_end; n0 += S::STEP) {
+    S::sync();
+    kr.put(Ks, ltid);
+    vr.put(Vs, ltid);
+    S::sync();
+    if (n0 + S::STEP < n_end) {
+      kr.fetch(kp, p.sk.l, n0 + S::STEP, min(F_TILE, p.Lk - n0 - S::STEP), ltid);
+      vr.fetch(vp, p.sv.l, n0 + S::STEP, min(F_TILE, p.Lk - n0 - S::STEP), ltid);
     }
     if (n0 >= w_end) continue;  // wavefront-uniform: nothing visible to this wavefront here
 
@@ -226,6 +280,39 @@ __global__ __launch_bounds__(F_THREADS, D == 64 ? 3 : 1) void attn_fwd_f32_kerne
   }
 
   l = half_swap_sum(l);
+  if constexpr (SPLIT) {
+    __shared__ float sm[S::WAVES][32], sl[S::WAVES][32];
+    if (g == 0) sm[wave][i] = m, sl[wave][i] = l;
+    __syncthreads();
+    float top = sm[0][i];
+#pragma unroll
+    for (int w = 1; w < S::WAVES; w++) top = fmaxf(top, sm[w][i]);
+    const float mine = ody_exp2(m - (top == -INFINITY ? 0.f : top));
+#pragma unroll
+    for (int db = 0; db < NDB; db++) o[db] *= mine;
+    auto total = [&](int r, float& ref) {
+      float t = sm[0][r], sum = 0.f;
+#pragma unroll
+      for (int w = 1; w < S::WAVES; w++) t = fmaxf(t, sm[w][r]);
+      ref = t == -INFINITY ? 0.f : t;
+#pragma unroll
+      for (int w = 0; w < S::WAVES; w++) sum += sl[w][r] * ody_exp2(sm[w][r] - ref);
+      return sum;
+    };
+    float* ob = static_cast<float*>(p.out) + b * p.so.b + h * p.so.h;
+    sum_wavefronts<D, S::WAVES>(smem, o, wave, i, g, tid, min(32, p.Lq - q0), false, [&](int r) { return ob + (int64_t)(q0 + r) * p.so.l; },
+                      [&](int r) {
+                        float ref;
+                        const float sum = total(r, ref);
+                        return sum > 0.f ? (DROP ? p.drop_scale : 1.f) / sum : 0.f;
+                      });
+    if (wave == 0 && g == 0 && qi < p.Lq) {
+      float ref;
+      const float sum = total(i, ref);
+      p.lse[((int64_t)b * p.Hq + h) * p.Lq + qi] = sum > 0.f ? (ref + __log2f(sum)) * LN2 : -INFINITY;
+    }
+    return;
+  }
   if (qi < p.Lq) {
     float* op = static_cast<float*>(p.out) + b * p.so.b + h * p.so.h + (int64_t)qi * p.so.l;
     store_rows<D>(op, o, g, l > 0.f ? (DROP ? p.drop_scale : 1.f) / l : 0.f, false);
@@ -236,17 +323,20 @@ __global__ __launch_bounds__(F_THREADS, D == 64 ? 3 : 1) void attn_fwd_f32_kerne
 // ---------------------------------------------------------------------------------------
 // dQ: the wavefront owns 32 queries, keys are streamed
 // ---------------------------------------------------------------------------------------
-template <int D, bool DROP>
-__global__ __launch_bounds__(F_THREADS) void attn_bwd_dq_f32_kernel(const AttnParams p) {
-  constexpr int LD = D + 4, NDB = D / 32;
-  __shared__ __attribute__((aligned(16))) float Ks[F_TILE * LD];
-  __shared__ __attribute__((aligned(16))) float Vs[F_TILE * LD];
+template <int D, bool DROP, bool SPLIT>
+__global__ __launch_bounds__((Shape<D, SPLIT>::THREADS), D == 64 && SPLIT ? 2 : 1) void attn_bwd_dq_f32_kernel(const AttnParams p) {
+  using S = Shape<D, SPLIT>;
+  constexpr int LD = S::LD, NDB = D / 32;
+  extern __shared__ __attribute__((aligned(16))) float smem[];   // [TILES][K tile, V tile]
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, i = lane & 31, g = lane >> 5;
   const BlockCoord bc = ody_block_coord(p.Hq, p.B);
   const int nqb = gridDim.x / (p.Hq * p.B);
   const int qblk = p.causal ? (nqb - 1 - bc.rank) : bc.rank;
   const int h = bc.h, b = bc.b, hk = h / p.group;
-  const int q0 = qblk * F_ROWS, wq0 = q0 + wave * 32, qi = wq0 + i;
+  const int q0 = qblk * S::ROWS, wq0 = SPLIT ? q0 : q0 + wave * 32, qi = wq0 + i;
+  const int ltid = SPLIT ? lane : tid;
+  float* Ks = smem + (SPLIT ? wave : 0) * 2 * F_TILE * LD;
+  float* Vs = Ks + F_TILE * LD;
   const float* qp = static_cast<const float*>(p.q) + b * p.sq.b + h * p.sq.h;
   const float* dop = static_cast<const float*>(p.dout) + b * p.sdo.b + h * p.sdo.h;
   const float* kp = static_cast<const float*>(p.k) + b * p.sk.b + hk * p.sk.h;
@@ -268,23 +358,24 @@ __global__ __launch_bounds__(F_THREADS) void attn_bwd_dq_f32_kernel(const AttnPa
 #pragma unroll
     for (int r = 0; r < 16; r++) dq[db][r] = 0.f;
 
-  const int blk_hi = min(q0 + F_ROWS, p.Lq) - 1, wav_hi = min(wq0 + 32, p.Lq) - 1;
+  const int blk_hi = min(q0 + S::ROWS, p.Lq) - 1, wav_hi = min(wq0 + 32, p.Lq) - 1;
   const int n_end = max(0, p.causal ? min(p.Lk, blk_hi + p.off + 1) : p.Lk);
   const int w_end = (wq0 < p.Lq) ? max(0, p.causal ? min(p.Lk, wav_hi + p.off + 1) : p.Lk) : 0;
 
-  TileRegs<D> kr, vr;
-  if (n_end > 0) {
-    kr.fetch(kp, p.sk.l, 0, min(F_TILE, p.Lk), tid);
-    vr.fetch(vp, p.sv.l, 0, min(F_TILE, p.Lk), tid);
+  TileRegs<D, S::LOADERS> kr, vr;
+  const int n_first = SPLIT ? wave * F_TILE : 0;
+  if (n_first < n_end) {
+    kr.fetch(kp, p.sk.l, n_first, min(F_TILE, p.Lk - n_first), ltid);
+    vr.fetch(vp, p.sv.l, n_first, min(F_TILE, p.Lk - n_first), ltid);
   }
-  for (int n0 = 0; n0 < n_end; n0 += F_TILE) {
-    __syncthreads();
-    kr.put(Ks, tid);
-    vr.put(Vs, tid);
-    __syncthreads();
-    if (n0 + F_TILE < n_end) {
-      kr.fetch(kp, p.sk.l, n0 + F_TILE, min(F_TILE, p.Lk - n0 - F_TILE), tid);
-      vr.fetch(vp, p.sv.l, n0 + F_TILE, min(F_TILE, p.Lk - n0 - F_TILE), tid);
+  for (int n0 = n_first; n0 < n_end; n0 += S::STEP) {
+    S::sync();
+    kr.put(Ks, ltid);
+    vr.put(Vs, ltid);
+    S::sync();
+    if (n0 + S::STEP < n_end) {
+      kr.fetch(kp, p.sk.l, n0 + S::STEP, min(F_TILE, p.Lk - n0 - S::STEP), ltid);
+      vr.fetch(vp, p.sv.l, n0 + S::STEP, min(F_TILE, p.Lk - n0 - S::STEP), ltid);
     }
     if (n0 >= w_end) continue;
 
@@ -301,6 +392,12 @@ __global__ __launch_bounds__(F_THREADS) void attn_bwd_dq_f32_kernel(const AttnPa
     }
     tile_t_times_regs<D>(Ks, i, g, s, dq);  // dQ^T += K^T dS^T
   }
+  if constexpr (SPLIT) {
+    float* qb = static_cast<float*>(p.dq) + b * p.sdq.b + h * p.sdq.h;
+    sum_wavefronts<D, S::WAVES>(smem, dq, wave, i, g, tid, min(32, p.Lq - q0), p.accumulate_dq != 0,
+                      [&](int r) { return qb + (int64_t)(q0 + r) * p.sdq.l; }, [](int) { return 1.f; });
+    return;
+  }
   if (qi < p.Lq) {
     float* dqp = static_cast<float*>(p.dq) + b * p.sdq.b + h * p.sdq.h + (int64_t)qi * p.sdq.l;
     store_rows<D>(dqp, dq, g, 1.f, p.accumulate_dq != 0);
@@ -312,19 +409,23 @@ __global__ __launch_bounds__(F_THREADS) void attn_bwd_dq_f32_kernel(const AttnPa
 // WHICH: 0 = dV only, 1 = dK only, 2 = both.  (At head_dim 128 the K and V fragments and both
 // accumulators do not fit the register file together, so dV and dK take a pass each.)
 // ---------------------------------------------------------------------------------------
-template <int D, int WHICH, bool DROP>
-__global__ __launch_bounds__(F_THREADS, (D == 64 || WHICH == 0) ? 2 : 1) void attn_bwd_dkdv_f32_kernel(const AttnParams p) {
-  constexpr int LD = D + 4, NDB = D / 32;
+template <int D, int WHICH, bool DROP, bool SPLIT>
+__global__ __launch_bounds__((Shape<D, SPLIT>::THREADS), (D == 64 || (WHICH == 0 && !SPLIT)) ? 2 : 1) void attn_bwd_dkdv_f32_kernel(const AttnParams p) {
+  using S = Shape<D, SPLIT>;
+  constexpr int LD = S::LD, NDB = D / 32;
   constexpr bool DO_DV = (WHICH != 1), DO_DK = (WHICH != 0);
-  __shared__ __attribute__((aligned(16))) float Qs[F_TILE * LD];
-  __shared__ __attribute__((aligned(16))) float Os[F_TILE * LD];
-  __shared__ __attribute__((aligned(16))) float Ls[F_TILE];  // lse in the log2 domain; +inf = row contributes nothing
-  __shared__ __attribute__((aligned(16))) float Ds[F_TILE];
+  extern __shared__ __attribute__((aligned(16))) float smem[];   // [TILES][Q tile, dO tile]
+  __shared__ __attribute__((aligned(16))) float stats[S::TILES][2][F_TILE];  // lse in the log2 domain (+inf = row contributes nothing), delta
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, i = lane & 31, g = lane >> 5;
   const BlockCoord bc = ody_block_coord(p.Hkv, p.B);
   const int kblk = bc.rank;  // with causal masking the first key block is the heaviest
   const int hk = bc.h, b = bc.b;
-  const int n0 = kblk * F_ROWS, wn0 = n0 + wave * 32, ki = wn0 + i;
+  const int n0 = kblk * S::ROWS, wn0 = SPLIT ? n0 : n0 + wave * 32, ki = wn0 + i;
+  const int ltid = SPLIT ? lane : tid;
+  float* Qs = smem + (SPLIT ? wave : 0) * 2 * F_TILE * LD;
+  float* Os = Qs + F_TILE * LD;
+  float* Ls = stats[SPLIT ? wave : 0][0];
+  float* Ds = stats[SPLIT ? wave : 0][1];
   const float* kp = static_cast<const float*>(p.k) + b * p.sk.b + hk * p.sk.h;
   const float* vp = static_cast<const float*>(p.v) + b * p.sv.b + hk * p.sv.h;
 
@@ -345,35 +446,36 @@ __global__ __launch_bounds__(F_THREADS, (D == 64 || WHICH == 0) ? 2 : 1) void at
   const int i_begin = p.causal ? (max(0, n0 - p.off) / F_TILE) * F_TILE : 0;
   const int w_begin = p.causal ? max(0, wn0 - p.off) : 0;
 
-  TileRegs<D> qr, dor;
-  float lr = 0.f, dr = 0.f;  // threads 0..31 carry lse and delta of the next tile
-  for (int hg = 0; hg < p.group; hg++) {
-    const int h = hk * p.group + hg;
-    const float* qp = static_cast<const float*>(p.q) + b * p.sq.b + h * p.sq.h;
-    const float* dop = static_cast<const float*>(p.dout) + b * p.sdo.b + h * p.sdo.h;
-    const int64_t rbase = ((int64_t)b * p.Hq + h) * p.Lq;
-    const unsigned dh = DROP ? ody_dropout_head(p.drop_seed, b * p.Hq + h) : 0u;
-    auto fetch = [&](int i0) {
-      const int valid = min(F_TILE, p.Lq - i0);
-      qr.fetch(qp, p.sq.l, i0, valid, tid);
-      dor.fetch(dop, p.sdo.l, i0, valid, tid);
-      if (tid < F_TILE) {
-        const float x = (tid < valid) ? p.lse[rbase + i0 + tid] : -INFINITY;
-        lr = (x == -INFINITY) ? INFINITY : x * ODY_LOG2E;
-        dr = (tid < valid) ? p.delta[rbase + i0 + tid] : 0.f;
+  // turns over the query tiles of every head of the group
+  const int ntq = p.Lq > i_begin ? (p.Lq - i_begin + F_TILE - 1) / F_TILE : 0, turns = ntq * p.group;
+  TileRegs<D, S::LOADERS> qr, dor;
+  float lr = 0.f, dr = 0.f;  // the first 32 loaders carry lse and delta of the next tile
+  auto fetch = [&](int it) {
+    const int h = hk * p.group + it / ntq, i0 = i_begin + (it % ntq) * F_TILE, valid = min(F_TILE, p.Lq - i0);
+    qr.fetch(static_cast<const float*>(p.q) + b * p.sq.b + h * p.sq.h, p.sq.l, i0, valid, ltid);
+    dor.fetch(static_cast<const float*>(p.dout) + b * p.sdo.b + h * p.sdo.h, p.sdo.l, i0, valid, ltid);
+    if (ltid < F_TILE) {
+      const int64_t rbase = ((int64_t)b * p.Hq + h) * p.Lq;
+      const float x = (ltid < valid) ? p.lse[rbase + i0 + ltid] : -INFINITY;
+      lr = (x == -INFINITY) ? INFINITY : x * ODY_LOG2E;
+      dr = (ltid < valid) ? p.delta[rbase + i0 + ltid] : 0.f;
+    }
+  };
+  const int it_first = SPLIT ? wave : 0, it_step = S::STEP / F_TILE;
+  if (it_first < turns) fetch(it_first);
+  {
+    for (int it = it_first; it < turns; it += it_step) {
+      const int h = hk * p.group + it / ntq, i0 = i_begin + (it % ntq) * F_TILE;
+      const unsigned dh = DROP ? ody_dropout_head(p.drop_seed, b * p.Hq + h) : 0u;
+      S::sync();
+      qr.put(Qs, ltid);
+      dor.put(Os, ltid);
+      if (ltid < F_TILE) {
+        Ls[ltid] = lr;
+        Ds[ltid] = dr;
       }
-    };
-    if (i_begin < p.Lq) fetch(i_begin);
-    for (int i0 = i_begin; i0 < p.Lq; i0 += F_TILE) {
-      __syncthreads();
-      qr.put(Qs, tid);
-      dor.put(Os, tid);
-      if (tid < F_TILE) {
-        Ls[tid] = lr;
-        Ds[tid] = dr;
-      }
-      __syncthreads();
-      if (i0 + F_TILE < p.Lq) fetch(i0 + F_TILE);
+      S::sync();
+      if (it + it_step < turns) fetch(it + it_step);
       if (i0 + F_TILE <= w_begin || wn0 >= p.Lk) continue;  // wavefront-uniform
 
       // S = Q K^T (log2 domain): rows = queries, column = this lane's key; dP = dO V^T
@@ -407,6 +509,19 @@ __global__ __launch_bounds__(F_THREADS, (D == 64 || WHICH == 0) ? 2 : 1) void at
       if constexpr (DO_DV) tile_t_times_regs<D>(Os, i, g, s, dv);   // dV^T += dO^T P
       if constexpr (DO_DK) tile_t_times_regs<D>(Qs, i, g, dp, dk);  // dK^T += Q^T dS
     }
+  }
+  if constexpr (SPLIT) {
+    if constexpr (DO_DK) {
+      float* base = static_cast<float*>(p.dk) + b * p.sdk.b + hk * p.sdk.h;
+      sum_wavefronts<D, S::WAVES>(smem, dk, wave, i, g, tid, min(32, p.Lk - n0), false, [&](int r) { return base + (int64_t)(n0 + r) * p.sdk.l; },
+                        [](int) { return 1.f; });
+    }
+    if constexpr (DO_DV) {
+      float* base = static_cast<float*>(p.dv) + b * p.sdv.b + hk * p.sdv.h;
+      sum_wavefronts<D, S::WAVES>(smem, dv, wave, i, g, tid, min(32, p.Lk - n0), false, [&](int r) { return base + (int64_t)(n0 + r) * p.sdv.l; },
+                        [](int) { return 1.f; });
+    }
+    return;
   }
   if (ki < p.Lk) {
     if constexpr (DO_DK) {
@@ -446,29 +561,44 @@ __global__ __launch_bounds__(256) void attn_delta_kernel(const AttnParams p) {
   if (row < total && sub == 0) p.delta[row] = acc;
 }
 
+// Whether `rows` per (head, batch) leave 128-row workgroups too few (two per compute unit even out a causal mask); beyond that
+// the shared tiles of the wider workgroup save memory traffic.
+bool few_rows(int rows, int heads) { return (int64_t)((rows + F_ROWS - 1) / F_ROWS) * heads < 1024; }
+
+template <int D, bool SPLIT, typename K>
+int launch_one(const char* name, K kern, int rows, int heads, const AttnParams& p, hipStream_t st) {
+  using S = Shape<D, SPLIT>;
+  constexpr size_t smem = sizeof(float) * S::TILES * 2 * F_TILE * S::LD;
+  if (int rc = ody_allow_dynamic_lds(reinterpret_cast<const void*>(kern), smem, name)) return rc;
+  ODY_LAUNCH(name, st, kern, dim3((unsigned)(((int64_t)rows + S::ROWS - 1) / S::ROWS * heads)), dim3(S::THREADS), smem, p);
+  return ody_check_launch(name);
+}
+
 template <int D, bool DROP>
 int launch_fwd(const AttnParams& p, hipStream_t st) {
-  const int nqb = (p.Lq + F_ROWS - 1) / F_ROWS;
-  ODY_LAUNCH("attn_fwd_f32", st, (attn_fwd_f32_kernel<D, DROP>), dim3(nqb * p.Hq * p.B), dim3(F_THREADS), 0, p);
-  return ody_check_launch("attn_fwd_f32");
+  const int heads = p.Hq * p.B;
+  if (few_rows(p.Lq, heads)) return launch_one<D, true>("attn_fwd_f32", &attn_fwd_f32_kernel<D, DROP, true>, p.Lq, heads, p, st);
+  return launch_one<D, false>("attn_fwd_f32", &attn_fwd_f32_kernel<D, DROP, false>, p.Lq, heads, p, st);
+}
+
+template <int D, bool DROP, bool SPLIT>
+int launch_dkdv(const AttnParams& p, hipStream_t st) {
+  const int heads = p.Hkv * p.B;
+  if constexpr (D == 64) {
+    return launch_one<D, SPLIT>("attn_bwd_dkdv_f32", &attn_bwd_dkdv_f32_kernel<D, 2, DROP, SPLIT>, p.Lk, heads, p, st);
+  } else {
+    if (int rc = launch_one<D, SPLIT>("attn_bwd_dv_f32", &attn_bwd_dkdv_f32_kernel<D, 0, DROP, SPLIT>, p.Lk, heads, p, st)) return rc;
+    return launch_one<D, SPLIT>("attn_bwd_dk_f32", &attn_bwd_dkdv_f32_kernel<D, 1, DROP, SPLIT>, p.Lk, heads, p, st);
+  }
 }
 
 template <int D, bool DROP>
 int launch_bwd(const AttnParams& p, hipStream_t st) {
-  const int nqb = (p.Lq + F_ROWS - 1) / F_ROWS, nkb = (p.Lk + F_ROWS - 1) / F_ROWS;
-  const dim3 gk(nkb * p.Hkv * p.B), blk(F_THREADS);
-  int rc;
-  if constexpr (D == 64) {
-    ODY_LAUNCH("attn_bwd_dkdv_f32", st, (attn_bwd_dkdv_f32_kernel<D, 2, DROP>), gk, blk, 0, p);
-    if ((rc = ody_check_launch("attn_bwd_dkdv_f32"))) return rc;
-  } else {
-    ODY_LAUNCH("attn_bwd_dv_f32", st, (attn_bwd_dkdv_f32_kernel<D, 0, DROP>), gk, blk, 0, p);
-    if ((rc = ody_check_launch("attn_bwd_dv_f32"))) return rc;
-    ODY_LAUNCH("attn_bwd_dk_f32", st, (attn_bwd_dkdv_f32_kernel<D, 1, DROP>), gk, blk, 0, p);
-    if ((rc = ody_check_launch("attn_bwd_dk_f32"))) return rc;
-  }
-  ODY_LAUNCH("attn_bwd_dq_f32", st, (attn_bwd_dq_f32_kernel<D, DROP>), dim3(nqb * p.Hq * p.B), blk, 0, p);
-  return ody_check_launch("attn_bwd_dq_f32");
+  const int rc = few_rows(p.Lk, p.Hkv * p.B) ? launch_dkdv<D, DROP, true>(p, st) : launch_dkdv<D, DROP, false>(p, st);
+  if (rc) return rc;
+  const int heads = p.Hq * p.B;
+  if (few_rows(p.Lq, heads)) return launch_one<D, true>("attn_bwd_dq_f32", &attn_bwd_dq_f32_kernel<D, DROP, true>, p.Lq, heads, p, st);
+  return launch_one<D, false>("attn_bwd_dq_f32", &attn_bwd_dq_f32_kernel<D, DROP, false>, p.Lq, heads, p, st);
 }
 
 template <typename T, int D>

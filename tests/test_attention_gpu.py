@@ -543,3 +543,24 @@ def test_attention_fwd_few_queries(case, D, dev):
     torch.cuda.synchronize()
     assert_parity(o, o_ref, TOL_BF16, "o")
     assert torch.allclose(lse.cpu(), lse_ref, atol=TOL_LSE, rtol=TOL_LSE)
+
+
+@pytest.mark.parametrize("D,heads", [(64, 2), (64, 1100), (128, 1), (128, 1100)])
+@pytest.mark.parametrize("case", [(1, 1, True), (31, 33, True), (257, 257, True), (300, 40, True), (70, 600, False)],
+                         ids=lambda c: "Lq%d_Lk%d_c%d" % c)
+def test_attention_fp32_few_and_many_rows(case, D, heads, dev):
+    """fp32 attention with the wavefronts of a workgroup on the same 32 rows (few heads) and on 128 (many), group size 2."""
+    from odysseus_transformer_amd import ops
+    Lq, Lk, causal = case
+    print(f"fp32 rows case={case} D={D} heads={heads}", flush=True)
+    q, k, v, do = _inputs(1, Lq, Lk, heads, max(1, heads // 2), D, torch.float32, seed=61)
+    o_ref, lse_ref = oracle.attention_fwd(q, k, v, causal=causal)
+    dq_ref, dk_ref, dv_ref = oracle.attention_bwd(q, k, v, o_ref, lse_ref, do, causal=causal)
+    qg, kg, vg, dog = (t.to(dev) for t in (q, k, v, do))
+    o, lse = ops.attn_fwd(qg, kg, vg, causal=causal)
+    dq, dk, dv = ops.attn_bwd(qg, kg, vg, o, lse, dog, causal=causal)
+    torch.cuda.synchronize()
+    floor = 1.0 if Lk == 1 else 1e-3
+    for got, ref, what in ((o, o_ref, "o"), (dq, dq_ref, "dq"), (dk, dk_ref, "dk"), (dv, dv_ref, "dv")):
+        assert_parity(got, ref, TOL_F32, what, floor)
+    assert torch.allclose(lse.cpu(), lse_ref, atol=TOL_LSE, rtol=TOL_LSE)
