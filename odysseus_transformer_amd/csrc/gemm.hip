@@ -374,12 +374,12 @@ struct F32Tile {
 // of 32 x 32 (a 64 x 64 or 128 x 128 workgroup tile).  One LDS slab; the next one is fetched into
 // registers while the current one is multiplied.  The product is computed as C^T = op(B)^T op(A)^T,
 // so a lane holds 4 consecutive N per register quad and writes 16-byte pieces of C rows.
-// VEC = false (unaligned pointers or extents that are not multiples of 4) moves single floats.
+// gridDim.y > 1: block y takes the y-th range of slabs and writes fp32 partial results to part[y][M][N] (VEC only).
+// VEC = false (unaligned pointers, or a contiguous extent that is no multiple of 4) moves single floats.
 template <int WT, bool A_KC, bool B_KC, bool VEC>
-__global__ __launch_bounds__(256) void gemm_f32_kernel(const float* __restrict__ A, const float* __restrict__ B,
-                                                       float* __restrict__ C, const float* __restrict__ bias, int M,
-                                                       int N, int K, int64_t lda, int64_t ldb, int64_t ldc,
-                                                       int accumulate, int ntn) {
+__global__ __launch_bounds__(256) void gemm_f32_kernel(const float* __restrict__ A, const float* __restrict__ B, float* C,
+                                                            const float* __restrict__ bias, int M, int N, int K, int64_t lda,
+                                                            int64_t ldb, int64_t ldc, int accumulate, int ntn, float* part) {
   constexpr int BT = 64 * WT;
   constexpr int NCH = (WT == 1) ? 2 : 1;  // never a single chain of dependent MFMAs
   using TA = F32Tile<BT, A_KC>;
@@ -402,14 +402,19 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(const float* __restrict__
 
   TA ta;
   TB tb;
-  ta.template gload<VEC>(A, lda, m0, 0, M, K, tid);
-  tb.template gload<VEC>(B, ldb, n0, 0, N, K, tid);
-  for (int k0 = 0; k0 < K; k0 += FK) {
+  int k_first = 0, k_last = K;
+  if (VEC && part) {
+    const int per = ((K + FK - 1) / FK + (int)gridDim.y - 1) / (int)gridDim.y * FK;
+    k_first = min((int)blockIdx.y * per, K), k_last = min(k_first + per, K);
+  }
+  ta.template gload<VEC>(A, lda, m0, k_first, M, K, tid);
+  tb.template gload<VEC>(B, ldb, n0, k_first, N, K, tid);
+  for (int k0 = k_first; k0 < k_last; k0 += FK) {
     __syncthreads();
     ta.put(As, tid);
     tb.put(Bs, tid);
     __syncthreads();
-    if (k0 + FK < K) {
+    if (k0 + FK < k_last) {
       ta.template gload<VEC>(A, lda, m0, k0 + FK, M, K, tid);
       tb.template gload<VEC>(B, ldb, n0, k0 + FK, N, K, tid);
     }
@@ -429,7 +434,6 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(const float* __restrict__
             acc[a][b][t % NCH] = mfma_f32(bf[b][t], af[a][t], acc[a][b][t % NCH]);
     }
   }
-
   // register r of lane (i, g) of tile (a, b): row m = 32 (wm WT + a) + i, column n = 32 (wn WT + b) + 8 (r / 4) + 4 g + r % 4
 #pragma unroll
   for (int a = 0; a < WT; a++) {
@@ -442,6 +446,11 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(const float* __restrict__
 #pragma unroll
       for (int q = 0; q < 4; q++) {
         const int n = n0 + 32 * (wn * WT + b) + 8 * q + 4 * g;
+        if (VEC && part) {
+          if (n < N)
+            *reinterpret_cast<f32x4*>(part + ((int64_t)blockIdx.y * M + m) * N + n) = f32x4{v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]};
+          continue;
+        }
         float* dst = C + (int64_t)m * ldc + n;
         if (VEC && n + 3 < N) {
           f32x4 o{v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]};
@@ -463,44 +472,91 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(const float* __restrict__
   }
 }
 
+// C (+)= sum of the fp32 partial results (+ bias); 4 elements per thread
+__global__ __launch_bounds__(256) void gemm_f32_sum_kernel(const float* __restrict__ part, int splits, float* C,
+                                                           const float* __restrict__ bias, int M, int N, int64_t ldc, int accumulate) {
+  const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (idx >= (int64_t)M * (N / 4)) return;
+  const int m = idx / (N / 4), n = (idx % (N / 4)) * 4;
+  f32x4 v = sum_parts(part, splits, (int64_t)M * N, (int64_t)m * N + n);
+  if (bias) v += *reinterpret_cast<const f32x4*>(bias + n);
+  f32x4* dst = reinterpret_cast<f32x4*>(C + (int64_t)m * ldc + n);
+  if (accumulate) v += *dst;
+  *dst = v;
+}
+
+// Tile and ranges of K of an fp32 product: 128 x 128 tiles once they fill the chip twice over, 64 x 64 tiles below that.  A lone
+// block of 4 wavefronts on a compute unit waits at its barriers half of the time (0.87 us per slab of 32 k), several blocks fill
+// each other's gaps (0.56 us per block and slab), so a long K is cut into ranges until the blocks outnumber the units a few times
+// -- as far as the trip of the partial results through memory pays for it.  (Weight gradients over 2048 tokens, us without / with
+// ranges: 2752 x 512 85 / 76, 1536 x 512 54 / 45, 512 x 512 51 / 20.  Sharing a tile's slabs between four times the wavefronts
+// of one block, or K over eight independent ones, took as long as the ranges.)
+struct PlanF32 { int tile, splits; };
+PlanF32 plan_f32(int M, int N, int K) {
+  const int64_t big = (int64_t)((M + 127) / 128) * ((N + 127) / 128), small = (int64_t)((M + 63) / 64) * ((N + 63) / 64);
+  if (big >= 512) return PlanF32{128, 1};
+  const int slabs = (K + FK - 1) / FK;
+  PlanF32 best{64, 1};
+  double best_us = 1e30;
+  for (int s = 1; s <= 16 && slabs >= 4 * s; s++) {
+    const double per_cu = (double)((small * s + 255) / 256);
+    double us = (slabs + s - 1) / s * std::max(0.87, 0.56 * per_cu);
+    if (s > 1) us += 3.0 + (double)s * M * N * 8.0 / 5.0e6;
+    if (us < best_us) best_us = us, best.splits = s;
+  }
+  return best;
+}
+
 template <int WT, bool A_KC, bool B_KC>
 int launch_f32(const float* a, const float* b, float* c, const float* bias, int M, int N, int K, int64_t lda,
-               int64_t ldb, int64_t ldc, int accumulate, bool vec, hipStream_t st) {
+               int64_t ldb, int64_t ldc, int accumulate, bool vec, int splits, float* part, hipStream_t st) {
   constexpr int BT = 64 * WT;
   const int64_t ntm = (M + BT - 1) / BT, ntn = (N + BT - 1) / BT;
   ODY_REQUIRE(ntm * ntn < ((int64_t)1 << 31), ODY_ERR_BAD_SHAPE, "ody_gemm: M=%d N=%d too large for one launch", M, N);
-  const dim3 grid((unsigned)(ntm * ntn)), blk(256);
+  const dim3 grid((unsigned)(ntm * ntn), splits), blk(256);
   if (vec)
     ODY_LAUNCH("gemm_f32", st, (gemm_f32_kernel<WT, A_KC, B_KC, true>), grid, blk, 0, a, b, c, bias, M, N, K, lda,
-               ldb, ldc, accumulate, (int)ntn);
+               ldb, ldc, accumulate, (int)ntn, part);
   else
     ODY_LAUNCH("gemm_f32", st, (gemm_f32_kernel<WT, A_KC, B_KC, false>), grid, blk, 0, a, b, c, bias, M, N, K, lda,
-               ldb, ldc, accumulate, (int)ntn);
-  return ody_check_launch("gemm_f32");
+               ldb, ldc, accumulate, (int)ntn, part);
+  int rc = ody_check_launch("gemm_f32");
+  if (rc || splits == 1) return rc;
+  const int64_t n4 = (int64_t)M * (N / 4);
+  ODY_LAUNCH("gemm_f32_sum", st, gemm_f32_sum_kernel, dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, part, splits, c, bias, M, N, ldc,
+             accumulate);
+  return ody_check_launch("gemm_f32_sum");
 }
 
 template <bool A_KC, bool B_KC>
 int dispatch_f32(const float* a, const float* b, float* c, const float* bias, int M, int N, int K, int64_t lda,
-                 int64_t ldb, int64_t ldc, int accumulate, hipStream_t st) {
+                 int64_t ldb, int64_t ldc, int accumulate, void* workspace, size_t workspace_bytes, hipStream_t st) {
   const bool vec = ody_aligned16(a) && ody_aligned16(b) && ody_aligned16(c) && (!bias || ody_aligned16(bias)) &&
-                   lda % 4 == 0 && ldb % 4 == 0 && ldc % 4 == 0 && M % 4 == 0 && N % 4 == 0 && K % 4 == 0;
-  // 128 x 128 tiles once they fill the chip twice over, 64 x 64 tiles below that
-  const int64_t big = (int64_t)((M + 127) / 128) * ((N + 127) / 128);
-  if (big >= 512) return launch_f32<2, A_KC, B_KC>(a, b, c, bias, M, N, K, lda, ldb, ldc, accumulate, vec, st);
-  return launch_f32<1, A_KC, B_KC>(a, b, c, bias, M, N, K, lda, ldb, ldc, accumulate, vec, st);
+                   lda % 4 == 0 && ldb % 4 == 0 && ldc % 4 == 0 && N % 4 == 0 && (A_KC ? K : M) % 4 == 0 && (!B_KC || K % 4 == 0);
+  PlanF32 pl = plan_f32(M, N, K);
+  if (pl.splits > 1 && (!vec || !workspace || !ody_aligned16(workspace) || workspace_bytes < (size_t)pl.splits * M * N * sizeof(float)))
+    pl.splits = 1;
+  float* part = pl.splits > 1 ? static_cast<float*>(workspace) : nullptr;
+  if (pl.tile == 128) return launch_f32<2, A_KC, B_KC>(a, b, c, bias, M, N, K, lda, ldb, ldc, accumulate, vec, 1, nullptr, st);
+  return launch_f32<1, A_KC, B_KC>(a, b, c, bias, M, N, K, lda, ldb, ldc, accumulate, vec, pl.splits, part, st);
 }
 
-int gemm_f32(int op, const float* a, const float* b, float* c, const float* bias, int M, int N, int K, int64_t lda,
-             int64_t ldb, int64_t ldc, int accumulate, hipStream_t st) {
-  if (op == ODY_GEMM_NT) return dispatch_f32<true, true>(a, b, c, bias, M, N, K, lda, ldb, ldc, accumulate, st);
-  if (op == ODY_GEMM_NN) return dispatch_f32<true, false>(a, b, c, bias, M, N, K, lda, ldb, ldc, accumulate, st);
-  return dispatch_f32<false, false>(a, b, c, bias, M, N, K, lda, ldb, ldc, accumulate, st);
+int gemm_f32(int op, const float* a, const float* b, float* c, const float* bias, int M, int N, int K, int64_t lda, int64_t ldb,
+             int64_t ldc, int accumulate, void* workspace, size_t workspace_bytes, hipStream_t st) {
+  if (op == ODY_GEMM_NT) return dispatch_f32<true, true>(a, b, c, bias, M, N, K, lda, ldb, ldc, accumulate, workspace, workspace_bytes, st);
+  if (op == ODY_GEMM_NN) return dispatch_f32<true, false>(a, b, c, bias, M, N, K, lda, ldb, ldc, accumulate, workspace, workspace_bytes, st);
+  return dispatch_f32<false, false>(a, b, c, bias, M, N, K, lda, ldb, ldc, accumulate, workspace, workspace_bytes, st);
 }
 
 }  // namespace
 
 extern "C" size_t ody_gemm_workspace_bytes(int op, int M, int N, int K, int dtype) {
-  if (dtype != ODY_BF16 || M <= 0 || N <= 0 || K <= 0) return 0;
+  if (M <= 0 || N <= 0 || K <= 0) return 0;
+  if (dtype == ODY_F32) {
+    const int splits = plan_f32(M, N, K).splits;
+    return splits > 1 ? (size_t)splits * M * N * sizeof(float) : 0;
+  }
+  if (dtype != ODY_BF16) return 0;
   if (op == ODY_GEMM_NT && ody_gemm_skinny_ok(EPI_NONE, M, N)) return 0;
   const int splits = plan_bf16(M, N, K, true).splits;
   return splits > 1 ? (size_t)splits * M * N * sizeof(float) : 0;
@@ -519,7 +575,7 @@ extern "C" int ody_gemm(int op, const void* A, const void* B, void* C, const voi
   hipStream_t st = static_cast<hipStream_t>(stream);
   if (dtype == ODY_F32)
     return gemm_f32(op, (const float*)A, (const float*)B, (float*)C, (const float*)bias, M, N, K, lda, ldb, ldc,
-                    accumulate, st);
+                    accumulate, workspace, workspace_bytes, st);
   ODY_REQUIRE(dtype == ODY_BF16, ODY_ERR_UNSUPPORTED, "ody_gemm: dtype %d unknown", dtype);
   // 16-byte vectors along the contiguous direction of every matrix
   ODY_REQUIRE(ody_aligned16(A) && ody_aligned16(B) && ((reinterpret_cast<uintptr_t>(C) & 7u) == 0) &&
@@ -619,7 +675,7 @@ extern "C" int ody_linear_residual_ws(const void* x, const void* w, const void* 
                                     hipMemcpyDeviceToDevice, st);
     ODY_REQUIRE(e == hipSuccess, ODY_ERR_LAUNCH, "ody_linear_residual: copy of the residual failed: %s", hipGetErrorString(e));
   }
-  return ody_gemm(ODY_GEMM_NT, x, w, y, nullptr, M, N, K, ldx, ldw, ldy, 1, dtype, nullptr, 0, stream);
+  return ody_gemm(ODY_GEMM_NT, x, w, y, nullptr, M, N, K, ldx, ldw, ldy, 1, dtype, workspace, workspace_bytes, stream);
 }
 
 extern "C" int ody_linear_residual(const void* x, const void* w, const void* residual, void* y, int M, int N, int K,

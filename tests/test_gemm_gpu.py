@@ -190,3 +190,17 @@ def test_row_pitch_beyond_the_tile_kernels_offsets(dev):
     a.copy_(randn((M, K), 44, dtype=torch.bfloat16))
     w = randn((N, K), 45, std=0.05, dtype=torch.bfloat16).to(dev)
     assert rel_err(ops.gemm(ops.GEMM_NT, a, w), a.float() @ w.float().t()) <= TOL_BF16
+
+
+@pytest.mark.parametrize("op", ["nt", "nn", "tn"])
+@pytest.mark.parametrize("M,N,K", [(64, 64, 4096), (68, 132, 1028), (129, 64, 640), (1111, 132, 516), (132, 1028, 2049)], ids=lambda v: str(v))
+def test_fp32_ranges_of_k(op, M, N, K, dev):
+    """fp32 products whose K is cut into ranges, ragged rows beside vector loads, and extents that vector loads cannot take."""
+    from odysseus_transformer_amd import ops
+    a = randn((K, M) if op == "tn" else (M, K), 46).to(dev)
+    b = randn((N, K) if op == "nt" else (K, N), 47).to(dev)
+    code = {"nt": ops.GEMM_NT, "nn": ops.GEMM_NN, "tn": ops.GEMM_TN}[op]
+    ref = ((a.double().t() if op == "tn" else a.double()) @ (b.double().t() if op == "nt" else b.double()))
+    bias, out = randn((N,), 48).to(dev), torch.ones((M, N), device=dev)
+    assert rel_err(ops.gemm(code, a, b), ref) <= 1e-5
+    assert rel_err(ops.gemm(code, a, b, bias=bias, out=out, accumulate=True), ref + bias.double() + 1.0) <= 1e-5
