@@ -667,6 +667,13 @@ def rope_(x, n_rot: int, position_ids=None, base: float = 10000.0, inverse: bool
 
 
 # --------------------------------------------------------------------------- autograd
+def _dense_dout(dout, out):
+    """The gradient that arrived for `out`, with a head dimension the kernels can read; zero if none did."""
+    if dout is None:
+        return torch.zeros_like(out)
+    return dout if dout.stride(3) == 1 else dout.contiguous()
+
+
 class FlashAttnFunc(torch.autograd.Function):
     """Causal/full attention with GQA over (B, L, H, D) tensors; returns (out, lse)."""
 
@@ -676,13 +683,13 @@ class FlashAttnFunc(torch.autograd.Function):
         ctx.save_for_backward(q, k, v, out, lse)
         ctx.softmax_scale, ctx.causal, ctx.dropout = softmax_scale, causal, (dropout_p, seed)
         ctx.mark_non_differentiable(lse)
+        ctx.set_materialize_grads(False)   # no zero tensor for the gradient of lse: a fill kernel and 10 us of host on every backward
         return out, lse
 
     @staticmethod
     def backward(ctx, dout, _dlse):
         q, k, v, out, lse = ctx.saved_tensors
-        if dout.stride(3) != 1:
-            dout = dout.contiguous()
+        dout = _dense_dout(dout, out)
         dq, dk, dv = attn_bwd(q, k, v, out, lse, dout, causal=ctx.causal, scale=ctx.softmax_scale,
                               dropout_p=ctx.dropout[0], seed=ctx.dropout[1])
         return dq, dk, dv, None, None, None, None
@@ -711,6 +718,7 @@ class RingBlocksAttnFunc(torch.autograd.Function):
         ctx.save_for_backward(q, out, lse, *kv)
         ctx.causal_block, ctx.softmax_scale = causal_block, softmax_scale
         ctx.mark_non_differentiable(lse)
+        ctx.set_materialize_grads(False)
         return out, lse
 
     @staticmethod
@@ -718,8 +726,7 @@ class RingBlocksAttnFunc(torch.autograd.Function):
         q, out, lse, *kv = ctx.saved_tensors
         nb = len(kv) // 2
         ks, vs = kv[:nb], kv[nb:]
-        if dout.stride(3) != 1:
-            dout = dout.contiguous()
+        dout = _dense_dout(dout, out)
         # the running dq stays in fp32 over the blocks and is rounded once; delta, the start values and the
         # Q / dO images depend on the queries only and are built by the first block's call
         dq = torch.empty(q.shape, dtype=torch.float32, device=q.device)
@@ -791,6 +798,7 @@ class ZigzagRingRankAttnFunc(torch.autograd.Function):
         ctx.save_for_backward(q, out, lse_full, *kv)
         ctx.rank, ctx.world, ctx.softmax_scale = rank, world, softmax_scale
         ctx.mark_non_differentiable(lse_full)
+        ctx.set_materialize_grads(False)
         return out, lse_full
 
     @staticmethod
@@ -799,19 +807,21 @@ class ZigzagRingRankAttnFunc(torch.autograd.Function):
         world = ctx.world
         ks, vs = kv[:world], kv[world:]
         c = q.shape[1] // 2
-        if dout.stride(3) != 1:
-            dout = dout.contiguous()
+        dout = _dense_dout(dout, out)
         dq = torch.empty(q.shape, dtype=torch.float32, device=q.device)
         lse_b = lse[:, :, c:].contiguous()
         steps = list(ZigzagRingRankAttnFunc._steps(ctx.rank, world))
         # sized for the largest step (both query chunks against both key chunks); a step with fewer queries asks for less
         ws, _ = _shared_bwd_workspace(q, [(ks[0], False)])
-        dks = [torch.zeros_like(k) for k in ks]
-        dvs = [torch.zeros_like(v) for v in vs]
+        dks = [torch.empty_like(k) for k in ks]
+        dvs = [torch.empty_like(v) for v in vs]
         prev = None
         for s, ((q0, q1), (k0, k1), causal) in enumerate(steps):
             qs, kr = slice(q0 * c, q1 * c), slice(k0 * c, k1 * c)
             kind = (q0, q1, k0, k1)
+            if k1 == 1:   # the chunk that this step does not read; everything else is written below
+                dks[s][:, c:].zero_()
+                dvs[s][:, c:].zero_()
             need = attn_bwd_workspace_bytes(q[:, qs], ks[s][:, kr], True, causal)
             attn_bwd(q[:, qs], ks[s][:, kr], vs[s][:, kr], out[:, qs], lse if q1 - q0 == 2 else lse_b, dout[:, qs],
                      causal=causal, scale=ctx.softmax_scale, dq=dq[:, qs], dk=dks[s][:, kr], dv=dvs[s][:, kr],
@@ -947,14 +957,14 @@ class QKVRoPEAttnFunc(torch.autograd.Function):
         ctx.save_for_backward(x2, weight, qkv, out, lse, table)
         ctx.dims = (n_heads, n_kv_heads, head_dim, softmax_scale, x.shape)
         ctx.mark_non_differentiable(lse, qkv)
+        ctx.set_materialize_grads(False)   # at 16384 tokens the zero gradient of qkv alone was a 26 us fill of 200 MB
         return qkv, out, lse
 
     @staticmethod
     def backward(ctx, _dqkv, dout, _dlse):
         x2, weight, qkv, out, lse, table = ctx.saved_tensors
         n_heads, n_kv_heads, head_dim, softmax_scale, x_shape = ctx.dims
-        if dout.stride(3) != 1:
-            dout = dout.contiguous()
+        dout = _dense_dout(dout, out)
         dqkv = torch.empty_like(qkv)
         a, b = n_heads, n_heads + n_kv_heads
         attn_bwd(qkv[:, :, :a], qkv[:, :, a:b], qkv[:, :, b:], out, lse, dout, causal=True, scale=softmax_scale,
