@@ -1,4 +1,5 @@
 // extern "C" entry points for attention.
+#include <algorithm>
 #include <cmath>
 #include <mutex>
 #include "attn_params.h"
@@ -89,6 +90,7 @@ int attn_fwd_impl(const char* who, const void* q, const void* k, const void* v, 
                 "%s: workspace must be 256-byte aligned", who);
     return ody_launch_attn_fwd_w8(p, workspace, workspace_bytes, st);
   }
+  if (dtype == ODY_BF16 && p.drop_thresh == 0) return ody_launch_attn_fwd_hd64(p, st);
   if (dtype == ODY_BF16) return ody_launch_attn_fwd_mfma(p, D, st);
   return ody_launch_attn_fwd_f32(p, D, st);
 }
@@ -190,6 +192,7 @@ extern "C" size_t ody_attn_bwd_workspace_bytes(int B, int Lq, int Lk, int Hq, in
   if (B <= 0 || Lq <= 0 || Lk <= 0 || Hq <= 0 || Hkv <= 0) return 0;
   size_t n = delta_bytes(B, Lq, Hq);
   if (dtype == ODY_BF16 && D == 128) n += ody_attn_bwd_pipe_workspace(B, Lq, Lk, Hq, Hkv);
+  if (dtype == ODY_BF16 && D == 64) n = std::max(n, ody_attn_bwd_hd64_workspace(B, Lq, Lk, Hq, Hkv));   // with dropout: delta
   return n;
 }
 
@@ -269,6 +272,7 @@ int attn_bwd_impl(const char* who, const void* rope_q, const void* rope_k,
   hipStream_t st = static_cast<hipStream_t>(stream);
   if (dtype == ODY_BF16 && D == 128 && p.drop_thresh == 0)   // its query-side pre-pass computes delta as well
     return ody_launch_attn_bwd_pipe(p, static_cast<char*>(workspace) + delta_bytes(B, Lq, Hq), st);
+  if (dtype == ODY_BF16 && p.drop_thresh == 0) return ody_launch_attn_bwd_hd64(p, workspace, st);
   if (!p.reuse_query_side && (rc = ody_launch_attn_delta(p, D, dtype, st))) return rc;
   if (dtype == ODY_BF16) return ody_launch_attn_bwd_mfma(p, D, st);
   return ody_launch_attn_bwd_f32(p, D, st);

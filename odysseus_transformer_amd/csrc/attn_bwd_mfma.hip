@@ -385,9 +385,7 @@ int ody_launch_attn_bwd_mfma(const AttnParams& p, int D, hipStream_t st) {
   if (p.drop_thresh != 0) {   // dropout: these kernels serve both head dims
     if (D == 64) return launch<64, true>(p, st);
     if (D == 128) return launch<128, true>(p, st);
-  } else if (D == 64) {
-    return launch<64, false>(p, st);   // head_dim 128 has its own kernels (attn_bwd_pipe.hip)
-  }
+  }   // without it: attn_bwd_pipe.hip, attn_hd64.hip
   ody_set_error("attn_bwd: head_dim %d not built here", D);
   return ODY_ERR_UNSUPPORTED;
 }

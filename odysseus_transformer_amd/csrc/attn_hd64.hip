@@ -1,0 +1,671 @@
+// Flash attention for bf16 and head_dim 64, forward and backward, deterministic, without images or atomics.
+//
+// At head_dim 64 a (query, key) pair costs half the MFMA work of head_dim 128 and the same exp, conversions and sums: the
+// vector pipe is the bound (forward: about 900 vector cycles per 512 matrix cycles of a 32 x 64 score tile), not LDS.  So, unlike
+// the head_dim-128 kernels, operands that a product contracts over their row index are read with the transposing LDS read from
+// the same tile as the row operands -- no transposed images, hence no pre-pass over V and K and half the tile bytes --, three
+// or four wavefronts share a SIMD to keep the vector pipe fed, and the softmax of the forward does no work that the result does
+// not need: a row's reference is the maximum of its first tile, nothing is compared or rescaled after it, and a block where a
+// later score outgrew that by more than fp32 holds walks its keys once more with a reference that follows.
+//
+// A block is 4 wavefronts of 32 rows each (queries; keys in the dK/dV kernel) against 64-row tiles of the other side, which go
+// straight to LDS (direct loads, two stages).  GROUPS = 2 gives a block a second set of 4 wavefronts over the same rows, which
+// takes every other tile; the sets add up through LDS at the end.  It is for calls with too few blocks to give every SIMD three
+// wavefronts.
+//
+// Tile layout in LDS: 64 rows of 128 bytes; 16-byte chunk c of row r sits at position c ^ swz(r), swz(r) = bits 3, 2, 1 of r in
+// bits 0, 1, 2.  Conflict-free for both kinds of read: the 16 rows that a 16-byte read serves together (attn_tile.h) have pairwise
+// different (r & 1, swz), and of the four rows of a transposing read those two that share a 128-byte half differ in bit 2 of swz.
+// The permutation is applied to the source chunk of each lane, as a direct load writes its lanes to consecutive addresses.
+//
+// Measured against the kernels these replace (register-staged tiles through padded LDS rows, rescaling on every tile, one block per
+// kv head), us: 16 heads, L = 8192, causal: forward 207 -> 158 (870 TFLOP/s), dK/dV 415 -> 285, dQ 323 -> 213; 2 x 8 heads, L = 500,
+// causal: 14 -> 10.7, 22.6 -> 16, 19.3 -> 11; 8 heads on 2 kv heads, L = 2000, full: 42 -> 26, 279 -> 45, 65 -> 30.  At the long
+// shape the vector pipe is 70 % and the matrix pipe 46 % busy in the forward (16 % of the units' time is the causal tail), matrix 52 %
+// and vector 45 % in dK/dV and dQ at 2.0 GHz.  Without effect: raised priority around the matrix steps, two wavefronts a SIMD
+// instead of three in the backward.
+#include <type_traits>
+#include <utility>
+#include "attn_params.h"
+#include "attn_tile.h"
+
+namespace {
+
+constexpr int D = 64, KS = D / 16, DT = D / 32, ROWS = 64, TILE = ROWS * D;   // elements of a tile: 8 KB
+constexpr int BLOCK_ROWS = 128;
+typedef __attribute__((address_space(3))) void* lds_ptr;
+typedef __attribute__((address_space(1))) const void* global_ptr;
+
+__device__ __forceinline__ int swz(int r) { return ((r & 2) << 1) | ((r & 4) >> 1) | ((r & 8) >> 3); }
+
+// Fragment reads go by LDS byte addresses: what depends on the lane and the stage sits in 8 registers that move from stage to
+// stage, the rest is in the offset field of the instruction.
+struct Readers {
+  unsigned row[KS], tr[4];
+  __device__ __forceinline__ void init(const bf16* stage, int g, int i) {
+    const unsigned a = (unsigned)(uintptr_t)(lds_ptr)const_cast<bf16*>(stage);
+    const int rb = i * D + 8 * (g ^ swz(i));
+#pragma unroll
+    for (int ks = 0; ks < KS; ks++) row[ks] = a + 2 * (rb ^ (16 * ks));
+    const int t = (i & 15) >> 2;
+    const int tb = (4 * g + t) * D + 8 * ((2 * (i >> 4) + ((i & 3) >> 1)) ^ (4 * (t >> 1) + 2 * g)) + 4 * (i & 1);
+    tr[0] = a + 2 * tb, tr[1] = a + 2 * (tb ^ 8), tr[2] = a + 2 * (tb ^ 32), tr[3] = a + 2 * (tb ^ 40);
+  }
+  __device__ __forceinline__ void move(int bytes) {
+#pragma unroll
+    for (int n = 0; n < 4; n++) row[n] += bytes, tr[n] += bytes;
+  }
+};
+// A operand, rows first .. first + 31 behind the stage's start: lane (g, i) holds row i, k = 16 ks + 8 g .. + 7
+__device__ __forceinline__ bf16x8 row_frag(const Readers& r, int first, int ks) {
+  typedef const bf16x8 __attribute__((address_space(3))) * frag_ptr;
+  return *(frag_ptr)(uintptr_t)(r.row[ks] + 2 * first * D);
+}
+// A operands of the transposed tile, 16 rows from FIRST on: lane (g, i) of f[dt] holds column 32 dt + i, and k element e is row
+// FIRST + 8 (e >> 2) + 4 g + (e & 3) -- the order in which accumulators hold their rows, so that P and dS go from accumulator to
+// B operand in place.  The reads and the wait for them are one piece of assembly: behind the intrinsic the compiler waits for
+// every direct load in flight, as for possible writers of what is read here.
+template <int FIRST>
+__device__ __forceinline__ void tr_frags(bf16x8 (&f)[DT], const Readers& r) {
+  s16x4 x0, x1, y0, y1;
+  asm volatile("ds_read_b64_tr_b16 %0, %4 offset:%8\n\tds_read_b64_tr_b16 %1, %5 offset:%9\n\t"
+               "ds_read_b64_tr_b16 %2, %6 offset:%8\n\tds_read_b64_tr_b16 %3, %7 offset:%9\n\ts_waitcnt lgkmcnt(0)"
+               : "=&v"(x0), "=&v"(x1), "=&v"(y0), "=&v"(y1)
+               : "v"(r.tr[0]), "v"(r.tr[1]), "v"(r.tr[2]), "v"(r.tr[3]), "n"(2 * FIRST * D), "n"(2 * (FIRST + 8) * D)
+               : "memory");
+  f[0] = concat4(__builtin_bit_cast(bf16x4, x0), __builtin_bit_cast(bf16x4, x1));
+  f[1] = concat4(__builtin_bit_cast(bf16x4, y0), __builtin_bit_cast(bf16x4, y1));
+}
+// Blocks heaviest first, all (head, batch) pairs of a rank together (ody_block_coord), and under a causal mask every other run
+// of 256 blocks with its ranks reversed: the three or four blocks that share a compute unit then add up to about the same
+// length.  In plain order the units with the first blocks of every run got 320 tiles where the mean was 260 (forward of 16 heads,
+// L = 8192: 182 us, 158 this way).
+__device__ __forceinline__ BlockCoord block_coord(int H, int B, int causal) {
+  BlockCoord c = ody_block_coord(H, B);
+  const int ranks = gridDim.x / (H * B), run = max(1, 256 / (H * B)), n = c.rank / run;
+  if (causal && (n & 1) && (n + 1) * run <= ranks) c.rank = n * run + run - 1 - c.rank % run;
+  return c;
+}
+// row of accumulator register r
+__device__ __forceinline__ int acc_row(int r, int g) { return 8 * (r >> 2) + 4 * g + (r & 3); }
+
+// Direct loads of 64-row tiles of one matrix: 8 instructions of 8 rows, two per wavefront of a group.  Rows at or beyond nrows
+// re-read the last one (finite filler that the caller masks); tiles start below nrows.
+struct TileLoader {
+  int64_t off, stride;   // of this lane's chunk in the first instruction; row stride
+  int row;
+  __device__ __forceinline__ void init(int64_t s, int w4, int lane) {
+    row = 8 * w4 + (lane >> 3);
+    off = (int64_t)row * s + 8 * ((lane & 7) ^ swz(row));
+    stride = s;
+  }
+  // base: the matrix of this (batch, head), uniform
+  __device__ __forceinline__ void load(bf16* tile, const bf16* base, int row0, int nrows, int w4) const {
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+      const bf16* src = base + (int64_t)(row0 + 32 * j) * stride + off;
+      if (row0 + ROWS > nrows) src += (int64_t)min(nrows - 1 - row0 - 32 * j - row, 0) * stride;
+      __builtin_amdgcn_global_load_lds((global_ptr)src, (lds_ptr)(tile + (4 * j + w4) * 512), 16, 0, 0);
+    }
+  }
+};
+
+// The 32 rows of a wavefront as B operands: lane (g, i) holds row `row`, k = 16 ks + 8 g .. + 7; zero beyond nrows
+__device__ __forceinline__ void load_rows(bf16x8 (&f)[KS], const bf16* base, int64_t stride, int row, int nrows, int g) {
+#pragma unroll
+  for (int ks = 0; ks < KS; ks++) {
+    f[ks] = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
+    if (row < nrows) f[ks] = *reinterpret_cast<const bf16x8*>(base + (int64_t)row * stride + 16 * ks + 8 * g);
+  }
+  // arrived before the loop: left pending, the wait for them would land on a use inside it, as a wait for the tile loads too
+#pragma unroll
+  for (int ks = 0; ks < KS; ks++) asm volatile("" : "+v"(f[ks]));
+}
+
+__device__ __forceinline__ void clear(f32x16 (&x)[DT]) {
+#pragma unroll
+  for (int dt = 0; dt < DT; dt++)
+#pragma unroll
+    for (int r = 0; r < 16; r++) x[dt][r] = 0.f;
+}
+
+// accumulators of the second group to LDS, and back into the first (dst [register][lane] of this wavefront)
+__device__ __forceinline__ void give(float* patch, const f32x16 (&x)[DT], int lane) {
+#pragma unroll
+  for (int dt = 0; dt < DT; dt++)
+#pragma unroll
+    for (int r = 0; r < 16; r++) patch[(16 * dt + r) * 64 + lane] = x[dt][r];
+}
+__device__ __forceinline__ void take(const float* patch, f32x16 (&x)[DT], int lane, float mine, float theirs) {
+#pragma unroll
+  for (int dt = 0; dt < DT; dt++)
+#pragma unroll
+    for (int r = 0; r < 16; r++) x[dt][r] = x[dt][r] * mine + patch[(16 * dt + r) * 64 + lane] * theirs;
+}
+
+// D accumulator columns of one row -> bf16 row
+__device__ __forceinline__ void store_row(bf16* dst, const f32x16 (&x)[DT], float scale, int g) {
+#pragma unroll
+  for (int dt = 0; dt < DT; dt++)
+#pragma unroll
+    for (int a = 0; a < 4; a++) {
+      bf16x4 w;
+#pragma unroll
+      for (int e = 0; e < 4; e++) w[e] = (bf16)(x[dt][4 * a + e] * scale);
+      *reinterpret_cast<bf16x4*>(dst + 32 * dt + 8 * a + 4 * g) = w;
+    }
+}
+
+constexpr size_t KV_STAGE = 2 * TILE;                    // elements: two tiles
+constexpr size_t QS_STAGE = 2 * TILE + 2 * 2 * ROWS;     // Q and dO tiles, -lse / scale and -delta of their rows in fp32
+static_assert(2 * 2 * KV_STAGE * sizeof(bf16) >= 4 * 34 * 64 * sizeof(float) && 2 * 2 * QS_STAGE * sizeof(bf16) >= 4 * 64 * 64 * sizeof(float),
+              "what a group hands over fits in the stages of two");
+
+// ---------------------------------------------------------------------------------------------------------- forward
+//   S^T = K Q^T      O^T += V^T P^T       lane = query column
+template <int GROUPS>
+__global__ __launch_bounds__(256 * GROUPS, 4) void attn_fwd_hd64_kernel(const AttnParams p) {
+  constexpr size_t STAGE_BYTES = KV_STAGE * sizeof(bf16);
+  extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, g = lane >> 5, i = lane & 31;
+  const int grp = wave >> 2, w4 = wave & 3;
+  bf16* ring = reinterpret_cast<bf16*>(smem) + grp * 2 * KV_STAGE;   // [2][K tile | V tile]
+  const BlockCoord bc = block_coord(p.Hq, p.B, p.causal);
+  const int nqb = gridDim.x / (p.Hq * p.B);
+  const int qblk = p.causal ? nqb - 1 - bc.rank : bc.rank;   // heaviest blocks first
+  const int h = bc.h, b = bc.b, hk = h / p.group;
+  const int q0 = qblk * BLOCK_ROWS, wq0 = q0 + w4 * 32, qi = wq0 + i;
+
+  int n_end = p.causal ? min(p.Lk, min(q0 + BLOCK_ROWS, p.Lq) + p.off) : p.Lk;
+  const int ntiles = n_end > 0 ? (n_end + ROWS - 1) / ROWS : 0;
+  TileLoader lk, lv;
+  lk.init(p.sk.l, w4, lane);
+  lv.init(p.sv.l, w4, lane);
+  const bf16* kp = static_cast<const bf16*>(p.k) + b * p.sk.b + hk * p.sk.h;
+  const bf16* vp = static_cast<const bf16*>(p.v) + b * p.sv.b + hk * p.sv.h;
+  auto load = [&](int t, int buf) {
+    lk.load(ring + buf * KV_STAGE, kp, t * ROWS, p.Lk, w4);
+    lv.load(ring + buf * KV_STAGE + TILE, vp, t * ROWS, p.Lk, w4);
+  };
+
+  bf16x8 qf[KS];
+  load_rows(qf, static_cast<const bf16*>(p.q) + b * p.sq.b + h * p.sq.h, p.sq.l, qi, p.Lq, g);
+  const int lim = p.causal ? min(p.Lk - 1, qi + p.off) : p.Lk - 1;   // last key this lane's query sees
+  const float c2 = p.scale_log2e;
+  f32x16 o[DT];
+  float ref;     // the row's reference in log2 units
+  float l4[4];   // this lane's partial row sums
+
+  // ONLINE = false: the reference of a row is the largest score of its first tile (a row that sees any key sees key 0) and stays.
+  // ONLINE = true: it follows the maximum, in steps of 2^8 and more.
+  const int iters = (ntiles + GROUPS - 1) / GROUPS;
+  auto walk = [&](auto online) {
+    constexpr bool ONLINE = decltype(online)::value;
+    clear(o);
+    ref = -1e30f;   // below any score until a key was seen
+#pragma unroll
+    for (int e = 0; e < 4; e++) l4[e] = 0.f;
+    Readers rd;
+    rd.init(ring, g, i);
+    auto tile = [&](int t, bool first) {
+      const int n0 = t * ROWS;
+      if (t >= ntiles || (p.causal && n0 > wq0 + 31 + p.off)) return;
+      f32x16 s[2];
+#pragma unroll
+      for (int ks = 0; ks < KS; ks++)
+#pragma unroll
+        for (int kt = 0; kt < 2; kt++) s[kt] = mfma32(row_frag(rd, 32 * kt, ks), qf[ks], ks == 0 ? f32x16{0} : s[kt]);
+      if (n0 + ROWS > p.Lk || (p.causal && n0 + ROWS - 1 > wq0 + p.off)) {
+#pragma unroll
+        for (int kt = 0; kt < 2; kt++)
+#pragma unroll
+          for (int r = 0; r < 16; r++)
+            if (n0 + 32 * kt + acc_row(r, g) > lim) s[kt][r] = -INFINITY;
+      }
+      if (ONLINE || first) {
+        float mx = fmaxf(s[0][0], s[1][0]);
+#pragma unroll
+        for (int r = 1; r < 16; r++) mx = fmaxf(mx, fmaxf(s[0][r], s[1][r]));
+        mx = half_swap_max(mx) * c2;
+        if (__builtin_amdgcn_ballot_w64(mx > ref + 8.f) != 0) {
+          const float next = fmaxf(ref, mx), alpha = ody_exp2(ref - next);
+          ref = next;
+#pragma unroll
+          for (int e = 0; e < 4; e++) l4[e] *= alpha;
+#pragma unroll
+          for (int dt = 0; dt < DT; dt++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) o[dt][r] *= alpha;
+        }
+      }
+      auto half = [&](auto which) {
+        constexpr int kt = decltype(which)::value;
+        bf16x8 pb[2], vf[DT];
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+          const float x = ody_exp2(fmaf(s[kt][r], c2, -ref));
+          l4[r & 3] += x;
+          pb[r >> 3][r & 7] = (bf16)x;
+        }
+        tr_frags<ROWS + 32 * kt>(vf, rd);
+#pragma unroll
+        for (int dt = 0; dt < DT; dt++) o[dt] = mfma32(vf[dt], pb[0], o[dt]);
+        tr_frags<ROWS + 32 * kt + 16>(vf, rd);
+#pragma unroll
+        for (int dt = 0; dt < DT; dt++) o[dt] = mfma32(vf[dt], pb[1], o[dt]);
+      };
+      half(std::integral_constant<int, 0>{});
+      half(std::integral_constant<int, 1>{});
+    };
+    if (grp < ntiles) load(grp, 0);
+    for (int it = 0; it < iters; it++) {
+      const int t = grp + GROUPS * it;
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __syncthreads();   // the tile has landed, and everyone is done with the one before
+      if (t + GROUPS < ntiles) load(t + GROUPS, (it + 1) & 1);
+      tile(t, it == 0);
+      rd.move((it & 1) ? -(int)STAGE_BYTES : (int)STAGE_BYTES);
+    }
+    __syncthreads();   // everyone is done with the stages
+  };
+  walk(std::false_type{});
+  {
+    // a later score that outgrew its row's reference by more than fp32 holds left a row sum beyond any real one (or a NaN)
+    int* flags = reinterpret_cast<int*>(smem);
+    const bool beyond = __builtin_amdgcn_ballot_w64(!(half_swap_sum((l4[0] + l4[1]) + (l4[2] + l4[3])) < 0x1p100f)) != 0;
+    if (lane == 0) flags[wave] = beyond;
+    __syncthreads();
+    int any = 0;
+#pragma unroll
+    for (int w = 0; w < 4 * GROUPS; w++) any |= flags[w];
+    __syncthreads();
+    if (any) walk(std::true_type{});
+  }
+
+  float l = (l4[0] + l4[1]) + (l4[2] + l4[3]);
+#pragma unroll 1
+  for (int from = 1; from < GROUPS; from++) {
+    float* patch = reinterpret_cast<float*>(smem) + w4 * 34 * 64;
+    if (grp == from) {
+      give(patch, o, lane);
+      patch[32 * 64 + lane] = ref;
+      patch[33 * 64 + lane] = l;
+    }
+    __syncthreads();
+    if (grp == 0) {
+      const float ref1 = patch[32 * 64 + lane], next = fmaxf(ref, ref1), a0 = ody_exp2(ref - next), a1 = ody_exp2(ref1 - next);
+      take(patch, o, lane, a0, a1);
+      l = l * a0 + patch[33 * 64 + lane] * a1;
+      ref = next;
+    }
+    __syncthreads();
+  }
+  if (grp != 0) return;
+  l = half_swap_sum(l);
+  if (qi < p.Lq) {
+    const float inv = l > 0.f ? 1.f / l : 0.f;
+    store_row(static_cast<bf16*>(p.out) + b * p.so.b + h * p.so.h + (int64_t)qi * p.so.l, o, inv, g);
+    if (g == 0) p.lse[((int64_t)b * p.Hq + h) * p.Lq + qi] = l > 0.f ? (ref + __log2f(l)) * ODY_LN2 : -INFINITY;
+  }
+}
+
+// ---------------------------------------------------------------------------------------------------------- backward
+// Per query row, [-lse / scale | -delta] in fp32, rows padded to whole tiles: what S and dP start from in the dK/dV kernel.  Rows
+// that must give P = 0 (padding, or a query that saw no key) hold -1e30.  8 lanes per row.
+__global__ __launch_bounds__(256) void attn_bwd_hd64_rows_kernel(const AttnParams p, float* __restrict__ stats, int rows) {
+  const int lane8 = threadIdx.x & 7, qi = blockIdx.x * 32 + (threadIdx.x >> 3), h = blockIdx.y, b = blockIdx.z;
+  float acc = 0.f;
+  if (qi < p.Lq) {
+    const bf16x8 ov = *reinterpret_cast<const bf16x8*>(static_cast<const bf16*>(p.out) + b * p.so.b + h * p.so.h + (int64_t)qi * p.so.l + 8 * lane8);
+    const bf16x8 dv = *reinterpret_cast<const bf16x8*>(static_cast<const bf16*>(p.dout) + b * p.sdo.b + h * p.sdo.h + (int64_t)qi * p.sdo.l + 8 * lane8);
+#pragma unroll
+    for (int e = 0; e < 8; e++) acc = fmaf((float)ov[e], (float)dv[e], acc);
+  }
+#pragma unroll
+  for (int sft = 4; sft > 0; sft >>= 1) acc += __shfl_xor(acc, sft, 64);
+  if (lane8 != 0) return;
+  const int64_t head = (int64_t)b * p.Hq + h;
+  const float l = qi < p.Lq ? p.lse[head * p.Lq + qi] : INFINITY;
+  stats[head * rows + qi] = (l == INFINITY || l == -INFINITY) ? -1e30f : -l / p.scale;
+  stats[((int64_t)p.B * p.Hq + head) * rows + qi] = -acc;
+}
+
+//   S = Q K^T - lse / scale     dP = dO V^T - delta     dV^T += dO^T P     dK^T += Q^T (P o dP)      lane = key column
+//
+// PART: the block takes ONE query head and leaves fp32 sums in part [dK | dV][B][Hq][Lk][D], which the kernel below adds over the
+// heads of a group; otherwise it walks all query heads of its kv head.
+template <int GROUPS, bool PART>
+__global__ __launch_bounds__(256 * GROUPS, GROUPS == 1 ? 3 : 2) void attn_bwd_hd64_dkdv_kernel(const AttnParams p, const float* __restrict__ stats, int rows,
+                                                                            float* __restrict__ part) {
+  constexpr size_t STAGE_BYTES = QS_STAGE * sizeof(bf16);
+  extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, g = lane >> 5, i = lane & 31;
+  const int grp = wave >> 2, w4 = wave & 3;
+  bf16* ring = reinterpret_cast<bf16*>(smem) + grp * 2 * QS_STAGE;   // [2][Q tile | dO tile | row values]
+  const BlockCoord bc = block_coord(PART ? p.Hq : p.Hkv, p.B, p.causal);   // rank 0 = first key block = most query tiles
+  const int b = bc.b, hk = PART ? bc.h / p.group : bc.h, h_first = PART ? bc.h : hk * p.group, heads = PART ? 1 : p.group;
+  const int n0 = bc.rank * BLOCK_ROWS, wn0 = n0 + w4 * 32, key = wn0 + i;
+
+  const int t_begin = p.causal ? max(0, n0 - p.off) / ROWS : 0, t_end = (p.Lq + ROWS - 1) / ROWS;
+  const int ntq = max(0, t_end - t_begin), total = ntq * heads;
+  // Tile `it` of the flattened (query head, query tile) range, last query tile first: the key blocks that run at one time on an
+  // XCD then read the same Q and dO tiles.
+  TileLoader lq, lo;
+  lq.init(p.sq.l, w4, lane);
+  lo.init(p.sdo.l, w4, lane);
+  auto load = [&](int it, int buf) {
+    const int h = h_first + it / ntq, t = t_end - 1 - it % ntq;
+    bf16* st = ring + buf * QS_STAGE;
+    lq.load(st, static_cast<const bf16*>(p.q) + b * p.sq.b + h * p.sq.h, t * ROWS, p.Lq, w4);
+    lo.load(st + TILE, static_cast<const bf16*>(p.dout) + b * p.sdo.b + h * p.sdo.h, t * ROWS, p.Lq, w4);
+    if (w4 < 2) {
+      const float* src = stats + ((int64_t)w4 * p.B * p.Hq + (int64_t)b * p.Hq + h) * rows + t * ROWS + lane;
+      __builtin_amdgcn_global_load_lds((global_ptr)src, (lds_ptr)(st + 2 * TILE + w4 * 2 * ROWS), 4, 0, 0);
+    }
+  };
+  if (grp < total) load(grp, 0);
+
+  bf16x8 kf[KS], vf[KS];
+  load_rows(kf, static_cast<const bf16*>(p.k) + b * p.sk.b + hk * p.sk.h, p.sk.l, key, p.Lk, g);
+  load_rows(vf, static_cast<const bf16*>(p.v) + b * p.sv.b + hk * p.sv.h, p.sv.l, key, p.Lk, g);
+  const float c2 = p.scale_log2e;
+  Readers rd;
+  rd.init(ring, g, i);
+  f32x16 dk[DT], dv[DT];
+  clear(dk);
+  clear(dv);
+
+  const int iters = (total + GROUPS - 1) / GROUPS;
+  for (int n = 0; n < iters; n++) {
+    const int it = grp + GROUPS * n, i0 = (t_end - 1 - it % max(ntq, 1)) * ROWS;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (it + GROUPS < total) load(it + GROUPS, (n + 1) & 1);
+    const bf16* stage = ring + (n & 1) * QS_STAGE;
+    const float* rv = reinterpret_cast<const float*>(stage + 2 * TILE) + 4 * g;
+    auto sub_tile = [&](auto which) {
+      __builtin_amdgcn_sched_barrier(0);   // one sub-tile's fragments at a time
+      constexpr int mt = decltype(which)::value;
+      const int m0 = i0 + 32 * mt;
+      // every query of the sub-tile comes before every key of this wavefront: nothing to do
+      if (it >= total || m0 >= p.Lq || (p.causal && m0 + 31 + p.off < wn0)) return;
+      f32x16 s, dp;
+#pragma unroll
+      for (int a = 0; a < 4; a++) {
+        const f32x4 x = *reinterpret_cast<const f32x4*>(rv + 32 * mt + 8 * a);
+        const f32x4 y = *reinterpret_cast<const f32x4*>(rv + ROWS + 32 * mt + 8 * a);
+#pragma unroll
+        for (int e = 0; e < 4; e++) s[4 * a + e] = x[e], dp[4 * a + e] = y[e];
+      }
+#pragma unroll
+      for (int ks = 0; ks < KS; ks++) {
+        s = mfma32(row_frag(rd, 32 * mt, ks), kf[ks], s);
+        dp = mfma32(row_frag(rd, ROWS + 32 * mt, ks), vf[ks], dp);
+      }
+      if (p.causal && m0 + p.off < wn0 + 31) {
+#pragma unroll
+        for (int r = 0; r < 16; r++)
+          if (m0 + acc_row(r, g) + p.off < key) s[r] = -INFINITY;
+      }
+      bf16x8 pf[2], dsf[2];
+#pragma unroll
+      for (int r = 0; r < 16; r++) {
+        const float pr = ody_exp2(s[r] * c2);
+        pf[r >> 3][r & 7] = (bf16)pr;
+        dsf[r >> 3][r & 7] = (bf16)(pr * dp[r]);
+      }
+      auto products = [&](auto half) {
+        constexpr int ss = decltype(half)::value;
+        bf16x8 of[DT], qf[DT];
+        tr_frags<ROWS + 32 * mt + 16 * ss>(of, rd);
+        tr_frags<32 * mt + 16 * ss>(qf, rd);
+#pragma unroll
+        for (int dt = 0; dt < DT; dt++) {
+          dv[dt] = mfma32(of[dt], pf[ss], dv[dt]);
+          dk[dt] = mfma32(qf[dt], dsf[ss], dk[dt]);
+        }
+      };
+      products(std::integral_constant<int, 0>{});
+      products(std::integral_constant<int, 1>{});
+    };
+    sub_tile(std::integral_constant<int, 0>{});
+    sub_tile(std::integral_constant<int, 1>{});
+    rd.move((n & 1) ? -(int)STAGE_BYTES : (int)STAGE_BYTES);
+  }
+
+#pragma unroll 1
+  for (int from = 1; from < GROUPS; from++) {
+    float* patch = reinterpret_cast<float*>(smem) + w4 * 64 * 64;
+    __syncthreads();
+    if (grp == from) {
+      give(patch, dk, lane);
+      give(patch + 32 * 64, dv, lane);
+    }
+    __syncthreads();
+    if (grp == 0) {
+      take(patch, dk, lane, 1.f, 1.f);
+      take(patch + 32 * 64, dv, lane, 1.f, 1.f);
+    }
+  }
+  if (grp != 0) return;
+  if (key >= p.Lk) return;
+  if (PART) {
+    float* pk = part + (((int64_t)b * p.Hq + bc.h) * p.Lk + key) * D;
+    float* pv = pk + (int64_t)p.B * p.Hq * p.Lk * D;
+#pragma unroll
+    for (int dt = 0; dt < DT; dt++)
+#pragma unroll
+      for (int a = 0; a < 4; a++) {
+        f32x4 wk, wv;
+#pragma unroll
+        for (int e = 0; e < 4; e++) wk[e] = dk[dt][4 * a + e], wv[e] = dv[dt][4 * a + e];
+        *reinterpret_cast<f32x4*>(pk + 32 * dt + 8 * a + 4 * g) = wk;
+        *reinterpret_cast<f32x4*>(pv + 32 * dt + 8 * a + 4 * g) = wv;
+      }
+  } else {
+    store_row(static_cast<bf16*>(p.dk) + b * p.sdk.b + hk * p.sdk.h + (int64_t)key * p.sdk.l, dk, p.scale, g);
+    store_row(static_cast<bf16*>(p.dv) + b * p.sdv.b + hk * p.sdv.h + (int64_t)key * p.sdv.l, dv, 1.f, g);
+  }
+}
+
+// dK, dV of a kv head = the sums of its query heads in their order; one thread per 4 elements
+__global__ __launch_bounds__(256) void attn_bwd_hd64_sum_kernel(const AttnParams p, const float* __restrict__ part) {
+  constexpr int Q = D / 4;
+  const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;   // over B * Hkv * Lk * D / 4
+  if (idx >= (int64_t)p.B * p.Hkv * p.Lk * Q) return;
+  const int d = 4 * (int)(idx % Q), key = (idx / Q) % p.Lk, hk = (idx / ((int64_t)Q * p.Lk)) % p.Hkv, b = idx / ((int64_t)Q * p.Lk * p.Hkv);
+  const int64_t plane = (int64_t)p.B * p.Hq * p.Lk * D;
+  const float* src = part + (((int64_t)b * p.Hq + hk * p.group) * p.Lk + key) * D + d;
+  f32x4 sk = {0.f, 0.f, 0.f, 0.f}, sv = sk;
+  for (int n = 0; n < p.group; n++, src += (int64_t)p.Lk * D) {
+    sk += *reinterpret_cast<const f32x4*>(src);
+    sv += *reinterpret_cast<const f32x4*>(src + plane);
+  }
+  bf16x4 wk, wv;
+#pragma unroll
+  for (int e = 0; e < 4; e++) wk[e] = (bf16)(sk[e] * p.scale), wv[e] = (bf16)sv[e];
+  *reinterpret_cast<bf16x4*>(static_cast<bf16*>(p.dk) + b * p.sdk.b + hk * p.sdk.h + (int64_t)key * p.sdk.l + d) = wk;
+  *reinterpret_cast<bf16x4*>(static_cast<bf16*>(p.dv) + b * p.sdv.b + hk * p.sdv.h + (int64_t)key * p.sdv.l + d) = wv;
+}
+
+//   S^T = K Q^T     dP^T = V dO^T - delta     dQ^T += K^T dS^T       lane = query column
+template <int GROUPS>
+__global__ __launch_bounds__(256 * GROUPS, GROUPS == 1 ? 3 : 2) void attn_bwd_hd64_dq_kernel(const AttnParams p, const float* __restrict__ stats,
+                                                                                           int rows) {
+  constexpr size_t STAGE_BYTES = KV_STAGE * sizeof(bf16);
+  extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, g = lane >> 5, i = lane & 31;
+  const int grp = wave >> 2, w4 = wave & 3;
+  bf16* ring = reinterpret_cast<bf16*>(smem) + grp * 2 * KV_STAGE;
+  const BlockCoord bc = block_coord(p.Hq, p.B, p.causal);
+  const int nqb = gridDim.x / (p.Hq * p.B);
+  const int qblk = p.causal ? nqb - 1 - bc.rank : bc.rank;
+  const int h = bc.h, b = bc.b, hk = h / p.group;
+  const int q0 = qblk * BLOCK_ROWS, wq0 = q0 + w4 * 32, qi = wq0 + i;
+
+  int n_end = p.causal ? min(p.Lk, min(q0 + BLOCK_ROWS, p.Lq) + p.off) : p.Lk;
+  const int ntiles = n_end > 0 ? (n_end + ROWS - 1) / ROWS : 0;
+  TileLoader lk, lv;
+  lk.init(p.sk.l, w4, lane);
+  lv.init(p.sv.l, w4, lane);
+  const bf16* kp = static_cast<const bf16*>(p.k) + b * p.sk.b + hk * p.sk.h;
+  const bf16* vp = static_cast<const bf16*>(p.v) + b * p.sv.b + hk * p.sv.h;
+  auto load = [&](int t, int buf) {
+    lk.load(ring + buf * KV_STAGE, kp, t * ROWS, p.Lk, w4);
+    lv.load(ring + buf * KV_STAGE + TILE, vp, t * ROWS, p.Lk, w4);
+  };
+  if (grp < ntiles) load(grp, 0);
+
+  bf16x8 qf[KS], dof[KS];
+  load_rows(qf, static_cast<const bf16*>(p.q) + b * p.sq.b + h * p.sq.h, p.sq.l, qi, p.Lq, g);
+  load_rows(dof, static_cast<const bf16*>(p.dout) + b * p.sdo.b + h * p.sdo.h, p.sdo.l, qi, p.Lq, g);
+  const int64_t head = (int64_t)b * p.Hq + h;
+  float lse2 = qi < p.Lq ? p.lse[head * p.Lq + qi] : INFINITY;
+  if (lse2 == -INFINITY) lse2 = INFINITY;   // a query that saw no key: P = 0
+  lse2 *= ODY_LOG2E;
+  const float nd = qi < p.Lq ? stats[((int64_t)p.B * p.Hq + head) * rows + qi] : 0.f;
+  f32x16 start;   // dP starts from -delta: one add less per element
+#pragma unroll
+  for (int r = 0; r < 16; r++) start[r] = nd;
+  const int lim = p.causal ? min(p.Lk - 1, qi + p.off) : p.Lk - 1;
+  const float c2 = p.scale_log2e;
+  Readers rd;
+  rd.init(ring, g, i);
+  f32x16 dq[DT];
+  clear(dq);
+
+  const int iters = (ntiles + GROUPS - 1) / GROUPS;
+  for (int it = 0; it < iters; it++) {
+    const int t = grp + GROUPS * it;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (t + GROUPS < ntiles) load(t + GROUPS, (it + 1) & 1);
+    auto sub_tile = [&](auto which) {
+      __builtin_amdgcn_sched_barrier(0);   // one sub-tile's fragments at a time
+      constexpr int kt = decltype(which)::value;
+      const int k0 = t * ROWS + 32 * kt;
+      if (t >= ntiles || k0 >= p.Lk || (p.causal && k0 > wq0 + 31 + p.off)) return;
+      f32x16 s, dp;
+#pragma unroll
+      for (int ks = 0; ks < KS; ks++) {
+        s = mfma32(row_frag(rd, 32 * kt, ks), qf[ks], ks == 0 ? f32x16{0} : s);
+        dp = mfma32(row_frag(rd, ROWS + 32 * kt, ks), dof[ks], ks == 0 ? start : dp);
+      }
+      if (k0 + 32 > p.Lk || (p.causal && k0 + 31 > wq0 + p.off)) {
+#pragma unroll
+        for (int r = 0; r < 16; r++)
+          if (k0 + acc_row(r, g) > lim) s[r] = -INFINITY;
+      }
+      bf16x8 dsf[2];
+#pragma unroll
+      for (int r = 0; r < 16; r++) dsf[r >> 3][r & 7] = (bf16)(ody_exp2(fmaf(s[r], c2, -lse2)) * dp[r]);
+      bf16x8 kf[DT];
+      tr_frags<32 * kt>(kf, rd);
+#pragma unroll
+      for (int dt = 0; dt < DT; dt++) dq[dt] = mfma32(kf[dt], dsf[0], dq[dt]);
+      tr_frags<32 * kt + 16>(kf, rd);
+#pragma unroll
+      for (int dt = 0; dt < DT; dt++) dq[dt] = mfma32(kf[dt], dsf[1], dq[dt]);
+    };
+    sub_tile(std::integral_constant<int, 0>{});
+    sub_tile(std::integral_constant<int, 1>{});
+    rd.move((it & 1) ? -(int)STAGE_BYTES : (int)STAGE_BYTES);
+  }
+
+#pragma unroll 1
+  for (int from = 1; from < GROUPS; from++) {
+    float* patch = reinterpret_cast<float*>(smem) + w4 * 32 * 64;
+    __syncthreads();
+    if (grp == from) give(patch, dq, lane);
+    __syncthreads();
+    if (grp == 0) take(patch, dq, lane, 1.f, 1.f);
+  }
+  if (grp != 0) return;
+  if (qi >= p.Lq) return;
+  const int64_t at = b * p.sdq.b + h * p.sdq.h + (int64_t)qi * p.sdq.l;
+  if (p.dq_f32) {   // the running dq of a ring step: exact accumulation over the key blocks
+    float* dst = static_cast<float*>(p.dq) + at;
+#pragma unroll
+    for (int dt = 0; dt < DT; dt++)
+#pragma unroll
+      for (int a = 0; a < 4; a++) {
+        f32x4* x = reinterpret_cast<f32x4*>(dst + 32 * dt + 8 * a + 4 * g);
+        f32x4 w = {0.f, 0.f, 0.f, 0.f};
+        if (p.accumulate_dq) w = *x;
+#pragma unroll
+        for (int e = 0; e < 4; e++) w[e] += dq[dt][4 * a + e] * p.scale;
+        *x = w;
+      }
+  } else if (p.accumulate_dq) {
+    bf16* dst = static_cast<bf16*>(p.dq) + at;
+#pragma unroll
+    for (int dt = 0; dt < DT; dt++)
+#pragma unroll
+      for (int a = 0; a < 4; a++) {
+        bf16x4* x = reinterpret_cast<bf16x4*>(dst + 32 * dt + 8 * a + 4 * g);
+        const bf16x4 old = *x;
+        bf16x4 w;
+#pragma unroll
+        for (int e = 0; e < 4; e++) w[e] = (bf16)(dq[dt][4 * a + e] * p.scale + (float)old[e]);
+        *x = w;
+      }
+  } else {
+    store_row(static_cast<bf16*>(p.dq) + at, dq, p.scale, g);
+  }
+}
+
+inline size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
+inline int padded_rows(int Lq) { return (Lq + ROWS - 1) / ROWS * ROWS; }
+inline size_t stats_bytes(int B, int Lq, int Hq) { return align256((size_t)2 * B * Hq * padded_rows(Lq) * sizeof(float)); }
+inline int64_t row_blocks(int B, int L, int H) { return (int64_t)B * H * ((L + BLOCK_ROWS - 1) / BLOCK_ROWS); }
+
+// Fewer blocks than this leave SIMDs with one wavefront: two groups per block.  (More groups per block for all calls, which evens
+// out a causal mask by itself, loses more to the wider barrier: dK/dV of 16 heads, L = 8192, with three groups 342 us against 311.)
+constexpr int FEW_BLOCKS = 512;
+// one block per query head instead of one per kv head where the latter leave compute units idle
+inline bool split_heads(int B, int Lk, int Hq, int Hkv) { return Hq != Hkv && row_blocks(B, Lk, Hkv) < 1024; }
+
+template <typename K, typename... A>
+int launch(const char* name, K kern, int64_t blocks, int groups, size_t stage_elems, hipStream_t st, const A&... args) {
+  const size_t smem = (size_t)groups * 2 * stage_elems * sizeof(bf16);
+  if (int rc = ody_allow_dynamic_lds(reinterpret_cast<const void*>(kern), smem, name)) return rc;
+  ODY_LAUNCH(name, st, kern, dim3((unsigned)blocks), dim3(256 * groups), smem, args...);
+  return ody_check_launch(name);
+}
+
+}  // namespace
+
+int ody_launch_attn_fwd_hd64(const AttnParams& p, hipStream_t st) {
+  const int64_t blocks = row_blocks(p.B, p.Lq, p.Hq);
+  return blocks < FEW_BLOCKS ? launch("attn_fwd_hd64", &attn_fwd_hd64_kernel<2>, blocks, 2, KV_STAGE, st, p)
+                             : launch("attn_fwd_hd64", &attn_fwd_hd64_kernel<1>, blocks, 1, KV_STAGE, st, p);
+}
+
+// [row values | fp32 dK / dV of every query head]
+size_t ody_attn_bwd_hd64_workspace(int B, int Lq, int Lk, int Hq, int Hkv) {
+  return stats_bytes(B, Lq, Hq) + (split_heads(B, Lk, Hq, Hkv) ? align256((size_t)2 * B * Hq * Lk * D * sizeof(float)) : 0);
+}
+
+int ody_launch_attn_bwd_hd64(const AttnParams& p, void* workspace, hipStream_t st) {
+  float* stats = static_cast<float*>(workspace);
+  float* part = reinterpret_cast<float*>(static_cast<char*>(workspace) + stats_bytes(p.B, p.Lq, p.Hq));
+  const int rows = padded_rows(p.Lq);
+  int rc;
+  if (!p.reuse_query_side) {
+    ODY_LAUNCH("attn_bwd_hd64_rows", st, attn_bwd_hd64_rows_kernel, dim3(rows / 32, p.Hq, p.B), dim3(256), 0, p, stats, rows);
+    if ((rc = ody_check_launch("attn_bwd_hd64_rows"))) return rc;
+  }
+  const bool heads = split_heads(p.B, p.Lk, p.Hq, p.Hkv);
+  const int64_t nkv = row_blocks(p.B, p.Lk, heads ? p.Hq : p.Hkv), nq = row_blocks(p.B, p.Lq, p.Hq);
+  auto dkdv = [&](auto kern, int groups) { return launch("attn_bwd_hd64_dkdv", kern, nkv, groups, QS_STAGE, st, p, stats, rows, part); };
+  if (nkv < FEW_BLOCKS) rc = heads ? dkdv(&attn_bwd_hd64_dkdv_kernel<2, true>, 2) : dkdv(&attn_bwd_hd64_dkdv_kernel<2, false>, 2);
+  else rc = heads ? dkdv(&attn_bwd_hd64_dkdv_kernel<1, true>, 1) : dkdv(&attn_bwd_hd64_dkdv_kernel<1, false>, 1);
+  if (rc) return rc;
+  if (heads) {
+    const int64_t n = (int64_t)p.B * p.Hkv * p.Lk * (D / 4);
+    ODY_LAUNCH("attn_bwd_hd64_sum", st, attn_bwd_hd64_sum_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, p, part);
+    if ((rc = ody_check_launch("attn_bwd_hd64_sum"))) return rc;
+  }
+  return nq < FEW_BLOCKS ? launch("attn_bwd_hd64_dq", &attn_bwd_hd64_dq_kernel<2>, nq, 2, KV_STAGE, st, p, stats, rows)
+                         : launch("attn_bwd_hd64_dq", &attn_bwd_hd64_dq_kernel<1>, nq, 1, KV_STAGE, st, p, stats, rows);
+}

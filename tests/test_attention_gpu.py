@@ -564,3 +564,56 @@ def test_attention_fp32_few_and_many_rows(case, D, heads, dev):
     for got, ref, what in ((o, o_ref, "o"), (dq, dq_ref, "dq"), (dk, dk_ref, "dk"), (dv, dv_ref, "dv")):
         assert_parity(got, ref, TOL_F32, what, floor)
     assert torch.allclose(lse.cpu(), lse_ref, atol=TOL_LSE, rtol=TOL_LSE)
+
+
+HD64_CASES = [
+    # B, Lq, Lk, Hq, Hkv, causal: edges of the 32-row wavefronts, 64-row tiles and 128-row blocks; one and two wavefront groups per
+    # block (fewer than 512 blocks: two); dK / dV per kv head, per query head with a sum, and per kv head over a whole group
+    (1, 1, 1, 1, 1, True), (1, 31, 33, 2, 1, True), (2, 65, 64, 3, 3, False), (1, 127, 129, 4, 2, True), (1, 129, 127, 4, 1, False),
+    (1, 200, 72, 4, 4, True), (1, 100, 700, 4, 4, False), (1, 700, 100, 2, 2, False), (1, 70, 331, 8, 2, True), (1, 1031, 1031, 2, 1, True),
+    (2, 130, 130, 140, 140, True), (2, 130, 193, 280, 140, False), (1, 97, 161, 1040, 260, True), (4, 65, 65, 256, 128, True),
+]
+
+
+@pytest.mark.parametrize("spread", [1.0, 60.0], ids=["unit", "moving_reference"])
+@pytest.mark.parametrize("case", HD64_CASES, ids=lambda c: "B%d_Lq%d_Lk%d_H%d_%d_c%d" % c)
+def test_attention_hd64(case, spread, dev):
+    """The head_dim-64 kernels against the oracle.  spread > 1: keys grow along the sequence, so that a row's maximum keeps
+    outgrowing the reference its first tiles set (scores up to a few hundred), and the softmax is all but one-hot."""
+    from odysseus_transformer_amd import ops
+    B, Lq, Lk, Hq, Hkv, causal = case
+    print(f"case={case} spread={spread}", flush=True)
+    q, k, v, do = _inputs(B, Lq, Lk, Hq, Hkv, 64, torch.bfloat16, seed=23)
+    k = (k.float() * torch.linspace(1.0, spread, Lk)[None, :, None, None]).bfloat16()
+    o_ref, lse_ref = oracle.attention_fwd(q.float(), k.float(), v.float(), causal=causal)
+    dq_ref, dk_ref, dv_ref = oracle.attention_bwd(q.float(), k.float(), v.float(), o_ref, lse_ref, do.float(), causal=causal)
+    qg, kg, vg, dog = (t.to(dev) for t in (q, k, v, do))
+    o, lse = ops.attn_fwd(qg, kg, vg, causal=causal)
+    assert_parity(o, o_ref, TOL_BF16, "o")
+    assert torch.allclose(lse.cpu(), lse_ref, atol=TOL_LSE, rtol=TOL_LSE)
+    grads = ops.attn_bwd(qg, kg, vg, o, lse, dog, causal=causal)
+    floor = 1.0 if Lk == 1 else 1e-3
+    assert_parity(grads[2], dv_ref, TOL_BF16, "dv")
+    if spread == 1.0:   # one-hot rows leave dS = P (dP - delta) with nothing but the rounding of out
+        assert_parity(grads[0], dq_ref, TOL_BF16, "dq", floor)
+        assert_parity(grads[1], dk_ref, TOL_BF16, "dk", floor)
+    again = (*ops.attn_fwd(qg, kg, vg, causal=causal), *ops.attn_bwd(qg, kg, vg, o, lse, dog, causal=causal))
+    for a, b in zip((o, lse, *grads), again):
+        assert torch.equal(a, b)
+
+
+def test_attention_hd64_running_fp32_dq(dev):
+    """Two key blocks against the same queries: dq in fp32 over both calls, the second one reusing the query side."""
+    from odysseus_transformer_amd import ops
+    q, k, v, do = _inputs(1, 150, 260, 4, 2, 64, torch.bfloat16, seed=5)
+    o_ref, lse_ref = oracle.attention_fwd(q.float(), k.float(), v.float(), causal=False)
+    refs = oracle.attention_bwd(q.float(), k.float(), v.float(), o_ref, lse_ref, do.float(), causal=False)
+    qg, kg, vg, dog = (t.to(dev) for t in (q, k, v, do))
+    o, lse = o_ref.bfloat16().to(dev), lse_ref.to(dev)
+    dq = torch.empty(q.shape, dtype=torch.float32, device=dev)
+    ws = ops.attn_bwd_workspace(qg, kg[:, :130])
+    parts = [ops.attn_bwd(qg, kg[:, s], vg[:, s], o, lse, dog, causal=False, dq=dq, accumulate_dq=n > 0, workspace=ws,
+                          reuse_query_side=n > 0) for n, s in enumerate((slice(0, 130), slice(130, 260)))]
+    for got, ref, name in ((dq, refs[0], "dq"), (torch.cat([p[1] for p in parts], 1), refs[1], "dk"),
+                           (torch.cat([p[2] for p in parts], 1), refs[2], "dv")):
+        assert_parity(got, ref, TOL_BF16, name)
