@@ -44,6 +44,7 @@ struct Args {
   int M, N, K;
   int64_t lda, ldb, ldc, ld_add;
   int tiles_m, tiles_n;
+  int halved;         // the last tiles of the walk, worked on as two half tiles each (256 x 256 only)
   int vec16;          // C (and add) have 16-byte aligned rows
   GemmEpi ep;
 };
@@ -132,8 +133,15 @@ __device__ __forceinline__ void read_tr(unsigned addr, s16x4& lo, s16x4& hi) {
                : "v"(addr), "n"(OFF0), "n"(OFF1));
 }
 
+// Consecutive block ids go round-robin over the 8 XCDs, each with its own L2: give every XCD a contiguous range of the n positions.
+__device__ __forceinline__ int xcd_position(int id, int n) {
+  const int x = id & 7, whole = n >> 3, extra = n & 7;
+  return x * whole + min(x, extra) + (id >> 3);
+}
+
+// The BM x BN results from row m0 and column n0 on (n0 / BN = tn), this wavefront's share
 template <bool A_KC, bool B_KC, int BM, int BN, bool SPLITK, int EPI>
-__global__ __launch_bounds__(THREADS, BM * BN <= 128 * 128 ? 4 : 2) void gemm_tile_kernel(const Args p) {
+__device__ __forceinline__ void gemm_tile_block(const Args& p, int m0, int tn) {
   constexpr int WM = BM / 32, WN = BN / 64;      // 16-row blocks per wavefront: rows BM / 2, columns BN / 4
   constexpr int HALF = BM / 2, NH = WN / 2;
   static_assert(EPI == EPI_NONE || !SPLITK, "fused epilogues: one pass over K");
@@ -144,19 +152,7 @@ __global__ __launch_bounds__(THREADS, BM * BN <= 128 * 128 ? 4 : 2) void gemm_ti
 
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, c = lane & 15, q = lane >> 4;
   const int wm = wave >> 2, wn = wave & 3;
-
-  // Block -> tile.  Consecutive ids go round-robin over the 8 XCDs, each with its own L2: give every XCD a contiguous range of
-  // tiles, and inside it walk down M in groups of 8 so that the tiles in flight share panels of both operands.
-  int pid = blockIdx.x;
-  const int nblk = p.tiles_m * p.tiles_n;
-  {
-    const int x = pid & 7, whole = nblk >> 3, extra = nblk & 7;
-    pid = x * whole + min(x, extra) + (pid >> 3);
-  }
-  constexpr int GROUP = 8;
-  const int per_group = GROUP * p.tiles_n, gid = pid / per_group, first_m = gid * GROUP, gsz = min(p.tiles_m - first_m, GROUP);
-  const int tm = first_m + (pid % per_group) % gsz, tn = (pid % per_group) / gsz;
-  const int m0 = tm * BM, n0 = tn * BN;
+  const int n0 = tn * BN;
 
   // slabs [s0, s0 + nk) of the K range
   const int slabs = (p.K + BK - 1) / BK;
@@ -457,6 +453,32 @@ __global__ __launch_bounds__(THREADS, BM * BN <= 128 * 128 ? 4 : 2) void gemm_ti
 }
 #undef ODY_FENCE
 
+// Block -> tile: a walk down M in groups of 8 tiles, so that the tiles in flight share panels of both operands; first the whole
+// tiles, then, two blocks each, those whose halves fill a last round better (plan_bf16).
+template <bool A_KC, bool B_KC, int BM, int BN, bool SPLITK, int EPI>
+__global__ __launch_bounds__(THREADS, BM * BN <= 128 * 128 ? 4 : 2) void gemm_tile_kernel(const Args p) {
+  const int whole = p.tiles_m * p.tiles_n - p.halved;
+  int pos = blockIdx.x, half = 0;
+  const bool in_half = BM == 256 && !SPLITK && pos >= whole;
+  if (in_half) {
+    pos = xcd_position(pos - whole, 2 * p.halved);
+    half = pos & 1;
+    pos = whole + (pos >> 1);
+  } else {
+    pos = xcd_position(pos, whole);
+  }
+  constexpr int GROUP = 8;
+  const int per_group = GROUP * p.tiles_n, first_m = pos / per_group * GROUP, gsz = min(p.tiles_m - first_m, GROUP);
+  const int m0 = (first_m + (pos % per_group) % gsz) * BM, tn = (pos % per_group) / gsz;
+  if constexpr (BM == 256 && !SPLITK) {
+    if (in_half) {
+      if (m0 + 128 * half < p.M) gemm_tile_block<A_KC, B_KC, 128, BN, SPLITK, EPI>(p, m0 + 128 * half, tn);
+      return;
+    }
+  }
+  gemm_tile_block<A_KC, B_KC, BM, BN, SPLITK, EPI>(p, m0, tn);
+}
+
 template <bool A_KC, bool B_KC, int BM, int BN, bool SPLITK, int EPI>
 int launch(const char* name, Args a, int splits, hipStream_t st) {
   constexpr size_t smem = sizeof(bf16) * BK * (A_STAGES * BM + B_STAGES * BN);
@@ -465,7 +487,7 @@ int launch(const char* name, Args a, int splits, hipStream_t st) {
   if (int rc = ody_allow_dynamic_lds(reinterpret_cast<const void*>(kern), smem, name)) return rc;
   a.tiles_m = (a.M + BM - 1) / BM, a.tiles_n = (a.N + BN - 1) / BN;
   if (EPI == EPI_SWIGLU_FWD) a.tiles_n = (a.ep.I + BN / 2 - 1) / (BN / 2);
-  ODY_LAUNCH(name, st, kern, dim3(a.tiles_m * a.tiles_n, splits), dim3(THREADS), smem, a);
+  ODY_LAUNCH(name, st, kern, dim3(a.tiles_m * a.tiles_n + a.halved, splits), dim3(THREADS), smem, a);
   return ody_check_launch(name);
 }
 

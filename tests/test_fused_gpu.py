@@ -271,9 +271,9 @@ def test_fused_epilogues_with_few_rows(M, dev):
     assert rel_err(got, want) <= TOL_BF16, "rope"
 
 
-@pytest.mark.parametrize("T,I,K", [(65, 128, 72), (200, 384, 4096), (1000, 640, 520), (3001, 1408, 264)])
+@pytest.mark.parametrize("T,I,K", [(65, 128, 72), (200, 384, 4096), (1000, 640, 520), (3001, 1408, 264), (4104, 4224, 72)])
 def test_fused_epilogues_on_ragged_rows(T, I, K, dev):
-    """Rows and K that fill no tile, with and without K cut into ranges: SwiGLU both ways bit for bit against the two-kernel
+    """Rows and K that fill no tile, with and without K cut into ranges or a last round in half tiles: SwiGLU both ways bit for bit against the two-kernel
     path, residual and rotary epilogues against fp32 products."""
     from odysseus_transformer_amd import ops
     x, wgu = randn((T, K), 9700, dtype=BF).to(dev), randn((2 * I, K), 9701, std=0.05, dtype=BF).to(dev)

@@ -156,10 +156,11 @@ def test_products_with_few_rows(M, N, K, dev):
 
 @pytest.mark.parametrize("op", ["nt", "nn", "tn"])
 @pytest.mark.parametrize("M,N,K", [(72, 8, 8), (128, 264, 72), (136, 248, 64), (248, 256, 1000), (264, 520, 200), (1000, 1096, 2056),
-                                   (2056, 4104, 136), (4104, 5128, 72)], ids=lambda v: str(v))
+                                   (2056, 4104, 136), (4104, 5128, 72), (4360, 4104, 136)], ids=lambda v: str(v))
 def test_tile_edges(op, M, N, K, dev):
     """The tile kernel around its edges in all three extents: rows and columns on both sides of 64, 128 and 256, a partial last
-    slab of K, K cut into ranges, padded pitches whose padding is not a number, bias and accumulation."""
+    slab of K, K cut into ranges, a last round in half tiles (289 and more tiles of 256 x 256), padded pitches whose padding is
+    not a number, bias and accumulation."""
     from odysseus_transformer_amd import ops
     print(f"tile edges {op} M={M} N={N} K={K}", flush=True)
     nan = float("nan")
