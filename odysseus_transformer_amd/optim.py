@@ -1,13 +1,16 @@
 """AdamW on the gfx950 HIP library: the optimizer of the reference's training loop
-(torch.optim.AdamW(model.parameters(), lr=...), train.py:170,216) with the update of a tensor in ONE pass.
+(torch.optim.AdamW(model.parameters(), lr=...), train.py:170,216) with the update in ONE pass and a
+launch per 48 tensors.
 
 The host framework's default implementation runs the update as seven element-wise passes over every parameter
-(about 1.2 TB/s of useful traffic on this chip); `ody_adamw` reads parameter, gradient and both moments once and
+(about 1.2 TB/s of useful traffic on this chip); `ody_adamw_many` reads parameter, gradient and both moments once and
 writes parameter and moments once.  Same hyper-parameters, same state layout (`step`, `exp_avg`, `exp_avg_sq`
 per parameter, moments in the parameter's dtype), so state dicts interchange with torch.optim.AdamW; the
 arithmetic is fp32 with one rounding per stored value, where the host rounds after each of its passes.
 """
 from __future__ import annotations
+
+import ctypes
 
 import torch
 
@@ -34,6 +37,7 @@ class AdamW(torch.optim.Optimizer):
             b1, b2 = group["betas"]
             if group.get("amsgrad") or group.get("maximize") or group.get("decoupled_weight_decay", True) is False:
                 raise NotImplementedError("amsgrad, maximize and coupled (L2) weight decay are not implemented")
+            batches = {}   # (device, dtype) -> [param, grad, exp_avg, exp_avg_sq, numel, step] columns of one launch
             for p in group["params"]:
                 if p.grad is None:
                     continue
@@ -52,9 +56,17 @@ class AdamW(torch.optim.Optimizer):
                     state["step"] = torch.tensor(0.0)
                     state["exp_avg"] = torch.zeros_like(p, memory_format=torch.preserve_format)
                     state["exp_avg_sq"] = torch.zeros_like(p, memory_format=torch.preserve_format)
-                state["step"] += 1
-                _lib.call("ody_adamw", p.data_ptr(), g.data_ptr(), state["exp_avg"].data_ptr(),
-                          state["exp_avg_sq"].data_ptr(), p.numel(), float(group["lr"]), float(b1), float(b2),
-                          float(group["eps"]), float(group["weight_decay"]), int(state["step"].item()),
-                          0 if p.dtype == torch.bfloat16 else 1, torch.cuda.current_stream(p.device).cuda_stream)
+                columns = batches.setdefault((p.device, p.dtype), ([], [], [], [], [], [], [], []))
+                for column, value in zip(columns, (p.data_ptr(), g.data_ptr(), state["exp_avg"].data_ptr(),
+                                                   state["exp_avg_sq"].data_ptr(), p.numel(), int(state["step"].item()) + 1,
+                                                   state["step"], g)):
+                    column.append(value)
+            for (device, dtype), (*columns, counters, _grads) in batches.items():
+                n = len(columns[0])
+                for counter in counters:
+                    counter += 1
+                tables = [(ctypes.c_int64 * n)(*c) for c in columns]
+                _lib.call("ody_adamw_many", *tables, n, float(group["lr"]), float(b1), float(b2), float(group["eps"]),
+                          float(group["weight_decay"]), 0 if dtype == torch.bfloat16 else 1,
+                          torch.cuda.current_stream(device).cuda_stream)
         return loss

@@ -70,3 +70,26 @@ def test_adamw_refuses_what_it_cannot_do(dev):
         AdamW([p]).step()                                  # a CPU parameter: there is no CPU path
     q = torch.nn.Parameter(torch.zeros(8, device=dev))
     AdamW([q]).step()                                      # no gradient yet: nothing to do, no state
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_adamw_many_tensors_are_each_updated_alone(dtype, dev):
+    """More tensors than one launch takes, lengths around a vector and a block's chunk, steps that differ: bit for bit what each
+    tensor gets in a call of its own."""
+    from odysseus_transformer_amd.optim import AdamW
+    g = torch.Generator().manual_seed(3)
+    sizes = [1, 7, 8, 9, 2047, 4096, 4097, 8191, 8192, 8200, 70001] * 5
+    init = [torch.randn(n, generator=g).to(dtype) for n in sizes]
+    grads = [[torch.randn(n, generator=g).to(dtype).to(dev) for n in sizes] for _ in range(2)]
+    together, alone = ([torch.nn.Parameter(t.to(dev)) for t in init] for _ in range(2))
+    one, each = AdamW(together, **HP), [AdamW([p], **HP) for p in alone]
+    for s in range(2):
+        for k, (a, b) in enumerate(zip(together, alone)):
+            a.grad = b.grad = grads[s][k] if s or k % 3 else None    # every third tensor starts a step late
+        one.step()
+        for o in each:
+            o.step()
+    for k, (a, b, o) in enumerate(zip(together, alone, each)):
+        assert torch.equal(a, b), k
+        for name in ("exp_avg", "exp_avg_sq", "step"):
+            assert torch.equal(one.state[a][name], o.state[b][name]), (k, name)
