@@ -310,9 +310,8 @@ __global__ __launch_bounds__(256 * GROUPS, 4) void attn_fwd_hd64_kernel(const At
 }
 
 // ---------------------------------------------------------------------------------------------------------- backward
-// Per query row, [-lse / scale | -delta] in fp32, rows padded to whole tiles: what S and dP start from in the dK/dV kernel.  Rows
-// that must give P = 0 (padding, or a query that saw no key) hold -1e30.  8 lanes per row.
-__global__ __launch_bounds__(256) void attn_bwd_hd64_rows_kernel(const AttnParams p, float* __restrict__ stats, int rows) {
+// -delta of every query row, (B, Hq, Lq) in fp32: what dP starts from.  8 lanes per row.
+__global__ __launch_bounds__(256) void attn_bwd_hd64_rows_kernel(const AttnParams p, float* __restrict__ neg_delta) {
   const int lane8 = threadIdx.x & 7, qi = blockIdx.x * 32 + (threadIdx.x >> 3), h = blockIdx.y, b = blockIdx.z;
   float acc = 0.f;
   if (qi < p.Lq) {
@@ -323,19 +322,19 @@ __global__ __launch_bounds__(256) void attn_bwd_hd64_rows_kernel(const AttnParam
   }
 #pragma unroll
   for (int sft = 4; sft > 0; sft >>= 1) acc += __shfl_xor(acc, sft, 64);
-  if (lane8 != 0) return;
-  const int64_t head = (int64_t)b * p.Hq + h;
-  const float l = qi < p.Lq ? p.lse[head * p.Lq + qi] : INFINITY;
-  stats[head * rows + qi] = (l == INFINITY || l == -INFINITY) ? -1e30f : -l / p.scale;
-  stats[((int64_t)p.B * p.Hq + head) * rows + qi] = -acc;
+  if (lane8 == 0 && qi < p.Lq) neg_delta[((int64_t)b * p.Hq + h) * p.Lq + qi] = -acc;
 }
 
 //   S = Q K^T - lse / scale     dP = dO V^T - delta     dV^T += dO^T P     dK^T += Q^T (P o dP)      lane = key column
 //
+// S starts from -lse / scale of its rows, which the first wavefront of a group forms from lse once per tile: a register load beside
+// the tile's direct loads, written to the tile's stage after the products of the tile before it.  (Kept in memory by the kernel
+// above they would double the workspace that a caller holds, for the same time.)
+//
 // PART: the block takes ONE query head and leaves fp32 sums in part [dK | dV][B][Hq][Lk][D], which the kernel below adds over the
 // heads of a group; otherwise it walks all query heads of its kv head.
 template <int GROUPS, bool PART>
-__global__ __launch_bounds__(256 * GROUPS, GROUPS == 1 ? 3 : 2) void attn_bwd_hd64_dkdv_kernel(const AttnParams p, const float* __restrict__ stats, int rows,
+__global__ __launch_bounds__(256 * GROUPS, GROUPS == 1 ? 3 : 2) void attn_bwd_hd64_dkdv_kernel(const AttnParams p, const float* __restrict__ neg_delta,
                                                                             float* __restrict__ part) {
   constexpr size_t STAGE_BYTES = QS_STAGE * sizeof(bf16);
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
@@ -353,17 +352,30 @@ __global__ __launch_bounds__(256 * GROUPS, GROUPS == 1 ? 3 : 2) void attn_bwd_hd
   TileLoader lq, lo;
   lq.init(p.sq.l, w4, lane);
   lo.init(p.sdo.l, w4, lane);
+  float l_next = INFINITY;   // first wavefront of a group: lse of row `lane` of the tile on its way
   auto load = [&](int it, int buf) {
     const int h = h_first + it / ntq, t = t_end - 1 - it % ntq;
+    const int64_t head = ((int64_t)b * p.Hq + h) * p.Lq;
+    if (w4 == 0) {
+      l_next = INFINITY;
+      if (t * ROWS + lane < p.Lq) l_next = p.lse[head + t * ROWS + lane];
+    }
     bf16* st = ring + buf * QS_STAGE;
     lq.load(st, static_cast<const bf16*>(p.q) + b * p.sq.b + h * p.sq.h, t * ROWS, p.Lq, w4);
     lo.load(st + TILE, static_cast<const bf16*>(p.dout) + b * p.sdo.b + h * p.sdo.h, t * ROWS, p.Lq, w4);
-    if (w4 < 2) {
-      const float* src = stats + ((int64_t)w4 * p.B * p.Hq + (int64_t)b * p.Hq + h) * rows + t * ROWS + lane;
-      __builtin_amdgcn_global_load_lds((global_ptr)src, (lds_ptr)(st + 2 * TILE + w4 * 2 * ROWS), 4, 0, 0);
+    if (w4 == 1) {   // rows past the end repeat the last one: their P is 0
+      const float* src = neg_delta + head + min(t * ROWS + lane, p.Lq - 1);
+      __builtin_amdgcn_global_load_lds((global_ptr)src, (lds_ptr)(st + 2 * TILE + 2 * ROWS), 4, 0, 0);
     }
   };
+  // -1e30 for rows that must give P = 0: past the end, or a query that saw no key
+  auto put_lse = [&](int buf) {
+    if (w4 != 0) return;
+    const bool none = l_next == INFINITY || l_next == -INFINITY;
+    reinterpret_cast<float*>(ring + buf * QS_STAGE + 2 * TILE)[lane] = none ? -1e30f : -l_next / p.scale;
+  };
   if (grp < total) load(grp, 0);
+  put_lse(0);
 
   bf16x8 kf[KS], vf[KS];
   load_rows(kf, static_cast<const bf16*>(p.k) + b * p.sk.b + hk * p.sk.h, p.sk.l, key, p.Lk, g);
@@ -430,6 +442,7 @@ __global__ __launch_bounds__(256 * GROUPS, GROUPS == 1 ? 3 : 2) void attn_bwd_hd
     };
     sub_tile(std::integral_constant<int, 0>{});
     sub_tile(std::integral_constant<int, 1>{});
+    put_lse((n + 1) & 1);
     rd.move((n & 1) ? -(int)STAGE_BYTES : (int)STAGE_BYTES);
   }
 
@@ -490,8 +503,8 @@ __global__ __launch_bounds__(256) void attn_bwd_hd64_sum_kernel(const AttnParams
 
 //   S^T = K Q^T     dP^T = V dO^T - delta     dQ^T += K^T dS^T       lane = query column
 template <int GROUPS>
-__global__ __launch_bounds__(256 * GROUPS, GROUPS == 1 ? 3 : 2) void attn_bwd_hd64_dq_kernel(const AttnParams p, const float* __restrict__ stats,
-                                                                                           int rows) {
+__global__ __launch_bounds__(256 * GROUPS, GROUPS == 1 ? 3 : 2) void attn_bwd_hd64_dq_kernel(const AttnParams p,
+                                                                                           const float* __restrict__ neg_delta) {
   constexpr size_t STAGE_BYTES = KV_STAGE * sizeof(bf16);
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, g = lane >> 5, i = lane & 31;
@@ -523,7 +536,7 @@ __global__ __launch_bounds__(256 * GROUPS, GROUPS == 1 ? 3 : 2) void attn_bwd_hd
   float lse2 = qi < p.Lq ? p.lse[head * p.Lq + qi] : INFINITY;
   if (lse2 == -INFINITY) lse2 = INFINITY;   // a query that saw no key: P = 0
   lse2 *= ODY_LOG2E;
-  const float nd = qi < p.Lq ? stats[((int64_t)p.B * p.Hq + head) * rows + qi] : 0.f;
+  const float nd = qi < p.Lq ? neg_delta[head * p.Lq + qi] : 0.f;
   f32x16 start;   // dP starts from -delta: one add less per element
 #pragma unroll
   for (int r = 0; r < 16; r++) start[r] = nd;
@@ -615,8 +628,7 @@ __global__ __launch_bounds__(256 * GROUPS, GROUPS == 1 ? 3 : 2) void attn_bwd_hd
 }
 
 inline size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
-inline int padded_rows(int Lq) { return (Lq + ROWS - 1) / ROWS * ROWS; }
-inline size_t stats_bytes(int B, int Lq, int Hq) { return align256((size_t)2 * B * Hq * padded_rows(Lq) * sizeof(float)); }
+inline size_t delta_bytes(int B, int Lq, int Hq) { return align256((size_t)B * Hq * Lq * sizeof(float)); }
 inline int64_t row_blocks(int B, int L, int H) { return (int64_t)B * H * ((L + BLOCK_ROWS - 1) / BLOCK_ROWS); }
 
 // Fewer blocks than this leave SIMDs with one wavefront: two groups per block.  (More groups per block for all calls, which evens
@@ -641,23 +653,22 @@ int ody_launch_attn_fwd_hd64(const AttnParams& p, hipStream_t st) {
                              : launch("attn_fwd_hd64", &attn_fwd_hd64_kernel<1>, blocks, 1, KV_STAGE, st, p);
 }
 
-// [row values | fp32 dK / dV of every query head]
+// [-delta | fp32 dK / dV of every query head]
 size_t ody_attn_bwd_hd64_workspace(int B, int Lq, int Lk, int Hq, int Hkv) {
-  return stats_bytes(B, Lq, Hq) + (split_heads(B, Lk, Hq, Hkv) ? align256((size_t)2 * B * Hq * Lk * D * sizeof(float)) : 0);
+  return delta_bytes(B, Lq, Hq) + (split_heads(B, Lk, Hq, Hkv) ? align256((size_t)2 * B * Hq * Lk * D * sizeof(float)) : 0);
 }
 
 int ody_launch_attn_bwd_hd64(const AttnParams& p, void* workspace, hipStream_t st) {
-  float* stats = static_cast<float*>(workspace);
-  float* part = reinterpret_cast<float*>(static_cast<char*>(workspace) + stats_bytes(p.B, p.Lq, p.Hq));
-  const int rows = padded_rows(p.Lq);
+  float* neg_delta = static_cast<float*>(workspace);
+  float* part = reinterpret_cast<float*>(static_cast<char*>(workspace) + delta_bytes(p.B, p.Lq, p.Hq));
   int rc;
   if (!p.reuse_query_side) {
-    ODY_LAUNCH("attn_bwd_hd64_rows", st, attn_bwd_hd64_rows_kernel, dim3(rows / 32, p.Hq, p.B), dim3(256), 0, p, stats, rows);
+    ODY_LAUNCH("attn_bwd_hd64_rows", st, attn_bwd_hd64_rows_kernel, dim3((p.Lq + 31) / 32, p.Hq, p.B), dim3(256), 0, p, neg_delta);
     if ((rc = ody_check_launch("attn_bwd_hd64_rows"))) return rc;
   }
   const bool heads = split_heads(p.B, p.Lk, p.Hq, p.Hkv);
   const int64_t nkv = row_blocks(p.B, p.Lk, heads ? p.Hq : p.Hkv), nq = row_blocks(p.B, p.Lq, p.Hq);
-  auto dkdv = [&](auto kern, int groups) { return launch("attn_bwd_hd64_dkdv", kern, nkv, groups, QS_STAGE, st, p, stats, rows, part); };
+  auto dkdv = [&](auto kern, int groups) { return launch("attn_bwd_hd64_dkdv", kern, nkv, groups, QS_STAGE, st, p, neg_delta, part); };
   if (nkv < FEW_BLOCKS) rc = heads ? dkdv(&attn_bwd_hd64_dkdv_kernel<2, true>, 2) : dkdv(&attn_bwd_hd64_dkdv_kernel<2, false>, 2);
   else rc = heads ? dkdv(&attn_bwd_hd64_dkdv_kernel<1, true>, 1) : dkdv(&attn_bwd_hd64_dkdv_kernel<1, false>, 1);
   if (rc) return rc;
@@ -666,6 +677,6 @@ int ody_launch_attn_bwd_hd64(const AttnParams& p, void* workspace, hipStream_t s
     ODY_LAUNCH("attn_bwd_hd64_sum", st, attn_bwd_hd64_sum_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, p, part);
     if ((rc = ody_check_launch("attn_bwd_hd64_sum"))) return rc;
   }
-  return nq < FEW_BLOCKS ? launch("attn_bwd_hd64_dq", &attn_bwd_hd64_dq_kernel<2>, nq, 2, KV_STAGE, st, p, stats, rows)
-                         : launch("attn_bwd_hd64_dq", &attn_bwd_hd64_dq_kernel<1>, nq, 1, KV_STAGE, st, p, stats, rows);
+  return nq < FEW_BLOCKS ? launch("attn_bwd_hd64_dq", &attn_bwd_hd64_dq_kernel<2>, nq, 2, KV_STAGE, st, p, neg_delta)
+                         : launch("attn_bwd_hd64_dq", &attn_bwd_hd64_dq_kernel<1>, nq, 1, KV_STAGE, st, p, neg_delta);
 }
