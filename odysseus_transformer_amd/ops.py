@@ -58,9 +58,11 @@ _NO_CONTEXT = _NoContext()
 
 
 def run_function(fn, *args):
-    """fn.apply(*args), or fn's forward alone under no_grad / inference mode: an inference step is a handful of small launches,
-    and the autograd machinery around each costs more host time (8-10 us) than the launch itself."""
-    if torch.is_grad_enabled():
+    """fn.apply(*args), or fn's forward alone where nothing looks at the call: under no_grad / inference mode an inference step is
+    a handful of small launches, and the autograd machinery around each costs more host time (8-10 us) than the launch itself.
+    Forward-mode differentiation, function transforms and tracing go on under no_grad and see the call only through apply."""
+    if (torch.is_grad_enabled() or torch.autograd.forward_ad._current_level >= 0 or torch._C._are_functorch_transforms_active()
+            or torch._C._get_tracing_state() is not None):
         return fn.apply(*args)
     return fn.forward(_NO_CONTEXT, *args)
 

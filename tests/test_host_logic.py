@@ -423,3 +423,35 @@ def test_general_attention_path_gathers_and_scatters_like_the_host(monkeypatch):
     y = m._attend_general(q1, k1, v1, mask3, cache, torch.tensor([L + 6]), scale)
     assert seen[-1] == (1, L + 7 - 8)
     torch.testing.assert_close(y.double(), dense(q1, torch.cat([k_all, k1], 1), torch.cat([v_all, v1], 1), mask3), atol=1e-5, rtol=1e-5)
+
+
+def test_functions_are_seen_by_forward_mode_transforms_and_tracing_without_grad():
+    """The short cut past an autograd function under no_grad must not drop a tangent, a transform's rule or a traced call."""
+    from odysseus_transformer_amd import ops
+    seen = []
+
+    class Fn:
+        @staticmethod
+        def apply(x):
+            seen.append("apply")
+            return x * 2
+
+        @staticmethod
+        def forward(ctx, x):
+            seen.append("forward")
+            return x * 2
+
+    x = torch.randn(4)
+    call = lambda v: ops.run_function(Fn, v)  # noqa: E731
+    call(x)
+    with torch.no_grad():
+        call(x)
+        with torch.autograd.forward_ad.dual_level():
+            call(torch.autograd.forward_ad.make_dual(x, x))
+        torch.func.jvp(call, (x,), (x,))
+        torch.func.vmap(call)(x)
+        torch.jit.trace(call, (x,), check_trace=False)
+        call(x)
+    with torch.inference_mode():
+        call(x)
+    assert seen == ["apply", "forward", "apply", "apply", "apply", "apply", "forward", "forward"]
