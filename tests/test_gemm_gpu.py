@@ -205,3 +205,26 @@ def test_fp32_ranges_of_k(op, M, N, K, dev):
     bias, out = randn((N,), 48).to(dev), torch.ones((M, N), device=dev)
     assert rel_err(ops.gemm(code, a, b), ref) <= 1e-5
     assert rel_err(ops.gemm(code, a, b, bias=bias, out=out, accumulate=True), ref + bias.double() + 1.0) <= 1e-5
+
+
+@pytest.mark.parametrize("op", ["nt", "nn", "tn"])
+@pytest.mark.parametrize("K", [4, 32, 36, 64, 68, 96, 100, 132, 160])
+@pytest.mark.parametrize("M,N", [(64, 64), (68, 132), (2052, 4100)], ids=lambda v: str(v))
+def test_fp32_slab_pipeline(op, M, N, K, dev):
+    """One to five slabs of 32 k, whole and ragged, through 64 and 128 wide tiles, inside buffers whose other elements are NaN: each
+    element within the bound of a sum of K products in fp32, (K + 2) 2^-24 sum |a| |b|."""
+    from odysseus_transformer_amd import ops
+    print(f"op={op} M={M} N={N} K={K}", flush=True)
+    a, b = randn((M, K), 11), randn((N, K), 12)
+
+    def inside(t):
+        big = torch.full((t.shape[0] + 8, t.shape[1] + 8), float("nan"), device=dev)
+        big[4:4 + t.shape[0], 4:4 + t.shape[1]] = t.to(dev)
+        return big[4:4 + t.shape[0], 4:4 + t.shape[1]]
+
+    ag = inside(a.t() if op == "tn" else a)
+    bg = inside(b if op == "nt" else b.t())
+    got = ops.gemm({"nt": ops.GEMM_NT, "nn": ops.GEMM_NN, "tn": ops.GEMM_TN}[op], ag, bg)
+    ad, bd = a.double().to(dev), b.double().to(dev)
+    want, bound = ad @ bd.t(), (K + 2) * 2.0 ** -24 * (ad.abs() @ bd.abs().t())
+    assert ((got.double() - want).abs() <= bound).all()
