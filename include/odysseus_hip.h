@@ -230,6 +230,12 @@ int ody_linear_residual_ws(const void* x, const void* w, const void* residual, v
                            size_t workspace_bytes, void* stream);
 int ody_linear_swiglu(const void* x, const void* w_gate_up, void* gate_up, void* h, int T, int I, int K,
                       int64_t ldx, int64_t ldw, int64_t ld_gu, int64_t ld_h, int dtype, void* stream);
+/* h alone, for a caller that has no backward pass to keep gate_up for: the product never leaves the kernel.  bf16 in sizes and
+ * alignments that the one-kernel path takes (16-byte aligned rows, K % 8 == 0, and I % 128 == 0 or few rows with I % 16 == 0);
+ * ody_linear_swiglu_h_fused says whether it does (1 or 0), otherwise ODY_ERR_UNSUPPORTED. */
+int ody_linear_swiglu_h_fused(const void* x, const void* w_gate_up, int T, int I, int K, int64_t ldx, int64_t ldw, int dtype);
+int ody_linear_swiglu_h(const void* x, const void* w_gate_up, void* h, int T, int I, int K, int64_t ldx, int64_t ldw, int64_t ld_h,
+                        int dtype, void* stream);
 size_t ody_linear_dgrad_swiglu_workspace_bytes(int T, int I, int K, int dtype);
 int ody_linear_dgrad_swiglu(const void* dy, const void* w_down, const void* gate_up, void* d_gate_up, int T, int I,
                             int K, int64_t ld_dy, int64_t ldw, int64_t ld_gu, int64_t ld_dgu, int dtype,

@@ -38,6 +38,8 @@ SIGNATURES = {
     "ody_linear_residual": (_i, [_p] * 4 + [_i] * 3 + [_i64] * 4 + [_i, _p]),
     "ody_linear_residual_ws": (_i, [_p] * 4 + [_i] * 3 + [_i64] * 4 + [_i, _p, _sz, _p]),
     "ody_linear_swiglu": (_i, [_p] * 4 + [_i] * 3 + [_i64] * 4 + [_i, _p]),
+    "ody_linear_swiglu_h_fused": (_i, [_p] * 2 + [_i] * 3 + [_i64] * 2 + [_i]),
+    "ody_linear_swiglu_h": (_i, [_p] * 3 + [_i] * 3 + [_i64] * 3 + [_i, _p]),
     "ody_linear_dgrad_swiglu_workspace_bytes": (_sz, [_i] * 4),
     "ody_linear_dgrad_swiglu": (_i, [_p] * 4 + [_i] * 3 + [_i64] * 4 + [_i, _p, _sz, _p]),
     "ody_swiglu_fwd": (_i, [_p, _p, _i, _i, _i64, _i64, _i, _p]),

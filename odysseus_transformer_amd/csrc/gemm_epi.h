@@ -1,7 +1,7 @@
 // What the epilogue of a bf16 product does besides rounding and storing.
 //   EPI_RESIDUAL    C = A B + R                      (R = aux, row pitch ld_aux; one rounding, after the add)
-//   EPI_SWIGLU_FWD  NT only.  B is the packed (2 I, K) gate_up weight.  Writes gate_up to C in its usual [gate | up] layout and
-//                   h = silu(gate) * up to out2, computed from the rounded gate / up values exactly as the stand-alone SwiGLU
+//   EPI_SWIGLU_FWD  NT only.  B is the packed (2 I, K) gate_up weight.  Writes gate_up to C in its usual [gate | up] layout (C NULL:
+//                   not at all) and h = silu(gate) * up to out2, computed from the rounded gate / up values exactly as the stand-alone SwiGLU
 //                   kernel would.
 //   EPI_ROPE        NT only, head_dim 128.  Columns below I (a multiple of 128) are rotated before the one rounding: with the
 //                   cos / sin table of ody_rope_table in aux (row pitch ld_aux), column j < 64 of a head pairs with column j + 64

@@ -102,8 +102,10 @@ __global__ __launch_bounds__(64 * SK_WAVES) void gemm_skinny_kernel(const bf16* 
       const float a1 = (float)g4[e], a3 = (float)u4[e];
       h4[e] = (bf16)(a1 / (1.f + __expf(-a1)) * a3);
     }
-    *reinterpret_cast<bf16x4*>(cp + n) = g4;
-    *reinterpret_cast<bf16x4*>(cp + ep.I + n) = u4;
+    if (C) {   // NULL: only h is wanted
+      *reinterpret_cast<bf16x4*>(cp + n) = g4;
+      *reinterpret_cast<bf16x4*>(cp + ep.I + n) = u4;
+    }
     *reinterpret_cast<bf16x4*>(ep.out2 + (int64_t)row * ep.ld_out2 + n) = h4;
   } else if constexpr (EPI == EPI_ROPE) {
     const int n = row0[0] + 4 * q, j = n & 127;

@@ -400,6 +400,7 @@ __device__ __forceinline__ void gemm_tile_block(const Args& p, int m0, int tn) {
     }
 #pragma unroll
     for (int pass = 0; pass < 32 / RPP; pass++) {
+      if (EPI == EPI_SWIGLU_FWD && p.C == nullptr) break;   // only h is wanted
       const int row = pass * RPP + lane / CPR, ch = lane % CPR, m = mw + 32 * a2 + row;
       const bf16x8 v = *reinterpret_cast<const bf16x8*>(band + row * EP + 8 * ch);
       const int b = ch >> 1;

@@ -295,3 +295,16 @@ def test_fused_epilogues_on_ragged_rows(T, I, K, dev):
     p = plain.view(T, I // 128, 128)
     a, b = p[:, :-1].split(64, dim=-1)
     assert rel_err(got, torch.cat([torch.cat([a * c - b * s, b * c + a * s], -1), p[:, -1:]], 1)) <= 1e-2
+
+
+@pytest.mark.parametrize("T,I,K", [(1, 128, 72), (16, 144, 64), (17, 128, 72), (200, 384, 4096), (1000, 640, 520), (3001, 1408, 264), (4104, 4224, 72),
+                                   (40, 144, 64)])
+def test_swiglu_without_gate_up(T, I, K, dev):
+    """h alone is the h of the kernel that keeps gate_up, bit for bit: tile edges, a last round in half tiles, few rows, columns of a
+    wider buffer, and a size that has no such kernel (40, 144)."""
+    from odysseus_transformer_amd import ops
+    print(f"swiglu_h T={T} I={I} K={K}", flush=True)
+    x, w = randn((T, K + 8), 9800, dtype=BF).to(dev)[:, 8:], randn((2 * I, K), 9801, std=0.05, dtype=BF).to(dev)
+    h, names = _kernels_of(lambda: ops.linear_swiglu_h(x, w))
+    assert (len(names) == 1) == ((T, I) != (40, 144)), names
+    assert torch.equal(h, ops.linear_swiglu(x, w)[1])
