@@ -439,13 +439,10 @@ def linear_residual(x, weight, residual):
 _ROPE_TABLE_LAST = None   # (position tensor, its version, rows, head_dim, base, device, stream, table) of the last table built
 
 
-def _tensor_version(t) -> int:
-    """The autograd version counter of `t`; inference tensors (torch.inference_mode) have none and cannot be
-    modified in place outside that mode: -1."""
-    try:
-        return t._version
-    except RuntimeError:
-        return -1
+def _tensor_version(t) -> Optional[int]:
+    """The autograd version counter of `t`, which counts its modifications in place; None for a tensor made under
+    torch.inference_mode(): it has no counter, although that mode may modify it."""
+    return None if t.is_inference() else t._version
 
 
 def rope_table(position_ids, rows: int, head_dim: int, base: float = 10000.0, device=None, inv_freq=None) -> torch.Tensor:
@@ -454,7 +451,8 @@ def rope_table(position_ids, rows: int, head_dim: int, base: float = 10000.0, de
     elements, one sequence that every batch entry shares, e.g. (1, L) for (B, L) rows -- or None for arange.
 
     The layers of a model are handed one and the same position tensor: the last table is kept and returned again
-    for the same tensor object (unmodified since), shape, base and stream.  Treat the result as read-only."""
+    for the same tensor object (unmodified since), shape, base and stream.  A tensor that cannot say whether it was
+    modified (made under torch.inference_mode()) gets a new table every time.  Treat the result as read-only."""
     global _ROPE_TABLE_LAST
     pos_arg = position_ids
     if position_ids is not None:
@@ -463,9 +461,11 @@ def rope_table(position_ids, rows: int, head_dim: int, base: float = 10000.0, de
     if device is None:
         raise ValueError("rope_table needs position_ids or a device")
     device = torch.device(device)
-    key = (None if pos_arg is None else _tensor_version(pos_arg), rows, head_dim, float(base), str(device), _stream())
+    version = 0 if pos_arg is None else _tensor_version(pos_arg)
+    keep = inv_freq is None and version is not None
+    key = (version, rows, head_dim, float(base), str(device), _stream())
     last = _ROPE_TABLE_LAST
-    if inv_freq is None and last is not None and last[0] is pos_arg and last[1] == key:
+    if keep and last is not None and last[0] is pos_arg and last[1] == key:
         return last[2]
     if position_ids is not None:
         position_ids = position_ids.to(torch.int64).reshape(-1)
@@ -475,7 +475,6 @@ def rope_table(position_ids, rows: int, head_dim: int, base: float = 10000.0, de
                 raise ValueError(f"{n} positions for {rows} rows")
             position_ids = position_ids.repeat(rows // n)     # one sequence shared by the batch
         position_ids = position_ids.contiguous()
-    custom_freq = inv_freq is not None
     if inv_freq is None:
         inv_freq = rope_inv_freq(head_dim, base, device)
     if inv_freq.dtype != torch.float32 or inv_freq.numel() != head_dim // 2 or not inv_freq.is_contiguous():
@@ -483,7 +482,7 @@ def rope_table(position_ids, rows: int, head_dim: int, base: float = 10000.0, de
     table = torch.empty((rows, head_dim), dtype=torch.bfloat16, device=device)
     _lib.call("ody_rope_table", position_ids.data_ptr() if position_ids is not None else 0, inv_freq.data_ptr(), rows,
               head_dim, float(base), table.data_ptr(), _stream())
-    if not custom_freq:
+    if keep:
         _ROPE_TABLE_LAST = (pos_arg, key, table)   # holding pos_arg keeps its identity from being reused
     return table
 

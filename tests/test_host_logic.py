@@ -455,3 +455,42 @@ def test_functions_are_seen_by_forward_mode_transforms_and_tracing_without_grad(
     with torch.inference_mode():
         call(x)
     assert seen == ["apply", "forward", "apply", "apply", "apply", "apply", "forward", "forward"]
+
+
+@pytest.fixture
+def fake_rope_kernel(monkeypatch):
+    """rope_table on CPU tensors, its kernel replaced by one that writes each row's position; yields the list of the positions of
+    every table that was built."""
+    import ctypes
+    from odysseus_transformer_amd import _lib, ops
+    built = []
+
+    def call(name, pos, _freq, rows, dim, _base, table, _stream):
+        assert name == "ody_rope_table"
+        p = list((ctypes.c_int64 * rows).from_address(pos))
+        built.append(p)
+        vals = torch.tensor(p, dtype=torch.bfloat16).repeat_interleave(dim)
+        ctypes.memmove(table, vals.data_ptr(), 2 * rows * dim)
+
+    monkeypatch.setattr(_lib, "call", call)
+    monkeypatch.setattr(ops, "_need_gpu", lambda *t: None)
+    monkeypatch.setattr(ops, "_stream", lambda: 0)
+    monkeypatch.setattr(ops, "_ROPE_TABLE_LAST", None)
+    return built
+
+
+def test_rope_table_of_a_position_tensor_advanced_under_inference_mode(fake_rope_kernel):
+    """Tensors made under inference_mode have no version counter, yet that mode modifies them: no table is reused for them."""
+    from odysseus_transformer_amd import ops
+    with torch.inference_mode():
+        pos = torch.tensor([[5]])
+        assert ops.rope_table(pos, 1, 128)[0, 0] == 5
+        pos += 1
+        assert ops.rope_table(pos, 1, 128)[0, 0] == 6
+        normal = ops.rope_table(pos.clone(), 1, 128)
+    pos = torch.tensor([[5]])        # a counter: one table while the positions stay, another behind a change
+    t = ops.rope_table(pos, 1, 128)
+    assert ops.rope_table(pos, 1, 128) is t and t is not normal
+    with torch.inference_mode():
+        pos += 1
+        assert ops.rope_table(pos, 1, 128)[0, 0] == 6
