@@ -454,20 +454,27 @@ def rope_table(position_ids, rows: int, head_dim: int, base: float = 10000.0, de
     for the same tensor object (unmodified since), shape, base and stream.  A tensor that cannot say whether it was
     modified (made under torch.inference_mode()) gets a new table every time.  Treat the result as read-only."""
     global _ROPE_TABLE_LAST
-    pos_arg = position_ids
     if position_ids is not None:
-        _need_gpu(position_ids)
         device = position_ids.device
     if device is None:
         raise ValueError("rope_table needs position_ids or a device")
     device = torch.device(device)
-    version = 0 if pos_arg is None else _tensor_version(pos_arg)
-    keep = inv_freq is None and version is not None
+    version = 0 if position_ids is None else _tensor_version(position_ids)
+    if inv_freq is not None or version is None:
+        return _new_rope_table(position_ids, rows, head_dim, base, device, inv_freq)
     key = (version, rows, head_dim, float(base), str(device), _stream())
     last = _ROPE_TABLE_LAST
-    if keep and last is not None and last[0] is pos_arg and last[1] == key:
+    if last is not None and last[0] is position_ids and last[1] == key:
         return last[2]
+    table = _new_rope_table(position_ids, rows, head_dim, base, device)
+    _ROPE_TABLE_LAST = (position_ids, key, table)   # holding position_ids keeps its identity from being reused
+    return table
+
+
+def _new_rope_table(position_ids, rows: int, head_dim: int, base: float, device, inv_freq=None) -> torch.Tensor:
+    """rope_table from the positions as they are now."""
     if position_ids is not None:
+        _need_gpu(position_ids)
         position_ids = position_ids.to(torch.int64).reshape(-1)
         n = position_ids.numel()
         if n != rows:
@@ -482,8 +489,6 @@ def rope_table(position_ids, rows: int, head_dim: int, base: float = 10000.0, de
     table = torch.empty((rows, head_dim), dtype=torch.bfloat16, device=device)
     _lib.call("ody_rope_table", position_ids.data_ptr() if position_ids is not None else 0, inv_freq.data_ptr(), rows,
               head_dim, float(base), table.data_ptr(), _stream())
-    if keep:
-        _ROPE_TABLE_LAST = (pos_arg, key, table)   # holding pos_arg keeps its identity from being reused
     return table
 
 
@@ -998,7 +1003,8 @@ class LinearRoPEFunc(torch.autograd.Function):
         B, L, K = x.shape
         x2 = x.reshape(B * L, K)
         x2 = x2 if x2.stride(1) == 1 else x2.contiguous()
-        table = rope_table(position_ids, B * L, head_dim, rope_base, device=x.device)
+        # evaluated on every call, as rope_ does: behind a cache the positions are new with every token
+        table = _new_rope_table(position_ids, B * L, head_dim, rope_base, x.device)
         ctx.save_for_backward(x2, weight, position_ids)
         ctx.dims = (n_rot, rope_base, x.shape)
         return linear_rope(x2, weight, table, n_rot, head_dim).view(B, L, -1, head_dim)

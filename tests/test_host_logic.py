@@ -494,3 +494,16 @@ def test_rope_table_of_a_position_tensor_advanced_under_inference_mode(fake_rope
     with torch.inference_mode():
         pos += 1
         assert ops.rope_table(pos, 1, 128)[0, 0] == 6
+
+
+def test_cached_path_evaluates_its_positions_on_every_call(fake_rope_kernel, monkeypatch):
+    """The projection behind a KV cache rotates by the positions as they are, whoever wrote them: no table outlives a call."""
+    from odysseus_transformer_amd import ops
+    monkeypatch.setattr(ops, "linear_rope", lambda x, w, table, n_rot, head_dim: table.clone())
+    x, pos = torch.zeros(1, 1, 128), torch.tensor([[5]])
+    project = lambda: ops.run_function(ops.LinearRoPEFunc, x, x[0], 1, 128, pos, 10000.0)[0, 0, 0, 0]  # noqa: E731
+    with torch.no_grad():
+        assert project() == 5
+        pos.data.add_(1)        # as a captured graph or another library writes it: no version counted
+        assert project() == 6
+    assert fake_rope_kernel == [[5], [6]]
