@@ -452,7 +452,9 @@ def rope_table(position_ids, rows: int, head_dim: int, base: float = 10000.0, de
 
     The layers of a model are handed one and the same position tensor: the last table is kept and returned again
     for the same tensor object (unmodified since), shape, base and stream.  A tensor that cannot say whether it was
-    modified (made under torch.inference_mode()) gets a new table every time.  Treat the result as read-only."""
+    modified (made under torch.inference_mode()) gets a new table every time, and so does a call under graph capture: a
+    replay has to read the positions again, and what a capture records has no values for later calls.  Treat the result
+    as read-only."""
     global _ROPE_TABLE_LAST
     if position_ids is not None:
         device = position_ids.device
@@ -460,7 +462,7 @@ def rope_table(position_ids, rows: int, head_dim: int, base: float = 10000.0, de
         raise ValueError("rope_table needs position_ids or a device")
     device = torch.device(device)
     version = 0 if position_ids is None else _tensor_version(position_ids)
-    if inv_freq is not None or version is None:
+    if inv_freq is not None or version is None or torch.cuda.is_current_stream_capturing():
         return _new_rope_table(position_ids, rows, head_dim, base, device, inv_freq)
     key = (version, rows, head_dim, float(base), str(device), _stream())
     last = _ROPE_TABLE_LAST

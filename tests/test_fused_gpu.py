@@ -308,3 +308,61 @@ def test_swiglu_without_gate_up(T, I, K, dev):
     h, names = _kernels_of(lambda: ops.linear_swiglu_h(x, w))
     assert (len(names) == 1) == ((T, I) != (40, 144)), names
     assert torch.equal(h, ops.linear_swiglu(x, w)[1])
+
+
+def test_rope_table_under_capture_follows_the_positions_of_each_replay(dev):
+    """Warm-up and capture on one stream, as a program with a stream of its own does; every replay against an eager table."""
+    from odysseus_transformer_amd import ops
+    pos = torch.arange(40, device=dev)[None]
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        ops.rope_table(pos, 40, 128)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=side):
+            captured = ops.rope_table(pos, 40, 128)
+        eager = ops.rope_table(pos, 40, 128)          # not the captured one: that has no values before the first replay
+        want = torch.equal(eager, ops.rope_table(pos.clone(), 40, 128))
+    torch.cuda.synchronize()
+    assert want
+    for step in (3, 500, 70000):
+        pos.add_(step)
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(captured, ops.rope_table(pos.clone(), 40, 128))
+
+
+def test_decoding_step_under_inference_mode_with_an_advancing_position_tensor(dev):
+    """Two steps through one position tensor that is advanced in place, against the same steps with tensors of their own."""
+    import types
+    from odysseus_transformer_amd.decoder.odysseus import LlamaFlashAttention2TPSP
+
+    class Cache:
+        def __init__(self):
+            self.k = self.v = None
+
+        def get_seq_length(self, layer_idx=0):
+            return 0 if self.k is None else self.k.shape[2]
+
+        def update(self, k, v, layer_idx, cache_kwargs=None):
+            self.k = k.clone() if self.k is None else torch.cat([self.k, k], 2)
+            self.v = v.clone() if self.v is None else torch.cat([self.v, v], 2)
+            return self.k, self.v
+
+    cfg = types.SimpleNamespace(hidden_size=512, num_attention_heads=4, num_key_value_heads=2, head_dim=128, attention_dropout=0.0,
+                                rope_theta=10000.0)
+    torch.manual_seed(0)
+    attn = LlamaFlashAttention2TPSP(cfg, 0).to(BF).to(dev).eval()
+    prompt, tokens = randn((1, 70, 512), 9700, dtype=BF).to(dev), randn((3, 1, 1, 512), 9701, dtype=BF).to(dev)
+    results = []
+    for in_place in (True, False):
+        with torch.inference_mode():
+            cache, pos, outs = Cache(), torch.tensor([[70]], device=dev), []
+            attn(prompt, position_ids=torch.arange(70, device=dev)[None], past_key_value=cache)
+            for n in range(3):
+                outs.append(attn(tokens[n], position_ids=pos if in_place else torch.tensor([[70 + n]], device=dev), past_key_value=cache)[0])
+                pos += 1
+            results.append((torch.cat(outs, 1), cache.k))
+    for a, b in zip(*results):
+        assert torch.equal(a, b)

@@ -507,3 +507,16 @@ def test_cached_path_evaluates_its_positions_on_every_call(fake_rope_kernel, mon
         pos.data.add_(1)        # as a captured graph or another library writes it: no version counted
         assert project() == 6
     assert fake_rope_kernel == [[5], [6]]
+
+
+def test_rope_table_neither_comes_from_nor_outlives_a_capture(fake_rope_kernel, monkeypatch):
+    """A replay must evaluate the positions of its own time, and a table that a capture recorded holds nothing yet."""
+    from odysseus_transformer_amd import ops
+    pos, capturing = torch.tensor([[5]]), [False]
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: capturing[0])
+    before = ops.rope_table(pos, 1, 128)
+    capturing[0] = True
+    captured = ops.rope_table(pos, 1, 128)
+    capturing[0] = False
+    after = ops.rope_table(pos, 1, 128)
+    assert captured is not before and after is not captured
