@@ -476,6 +476,7 @@ def fake_rope_kernel(monkeypatch):
     monkeypatch.setattr(ops, "_need_gpu", lambda *t: None)
     monkeypatch.setattr(ops, "_stream", lambda: 0)
     monkeypatch.setattr(ops, "_ROPE_TABLE_LAST", None)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
     return built
 
 
