@@ -606,6 +606,15 @@ def check_rmsnorm_args(x, weight, rstd=None, dy=None) -> None:
                              f"{tuple(rstd.shape)}, {rstd.dtype}, {rstd.device}")
 
 
+def check_position_ids(position_ids, B: int, L: int, device) -> None:
+    """Integers on `device`, one row of L positions or one per batch entry."""
+    if position_ids.dtype not in (torch.int64, torch.int32) or position_ids.device != device:
+        raise ValueError(f"rope: position_ids must be an integer tensor on {device}; got "
+                         f"{position_ids.dtype} on {position_ids.device}")
+    if position_ids.shape[-1] != L or position_ids.numel() not in (L, B * L):
+        raise ValueError(f"rope: position_ids {tuple(position_ids.shape)} do not cover (B={B}, L={L})")
+
+
 def check_rope_args(x, n_rot, position_ids, inv_freq) -> None:
     B, L, H, D = x.shape
     if not 0 <= n_rot <= H:
@@ -617,11 +626,7 @@ def check_rope_args(x, n_rot, position_ids, inv_freq) -> None:
         raise ValueError(f"rope: inv_freq must be a contiguous float32 ({D // 2},) tensor on {x.device}; got "
                          f"{tuple(inv_freq.shape)}, {inv_freq.dtype}, {inv_freq.device}")
     if position_ids is not None:
-        if position_ids.dtype not in (torch.int64, torch.int32) or position_ids.device != x.device:
-            raise ValueError(f"rope: position_ids must be an integer tensor on {x.device}; got "
-                             f"{position_ids.dtype} on {position_ids.device}")
-        if position_ids.shape[-1] != L or position_ids.numel() not in (L, B * L):
-            raise ValueError(f"rope: position_ids {tuple(position_ids.shape)} do not cover (B={B}, L={L})")
+        check_position_ids(position_ids, B, L, x.device)
 
 
 def rmsnorm_fwd(x, weight, eps: float = 1e-6):
@@ -1005,6 +1010,8 @@ class LinearRoPEFunc(torch.autograd.Function):
         B, L, K = x.shape
         x2 = x.reshape(B * L, K)
         x2 = x2 if x2.stride(1) == 1 else x2.contiguous()
+        if position_ids is not None:
+            check_position_ids(position_ids, B, L, x.device)
         # evaluated on every call, as rope_ does: behind a cache the positions are new with every token
         table = _new_rope_table(position_ids, B * L, head_dim, rope_base, x.device)
         ctx.save_for_backward(x2, weight, position_ids)

@@ -521,3 +521,15 @@ def test_rope_table_neither_comes_from_nor_outlives_a_capture(fake_rope_kernel, 
     capturing[0] = False
     after = ops.rope_table(pos, 1, 128)
     assert captured is not before and after is not captured
+
+
+@pytest.mark.parametrize("pos", [torch.tensor([[5]]), torch.arange(2)[None], torch.arange(4.0)[None], torch.arange(4)[:, None]],
+                         ids=["one for all", "half", "float", "column"])
+def test_cached_path_refuses_positions_that_do_not_cover_its_tokens(pos, fake_rope_kernel, monkeypatch):
+    """What rope_ refuses is refused here too, and not repeated over the rows or rounded."""
+    from odysseus_transformer_amd import ops
+    monkeypatch.setattr(ops, "linear_rope", lambda x, w, table, n_rot, head_dim: table.clone())
+    with torch.no_grad(), pytest.raises(ValueError):
+        ops.run_function(ops.LinearRoPEFunc, torch.zeros(1, 4, 128), torch.zeros(128, 128), 1, 128, pos, 10000.0)
+    with pytest.raises(ValueError):
+        ops.check_rope_args(torch.zeros(1, 4, 1, 128), 1, pos, None)
