@@ -322,24 +322,26 @@ def attn_bwd_workspace_bytes(q, k, keep_ds: bool = False, causal: bool = True) -
     return n
 
 
-def _shared_bwd_workspace(q, calls):
-    """One workspace for a sequence of attn_bwd calls with the same queries: `calls` is a list of (k, causal).
+def _shared_bwd_workspace(calls):
+    """One workspace for a sequence of attn_bwd calls: `calls` is a list of (q, k, causal).  It is sized by every call of the
+    sequence, for a call on fewer rows may need more: kernels that cut their work into fp32 parts do so where blocks are few.
     Returns it with the keep_ds setting of every call: on where the shape qualifies and the scratch stays within
     keep_ds_max_bytes(), all off if that much memory is not there."""
-    B, Lq, Hq, D = q.shape
     lib = _lib.load()
-    base = [lib.ody_attn_bwd_workspace_bytes(B, Lq, k.shape[1], Hq, k.shape[2], D, _dt(q)) for k, _ in calls]
-    ds = [lib.ody_attn_bwd_ds_bytes(B, Lq, k.shape[1], Hq, k.shape[2], D, _dt(q), int(c)) for k, c in calls]
-    limit = keep_ds_max_bytes(q.device)
-    failed = _KEEP_DS_OOM.get(str(q.device), 1 << 62)
+    dims = [(q.shape[0], q.shape[1], k.shape[1], q.shape[2], k.shape[2], q.shape[3], _dt(q)) for q, k, _ in calls]
+    base = [lib.ody_attn_bwd_workspace_bytes(*d) for d in dims]
+    ds = [lib.ody_attn_bwd_ds_bytes(*d, int(c)) for d, (_, _, c) in zip(dims, calls)]
+    device = calls[0][0].device
+    limit = keep_ds_max_bytes(device)
+    failed = _KEEP_DS_OOM.get(str(device), 1 << 62)
     keeps = [0 < d <= limit and d < failed for d in ds]
     if any(keeps):
         try:
             n = max(b + (d if kp else 0) for b, d, kp in zip(base, ds, keeps))
-            return torch.empty(n, dtype=torch.uint8, device=q.device), keeps
+            return torch.empty(n, dtype=torch.uint8, device=device), keeps
         except torch.OutOfMemoryError:
-            _KEEP_DS_OOM[str(q.device)] = min(failed, min(d for d, kp in zip(ds, keeps) if kp))
-    return torch.empty(max(base), dtype=torch.uint8, device=q.device), [False] * len(calls)
+            _KEEP_DS_OOM[str(device)] = min(failed, min(d for d, kp in zip(ds, keeps) if kp))
+    return torch.empty(max(base), dtype=torch.uint8, device=device), [False] * len(calls)
 
 
 def cast_from_f32(src, dtype) -> torch.Tensor:
@@ -757,7 +759,7 @@ class RingBlocksAttnFunc(torch.autograd.Function):
         # Q / dO images depend on the queries only and are built by the first block's call
         dq = torch.empty(q.shape, dtype=torch.float32, device=q.device)
         same_kv_shape = all(k.shape == ks[0].shape for k in ks)
-        ws, keeps = _shared_bwd_workspace(q, [(ks[b], b == ctx.causal_block) for b in range(nb)]) if nb else (None, [])
+        ws, keeps = _shared_bwd_workspace([(q, ks[b], b == ctx.causal_block) for b in range(nb)]) if nb else (None, [])
         dks, dvs = [], []
         for b in range(nb):
             _, dk, dv = attn_bwd(q, ks[b], vs[b], out, lse, dout, causal=(b == ctx.causal_block),
@@ -837,8 +839,8 @@ class ZigzagRingRankAttnFunc(torch.autograd.Function):
         dq = torch.empty(q.shape, dtype=torch.float32, device=q.device)
         lse_b = lse[:, :, c:].contiguous()
         steps = list(ZigzagRingRankAttnFunc._steps(ctx.rank, world))
-        # sized for the largest step (both query chunks against both key chunks); a step with fewer queries asks for less
-        ws, _ = _shared_bwd_workspace(q, [(ks[0], False)])
+        ws, keeps = _shared_bwd_workspace([(q[:, q0 * c:q1 * c], ks[s][:, k0 * c:k1 * c], causal)
+                                           for s, ((q0, q1), (k0, k1), causal) in enumerate(steps)])
         dks = [torch.empty_like(k) for k in ks]
         dvs = [torch.empty_like(v) for v in vs]
         prev = None
@@ -848,11 +850,9 @@ class ZigzagRingRankAttnFunc(torch.autograd.Function):
             if k1 == 1:   # the chunk that this step does not read; everything else is written below
                 dks[s][:, c:].zero_()
                 dvs[s][:, c:].zero_()
-            need = attn_bwd_workspace_bytes(q[:, qs], ks[s][:, kr], True, causal)
             attn_bwd(q[:, qs], ks[s][:, kr], vs[s][:, kr], out[:, qs], lse if q1 - q0 == 2 else lse_b, dout[:, qs],
                      causal=causal, scale=ctx.softmax_scale, dq=dq[:, qs], dk=dks[s][:, kr], dv=dvs[s][:, kr],
-                     accumulate_dq=(s > 0), workspace=ws, reuse_query_side=(kind == prev),
-                     keep_ds=(need is not None and need <= ws.numel()))
+                     accumulate_dq=(s > 0), workspace=ws, reuse_query_side=(kind == prev), keep_ds=keeps[s])
             prev = kind
         return (cast_from_f32(dq, q.dtype), None, None, None, *dks, *dvs)
 

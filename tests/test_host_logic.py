@@ -533,3 +533,27 @@ def test_cached_path_refuses_positions_that_do_not_cover_its_tokens(pos, fake_ro
         ops.run_function(ops.LinearRoPEFunc, torch.zeros(1, 4, 128), torch.zeros(128, 128), 1, 128, pos, 10000.0)
     with pytest.raises(ValueError):
         ops.check_rope_args(torch.zeros(1, 4, 1, 128), 1, pos, None)
+
+
+@pytest.mark.parametrize("keep_ds", [0, 1 << 40])
+@pytest.mark.parametrize("Hq,Hkv,D,c", [(32, 8, 64, 8192), (32, 8, 64, 8064), (16, 4, 64, 16384), (8, 2, 64, 32768), (4, 4, 128, 8256),
+                                        (4, 4, 128, 8192), (4, 1, 128, 512), (2, 2, 64, 96)])
+def test_zigzag_backward_workspace_has_room_for_every_step(Hq, Hkv, D, c, keep_ds, monkeypatch):
+    """Steps on fewer keys may need more scratch than the one on all of them (their kernels cut the work into fp32 parts): shapes on
+    both sides of those lines, through the real byte counts; tensors without memory, launches left out."""
+    from odysseus_transformer_amd import _lib, ops
+    calls = []
+    monkeypatch.setattr(_lib, "call", lambda name, *a: calls.append(name))
+    monkeypatch.setattr(ops, "_need_gpu", lambda *t: None)
+    monkeypatch.setattr(ops, "_stream", lambda: 0)
+    ops.set_keep_ds_max_bytes(keep_ds)
+    try:
+        for rank in range(3):
+            t = lambda h: torch.empty((1, 2 * c, h, D), dtype=torch.bfloat16, device="meta", requires_grad=True)  # noqa: E731
+            q, ks, vs = t(Hq), [t(Hkv) for _ in range(3)], [t(Hkv) for _ in range(3)]
+            out, _ = ops.zigzag_ring_rank_attn(q, ks, vs, rank, 3)
+            out.backward(torch.empty_like(out))
+            assert q.grad.shape == q.shape and ks[2].grad.shape == ks[2].shape
+    finally:
+        ops.set_keep_ds_max_bytes(None)
+    assert calls.count("ody_attn_bwd") == 9

@@ -35,7 +35,9 @@ def _scatter_add(full, local, rank, world, dim=1):
 
 
 @pytest.mark.parametrize("world,c,Hq,Hkv,D,dtype", [(4, 96, 4, 2, 128, torch.bfloat16), (2, 160, 2, 2, 128, torch.bfloat16),
-                                                   (3, 64, 4, 4, 64, torch.float32)])
+                                                   (3, 64, 4, 4, 64, torch.float32), (4, 96, 4, 2, 64, torch.bfloat16),
+                                                   # a block of 256 keys: one scratch part per kv head; half of it: one per query head
+                                                   (2, 128, 1024, 512, 64, torch.bfloat16)])
 def test_zigzag_ranks_assemble_to_full_causal_attention(world, c, Hq, Hkv, D, dtype, dev):
     from odysseus_transformer_amd import ops
     L = 2 * world * c
