@@ -29,6 +29,7 @@ SIGNATURES = {
     "ody_attn_fwd": (_i, [_p] * 5 + [_i] * 6 + [_i64] * 12 + [_f, _i, _i, _p, _sz, _p]),
     "ody_attn_fwd_noalloc": (_i, [_p] * 5 + [_i] * 6 + [_i64] * 12 + [_f, _i, _i, _p]),
     "ody_attn_bwd_workspace_bytes": (_sz, [_i] * 7),
+    "ody_attn_bwd_workspace_least_bytes": (_sz, [_i] * 7),
     "ody_attn_bwd_ds_bytes": (_sz, [_i] * 8),
     "ody_attn_bwd": (_i, [_p] * 9 + [_i] * 6 + [_i64] * 24 + [_f, _i, _i, _i, _p, _sz, _p]),
     "ody_cast_from_f32": (_i, [_p, _p, _i64, _i, _p]),

@@ -196,6 +196,11 @@ extern "C" size_t ody_attn_bwd_workspace_bytes(int B, int Lq, int Lk, int Hq, in
   return n;
 }
 
+extern "C" size_t ody_attn_bwd_workspace_least_bytes(int B, int Lq, int Lk, int Hq, int Hkv, int D, int dtype) {
+  if (B <= 0 || Lq <= 0 || Lk <= 0 || Hq <= 0 || Hkv <= 0) return 0;
+  return dtype == ODY_BF16 && D == 128 ? ody_attn_bwd_workspace_bytes(B, Lq, Lk, Hq, Hkv, D, dtype) : delta_bytes(B, Lq, Hq);
+}
+
 extern "C" size_t ody_attn_bwd_ds_bytes(int B, int Lq, int Lk, int Hq, int Hkv, int D, int dtype, int causal) {
   if (B <= 0 || Lq <= 0 || Lk <= 0 || Hq <= 0 || Hkv <= 0 || dtype != ODY_BF16 || D != 128) return 0;
   return (ody_attn_bwd_pipe_ds_bytes(B, Lq, Lk, Hq, causal) + 255) & ~(size_t)255;
@@ -254,8 +259,8 @@ int attn_bwd_impl(const char* who, const void* rope_q, const void* rope_k,
     ODY_REQUIRE(ws_ds > 0, ODY_ERR_UNSUPPORTED,
                 "%s: ODY_BWD_KEEP_DS needs bf16, head_dim 128, Lq and Lk multiples of 256 and, if causal, Lq == Lk", who);
   }
-  ODY_REQUIRE(workspace_bytes >= ws_base + ws_ds, ODY_ERR_WORKSPACE, "%s: workspace of %zu bytes, %zu needed", who,
-              workspace_bytes, ws_base + ws_ds);
+  const size_t ws_least = ody_attn_bwd_workspace_least_bytes(B, Lq, Lk, Hq, Hkv, D, dtype) + ws_ds;
+  ODY_REQUIRE(workspace_bytes >= ws_least, ODY_ERR_WORKSPACE, "%s: workspace of %zu bytes, %zu needed", who, workspace_bytes, ws_least);
   ODY_REQUIRE((reinterpret_cast<uintptr_t>(workspace) & 255u) == 0, ODY_ERR_MISALIGNED,
               "%s: workspace must be 256-byte aligned", who);
   if (rope_q || rope_k) {
@@ -272,7 +277,7 @@ int attn_bwd_impl(const char* who, const void* rope_q, const void* rope_k,
   hipStream_t st = static_cast<hipStream_t>(stream);
   if (dtype == ODY_BF16 && D == 128 && p.drop_thresh == 0)   // its query-side pre-pass computes delta as well
     return ody_launch_attn_bwd_pipe(p, static_cast<char*>(workspace) + delta_bytes(B, Lq, Hq), st);
-  if (dtype == ODY_BF16 && p.drop_thresh == 0) return ody_launch_attn_bwd_hd64(p, workspace, st);
+  if (dtype == ODY_BF16 && p.drop_thresh == 0) return ody_launch_attn_bwd_hd64(p, workspace, workspace_bytes, st);
   if (!p.reuse_query_side && (rc = ody_launch_attn_delta(p, D, dtype, st))) return rc;
   if (dtype == ODY_BF16) return ody_launch_attn_bwd_mfma(p, D, st);
   return ody_launch_attn_bwd_f32(p, D, st);

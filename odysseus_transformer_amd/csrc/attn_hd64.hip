@@ -658,7 +658,7 @@ size_t ody_attn_bwd_hd64_workspace(int B, int Lq, int Lk, int Hq, int Hkv) {
   return delta_bytes(B, Lq, Hq) + (split_heads(B, Lk, Hq, Hkv) ? align256((size_t)2 * B * Hq * Lk * D * sizeof(float)) : 0);
 }
 
-int ody_launch_attn_bwd_hd64(const AttnParams& p, void* workspace, hipStream_t st) {
+int ody_launch_attn_bwd_hd64(const AttnParams& p, void* workspace, size_t workspace_bytes, hipStream_t st) {
   float* neg_delta = static_cast<float*>(workspace);
   float* part = reinterpret_cast<float*>(static_cast<char*>(workspace) + delta_bytes(p.B, p.Lq, p.Hq));
   int rc;
@@ -666,7 +666,7 @@ int ody_launch_attn_bwd_hd64(const AttnParams& p, void* workspace, hipStream_t s
     ODY_LAUNCH("attn_bwd_hd64_rows", st, attn_bwd_hd64_rows_kernel, dim3((p.Lq + 31) / 32, p.Hq, p.B), dim3(256), 0, p, neg_delta);
     if ((rc = ody_check_launch("attn_bwd_hd64_rows"))) return rc;
   }
-  const bool heads = split_heads(p.B, p.Lk, p.Hq, p.Hkv);
+  const bool heads = split_heads(p.B, p.Lk, p.Hq, p.Hkv) && workspace_bytes >= ody_attn_bwd_hd64_workspace(p.B, p.Lq, p.Lk, p.Hq, p.Hkv);
   const int64_t nkv = row_blocks(p.B, p.Lk, heads ? p.Hq : p.Hkv), nq = row_blocks(p.B, p.Lq, p.Hq);
   auto dkdv = [&](auto kern, int groups) { return launch("attn_bwd_hd64_dkdv", kern, nkv, groups, QS_STAGE, st, p, neg_delta, part); };
   if (nkv < FEW_BLOCKS) rc = heads ? dkdv(&attn_bwd_hd64_dkdv_kernel<2, true>, 2) : dkdv(&attn_bwd_hd64_dkdv_kernel<2, false>, 2);

@@ -98,11 +98,11 @@ size_t ody_attn_bwd_pipe_workspace(int B, int Lq, int Lk, int Hq, int Hkv);
 // bytes of the kept dS tiles (AttnParams::ds), 0 where the shape does not qualify
 size_t ody_attn_bwd_pipe_ds_bytes(int B, int Lq, int Lk, int Hq, int causal);
 int ody_launch_attn_bwd_pipe(const AttnParams& p, void* workspace, hipStream_t st);
-// head_dim 64, bf16, no dropout; the forward needs no workspace, the backward one of ody_attn_bwd_hd64_workspace(...) bytes (its
-// row values take the place of p.delta)
+// head_dim 64, bf16, no dropout; the forward needs no workspace, the backward room for its row values, which take the place of
+// p.delta.  With ody_attn_bwd_hd64_workspace(...) bytes it can take the query heads of a group apart; with less it does not.
 int ody_launch_attn_fwd_hd64(const AttnParams& p, hipStream_t st);
 size_t ody_attn_bwd_hd64_workspace(int B, int Lq, int Lk, int Hq, int Hkv);
-int ody_launch_attn_bwd_hd64(const AttnParams& p, void* workspace, hipStream_t st);
+int ody_launch_attn_bwd_hd64(const AttnParams& p, void* workspace, size_t workspace_bytes, hipStream_t st);
 // with dropout, both head dims
 int ody_launch_attn_bwd_mfma(const AttnParams& p, int D, hipStream_t st);
 // fp32 on the fp32 matrix cores

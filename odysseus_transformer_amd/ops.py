@@ -199,6 +199,7 @@ def attn_bwd(q, k, v, out, lse, dout, causal: bool = True, scale: Optional[float
     scale = 1.0 / math.sqrt(D) if scale is None else float(scale)
     lib = _lib.load()
     ws_bytes = lib.ody_attn_bwd_workspace_bytes(B, Lq, Lk, Hq, Hkv, D, _dt(q))
+    least = lib.ody_attn_bwd_workspace_least_bytes(B, Lq, Lk, Hq, Hkv, D, _dt(q))
     ds_bytes = lib.ody_attn_bwd_ds_bytes(B, Lq, Lk, Hq, Hkv, D, _dt(q), int(causal)) if keep_ds is not False else 0
     if keep_ds and ds_bytes == 0:
         raise ValueError(_KEEP_DS_SHAPES)
@@ -213,15 +214,17 @@ def attn_bwd(q, k, v, out, lse, dout, causal: bool = True, scale: Optional[float
                 _KEEP_DS_OOM[str(q.device)] = min(ds_bytes, _KEEP_DS_OOM.get(str(q.device), 1 << 62))
     if keep_ds:
         ws_bytes += ds_bytes
+        least += ds_bytes
     if workspace is None:
         if reuse_query_side:
             raise ValueError("reuse_query_side needs the workspace of the previous call")
         if ws is None:
-            ws = scratch(ws_bytes, "attn_bwd_workspace", q.device)
+            ws = _scratch_or_least(ws_bytes, least, lambda n: scratch(n, "attn_bwd_workspace", q.device))
     else:
         ws = workspace
-        if ws.dtype != torch.uint8 or ws.numel() < ws_bytes or ws.device != q.device or not ws.is_contiguous():
-            raise ValueError(f"workspace must be a contiguous uint8 tensor of at least {ws_bytes} bytes on {q.device}")
+        if ws.dtype != torch.uint8 or ws.numel() < least or ws.device != q.device or not ws.is_contiguous():
+            raise ValueError(f"workspace must be a contiguous uint8 tensor of at least {least} bytes on {q.device}")
+    ws_bytes = ws.numel()
     flags = (_lib.BWD_ACCUMULATE_DQ if accumulate_dq else 0) | (_lib.BWD_DQ_F32 if dq_f32 else 0) | \
             (_lib.BWD_REUSE_QUERY_SIDE if reuse_query_side else 0) | (_lib.BWD_KEEP_DS if keep_ds else 0)
     if lse.dtype != torch.float32 or not lse.is_contiguous():
@@ -243,6 +246,16 @@ def attn_bwd(q, k, v, out, lse, dout, causal: bool = True, scale: Optional[float
                 raise ValueError(f"{n} must be a contiguous bfloat16 ({rows}, {D}) tensor on {q.device}")
         _lib.call("ody_attn_bwd_rope", *args, tq.data_ptr(), tk.data_ptr())
     return dq, dk, dv
+
+
+def _scratch_or_least(nbytes: int, least: int, allocate) -> torch.Tensor:
+    """allocate(nbytes), or allocate(least) where that much memory is not there and the kernels can do with less."""
+    try:
+        return allocate(nbytes)
+    except torch.OutOfMemoryError:
+        if least >= nbytes:
+            raise
+    return allocate(least)
 
 
 _KEEP_DS_MAX_BYTES: Optional[int] = None
@@ -341,7 +354,9 @@ def _shared_bwd_workspace(calls):
             return torch.empty(n, dtype=torch.uint8, device=device), keeps
         except torch.OutOfMemoryError:
             _KEEP_DS_OOM[str(device)] = min(failed, min(d for d, kp in zip(ds, keeps) if kp))
-    return torch.empty(max(base), dtype=torch.uint8, device=device), [False] * len(calls)
+    least = max(lib.ody_attn_bwd_workspace_least_bytes(*d) for d in dims)
+    ws = _scratch_or_least(max(base), least, lambda n: torch.empty(n, dtype=torch.uint8, device=device))
+    return ws, [False] * len(calls)
 
 
 def cast_from_f32(src, dtype) -> torch.Tensor:

@@ -617,3 +617,25 @@ def test_attention_hd64_running_fp32_dq(dev):
     for got, ref, name in ((dq, refs[0], "dq"), (torch.cat([p[1] for p in parts], 1), refs[1], "dk"),
                            (torch.cat([p[2] for p in parts], 1), refs[2], "dv")):
         assert_parity(got, ref, TOL_BF16, name)
+
+
+@pytest.mark.parametrize("case", [(1, 70, 331, 8, 2, True), (2, 130, 193, 12, 3, False)], ids=lambda c: "B%d_Lq%d_Lk%d_H%d_%d_c%d" % c)
+def test_attention_hd64_backward_in_the_least_workspace(case, dev):
+    """Without room for the fp32 dK / dV of every query head a group's heads are walked in turn: same dQ, and dK / dV that differ by
+    the order of a sum."""
+    from odysseus_transformer_amd import _lib, ops
+    B, Lq, Lk, Hq, Hkv, causal = case
+    q, k, v, do = _inputs(B, Lq, Lk, Hq, Hkv, 64, torch.bfloat16, seed=31)
+    o_ref, lse_ref = oracle.attention_fwd(q.float(), k.float(), v.float(), causal=causal)
+    refs = oracle.attention_bwd(q.float(), k.float(), v.float(), o_ref, lse_ref, do.float(), causal=causal)
+    args = [t.to(dev) for t in (q, k, v, o_ref.bfloat16(), lse_ref, do)]
+    least = _lib.load().ody_attn_bwd_workspace_least_bytes(B, Lq, Lk, Hq, Hkv, 64, _lib.ODY_BF16)
+    assert least < ops.attn_bwd_workspace(args[0], args[1]).numel()
+    ws = torch.full((least + 256,), 0xA5, dtype=torch.uint8, device=dev)
+    split = ops.attn_bwd(*args, causal=causal)
+    whole = ops.attn_bwd(*args, causal=causal, workspace=ws[:least])
+    torch.cuda.synchronize()
+    assert bool((ws[least:] == 0xA5).all())
+    assert torch.equal(split[0], whole[0])
+    for got, ref, name in zip(whole, refs, ("dq", "dk", "dv")):
+        assert_parity(got, ref, TOL_BF16, name)

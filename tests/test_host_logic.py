@@ -557,3 +557,35 @@ def test_zigzag_backward_workspace_has_room_for_every_step(Hq, Hkv, D, c, keep_d
     finally:
         ops.set_keep_ds_max_bytes(None)
     assert calls.count("ody_attn_bwd") == 9
+
+
+@pytest.mark.parametrize("ring", [False, True])
+def test_grouped_heads_of_64_backward_without_memory_for_the_parts(ring, monkeypatch):
+    """The fp32 dK / dV of every query head (here 2.1 GB) are an offer: where that much is not there, or a caller's workspace is
+    smaller, the call takes the delta-sized scratch that it always took."""
+    from odysseus_transformer_amd import _lib, ops
+    sizes, real = [], torch.empty
+    monkeypatch.setattr(_lib, "call", lambda name, *a: sizes.append(a[-2]) if name == "ody_attn_bwd" else None)
+    monkeypatch.setattr(ops, "_need_gpu", lambda *t: None)
+    monkeypatch.setattr(ops, "_stream", lambda: 0)
+
+    def short_of_memory(*args, **kw):
+        if kw.get("dtype") is torch.uint8 and args[0] > 1 << 30:
+            raise torch.OutOfMemoryError("out of memory")
+        return real(*args, **kw)
+
+    B, L, Hq, Hkv, D = 1, 130000, 32, 1, 64
+    delta = (4 * B * L * Hq + 255) // 256 * 256
+    t = lambda h: real((B, L, h, D), dtype=torch.bfloat16, device="meta", requires_grad=True)  # noqa: E731
+    q, k, v = t(Hq), t(Hkv), t(Hkv)
+    monkeypatch.setattr(torch, "empty", short_of_memory)
+    if ring:
+        ops.ring_blocks_attn(q, [k], [v])[0].backward(real(q.shape, dtype=q.dtype, device="meta"))
+    else:
+        lse = real((B, Hq, L), dtype=torch.float32, device="meta")
+        ops.attn_bwd(q, k, v, q, lse, q)
+        ws = real(delta, dtype=torch.uint8, device="meta")
+        ops.attn_bwd(q, k, v, q, lse, q, workspace=ws)
+        with pytest.raises(ValueError):
+            ops.attn_bwd(q, k, v, q, lse, q, workspace=ws[:-256])
+    assert set(sizes) == {delta}
