@@ -270,6 +270,7 @@ Plan plan_with_workspace(int M, int N, int K, const void* workspace, size_t work
 }
 
 bool vec16(const void* p, int64_t ld) { return ody_aligned16(p) && ld % 8 == 0; }
+bool vec8(const void* p, int64_t ld) { return (reinterpret_cast<uintptr_t>(p) & 7u) == 0 && ld % 4 == 0; }
 
 // whether the byte offsets inside a tile fit the tile kernel's 32 bits
 bool tile_pitch_ok(int op, int64_t lda, int64_t ldb) {
@@ -727,13 +728,14 @@ extern "C" int ody_linear_residual_ws(const void* x, const void* w, const void* 
     return ody_launch_gemm_skinny(EPI_RESIDUAL, static_cast<const bf16*>(x), static_cast<const bf16*>(w), static_cast<bf16*>(y),
                                   nullptr, M, N, K, ldx, ldw, ldy, 0, ep, st);
   }
-  if (dtype == ODY_BF16 && K % 8 == 0 && N % 8 == 0 && tile_pitch_ok(ODY_GEMM_NT, ldx, ldw) && vec16(x, ldx) && vec16(w, ldw))
+  if (dtype == ODY_BF16 && K % 8 == 0 && N % 8 == 0 && tile_pitch_ok(ODY_GEMM_NT, ldx, ldw) && vec16(x, ldx) && vec16(w, ldw) &&
+      vec8(residual, ld_res) && vec8(y, ldy))   // the epilogues move at least four elements at a time
     return gemm_bf16(ODY_GEMM_NT, static_cast<const bf16*>(x), static_cast<const bf16*>(w), static_cast<bf16*>(y), nullptr,
                      static_cast<const bf16*>(residual), M, N, K, ldx, ldw, ldy, ld_res, workspace, workspace_bytes, st);
   if (dtype == ODY_F32)
     return gemm_f32(ODY_GEMM_NT, static_cast<const float*>(x), static_cast<const float*>(w), static_cast<float*>(y), nullptr, M, N, K, ldx,
                     ldw, ldy, static_cast<const float*>(residual), y == residual ? ldy : ld_res, workspace, workspace_bytes, st);
-  // any other shape: y = residual, then y += x W^T (added in fp32 before the one rounding, as above)
+  // any other shape or alignment: y = residual, then y += x W^T (added in fp32 before the one rounding, as above)
   if (y != residual) {
     hipError_t e = hipMemcpy2DAsync(y, (size_t)ldy * sizeof(bf16), residual, (size_t)ld_res * sizeof(bf16), (size_t)N * sizeof(bf16), (size_t)M,
                                     hipMemcpyDeviceToDevice, st);

@@ -48,6 +48,12 @@ def test_validation_returns_codes_without_a_gpu():
     with pytest.raises(_lib.OdysseusHipError) as e:
         _lib.call("ody_rmsnorm_fwd", 16, 16, 16, 0, 4, 7, 1e-6, 0, 0)
     assert e.value.code == -2
+    # a result that 8-byte pieces cannot address, in place on the residual: by its address, by its pitch
+    for y, ldy in ((18, 64), (20, 64), (16, 66)):
+        for M in (4, 40):
+            with pytest.raises(_lib.OdysseusHipError) as e:
+                _lib.call("ody_linear_residual_ws", 16, 16, y, y, M, 64, 64, 64, 64, ldy, ldy, 0, 0, 0, 0)
+            assert e.value.code == -3
     assert lib.ody_attn_bwd_workspace_bytes(1, 1000, 1000, 4, 4, 64, 0) == 16128
     assert lib.ody_rmsnorm_bwd_partials(100) == 100 and lib.ody_rmsnorm_bwd_partials(100000) == 256
 

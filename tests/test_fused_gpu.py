@@ -366,3 +366,15 @@ def test_decoding_step_under_inference_mode_with_an_advancing_position_tensor(de
             results.append((torch.cat(outs, 1), cache.k))
     for a, b in zip(*results):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("M,N,K", [(5, 264, 136), (40, 264, 136), (200, 128, 4096)], ids=["few rows", "one pass", "K in ranges"])
+@pytest.mark.parametrize("offset,pitch", [(1, 3), (2, 2), (4, 4), (8, 8), (0, 1)])
+def test_linear_residual_with_a_residual_of_any_alignment(M, N, K, offset, pitch, dev):
+    """The residual as a column slice that starts `offset` elements into rows N + offset + pitch apart: pieces of 16, 8, 4 and 2 bytes."""
+    from odysseus_transformer_amd import _lib, ops
+    x, w, wide = randn((M, K), 9800, dtype=BF), randn((N, K), 9801, std=0.05, dtype=BF), randn((M, N + offset + pitch), 9802, dtype=BF)
+    if K > 1000:
+        assert _lib.load().ody_gemm_workspace_bytes(ops.GEMM_NT, M, N, K, _lib.ODY_BF16) > 0
+    y = ops.linear_residual(x.to(dev), w.to(dev), wide.to(dev)[:, offset:offset + N])
+    assert rel_err(y, x.float() @ w.float().t() + wide[:, offset:offset + N].float()) <= TOL_BF16
