@@ -6,7 +6,8 @@
 // the same tile as the row operands -- no transposed images, hence no pre-pass over V and K and half the tile bytes --, three
 // or four wavefronts share a SIMD to keep the vector pipe fed, and the softmax of the forward does no work that the result does
 // not need: a row's reference is the maximum of its first tile, nothing is compared or rescaled after it, and a block where a
-// later score outgrew that by more than fp32 holds walks its keys once more with a reference that follows.
+// later score outgrew that by more than fp32 holds, in a row sum or in a sum of P V, walks its keys once more with a reference
+// that follows.
 //
 // A block is 4 wavefronts of 32 rows each (queries; keys in the dK/dV kernel) against 64-row tiles of the other side, which go
 // straight to LDS (direct loads, two stages).  GROUPS = 2 gives a block a second set of 4 wavefronts over the same rows, which
@@ -197,7 +198,7 @@ __global__ __launch_bounds__(256 * GROUPS, 4) void attn_fwd_hd64_kernel(const At
   float l4[4];   // this lane's partial row sums
 
   // ONLINE = false: the reference of a row is the largest score of its first tile (a row that sees any key sees key 0) and stays.
-  // ONLINE = true: it follows the maximum, in steps of 2^8 and more.
+  // ONLINE = true: it is the maximum so far, so that P <= 1 and P V overflows for no values that P = 1 would hold.
   const int iters = (ntiles + GROUPS - 1) / GROUPS;
   auto walk = [&](auto online) {
     constexpr bool ONLINE = decltype(online)::value;
@@ -227,7 +228,7 @@ __global__ __launch_bounds__(256 * GROUPS, 4) void attn_fwd_hd64_kernel(const At
 #pragma unroll
         for (int r = 1; r < 16; r++) mx = fmaxf(mx, fmaxf(s[0][r], s[1][r]));
         mx = half_swap_max(mx) * c2;
-        if (__builtin_amdgcn_ballot_w64(mx > ref + 8.f) != 0) {
+        if (__builtin_amdgcn_ballot_w64(mx > ref) != 0) {
           const float next = fmaxf(ref, mx), alpha = ody_exp2(ref - next);
           ref = next;
 #pragma unroll
@@ -270,9 +271,16 @@ __global__ __launch_bounds__(256 * GROUPS, 4) void attn_fwd_hd64_kernel(const At
   };
   walk(std::false_type{});
   {
-    // a later score that outgrew its row's reference by more than fp32 holds left a row sum beyond any real one (or a NaN)
+    // a later score that outgrew its row's reference by more than fp32 holds left a row sum beyond any real one (or a NaN), or,
+    // times large values, an infinity in O: 0 times the accumulators is 0 unless one of them is not finite
     int* flags = reinterpret_cast<int*>(smem);
-    const bool beyond = __builtin_amdgcn_ballot_w64(!(half_swap_sum((l4[0] + l4[1]) + (l4[2] + l4[3])) < 0x1p100f)) != 0;
+    float zero[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int dt = 0; dt < DT; dt++)
+#pragma unroll
+      for (int r = 0; r < 16; r++) zero[r & 3] = fmaf(o[dt][r], 0.f, zero[r & 3]);
+    const bool finite = (zero[0] + zero[1]) + (zero[2] + zero[3]) == 0.f;
+    const bool beyond = __builtin_amdgcn_ballot_w64(!finite || !(half_swap_sum((l4[0] + l4[1]) + (l4[2] + l4[3])) < 0x1p100f)) != 0;
     if (lane == 0) flags[wave] = beyond;
     __syncthreads();
     int any = 0;

@@ -639,3 +639,26 @@ def test_attention_hd64_backward_in_the_least_workspace(case, dev):
     assert torch.equal(split[0], whole[0])
     for got, ref, name in zip(whole, refs, ("dq", "dk", "dv")):
         assert_parity(got, ref, TOL_BF16, name)
+
+
+def _outgrown(B, Lq, Lk, H, D, late, seed):
+    """Inputs whose scores are small on the first keys and reach about `late` (natural log) on the last quarter of them, with values
+    of 2^48: P V, relative to the first keys' maximum, then leaves fp32 long before the row sum does."""
+    q, k, v, _ = _inputs(B, Lq, Lk, H, H, D, torch.bfloat16, seed=seed)
+    q[..., 0], k[..., 0] = 8.0, 0.0
+    k[:, -(Lk // 4):, :, 0] = late * D ** 0.5 / 8.0
+    return q, k, (v.float() * 2.0 ** 48).bfloat16()
+
+
+@pytest.mark.parametrize("case", [(1, 200, 320, 2, False), (1, 331, 331, 2, True), (1, 70, 1000, 600, False)],
+                         ids=lambda c: "Lq%d_Lk%d_H%d_c%d" % c[1:])
+def test_attention_hd64_large_values_behind_an_outgrown_reference(case, dev):
+    """Scores 56 above a row's first tile with |v| around 2^48: finite, and nothing may overflow on the way."""
+    from odysseus_transformer_amd import ops
+    B, Lq, Lk, H, causal = case
+    q, k, v = _outgrown(B, Lq, Lk, H, 64, 56.0, seed=71)
+    o_ref, lse_ref = oracle.attention_fwd(q.float(), k.float(), v.float(), causal=causal)
+    o, lse = ops.attn_fwd(q.to(dev), k.to(dev), v.to(dev), causal=causal)
+    assert bool(o.isfinite().all())
+    assert_parity(o, o_ref, TOL_BF16, "o")
+    assert torch.allclose(lse.cpu(), lse_ref, atol=TOL_LSE, rtol=TOL_LSE)
