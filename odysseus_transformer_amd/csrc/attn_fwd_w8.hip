@@ -9,8 +9,8 @@
 //
 // The reference m of a query is fixed by its first 32 keys (key 0 is among them, and a query that
 // sees any key sees key 0): the loop neither tracks maxima nor rescales O.  A later score that
-// outgrows the reference by more than fp32 can hold shows up as a row sum that overflowed; the
-// 256-query block is then flagged and redone by the online-rescaling kernel.
+// outgrows the reference by more than fp32 can hold shows up as a row sum that overflowed, or, with large values, as an
+// accumulator of O that did; the 256-query block is then flagged and redone by the online-rescaling kernel.
 //
 // A call with few query blocks (16384 queries are 64 per head; the off-diagonal steps of a zigzag ring have 32) leaves
 // compute units idle or, under a causal mask, waiting for the one with the longest block: then every block's key range
@@ -191,7 +191,13 @@ __global__ __launch_bounds__(FW_THREADS) void attn_fwd_w8_kernel(const AttnParam
 
   // ---- epilogue
   const float lt = half_swap_sum((l4[0] + l4[1]) + (l4[2] + l4[3]));
-  if (__builtin_amdgcn_ballot_w64(!(lt < 0x1p100f)) != 0 && lane == 0)
+  float zero[4] = {0.f, 0.f, 0.f, 0.f};   // 0 times the accumulators of O: 0 unless one of them is not finite
+#pragma unroll
+  for (int dt = 0; dt < DT; dt++)
+#pragma unroll
+    for (int r = 0; r < 16; r++) zero[r & 3] = fmaf(o[dt][r], 0.f, zero[r & 3]);
+  const bool finite = (zero[0] + zero[1]) + (zero[2] + zero[3]) == 0.f;
+  if (__builtin_amdgcn_ballot_w64(!finite || !(lt < 0x1p100f)) != 0 && lane == 0)
     atomicOr(bail_flags + ((int64_t)b * p.Hq + h) * nqb + qblk, 1);
   if (nsplit > 1) {
     if (qi < p.Lq) {   // this part's normalised result and log-sum-exp, for the merge kernel

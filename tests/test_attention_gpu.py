@@ -662,3 +662,17 @@ def test_attention_hd64_large_values_behind_an_outgrown_reference(case, dev):
     assert bool(o.isfinite().all())
     assert_parity(o, o_ref, TOL_BF16, "o")
     assert torch.allclose(lse.cpu(), lse_ref, atol=TOL_LSE, rtol=TOL_LSE)
+
+
+@pytest.mark.parametrize("case", [(1, 300, 320, 2, False), (1, 331, 331, 2, True), (1, 200, 2048, 2, False), (1, 2100, 2100, 1, True)],
+                         ids=lambda c: "Lq%d_Lk%d_H%d_c%d" % c[1:])
+def test_attention_hd128_large_values_behind_an_outgrown_reference(case, dev):
+    """The same for the kernels of head_dim 128, whole and with the keys cut into parts."""
+    from odysseus_transformer_amd import ops
+    B, Lq, Lk, H, causal = case
+    q, k, v = _outgrown(B, Lq, Lk, H, 128, 56.0, seed=73)
+    o_ref, lse_ref = oracle.attention_fwd(q.float(), k.float(), v.float(), causal=causal)
+    o, lse = ops.attn_fwd(q.to(dev), k.to(dev), v.to(dev), causal=causal)
+    assert bool(o.isfinite().all())
+    assert_parity(o, o_ref, TOL_BF16, "o")
+    assert torch.allclose(lse.cpu(), lse_ref, atol=TOL_LSE, rtol=TOL_LSE)
