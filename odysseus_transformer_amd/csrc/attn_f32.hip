@@ -17,9 +17,9 @@
 // SPLIT instances serve calls with few rows, whose 128-row workgroups would leave compute units idle (and, under a causal
 // mask, wait for the longest): the wavefronts (eight at head_dim 64) own the SAME 32 rows and take the streamed tiles in turn, each through
 // LDS of its own (no barrier in the loop), and add their results up through LDS at the end.  8 heads x 64, L = 2048,
-// causal: forward 162 -> 63 us, dQ 237 -> 81, dK / dV 304 -> 109; 8 x 64, L = 8192 (one 128-row workgroup per half compute
-// unit): 840 -> 688, 1238 -> 913, 1610 -> 1275; the line lies at the
-// widest launches tried.
+// causal: forward 160 -> 56 us, dQ 237 -> 73, dK / dV 298 -> 97; 8 x 64, L = 8192: 842 -> 689, 1262 -> 913, 1600 -> 1287.
+// Where they do not serve, few_rows() below: 16 heads x 64, 4096 rows against 4096 full: 572 us whole, 691 split, against 32: 15
+// and 57; 16 x 128, L = 4096, causal: 658 and 829.
 //
 // Two index permutations keep every LDS read conflict-free and 16 bytes wide where it
 // can be:
@@ -29,6 +29,8 @@
 //  * contraction over the 32 streamed rows: k-step ks multiplies row 8 (ks / 4) + 4 g +
 //    ks % 4, which is the row that result register ks of this lane already holds.
 // Everything is deterministic: no atomics, fixed summation order.
+#include <algorithm>
+#include <cmath>
 #include "attn_params.h"
 #include "attn_tile.h"
 
@@ -561,9 +563,35 @@ __global__ __launch_bounds__(256) void attn_delta_kernel(const AttnParams p) {
   if (row < total && sub == 0) p.delta[row] = acc;
 }
 
-// Whether `rows` per (head, batch) leave 128-row workgroups too few (two per compute unit even out a causal mask); beyond that
-// the shared tiles of the wider workgroup save memory traffic.
-bool few_rows(int rows, int heads) { return (int64_t)((rows + F_ROWS - 1) / F_ROWS) * heads < 1024; }
+// Tiles of the streamed side that a row block walks: the longest walk and the mean.
+struct Walk { double longest, mean; };
+Walk walk(const AttnParams& p, bool own_keys) {
+  double pairs = (double)p.Lq * p.Lk, longest = own_keys ? p.Lq : p.Lk;
+  if (p.causal) {   // a query sees keys up to its own position + off; before that, none
+    pairs = p.off >= 0 ? (double)p.Lq * (p.off + 0.5 * p.Lq) : 0.5 * p.Lk * p.Lk;
+    if (own_keys) longest = std::min(p.Lq, p.Lk);
+  }
+  const double share = own_keys ? (double)p.group / p.Lk : 1.0 / p.Lq;
+  if (own_keys) longest *= p.group;
+  return Walk{std::ceil(longest / F_TILE), std::min(pairs * share, longest) / F_TILE};
+}
+
+// Whether the SPLIT instance is the faster one, in units of the time that a lone 128-row workgroup takes per tile (2.4 us in the
+// forward of head_dim 64, 4.7 at 128).  That workgroup's walk is as long as its tiles; where several share a unit, the unit is
+// at 0.9 per tile, and behind a causal mask's longest walk most of the unit idles at head_dim 64 (three workgroups share one) and
+// little at 128 (one each).  A round of 256 split workgroups costs its start and end and 0.32 (head_dim 128: 0.34) per tile, and
+// no less than one tile for each wavefront.  Fitted to 1100 shapes of 32 to 16384 rows and tokens, 1 to 256 heads, both masks:
+// never slower than the whole instance by more than 2 us, and 0.2 % off the better one in the mean.  Beyond 1024 whole
+// workgroups it was not measured.
+template <int D>
+bool few_rows(int rows, int heads, Walk w) {
+  constexpr double start = D == 64 ? 1.0 : 1.6, tile = D == 64 ? 0.32 : 0.34, idle = D == 64 ? 0.9 : 0.2;
+  const int64_t whole = (int64_t)((rows + F_ROWS - 1) / F_ROWS) * heads, split = (int64_t)((rows + 31) / 32) * heads;
+  if (whole >= 1024 || w.longest < 2) return false;
+  const double rounds = (double)((split + 255) / 256), per_unit = 0.9 * whole / 256.0;
+  return rounds * (start + tile * std::max(w.mean, (double)Shape<D, true>::WAVES)) <
+         1.75 + std::max(w.longest, per_unit * w.mean + idle * (w.longest - w.mean));
+}
 
 template <int D, bool SPLIT, typename K>
 int launch_one(const char* name, K kern, int rows, int heads, const AttnParams& p, hipStream_t st) {
@@ -577,7 +605,7 @@ int launch_one(const char* name, K kern, int rows, int heads, const AttnParams& 
 template <int D, bool DROP>
 int launch_fwd(const AttnParams& p, hipStream_t st) {
   const int heads = p.Hq * p.B;
-  if (few_rows(p.Lq, heads)) return launch_one<D, true>("attn_fwd_f32", &attn_fwd_f32_kernel<D, DROP, true>, p.Lq, heads, p, st);
+  if (few_rows<D>(p.Lq, heads, walk(p, false))) return launch_one<D, true>("attn_fwd_f32_split", &attn_fwd_f32_kernel<D, DROP, true>, p.Lq, heads, p, st);
   return launch_one<D, false>("attn_fwd_f32", &attn_fwd_f32_kernel<D, DROP, false>, p.Lq, heads, p, st);
 }
 
@@ -585,19 +613,19 @@ template <int D, bool DROP, bool SPLIT>
 int launch_dkdv(const AttnParams& p, hipStream_t st) {
   const int heads = p.Hkv * p.B;
   if constexpr (D == 64) {
-    return launch_one<D, SPLIT>("attn_bwd_dkdv_f32", &attn_bwd_dkdv_f32_kernel<D, 2, DROP, SPLIT>, p.Lk, heads, p, st);
+    return launch_one<D, SPLIT>(SPLIT ? "attn_bwd_dkdv_f32_split" : "attn_bwd_dkdv_f32", &attn_bwd_dkdv_f32_kernel<D, 2, DROP, SPLIT>, p.Lk, heads, p, st);
   } else {
-    if (int rc = launch_one<D, SPLIT>("attn_bwd_dv_f32", &attn_bwd_dkdv_f32_kernel<D, 0, DROP, SPLIT>, p.Lk, heads, p, st)) return rc;
-    return launch_one<D, SPLIT>("attn_bwd_dk_f32", &attn_bwd_dkdv_f32_kernel<D, 1, DROP, SPLIT>, p.Lk, heads, p, st);
+    if (int rc = launch_one<D, SPLIT>(SPLIT ? "attn_bwd_dv_f32_split" : "attn_bwd_dv_f32", &attn_bwd_dkdv_f32_kernel<D, 0, DROP, SPLIT>, p.Lk, heads, p, st)) return rc;
+    return launch_one<D, SPLIT>(SPLIT ? "attn_bwd_dk_f32_split" : "attn_bwd_dk_f32", &attn_bwd_dkdv_f32_kernel<D, 1, DROP, SPLIT>, p.Lk, heads, p, st);
   }
 }
 
 template <int D, bool DROP>
 int launch_bwd(const AttnParams& p, hipStream_t st) {
-  const int rc = few_rows(p.Lk, p.Hkv * p.B) ? launch_dkdv<D, DROP, true>(p, st) : launch_dkdv<D, DROP, false>(p, st);
+  const int rc = few_rows<D>(p.Lk, p.Hkv * p.B, walk(p, true)) ? launch_dkdv<D, DROP, true>(p, st) : launch_dkdv<D, DROP, false>(p, st);
   if (rc) return rc;
   const int heads = p.Hq * p.B;
-  if (few_rows(p.Lq, heads)) return launch_one<D, true>("attn_bwd_dq_f32", &attn_bwd_dq_f32_kernel<D, DROP, true>, p.Lq, heads, p, st);
+  if (few_rows<D>(p.Lq, heads, walk(p, false))) return launch_one<D, true>("attn_bwd_dq_f32_split", &attn_bwd_dq_f32_kernel<D, DROP, true>, p.Lq, heads, p, st);
   return launch_one<D, false>("attn_bwd_dq_f32", &attn_bwd_dq_f32_kernel<D, DROP, false>, p.Lq, heads, p, st);
 }
 
