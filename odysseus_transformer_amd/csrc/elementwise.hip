@@ -523,6 +523,8 @@ __global__ __launch_bounds__(256) void lse_merge_kernel(float* __restrict__ out_
   if (sub == 0) lse_acc[li] = nw;
 }
 
+constexpr int64_t MOST_BLOCKS = (1 << 24) - 1;   // of 256 threads: a launch takes fewer than 2^32 threads
+
 inline unsigned blocks_for(int64_t n) { return (unsigned)((n + 255) / 256); }
 
 template <typename T> constexpr int vecn() { return Vec16B<T>::N; }
@@ -543,8 +545,9 @@ extern "C" int ody_rmsnorm_fwd(const void* x, const void* w, void* y, float* rst
   ODY_REQUIRE(ody_aligned16(x) && ody_aligned16(w) && ody_aligned16(y), ODY_ERR_MISALIGNED,
               "ody_rmsnorm_fwd: pointers must be 16-byte aligned");
   hipStream_t st = static_cast<hipStream_t>(stream);
-  // a wavefront per row only where a row is too narrow for a block and there are many (see rmsnorm_fwd_row_kernel)
-  if (T <= 2048 || d / n >= 256) {
+  // a wavefront per row only where a row is too narrow for a block and there are many (see rmsnorm_fwd_row_kernel), or more than
+  // one launch of a block per row takes
+  if (T <= MOST_BLOCKS && (T <= 2048 || d / n >= 256)) {
     ODY_BY_DTYPE(dtype,
                  ODY_LAUNCH("rmsnorm_fwd", st, rmsnorm_fwd_row_kernel<bf16>, dim3(T), dim3(256), 0, (const bf16*)x, (const bf16*)w,
                             (bf16*)y, rstd, d, eps),

@@ -1,0 +1,74 @@
+"""What the entry points of elementwise.hip launch at sizes near the limits of a launch, without a GPU: the library runs in a process
+of its own against a stand-in for the runtime's launch call, which refuses what the runtime refuses (2^32 threads and more in a
+dimension) and hands grids and kernel arguments to the test."""
+import subprocess
+import sys
+import textwrap
+from pathlib import Path
+
+import pytest
+
+ROOT = Path(__file__).resolve().parent.parent
+
+STAND_IN = r"""
+#include <cstddef>
+#include <cstdint>
+struct dim3 { uint32_t x, y, z; };
+static thread_local struct { dim3 grid, block; size_t smem; void* stream; } pending;
+static thread_local int error = 0;
+static void (*seen)(uint32_t, uint32_t, void**) = nullptr;
+extern "C" {
+void on_launch(void (*f)(uint32_t, uint32_t, void**)) { seen = f; }
+int __hipPushCallConfiguration(dim3 grid, dim3 block, size_t smem, void* stream) { pending = {grid, block, smem, stream}; return 0; }
+int __hipPopCallConfiguration(dim3* grid, dim3* block, size_t* smem, void** stream) {
+  *grid = pending.grid, *block = pending.block, *smem = pending.smem, *stream = pending.stream;
+  return 0;
+}
+int hipLaunchKernel(const void*, dim3 grid, dim3 block, void** args, size_t, void*) {
+  if (grid.x == 0 || (uint64_t)grid.x * block.x >> 32) return error = 9;   // hipErrorInvalidConfiguration
+  seen(grid.x, block.x, args);
+  return 0;
+}
+int hipGetLastError() { const int e = error; error = 0; return e; }
+}
+"""
+
+PROLOGUE = """
+import ctypes as C, os, sys
+sys.path.insert(0, sys.argv[2])
+shim = C.CDLL(sys.argv[1], os.RTLD_GLOBAL | os.RTLD_NOW)   # before the library: its calls bind to the stand-in
+from odysseus_transformer_amd import _lib
+assert "torch" not in sys.modules
+launches = []
+@C.CFUNCTYPE(None, C.c_uint32, C.c_uint32, C.POINTER(C.c_void_p))
+def seen(grid, block, args):
+    launches.append((grid, block, read(args)))
+def value(args, k, kind):
+    return C.cast(args[k], C.POINTER(kind)).contents.value
+shim.on_launch(seen)
+A = 1 << 20   # an aligned address; nothing is read or written
+"""
+
+
+@pytest.fixture(scope="module")
+def stand_in(tmp_path_factory):
+    folder = tmp_path_factory.mktemp("stand_in")
+    (folder / "launch.cpp").write_text(STAND_IN)
+    subprocess.run(["g++", "-O1", "-shared", "-fPIC", "-o", str(folder / "launch.so"), str(folder / "launch.cpp")], check=True)
+    return str(folder / "launch.so")
+
+
+def run(stand_in, program):
+    r = subprocess.run([sys.executable, "-c", PROLOGUE + textwrap.dedent(program), stand_in, str(ROOT)], capture_output=True, text=True,
+                       timeout=120)
+    assert r.returncode == 0, r.stdout + r.stderr
+
+
+@pytest.mark.parametrize("rows", [(1 << 24) - 1, 1 << 24, (1 << 26) - 4])
+def test_rmsnorm_rows(stand_in, rows):
+    """A block per row up to 2^24 - 1 rows, a wavefront per row from there: the most rows of that kernel are the most of the call."""
+    run(stand_in, f"""
+        read = lambda args: None
+        _lib.call("ody_rmsnorm_fwd", A, A, A, 0, {rows}, 2048, 1e-6, _lib.ODY_BF16, 0)
+        assert launches == [({rows} if {rows} < 1 << 24 else ({rows} + 3) // 4, 256, None)], launches
+    """)
