@@ -335,11 +335,11 @@ __global__ __launch_bounds__(256) void colsum_kernel(const float* __restrict__ p
 template <typename T>
 __global__ __launch_bounds__(256) void rope_kernel(T* __restrict__ x, const int64_t* __restrict__ pos_ids,
                                                    const float* __restrict__ inv_freq, int B, int L, int n_rot, int D,
-                                                   int64_t sb, int64_t sl, int64_t sh, float log2_base, int inverse) {
+                                                   int64_t sb, int64_t sl, int64_t sh, float log2_base, int inverse, int64_t token0) {
   constexpr int N = VecIO<T>::N, MOST = 256;
   __shared__ __attribute__((aligned(16))) float cs[MOST], sn[MOST];   // [token][frequency of the pass]
   const int half = D / 2, tokens = max(1, MOST / half);
-  const int64_t first = (int64_t)blockIdx.x * tokens;
+  const int64_t first = token0 + (int64_t)blockIdx.x * tokens;   // token0: where this launch begins
   const int b0 = (int)(first / L), l0 = (int)(first % L), mine = (int)min((int64_t)tokens, (int64_t)B * L - first);
   for (int j0 = 0; j0 < half; j0 += MOST) {
     const int width = min(half - j0, MOST), vecs = width / N;
@@ -606,14 +606,17 @@ extern "C" int ody_rope(void* x, const int64_t* position_ids, const float* inv_f
   if (n_rot == 0) return ODY_OK;
   hipStream_t st = static_cast<hipStream_t>(stream);
   const int64_t tokens = std::max(1, 256 / (D / 2)), blocks = ((int64_t)B * L + tokens - 1) / tokens;
-  ODY_REQUIRE(blocks < (int64_t)1 << 31, ODY_ERR_BAD_SHAPE, "ody_rope: too many blocks for one launch");
   const float l2b = inv_freq ? 0.f : log2f(base);
-  ODY_BY_DTYPE(dtype,
-               ODY_LAUNCH("rope", st, rope_kernel<bf16>, dim3((unsigned)blocks), dim3(256), 0, (bf16*)x, position_ids,
-                                  inv_freq, B, L, n_rot, D, sx_b, sx_l, sx_h, l2b, inverse),
-               ODY_LAUNCH("rope", st, rope_kernel<float>, dim3((unsigned)blocks), dim3(256), 0, (float*)x,
-                                  position_ids, inv_freq, B, L, n_rot, D, sx_b, sx_l, sx_h, l2b, inverse));
-  return ody_check_launch("rope");
+  for (int64_t at = 0; at < blocks; at += MOST_BLOCKS) {
+    const dim3 grid((unsigned)std::min(blocks - at, MOST_BLOCKS));
+    ODY_BY_DTYPE(dtype,
+                 ODY_LAUNCH("rope", st, rope_kernel<bf16>, grid, dim3(256), 0, (bf16*)x, position_ids, inv_freq, B, L, n_rot, D, sx_b,
+                            sx_l, sx_h, l2b, inverse, at * tokens),
+                 ODY_LAUNCH("rope", st, rope_kernel<float>, grid, dim3(256), 0, (float*)x, position_ids, inv_freq, B, L, n_rot, D, sx_b,
+                            sx_l, sx_h, l2b, inverse, at * tokens));
+    if (int rc = ody_check_launch("rope")) return rc;
+  }
+  return ODY_OK;
 }
 
 extern "C" int ody_rope_table(const int64_t* position_ids, const float* inv_freq, int64_t rows, int D, float base,

@@ -72,3 +72,17 @@ def test_rmsnorm_rows(stand_in, rows):
         _lib.call("ody_rmsnorm_fwd", A, A, A, 0, {rows}, 2048, 1e-6, _lib.ODY_BF16, 0)
         assert launches == [({rows} if {rows} < 1 << 24 else ({rows} + 3) // 4, 256, None)], launches
     """)
+
+
+@pytest.mark.parametrize("B,L,D,dtype", [(1, 5, 128, 0), (3, 1 << 25, 128, 0), (2, (1 << 25) + 1, 64, 1), (1, (1 << 24) + 7, 1024, 1)])
+def test_rope_tokens(stand_in, B, L, D, dtype):
+    """One launch, or several that together take every token once."""
+    run(stand_in, f"""
+        read = lambda args: value(args, 12, C.c_int64)
+        _lib.call("ody_rope", A, 0, 0, {B}, {L}, 2, {D}, {L} * 4 * {D}, 4 * {D}, {D}, 10000.0, 0, {dtype}, 0)
+        tokens, at = max(1, 256 // ({D} // 2)), 0
+        for grid, block, token0 in launches:
+            assert token0 == at and block == 256, (token0, at)
+            at += grid * tokens
+        assert {B} * {L} <= at < {B} * {L} + tokens, (at, launches)
+    """)
