@@ -809,20 +809,22 @@ extern "C" int ody_adamw_many(void* const* params, const void* const* grads, voi
   }
   const float decay = 1.f - lr * weight_decay;
   hipStream_t st = static_cast<hipStream_t>(stream);
-  const int64_t chunk = (int64_t)256 * (dtype == ODY_BF16 ? 8 : 4), most = (int64_t)1 << 30;
+  const int64_t size = dtype == ODY_BF16 ? 2 : 4, chunk = 256 * 16 / size;   // elements per block
+  int64_t done = 0;   // elements of tensor k in the launches before
   for (int k = 0; k < count;) {
     AdamwTable tab{};
     int64_t blocks = 0;
     int c = 0;
-    for (; k < count && c < ADAMW_TENSORS; k++, c++) {
-      const int64_t more = (n[k] + chunk - 1) / chunk;
-      ODY_REQUIRE(more <= most, ODY_ERR_BAD_SHAPE, "ody_adamw: n=%lld", (long long)n[k]);
-      if (blocks + more > most) break;
-      blocks += more;
-      tab.p[c] = params[k], tab.g[c] = grads[k], tab.m[c] = exp_avgs[k], tab.v[c] = exp_avg_sqs[k], tab.n[c] = n[k];
+    while (k < count && c < ADAMW_TENSORS && blocks < MOST_BLOCKS) {
+      const int64_t at = done * size, take = std::min(n[k] - done, (MOST_BLOCKS - blocks) * chunk);
+      tab.p[c] = static_cast<char*>(params[k]) + at, tab.g[c] = static_cast<const char*>(grads[k]) + at;
+      tab.m[c] = static_cast<char*>(exp_avgs[k]) + at, tab.v[c] = static_cast<char*>(exp_avg_sqs[k]) + at, tab.n[c] = take;
       const double bc1 = 1.0 - pow((double)beta1, (double)steps[k]), bc2 = 1.0 - pow((double)beta2, (double)steps[k]);
       tab.step_size[c] = (float)((double)lr / bc1), tab.inv_sqrt_bc2[c] = (float)(1.0 / sqrt(bc2));
-      tab.end[c] = (unsigned)blocks;
+      blocks += (take + chunk - 1) / chunk;
+      tab.end[c++] = (unsigned)blocks;
+      done += take;
+      if (done == n[k]) k++, done = 0;
     }
     for (; c < ADAMW_TENSORS; c++) tab.end[c] = (unsigned)blocks;
     if (dtype == ODY_BF16) ODY_LAUNCH("adamw", st, adamw_kernel<bf16>, dim3((unsigned)blocks), dim3(256), 0, tab, decay, beta1, beta2, eps);

@@ -86,3 +86,48 @@ def test_rope_tokens(stand_in, B, L, D, dtype):
             at += grid * tokens
         assert {B} * {L} <= at < {B} * {L} + tokens, (at, launches)
     """)
+
+
+ADAMW = """
+N = 48
+class Table(C.Structure):
+    _fields_ = [("p", C.c_uint64 * N), ("g", C.c_uint64 * N), ("m", C.c_uint64 * N), ("v", C.c_uint64 * N), ("n", C.c_int64 * N),
+                ("step_size", C.c_float * N), ("inv_sqrt_bc2", C.c_float * N), ("end", C.c_uint32 * N)]
+def read(args):
+    return Table.from_buffer_copy(C.cast(args[0], C.POINTER(Table)).contents)
+def step(dtype, tensors):   # (address of the parameter, elements, step); gradient and moments 1, 2 and 3 << 44 behind it
+    n = len(tensors)
+    p, e, s = ((C.c_int64 * n)(*c) for c in zip(*tensors))
+    g, m, v = ((C.c_int64 * n)(*(t[0] + (k << 44) for t in tensors)) for k in (1, 2, 3))
+    _lib.call("ody_adamw_many", p, g, m, v, e, s, n, 1e-3, 0.9, 0.99, 1e-8, 0.01, dtype, 0)
+    covered = []   # per launch: (address, elements, step size) of its entries
+    for grid, block, t in launches:
+        size, first, entries = 2 if dtype == 0 else 4, 0, []
+        for k in range(N):
+            if t.end[k] == first:
+                break
+            assert t.end[k] - first == -(-t.n[k] * size // 4096) and t.p[k] % 16 == 0
+            assert [t.g[k], t.m[k], t.v[k]] == [t.p[k] + (j << 44) for j in (1, 2, 3)]
+            entries.append((t.p[k], t.n[k], t.step_size[k]))
+            first = t.end[k]
+        assert first == grid == t.end[N - 1] and block == 256
+        covered.append(entries)
+    return covered
+"""
+
+
+@pytest.mark.parametrize("dtype", [0, 1])
+def test_adamw_elements(stand_in, dtype):
+    """Tensors beyond a launch, alone and between small ones: every element in one launch, with its own tensor's step size."""
+    run(stand_in, ADAMW + f"""
+size, most = 2 if {dtype} == 0 else 4, ((1 << 24) - 1) * 4096
+sizes = [7, most // size - 2048, 5, 2 * most // size + 11, 4096] + [9] * 60
+tensors = [(A + (k << 38), n, k + 1) for k, n in enumerate(sizes)]
+covered = sum(step({dtype}, tensors), [])
+for p, n, s in tensors:
+    at, own = p, [e for e in covered if p <= e[0] < p + (1 << 38)]
+    for e in own:
+        assert e[0] == at and abs(e[2] / (1e-3 / (1 - 0.9 ** s)) - 1) < 1e-6, (e, at)
+        at += e[1] * size
+    assert at == p + n * size, (at, p, n)
+""")
