@@ -372,7 +372,8 @@ int ody_attn_bwd_dropout(const void* q, const void* k, const void* v, const void
 int ody_adamw(void* param, const void* grad, void* exp_avg, void* exp_avg_sq, int64_t n, float lr, float beta1,
               float beta2, float eps, float weight_decay, int64_t step, int dtype, void* stream);
 /* The same for `count` tensors of one dtype with the same hyper-parameters, a launch per 48 of them.  The tables are host
- * arrays, read before the call returns; n[k] elements, steps[k] as above; no two tensors may overlap. */
+ * arrays, read before the call returns; n[k] elements, steps[k] as above.  Parameters that share memory are updated one after
+ * the other, in their order; apart from that, no two of all these arrays may overlap. */
 int ody_adamw_many(void* const* params, const void* const* grads, void* const* exp_avgs, void* const* exp_avg_sqs,
                    const int64_t* n, const int64_t* steps, int count, float lr, float beta1, float beta2, float eps,
                    float weight_decay, int dtype, void* stream);

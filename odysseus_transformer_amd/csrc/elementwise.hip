@@ -791,6 +791,16 @@ __global__ __launch_bounds__(256) void adamw_kernel(const AdamwTable tab, float 
     v[k] = (T)vf;
   }
 }
+
+// whether a parameter shares memory with one of the table's first c
+bool overlaps(const AdamwTable& tab, int c, const void* param, int64_t bytes, int64_t size) {
+  const char* p = static_cast<const char*>(param);
+  for (int k = 0; k < c; k++) {
+    const char* q = static_cast<const char*>(tab.p[k]);
+    if (p < q + tab.n[k] * size && q < p + bytes) return true;
+  }
+  return false;
+}
 }  // namespace
 
 extern "C" int ody_adamw_many(void* const* params, const void* const* grads, void* const* exp_avgs, void* const* exp_avg_sqs,
@@ -817,6 +827,7 @@ extern "C" int ody_adamw_many(void* const* params, const void* const* grads, voi
     int c = 0;
     while (k < count && c < ADAMW_TENSORS && blocks < MOST_BLOCKS) {
       const int64_t at = done * size, take = std::min(n[k] - done, (MOST_BLOCKS - blocks) * chunk);
+      if (overlaps(tab, c, params[k], n[k] * size, size)) break;   // one after the other, in launches of their own
       tab.p[c] = static_cast<char*>(params[k]) + at, tab.g[c] = static_cast<const char*>(grads[k]) + at;
       tab.m[c] = static_cast<char*>(exp_avgs[k]) + at, tab.v[c] = static_cast<char*>(exp_avg_sqs[k]) + at, tab.n[c] = take;
       const double bc1 = 1.0 - pow((double)beta1, (double)steps[k]), bc2 = 1.0 - pow((double)beta2, (double)steps[k]);

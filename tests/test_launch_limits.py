@@ -131,3 +131,12 @@ for p, n, s in tensors:
         at += e[1] * size
     assert at == p + n * size, (at, p, n)
 """)
+
+
+def test_adamw_parameters_that_share_memory(stand_in):
+    """Their updates follow each other: never two in one launch, and in the order of the call."""
+    run(stand_in, ADAMW + """
+whole, part, behind, again = (A, 4096, 1), (A + 4096, 512, 2), (A + 8192, 512, 3), (A, 4096, 4)
+covered = [[e[0] for e in launch] for launch in step(0, [whole, behind, part, again])]
+assert covered == [[A, A + 8192], [A + 4096], [A]], covered
+""")
