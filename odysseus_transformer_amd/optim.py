@@ -63,10 +63,10 @@ class AdamW(torch.optim.Optimizer):
                     column.append(value)
             for (device, dtype), (*columns, counters, _grads) in batches.items():
                 n = len(columns[0])
-                for counter in counters:
-                    counter += 1
                 tables = [(ctypes.c_int64 * n)(*c) for c in columns]
                 _lib.call("ody_adamw_many", *tables, n, float(group["lr"]), float(b1), float(b2), float(group["eps"]),
                           float(group["weight_decay"]), 0 if dtype == torch.bfloat16 else 1,
                           torch.cuda.current_stream(device).cuda_stream)
+                for counter in counters:   # not before: a refused call updates nothing
+                    counter += 1
         return loss

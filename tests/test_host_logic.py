@@ -589,3 +589,37 @@ def test_grouped_heads_of_64_backward_without_memory_for_the_parts(ring, monkeyp
         with pytest.raises(ValueError):
             ops.attn_bwd(q, k, v, q, lse, q, workspace=ws[:-256])
     assert set(sizes) == {delta}
+
+
+@pytest.fixture
+def adamw_on_cpu(monkeypatch):
+    """AdamW on CPU parameters that call themselves device tensors, its kernel replaced by `calls.append`; yields (calls, parameter)."""
+    import types
+    from odysseus_transformer_amd import _lib
+    calls = []
+    monkeypatch.setattr(_lib, "call", lambda name, *args: calls.append(args))
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda device=None: types.SimpleNamespace(cuda_stream=0))
+
+    class OnDevice(torch.nn.Parameter):
+        is_cuda = True
+
+    def parameter(shape, grad=None):
+        p = OnDevice(torch.zeros(shape, dtype=torch.bfloat16))
+        p.grad = torch.ones(shape, dtype=torch.bfloat16) if grad is None else grad
+        return p
+    return calls, parameter
+
+
+def test_adamw_counts_no_step_that_was_refused(adamw_on_cpu, monkeypatch):
+    from odysseus_transformer_amd import _lib
+    from odysseus_transformer_amd.optim import AdamW
+    _, parameter = adamw_on_cpu
+    opt = AdamW([parameter((8,)), parameter((16,))])
+    opt.step()
+
+    def refuse(name, *args):
+        raise _lib.OdysseusHipError(name, -3, "misaligned")
+    monkeypatch.setattr(_lib, "call", refuse)
+    with pytest.raises(_lib.OdysseusHipError):
+        opt.step()
+    assert [int(s["step"]) for s in opt.state.values()] == [1, 1]
