@@ -37,7 +37,18 @@ class AdamW(torch.optim.Optimizer):
             b1, b2 = group["betas"]
             if group.get("amsgrad") or group.get("maximize") or group.get("decoupled_weight_decay", True) is False:
                 raise NotImplementedError("amsgrad, maximize and coupled (L2) weight decay are not implemented")
-            batches = {}   # (device, dtype) -> [param, grad, exp_avg, exp_avg_sq, numel, step] columns of one launch
+            batches = {}   # (device, dtype) -> rows of one call
+
+            def update(device, dtype, rows):
+                *columns, counters = zip(*rows)
+                n = len(rows)
+                tables = [(ctypes.c_int64 * n)(*c) for c in columns]
+                _lib.call("ody_adamw_many", *tables, n, float(group["lr"]), float(b1), float(b2), float(group["eps"]),
+                          float(group["weight_decay"]), 0 if dtype == torch.bfloat16 else 1,
+                          torch.cuda.current_stream(device).cuda_stream)
+                for counter in counters:   # not before: a refused call updates nothing
+                    counter += 1
+
             for p in group["params"]:
                 if p.grad is None:
                     continue
@@ -49,24 +60,21 @@ class AdamW(torch.optim.Optimizer):
                                        f"{p.device}); there is no CPU implementation in this package")
                 if p.dtype not in (torch.bfloat16, torch.float32) or not p.is_contiguous():
                     raise ValueError(f"parameters must be contiguous bfloat16 or float32 tensors, got {p.dtype}")
-                if g.dtype != p.dtype or not g.is_contiguous():
+                copied = g.dtype != p.dtype or not g.is_contiguous()
+                if copied:
                     g = g.to(p.dtype).contiguous()
                 state = self.state[p]
                 if len(state) == 0:
                     state["step"] = torch.tensor(0.0)
                     state["exp_avg"] = torch.zeros_like(p, memory_format=torch.preserve_format)
                     state["exp_avg_sq"] = torch.zeros_like(p, memory_format=torch.preserve_format)
-                columns = batches.setdefault((p.device, p.dtype), ([], [], [], [], [], [], [], []))
-                for column, value in zip(columns, (p.data_ptr(), g.data_ptr(), state["exp_avg"].data_ptr(),
-                                                   state["exp_avg_sq"].data_ptr(), p.numel(), int(state["step"].item()) + 1,
-                                                   state["step"], g)):
-                    column.append(value)
-            for (device, dtype), (*columns, counters, _grads) in batches.items():
-                n = len(columns[0])
-                tables = [(ctypes.c_int64 * n)(*c) for c in columns]
-                _lib.call("ody_adamw_many", *tables, n, float(group["lr"]), float(b1), float(b2), float(group["eps"]),
-                          float(group["weight_decay"]), 0 if dtype == torch.bfloat16 else 1,
-                          torch.cuda.current_stream(device).cuda_stream)
-                for counter in counters:   # not before: a refused call updates nothing
-                    counter += 1
+                row = (p.data_ptr(), g.data_ptr(), state["exp_avg"].data_ptr(), state["exp_avg_sq"].data_ptr(), p.numel(),
+                       int(state["step"].item()) + 1, state["step"])
+                if copied:   # used at once, so that no two copies are held
+                    update(p.device, p.dtype, [row])
+                    del g
+                else:
+                    batches.setdefault((p.device, p.dtype), []).append(row)
+            for (device, dtype), rows in batches.items():
+                update(device, dtype, rows)
         return loss

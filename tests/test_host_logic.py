@@ -623,3 +623,25 @@ def test_adamw_counts_no_step_that_was_refused(adamw_on_cpu, monkeypatch):
     with pytest.raises(_lib.OdysseusHipError):
         opt.step()
     assert [int(s["step"]) for s in opt.state.values()] == [1, 1]
+
+
+def test_adamw_holds_one_converted_gradient_at_a_time(adamw_on_cpu, monkeypatch):
+    """Gradients that must be copied into the parameter's dtype or layout: updated one by one, each copy gone before the next is made;
+    the others together."""
+    import weakref
+    from odysseus_transformer_amd import _lib
+    from odysseus_transformer_amd.optim import AdamW
+    calls, parameter = adamw_on_cpu
+    copies, alive = [], []
+    contiguous = torch.Tensor.contiguous
+
+    def seen(t):
+        alive.append(sum(r() is not None for r in copies))
+        c = contiguous(t)
+        copies.append(weakref.ref(c))
+        return c
+    monkeypatch.setattr(torch.Tensor, "contiguous", seen)
+    strided = [parameter((4, 6), torch.ones(6, 4, dtype=torch.bfloat16).t()) for _ in range(3)]
+    AdamW([parameter((8,)), strided[0], parameter((16,)), *strided[1:]]).step()
+    assert alive == [0, 0, 0]
+    assert sorted(args[6] for args in calls) == [1, 1, 1, 2]   # tensors per call
