@@ -79,6 +79,7 @@ __global__ __launch_bounds__(64 * DC_WAVES) void attn_decode_kernel(const AttnPa
 #pragma unroll
         for (int ks = 0; ks < KS; ks++) s[m][st] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[st][ks], qf[m][ks], s[m][st], 0, 0, 0);
       }
+    wavefront_sync();   // the tile before has been read
 #pragma unroll
     for (int j = 0; j < VL; j++) *reinterpret_cast<bf16x8*>(Vs + (RPL * j + lane / CPR) * VP + 8 * (lane % CPR)) = vr[j];
     // keys of a lane: k0 + 16 st + 4 q + r
@@ -114,7 +115,8 @@ __global__ __launch_bounds__(64 * DC_WAVES) void attn_decode_kernel(const AttnPa
 #pragma unroll
       for (int dt = 0; dt < DT; dt++) o[m][dt] *= alpha;
     }
-    // contraction index 8 q + j <-> key 16 (j >> 2) + 4 q + (j & 3); a wavefront's LDS operations complete in order
+    // contraction index 8 q + j <-> key 16 (j >> 2) + 4 q + (j & 3)
+    wavefront_sync();
     const bf16* vt = Vs + (4 * q + (c >> 2)) * VP + 4 * (c & 3);
 #pragma unroll
     for (int dt = 0; dt < DT; dt++) {

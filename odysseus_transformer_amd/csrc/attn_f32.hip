@@ -83,7 +83,8 @@ struct Shape {
   static constexpr int STEP = SPLIT ? WAVES * F_TILE : F_TILE;   // streamed rows between two turns of a wavefront
   static constexpr int TILES = SPLIT ? WAVES : 1;                // tiles of each kind in LDS
   __device__ static __forceinline__ void sync() {
-    if (!SPLIT) __syncthreads();   // a wavefront's own LDS operations complete in order
+    if (SPLIT) wavefront_sync();   // its tiles are its own
+    else __syncthreads();
   }
 };
 

@@ -305,10 +305,12 @@ __device__ __forceinline__ void gemm_tile_block(const Args& p, int m0, int tn) {
 #pragma unroll
     for (int a2 = 0; a2 < WM / 2; a2++) {
       ODY_FENCE();
+      wavefront_sync();   // the band before has been read
 #pragma unroll
       for (int t = 0; t < 2; t++)
 #pragma unroll
         for (int b = 0; b < WN; b++) *reinterpret_cast<f32x4*>(band + (16 * t + c) * EP + 16 * b + 4 * q) = acc[2 * a2 + t][b];
+      wavefront_sync();
 #pragma unroll
       for (int pass = 0; pass < 32 / RPP; pass++) {
         const int row = pass * RPP + lane / CPR, ch = lane % CPR, m = mw + 32 * a2 + row, n = n0 + wn * COLS + 4 * ch;
@@ -346,10 +348,12 @@ __device__ __forceinline__ void gemm_tile_block(const Args& p, int m0, int tn) {
 #pragma unroll
       for (int a2 = 0; a2 < WM / 2; a2++) {
         ODY_FENCE();
+        wavefront_sync();
 #pragma unroll
         for (int t = 0; t < 2; t++)
 #pragma unroll
           for (int b = 0; b < WN; b++) *reinterpret_cast<f32x4*>(band + (16 * t + c) * EP + 16 * b + 4 * q) = biased(acc[2 * a2 + t][b], b);
+        wavefront_sync();
 #pragma unroll
         for (int pass = 0; pass < 32 / RPP; pass++) {
           const int row = pass * RPP + lane / CPR, ch = lane % CPR, m = mw + 32 * a2 + row, n = n0 + wn * COLS + 8 * ch;
@@ -373,6 +377,7 @@ __device__ __forceinline__ void gemm_tile_block(const Args& p, int m0, int tn) {
 #pragma unroll
   for (int a2 = 0; a2 < WM / 2; a2++) {
     ODY_FENCE();
+    wavefront_sync();
     bf16x4 w[2][WN];
 #pragma unroll
     for (int t = 0; t < 2; t++) {
@@ -398,6 +403,7 @@ __device__ __forceinline__ void gemm_tile_block(const Args& p, int m0, int tn) {
 #pragma unroll
       for (int b = 0; b < WN; b++) *reinterpret_cast<bf16x4*>(band + (16 * t + c) * EP + 16 * b + 4 * q) = w[t][b];
     }
+    wavefront_sync();
 #pragma unroll
     for (int pass = 0; pass < 32 / RPP; pass++) {
       if (EPI == EPI_SWIGLU_FWD && p.C == nullptr) break;   // only h is wanted
@@ -431,6 +437,7 @@ __device__ __forceinline__ void gemm_tile_block(const Args& p, int m0, int tn) {
     if constexpr (EPI == EPI_SWIGLU_FWD) {
       // h from the rounded values: block b of the first half is the gate of block b of the second
       constexpr int EPH = COLS / 2 + 8, CPH = COLS / 16, RPH = 64 / CPH;
+      wavefront_sync();
 #pragma unroll
       for (int t = 0; t < 2; t++)
 #pragma unroll
@@ -443,6 +450,7 @@ __device__ __forceinline__ void gemm_tile_block(const Args& p, int m0, int tn) {
           }
           *reinterpret_cast<bf16x4*>(band + (16 * t + c) * EPH + 16 * b + 4 * q) = hv;
         }
+      wavefront_sync();
 #pragma unroll
       for (int pass = 0; pass < (32 + RPH - 1) / RPH; pass++) {
         const int row = pass * RPH + lane / CPH, ch = lane % CPH, m = mw + 32 * a2 + row, j = j0 + wn * 16 * NH + 8 * ch;

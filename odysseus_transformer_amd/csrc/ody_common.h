@@ -85,6 +85,15 @@ __device__ __forceinline__ bf16x8 concat4(bf16x4 lo, bf16x4 hi) {
   return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
 }
 
+// Between LDS writes of a wavefront's lanes and reads by its other lanes, and the other way round.  The hardware runs a wavefront's
+// LDS operations in order; the compiler, which looks at one lane, may swap a write and a read whose addresses differ there.  No
+// instruction comes of it.
+__device__ __forceinline__ void wavefront_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+}
+
 __device__ __forceinline__ f32x16 mfma32(bf16x8 a, bf16x8 b, f32x16 c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
 }
