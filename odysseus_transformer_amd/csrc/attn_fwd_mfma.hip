@@ -264,13 +264,8 @@ int launch(const AttnParams& p, const int* flags, int flag_block, hipStream_t st
 }  // namespace
 
 int ody_launch_attn_fwd_mfma(const AttnParams& p, int D, hipStream_t st) {
-  if (p.drop_thresh != 0) {
-    if (D == 128) return launch<128, 1, true>(p, nullptr, 1, st);
-    if (D == 64) return launch<64, 1, true>(p, nullptr, 1, st);
-  } else {
-    if (D == 128) return launch<128, 1, false>(p, nullptr, 1, st);
-    if (D == 64) return launch<64, 1, false>(p, nullptr, 1, st);
-  }
+  if (D == 128) return launch<128, 1, true>(p, nullptr, 1, st);
+  if (D == 64) return launch<64, 1, true>(p, nullptr, 1, st);
   ody_set_error("attn_fwd: head_dim %d not built (64, 128)", D);
   return ODY_ERR_UNSUPPORTED;
 }

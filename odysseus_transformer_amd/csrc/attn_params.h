@@ -72,6 +72,7 @@ __device__ __forceinline__ unsigned ody_dropout_hash(unsigned row, int k) { retu
 #endif
 
 // Launchers (one per translation unit); each returns an ody_status.
+// with dropout, both head dims
 int ody_launch_attn_fwd_mfma(const AttnParams& p, int D, hipStream_t st);
 // transposed 64-row tile images of a (B, L, H, 128) bf16 matrix (attn_tile.h)
 size_t ody_attn_images_bytes(int B, int L, int H);
