@@ -462,6 +462,11 @@ def _tensor_version(t) -> Optional[int]:
     return None if t.is_inference() else t._version
 
 
+def _recordable(t) -> bool:
+    """Whether autograd can keep `t` for a backward: outside torch.inference_mode() it refuses tensors made inside."""
+    return torch.is_inference_mode_enabled() or not t.is_inference()
+
+
 def rope_table(position_ids, rows: int, head_dim: int, base: float = 10000.0, device=None, inv_freq=None) -> torch.Tensor:
     """(rows, head_dim) bfloat16: [r, 2 j] = cos, [r, 2 j + 1] = sin of position r times frequency j, rounded
     as rope_ rounds them.  position_ids: int64 with `rows` elements in the order of the rows -- or with rows / B
@@ -470,8 +475,8 @@ def rope_table(position_ids, rows: int, head_dim: int, base: float = 10000.0, de
     The layers of a model are handed one and the same position tensor: the last table is kept and returned again
     for the same tensor object (unmodified since), shape, base and stream.  A tensor that cannot say whether it was
     modified (made under torch.inference_mode()) gets a new table every time, and so does a call under graph capture: a
-    replay has to read the positions again, and what a capture records has no values for later calls.  Treat the result
-    as read-only."""
+    replay has to read the positions again, and what a capture records has no values for later calls.  A table made under
+    inference mode is not handed out behind it, where autograd would refuse to keep it.  Treat the result as read-only."""
     global _ROPE_TABLE_LAST
     if position_ids is not None:
         device = position_ids.device
@@ -483,7 +488,7 @@ def rope_table(position_ids, rows: int, head_dim: int, base: float = 10000.0, de
         return _new_rope_table(position_ids, rows, head_dim, base, device, inv_freq)
     key = (version, rows, head_dim, float(base), str(device), _stream())
     last = _ROPE_TABLE_LAST
-    if last is not None and last[0] is position_ids and last[1] == key:
+    if last is not None and last[0] is position_ids and last[1] == key and _recordable(last[2]):
         return last[2]
     table = _new_rope_table(position_ids, rows, head_dim, base, device)
     _ROPE_TABLE_LAST = (position_ids, key, table)   # holding position_ids keeps its identity from being reused

@@ -523,6 +523,31 @@ def test_rope_table_neither_comes_from_nor_outlives_a_capture(fake_rope_kernel, 
     assert captured is not before and after is not captured
 
 
+def test_rope_table_of_an_evaluation_is_not_kept_for_training(fake_rope_kernel):
+    """One position tensor for an evaluation under inference_mode and the training step behind it: autograd keeps the step's table,
+    which it refuses for one made under that mode."""
+    from odysseus_transformer_amd import ops
+
+    class Keeps(torch.autograd.Function):
+        @staticmethod
+        def forward(ctx, x, pos):
+            ctx.save_for_backward(ops.rope_table(pos, 1, 128))
+            return x.clone()
+
+        @staticmethod
+        def backward(ctx, dy):
+            return dy, None
+
+    pos, x = torch.tensor([[5]]), torch.zeros(1, requires_grad=True)
+    with torch.inference_mode():
+        assert ops.rope_table(pos, 1, 128) is ops.rope_table(pos, 1, 128)
+    Keeps.apply(x, pos).backward()
+    t = ops.rope_table(pos, 1, 128)
+    with torch.inference_mode():
+        assert ops.rope_table(pos, 1, 128) is t
+    assert fake_rope_kernel == [[5], [5]]
+
+
 @pytest.mark.parametrize("pos", [torch.tensor([[5]]), torch.arange(2)[None], torch.arange(4.0)[None], torch.arange(4)[:, None]],
                          ids=["one for all", "half", "float", "column"])
 def test_cached_path_refuses_positions_that_do_not_cover_its_tokens(pos, fake_rope_kernel, monkeypatch):
