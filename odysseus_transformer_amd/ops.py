@@ -1034,6 +1034,8 @@ class LinearRoPEFunc(torch.autograd.Function):
             check_position_ids(position_ids, B, L, x.device)
         # evaluated on every call, as rope_ does: behind a cache the positions are new with every token
         table = _new_rope_table(position_ids, B * L, head_dim, rope_base, x.device)
+        if ctx is not _NO_CONTEXT and position_ids is not None and not _recordable(position_ids):
+            position_ids = position_ids.clone()
         ctx.save_for_backward(x2, weight, position_ids)
         ctx.dims = (n_rot, rope_base, x.shape)
         return linear_rope(x2, weight, table, n_rot, head_dim).view(B, L, -1, head_dim)

@@ -510,6 +510,23 @@ def test_cached_path_evaluates_its_positions_on_every_call(fake_rope_kernel, mon
     assert fake_rope_kernel == [[5], [6]]
 
 
+def test_cached_path_records_positions_made_under_inference_mode(fake_rope_kernel, monkeypatch):
+    """A position tensor of an inference program serves a training step too, and the backward turns by what it held in the forward."""
+    from odysseus_transformer_amd import ops
+    monkeypatch.setattr(ops, "linear_rope", lambda x, w, table, n_rot, head_dim: table.clone())
+    monkeypatch.setattr(ops, "gemm", lambda op, a, b: torch.zeros_like(a))
+    turned = []
+    monkeypatch.setattr(ops, "rope_", lambda d, n_rot, pos, base, inverse: turned.append(pos.item()))
+    with torch.inference_mode():
+        pos = torch.tensor([[5]])
+    x, w = torch.zeros(1, 1, 128, requires_grad=True), torch.zeros(128, 128)
+    y = ops.run_function(ops.LinearRoPEFunc, x, w, 1, 128, pos, 10000.0)
+    with torch.inference_mode():
+        pos += 1
+    y.sum().backward()
+    assert y[0, 0, 0, 0] == 5 and turned == [5]
+
+
 def test_rope_table_neither_comes_from_nor_outlives_a_capture(fake_rope_kernel, monkeypatch):
     """A replay must evaluate the positions of its own time, and a table that a capture recorded holds nothing yet."""
     from odysseus_transformer_amd import ops
