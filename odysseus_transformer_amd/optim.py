@@ -70,11 +70,17 @@ class AdamW(torch.optim.Optimizer):
                     state["exp_avg_sq"] = torch.zeros_like(p, memory_format=torch.preserve_format)
                 row = (p.data_ptr(), g.data_ptr(), state["exp_avg"].data_ptr(), state["exp_avg_sq"].data_ptr(), p.numel(),
                        int(state["step"].item()) + 1, state["step"])
-                if copied:   # used at once, so that no two copies are held
+                waiting = batches.setdefault((p.device, p.dtype), [])
+                if copied:   # used at once, so that no two copies are held; behind earlier parameters over the same memory
+                    size = p.element_size()
+                    if any(row[0] < r[0] + r[4] * size and r[0] < row[0] + row[4] * size for r in waiting):
+                        update(p.device, p.dtype, waiting)
+                        waiting.clear()
                     update(p.device, p.dtype, [row])
                     del g
                 else:
-                    batches.setdefault((p.device, p.dtype), []).append(row)
+                    waiting.append(row)
             for (device, dtype), rows in batches.items():
-                update(device, dtype, rows)
+                if rows:
+                    update(device, dtype, rows)
         return loss

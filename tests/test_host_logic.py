@@ -687,3 +687,15 @@ def test_adamw_holds_one_converted_gradient_at_a_time(adamw_on_cpu, monkeypatch)
     AdamW([parameter((8,)), strided[0], parameter((16,)), *strided[1:]]).step()
     assert alive == [0, 0, 0]
     assert sorted(args[6] for args in calls) == [1, 1, 1, 2]   # tensors per call
+
+
+def test_adamw_keeps_the_order_of_parameters_over_the_same_memory(adamw_on_cpu):
+    """A parameter whose gradient must be copied follows an earlier one that shares its memory; others do not hold it up."""
+    from odysseus_transformer_amd.optim import AdamW
+    calls, parameter = adamw_on_cpu
+    strided = lambda: torch.ones(6, 4, dtype=torch.bfloat16).t()  # noqa: E731
+    apart, first, second = parameter((4, 6), strided()), parameter((4, 6)), parameter((4, 6), strided())
+    second.data = first.data
+    AdamW([parameter((8,)), first, apart, second, parameter((16,))]).step()
+    assert [list(args[0]) for args in calls][0] == [apart.data_ptr()]
+    assert [args[6] for args in calls] == [1, 2, 1, 1] and calls[1][0][1] == calls[2][0][0] == first.data_ptr()
