@@ -594,9 +594,12 @@ def test_attention_hd64(case, spread, dev):
     grads = ops.attn_bwd(qg, kg, vg, o, lse, dog, causal=causal)
     floor = 1.0 if Lk == 1 else 1e-3
     assert_parity(grads[2], dv_ref, TOL_BF16, "dv")
-    if spread == 1.0:   # one-hot rows leave dS = P (dP - delta) with nothing but the rounding of out
-        assert_parity(grads[0], dq_ref, TOL_BF16, "dq", floor)
-        assert_parity(grads[1], dk_ref, TOL_BF16, "dk", floor)
+    if spread > 1.0:
+        # one-hot rows leave dS = P (dP - delta) with little but the rounding of out: the oracle gets out and lse as the kernels
+        # had them.  Then P and dS in bf16, dP and lse off by 1e-6 come to 8e-3 in a plain emulation of all these cases
+        dq_ref, dk_ref, _ = oracle.attention_bwd(q.float(), k.float(), v.float(), o.float().cpu(), lse.cpu(), do.float(), causal=causal)
+    assert_parity(grads[0], dq_ref, TOL_BF16, "dq", floor)
+    assert_parity(grads[1], dk_ref, TOL_BF16, "dk", floor)
     again = (*ops.attn_fwd(qg, kg, vg, causal=causal), *ops.attn_bwd(qg, kg, vg, o, lse, dog, causal=causal))
     for a, b in zip((o, lse, *grads), again):
         assert torch.equal(a, b)
