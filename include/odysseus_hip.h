@@ -221,9 +221,10 @@ int ody_gemm(int op, const void* A, const void* B, void* C, const void* bias,
  *                         backward of decoder/odysseus.py:295; dh itself is never stored.  workspace:
  *                         ody_linear_dgrad_swiglu_workspace_bytes(...) bytes (0 when the shape takes the fused
  *                         kernel; otherwise room for dh), 16-byte aligned.  The query goes by the shape alone and
- *                         assumes 16-byte aligned pointers and leading dimensions that are multiples of 8: operands
- *                         without them take the two-kernel path whatever the shape and need T * I elements of
- *                         workspace (the call returns ODY_ERR_WORKSPACE and says so if it is missing).
+ *                         assumes 16-byte aligned pointers and leading dimensions that are multiples of 8, below 2^22
+ *                         (dy) and 2^24 (w_down): operands without them take the two-kernel path whatever the shape
+ *                         and need T * I elements of workspace (the call returns ODY_ERR_WORKSPACE and says so if it
+ *                         is missing).
  */
 int ody_linear_residual(const void* x, const void* w, const void* residual, void* y, int M, int N, int K,
                         int64_t ldx, int64_t ldw, int64_t ld_res, int64_t ldy, int dtype, void* stream);

@@ -573,9 +573,10 @@ def linear_dgrad_swiglu(dy, w_down, gate_up):
                          f"{tuple(gate_up.shape)} {gate_up.dtype} do not fit")
     dgu = torch.empty((T, 2 * I), dtype=dy.dtype, device=dy.device)
     ws_bytes = _lib.load().ody_linear_dgrad_swiglu_workspace_bytes(T, I, K, _dt(dy))
-    if ws_bytes == 0 and any(t.data_ptr() % 16 or t.stride(0) % 8 for t in (dy, w_down, gate_up, dgu)):
-        # the size query goes by the shape alone; the one-kernel path also wants 16-byte aligned rows, and a
-        # column-sliced view without them takes the two-kernel path, which keeps dh (T, I) in a workspace
+    if ws_bytes == 0 and (any(t.data_ptr() % 16 or t.stride(0) % 8 for t in (dy, w_down, gate_up, dgu))
+                          or _rowmajor2d(dy, "dy") >= 1 << 22 or _rowmajor2d(w_down, "w_down") >= 1 << 24):
+        # the size query goes by the shape alone; the one-kernel path also wants 16-byte aligned rows and pitches inside its
+        # 32-bit offsets, and a column-sliced view without them takes the two-kernel path, which keeps dh (T, I) in a workspace
         ws_bytes = (T * I * dy.element_size() + 255) & ~255
     ws = scratch(ws_bytes, "dgrad_swiglu_workspace", dy.device) if ws_bytes else None
     _lib.call("ody_linear_dgrad_swiglu", dy.data_ptr(), w_down.data_ptr(), gate_up.data_ptr(), dgu.data_ptr(), T, I, K,

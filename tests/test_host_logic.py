@@ -699,3 +699,29 @@ def test_adamw_keeps_the_order_of_parameters_over_the_same_memory(adamw_on_cpu):
     AdamW([parameter((8,)), first, apart, second, parameter((16,))]).step()
     assert [list(args[0]) for args in calls][0] == [apart.data_ptr()]
     assert [args[6] for args in calls] == [1, 2, 1, 1] and calls[1][0][1] == calls[2][0][0] == first.data_ptr()
+
+
+@pytest.mark.parametrize("operand", ["dy", "w_down"])
+def test_swiglu_backward_of_pitches_beyond_the_tile_kernel_has_room_for_dh(operand, monkeypatch):
+    """Row pitches that the one-kernel path does not take run as two kernels, which keep dh (T, I) in the workspace: the size query, which
+    knows the shape alone, asks for none here."""
+    from odysseus_transformer_amd import _lib, ops
+    calls = []
+    monkeypatch.setattr(_lib, "call", lambda name, *a: calls.append(a))
+    monkeypatch.setattr(ops, "_need_gpu", lambda *t: None)
+    monkeypatch.setattr(ops, "_stream", lambda: 0)
+    T, K, I = 3, 64, 128
+    assert _lib.load().ody_linear_dgrad_swiglu_workspace_bytes(T, I, K, 0) == 0
+
+    def rows(n, width, pitch):
+        return torch.empty(n * pitch, dtype=torch.bfloat16, device="meta").as_strided((n, width), (pitch, 1))
+
+    def given(ld_dy, ld_w):
+        ops.linear_dgrad_swiglu(rows(T, K, ld_dy), rows(K, I, ld_w), rows(T, 2 * I, 2 * I))
+        return calls[-1][-2]
+
+    assert given(K, I) == 0
+    limit = 1 << (22 if operand == "dy" else 24)
+    below, at = ((limit - 8, I), (limit, I)) if operand == "dy" else ((K, limit - 8), (K, limit))
+    assert given(*below) == 0
+    assert given(*at) >= T * I * 2
