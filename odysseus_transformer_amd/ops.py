@@ -199,7 +199,6 @@ def attn_bwd(q, k, v, out, lse, dout, causal: bool = True, scale: Optional[float
     scale = 1.0 / math.sqrt(D) if scale is None else float(scale)
     lib = _lib.load()
     ws_bytes = lib.ody_attn_bwd_workspace_bytes(B, Lq, Lk, Hq, Hkv, D, _dt(q))
-    least = lib.ody_attn_bwd_workspace_least_bytes(B, Lq, Lk, Hq, Hkv, D, _dt(q))
     ds_bytes = lib.ody_attn_bwd_ds_bytes(B, Lq, Lk, Hq, Hkv, D, _dt(q), int(causal)) if keep_ds is not False else 0
     if keep_ds and ds_bytes == 0:
         raise ValueError(_KEEP_DS_SHAPES)
@@ -214,7 +213,10 @@ def attn_bwd(q, k, v, out, lse, dout, causal: bool = True, scale: Optional[float
                 _KEEP_DS_OOM[str(q.device)] = min(ds_bytes, _KEEP_DS_OOM.get(str(q.device), 1 << 62))
     if keep_ds:
         ws_bytes += ds_bytes
-        least += ds_bytes
+
+    def least():   # asked only where ws_bytes are not to be had
+        return lib.ody_attn_bwd_workspace_least_bytes(B, Lq, Lk, Hq, Hkv, D, _dt(q)) + (ds_bytes if keep_ds else 0)
+
     if workspace is None:
         if reuse_query_side:
             raise ValueError("reuse_query_side needs the workspace of the previous call")
@@ -222,8 +224,9 @@ def attn_bwd(q, k, v, out, lse, dout, causal: bool = True, scale: Optional[float
             ws = _scratch_or_least(ws_bytes, least, lambda n: scratch(n, "attn_bwd_workspace", q.device))
     else:
         ws = workspace
-        if ws.dtype != torch.uint8 or ws.numel() < least or ws.device != q.device or not ws.is_contiguous():
-            raise ValueError(f"workspace must be a contiguous uint8 tensor of at least {least} bytes on {q.device}")
+        if ws.dtype != torch.uint8 or ws.device != q.device or not ws.is_contiguous() or \
+                (ws.numel() < ws_bytes and ws.numel() < least()):
+            raise ValueError(f"workspace must be a contiguous uint8 tensor of at least {least()} bytes on {q.device}")
     ws_bytes = ws.numel()
     flags = (_lib.BWD_ACCUMULATE_DQ if accumulate_dq else 0) | (_lib.BWD_DQ_F32 if dq_f32 else 0) | \
             (_lib.BWD_REUSE_QUERY_SIDE if reuse_query_side else 0) | (_lib.BWD_KEEP_DS if keep_ds else 0)
@@ -248,14 +251,14 @@ def attn_bwd(q, k, v, out, lse, dout, causal: bool = True, scale: Optional[float
     return dq, dk, dv
 
 
-def _scratch_or_least(nbytes: int, least: int, allocate) -> torch.Tensor:
-    """allocate(nbytes), or allocate(least) where that much memory is not there and the kernels can do with less."""
+def _scratch_or_least(nbytes: int, least, allocate) -> torch.Tensor:
+    """allocate(nbytes), or allocate(least()) where that much memory is not there and the kernels can do with less."""
     try:
         return allocate(nbytes)
     except torch.OutOfMemoryError:
-        if least >= nbytes:
+        if least() >= nbytes:
             raise
-    return allocate(least)
+    return allocate(least())
 
 
 _KEEP_DS_MAX_BYTES: Optional[int] = None
@@ -354,8 +357,8 @@ def _shared_bwd_workspace(calls):
             return torch.empty(n, dtype=torch.uint8, device=device), keeps
         except torch.OutOfMemoryError:
             _KEEP_DS_OOM[str(device)] = min(failed, min(d for d, kp in zip(ds, keeps) if kp))
-    least = max(lib.ody_attn_bwd_workspace_least_bytes(*d) for d in dims)
-    ws = _scratch_or_least(max(base), least, lambda n: torch.empty(n, dtype=torch.uint8, device=device))
+    ws = _scratch_or_least(max(base), lambda: max(lib.ody_attn_bwd_workspace_least_bytes(*d) for d in dims),
+                           lambda n: torch.empty(n, dtype=torch.uint8, device=device))
     return ws, [False] * len(calls)
 
 
