@@ -25,6 +25,10 @@
 // shape the vector pipe is 70 % and the matrix pipe 46 % busy in the forward (16 % of the units' time is the causal tail), matrix 52 %
 // and vector 45 % in dK/dV and dQ at 2.0 GHz.  Without effect: raised priority around the matrix steps, two wavefronts a SIMD
 // instead of three in the backward.
+//
+// Error of the forward against 64 bits, standard normal inputs (running maximum / first tile's): 16 heads, L = 4096, causal 2.05e-3 /
+// 2.11e-3; L = 700, full 2.21e-3 / 2.31e-3.  The roundings are the same ones; bf16 is finest just below a power of two, and that is
+// where the largest P of a row lie if the reference is its maximum (an emulation in 64 bits that rounds P and out gives these figures).
 #include <type_traits>
 #include <utility>
 #include "attn_params.h"

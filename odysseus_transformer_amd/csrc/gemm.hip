@@ -403,8 +403,9 @@ struct F32Tile {
 // rows.
 // Bound by the fp32 matrix rate where blocks are many (0.50 us per slab and block, 0.43 at 2.4 GHz), by latency where they are few.
 // Measured against one slab in LDS and one in registers, loaded behind bounds checks that made every wait one for all loads: NT / NN
-// / TN 4096^3 130 / 127 / 128 -> 136 / 137 / 136 TFLOP/s; 2048 x 2752 x 512 NT 63 -> 53 us, 2048 x 1536 x 512 33 -> 30; 2752 x 512 x
-// 2048 TN 66 -> 58.  With the bounds checks left in, the deeper pipeline alone was 2 % slower than none.
+// / TN 4096^3 130 / 127 / 128 -> 136 / 137 / 136 TFLOP/s in loops of 30 calls and more (three calls behind one, by the wall clock: 111 /
+// 118 / 122); 2048 x 2752 x 512 NT 63 -> 53 us, 2048 x 1536 x 512 33 -> 30; 2752 x 512 x 2048 TN 66 -> 58.  With the bounds checks left
+// in, the deeper pipeline alone was 2 % slower than none.
 // gridDim.y > 1: block y takes the y-th range of slabs and writes fp32 partial results to part[y][M][N] (VEC only).
 // VEC = false (unaligned pointers, or a contiguous extent that is no multiple of 4) moves single floats.
 template <int WT, bool A_KC, bool B_KC, bool VEC>

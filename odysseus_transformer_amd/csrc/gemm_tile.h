@@ -24,8 +24,10 @@
 //
 // Bound: the package power limit.  With constant operands the NT instance sustains 2170 TFLOP/s (4096 x 4096 x 11008, 87 % of
 // the matrix peak), with random ones 1500.  Measured against the kernel it replaced (4 wavefronts, operands staged through
-// registers), TFLOP/s, 8192^3 / 4096 x 4096 x 11008: NT 1305 -> 1450 / 1347 -> 1520, NN 1283 -> 1443 / 1343 -> 1500, TN
-// 1266 -> 1376 / 1265 -> 1398.
+// registers), TFLOP/s in loops of 30 calls and more, 8192^3 / 4096 x 4096 x 11008: NT 1305 -> 1450 / 1347 -> 1520, NN 1283 ->
+// 1443 / 1343 -> 1500, TN 1266 -> 1376 / 1265 -> 1398 (another box: 1565 / 1545, 1506 / 1500, 1402 / 1400; torch.matmul there, NT,
+// 1614 / 1600).  A call between two events of its own shows the launch and the clock's way up as well: the second NT product
+// 1320 right after idling (torch.matmul 1300 to 1550), 1480 once the card has worked for a second (1470).
 #pragma once
 #include "gemm_epi.h"
 
