@@ -582,8 +582,10 @@ Walk walk(const AttnParams& p, bool own_keys) {
 // at 0.9 per tile, and behind a causal mask's longest walk most of the unit idles at head_dim 64 (three workgroups share one) and
 // little at 128 (one each).  A round of 256 split workgroups costs its start and end and 0.32 (head_dim 128: 0.34) per tile, and
 // no less than one tile for each wavefront.  Fitted to 1100 shapes of 32 to 16384 rows and tokens, 1 to 256 heads, both masks:
-// never slower than the whole instance by more than 2 us, and 0.2 % off the better one in the mean.  Beyond 1024 whole
-// workgroups it was not measured.
+// never slower than the whole instance by more than 2 us, and 0.2 % off the better one in the mean.  From 1024 whole workgroups on these
+// are ahead, whole / split in us: 8 x 64, L = 16384, causal 2443 / 2629 forward, 4731 / 4955 dK / dV (dQ 3684 / 3522, the one exception
+// of 42 timed); 2 x 16 x 64, L = 4096, causal 612 / 735, 1192 / 1351, dQ 928 / 975; 8 x 32 x 64, L = 512, causal 96 / 195, 194 / 323,
+// 155 / 249; 32 x 128, L = 4096, causal 1277 / 1641 forward, dQ 1813 / 2116.
 template <int D>
 bool few_rows(int rows, int heads, Walk w) {
   constexpr double start = D == 64 ? 1.0 : 1.6, tile = D == 64 ? 0.32 : 0.34, idle = D == 64 ? 0.9 : 0.2;
