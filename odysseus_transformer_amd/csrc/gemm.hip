@@ -1,13 +1,9 @@
 // Dense linears: C (M, N) = op(A) . op(B) for the three products of a linear
-// layer (forward NT, dgrad NN, wgrad TN): the choice of a kernel and a plan, the entry points, and the fp32 kernel.
+// layer (forward NT, dgrad NN, wgrad TN): the choice of a kernel and a plan, and the entry points.
 //
 // bf16 products run on gemm_tile.h (LDS tiles) or gemm_skinny.hip (few rows); the small kernel below only takes matrices whose
-// row pitch does not fit those kernels' 32-bit tile offsets.
-//
-// fp32 (its 1e-4 tolerance rules out bf16 inputs): v_mfma_f32_32x32x2_f32 on
-// 64 x 64 or 128 x 128 workgroup tiles, any shape and alignment.
+// row pitch does not fit those kernels' 32-bit tile offsets.  fp32 products: gemm_f32.hip.
 #include <algorithm>
-#include <type_traits>
 #include "gemm_tile.h"
 
 namespace {
@@ -321,305 +317,11 @@ int gemm_bf16(int op, const bf16* A, const bf16* B, bf16* C, const bf16* bias, c
   return ody_check_launch("gemm_splitk_sum");
 }
 
-// ------------------------------------------------------------------ fp32 MFMA
-constexpr int FK = 32;  // K-slab of the fp32 kernel
-// largest row pitch (exclusive) whose byte offsets inside a slab, 128 rows or 32 rows of K, stay below 2^31
-constexpr int64_t f32_max_pitch(bool kc) { return (int64_t)1 << (kc ? 22 : 24); }
-
-__device__ __forceinline__ f32x16 mfma_f32(float a, float b, f32x16 c) {
-  return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
-}
-
-// One operand slab (BT rows x FK of K) on its way from global memory to LDS and out again as
-// MFMA fragments.  KC = true: memory is (rows, K) row-major, LDS [BT][FK + 4], a fragment is one
-// 16-byte read.  KC = false: memory is (K, rows) row-major, LDS [FK][BT + 8], a fragment is four
-// 4-byte reads.  Either way k-step 4 j + t of lane half g multiplies K index 8 j + 4 g + t, so
-// both operands of a product agree, and both pitches keep the reads conflict-free.
-template <int BT, bool KC>
-struct F32Tile {
-  static constexpr int PITCH = KC ? FK + 4 : BT + 8;
-  static constexpr int ELEMS = (KC ? BT : FK) * PITCH;
-  static constexpr int CHUNKS = BT * FK / 4 / 256;  // 16-byte pieces per thread
-  f32x4 r[CHUNKS];
-
-  static __device__ __forceinline__ void coord(int c, int& rr, int& kk) {
-    if (KC) { rr = c / (FK / 4); kk = (c % (FK / 4)) * 4; }
-    else { kk = c / (BT / 4); rr = (c % (BT / 4)) * 4; }
-  }
-  // Byte offset of piece j in the slab, beyond the buffer's range for a row past the end.  Pitches below f32_max_pitch.
-  static __device__ __forceinline__ unsigned offset(int j, int64_t ld, int row0, int nrows, int tid) {
-    int rr, kk;
-    coord(tid + 256 * j, rr, kk);
-    return row0 + rr < nrows ? 4u * (unsigned)(KC ? rr * (int)ld + kk : kk * (int)ld + rr) : gemm_tile::PAST_END;
-  }
-  // Vectors, without a branch: behind one the compiler loses count of the loads in flight and waits for all of them.
-  __device__ __forceinline__ void gload_vec(const float* base, int64_t ld, const unsigned (&off)[CHUNKS], int row0, int k0, int K, int tid) {
-    auto rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(base + (KC ? (int64_t)row0 * ld + k0 : (int64_t)k0 * ld + row0)), 0,
-                                                  0x7fffffff, 0x00020000);
-#pragma unroll
-    for (int j = 0; j < CHUNKS; j++) {
-      int rr, kk;
-      coord(tid + 256 * j, rr, kk);
-      r[j] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, k0 + kk < K ? off[j] : gemm_tile::PAST_END, 0, 0));
-    }
-  }
-  // Single floats.  row0: first row (M or N index) of the tile; k0: first K index; out-of-range elements read as 0
-  __device__ __forceinline__ void gload(const float* base, int64_t ld, int row0, int k0, int nrows, int K, int tid) {
-#pragma unroll
-    for (int j = 0; j < CHUNKS; j++) {
-      int rr, kk;
-      coord(tid + 256 * j, rr, kk);
-      const int row = row0 + rr, k = k0 + kk;
-      const float* src = KC ? base + (int64_t)row * ld + k : base + (int64_t)k * ld + row;
-#pragma unroll
-      for (int e = 0; e < 4; e++) {
-        const bool ok = KC ? (row < nrows && k + e < K) : (row + e < nrows && k < K);
-        r[j][e] = ok ? src[e] : 0.f;
-      }
-    }
-  }
-  __device__ __forceinline__ void put(float* lds, int tid) const {
-#pragma unroll
-    for (int j = 0; j < CHUNKS; j++) {
-      int rr, kk;
-      coord(tid + 256 * j, rr, kk);
-      *reinterpret_cast<f32x4*>(lds + (KC ? rr * PITCH + kk : kk * PITCH + rr)) = r[j];
-    }
-  }
-  // k-steps 4 j .. 4 j + 3 of row r0 + i
-  static __device__ __forceinline__ f32x4 frag(const float* lds, int r0, int i, int g, int j) {
-    if (KC) return *reinterpret_cast<const f32x4*>(lds + (r0 + i) * PITCH + 8 * j + 4 * g);
-    f32x4 v;
-#pragma unroll
-    for (int t = 0; t < 4; t++) v[t] = lds[(8 * j + 4 * g + t) * PITCH + r0 + i];
-    return v;
-  }
-};
-
-// v_mfma_f32_32x32x2_f32, 4 wavefronts in a 2 x 2 arrangement, each owning WT x WT result tiles
-// of 32 x 32 (a 64 x 64 or 128 x 128 workgroup tile).  Two slabs in LDS and two on their way in registers, so that a slab has two
-// others to land behind and one barrier suffices; the fragments of the next four k-steps are read while four are multiplied.  The
-// product is computed as C^T = op(B)^T op(A)^T, so a lane holds 4 consecutive N per register quad and writes 16-byte pieces of C
-// rows.
-// Bound by the fp32 matrix rate where blocks are many (0.50 us per slab and block, 0.43 at 2.4 GHz), by latency where they are few.
-// Measured against one slab in LDS and one in registers, loaded behind bounds checks that made every wait one for all loads: NT / NN
-// / TN 4096^3 130 / 127 / 128 -> 136 / 137 / 136 TFLOP/s in loops of 30 calls and more (three calls behind one, by the wall clock: 111 /
-// 118 / 122); 2048 x 2752 x 512 NT 63 -> 53 us, 2048 x 1536 x 512 33 -> 30; 2752 x 512 x 2048 TN 66 -> 58.  With the bounds checks left
-// in, the deeper pipeline alone was 2 % slower than none.
-// gridDim.y > 1: block y takes the y-th range of slabs and writes fp32 partial results to part[y][M][N] (VEC only).
-// VEC = false (unaligned pointers, or a contiguous extent that is no multiple of 4) moves single floats.
-template <int WT, bool A_KC, bool B_KC, bool VEC>
-__global__ __launch_bounds__(256, WT == 1 ? 4 : 2) void gemm_f32_kernel(const float* __restrict__ A, const float* __restrict__ B, float* C,
-                                                            const float* __restrict__ bias, int M, int N, int K, int64_t lda,
-                                                            int64_t ldb, int64_t ldc, const float* add, int64_t ld_add, int ntn, float* part) {
-  constexpr int BT = 64 * WT;
-  constexpr int NCH = (WT == 1) ? 2 : 1;  // never a single chain of dependent MFMAs
-  using TA = F32Tile<BT, A_KC>;
-  using TB = F32Tile<BT, B_KC>;
-  __shared__ __attribute__((aligned(16))) float As[2][TA::ELEMS];
-  __shared__ __attribute__((aligned(16))) float Bs[2][TB::ELEMS];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, i = lane & 31, g = lane >> 5;
-  const int wm = wave >> 1, wn = wave & 1;
-  const int m0 = (blockIdx.x / ntn) * BT, n0 = (blockIdx.x % ntn) * BT;
-
-  f32x16 acc[WT][WT][NCH];
-#pragma unroll
-  for (int a = 0; a < WT; a++)
-#pragma unroll
-    for (int b = 0; b < WT; b++)
-#pragma unroll
-      for (int c = 0; c < NCH; c++)
-#pragma unroll
-        for (int r = 0; r < 16; r++) acc[a][b][c][r] = 0.f;
-
-  TA ta[2];
-  TB tb[2];
-  int k_first = 0, k_last = K;
-  if (VEC && part) {
-    const int per = ((K + FK - 1) / FK + (int)gridDim.y - 1) / (int)gridDim.y * FK;
-    k_first = min((int)blockIdx.y * per, K), k_last = min(k_first + per, K);
-  }
-  unsigned oa[TA::CHUNKS], ob[TB::CHUNKS];
-  if (VEC) {
-#pragma unroll
-    for (int j = 0; j < TA::CHUNKS; j++) oa[j] = TA::offset(j, lda, m0, M, tid);
-#pragma unroll
-    for (int j = 0; j < TB::CHUNKS; j++) ob[j] = TB::offset(j, ldb, n0, N, tid);
-  }
-  auto fetch = [&](int set, int k0) {   // past K: zeros, nothing is read
-    if (VEC) {
-      ta[set].gload_vec(A, lda, oa, m0, k0, K, tid);
-      tb[set].gload_vec(B, ldb, ob, n0, k0, K, tid);
-    } else {
-      ta[set].gload(A, lda, m0, k0, M, K, tid);
-      tb[set].gload(B, ldb, n0, k0, N, K, tid);
-    }
-  };
-  auto put = [&](int set) {
-    ta[set].put(As[set], tid);
-    tb[set].put(Bs[set], tid);
-  };
-  fetch(0, k_first);
-  fetch(1, k_first + FK);
-  put(0);
-  // the slab at k0, in LDS set `cur`; the one behind it goes from registers to the other set, the one after that sets out
-  auto slab = [&](auto which, int k0) {
-    constexpr int cur = decltype(which)::value;
-    __syncthreads();
-    f32x4 af[2][WT], bf[2][WT];
-    auto frags = [&](int j) {
-#pragma unroll
-      for (int a = 0; a < WT; a++) af[j & 1][a] = TA::frag(As[cur], 32 * (wm * WT + a), i, g, j);
-#pragma unroll
-      for (int b = 0; b < WT; b++) bf[j & 1][b] = TB::frag(Bs[cur], 32 * (wn * WT + b), i, g, j);
-    };
-    frags(0);
-    fetch(cur, k0 + 2 * FK);
-#pragma unroll
-    for (int j = 0; j < FK / 8; j++) {
-      // the next fragments are on their way while these are multiplied
-      if (j + 1 < FK / 8) frags(j + 1);
-      else put(cur ^ 1);
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int t = 0; t < 4; t++)
-#pragma unroll
-        for (int a = 0; a < WT; a++)
-#pragma unroll
-          for (int b = 0; b < WT; b++)
-            acc[a][b][t % NCH] = mfma_f32(bf[j & 1][b][t], af[j & 1][a][t], acc[a][b][t % NCH]);
-      __builtin_amdgcn_sched_barrier(0);
-    }
-  };
-  int k0 = k_first;
-  for (; k0 + FK < k_last; k0 += 2 * FK) {
-    slab(std::integral_constant<int, 0>{}, k0);
-    slab(std::integral_constant<int, 1>{}, k0 + FK);
-  }
-  if (k0 < k_last) slab(std::integral_constant<int, 0>{}, k0);
-  // register r of lane (i, g) of tile (a, b): row m = 32 (wm WT + a) + i, column n = 32 (wn WT + b) + 8 (r / 4) + 4 g + r % 4
-#pragma unroll
-  for (int a = 0; a < WT; a++) {
-    const int m = m0 + 32 * (wm * WT + a) + i;
-    if (m >= M) continue;
-#pragma unroll
-    for (int b = 0; b < WT; b++) {
-      f32x16 v = acc[a][b][0];
-      if (NCH == 2) v += acc[a][b][NCH - 1];
-#pragma unroll
-      for (int q = 0; q < 4; q++) {
-        const int n = n0 + 32 * (wn * WT + b) + 8 * q + 4 * g;
-        if (VEC && part) {
-          if (n < N)
-            *reinterpret_cast<f32x4*>(part + ((int64_t)blockIdx.y * M + m) * N + n) = f32x4{v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]};
-          continue;
-        }
-        float* dst = C + (int64_t)m * ldc + n;
-        if (VEC && n + 3 < N) {
-          f32x4 o{v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]};
-          if (bias) o += *reinterpret_cast<const f32x4*>(bias + n);
-          if (add) o += *reinterpret_cast<const f32x4*>(add + (int64_t)m * ld_add + n);
-          *reinterpret_cast<f32x4*>(dst) = o;
-        } else {
-#pragma unroll
-          for (int e = 0; e < 4; e++) {
-            if (n + e >= N) continue;
-            float o = v[4 * q + e];
-            if (bias) o += bias[n + e];
-            if (add) o += add[(int64_t)m * ld_add + n + e];
-            dst[e] = o;
-          }
-        }
-      }
-    }
-  }
-}
-
-// C (+)= sum of the fp32 partial results (+ bias); 4 elements per thread
-__global__ __launch_bounds__(256) void gemm_f32_sum_kernel(const float* __restrict__ part, int splits, float* C,
-                                                           const float* __restrict__ bias, int M, int N, int64_t ldc, const float* add,
-                                                           int64_t ld_add) {
-  const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (idx >= (int64_t)M * (N / 4)) return;
-  const int m = idx / (N / 4), n = (idx % (N / 4)) * 4;
-  f32x4 v = sum_parts(part, splits, (int64_t)M * N, (int64_t)m * N + n);
-  if (bias) v += *reinterpret_cast<const f32x4*>(bias + n);
-  f32x4* dst = reinterpret_cast<f32x4*>(C + (int64_t)m * ldc + n);
-  if (add) v += *reinterpret_cast<const f32x4*>(add + (int64_t)m * ld_add + n);
-  *dst = v;
-}
-
-// Tile and ranges of K of an fp32 product: 128 x 128 tiles once they fill the chip twice over, 64 x 64 tiles below that.  A lone
-// block of 4 wavefronts on a compute unit waits a third of the time (0.74 us per slab of 32 k), several blocks fill
-// each other's gaps (0.50 us per block and slab), so a long K is cut into ranges until the blocks outnumber the units a few times
-// -- as far as the trip of the partial results through memory pays for it.  (Weight gradients over 2048 tokens, us without / with
-// ranges, before the deeper pipeline: 2752 x 512 85 / 76, 1536 x 512 54 / 45, 512 x 512 51 / 20.  Sharing a tile's slabs between four times the wavefronts
-// of one block, or K over eight independent ones, took as long as the ranges.)
-struct PlanF32 { int tile, splits; };
-PlanF32 plan_f32(int M, int N, int K) {
-  const int64_t big = (int64_t)((M + 127) / 128) * ((N + 127) / 128), small = (int64_t)((M + 63) / 64) * ((N + 63) / 64);
-  if (big >= 512) return PlanF32{128, 1};
-  const int slabs = (K + FK - 1) / FK;
-  PlanF32 best{64, 1};
-  double best_us = 1e30;
-  for (int s = 1; s <= 16 && slabs >= 4 * s; s++) {
-    const double per_cu = (double)((small * s + 255) / 256);
-    double us = (slabs + s - 1) / s * std::max(0.74, 0.50 * per_cu);
-    if (s > 1) us += 3.0 + (double)s * M * N * 8.0 / 5.0e6;
-    if (us < best_us) best_us = us, best.splits = s;
-  }
-  return best;
-}
-
-template <int WT, bool A_KC, bool B_KC>
-int launch_f32(const float* a, const float* b, float* c, const float* bias, int M, int N, int K, int64_t lda,
-               int64_t ldb, int64_t ldc, const float* add, int64_t ld_add, bool vec, int splits, float* part, hipStream_t st) {
-  constexpr int BT = 64 * WT;
-  const int64_t ntm = (M + BT - 1) / BT, ntn = (N + BT - 1) / BT;
-  ODY_REQUIRE(ntm * ntn < ((int64_t)1 << 31), ODY_ERR_BAD_SHAPE, "ody_gemm: M=%d N=%d too large for one launch", M, N);
-  const dim3 grid((unsigned)(ntm * ntn), splits), blk(256);
-  if (vec)
-    ODY_LAUNCH("gemm_f32", st, (gemm_f32_kernel<WT, A_KC, B_KC, true>), grid, blk, 0, a, b, c, bias, M, N, K, lda,
-               ldb, ldc, add, ld_add, (int)ntn, part);
-  else
-    ODY_LAUNCH("gemm_f32", st, (gemm_f32_kernel<WT, A_KC, B_KC, false>), grid, blk, 0, a, b, c, bias, M, N, K, lda,
-               ldb, ldc, add, ld_add, (int)ntn, part);
-  int rc = ody_check_launch("gemm_f32");
-  if (rc || splits == 1) return rc;
-  const int64_t n4 = (int64_t)M * (N / 4);
-  ODY_LAUNCH("gemm_f32_sum", st, gemm_f32_sum_kernel, dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, part, splits, c, bias, M, N, ldc,
-             add, ld_add);
-  return ody_check_launch("gemm_f32_sum");
-}
-
-template <bool A_KC, bool B_KC>
-int dispatch_f32(const float* a, const float* b, float* c, const float* bias, int M, int N, int K, int64_t lda,
-                 int64_t ldb, int64_t ldc, const float* add, int64_t ld_add, void* workspace, size_t workspace_bytes, hipStream_t st) {
-  const bool vec = ody_aligned16(a) && ody_aligned16(b) && ody_aligned16(c) && (!bias || ody_aligned16(bias)) &&
-                   lda < f32_max_pitch(A_KC) && ldb < f32_max_pitch(B_KC) && lda % 4 == 0 && ldb % 4 == 0 && ldc % 4 == 0 && (!add || (ody_aligned16(add) && ld_add % 4 == 0)) && N % 4 == 0 && (A_KC ? K : M) % 4 == 0 && (!B_KC || K % 4 == 0);
-  PlanF32 pl = plan_f32(M, N, K);
-  if (pl.splits > 1 && (!vec || !workspace || !ody_aligned16(workspace) || workspace_bytes < (size_t)pl.splits * M * N * sizeof(float)))
-    pl.splits = 1;
-  float* part = pl.splits > 1 ? static_cast<float*>(workspace) : nullptr;
-  if (pl.tile == 128) return launch_f32<2, A_KC, B_KC>(a, b, c, bias, M, N, K, lda, ldb, ldc, add, ld_add, vec, 1, nullptr, st);
-  return launch_f32<1, A_KC, B_KC>(a, b, c, bias, M, N, K, lda, ldb, ldc, add, ld_add, vec, pl.splits, part, st);
-}
-
-int gemm_f32(int op, const float* a, const float* b, float* c, const float* bias, int M, int N, int K, int64_t lda, int64_t ldb,
-             int64_t ldc, const float* add, int64_t ld_add, void* workspace, size_t workspace_bytes, hipStream_t st) {
-  if (op == ODY_GEMM_NT) return dispatch_f32<true, true>(a, b, c, bias, M, N, K, lda, ldb, ldc, add, ld_add, workspace, workspace_bytes, st);
-  if (op == ODY_GEMM_NN) return dispatch_f32<true, false>(a, b, c, bias, M, N, K, lda, ldb, ldc, add, ld_add, workspace, workspace_bytes, st);
-  return dispatch_f32<false, false>(a, b, c, bias, M, N, K, lda, ldb, ldc, add, ld_add, workspace, workspace_bytes, st);
-}
-
 }  // namespace
 
 extern "C" size_t ody_gemm_workspace_bytes(int op, int M, int N, int K, int dtype) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
-  if (dtype == ODY_F32) {
-    const int splits = plan_f32(M, N, K).splits;
-    return splits > 1 ? (size_t)splits * M * N * sizeof(float) : 0;
-  }
+  if (dtype == ODY_F32) return ody_gemm_f32_workspace(M, N, K);
   if (dtype != ODY_BF16) return 0;
   if (op == ODY_GEMM_NT && ody_gemm_skinny_ok(EPI_NONE, M, N)) return 0;
   const int splits = plan_bf16(M, N, K, true).splits;
@@ -638,7 +340,7 @@ extern "C" int ody_gemm(int op, const void* A, const void* B, void* C, const voi
               (long long)ldb, (long long)ldc);
   hipStream_t st = static_cast<hipStream_t>(stream);
   if (dtype == ODY_F32)
-    return gemm_f32(op, (const float*)A, (const float*)B, (float*)C, (const float*)bias, M, N, K, lda, ldb, ldc,
+    return ody_launch_gemm_f32(op, (const float*)A, (const float*)B, (float*)C, (const float*)bias, M, N, K, lda, ldb, ldc,
                     accumulate ? (const float*)C : nullptr, ldc, workspace, workspace_bytes, st);
   ODY_REQUIRE(dtype == ODY_BF16, ODY_ERR_UNSUPPORTED, "ody_gemm: dtype %d unknown", dtype);
   // 16-byte vectors along the contiguous direction of every matrix
@@ -734,7 +436,7 @@ extern "C" int ody_linear_residual_ws(const void* x, const void* w, const void* 
     return gemm_bf16(ODY_GEMM_NT, static_cast<const bf16*>(x), static_cast<const bf16*>(w), static_cast<bf16*>(y), nullptr,
                      static_cast<const bf16*>(residual), M, N, K, ldx, ldw, ldy, ld_res, workspace, workspace_bytes, st);
   if (dtype == ODY_F32)
-    return gemm_f32(ODY_GEMM_NT, static_cast<const float*>(x), static_cast<const float*>(w), static_cast<float*>(y), nullptr, M, N, K, ldx,
+    return ody_launch_gemm_f32(ODY_GEMM_NT, static_cast<const float*>(x), static_cast<const float*>(w), static_cast<float*>(y), nullptr, M, N, K, ldx,
                     ldw, ldy, static_cast<const float*>(residual), y == residual ? ldy : ld_res, workspace, workspace_bytes, st);
   // any other shape or alignment: y = residual, then y += x W^T (added in fp32 before the one rounding, as above)
   if (y != residual) {

@@ -23,3 +23,8 @@ constexpr int ODY_SKINNY_MAX_M = 16;
 bool ody_gemm_skinny_ok(int epi, int M, int N);
 int ody_launch_gemm_skinny(int epi, const bf16* A, const bf16* W, bf16* C, const bf16* bias, int M, int N, int K, int64_t lda,
                            int64_t ldw, int64_t ldc, int accumulate, const GemmEpi& ep, hipStream_t st);
+
+// fp32 products (gemm_f32.hip), any shape and alignment; `add` may be C itself
+size_t ody_gemm_f32_workspace(int M, int N, int K);
+int ody_launch_gemm_f32(int op, const float* A, const float* B, float* C, const float* bias, int M, int N, int K, int64_t lda, int64_t ldb,
+                        int64_t ldc, const float* add, int64_t ld_add, void* workspace, size_t workspace_bytes, hipStream_t st);
