@@ -1,4 +1,4 @@
-"""Builds libodysseus_hip.so (gfx950) from csrc/*.hip with hipcc.
+"""Builds libodysseus_hip.so (gfx950) from csrc/*.hip with hipcc, and the host module of csrc/host/ with the host compiler.
 
 Usage:  python -m odysseus_transformer_amd.build [--force] [--jobs N]
 
@@ -14,6 +14,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 from pathlib import Path
 
 PKG = Path(__file__).resolve().parent
@@ -24,6 +25,9 @@ LIB = PKG / "lib" / "libodysseus_hip.so"
 BENCH_SRC = CSRC / "bench" / "probes.hip"
 BENCH_LIB = PKG / "lib" / "libodysseus_bench.so"
 INCLUDE = PKG.parent / "include"
+# the ops' host path: a CPython module against torch's C++ library, which finds the kernels' library through Python (_native.py)
+NATIVE_SRC = CSRC / "host" / "native.cpp"
+NATIVE_LIB = PKG / "lib" / "_odysseus_native.so"
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",
@@ -60,12 +64,33 @@ def _compile(src: Path, force: bool) -> Path:
     return obj
 
 
+def _build_native(force: bool) -> None:
+    if not force and not _newer(NATIVE_SRC, NATIVE_LIB, INCLUDE.glob("*.h")):
+        return
+    import torch
+    root = Path(torch.__file__).resolve().parent
+    rocm = Path(_hipcc()).resolve().parent.parent
+    cxx = shutil.which("g++") or shutil.which("c++")
+    if cxx is None:
+        raise RuntimeError("no host C++ compiler found")
+    cmd = [cxx, "-O2", "-std=c++17", "-fPIC", "-shared", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", "-I", str(INCLUDE), "-isystem", str(root / "include"), "-isystem",
+           str(root / "include" / "torch" / "csrc" / "api" / "include"), "-isystem", str(rocm / "include"), "-isystem", "/opt/rocm/include",
+           "-isystem", sysconfig.get_paths()["include"], str(NATIVE_SRC), "-o", str(NATIVE_LIB), "-L", str(root / "lib"), "-lc10", "-lc10_hip",
+           "-ltorch_cpu", "-ltorch_python"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"{cxx} failed for {NATIVE_SRC.name}:\n{r.stderr}")
+
+
 def build(force: bool = False, jobs: int = 4, verbose: bool = True) -> Path:
     OBJ.mkdir(parents=True, exist_ok=True)
     LIB.parent.mkdir(parents=True, exist_ok=True)
     srcs = sorted(CSRC.glob("*.hip"))
     with cf.ThreadPoolExecutor(max_workers=max(1, jobs)) as ex:
+        host = ex.submit(_build_native, force)
         objs = list(ex.map(lambda s: _compile(s, force), srcs))
+        host.result()
     if force or not LIB.exists() or any(o.stat().st_mtime > LIB.stat().st_mtime for o in objs):
         cmd = [_hipcc(), "--offload-arch=gfx950", "-shared", "-fPIC", "-o", str(LIB), *map(str, objs)]
         r = subprocess.run(cmd, capture_output=True, text=True)
@@ -77,7 +102,7 @@ def build(force: bool = False, jobs: int = 4, verbose: bool = True) -> Path:
         if r.returncode != 0:
             raise RuntimeError(f"hipcc failed for {BENCH_SRC.name}:\n{r.stderr}")
     if verbose:
-        print(f"built {LIB} ({LIB.stat().st_size} bytes) from {len(srcs)} sources, and {BENCH_LIB.name}")
+        print(f"built {LIB} ({LIB.stat().st_size} bytes) from {len(srcs)} sources, {NATIVE_LIB.name} and {BENCH_LIB.name}")
     return LIB
 
 

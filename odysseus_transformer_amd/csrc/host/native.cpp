@@ -1,0 +1,449 @@
+// The ops of ops.py in their plain form -- checks, allocations and the call of the C ABI -- without a trip through Python and ctypes
+// for each of them.
+//
+// Bound by the interpreter: the wrappers in ops.py take 9 to 15 us per op, of which the launch is 2; a decoding step, a short sequence
+// or a small layer is a row of ops whose kernels take no longer.  A decoding step of hidden 4096 behind 8191 tokens (8 ops of 110 us of
+// kernels): 176 us a pass through Python, 110 through here; attention of 4 x 331 tokens, forward and backward: 88 us of host work, now 65.
+//
+// A function here answers None for whatever is not the plain form of its op: a tensor that is not a dense CUDA tensor of the current
+// device (subclasses, wrappers of function transforms, conjugate or negative views included), a shape or stride that needs a copy or an
+// error message, a workspace that does not fit.  Its caller then goes on with the checks and copies written in Python, which stay the
+// definition of what an op accepts and of the error it raises.
+//
+// No state but what bind() is given once: the addresses of the library's entry points, so that this module uses the library that
+// Python loaded, and three Python objects.
+#define PY_SSIZE_T_CLEAN
+#include <Python.h>
+
+#include <ATen/core/Tensor.h>
+#include <ATen/ops/empty.h>
+#include <ATen/ops/empty_like.h>
+#include <c10/hip/HIPFunctions.h>
+#include <c10/hip/HIPStream.h>
+#include <c10/util/Exception.h>
+#include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/python_variable.h>
+
+#include <cmath>
+#include <cstring>
+
+#include "odysseus_hip.h"
+
+namespace {
+
+// ------------------------------------------------------------------------------------------------ the library and Python's side
+#define ODY_ENTRY_POINTS(X)                                                                                                       \
+  X(ody_rmsnorm_fwd) X(ody_rmsnorm_bwd_partials) X(ody_rmsnorm_bwd) X(ody_gemm_workspace_bytes) X(ody_gemm) X(ody_linear_residual_ws) \
+  X(ody_linear_rope_ws) X(ody_linear_swiglu) X(ody_linear_swiglu_h_fused) X(ody_linear_swiglu_h)                                  \
+  X(ody_linear_dgrad_swiglu_workspace_bytes) X(ody_linear_dgrad_swiglu) X(ody_attn_fwd_workspace_bytes) X(ody_attn_fwd)           \
+  X(ody_attn_bwd_workspace_bytes) X(ody_attn_bwd) X(ody_attn_bwd_rope) X(ody_rope) X(ody_rope_table)
+
+struct Library {
+#define X(name) decltype(&::name) name = nullptr;
+  ODY_ENTRY_POINTS(X)
+#undef X
+} lib;
+PyObject* arena_holder = nullptr;   // class whose attribute `instance` is the scratch arena, or None
+PyObject* scratch_fn = nullptr;     // scratch(nbytes, name, device) of ops.py
+PyObject* raise_fn = nullptr;       // raises for (name, status)
+
+struct NotPlain {};      // the caller answers None
+struct PythonError {};   // a Python exception is set
+
+// ------------------------------------------------------------------------------------------------ arguments
+constexpr c10::DispatchKeySet special{c10::DispatchKey::Python,          c10::DispatchKey::PythonTLSSnapshot, c10::DispatchKey::FuncTorchBatched,
+                                      c10::DispatchKey::FuncTorchGradWrapper, c10::DispatchKey::Functionalize, c10::DispatchKey::Batched,
+                                      c10::DispatchKey::Conjugate,       c10::DispatchKey::Negative,          c10::DispatchKey::ZeroTensor};
+
+void need(bool plain) {
+  if (!plain) throw NotPlain{};
+}
+
+// The arguments of one call; `like` (the first tensor) sets device and dtype.
+struct Call {
+  PyObject* const* args;
+  Py_ssize_t n;
+  c10::DeviceIndex device;
+  hipStream_t stream;
+
+  Call(PyObject* const* a, Py_ssize_t count, Py_ssize_t expected) : args(a), n(count), device(-1), stream(nullptr) { need(count == expected); }
+
+  // any strided tensor of the current device
+  const at::Tensor& any(Py_ssize_t i) {
+    PyObject* o = args[i];
+    need(THPVariable_CheckExact(o));
+    const at::Tensor& t = THPVariable_Unpack(o);
+    need(t.defined() && t.is_cuda() && t.layout() == c10::Layout::Strided && !t.unsafeGetTensorImpl()->key_set().has_any(special) && t.numel() > 0);
+    if (device < 0) {
+      device = c10::hip::current_device();
+      stream = c10::hip::getCurrentHIPStream(device).stream();
+    }
+    need(t.get_device() == device);
+    return t;
+  }
+  // ... that the kernels compute with
+  const at::Tensor& values(Py_ssize_t i) {
+    const at::Tensor& t = any(i);
+    need(t.scalar_type() == at::kBFloat16 || t.scalar_type() == at::kFloat);
+    return t;
+  }
+  const at::Tensor& like(Py_ssize_t i, const at::Tensor& ref) {
+    const at::Tensor& t = any(i);
+    need(t.scalar_type() == ref.scalar_type());
+    return t;
+  }
+  // row-major, rows any distance apart
+  const at::Tensor& matrix(Py_ssize_t i, const at::Tensor* ref) {
+    const at::Tensor& t = ref ? like(i, *ref) : values(i);
+    need(t.dim() == 2 && t.stride(1) == 1 && t.size(0) < INT32_MAX && t.size(1) < INT32_MAX);
+    return t;
+  }
+  // (B, L, H, D)
+  const at::Tensor& heads(Py_ssize_t i, const at::Tensor* ref) {
+    const at::Tensor& t = ref ? like(i, *ref) : values(i);
+    need(t.dim() == 4 && t.stride(3) == 1);
+    for (int d = 0; d < 4; d++) need(t.size(d) < INT32_MAX);
+    return t;
+  }
+  bool none(Py_ssize_t i) const { return args[i] == Py_None; }
+  bool flag(Py_ssize_t i) const {
+    need(PyBool_Check(args[i]));
+    return args[i] == Py_True;
+  }
+  int64_t whole(Py_ssize_t i) const {
+    need(PyLong_CheckExact(args[i]));
+    const int64_t v = PyLong_AsLongLong(args[i]);
+    if (v == -1 && PyErr_Occurred()) throw PythonError{};
+    return v;
+  }
+  double real(Py_ssize_t i) const {
+    need(PyFloat_Check(args[i]) || PyLong_CheckExact(args[i]));
+    const double v = PyFloat_AsDouble(args[i]);
+    if (v == -1 && PyErr_Occurred()) throw PythonError{};
+    return v;
+  }
+};
+
+int dt(const at::Tensor& t) { return t.scalar_type() == at::kBFloat16 ? ODY_BF16 : ODY_F32; }
+int64_t pitch(const at::Tensor& t) { return t.size(0) > 1 ? t.stride(0) : std::max(t.stride(0), t.size(1)); }
+at::Tensor make(at::IntArrayRef shape, const at::Tensor& like) { return at::empty(shape, like.options().requires_grad(false)); }
+at::Tensor make_f32(at::IntArrayRef shape, const at::Tensor& like) { return at::empty(shape, like.options().dtype(at::kFloat).requires_grad(false)); }
+
+// Kernel scratch, from the arena where one is set up.  Nothing: no such memory; the caller of the op has other ways.
+struct Scratch {
+  at::Tensor t;
+  size_t bytes;
+  Scratch(size_t nbytes, const char* name, const at::Tensor& like) : bytes(nbytes) {
+    if (nbytes == 0) return;
+    PyObject* arena = PyObject_GetAttrString(arena_holder, "instance");
+    if (!arena) throw PythonError{};
+    const bool have = arena != Py_None;
+    Py_DECREF(arena);
+    if (have) {
+      PyObject* device = THPDevice_New_(like);
+      PyObject* r = PyObject_CallFunction(scratch_fn, "nsO", (Py_ssize_t)nbytes, name, device);
+      Py_XDECREF(device);
+      if (!r) throw PythonError{};
+      t = THPVariable_Unpack(r);
+      Py_DECREF(r);
+      return;
+    }
+    try {
+      t = at::empty({(int64_t)nbytes}, like.options().dtype(at::kByte).requires_grad(false));
+    } catch (const c10::OutOfMemoryError&) {
+      throw NotPlain{};
+    }
+  }
+  void* ptr() const { return t.defined() ? t.data_ptr() : nullptr; }
+
+ private:
+  static PyObject* THPDevice_New_(const at::Tensor& like) {
+    PyObject* o = THPVariable_Wrap(like);
+    PyObject* d = o ? PyObject_GetAttrString(o, "device") : nullptr;
+    Py_XDECREF(o);
+    if (!d) throw PythonError{};
+    return d;
+  }
+};
+
+// an entry point's answer; the interpreter is free meanwhile (a launch waits where the queue is full)
+template <typename F, typename... A>
+void call(const char* name, F fn, A... a) {
+  int rc;
+  {
+    PyThreadState* save = PyEval_SaveThread();
+    rc = fn(a...);
+    PyEval_RestoreThread(save);
+  }
+  if (rc == 0) return;
+  PyObject* r = PyObject_CallFunction(raise_fn, "si", name, rc);
+  Py_XDECREF(r);
+  if (r) PyErr_Format(PyExc_RuntimeError, "%s failed with status %d", name, rc);
+  throw PythonError{};
+}
+#define CALL(name, ...) call(#name, lib.name, __VA_ARGS__)
+
+PyObject* wrap(const at::Tensor& t) {
+  PyObject* o = THPVariable_Wrap(t);
+  if (!o) throw PythonError{};
+  return o;
+}
+template <typename... T>
+PyObject* tuple(const T&... t) {
+  PyObject* r = PyTuple_New(sizeof...(T));
+  if (!r) throw PythonError{};
+  Py_ssize_t i = 0;
+  (PyTuple_SET_ITEM(r, i++, wrap(t)), ...);
+  return r;
+}
+
+// ------------------------------------------------------------------------------------------------ the ops
+// (x, weight, eps) -> (y, rstd)
+PyObject* rmsnorm_fwd(Call c) {
+  const at::Tensor &x = c.values(0), &w = c.like(1, x);
+  need(x.dim() >= 1 && x.is_contiguous() && w.dim() == 1 && w.is_contiguous() && w.size(0) == x.size(-1));
+  const int64_t d = x.size(-1), T = x.numel() / d;
+  need(T < INT32_MAX && d < INT32_MAX);
+  const float eps = (float)c.real(2);
+  at::Tensor y = make(x.sizes(), x), rstd = make_f32({T}, x);
+  CALL(ody_rmsnorm_fwd, x.data_ptr(), w.data_ptr(), y.data_ptr(), rstd.data_ptr<float>(), (int)T, (int)d, eps, dt(x), (void*)c.stream);
+  return tuple(y, rstd);
+}
+
+// (x, weight, rstd, dy, dx_add or None) -> (dx, dw)
+PyObject* rmsnorm_bwd(Call c) {
+  const at::Tensor &x = c.values(0), &w = c.like(1, x), &rstd = c.any(2), &dy = c.like(3, x);
+  need(x.dim() >= 1 && x.is_contiguous() && w.dim() == 1 && w.is_contiguous() && w.size(0) == x.size(-1));
+  const int64_t d = x.size(-1), T = x.numel() / d;
+  need(T < INT32_MAX && d < INT32_MAX && rstd.scalar_type() == at::kFloat && rstd.is_contiguous() && rstd.numel() == T);
+  need(dy.sizes() == x.sizes() && dy.is_contiguous());
+  const at::Tensor* add = c.none(4) ? nullptr : &c.like(4, x);
+  need(!add || (add->sizes() == x.sizes() && add->is_contiguous()));
+  at::Tensor dx = make(x.sizes(), x), dw = make(w.sizes(), w);
+  Scratch part((size_t)lib.ody_rmsnorm_bwd_partials((int)T) * d * 4, "rmsnorm_dw_partials", x);
+  CALL(ody_rmsnorm_bwd, x.data_ptr(), w.data_ptr(), rstd.data_ptr<float>(), dy.data_ptr(), add ? add->data_ptr() : nullptr, dx.data_ptr(),
+       (float*)part.ptr(), dw.data_ptr(), (int)T, (int)d, dt(x), (void*)c.stream);
+  return tuple(dx, dw);
+}
+
+// (op, a, b) -> out
+PyObject* gemm(Call c) {
+  const int64_t op = c.whole(0);
+  const at::Tensor &a = c.matrix(1, nullptr), &b = c.matrix(2, &a);
+  need(op == ODY_GEMM_NT || op == ODY_GEMM_NN || op == ODY_GEMM_TN);
+  const int64_t M = a.size(op == ODY_GEMM_TN ? 1 : 0), K = a.size(op == ODY_GEMM_TN ? 0 : 1), N = b.size(op == ODY_GEMM_NT ? 0 : 1);
+  need(b.size(op == ODY_GEMM_NT ? 1 : 0) == K);
+  at::Tensor out = make({M, N}, a);
+  Scratch ws(lib.ody_gemm_workspace_bytes((int)op, (int)M, (int)N, (int)K, dt(a)), "gemm_workspace", a);
+  CALL(ody_gemm, (int)op, a.data_ptr(), b.data_ptr(), out.data_ptr(), nullptr, (int)M, (int)N, (int)K, pitch(a), pitch(b), pitch(out), 0, dt(a),
+       ws.ptr(), ws.bytes, (void*)c.stream);
+  return wrap(out);
+}
+
+// (x, weight, residual) -> y
+PyObject* linear_residual(Call c) {
+  const at::Tensor &x = c.matrix(0, nullptr), &w = c.matrix(1, &x), &r = c.matrix(2, &x);
+  const int64_t M = x.size(0), K = x.size(1), N = w.size(0);
+  need(w.size(1) == K && r.size(0) == M && r.size(1) == N);
+  at::Tensor y = make({M, N}, x);
+  Scratch ws(lib.ody_gemm_workspace_bytes(ODY_GEMM_NT, (int)M, (int)N, (int)K, dt(x)), "gemm_workspace", x);
+  CALL(ody_linear_residual_ws, x.data_ptr(), w.data_ptr(), r.data_ptr(), y.data_ptr(), (int)M, (int)N, (int)K, pitch(x), pitch(w), pitch(r),
+       y.stride(0), dt(x), ws.ptr(), ws.bytes, (void*)c.stream);
+  return wrap(y);
+}
+
+// (x, weight, table, n_rot, head_dim) -> y
+PyObject* linear_rope(Call c) {
+  const at::Tensor &x = c.matrix(0, nullptr), &w = c.matrix(1, &x), &table = c.matrix(2, &x);
+  const int64_t n_rot = c.whole(3), D = c.whole(4), M = x.size(0), K = x.size(1), N = w.size(0);
+  need(x.scalar_type() == at::kBFloat16 && D == 128 && w.size(1) == K && N % D == 0 && n_rot >= 0 && n_rot <= N / D);
+  need(table.is_contiguous() && table.size(0) == M && table.size(1) == D);
+  at::Tensor y = make({M, N}, x);
+  Scratch ws(lib.ody_gemm_workspace_bytes(ODY_GEMM_NT, (int)M, (int)N, (int)K, dt(x)), "gemm_workspace", x);
+  CALL(ody_linear_rope_ws, x.data_ptr(), w.data_ptr(), table.data_ptr(), y.data_ptr(), (int)M, (int)N, (int)K, (int)n_rot, (int)D, pitch(x),
+       pitch(w), table.stride(0), y.stride(0), dt(x), ws.ptr(), ws.bytes, (void*)c.stream);
+  return wrap(y);
+}
+
+// (x, w_gate_up) -> (gate_up, h)
+PyObject* linear_swiglu(Call c) {
+  const at::Tensor &x = c.matrix(0, nullptr), &w = c.matrix(1, &x);
+  const int64_t T = x.size(0), K = x.size(1), I2 = w.size(0);
+  need(w.size(1) == K && I2 % 2 == 0);
+  at::Tensor gu = make({T, I2}, x), h = make({T, I2 / 2}, x);
+  CALL(ody_linear_swiglu, x.data_ptr(), w.data_ptr(), gu.data_ptr(), h.data_ptr(), (int)T, (int)(I2 / 2), (int)K, pitch(x), pitch(w), gu.stride(0),
+       h.stride(0), dt(x), (void*)c.stream);
+  return tuple(gu, h);
+}
+
+// (x, w_gate_up) -> h, where one kernel does it
+PyObject* linear_swiglu_h(Call c) {
+  const at::Tensor &x = c.matrix(0, nullptr), &w = c.matrix(1, &x);
+  const int64_t T = x.size(0), K = x.size(1), I2 = w.size(0);
+  need(w.size(1) == K && I2 % 2 == 0 &&
+       lib.ody_linear_swiglu_h_fused(x.data_ptr(), w.data_ptr(), (int)T, (int)(I2 / 2), (int)K, pitch(x), pitch(w), dt(x)) != 0);
+  at::Tensor h = make({T, I2 / 2}, x);
+  CALL(ody_linear_swiglu_h, x.data_ptr(), w.data_ptr(), h.data_ptr(), (int)T, (int)(I2 / 2), (int)K, pitch(x), pitch(w), h.stride(0), dt(x),
+       (void*)c.stream);
+  return wrap(h);
+}
+
+// (dy, w_down, gate_up) -> d_gate_up
+PyObject* linear_dgrad_swiglu(Call c) {
+  const at::Tensor &dy = c.matrix(0, nullptr), &w = c.matrix(1, &dy), &gu = c.matrix(2, &dy);
+  const int64_t T = dy.size(0), K = dy.size(1), I = w.size(1);
+  need(w.size(0) == K && gu.size(0) == T && gu.size(1) == 2 * I);
+  for (const at::Tensor* t : {&dy, &w, &gu})   // what one kernel wants where the size query goes by the shape alone
+    need(reinterpret_cast<uintptr_t>(t->data_ptr()) % 16 == 0 && t->stride(0) % 8 == 0);
+  need(pitch(dy) < (1 << 22) && pitch(w) < (1 << 24));
+  at::Tensor dgu = make({T, 2 * I}, dy);
+  Scratch ws(lib.ody_linear_dgrad_swiglu_workspace_bytes((int)T, (int)I, (int)K, dt(dy)), "dgrad_swiglu_workspace", dy);
+  CALL(ody_linear_dgrad_swiglu, dy.data_ptr(), w.data_ptr(), gu.data_ptr(), dgu.data_ptr(), (int)T, (int)I, (int)K, pitch(dy), pitch(w), pitch(gu),
+       dgu.stride(0), dt(dy), ws.ptr(), ws.bytes, (void*)c.stream);
+  return wrap(dgu);
+}
+
+#define STRIDES(t) (t).stride(0), (t).stride(1), (t).stride(2)
+
+void check_kv(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v) {
+  need(k.sizes() == v.sizes() && k.size(0) == q.size(0) && k.size(3) == q.size(3));
+}
+
+// (q, k, v, causal, scale) -> (out, lse)
+PyObject* attn_fwd(Call c) {
+  const at::Tensor &q = c.heads(0, nullptr), &k = c.heads(1, &q), &v = c.heads(2, &q);
+  check_kv(q, k, v);
+  const bool causal = c.flag(3);
+  const float scale = (float)c.real(4);
+  const int B = q.size(0), Lq = q.size(1), Hq = q.size(2), D = q.size(3), Lk = k.size(1), Hkv = k.size(2);
+  at::Tensor out = make({B, Lq, Hq, D}, q), lse = make_f32({B, Hq, Lq}, q);
+  Scratch ws(lib.ody_attn_fwd_workspace_bytes(B, Lq, Lk, Hq, Hkv, D, dt(q)), "attn_fwd_workspace", q);
+  CALL(ody_attn_fwd, q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), lse.data_ptr<float>(), B, Lq, Lk, Hq, Hkv, D, STRIDES(q), STRIDES(k),
+       STRIDES(v), STRIDES(out), scale, (int)causal, dt(q), ws.ptr(), ws.bytes, (void*)c.stream);
+  return tuple(out, lse);
+}
+
+// (q, k, v, out, lse, dout, causal, scale, dq or None, dk or None, dv or None, table_q or None, table_k or None) -> (dq, dk, dv)
+PyObject* attn_bwd(Call c) {
+  const at::Tensor &q = c.heads(0, nullptr), &k = c.heads(1, &q), &v = c.heads(2, &q), &out = c.heads(3, &q), &lse = c.any(4), &dout = c.heads(5, &q);
+  check_kv(q, k, v);
+  const bool causal = c.flag(6);
+  const float scale = (float)c.real(7);
+  const int B = q.size(0), Lq = q.size(1), Hq = q.size(2), D = q.size(3), Lk = k.size(1), Hkv = k.size(2);
+  need(out.sizes() == q.sizes() && dout.sizes() == q.sizes());
+  need(lse.scalar_type() == at::kFloat && lse.is_contiguous() && lse.dim() == 3 && lse.size(0) == B && lse.size(1) == Hq && lse.size(2) == Lq);
+  at::Tensor g[3];
+  const at::Tensor* of[3] = {&q, &k, &v};
+  for (int i = 0; i < 3; i++) {
+    g[i] = c.none(8 + i) ? at::empty_like(*of[i], of[i]->options().requires_grad(false)) : c.heads(8 + i, &q);
+    need(g[i].sizes() == of[i]->sizes() && g[i].stride(3) == 1);
+  }
+  need(c.none(11) == c.none(12));
+  const at::Tensor* table[2] = {nullptr, nullptr};
+  if (!c.none(11))
+    for (int i = 0; i < 2; i++) {
+      table[i] = &c.matrix(11 + i, &q);
+      need(q.scalar_type() == at::kBFloat16 && table[i]->is_contiguous() && table[i]->size(0) == (int64_t)B * (i ? Lk : Lq) && table[i]->size(1) == D);
+    }
+  Scratch ws(lib.ody_attn_bwd_workspace_bytes(B, Lq, Lk, Hq, Hkv, D, dt(q)), "attn_bwd_workspace", q);
+#define BWD_ARGS                                                                                                                   \
+  q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), lse.data_ptr<float>(), dout.data_ptr(), g[0].data_ptr(), g[1].data_ptr(), \
+      g[2].data_ptr(), B, Lq, Lk, Hq, Hkv, D, STRIDES(q), STRIDES(k), STRIDES(v), STRIDES(out), STRIDES(dout), STRIDES(g[0]),       \
+      STRIDES(g[1]), STRIDES(g[2]), scale, (int)causal, 0, dt(q), ws.ptr(), ws.bytes, (void*)c.stream
+  if (table[0]) CALL(ody_attn_bwd_rope, BWD_ARGS, table[0]->data_ptr(), table[1]->data_ptr());
+  else CALL(ody_attn_bwd, BWD_ARGS);
+  return tuple(g[0], g[1], g[2]);
+}
+
+const int64_t* positions(Call& c, Py_ssize_t i, int64_t rows) {
+  if (c.none(i)) return nullptr;
+  const at::Tensor& p = c.any(i);
+  need(p.scalar_type() == at::kLong && p.is_contiguous() && p.numel() == rows);
+  return p.data_ptr<int64_t>();
+}
+const at::Tensor& frequencies(Call& c, Py_ssize_t i, int64_t D) {
+  const at::Tensor& f = c.any(i);
+  need(D % 2 == 0 && f.scalar_type() == at::kFloat && f.is_contiguous() && f.numel() == D / 2);
+  return f;
+}
+
+// (x, n_rot, position_ids or None, inv_freq, base, inverse) -> True: x (B, L, H, D) is rotated in place
+PyObject* rope(Call c) {
+  const at::Tensor& x = c.heads(0, nullptr);
+  const int64_t n_rot = c.whole(1);
+  const int B = x.size(0), L = x.size(1), D = x.size(3);
+  need(n_rot >= 0 && n_rot <= x.size(2));
+  need(c.none(2) || THPVariable_CheckExact(c.args[2]));
+  if (!c.none(2)) need(THPVariable_Unpack(c.args[2]).dim() >= 1 && THPVariable_Unpack(c.args[2]).size(-1) == L);
+  const int64_t* pos = positions(c, 2, (int64_t)B * L);
+  const at::Tensor& f = frequencies(c, 3, D);
+  CALL(ody_rope, x.data_ptr(), pos, f.data_ptr<float>(), B, L, (int)n_rot, D, STRIDES(x), (float)c.real(4), (int)c.flag(5), dt(x), (void*)c.stream);
+  Py_RETURN_TRUE;
+}
+
+// (position_ids or None, rows, head_dim, inv_freq, base) -> table
+PyObject* rope_table(Call c) {
+  const int64_t rows = c.whole(1), D = c.whole(2);
+  const at::Tensor& f = frequencies(c, 3, D);
+  need(rows > 0);
+  const int64_t* pos = positions(c, 0, rows);
+  at::Tensor table = at::empty({rows, D}, f.options().dtype(at::kBFloat16).requires_grad(false));
+  CALL(ody_rope_table, pos, f.data_ptr<float>(), rows, (int)D, (float)c.real(4), table.data_ptr(), (void*)c.stream);
+  return wrap(table);
+}
+
+// the raw stream that the ops above launch on
+PyObject* current_stream(Call) {
+  return PyLong_FromVoidPtr((void*)c10::hip::getCurrentHIPStream(c10::hip::current_device()).stream());
+}
+
+template <PyObject* (*OP)(Call), int N>
+PyObject* method(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  try {
+    return OP(Call(args, n, N));
+  } catch (const NotPlain&) {
+    Py_RETURN_NONE;
+  } catch (const PythonError&) {
+    return nullptr;
+  }
+  END_HANDLE_TH_ERRORS
+}
+
+// (addresses by name, arena holder, scratch, raise)
+PyObject* bind(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  if (n != 4 || !PyDict_Check(args[0])) {
+    PyErr_SetString(PyExc_TypeError, "bind(addresses, arena_holder, scratch, raise)");
+    return nullptr;
+  }
+#define X(name)                                                                      \
+  {                                                                                  \
+    PyObject* a = PyDict_GetItemString(args[0], #name);                              \
+    void* p = a ? PyLong_AsVoidPtr(a) : nullptr;                                     \
+    if (!p) {                                                                        \
+      if (!PyErr_Occurred()) PyErr_SetString(PyExc_KeyError, #name);                 \
+      return nullptr;                                                                \
+    }                                                                                \
+    lib.name = reinterpret_cast<decltype(lib.name)>(p);                              \
+  }
+  ODY_ENTRY_POINTS(X)
+#undef X
+  PyObject** to[3] = {&arena_holder, &scratch_fn, &raise_fn};
+  for (int i = 0; i < 3; i++) {
+    Py_INCREF(args[1 + i]);
+    Py_XSETREF(*to[i], args[1 + i]);
+  }
+  Py_RETURN_NONE;
+}
+
+#define METHOD(name, n) {#name, (PyCFunction)(void (*)(void))method<name, n>, METH_FASTCALL, nullptr}
+PyMethodDef methods[] = {
+    {"bind", (PyCFunction)(void (*)(void))bind, METH_FASTCALL, nullptr},
+    METHOD(rmsnorm_fwd, 3), METHOD(rmsnorm_bwd, 5), METHOD(gemm, 3), METHOD(linear_residual, 3), METHOD(linear_rope, 5), METHOD(linear_swiglu, 2),
+    METHOD(linear_swiglu_h, 2), METHOD(linear_dgrad_swiglu, 3), METHOD(attn_fwd, 5), METHOD(attn_bwd, 13), METHOD(rope, 6), METHOD(rope_table, 5),
+    METHOD(current_stream, 0), {nullptr, nullptr, 0, nullptr}};
+PyModuleDef module = {PyModuleDef_HEAD_INIT, "_odysseus_native", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__odysseus_native() { return PyModule_Create(&module); }

@@ -2,7 +2,8 @@
 stream, nothing else) and the autograd functions built from them.
 
 Every function requires CUDA(HIP) tensors and raises otherwise: the HIP library
-is the only compute path.
+is the only compute path.  `native` holds the plain form of the ops that a layer is made
+of, in C++; where it answers None the Python below it decides.
 """
 from __future__ import annotations
 
@@ -14,6 +15,7 @@ import torch
 
 from . import _lib
 from ._lib import GEMM_NN, GEMM_NT, GEMM_TN
+from ._native import native
 
 
 def _dt(t: torch.Tensor) -> int:
@@ -114,6 +116,10 @@ def attn_fwd(q, k, v, causal: bool = True, scale: Optional[float] = None, out=No
     dropout_p > 0 drops entries of the softmax matrix before P . V, scaling the kept ones by
     1 / (1 - dropout_p); which entries is a fixed function of `seed` (an int) and the entry's (batch, head,
     query, key), so attn_bwd with the same dropout_p and seed sees the same mask.  lse is that of the full P."""
+    if q.is_cuda and out is None and dropout_p == 0.0:
+        plain = native.attn_fwd(q, k, v, bool(causal), 1.0 / math.sqrt(q.shape[-1]) if scale is None else scale)
+        if plain is not None:
+            return plain
     _need_gpu(q, k, v)
     _check_dropout(dropout_p, seed)
     B, Lq, Hq, D = q.shape
@@ -175,6 +181,13 @@ def attn_bwd(q, k, v, out, lse, dout, causal: bool = True, scale: Optional[float
     opt-in: None (the default) turns it on only where the shape qualifies, no `workspace` is passed and the
     scratch stays within the budget of set_keep_ds_max_bytes() / ODYSSEUS_KEEP_DS_MAX_BYTES (0 unless set) or is
     already there in the arena; True insists (ValueError where the shape does not qualify); False never."""
+    if q.is_cuda and dropout_p == 0.0 and not accumulate_dq and workspace is None and not reuse_query_side and \
+            (keep_ds is False or (keep_ds is None and _never_keeps_ds())):
+        tq, tk = (None, None) if rope_tables is None else rope_tables
+        plain = native.attn_bwd(q, k, v, out, lse, dout, bool(causal), 1.0 / math.sqrt(q.shape[-1]) if scale is None else scale, dq, dk, dv,
+                                tq, tk)
+        if plain is not None:
+            return plain
     _need_gpu(q, k, v, out, lse, dout)
     _check_dropout(dropout_p, seed)
     if dropout_p > 0.0:
@@ -301,6 +314,12 @@ def _arena_holds(name: str, device) -> int:
     return 0 if backing is None else backing.numel()
 
 
+def _never_keeps_ds() -> bool:
+    """Whether keep_ds=None stays off whatever the shape: no budget, and no arena whose buffer might hold dS already."""
+    from .utils import globals as _globals
+    return _globals._Arena.instance is None and keep_ds_max_bytes() == 0
+
+
 def _keep_ds_fits(ws_bytes: int, ds_bytes: int, device) -> bool:
     """The policy of keep_ds=None: within the budget (and not a size that already failed to allocate on this device),
     or free because the arena's buffer is that large already."""
@@ -404,6 +423,10 @@ def _gemm_scratch(op: int, M: int, N: int, K: int, like):
 
 def gemm(op: int, a, b, bias=None, out=None, accumulate: bool = False):
     """op NT: a (M,K) b (N,K); NN: a (M,K) b (K,N); TN: a (K,M) b (K,N) -> (M,N)."""
+    if a.is_cuda and bias is None and out is None and not accumulate:
+        plain = native.gemm(op, a, b)
+        if plain is not None:
+            return plain
     _need_gpu(a, b, bias, out)
     if op == GEMM_NT:
         (M, K), (N, K2) = a.shape, b.shape
@@ -442,6 +465,10 @@ def _lin_args(x, w, name):
 
 def linear_residual(x, weight, residual):
     """x (M, K) W (N, K)^T + residual (M, N), the add in the product's epilogue."""
+    if x.is_cuda:
+        plain = native.linear_residual(x, weight, residual)
+        if plain is not None:
+            return plain
     _need_gpu(x, weight, residual)
     _lin_args(x, weight, "linear_residual")
     (M, K), N = x.shape, weight.shape[0]
@@ -500,6 +527,10 @@ def rope_table(position_ids, rows: int, head_dim: int, base: float = 10000.0, de
 
 def _new_rope_table(position_ids, rows: int, head_dim: int, base: float, device, inv_freq=None) -> torch.Tensor:
     """rope_table from the positions as they are now."""
+    if position_ids is not None and position_ids.is_cuda and position_ids.device == device:
+        plain = native.rope_table(position_ids, rows, head_dim, rope_inv_freq(head_dim, base, device) if inv_freq is None else inv_freq, base)
+        if plain is not None:
+            return plain
     if position_ids is not None:
         _need_gpu(position_ids)
         position_ids = position_ids.to(torch.int64).reshape(-1)
@@ -522,6 +553,10 @@ def _new_rope_table(position_ids, rows: int, head_dim: int, base: float, device,
 def linear_rope(x, weight, table, n_rot: int, head_dim: int):
     """x (M, K) W (N, K)^T with the first n_rot heads of head_dim columns rotated by row m of `table`
     (rope_table) in the product's epilogue: the packed QKV projection and its rotary embedding in one kernel."""
+    if x.is_cuda:
+        plain = native.linear_rope(x, weight, table, n_rot, head_dim)
+        if plain is not None:
+            return plain
     _need_gpu(x, weight, table)
     _lin_args(x, weight, "linear_rope")
     (M, K), N = x.shape, weight.shape[0]
@@ -541,6 +576,10 @@ def linear_rope(x, weight, table, n_rot: int, head_dim: int):
 
 def linear_swiglu(x, w_gate_up):
     """gate_up = x (T, K) Wgu (2 I, K)^T and h = silu(gate) * up in one kernel -> (gate_up, h)."""
+    if x.is_cuda:
+        plain = native.linear_swiglu(x, w_gate_up)
+        if plain is not None:
+            return plain
     _need_gpu(x, w_gate_up)
     _lin_args(x, w_gate_up, "linear_swiglu")
     (T, K), I2 = x.shape, w_gate_up.shape[0]
@@ -555,6 +594,10 @@ def linear_swiglu(x, w_gate_up):
 
 def linear_swiglu_h(x, w_gate_up):
     """The h of linear_swiglu alone, where nothing will ask for gate_up again: the product is not written to memory at all."""
+    if x.is_cuda:
+        plain = native.linear_swiglu_h(x, w_gate_up)
+        if plain is not None:
+            return plain
     _need_gpu(x, w_gate_up)
     _lin_args(x, w_gate_up, "linear_swiglu")
     (T, K), I2 = x.shape, w_gate_up.shape[0]
@@ -568,6 +611,10 @@ def linear_swiglu_h(x, w_gate_up):
 
 def linear_dgrad_swiglu(dy, w_down, gate_up):
     """d_gate_up from dy (T, K) and the down weight (K, I): dh = dy Wd never leaves the kernel."""
+    if dy.is_cuda:
+        plain = native.linear_dgrad_swiglu(dy, w_down, gate_up)
+        if plain is not None:
+            return plain
     _need_gpu(dy, w_down, gate_up)
     _lin_args(dy, w_down, "linear_dgrad_swiglu")
     (T, K), I = dy.shape, w_down.shape[1]
@@ -656,6 +703,10 @@ def check_rope_args(x, n_rot, position_ids, inv_freq) -> None:
 
 
 def rmsnorm_fwd(x, weight, eps: float = 1e-6):
+    if x.is_cuda:
+        plain = native.rmsnorm_fwd(x, weight, eps)
+        if plain is not None:
+            return plain
     _need_gpu(x, weight)
     check_rmsnorm_args(x, weight)
     x2 = x.reshape(-1, x.shape[-1]).contiguous()
@@ -670,6 +721,10 @@ def rmsnorm_fwd(x, weight, eps: float = 1e-6):
 def rmsnorm_bwd(x, weight, rstd, dy, dx_add=None):
     """dx, dw of rmsnorm; `dx_add` (same shape as x) is added to dx inside the kernel: the
     gradient that reaches the norm's input over the residual connection."""
+    if x.is_cuda:
+        plain = native.rmsnorm_bwd(x, weight, rstd, dy, dx_add)
+        if plain is not None:
+            return plain
     _need_gpu(x, weight, rstd, dy, dx_add)
     check_rmsnorm_args(x, weight, rstd, dy)
     x2 = x.reshape(-1, x.shape[-1]).contiguous()
@@ -705,6 +760,9 @@ def rope_inv_freq(head_dim: int, base: float, device) -> torch.Tensor:
 
 def rope_(x, n_rot: int, position_ids=None, base: float = 10000.0, inverse: bool = False, inv_freq=None) -> None:
     """Rotates heads [0, n_rot) of x (B, L, H, D) in place."""
+    if x.is_cuda and native.rope(x, n_rot, position_ids, rope_inv_freq(x.shape[-1], base, x.device) if inv_freq is None else inv_freq,
+                                 base, bool(inverse)):
+        return
     _need_gpu(x, position_ids, inv_freq)
     B, L, H, D = x.shape
     if inv_freq is None:

@@ -1,0 +1,194 @@
+"""The host path in C++ against the one in Python: the same results bit for bit over the forms that it takes, and the same answers to
+what it leaves alone."""
+import pytest
+import torch
+
+from conftest import randn
+
+pytestmark = pytest.mark.gpu
+
+
+class _Off:
+    """Stands for the module where it answers None to everything."""
+
+    def __getattr__(self, name):
+        return lambda *a: None
+
+
+def _both(monkeypatch, fn):
+    """fn() on either path, and how many calls the C++ one answered."""
+    from odysseus_transformer_amd import ops
+    taken = []
+
+    class Counting:
+        def __getattr__(self, name):
+            def call(*a):
+                r = getattr(ops_native, name)(*a)
+                if r is not None:
+                    taken.append(name)
+                return r
+            return call
+
+    ops_native = ops.native
+    with monkeypatch.context() as m:
+        m.setattr(ops, "native", Counting())
+        here = fn()
+    with monkeypatch.context() as m:
+        m.setattr(ops, "native", _Off())
+        there = fn()
+    torch.cuda.synchronize()
+    return here, there, taken
+
+
+def _same(a, b):
+    a, b = (x if isinstance(x, (tuple, list)) else (x,) for x in (a, b))
+    assert len(a) == len(b)
+    for x, y in zip(a, b):
+        assert x.shape == y.shape and x.dtype == y.dtype and x.stride() == y.stride() and x.requires_grad == y.requires_grad
+        assert torch.equal(x, y)
+
+
+def _matrix(rows, cols, seed, dtype, form, dev):
+    """A (rows, cols) matrix: dense, with padded rows, or starting off a 16-byte boundary (fp32: off any vector)."""
+    pad = {"dense": 0, "padded": 16, "shifted": 16}[form]
+    t = randn((rows, cols + pad), seed, std=0.1, dtype=dtype).to(dev)
+    off = 0 if form != "shifted" else (1 if dtype == torch.float32 else 8)
+    return t[:, off:off + cols]
+
+
+@pytest.mark.parametrize("form", ["dense", "padded", "shifted"])
+@pytest.mark.parametrize("rows", [1, 7, 300])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32], ids=["bf16", "f32"])
+def test_linears(dtype, rows, form, dev, monkeypatch):
+    from odysseus_transformer_amd import ops
+    K, N, I = 256, 384, 256
+    x, w = _matrix(rows, K, 1, dtype, form, dev), _matrix(N, K, 2, dtype, form, dev)
+    r, wgu = _matrix(rows, N, 3, dtype, form, dev), _matrix(2 * I, K, 4, dtype, form, dev)
+    wd, gu, dy = _matrix(K, I, 5, dtype, form, dev), _matrix(rows, 2 * I, 6, dtype, form, dev), _matrix(rows, N, 7, dtype, form, dev)
+    calls = {"nt": lambda: ops.gemm(ops.GEMM_NT, x, w), "nn": lambda: ops.gemm(ops.GEMM_NN, dy, w),
+             "residual": lambda: ops.linear_residual(x, w, r), "swiglu": lambda: ops.linear_swiglu(x, wgu),
+             "swiglu_h": lambda: ops.linear_swiglu_h(x, wgu), "dgrad": lambda: ops.linear_dgrad_swiglu(x, wd, gu)}
+    if dtype == torch.float32 and form == "shifted":   # refused on either path: the SwiGLU backward wants vectors
+        del calls["dgrad"]
+    if dtype == torch.float32 or rows % 8 == 0:
+        calls["tn"] = lambda: ops.gemm(ops.GEMM_TN, dy, x)
+    if dtype == torch.bfloat16:
+        table = ops.rope_table(torch.arange(rows, device=dev)[None], rows, 128)
+        calls["rope"] = lambda: ops.linear_rope(x, w, table, 2, 128)
+    for name, fn in calls.items():
+        print(f"{name} rows={rows} {dtype} {form}", flush=True)
+        here, there, taken = _both(monkeypatch, fn)
+        _same(here, there)
+        assert taken or name in ("swiglu_h", "dgrad"), name
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32], ids=["bf16", "f32"])
+def test_norm_and_rotation(dtype, dev, monkeypatch):
+    from odysseus_transformer_amd import ops
+    x, w = randn((1, 33, 512), 1, dtype=dtype).to(dev), randn((512,), 2, dtype=dtype).to(dev)
+    dy, add = randn((1, 33, 512), 3, dtype=dtype).to(dev), randn((1, 33, 512), 4, dtype=dtype).to(dev)
+    here, there, taken = _both(monkeypatch, lambda: ops.rmsnorm_fwd(x, w, 1e-6))
+    _same(here, there)
+    rstd = here[1]
+    for a in (None, add):
+        h, t, k = _both(monkeypatch, lambda: ops.rmsnorm_bwd(x, w, rstd, dy, a))
+        _same(h, t)
+        taken += k
+    assert taken == ["rmsnorm_fwd", "rmsnorm_bwd", "rmsnorm_bwd"]
+    # rows that are not dense: the copies are Python's
+    here, there, taken = _both(monkeypatch, lambda: ops.rmsnorm_fwd(x[..., :256], w[:256], 1e-6))
+    _same(here, there)
+    assert not taken
+    for B, pos in ((1, None), (1, torch.arange(5, 38, device=dev)[None]), (2, torch.arange(33, device=dev)[None]),
+                   (2, torch.randint(0, 99, (2, 33), device=dev)), (1, torch.arange(33, device=dev, dtype=torch.int32)[None])):
+        q = randn((B, 33, 6, 64), 5, dtype=dtype).to(dev)
+
+        def rotated(inverse):
+            y = q.clone()
+            ops.rope_(y, 4, pos, inverse=inverse)
+            return y
+
+        for inverse in (False, True):
+            here, there, taken = _both(monkeypatch, lambda: rotated(inverse))
+            _same(here, there)
+            assert bool(taken) == (pos is None or (pos.dtype == torch.int64 and pos.numel() == B * 33))
+
+
+@pytest.mark.parametrize("packed", [False, True], ids=["dense", "packed"])
+@pytest.mark.parametrize("shape", [(1, 1, 200, 4, 1, 128), (2, 65, 65, 4, 2, 128), (1, 130, 130, 2, 2, 64), (1, 300, 170, 4, 4, 64)],
+                         ids=lambda s: "B%d_Lq%d_Lk%d_H%d_%d_D%d" % s)
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32], ids=["bf16", "f32"])
+def test_attention(dtype, shape, packed, dev, monkeypatch):
+    from odysseus_transformer_amd import ops
+    B, Lq, Lk, Hq, Hkv, D = shape
+    print(f"shape={shape} {dtype} packed={packed}", flush=True)
+    if packed:
+        L = max(Lq, Lk)
+        qkv = randn((B, L, Hq + 2 * Hkv, D), 1, dtype=dtype).to(dev)
+        q, k, v = qkv[:, :Lq, :Hq], qkv[:, :Lk, Hq:Hq + Hkv], qkv[:, :Lk, Hq + Hkv:]
+    else:
+        q, k, v = (randn((B, L, H, D), s, dtype=dtype).to(dev) for L, H, s in ((Lq, Hq, 1), (Lk, Hkv, 2), (Lk, Hkv, 3)))
+    dout = randn((B, Lq, Hq, D), 4, dtype=dtype).to(dev)
+    for causal in (False, True):
+        here, there, taken = _both(monkeypatch, lambda: ops.attn_fwd(q, k, v, causal=causal, scale=None if causal else 0.1))
+        _same(here, there)
+        out, lse = here
+        for keep in (None, False):
+            h, t, kk = _both(monkeypatch, lambda: ops.attn_bwd(q, k, v, out, lse, dout, causal=causal, keep_ds=keep))
+            _same(h, t)
+            taken += kk
+        assert taken == ["attn_fwd", "attn_bwd", "attn_bwd"]
+        if dtype == torch.bfloat16 and D == 128 and packed and Lq == Lk:
+            tables = (ops.rope_table(None, B * Lq, D, device=dev),) * 2
+
+            def into():
+                d = torch.zeros_like(qkv)
+                ops.attn_bwd(q, k, v, out, lse, dout, causal=causal, dq=d[:, :, :Hq], dk=d[:, :, Hq:Hq + Hkv], dv=d[:, :, Hq + Hkv:],
+                             rope_tables=tables)
+                return d
+
+            h, t, kk = _both(monkeypatch, into)
+            _same(h, t)
+            assert kk == ["attn_bwd"]
+
+
+def test_what_it_leaves_alone(dev, monkeypatch):
+    """Errors, transforms, budgets and the arena go the way they went."""
+    from odysseus_transformer_amd import _lib, ops
+    from odysseus_transformer_amd.utils import globals as g
+    x, w = randn((16, 64), 1).to(dev), randn((64, 64), 2).to(dev)
+    for bad, err in ((lambda: ops.gemm(ops.GEMM_NT, x, w[:, :32]), ValueError), (lambda: ops.gemm(7, x, w), ValueError),
+                     (lambda: ops.gemm(ops.GEMM_NT, x, w.bfloat16()), TypeError), (lambda: ops.gemm(ops.GEMM_NT, x, w.cpu()), RuntimeError),
+                     (lambda: ops.gemm(ops.GEMM_NT, x.double(), w.double()), TypeError),
+                     (lambda: ops.gemm(ops.GEMM_NT, x.t(), w), ValueError),
+                     (lambda: ops.gemm(ops.GEMM_NT, x.bfloat16()[:, :60], w.bfloat16()[:, :60]), _lib.OdysseusHipError),
+                     (lambda: ops.rmsnorm_fwd(x, w[0].bfloat16()), TypeError), (lambda: ops.linear_residual(x, w, x[:, :8]), ValueError)):
+        with pytest.raises(err):
+            bad()
+
+    class Sub(torch.Tensor):
+        pass
+
+    q = randn((1, 256, 2, 128), 3, dtype=torch.bfloat16).to(dev)
+    for t in (q.as_subclass(Sub), q.cpu(), None, torch._neg_view(q)):
+        assert ops.native.attn_fwd(t, q, q, True, 0.1) is None
+    assert ops.native.attn_fwd(q, q, q, 1, 0.1) is None and ops.native.attn_fwd(q, q, q, True) is None
+    side = torch.cuda.Stream()
+    assert ops.native.current_stream() == ops._stream()
+    with torch.cuda.stream(side):
+        assert ops.native.current_stream() == ops._stream() == side.cuda_stream
+    out, lse = ops.attn_fwd(q, q, q)
+    ops.set_keep_ds_max_bytes(1 << 30)
+    try:
+        _, _, taken = _both(monkeypatch, lambda: ops.attn_bwd(q, q, q, out, lse, out))
+        assert not taken
+    finally:
+        ops.set_keep_ds_max_bytes(None)
+    g._set_global_memory_buffer(dev)
+    try:
+        a, b = randn((2048, 512), 4).to(dev), randn((2048, 512), 5).to(dev)
+        here, there, taken = _both(monkeypatch, lambda: ops.gemm(ops.GEMM_TN, a, b))
+        assert taken == ["gemm"] and torch.equal(here, there)
+        assert g.get_global_memory_buffer().buffer[("gemm_workspace", torch.uint8)].numel() > 0
+    finally:
+        g._destroy_global_memory_buffer()
