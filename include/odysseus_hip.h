@@ -328,6 +328,19 @@ int ody_attn_bwd_rope(const void* q, const void* k, const void* v, const void* o
                       void* workspace, size_t workspace_bytes, void* stream,
                       const void* rope_table_q, const void* rope_table_k);
 
+/* The RMSNorm in front of a product of few rows (a decoding step) inside the product, so that the normalised rows are never stored:
+ * bf16, at most 4 rows that take 64 KiB together (2 M (K + 8)), K a multiple of 8, 16-byte aligned rows (ODY_ERR_UNSUPPORTED
+ * otherwise: ody_rmsnorm_fwd and the product do).  Same arithmetic as the two kernels.
+ * ody_norm_linear_rope      ody_linear_rope of ody_rmsnorm_fwd(x); head_dim 128, the angles from position_ids (M) and
+ *                           inv_freq (D / 2) directly, rounded as ody_rope_table rounds them (decoder/odysseus.py:180-213 behind
+ *                           decoder/ring.py:67).
+ * ody_norm_linear_swiglu_h  ody_linear_swiglu_h of ody_rmsnorm_fwd(x); I a multiple of 16 (decoder/ring.py:84, decoder/odysseus.py:293-295).
+ */
+int ody_norm_linear_rope(const void* x, const void* norm_w, float eps, const void* w, const int64_t* position_ids, const float* inv_freq,
+                         void* y, int M, int N, int K, int n_rot, int D, int64_t ldx, int64_t ldw, int64_t ldy, int dtype, void* stream);
+int ody_norm_linear_swiglu_h(const void* x, const void* norm_w, float eps, const void* w_gate_up, void* h, int T, int I, int K,
+                             int64_t ldx, int64_t ldw, int64_t ld_h, int dtype, void* stream);
+
 /* ---- attention dropout ------------------------------------------------------
  * The dropout_p argument of the attention routine the reference calls (decoder/odysseus.py:228, 256-263; it
  * passes config.attention_dropout while training, 0.0 in its own configurations).  ody_attn_fwd / ody_attn_bwd with

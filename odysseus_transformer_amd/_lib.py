@@ -56,6 +56,8 @@ SIGNATURES = {
     "ody_adamw": (_i, [_p, _p, _p, _p, _i64, _f, _f, _f, _f, _f, _i64, _i, _p]),
     "ody_linear_rope": (_i, [_p] * 4 + [_i] * 5 + [_i64] * 4 + [_i, _p]),
     "ody_linear_rope_ws": (_i, [_p] * 4 + [_i] * 5 + [_i64] * 4 + [_i, _p, _sz, _p]),
+    "ody_norm_linear_rope": (_i, [_p, _p, _f] + [_p] * 4 + [_i] * 5 + [_i64] * 3 + [_i, _p]),
+    "ody_norm_linear_swiglu_h": (_i, [_p, _p, _f, _p, _p] + [_i] * 3 + [_i64] * 3 + [_i, _p]),
     "ody_attn_bwd_rope": (_i, [_p] * 9 + [_i] * 6 + [_i64] * 24 + [_f, _i, _i, _i, _p, _sz, _p, _p, _p]),
     "ody_attn_fwd_dropout": (_i, [_p] * 5 + [_i] * 6 + [_i64] * 12 + [_f, _i, _i, _p, _sz, _p, _f, _u64]),
     "ody_attn_bwd_dropout": (_i, [_p] * 9 + [_i] * 6 + [_i64] * 24 + [_f, _i, _i, _i, _p, _sz, _p, _f, _u64]),

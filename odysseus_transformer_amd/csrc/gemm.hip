@@ -510,6 +510,44 @@ extern "C" int ody_linear_swiglu(const void* x, const void* w_gate_up, void* gat
   return ody_swiglu_fwd(gate_up, h, T, I, ld_gu, ld_h, dtype, stream);
 }
 
+// The RMSNorm in front of a product of few rows, inside it: 16-byte rows, K % 8 == 0, rows that fit a block's LDS.
+namespace {
+bool norm_fits(const void* x, const void* norm_w, const void* w, const void* y, int M, int K, int64_t ldx, int64_t ldw, int64_t ldy) {
+  return M <= ODY_SKINNY_NORM_MAX_M && (size_t)M * (K + 8) * sizeof(bf16) <= ODY_SKINNY_NORM_BYTES && K % 8 == 0 && vec16(x, ldx) && vec16(w, ldw) && vec16(y, ldy) && ody_aligned16(norm_w);
+}
+}  // namespace
+
+extern "C" int ody_norm_linear_rope(const void* x, const void* norm_w, float eps, const void* w, const int64_t* position_ids,
+                                    const float* inv_freq, void* y, int M, int N, int K, int n_rot, int D, int64_t ldx, int64_t ldw,
+                                    int64_t ldy, int dtype, void* stream) {
+  int rc = check_lin("ody_norm_linear_rope", x, w, y, M, N, K, dtype);
+  if (rc) return rc;
+  ODY_REQUIRE(norm_w && position_ids && inv_freq, ODY_ERR_NULL, "ody_norm_linear_rope: NULL pointer");
+  ODY_REQUIRE(ldx >= K && ldw >= K && ldy >= N, ODY_ERR_BAD_SHAPE, "ody_norm_linear_rope: leading dimension smaller than the row length");
+  ODY_REQUIRE(n_rot >= 0 && D > 0 && N % D == 0 && n_rot <= N / D, ODY_ERR_BAD_SHAPE, "ody_norm_linear_rope: N=%d n_rot=%d D=%d", N, n_rot, D);
+  ODY_REQUIRE(dtype == ODY_BF16 && D == 128 && ody_gemm_skinny_ok(EPI_ROPE, M, N) && norm_fits(x, norm_w, w, y, M, K, ldx, ldw, ldy),
+              ODY_ERR_UNSUPPORTED, "ody_norm_linear_rope: bf16, head_dim 128, few rows on 16-byte boundaries");
+  GemmEpi ep{nullptr, nullptr, 0, 0, n_rot * D};
+  ep.norm = static_cast<const bf16*>(norm_w), ep.eps = eps, ep.positions = position_ids, ep.inv_freq = inv_freq;
+  return ody_launch_gemm_skinny(EPI_ROPE, static_cast<const bf16*>(x), static_cast<const bf16*>(w), static_cast<bf16*>(y), nullptr, M, N, K, ldx,
+                                ldw, ldy, 0, ep, static_cast<hipStream_t>(stream));
+}
+
+extern "C" int ody_norm_linear_swiglu_h(const void* x, const void* norm_w, float eps, const void* w_gate_up, void* h, int T, int I, int K,
+                                        int64_t ldx, int64_t ldw, int64_t ld_h, int dtype, void* stream) {
+  int rc = check_lin("ody_norm_linear_swiglu_h", x, w_gate_up, h, T, I, K, dtype);
+  if (rc) return rc;
+  ODY_REQUIRE(norm_w != nullptr, ODY_ERR_NULL, "ody_norm_linear_swiglu_h: NULL pointer");
+  ODY_REQUIRE(ldx >= K && ldw >= K && ld_h >= I, ODY_ERR_BAD_SHAPE, "ody_norm_linear_swiglu_h: leading dimension smaller than the row length");
+  ODY_REQUIRE(dtype == ODY_BF16 && I < (1 << 30) && ody_gemm_skinny_ok(EPI_SWIGLU_FWD, T, 2 * I) &&
+                  norm_fits(x, norm_w, w_gate_up, h, T, K, ldx, ldw, ld_h),
+              ODY_ERR_UNSUPPORTED, "ody_norm_linear_swiglu_h: bf16, few rows on 16-byte boundaries, I a multiple of 16");
+  GemmEpi ep{nullptr, static_cast<bf16*>(h), 0, ld_h, I};
+  ep.norm = static_cast<const bf16*>(norm_w), ep.eps = eps;
+  return ody_launch_gemm_skinny(EPI_SWIGLU_FWD, static_cast<const bf16*>(x), static_cast<const bf16*>(w_gate_up), nullptr, nullptr, T, 2 * I, K,
+                                ldx, ldw, 0, 0, ep, static_cast<hipStream_t>(stream));
+}
+
 extern "C" size_t ody_linear_dgrad_swiglu_workspace_bytes(int T, int I, int K, int dtype) {
   if (T <= 0 || I <= 0 || K <= 0) return 0;
   if (dtype == ODY_BF16 && I % 128 == 0 && K % 8 == 0) return 0;

@@ -16,10 +16,20 @@ struct GemmEpi {
   bf16* out2;
   int64_t ld_aux, ld_out2;
   int I;
+  // few rows only (gemm_skinny.hip): A is x, and the product that of its RMS-normalised rows (weight `norm` of K elements, or NULL);
+  // EPI_ROPE takes its angles from positions[row] * inv_freq[j], rounded as ody_rope_table rounds them, where there is no table
+  const bf16* norm;
+  float eps;
+  const int64_t* positions;
+  const float* inv_freq;
 };
 
 // C (M, N) = A (M, K) . W (N, K)^T for few rows of A (gemm_skinny.hip); EPI_NONE also takes a bias and accumulation into C.
 constexpr int ODY_SKINNY_MAX_M = 16;
+// The norm in front of a product of few rows (GemmEpi::norm): every block normalises them for itself, so only where that is quicker than
+// a launch of its own, and where the rows, 2 M (K + 8) bytes, fit the LDS.
+constexpr int ODY_SKINNY_NORM_MAX_M = 4;
+constexpr size_t ODY_SKINNY_NORM_BYTES = 64 << 10;
 bool ody_gemm_skinny_ok(int epi, int M, int N);
 int ody_launch_gemm_skinny(int epi, const bf16* A, const bf16* W, bf16* C, const bf16* bias, int M, int N, int K, int64_t lda,
                            int64_t ldw, int64_t ldc, int accumulate, const GemmEpi& ep, hipStream_t st);

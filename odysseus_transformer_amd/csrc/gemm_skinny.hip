@@ -15,12 +15,20 @@ namespace {
 
 constexpr int SK_WAVES = 8;
 
-template <int NT, int U, int EPI>
+// NORM: A is x, and the product that of its RMS-normalised rows.  Every block normalises them for itself, into LDS, with the arithmetic of
+// the RMSNorm kernel, while its first fragments of W are on their way; EPI_ROPE then takes its angles from the positions too.  Weights
+// cold, us without the norm / with it, one row: 6144 x 4096 with rotation 13.3 / 15.9, 22016 x 4096 SwiGLU 41.1 / 43.2, 5632 x 1024
+// 5.9 / 6.8; four rows 13.6 / 18.1, 43.4 / 47.1, 6.1 / 8.6.  The norm's own launch takes 2.6, the table's 2.0, and each its gap and 5 of host
+// work.  (The norm inside the K loop, on every fragment, took 16.2 and 46.6; a ring of fragments refilled one by one instead of a batch
+// at a time, without the norm, 14.9 and 41.6.)
+template <int NT, int U, int EPI, bool NORM>
 __global__ __launch_bounds__(64 * SK_WAVES) void gemm_skinny_kernel(const bf16* __restrict__ A, const bf16* __restrict__ W,
                                                                     bf16* __restrict__ C, const bf16* __restrict__ bias, int M,
                                                                     int N, int K, int64_t lda, int64_t ldw, int64_t ldc,
                                                                     int accumulate, GemmEpi ep) {
   __shared__ f32x4 red[SK_WAVES][NT][64];
+  __shared__ __attribute__((aligned(16))) bf16 angles[NORM && EPI == EPI_ROPE ? ODY_SKINNY_NORM_MAX_M : 1][16][2];
+  extern __shared__ __attribute__((aligned(16))) bf16 rows[];   // NORM: [M][K + 8]
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, c = lane & 15, q = lane >> 4;
   // first W row of group t of this block
   int row0[NT];
@@ -33,7 +41,7 @@ __global__ __launch_bounds__(64 * SK_WAVES) void gemm_skinny_kernel(const bf16* 
   const bf16* wp[NT];
 #pragma unroll
   for (int t = 0; t < NT; t++) wp[t] = W + (int64_t)min(row0[t] + c, N - 1) * ldw + 8 * q;
-  const bf16* ap = A + (int64_t)min(c, M - 1) * lda + 8 * q;
+  const bf16* ap = (NORM ? rows + min(c, M - 1) * (K + 8) : A + (int64_t)min(c, M - 1) * lda) + 8 * q;
 
   f32x4 acc[NT];
 #pragma unroll
@@ -51,13 +59,62 @@ __global__ __launch_bounds__(64 * SK_WAVES) void gemm_skinny_kernel(const bf16* 
   };
   int s = s0;
   const int whole = K / 32;   // steps that lie inside K for every lane
-  for (; s + U <= min(s1, whole); s += U) {
+  const int s_whole = min(s1, whole);
+  bool fetched = false;       // NORM: the first W fragments
+  if constexpr (NORM) {
+    fetched = s + U <= s_whole;
+    float* sums = reinterpret_cast<float*>(red);   // [M][SK_WAVES]
+    const int nvec = K / 8;
+    bf16x8 first = bf16x8{0, 0, 0, 0, 0, 0, 0, 0}, scale = first;
+    if (tid < nvec) first = *reinterpret_cast<const bf16x8*>(A + 8 * tid), scale = *reinterpret_cast<const bf16x8*>(ep.norm + 8 * tid);
+    if (fetched) {
+#pragma unroll
+      for (int u = 0; u < U; u++)
+#pragma unroll
+        for (int t = 0; t < NT; t++) wf[u][t] = *reinterpret_cast<const bf16x8*>(wp[t] + (int64_t)(s + u) * 32);
+    }
+    auto vector_of = [&](int r, int v) { return r == 0 && v == tid ? first : *reinterpret_cast<const bf16x8*>(A + (int64_t)r * lda + 8 * v); };
+    for (int r = 0; r < M; r++) {
+      float ss = 0.f;
+      for (int v = tid; v < nvec; v += 64 * SK_WAVES) {
+        const bf16x8 x = vector_of(r, v);
+#pragma unroll
+        for (int e = 0; e < 8; e++) ss = fmaf((float)x[e], (float)x[e], ss);
+      }
+#pragma unroll
+      for (int d = 32; d > 0; d >>= 1) ss += __shfl_xor(ss, d, 64);
+      if (lane == 0) sums[r * SK_WAVES + wave] = ss;
+    }
+    if (EPI == EPI_ROPE && tid < 16 * M) {   // the angles of this block's columns, one per thread, rounded as the table's
+      const float th = (float)ep.positions[tid >> 4] * ep.inv_freq[(row0[0] & 127) + (tid & 15)];
+      angles[tid >> 4][tid & 15][0] = (bf16)cosf(th), angles[tid >> 4][tid & 15][1] = (bf16)sinf(th);
+    }
+    __syncthreads();
+    for (int r = 0; r < M; r++) {
+      float ss = 0.f;
+#pragma unroll
+      for (int w = 0; w < SK_WAVES; w++) ss += sums[r * SK_WAVES + w];
+      const float rstd = rsqrtf(ss / (float)K + ep.eps);
+      for (int v = tid; v < nvec; v += 64 * SK_WAVES) {
+        const bf16x8 x = vector_of(r, v), n = v == tid ? scale : *reinterpret_cast<const bf16x8*>(ep.norm + 8 * v);
+        bf16x8 y;
+#pragma unroll
+        for (int e = 0; e < 8; e++) y[e] = (bf16)((float)n[e] * (float)(bf16)((float)x[e] * rstd));
+        *reinterpret_cast<bf16x8*>(rows + r * (K + 8) + 8 * v) = y;
+      }
+    }
+    __syncthreads();
+  }
+  for (; s + U <= s_whole; s += U) {
 #pragma unroll
     for (int u = 0; u < U; u++) {
+      if (!NORM || !fetched) {
 #pragma unroll
-      for (int t = 0; t < NT; t++) wf[u][t] = *reinterpret_cast<const bf16x8*>(wp[t] + (int64_t)(s + u) * 32);
+        for (int t = 0; t < NT; t++) wf[u][t] = *reinterpret_cast<const bf16x8*>(wp[t] + (int64_t)(s + u) * 32);
+      }
       af[u] = *reinterpret_cast<const bf16x8*>(ap + (int64_t)(s + u) * 32);
     }
+    fetched = false;
     multiply();
   }
   if (s < s1) {   // the remainder, all of it in flight at once
@@ -111,7 +168,7 @@ __global__ __launch_bounds__(64 * SK_WAVES) void gemm_skinny_kernel(const bf16* 
     const int n = row0[0] + 4 * q, j = n & 127;
     f32x4 o1 = v[0], o2 = v[1];
     if (n < ep.I) {
-      const bf16x8 cs = *reinterpret_cast<const bf16x8*>(ep.aux + (int64_t)row * ep.ld_aux + 2 * j);
+      const bf16x8 cs = *reinterpret_cast<const bf16x8*>(NORM ? angles[row][4 * q] : ep.aux + (int64_t)row * ep.ld_aux + 2 * j);
 #pragma unroll
       for (int e = 0; e < 4; e++) {
         const float co = (float)cs[2 * e], sn = (float)cs[2 * e + 1];
@@ -147,11 +204,14 @@ __global__ __launch_bounds__(64 * SK_WAVES) void gemm_skinny_kernel(const bf16* 
   }
 }
 
-template <int NT, int U, int EPI>
+template <int NT, int U, int EPI, bool NORM = false>
 int launch(const char* name, int blocks, const bf16* A, const bf16* W, bf16* C, const bf16* bias, int M, int N, int K, int64_t lda,
            int64_t ldw, int64_t ldc, int accumulate, const GemmEpi& ep, hipStream_t st) {
-  ODY_LAUNCH(name, st, (gemm_skinny_kernel<NT, U, EPI>), dim3(blocks), dim3(64 * SK_WAVES), 0, A, W, C, bias, M, N, K, lda, ldw,
-             ldc, accumulate, ep);
+  const size_t smem = NORM ? sizeof(bf16) * M * (K + 8) : 0;
+  auto kern = &gemm_skinny_kernel<NT, U, EPI, NORM>;
+  if (NORM)
+    if (int rc = ody_allow_dynamic_lds(reinterpret_cast<const void*>(kern), ODY_SKINNY_NORM_BYTES, name)) return rc;
+  ODY_LAUNCH(name, st, kern, dim3(blocks), dim3(64 * SK_WAVES), smem, A, W, C, bias, M, N, K, lda, ldw, ldc, accumulate, ep);
   return ody_check_launch(name);
 }
 
@@ -170,6 +230,11 @@ bool ody_gemm_skinny_ok(int epi, int M, int N) {
 int ody_launch_gemm_skinny(int epi, const bf16* A, const bf16* W, bf16* C, const bf16* bias, int M, int N, int K, int64_t lda,
                            int64_t ldw, int64_t ldc, int accumulate, const GemmEpi& ep, hipStream_t st) {
   const int groups = (N + 15) / 16;
+  if (ep.norm) {
+    if (epi == EPI_SWIGLU_FWD)
+      return launch<2, 8, EPI_SWIGLU_FWD, true>("gemm_skinny_norm_swiglu", groups / 2, A, W, C, bias, M, N, K, lda, ldw, ldc, accumulate, ep, st);
+    return launch<2, 8, EPI_ROPE, true>("gemm_skinny_norm_rope", groups / 2, A, W, C, bias, M, N, K, lda, ldw, ldc, accumulate, ep, st);
+  }
   if (epi == EPI_SWIGLU_FWD)
     return launch<2, 8, EPI_SWIGLU_FWD>("gemm_skinny_swiglu", groups / 2, A, W, C, bias, M, N, K, lda, ldw, ldc, accumulate, ep, st);
   if (epi == EPI_ROPE)

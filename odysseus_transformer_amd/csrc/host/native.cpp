@@ -36,7 +36,8 @@ namespace {
   X(ody_rmsnorm_fwd) X(ody_rmsnorm_bwd_partials) X(ody_rmsnorm_bwd) X(ody_gemm_workspace_bytes) X(ody_gemm) X(ody_linear_residual_ws) \
   X(ody_linear_rope_ws) X(ody_linear_swiglu) X(ody_linear_swiglu_h_fused) X(ody_linear_swiglu_h)                                  \
   X(ody_linear_dgrad_swiglu_workspace_bytes) X(ody_linear_dgrad_swiglu) X(ody_attn_fwd_workspace_bytes) X(ody_attn_fwd)           \
-  X(ody_attn_bwd_workspace_bytes) X(ody_attn_bwd) X(ody_attn_bwd_rope) X(ody_rope) X(ody_rope_table)
+  X(ody_attn_bwd_workspace_bytes) X(ody_attn_bwd) X(ody_attn_bwd_rope) X(ody_rope) X(ody_rope_table)           \
+  X(ody_norm_linear_rope) X(ody_norm_linear_swiglu_h)
 
 struct Library {
 #define X(name) decltype(&::name) name = nullptr;
@@ -392,6 +393,42 @@ PyObject* rope_table(Call c) {
   return wrap(table);
 }
 
+// What ody_norm_linear_* take: bf16 rows of x and of the weight on 16-byte boundaries, few of x.
+void check_norm_linear(const at::Tensor& x, const at::Tensor& norm, const at::Tensor& w) {
+  need(x.scalar_type() == at::kBFloat16 && x.size(0) <= 4 && x.size(0) * (x.size(1) + 8) * 2 <= 64 * 1024 && x.size(1) % 8 == 0 && w.size(1) == x.size(1));
+  need(norm.dim() == 1 && norm.is_contiguous() && norm.size(0) == x.size(1));
+  for (const at::Tensor* t : {&x, &norm, &w}) need(reinterpret_cast<uintptr_t>(t->data_ptr()) % 16 == 0);
+  need(pitch(x) % 8 == 0 && pitch(w) % 8 == 0);
+}
+
+// (x, norm_weight, eps, weight, n_rot, head_dim, position_ids, inv_freq) -> y
+PyObject* norm_linear_rope(Call c) {
+  const at::Tensor &x = c.matrix(0, nullptr), &norm = c.like(1, x), &w = c.matrix(3, &x);
+  check_norm_linear(x, norm, w);
+  const int64_t n_rot = c.whole(4), D = c.whole(5), M = x.size(0), K = x.size(1), N = w.size(0);
+  need(D == 128 && N % D == 0 && n_rot >= 0 && n_rot <= N / D && !c.none(6));
+  const float eps = (float)c.real(2);
+  const int64_t* pos = positions(c, 6, M);
+  const at::Tensor& f = frequencies(c, 7, D);
+  at::Tensor y = make({M, N}, x);
+  CALL(ody_norm_linear_rope, x.data_ptr(), norm.data_ptr(), eps, w.data_ptr(), pos, f.data_ptr<float>(), y.data_ptr(), (int)M, (int)N, (int)K,
+       (int)n_rot, (int)D, pitch(x), pitch(w), y.stride(0), dt(x), (void*)c.stream);
+  return wrap(y);
+}
+
+// (x, norm_weight, eps, w_gate_up) -> h
+PyObject* norm_linear_swiglu_h(Call c) {
+  const at::Tensor &x = c.matrix(0, nullptr), &norm = c.like(1, x), &w = c.matrix(3, &x);
+  check_norm_linear(x, norm, w);
+  const int64_t T = x.size(0), K = x.size(1), I = w.size(0) / 2;
+  need(w.size(0) % 32 == 0);
+  const float eps = (float)c.real(2);
+  at::Tensor h = make({T, I}, x);
+  CALL(ody_norm_linear_swiglu_h, x.data_ptr(), norm.data_ptr(), eps, w.data_ptr(), h.data_ptr(), (int)T, (int)I, (int)K, pitch(x), pitch(w),
+       h.stride(0), dt(x), (void*)c.stream);
+  return wrap(h);
+}
+
 // the raw stream that the ops above launch on
 PyObject* current_stream(Call) {
   return PyLong_FromVoidPtr((void*)c10::hip::getCurrentHIPStream(c10::hip::current_device()).stream());
@@ -441,6 +478,7 @@ PyMethodDef methods[] = {
     {"bind", (PyCFunction)(void (*)(void))bind, METH_FASTCALL, nullptr},
     METHOD(rmsnorm_fwd, 3), METHOD(rmsnorm_bwd, 5), METHOD(gemm, 3), METHOD(linear_residual, 3), METHOD(linear_rope, 5), METHOD(linear_swiglu, 2),
     METHOD(linear_swiglu_h, 2), METHOD(linear_dgrad_swiglu, 3), METHOD(attn_fwd, 5), METHOD(attn_bwd, 13), METHOD(rope, 6), METHOD(rope_table, 5),
+    METHOD(norm_linear_rope, 8), METHOD(norm_linear_swiglu_h, 4),
     METHOD(current_stream, 0), {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_odysseus_native", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 

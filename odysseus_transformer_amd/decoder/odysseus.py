@@ -150,12 +150,21 @@ class LlamaFlashAttention2TPSP(nn.Module):
         scale = 1.0 / math.sqrt(self.head_dim)
         nh, nkv, D = self.n_local_heads, self.n_local_kv_heads, self.head_dim
 
+        norm = kwargs.get("input_norm")   # an extension: hidden_states come before this norm, see OdysseusDecoderLayer._folds_norms
+        if norm is not None and not (general and self.pack_weight and self._can_fuse_rope(hidden_states)):
+            hidden_states, norm = norm(hidden_states), None
+
         if self.pack_weight:
             q_len = local_q_len * get_model_parallel_world_size()
             if not self.sequence_parallel:
                 hidden_states = allgather_bsz1(hidden_states)
             if general:
-                if self._can_fuse_rope(hidden_states):   # the rotation rides in the projection's epilogue
+                if norm is not None:   # ... and the norm in its prologue
+                    if position_ids is not None:
+                        ops.check_position_ids(position_ids, bsz, q_len, hidden_states.device)
+                    qkv = ops.norm_linear_rope(hidden_states.reshape(q_len, -1), norm.weight, norm.variance_epsilon, self.qkv_proj.weight,
+                                               nh + nkv, D, position_ids, self.rope_theta).view(bsz, q_len, nh + 2 * nkv, D)
+                elif self._can_fuse_rope(hidden_states):   # the rotation rides in the projection's epilogue
                     qkv = ops.run_function(ops.LinearRoPEFunc, hidden_states, self.qkv_proj.weight, nh + nkv, D, position_ids,
                                            self.rope_theta)
                 else:
@@ -276,9 +285,10 @@ class LlamaMLPZeRO(nn.Module):
         # SwiGLU (and its backward) inside the products' epilogues; False keeps one kernel per step
         self.fuse_elementwise = True
 
-    def forward(self, x, residual=None):
+    def forward(self, x, residual=None, input_norm=None):
         """`residual` (an extension: the reference's module takes x only) makes the result
-        residual + mlp(x) with every elementwise step fused into the products' epilogues."""
+        residual + mlp(x) with every elementwise step fused into the products' epilogues.  `input_norm`: x comes
+        before this norm (OdysseusDecoderLayer._folds_norms)."""
         if getattr(self.config, "pretraining_tp", 1) > 1:
             raise NotImplementedError("pretraining_tp > 1 is not supported yet.")
         w1, w2 = self.gate_up_proj.weight, self.down_proj.weight
@@ -286,6 +296,11 @@ class LlamaMLPZeRO(nn.Module):
                    and x.dtype == w1.dtype == w2.dtype and (residual is None or residual.dtype == x.dtype)
                    and not _has_hooks(self.gate_up_proj, self.down_proj)
                    and not torch.is_autocast_enabled("cuda"))
+        if input_norm is not None:
+            if fusable and self.fuse_elementwise and residual is not None:
+                h = ops.norm_linear_swiglu_h(x.reshape(-1, x.shape[-1]), input_norm.weight, input_norm.variance_epsilon, w1)
+                return ops.linear_residual(h, w2, residual.reshape(-1, residual.shape[-1])).view(residual.shape)
+            x = input_norm(x)
         if fusable and self.fuse_elementwise:
             return ops.run_function(ops.SwiGLUMLPResidualFunc, x, w1, w2, residual)
         y = self.down_proj(ops.swiglu(self.gate_up_proj(x)))
@@ -338,6 +353,10 @@ class OdysseusDecoderLayer(nn.Module):
     def _forward(self, hidden_states, attention_mask=None, position_ids=None, **kwargs):
         # what a host model hands its decoder layers besides (a cache to fill during a prefill)
         cache = {k: kwargs[k] for k in ("past_key_value", "past_key_values", "cache_position") if kwargs.get(k) is not None}
+        if self.fused and self._folds_norms(hidden_states):
+            h = self.self_attn(hidden_states, attention_mask=attention_mask, position_ids=position_ids, residual=hidden_states,
+                               input_norm=self.input_layernorm, **cache)[0]
+            return self.mlp(h, residual=h, input_norm=self.post_attention_layernorm)
         if self.fused:
             n1, skip = ops.rmsnorm_fork(hidden_states, self.input_layernorm.weight, self.input_layernorm.variance_epsilon)
             h = self.self_attn(n1, attention_mask=attention_mask, position_ids=position_ids, residual=skip, **cache)[0]
@@ -351,6 +370,17 @@ class OdysseusDecoderLayer(nn.Module):
         residual = hidden_states
         hidden_states = self.mlp(self.post_attention_layernorm(hidden_states))
         return residual + hidden_states
+
+
+    def _folds_norms(self, hidden_states) -> bool:
+        """A decoding step, or a handful of tokens that nothing records: the modules get the rows before their norm and the norm, which
+        then rides in the prologue of their first product.  Only where nobody else would see those rows instead of the normalised
+        ones: no hooks, and the modules that this class made."""
+        attn, mlp, norms = self.self_attn, self.mlp, (self.input_layernorm, self.post_attention_layernorm)
+        return (hidden_states.is_cuda and hidden_states.dtype == torch.bfloat16 and hidden_states.dim() == 3
+                and hidden_states.shape[0] * hidden_states.shape[1] <= ops.NORM_LINEAR_MAX_ROWS and not ops.watched()
+                and type(attn) is LlamaFlashAttention2TPSP and type(mlp) is LlamaMLPZeRO
+                and all(type(n) is LlamaRMSNorm and n.weight.dtype == torch.bfloat16 for n in norms) and not _has_hooks(attn, mlp, *norms))
 
 
 def _has_hooks(*modules) -> bool:

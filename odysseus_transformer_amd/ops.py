@@ -63,10 +63,15 @@ def run_function(fn, *args):
     """fn.apply(*args), or fn's forward alone where nothing looks at the call: under no_grad / inference mode an inference step is
     a handful of small launches, and the autograd machinery around each costs more host time (8-10 us) than the launch itself.
     Forward-mode differentiation, function transforms and tracing go on under no_grad and see the call only through apply."""
-    if (torch.is_grad_enabled() or torch.autograd.forward_ad._current_level >= 0 or torch._C._are_functorch_transforms_active()
-            or torch._C._get_tracing_state() is not None):
+    if watched():
         return fn.apply(*args)
     return fn.forward(_NO_CONTEXT, *args)
+
+
+def watched() -> bool:
+    """Whether anything may look at a call through autograd's machinery."""
+    return (torch.is_grad_enabled() or torch.autograd.forward_ad._current_level >= 0 or torch._C._are_functorch_transforms_active()
+            or torch._C._get_tracing_state() is not None)
 
 
 def scratch(nbytes: int, name: str, device) -> torch.Tensor:
@@ -572,6 +577,29 @@ def linear_rope(x, weight, table, n_rot: int, head_dim: int):
               _rowmajor2d(x, "x"), _rowmajor2d(weight, "weight"), table.stride(0), y.stride(0), _dt(x),
               0 if ws is None else ws.data_ptr(), ws_bytes, _stream())
     return y
+
+
+NORM_LINEAR_MAX_ROWS = 4   # the C ABI's limit for the two below
+
+
+def norm_linear_rope(x, norm_weight, eps: float, weight, n_rot: int, head_dim: int, position_ids, base: float = 10000.0):
+    """linear_rope of the RMS-normalised rows of x (M, K), the angles from the M positions: one kernel for few rows, the norm, the
+    table and the product for others.  No autograd."""
+    if x.is_cuda and position_ids is not None:
+        plain = native.norm_linear_rope(x, norm_weight, eps, weight, n_rot, head_dim, position_ids, rope_inv_freq(head_dim, base, x.device))
+        if plain is not None:
+            return plain
+    table = _new_rope_table(position_ids, x.shape[0], head_dim, base, x.device)
+    return linear_rope(rmsnorm_fwd(x, norm_weight, eps)[0], weight, table, n_rot, head_dim)
+
+
+def norm_linear_swiglu_h(x, norm_weight, eps: float, w_gate_up):
+    """linear_swiglu_h of the RMS-normalised rows of x (T, K): one kernel for few rows.  No autograd."""
+    if x.is_cuda:
+        plain = native.norm_linear_swiglu_h(x, norm_weight, eps, w_gate_up)
+        if plain is not None:
+            return plain
+    return linear_swiglu_h(rmsnorm_fwd(x, norm_weight, eps)[0], w_gate_up)
 
 
 def linear_swiglu(x, w_gate_up):

@@ -192,3 +192,76 @@ def test_what_it_leaves_alone(dev, monkeypatch):
         assert g.get_global_memory_buffer().buffer[("gemm_workspace", torch.uint8)].numel() > 0
     finally:
         g._destroy_global_memory_buffer()
+
+
+@pytest.mark.parametrize("rows", [1, 3, 4, 5])
+@pytest.mark.parametrize("K", [8, 40, 512, 4096, 9000], ids=lambda k: "K%d" % k)
+def test_norm_inside_a_product_of_few_rows(K, rows, dev, monkeypatch):
+    """One kernel against the norm, the table and the product: the same but for the order of the norm's sum (an ulp of 1 / rms, which
+    can move a rounding of the normalised row); beyond 4 rows and 64 KiB the three of them."""
+    from odysseus_transformer_amd import ops
+    print(f"K={K} rows={rows}", flush=True)
+    x, nw = randn((rows, K), 1, dtype=torch.bfloat16).to(dev), (1 + 0.1 * randn((K,), 2)).bfloat16().to(dev)
+    wq, wg = randn((640, K), 3, std=0.05, dtype=torch.bfloat16).to(dev), randn((96, K), 4, std=0.05, dtype=torch.bfloat16).to(dev)
+    pos = torch.tensor([0, 70001, 5, 1 << 20, 9], device=dev)[:rows]
+    for fn, one in ((lambda: ops.norm_linear_rope(x, nw, 1e-6, wq, 3, 128, pos), "norm_linear_rope"),
+                    (lambda: ops.norm_linear_swiglu_h(x, nw, 1e-6, wg), "norm_linear_swiglu_h")):
+        here, there, taken = _both(monkeypatch, fn)
+        assert (one in taken) == (rows <= 4 and 2 * rows * (K + 8) <= 1 << 16)
+        assert here.shape == there.shape and here.dtype == there.dtype
+        assert (here.float() - there.float()).norm() <= 2.0 ** -9 * there.float().norm()
+    n = (x.double() * (x.double().square().mean(-1, keepdim=True) + 1e-6).rsqrt() * nw.double())
+    g, u = (n @ wg.double().t()).chunk(2, -1)
+    ref = torch.nn.functional.silu(g) * u
+    assert (ops.norm_linear_swiglu_h(x, nw, 1e-6, wg).double() - ref).norm() <= 1e-2 * ref.norm()
+
+
+def test_norm_inside_a_product_with_infinities(dev):
+    from odysseus_transformer_amd import ops
+    x, nw = randn((3, 256), 1, dtype=torch.bfloat16), torch.ones(256, dtype=torch.bfloat16)
+    x[0, 3], x[1, 7] = float("inf"), float("nan")
+    w = randn((64, 256), 2, std=0.05, dtype=torch.bfloat16)
+    w[5, 250] = float("inf")
+    x, nw, w = x.to(dev), nw.to(dev), w.to(dev)
+    here, there = ops.norm_linear_swiglu_h(x, nw, 1e-6, w), ops.linear_swiglu_h(ops.rmsnorm_fwd(x, nw)[0], w)
+    assert torch.equal(here.isnan(), there.isnan()) and torch.equal(here.isinf(), there.isinf())
+    ok = there.isfinite()
+    assert (here[ok].float() - there[ok].float()).norm() <= 2.0 ** -9 * there[ok].float().norm()
+
+
+def test_decoding_layer_folds_its_norms_and_gives_hooks_what_they_had(dev):
+    import types
+    from transformers import DynamicCache
+    from odysseus_transformer_amd import _lib, ops
+    from odysseus_transformer_amd.decoder.odysseus import OdysseusDecoderLayer
+    cfg = types.SimpleNamespace(hidden_size=512, num_attention_heads=4, num_key_value_heads=2, head_dim=128, intermediate_size=1408,
+                                hidden_act="silu", attention_dropout=0.0, rms_norm_eps=1e-6, rope_theta=10000.0, pretraining_tp=1)
+    torch.manual_seed(0)
+    layer = OdysseusDecoderLayer(cfg).bfloat16().to(dev)
+    with torch.no_grad():
+        for p in layer.parameters():
+            p.normal_(0.0 if p.dim() > 1 else 1.0, 0.05)
+    x = randn((1, 34, 512), 1, dtype=torch.bfloat16).to(dev)
+
+    def step(hooked):
+        cache = DynamicCache()
+        with torch.no_grad():
+            layer(x[:, :33], position_ids=torch.arange(33, device=dev)[None], past_key_values=cache)
+            seen = []
+            h = layer.self_attn.register_forward_pre_hook(lambda m, a: seen.append(a[0])) if hooked else None
+            _lib.profile_enable(True)
+            _lib.profile_collect()
+            try:
+                y = layer(x[:, 33:], position_ids=torch.arange(33, 34, device=dev)[None], past_key_values=cache)
+                ran = set(_lib.profile_collect())
+            finally:
+                _lib.profile_enable(False)
+                if h is not None:
+                    h.remove()
+        return y, ran, seen
+
+    y, ran, _ = step(False)
+    assert {"gemm_skinny_norm_rope", "gemm_skinny_norm_swiglu"} <= ran and "rmsnorm_fwd" not in ran
+    z, ran, seen = step(True)
+    assert "rmsnorm_fwd" in ran and torch.equal(seen[0], ops.rmsnorm(x[:, 33:], layer.input_layernorm.weight, 1e-6))
+    assert (y.float() - z.float()).norm() <= 1e-2 * z.float().norm()
