@@ -226,17 +226,19 @@ __global__ __launch_bounds__(256) void gemm_splitk_rope_kernel(const float* __re
 // 128 x 256, 1200 with 128 x 128); with 1000 rows, for instance, 4096 x 11008 takes 156 us on its 64 tiles of 256 x 256, 99 us
 // on 256 tiles of 128 x 128 and 84 us on 128 tiles of 128 x 256 with K in two ranges.
 //
-// Where a last round of 256 x 256 tiles would leave more than half of the units idle, its tiles are worked on as two half tiles
-// each, by other blocks of the same launch: a round of half tiles takes 0.58 of a whole one.  (Same sums in the same order: the
-// result does not depend on it.)  Same box, us without / with: QKV of 3001 tokens (288 tiles) 183 / 150, gate_up of 1000 tokens
-// (344) 183 / 161, of 3001 (1032) 484 / 453, four weight gradients over 1000 tokens 394 / 371.
-struct Plan { int bm, bn, splits, halved; };
+// Where a last round of 256 x 256 tiles would leave more than half of the units idle, its tiles are worked on as two half or four
+// quarter tiles each, by other blocks of the same launch: a round of halves takes 0.58 of a whole one, of quarters 0.44 (0.27 where
+// they are few).  (Same sums in the same order: the result does not depend on it.)  Same box, us whole / halves: QKV of 3001 tokens (288
+// tiles) 183 / 150, gate_up of 1000 tokens (344) 183 / 161, of 3001 (1032) 484 / 453, four weight gradients over 1000 tokens 394 / 371.
+// Halves / quarters: QKV of 3001 tokens 141 / 136, gate_up of 2100 (774) 333 / 325, of 3001 428 / 421, its input gradient of 5000 (320)
+// 778 / 745.
+struct Plan { int bm, bn, splits, cut, cut_parts; };
 
 Plan plan_bf16(int M, int N, int K, bool may_split) {
   struct Tile { int bm, bn, per_cu; double idle_us, full_us; };
   static const Tile tiles[] = {{256, 256, 1, 0.80, 1.42}, {128, 256, 1, 0.55, 0.83}, {128, 128, 2, 0.35, 0.90}};
   const int slabs = (K + BK - 1) / BK;
-  Plan best{256, 256, 1, 0};
+  Plan best{256, 256, 1, 0, 1};
   double best_us = 1e30;
   for (const Tile& t : tiles) {
     const int64_t tiles_mn = (int64_t)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
@@ -247,11 +249,13 @@ Plan plan_bf16(int M, int N, int K, bool may_split) {
       if (rest) per_slab += t.idle_us + (t.full_us - t.idle_us) * rest / slots;
       double us = per_slab * ((slabs + s - 1) / s) + 4.0 * (full + (rest > 0));
       if (s > 1) us += 2.0 + (double)s * M * N * 8.0 / 6.0e6;
-      if (us < best_us) best_us = us, best = Plan{t.bm, t.bn, s, 0};
-      if (t.bm == 256 && s == 1 && full > 0 && rest > 0 && 2 * rest <= slots) {
-        const Tile& h = tiles[1];
-        const double with_halves = (full * t.full_us + h.idle_us + (h.full_us - h.idle_us) * 2 * rest / slots) * slabs + 4.0 * (full + 1);
-        if (with_halves < best_us) best_us = with_halves, best = Plan{t.bm, t.bn, 1, (int)rest};
+      if (us < best_us) best_us = us, best = Plan{t.bm, t.bn, s, 0, 1};
+      if (t.bm != 256 || s != 1 || full == 0 || rest == 0) continue;
+      for (int parts = 2; parts <= 4 && parts * rest <= 256; parts *= 2) {
+        const Tile& h = tiles[parts / 2];
+        const double last = h.idle_us + (h.full_us - h.idle_us) * parts * rest / (256 * h.per_cu);
+        const double cut_us = (full * t.full_us + last) * slabs + 4.0 * (full + 1);
+        if (cut_us < best_us) best_us = cut_us, best = Plan{t.bm, t.bn, 1, (int)rest, parts};
       }
     }
   }
@@ -286,7 +290,7 @@ int launch_any_pitch(const gemm_tile::Args& a, int accumulate, hipStream_t st) {
 }
 
 int launch_tiles(int op, int epi, const Plan& pl, gemm_tile::Args a, hipStream_t st) {
-  a.halved = pl.halved;
+  a.cut = pl.cut, a.cut_parts = pl.cut_parts;
   if (op == ODY_GEMM_NT) return ody_launch_gemm_nt(epi, pl.bm, pl.bn, pl.splits, a, st);
   if (op == ODY_GEMM_NN) return ody_launch_gemm_nn(epi, pl.bm, pl.bn, pl.splits, a, st);
   return ody_launch_gemm_tn(pl.bm, pl.bn, pl.splits, a, st);

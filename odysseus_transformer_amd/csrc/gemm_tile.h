@@ -46,7 +46,7 @@ struct Args {
   int M, N, K;
   int64_t lda, ldb, ldc, ld_add;
   int tiles_m, tiles_n;
-  int halved;         // the last tiles of the walk, worked on as two half tiles each (256 x 256 only)
+  int cut, cut_parts; // the last `cut` tiles of the walk are worked on as 2 half or 4 quarter tiles each (256 x 256, K in one range)
   int vec16;          // C (and add) have 16-byte aligned rows
   GemmEpi ep;
 };
@@ -465,16 +465,17 @@ __device__ __forceinline__ void gemm_tile_block(const Args& p, int m0, int tn) {
 #undef ODY_FENCE
 
 // Block -> tile: a walk down M in groups of 8 tiles, so that the tiles in flight share panels of both operands; first the whole
-// tiles, then, two blocks each, those whose halves fill a last round better (plan_bf16).
-template <bool A_KC, bool B_KC, int BM, int BN, bool SPLITK, int EPI>
+// tiles, then, PARTS blocks each, those whose halves or quarters fill a last round better (plan_bf16).  (One kernel for both: 0.3 %
+// slower where halves are taken.)
+template <bool A_KC, bool B_KC, int BM, int BN, bool SPLITK, int EPI, int PARTS>
 __global__ __launch_bounds__(THREADS, BM * BN <= 128 * 128 ? 4 : 2) void gemm_tile_kernel(const Args p) {
-  const int whole = p.tiles_m * p.tiles_n - p.halved;
-  int pos = blockIdx.x, half = 0;
-  const bool in_half = BM == 256 && !SPLITK && pos >= whole;
-  if (in_half) {
-    pos = xcd_position(pos - whole, 2 * p.halved);
-    half = pos & 1;
-    pos = whole + (pos >> 1);
+  const int whole = p.tiles_m * p.tiles_n - p.cut;
+  int pos = blockIdx.x, part = 0;
+  const bool in_part = BM == 256 && !SPLITK && pos >= whole;
+  if (in_part) {
+    pos = xcd_position(pos - whole, PARTS * p.cut);
+    part = pos % PARTS;
+    pos = whole + pos / PARTS;
   } else {
     pos = xcd_position(pos, whole);
   }
@@ -482,24 +483,38 @@ __global__ __launch_bounds__(THREADS, BM * BN <= 128 * 128 ? 4 : 2) void gemm_ti
   const int per_group = GROUP * p.tiles_n, first_m = pos / per_group * GROUP, gsz = min(p.tiles_m - first_m, GROUP);
   const int m0 = (first_m + (pos % per_group) % gsz) * BM, tn = (pos % per_group) / gsz;
   if constexpr (BM == 256 && !SPLITK) {
-    if (in_half) {
-      if (m0 + 128 * half < p.M) gemm_tile_block<A_KC, B_KC, 128, BN, SPLITK, EPI>(p, m0 + 128 * half, tn);
+    if (in_part) {
+      const int mp = m0 + 128 * (part & 1);
+      if (mp >= p.M) return;
+      if constexpr (PARTS == 2) {
+        gemm_tile_block<A_KC, B_KC, 128, BN, SPLITK, EPI>(p, mp, tn);
+      } else {
+        const int np = 2 * tn + (part >> 1);
+        if (np * (EPI == EPI_SWIGLU_FWD ? BN / 4 : BN / 2) < (EPI == EPI_SWIGLU_FWD ? p.ep.I : p.N))
+          gemm_tile_block<A_KC, B_KC, 128, BN / 2, SPLITK, EPI>(p, mp, np);
+      }
       return;
     }
   }
   gemm_tile_block<A_KC, B_KC, BM, BN, SPLITK, EPI>(p, m0, tn);
 }
 
-template <bool A_KC, bool B_KC, int BM, int BN, bool SPLITK, int EPI>
-int launch(const char* name, Args a, int splits, hipStream_t st) {
+template <bool A_KC, bool B_KC, int BM, int BN, bool SPLITK, int EPI, int PARTS>
+int launch_parts(const char* name, Args a, int splits, hipStream_t st) {
   constexpr size_t smem = sizeof(bf16) * BK * (A_STAGES * BM + B_STAGES * BN);
   static_assert(smem >= 8 * 32 * (BN / 4 + 4) * sizeof(float), "the fp32 bands fit in the operand stages");
-  auto kern = &gemm_tile_kernel<A_KC, B_KC, BM, BN, SPLITK, EPI>;
+  auto kern = &gemm_tile_kernel<A_KC, B_KC, BM, BN, SPLITK, EPI, PARTS>;
   if (int rc = ody_allow_dynamic_lds(reinterpret_cast<const void*>(kern), smem, name)) return rc;
   a.tiles_m = (a.M + BM - 1) / BM, a.tiles_n = (a.N + BN - 1) / BN;
   if (EPI == EPI_SWIGLU_FWD) a.tiles_n = (a.ep.I + BN / 2 - 1) / (BN / 2);
-  ODY_LAUNCH(name, st, kern, dim3(a.tiles_m * a.tiles_n + a.halved, splits), dim3(THREADS), smem, a);
+  ODY_LAUNCH(name, st, kern, dim3(a.tiles_m * a.tiles_n + (PARTS - 1) * a.cut, splits), dim3(THREADS), smem, a);
   return ody_check_launch(name);
+}
+template <bool A_KC, bool B_KC, int BM, int BN, bool SPLITK, int EPI>
+int launch(const char* name, const Args& a, int splits, hipStream_t st) {
+  if constexpr (BM == 256 && !SPLITK)
+    if (a.cut_parts == 4) return launch_parts<A_KC, B_KC, BM, BN, SPLITK, EPI, 4>(name, a, splits, st);
+  return launch_parts<A_KC, B_KC, BM, BN, SPLITK, EPI, 2>(name, a, splits, st);
 }
 
 }  // namespace gemm_tile

@@ -228,3 +228,42 @@ def test_fp32_slab_pipeline(op, M, N, K, dev):
     ad, bd = a.double().to(dev), b.double().to(dev)
     want, bound = ad @ bd.t(), (K + 2) * 2.0 ** -24 * (ad.abs() @ bd.abs().t())
     assert ((got.double() - want).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("M", [4100, 4104, 4216, 4360, 8200], ids=lambda m: "M%d" % m)
+@pytest.mark.parametrize("what", ["nt", "nn", "tn", "rope", "swiglu", "residual"])
+def test_tiles_of_a_nearly_empty_last_round(what, M, dev):
+    """272 to 528 tiles of 256 x 256 on 256 compute units: the last ones run in halves or quarters, some of them past the edge.  Same
+    bits as a call whose tiles fill its one round, and right beyond it."""
+    from odysseus_transformer_amd import ops
+    dt, K, N = torch.bfloat16, 192, 3968
+    print(f"what={what} M={M}", flush=True)
+    M = (M + 7) // 8 * 8 if what == "tn" else M
+    x, w = randn((M, K), 1, dtype=dt).to(dev), randn((N, K), 2, std=0.05, dtype=dt).to(dev)
+    r = randn((M, N), 3, dtype=dt).to(dev)
+
+    def run(x, r):
+        if what == "nt":
+            return ops.gemm(ops.GEMM_NT, x, w)
+        if what == "nn":
+            return ops.gemm(ops.GEMM_NN, x, w.t().contiguous())
+        if what == "tn":
+            return ops.gemm(ops.GEMM_TN, x.t().contiguous(), w.t().contiguous())
+        if what == "rope":
+            return ops.linear_rope(x, w, ops.rope_table(torch.arange(x.shape[0], device=dev), x.shape[0], 128), 20, 128)
+        if what == "swiglu":
+            return ops.linear_swiglu(x, w)[1]
+        return ops.linear_residual(x, w, r)
+
+    y = run(x, r)
+    assert torch.equal(y[:4096], run(x[:4096], r[:4096]))
+    ref = x.float() @ w.float().t()
+    if what == "rope":
+        return   # the rows beyond the first round: one more call on them alone, with their own positions, is another table
+    if what == "swiglu":
+        g, u = ref.chunk(2, -1)
+        ref = torch.nn.functional.silu(g.to(dt).float()) * u.to(dt).float()
+    if what == "residual":
+        ref = ref + r.float()
+    assert rel_err(y, ref.cpu()) <= TOL_BF16
+    assert rel_err(y[4096:], ref[4096:].cpu()) <= TOL_BF16
