@@ -17,7 +17,7 @@
 #include <algorithm>
 #include <type_traits>
 #include <utility>
-#include "attn_params.h"
+#include "attn_store.h"
 #include "attn_tile.h"
 
 namespace {
@@ -26,61 +26,6 @@ using namespace tile128;
 
 constexpr int D = 128, KS = D / 16, DT = D / 32;
 #define FENCE() __builtin_amdgcn_sched_barrier(0)
-
-// dQ^T of one query held by lane group g (accumulator rows 8 (r >> 2) + 4 g + (r & 3) of each 32-wide slice of the
-// head dimension) -> row qi of dq: scaled, then added to an fp32 or bf16 destination, rotated back by the rotary
-// table, or rounded and stored.
-__device__ __forceinline__ void store_dq_row(const AttnParams& p, const f32x16 (&dq)[DT], int b, int h, int qi, int g) {
-  if (qi >= p.Lq) return;
-  if (p.dq_f32) {
-    // fp32 destination (the ring step's running dq): exact accumulation over the key blocks, no rounding here
-    float* dqp = static_cast<float*>(p.dq) + b * p.sdq.b + h * p.sdq.h + (int64_t)qi * p.sdq.l;
-#pragma unroll
-    for (int dt = 0; dt < DT; dt++)
-#pragma unroll
-      for (int a = 0; a < 4; a++) {
-        f32x4* dst = reinterpret_cast<f32x4*>(dqp + 32 * dt + 8 * a + 4 * g);
-        f32x4 w = {0.f, 0.f, 0.f, 0.f};
-        if (p.accumulate_dq) w = *dst;
-#pragma unroll
-        for (int e = 0; e < 4; e++) w[e] += dq[dt][4 * a + e] * p.scale;
-        *dst = w;
-      }
-  } else if (p.rope_q) {
-    // the gradient of the un-rotated projection: element d < 64 pairs with d + 64, both in this lane
-    bf16* dqp = static_cast<bf16*>(p.dq) + b * p.sdq.b + h * p.sdq.h + (int64_t)qi * p.sdq.l;
-    const bf16* trow = p.rope_q + ((int64_t)b * p.Lq + qi) * D;
-#pragma unroll
-    for (int dt = 0; dt < 2; dt++)
-#pragma unroll
-      for (int a = 0; a < 4; a++) {
-        const bf16x8 cs = *reinterpret_cast<const bf16x8*>(trow + 2 * (32 * dt + 8 * a + 4 * g));
-        bf16x4 w1, w2;
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-          const float c = (float)cs[2 * e], sn = (float)cs[2 * e + 1];
-          const float g1 = dq[dt][4 * a + e] * p.scale, g2 = dq[dt + 2][4 * a + e] * p.scale;
-          w1[e] = (bf16)(g1 * c + g2 * sn);
-          w2[e] = (bf16)(g2 * c - g1 * sn);
-        }
-        *reinterpret_cast<bf16x4*>(dqp + 32 * dt + 8 * a + 4 * g) = w1;
-        *reinterpret_cast<bf16x4*>(dqp + 32 * (dt + 2) + 8 * a + 4 * g) = w2;
-      }
-  } else {
-    bf16* dqp = static_cast<bf16*>(p.dq) + b * p.sdq.b + h * p.sdq.h + (int64_t)qi * p.sdq.l;
-#pragma unroll
-    for (int dt = 0; dt < DT; dt++)
-#pragma unroll
-      for (int a = 0; a < 4; a++) {
-        bf16x4* dst = reinterpret_cast<bf16x4*>(dqp + 32 * dt + 8 * a + 4 * g);
-        bf16x4 w, old = {0, 0, 0, 0};
-        if (p.accumulate_dq) old = *dst;
-#pragma unroll
-        for (int e = 0; e < 4; e++) w[e] = (bf16)(dq[dt][4 * a + e] * p.scale + (float)old[e]);
-        *dst = w;
-      }
-  }
-}
 
 // The same accumulators as one part's unscaled fp32 sum (a dQ kernel whose key range is cut into parts):
 // dq_part [part][B][Lq][Hq][D]; attn_bwd_dq_sum_kernel adds the parts and finishes dq as store_dq_row would.
@@ -545,9 +490,7 @@ __global__ __launch_bounds__(KV_THREADS) void attn_bwd_dkdv_pipe_kernel(const At
         }
     }
   } else if (key < p.Lk) {
-    bf16* dkp = static_cast<bf16*>(p.dk) + b * p.sdk.b + hk * p.sdk.h + (int64_t)key * p.sdk.l;
     bf16* dvp = static_cast<bf16*>(p.dv) + b * p.sdv.b + hk * p.sdv.h + (int64_t)key * p.sdv.l;
-    const bf16* trow = p.rope_k ? p.rope_k + ((int64_t)b * p.Lk + key) * D : nullptr;
 #pragma unroll
     for (int dt = 0; dt < DT; dt++)
 #pragma unroll
@@ -557,34 +500,7 @@ __global__ __launch_bounds__(KV_THREADS) void attn_bwd_dkdv_pipe_kernel(const At
         for (int e = 0; e < 4; e++) wv[e] = (bf16)dv[dt][4 * a + e];
         *reinterpret_cast<bf16x4*>(dvp + 32 * dt + 8 * a + 4 * g) = wv;
       }
-    if (trow) {   // dK of the un-rotated projection: element d < 64 pairs with d + 64, both in this lane
-#pragma unroll
-      for (int dt = 0; dt < 2; dt++)
-#pragma unroll
-        for (int a = 0; a < 4; a++) {
-          const bf16x8 cs = *reinterpret_cast<const bf16x8*>(trow + 2 * (32 * dt + 8 * a + 4 * g));
-          bf16x4 w1, w2;
-#pragma unroll
-          for (int e = 0; e < 4; e++) {
-            const float c = (float)cs[2 * e], sn = (float)cs[2 * e + 1];
-            const float g1 = dk[dt][4 * a + e] * p.scale, g2 = dk[dt + 2][4 * a + e] * p.scale;
-            w1[e] = (bf16)(g1 * c + g2 * sn);
-            w2[e] = (bf16)(g2 * c - g1 * sn);
-          }
-          *reinterpret_cast<bf16x4*>(dkp + 32 * dt + 8 * a + 4 * g) = w1;
-          *reinterpret_cast<bf16x4*>(dkp + 32 * (dt + 2) + 8 * a + 4 * g) = w2;
-        }
-    } else {
-#pragma unroll
-      for (int dt = 0; dt < DT; dt++)
-#pragma unroll
-        for (int a = 0; a < 4; a++) {
-          bf16x4 wk;
-#pragma unroll
-          for (int e = 0; e < 4; e++) wk[e] = (bf16)(dk[dt][4 * a + e] * p.scale);
-          *reinterpret_cast<bf16x4*>(dkp + 32 * dt + 8 * a + 4 * g) = wk;
-        }
-    }
+    store_dk_row(p, dk, b, hk, key, g);
   }
 }
 
@@ -913,12 +829,25 @@ int ody_launch_attn_bwd_pipe(const AttnParams& p, void* workspace, hipStream_t s
   int rc;
   // everything that depends on q, dout, out and lse only: delta, Q / dO images, start values
   if (!p.reuse_query_side && (rc = ody_launch_attn_bwd_prepass(p, qimg, doimg, stats, st))) return rc;
-  if ((rc = ody_launch_attn_images(p.k, p.sk, p.B, p.Lk, p.Hkv, kimg, nullptr, 0, st))) return rc;
-  const int key_blocks = (p.Lk + KV_BN - 1) / KV_BN;
   float* part = reinterpret_cast<float*>(
       reinterpret_cast<unsigned char*>(stats) +
       align256((size_t)p.B * p.Hq * ((p.Lq + KV_BQ - 1) / KV_BQ) * KV_STAT_ELEMS * sizeof(bf16)));
+  auto group_sum = [&](int qparts) {
+    const int64_t n8 = (int64_t)p.B * p.Hkv * p.Lk * (D / 8);
+    ODY_LAUNCH("attn_bwd_group_sum", st, attn_bwd_group_sum_kernel, dim3((unsigned)((n8 + 255) / 256)), dim3(256), 0, p,
+               part, qparts);
+    return ody_check_launch("attn_bwd_group_sum");
+  };
   const int qparts = query_parts(p.B, p.Lq, p.Lk, p.Hq, p.Hkv, p.causal != 0);
+  // dK and dV are the same bits whether dS is kept or not; where that is a choice, a cut query range keeps a call on the kernels below
+  const bool same_sums = qparts == 1 || ody_attn_bwd_pipe_ds_bytes(p.B, p.Lq, p.Lk, p.Hq, p.causal) == 0;
+  if (!p.ds && same_sums && ody_attn_bwd_short_ok(p.B, p.Lq, p.Lk, p.Hq, p.causal)) {
+    // the pre-pass wrote the query side whole: a later call that reuses it may run on the kernels below
+    if ((rc = ody_launch_attn_bwd_short(p, stats, part, st)) || p.group == 1) return rc;
+    return group_sum(1);
+  }
+  if ((rc = ody_launch_attn_images(p.k, p.sk, p.B, p.Lk, p.Hkv, kimg, nullptr, 0, st))) return rc;
+  const int key_blocks = (p.Lk + KV_BN - 1) / KV_BN;
   if (p.group == 1 && qparts == 1) {
     if (p.ds)
       ODY_LAUNCH("attn_bwd_dkdv_pipe", st, (attn_bwd_dkdv_pipe_kernel<false, true>), dim3(key_blocks * p.Hkv * p.B),
@@ -935,10 +864,7 @@ int ody_launch_attn_bwd_pipe(const AttnParams& p, void* workspace, hipStream_t s
       ODY_LAUNCH("attn_bwd_dkdv_pipe", st, (attn_bwd_dkdv_pipe_kernel<true, false>), dim3(key_blocks * p.Hq * qparts * p.B),
                  dim3(KV_THREADS), smem_kv, p, qimg, doimg, stats, part, qparts);
     if ((rc = ody_check_launch("attn_bwd_dkdv_pipe"))) return rc;
-    const int64_t n8 = (int64_t)p.B * p.Hkv * p.Lk * (D / 8);
-    ODY_LAUNCH("attn_bwd_group_sum", st, attn_bwd_group_sum_kernel, dim3((unsigned)((n8 + 255) / 256)), dim3(256), 0, p,
-               part, qparts);
-    if ((rc = ody_check_launch("attn_bwd_group_sum"))) return rc;
+    if ((rc = group_sum(qparts))) return rc;
   }
   dim3 gq(((p.Lq + DQ_BM - 1) / DQ_BM) * p.Hq * p.B);
   if (p.ds) {

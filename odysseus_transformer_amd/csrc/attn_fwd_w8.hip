@@ -285,6 +285,8 @@ int key_splits(int B, int Lq, int Lk, int Hq, bool causal) {
 
 }  // namespace
 
+int ody_attn_fwd_w8_parts(int B, int Lq, int Lk, int Hq, int causal) { return key_splits(B, Lq, Lk, Hq, causal != 0); }
+
 // workspace: [flags of the 256-query blocks | transposed images of V | fp32 parts of a key-split call: out, lse]
 size_t ody_attn_fwd_w8_workspace(int B, int Lq, int Lk, int Hq, int Hkv, bool with_split) {
   const size_t flags = align256((size_t)B * Hq * ((Lq + FW_BM - 1) / FW_BM) * sizeof(int));

@@ -14,10 +14,7 @@
 // takes every other tile; the sets add up through LDS at the end.  It is for calls with too few blocks to give every SIMD three
 // wavefronts.
 //
-// Tile layout in LDS: 64 rows of 128 bytes; 16-byte chunk c of row r sits at position c ^ swz(r), swz(r) = bits 3, 2, 1 of r in
-// bits 0, 1, 2.  Conflict-free for both kinds of read: the 16 rows that a 16-byte read serves together (attn_tile.h) have pairwise
-// different (r & 1, swz), and of the four rows of a transposing read those two that share a 128-byte half differ in bit 2 of swz.
-// The permutation is applied to the source chunk of each lane, as a direct load writes its lanes to consecutive addresses.
+// Tiles and fragments: attn_rowtile.h.
 //
 // Measured against the kernels these replace (register-staged tiles through padded LDS rows, rescaling on every tile, one block per
 // kv head), us: 16 heads, L = 8192, causal: forward 207 -> 158 (870 TFLOP/s), dK/dV 415 -> 285, dQ 323 -> 213; 2 x 8 heads, L = 500,
@@ -31,56 +28,16 @@
 // where the largest P of a row lie if the reference is its maximum (an emulation in 64 bits that rounds P and out gives these figures).
 #include <type_traits>
 #include <utility>
-#include "attn_params.h"
-#include "attn_tile.h"
+#include "attn_rowtile.h"
 
 namespace {
 
-constexpr int D = 64, KS = D / 16, DT = D / 32, ROWS = 64, TILE = ROWS * D;   // elements of a tile: 8 KB
+using namespace rowtile;
+
+constexpr int D = 64, KS = D / 16, DT = D / 32, TILE = ROWS * D;   // elements of a tile: 8 KB
 constexpr int BLOCK_ROWS = 128;
-typedef __attribute__((address_space(3))) void* lds_ptr;
-typedef __attribute__((address_space(1))) const void* global_ptr;
+typedef TileLoader<D, 4> Loader;
 
-__device__ __forceinline__ int swz(int r) { return ((r & 2) << 1) | ((r & 4) >> 1) | ((r & 8) >> 3); }
-
-// Fragment reads go by LDS byte addresses: what depends on the lane and the stage sits in 8 registers that move from stage to
-// stage, the rest is in the offset field of the instruction.
-struct Readers {
-  unsigned row[KS], tr[4];
-  __device__ __forceinline__ void init(const bf16* stage, int g, int i) {
-    const unsigned a = (unsigned)(uintptr_t)(lds_ptr)const_cast<bf16*>(stage);
-    const int rb = i * D + 8 * (g ^ swz(i));
-#pragma unroll
-    for (int ks = 0; ks < KS; ks++) row[ks] = a + 2 * (rb ^ (16 * ks));
-    const int t = (i & 15) >> 2;
-    const int tb = (4 * g + t) * D + 8 * ((2 * (i >> 4) + ((i & 3) >> 1)) ^ (4 * (t >> 1) + 2 * g)) + 4 * (i & 1);
-    tr[0] = a + 2 * tb, tr[1] = a + 2 * (tb ^ 8), tr[2] = a + 2 * (tb ^ 32), tr[3] = a + 2 * (tb ^ 40);
-  }
-  __device__ __forceinline__ void move(int bytes) {
-#pragma unroll
-    for (int n = 0; n < 4; n++) row[n] += bytes, tr[n] += bytes;
-  }
-};
-// A operand, rows first .. first + 31 behind the stage's start: lane (g, i) holds row i, k = 16 ks + 8 g .. + 7
-__device__ __forceinline__ bf16x8 row_frag(const Readers& r, int first, int ks) {
-  typedef const bf16x8 __attribute__((address_space(3))) * frag_ptr;
-  return *(frag_ptr)(uintptr_t)(r.row[ks] + 2 * first * D);
-}
-// A operands of the transposed tile, 16 rows from FIRST on: lane (g, i) of f[dt] holds column 32 dt + i, and k element e is row
-// FIRST + 8 (e >> 2) + 4 g + (e & 3) -- the order in which accumulators hold their rows, so that P and dS go from accumulator to
-// B operand in place.  The reads and the wait for them are one piece of assembly: behind the intrinsic the compiler waits for
-// every direct load in flight, as for possible writers of what is read here.
-template <int FIRST>
-__device__ __forceinline__ void tr_frags(bf16x8 (&f)[DT], const Readers& r) {
-  s16x4 x0, x1, y0, y1;
-  asm volatile("ds_read_b64_tr_b16 %0, %4 offset:%8\n\tds_read_b64_tr_b16 %1, %5 offset:%9\n\t"
-               "ds_read_b64_tr_b16 %2, %6 offset:%8\n\tds_read_b64_tr_b16 %3, %7 offset:%9\n\ts_waitcnt lgkmcnt(0)"
-               : "=&v"(x0), "=&v"(x1), "=&v"(y0), "=&v"(y1)
-               : "v"(r.tr[0]), "v"(r.tr[1]), "v"(r.tr[2]), "v"(r.tr[3]), "n"(2 * FIRST * D), "n"(2 * (FIRST + 8) * D)
-               : "memory");
-  f[0] = concat4(__builtin_bit_cast(bf16x4, x0), __builtin_bit_cast(bf16x4, x1));
-  f[1] = concat4(__builtin_bit_cast(bf16x4, y0), __builtin_bit_cast(bf16x4, y1));
-}
 // Blocks heaviest first, all (head, batch) pairs of a rank together (ody_block_coord), and under a causal mask every other run
 // of 256 blocks with its ranks reversed: the three or four blocks that share a compute unit then add up to about the same
 // length.  In plain order the units with the first blocks of every run got 320 tiles where the mean was 260 (forward of 16 heads,
@@ -91,76 +48,6 @@ __device__ __forceinline__ BlockCoord block_coord(int H, int B, int causal) {
   if (causal && (n & 1) && (n + 1) * run <= ranks) c.rank = n * run + run - 1 - c.rank % run;
   return c;
 }
-// row of accumulator register r
-__device__ __forceinline__ int acc_row(int r, int g) { return 8 * (r >> 2) + 4 * g + (r & 3); }
-
-// Direct loads of 64-row tiles of one matrix: 8 instructions of 8 rows, two per wavefront of a group.  Rows at or beyond nrows
-// re-read the last one (finite filler that the caller masks); tiles start below nrows.
-struct TileLoader {
-  int64_t off, stride;   // of this lane's chunk in the first instruction; row stride
-  int row;
-  __device__ __forceinline__ void init(int64_t s, int w4, int lane) {
-    row = 8 * w4 + (lane >> 3);
-    off = (int64_t)row * s + 8 * ((lane & 7) ^ swz(row));
-    stride = s;
-  }
-  // base: the matrix of this (batch, head), uniform
-  __device__ __forceinline__ void load(bf16* tile, const bf16* base, int row0, int nrows, int w4) const {
-#pragma unroll
-    for (int j = 0; j < 2; j++) {
-      const bf16* src = base + (int64_t)(row0 + 32 * j) * stride + off;
-      if (row0 + ROWS > nrows) src += (int64_t)min(nrows - 1 - row0 - 32 * j - row, 0) * stride;
-      __builtin_amdgcn_global_load_lds((global_ptr)src, (lds_ptr)(tile + (4 * j + w4) * 512), 16, 0, 0);
-    }
-  }
-};
-
-// The 32 rows of a wavefront as B operands: lane (g, i) holds row `row`, k = 16 ks + 8 g .. + 7; zero beyond nrows
-__device__ __forceinline__ void load_rows(bf16x8 (&f)[KS], const bf16* base, int64_t stride, int row, int nrows, int g) {
-#pragma unroll
-  for (int ks = 0; ks < KS; ks++) {
-    f[ks] = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
-    if (row < nrows) f[ks] = *reinterpret_cast<const bf16x8*>(base + (int64_t)row * stride + 16 * ks + 8 * g);
-  }
-  // arrived before the loop: left pending, the wait for them would land on a use inside it, as a wait for the tile loads too
-#pragma unroll
-  for (int ks = 0; ks < KS; ks++) asm volatile("" : "+v"(f[ks]));
-}
-
-__device__ __forceinline__ void clear(f32x16 (&x)[DT]) {
-#pragma unroll
-  for (int dt = 0; dt < DT; dt++)
-#pragma unroll
-    for (int r = 0; r < 16; r++) x[dt][r] = 0.f;
-}
-
-// accumulators of the second group to LDS, and back into the first (dst [register][lane] of this wavefront)
-__device__ __forceinline__ void give(float* patch, const f32x16 (&x)[DT], int lane) {
-#pragma unroll
-  for (int dt = 0; dt < DT; dt++)
-#pragma unroll
-    for (int r = 0; r < 16; r++) patch[(16 * dt + r) * 64 + lane] = x[dt][r];
-}
-__device__ __forceinline__ void take(const float* patch, f32x16 (&x)[DT], int lane, float mine, float theirs) {
-#pragma unroll
-  for (int dt = 0; dt < DT; dt++)
-#pragma unroll
-    for (int r = 0; r < 16; r++) x[dt][r] = x[dt][r] * mine + patch[(16 * dt + r) * 64 + lane] * theirs;
-}
-
-// D accumulator columns of one row -> bf16 row
-__device__ __forceinline__ void store_row(bf16* dst, const f32x16 (&x)[DT], float scale, int g) {
-#pragma unroll
-  for (int dt = 0; dt < DT; dt++)
-#pragma unroll
-    for (int a = 0; a < 4; a++) {
-      bf16x4 w;
-#pragma unroll
-      for (int e = 0; e < 4; e++) w[e] = (bf16)(x[dt][4 * a + e] * scale);
-      *reinterpret_cast<bf16x4*>(dst + 32 * dt + 8 * a + 4 * g) = w;
-    }
-}
-
 constexpr size_t KV_STAGE = 2 * TILE;                    // elements: two tiles
 constexpr size_t QS_STAGE = 2 * TILE + 2 * 2 * ROWS;     // Q and dO tiles, -lse / scale and -delta of their rows in fp32
 static_assert(2 * 2 * KV_STAGE * sizeof(bf16) >= 4 * 34 * 64 * sizeof(float) && 2 * 2 * QS_STAGE * sizeof(bf16) >= 4 * 64 * 64 * sizeof(float),
@@ -183,7 +70,7 @@ __global__ __launch_bounds__(256 * GROUPS, 4) void attn_fwd_hd64_kernel(const At
 
   int n_end = p.causal ? min(p.Lk, min(q0 + BLOCK_ROWS, p.Lq) + p.off) : p.Lk;
   const int ntiles = n_end > 0 ? (n_end + ROWS - 1) / ROWS : 0;
-  TileLoader lk, lv;
+  Loader lk, lv;
   lk.init(p.sk.l, w4, lane);
   lv.init(p.sv.l, w4, lane);
   const bf16* kp = static_cast<const bf16*>(p.k) + b * p.sk.b + hk * p.sk.h;
@@ -210,7 +97,7 @@ __global__ __launch_bounds__(256 * GROUPS, 4) void attn_fwd_hd64_kernel(const At
     ref = -1e30f;   // below any score until a key was seen
 #pragma unroll
     for (int e = 0; e < 4; e++) l4[e] = 0.f;
-    Readers rd;
+    Readers<D> rd;
     rd.init(ring, g, i);
     auto tile = [&](int t, bool first) {
       const int n0 = t * ROWS;
@@ -252,10 +139,10 @@ __global__ __launch_bounds__(256 * GROUPS, 4) void attn_fwd_hd64_kernel(const At
           l4[r & 3] += x;
           pb[r >> 3][r & 7] = (bf16)x;
         }
-        tr_frags<ROWS + 32 * kt>(vf, rd);
+        tr_frags<ROWS + 32 * kt, 0>(vf, rd);
 #pragma unroll
         for (int dt = 0; dt < DT; dt++) o[dt] = mfma32(vf[dt], pb[0], o[dt]);
-        tr_frags<ROWS + 32 * kt + 16>(vf, rd);
+        tr_frags<ROWS + 32 * kt + 16, 0>(vf, rd);
 #pragma unroll
         for (int dt = 0; dt < DT; dt++) o[dt] = mfma32(vf[dt], pb[1], o[dt]);
       };
@@ -361,7 +248,7 @@ __global__ __launch_bounds__(256 * GROUPS, GROUPS == 1 ? 3 : 2) void attn_bwd_hd
   const int ntq = max(0, t_end - t_begin), total = ntq * heads;
   // Tile `it` of the flattened (query head, query tile) range, last query tile first: the key blocks that run at one time on an
   // XCD then read the same Q and dO tiles.
-  TileLoader lq, lo;
+  Loader lq, lo;
   lq.init(p.sq.l, w4, lane);
   lo.init(p.sdo.l, w4, lane);
   float l_next = INFINITY;   // first wavefront of a group: lse of row `lane` of the tile on its way
@@ -393,7 +280,7 @@ __global__ __launch_bounds__(256 * GROUPS, GROUPS == 1 ? 3 : 2) void attn_bwd_hd
   load_rows(kf, static_cast<const bf16*>(p.k) + b * p.sk.b + hk * p.sk.h, p.sk.l, key, p.Lk, g);
   load_rows(vf, static_cast<const bf16*>(p.v) + b * p.sv.b + hk * p.sv.h, p.sv.l, key, p.Lk, g);
   const float c2 = p.scale_log2e;
-  Readers rd;
+  Readers<D> rd;
   rd.init(ring, g, i);
   f32x16 dk[DT], dv[DT];
   clear(dk);
@@ -441,8 +328,8 @@ __global__ __launch_bounds__(256 * GROUPS, GROUPS == 1 ? 3 : 2) void attn_bwd_hd
       auto products = [&](auto half) {
         constexpr int ss = decltype(half)::value;
         bf16x8 of[DT], qf[DT];
-        tr_frags<ROWS + 32 * mt + 16 * ss>(of, rd);
-        tr_frags<32 * mt + 16 * ss>(qf, rd);
+        tr_frags<ROWS + 32 * mt + 16 * ss, 0>(of, rd);
+        tr_frags<32 * mt + 16 * ss, 0>(qf, rd);
 #pragma unroll
         for (int dt = 0; dt < DT; dt++) {
           dv[dt] = mfma32(of[dt], pf[ss], dv[dt]);
@@ -530,7 +417,7 @@ __global__ __launch_bounds__(256 * GROUPS, GROUPS == 1 ? 3 : 2) void attn_bwd_hd
 
   int n_end = p.causal ? min(p.Lk, min(q0 + BLOCK_ROWS, p.Lq) + p.off) : p.Lk;
   const int ntiles = n_end > 0 ? (n_end + ROWS - 1) / ROWS : 0;
-  TileLoader lk, lv;
+  Loader lk, lv;
   lk.init(p.sk.l, w4, lane);
   lv.init(p.sv.l, w4, lane);
   const bf16* kp = static_cast<const bf16*>(p.k) + b * p.sk.b + hk * p.sk.h;
@@ -554,7 +441,7 @@ __global__ __launch_bounds__(256 * GROUPS, GROUPS == 1 ? 3 : 2) void attn_bwd_hd
   for (int r = 0; r < 16; r++) start[r] = nd;
   const int lim = p.causal ? min(p.Lk - 1, qi + p.off) : p.Lk - 1;
   const float c2 = p.scale_log2e;
-  Readers rd;
+  Readers<D> rd;
   rd.init(ring, g, i);
   f32x16 dq[DT];
   clear(dq);
@@ -585,10 +472,10 @@ __global__ __launch_bounds__(256 * GROUPS, GROUPS == 1 ? 3 : 2) void attn_bwd_hd
 #pragma unroll
       for (int r = 0; r < 16; r++) dsf[r >> 3][r & 7] = (bf16)(ody_exp2(fmaf(s[r], c2, -lse2)) * dp[r]);
       bf16x8 kf[DT];
-      tr_frags<32 * kt>(kf, rd);
+      tr_frags<32 * kt, 0>(kf, rd);
 #pragma unroll
       for (int dt = 0; dt < DT; dt++) dq[dt] = mfma32(kf[dt], dsf[0], dq[dt]);
-      tr_frags<32 * kt + 16>(kf, rd);
+      tr_frags<32 * kt + 16, 0>(kf, rd);
 #pragma unroll
       for (int dt = 0; dt < DT; dt++) dq[dt] = mfma32(kf[dt], dsf[1], dq[dt]);
     };

@@ -87,6 +87,7 @@ int ody_launch_attn_bwd_prepass(const AttnParams& p, void* qimg, void* doimg, vo
 // blocks against many keys); a workspace without that room makes such a call run unsplit.
 int ody_launch_attn_fwd_w8(const AttnParams& p, void* workspace, size_t workspace_bytes, hipStream_t st);
 size_t ody_attn_fwd_w8_workspace(int B, int Lq, int Lk, int Hq, int Hkv, bool with_split);
+int ody_attn_fwd_w8_parts(int B, int Lq, int Lk, int Hq, int causal);   // of every block's key range, where the workspace has the room
 // forward for at most 64 rows per kv head (rows = queries x query heads of its group), key ranges cut over blocks; a workspace
 // without room for the parts makes the call run on one block per kv head
 bool ody_attn_decode_ok(int Lq, int Hq, int Hkv, int D);
@@ -104,6 +105,12 @@ int ody_launch_attn_bwd_pipe(const AttnParams& p, void* workspace, hipStream_t s
 int ody_launch_attn_fwd_hd64(const AttnParams& p, hipStream_t st);
 size_t ody_attn_bwd_hd64_workspace(int B, int Lq, int Lk, int Hq, int Hkv);
 int ody_launch_attn_bwd_hd64(const AttnParams& p, void* workspace, size_t workspace_bytes, hipStream_t st);
+// head_dim 128 where those two leave compute units idle; neither workspace nor images.  The backward runs behind the pre-pass, from
+// p.delta and its start values, and leaves fp32 dK / dV of every query head in `part` if Hq != Hkv.
+bool ody_attn_fwd_short_ok(int B, int Lq, int Lk, int Hq, int causal);
+bool ody_attn_bwd_short_ok(int B, int Lq, int Lk, int Hq, int causal);
+int ody_launch_attn_fwd_short(const AttnParams& p, hipStream_t st);
+int ody_launch_attn_bwd_short(const AttnParams& p, const void* stats, float* part, hipStream_t st);
 // with dropout, both head dims
 int ody_launch_attn_bwd_mfma(const AttnParams& p, int D, hipStream_t st);
 // fp32 on the fp32 matrix cores

@@ -1,0 +1,458 @@
+// Flash attention for bf16 and head_dim 128 where the kernels for long sequences (attn_fwd_w8.hip, attn_bwd_pipe.hip) leave compute units
+// idle or wait for latency: few blocks of 256 rows, each a few tiles long, behind passes that write transposed images.
+//
+// A block is 128 rows: 4 wavefronts of 32 rows, twice.  In the forward and for dQ the second four take every other key tile, so that the
+// serial chain of tiles is half as long; the halves add up through LDS at the end.  For dK and dV the two sets share the tiles and the
+// work: one holds dV, the other dK (S is formed twice, which costs less than the registers of both: a chain of three products instead of
+// four).  Tiles come straight to LDS, two stages, and serve as row operands and, through the transposing read, as transposed ones
+// (attn_rowtile.h), at half the LDS rate but without an image, its pass and its launch.  All of the backward behind the pre-pass is one launch.
+//
+// What bounds it: latency of a chain of tiles in a block (about 2.5 us for 128 rows against 128 keys in the forward) on 1 block a unit.
+// Before / here, us, launches included: forward of 4 x 8 heads, L = 331, causal 19.8 / 12.7 (three launches / one), backward on 2 kv heads
+// 62.2 / 33.6 (five / three); 32 heads on 8, L = 1000, causal 41.5 / 24.4 and 119 / 74; 8 heads, L = 1500, full 43 / 31 and 148 / 68.
+// Error against 64 bits, standard normal inputs, before / here: out 2.07e-3 / 1.96e-3 (4 x 8 heads, L = 331), 2.34e-3 / 2.31e-3 (640 rows,
+// full); dQ, dK, dV the same within the spread of one input to the next (2.5e-3, 2.5e-3, 2.3e-3).
+#include <algorithm>
+#include <type_traits>
+#include <utility>
+#include "attn_rowtile.h"
+#include "attn_store.h"
+
+namespace {
+
+using namespace rowtile;
+
+constexpr int D = 128, KS = D / 16, DT = D / 32, TILE = ROWS * D;   // elements of a tile: 16 KB
+constexpr int BLOCK_ROWS = 128, WAVES = 8, GROUPS = 2;
+constexpr size_t KV_STAGE = 2 * TILE;                    // elements: two tiles
+constexpr size_t QS_STAGE = 2 * TILE + 512;              // Q and dO tiles, start values of S and dP (1 KB, written by the pre-pass)
+constexpr size_t SMEM = GROUPS * 2 * KV_STAGE * sizeof(bf16);
+static_assert(SMEM >= 4 * (16 * DT + 2) * 64 * sizeof(float) && SMEM >= 2 * QS_STAGE * sizeof(bf16) && SMEM <= 160 * 1024, "one block per unit");
+typedef TileLoader<D, 4> GroupLoader;
+
+// ---------------------------------------------------------------------------------------------------------- forward
+//   S^T = K Q^T      O^T += V^T P^T       lane = query column
+__global__ __launch_bounds__(64 * WAVES, 2) void attn_fwd_short_kernel(const AttnParams p) {
+  constexpr size_t STAGE_BYTES = KV_STAGE * sizeof(bf16);
+  extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, g = lane >> 5, i = lane & 31;
+  const int grp = wave >> 2, w4 = wave & 3;
+  bf16* ring = reinterpret_cast<bf16*>(smem) + grp * 2 * KV_STAGE;   // [2][K tile | V tile]
+  const BlockCoord bc = ody_block_coord(p.Hq, p.B);
+  const int nqb = gridDim.x / (p.Hq * p.B);
+  const int qblk = p.causal ? nqb - 1 - bc.rank : bc.rank;   // heaviest blocks first
+  const int h = bc.h, b = bc.b, hk = h / p.group;
+  const int q0 = qblk * BLOCK_ROWS, wq0 = q0 + w4 * 32, qi = wq0 + i;
+
+  int n_end = p.causal ? min(p.Lk, min(q0 + BLOCK_ROWS, p.Lq) + p.off) : p.Lk;
+  const int ntiles = n_end > 0 ? (n_end + ROWS - 1) / ROWS : 0;
+  GroupLoader lk, lv;
+  lk.init(p.sk.l, w4, lane);
+  lv.init(p.sv.l, w4, lane);
+  const bf16* kp = static_cast<const bf16*>(p.k) + b * p.sk.b + hk * p.sk.h;
+  const bf16* vp = static_cast<const bf16*>(p.v) + b * p.sv.b + hk * p.sv.h;
+  auto load = [&](int t, int buf) {
+    lk.load(ring + buf * KV_STAGE, kp, t * ROWS, p.Lk, w4);
+    lv.load(ring + buf * KV_STAGE + TILE, vp, t * ROWS, p.Lk, w4);
+  };
+
+  bf16x8 qf[KS];
+  load_rows(qf, static_cast<const bf16*>(p.q) + b * p.sq.b + h * p.sq.h, p.sq.l, qi, p.Lq, g);
+  const int lim = p.causal ? min(p.Lk - 1, qi + p.off) : p.Lk - 1;   // last key this lane's query sees
+  const float c2 = p.scale_log2e;
+  f32x16 o[DT];
+  float ref;     // the row's reference in log2 units
+  float l4[4];   // this lane's partial row sums
+
+  // ONLINE = false: the reference of a row is the largest score of its first tile (a row that sees any key sees key 0) and stays.
+  // ONLINE = true: it is the maximum so far, so that P <= 1 and P V overflows for no values that P = 1 would hold.
+  const int iters = (ntiles + GROUPS - 1) / GROUPS;
+  auto walk = [&](auto online) {
+    constexpr bool ONLINE = decltype(online)::value;
+    clear(o);
+    ref = -1e30f;   // below any score until a key was seen
+#pragma unroll
+    for (int e = 0; e < 4; e++) l4[e] = 0.f;
+    Readers<D> rd;
+    rd.init(ring, g, i);
+    auto tile = [&](int t, bool first) {
+      const int n0 = t * ROWS;
+      if (t >= ntiles || (p.causal && n0 > wq0 + 31 + p.off)) return;
+      f32x16 s[2];
+#pragma unroll
+      for (int ks = 0; ks < KS; ks++)
+#pragma unroll
+        for (int kt = 0; kt < 2; kt++) s[kt] = mfma32(row_frag(rd, 32 * kt, ks), qf[ks], ks == 0 ? f32x16{0} : s[kt]);
+      if (n0 + ROWS > p.Lk || (p.causal && n0 + ROWS - 1 > wq0 + p.off)) {
+#pragma unroll
+        for (int kt = 0; kt < 2; kt++)
+#pragma unroll
+          for (int r = 0; r < 16; r++)
+            if (n0 + 32 * kt + acc_row(r, g) > lim) s[kt][r] = -INFINITY;
+      }
+      if (ONLINE || first) {
+        float mx = fmaxf(s[0][0], s[1][0]);
+#pragma unroll
+        for (int r = 1; r < 16; r++) mx = fmaxf(mx, fmaxf(s[0][r], s[1][r]));
+        mx = half_swap_max(mx) * c2;
+        if (__builtin_amdgcn_ballot_w64(mx > ref) != 0) {
+          const float next = fmaxf(ref, mx), alpha = ody_exp2(ref - next);
+          ref = next;
+#pragma unroll
+          for (int e = 0; e < 4; e++) l4[e] *= alpha;
+#pragma unroll
+          for (int dt = 0; dt < DT; dt++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) o[dt][r] *= alpha;
+        }
+      }
+      auto half = [&](auto which) {
+        constexpr int kt = decltype(which)::value;
+        bf16x8 pb[2], vf[2];
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+          const float x = ody_exp2(fmaf(s[kt][r], c2, -ref));
+          l4[r & 3] += x;
+          pb[r >> 3][r & 7] = (bf16)x;
+        }
+        auto product = [&](auto slice) {   // 16 keys, 64 columns of the head
+          constexpr int ss = decltype(slice)::value & 1, hf = decltype(slice)::value >> 1;
+          tr_frags<ROWS + 32 * kt + 16 * ss, hf>(vf, rd);
+#pragma unroll
+          for (int dt = 0; dt < 2; dt++) o[2 * hf + dt] = mfma32(vf[dt], pb[ss], o[2 * hf + dt]);
+        };
+        product(std::integral_constant<int, 0>{});
+        product(std::integral_constant<int, 2>{});
+        product(std::integral_constant<int, 1>{});
+        product(std::integral_constant<int, 3>{});
+      };
+      half(std::integral_constant<int, 0>{});
+      half(std::integral_constant<int, 1>{});
+    };
+    if (grp < ntiles) load(grp, 0);
+    for (int it = 0; it < iters; it++) {
+      const int t = grp + GROUPS * it;
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __syncthreads();   // the tile has landed, and everyone is done with the one before
+      if (t + GROUPS < ntiles) load(t + GROUPS, (it + 1) & 1);
+      tile(t, it == 0);
+      rd.move((it & 1) ? -(int)STAGE_BYTES : (int)STAGE_BYTES);
+    }
+    __syncthreads();   // everyone is done with the stages
+  };
+  walk(std::false_type{});
+  {
+    // a later score that outgrew its row's reference by more than fp32 holds left a row sum beyond any real one (or a NaN), or,
+    // times large values, an infinity in O: 0 times the accumulators is 0 unless one of them is not finite
+    int* flags = reinterpret_cast<int*>(smem);
+    float zero[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int dt = 0; dt < DT; dt++)
+#pragma unroll
+      for (int r = 0; r < 16; r++) zero[r & 3] = fmaf(o[dt][r], 0.f, zero[r & 3]);
+    const bool finite = (zero[0] + zero[1]) + (zero[2] + zero[3]) == 0.f;
+    const bool beyond = __builtin_amdgcn_ballot_w64(!finite || !(half_swap_sum((l4[0] + l4[1]) + (l4[2] + l4[3])) < 0x1p100f)) != 0;
+    if (lane == 0) flags[wave] = beyond;
+    __syncthreads();
+    int any = 0;
+#pragma unroll
+    for (int w = 0; w < 4 * GROUPS; w++) any |= flags[w];
+    __syncthreads();
+    if (any) walk(std::true_type{});
+  }
+
+  float l = (l4[0] + l4[1]) + (l4[2] + l4[3]);
+#pragma unroll 1
+  for (int from = 1; from < GROUPS; from++) {
+    float* patch = reinterpret_cast<float*>(smem) + w4 * (16 * DT + 2) * 64;
+    if (grp == from) {
+      give(patch, o, lane);
+      patch[16 * DT * 64 + lane] = ref;
+      patch[(16 * DT + 1) * 64 + lane] = l;
+    }
+    __syncthreads();
+    if (grp == 0) {
+      const float ref1 = patch[16 * DT * 64 + lane], next = fmaxf(ref, ref1), a0 = ody_exp2(ref - next), a1 = ody_exp2(ref1 - next);
+      take(patch, o, lane, a0, a1);
+      l = l * a0 + patch[(16 * DT + 1) * 64 + lane] * a1;
+      ref = next;
+    }
+    __syncthreads();
+  }
+  if (grp != 0) return;
+  l = half_swap_sum(l);
+  if (qi < p.Lq) {
+    const float inv = l > 0.f ? 1.f / l : 0.f;
+    store_row(static_cast<bf16*>(p.out) + b * p.so.b + h * p.so.h + (int64_t)qi * p.so.l, o, inv, g);
+    if (g == 0) p.lse[((int64_t)b * p.Hq + h) * p.Lq + qi] = l > 0.f ? (ref + __log2f(l)) * ODY_LN2 : -INFINITY;
+  }
+}
+
+
+// ---------------------------------------------------------------------------------------------------------- backward
+// dQ of 128 queries of a head: 4 wavefronts of 32 queries, two groups that take every other key tile.
+//   S^T = K Q^T     dP^T = V dO^T - delta     dQ^T += K^T dS^T       lane = query column
+__device__ __forceinline__ void dq_block(const AttnParams& p, unsigned char* smem, int q0, int h, int b) {
+  constexpr size_t STAGE_BYTES = KV_STAGE * sizeof(bf16);
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, g = lane >> 5, i = lane & 31;
+  const int grp = wave >> 2, w4 = wave & 3, hk = h / p.group, wq0 = q0 + w4 * 32, qi = wq0 + i;
+  bf16* ring = reinterpret_cast<bf16*>(smem) + grp * 2 * KV_STAGE;   // [2][K tile | V tile]
+
+  int n_end = p.causal ? min(p.Lk, min(q0 + BLOCK_ROWS, p.Lq) + p.off) : p.Lk;
+  const int ntiles = n_end > 0 ? (n_end + ROWS - 1) / ROWS : 0;
+  GroupLoader lk, lv;
+  lk.init(p.sk.l, w4, lane);
+  lv.init(p.sv.l, w4, lane);
+  const bf16* kp = static_cast<const bf16*>(p.k) + b * p.sk.b + hk * p.sk.h;
+  const bf16* vp = static_cast<const bf16*>(p.v) + b * p.sv.b + hk * p.sv.h;
+  auto load = [&](int t, int buf) {
+    lk.load(ring + buf * KV_STAGE, kp, t * ROWS, p.Lk, w4);
+    lv.load(ring + buf * KV_STAGE + TILE, vp, t * ROWS, p.Lk, w4);
+  };
+  if (grp < ntiles) load(grp, 0);
+
+  bf16x8 qf[KS], dof[KS];
+  load_rows(qf, static_cast<const bf16*>(p.q) + b * p.sq.b + h * p.sq.h, p.sq.l, qi, p.Lq, g);
+  load_rows(dof, static_cast<const bf16*>(p.dout) + b * p.sdo.b + h * p.sdo.h, p.sdo.l, qi, p.Lq, g);
+  const int64_t head = (int64_t)b * p.Hq + h;
+  float lse2 = qi < p.Lq ? p.lse[head * p.Lq + qi] : INFINITY;
+  if (lse2 == -INFINITY) lse2 = INFINITY;   // a query that saw no key: P = 0
+  lse2 *= ODY_LOG2E;
+  const float nd = qi < p.Lq ? -p.delta[head * p.Lq + qi] : 0.f;
+  f32x16 start;   // dP starts from -delta: one add less per element
+#pragma unroll
+  for (int r = 0; r < 16; r++) start[r] = nd;
+  const int lim = p.causal ? min(p.Lk - 1, qi + p.off) : p.Lk - 1;
+  const float c2 = p.scale_log2e;
+  Readers<D> rd;
+  rd.init(ring, g, i);
+  f32x16 dq[DT];
+  clear(dq);
+
+  const int iters = (ntiles + GROUPS - 1) / GROUPS;
+  for (int it = 0; it < iters; it++) {
+    const int t = grp + GROUPS * it;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (t + GROUPS < ntiles) load(t + GROUPS, (it + 1) & 1);
+    auto sub_tile = [&](auto which) {
+      __builtin_amdgcn_sched_barrier(0);   // one sub-tile's fragments at a time
+      constexpr int kt = decltype(which)::value;
+      const int k0 = t * ROWS + 32 * kt;
+      if (t >= ntiles || k0 >= p.Lk || (p.causal && k0 > wq0 + 31 + p.off)) return;
+      f32x16 s, dp;
+#pragma unroll
+      for (int ks = 0; ks < KS; ks++) {
+        s = mfma32(row_frag(rd, 32 * kt, ks), qf[ks], ks == 0 ? f32x16{0} : s);
+        dp = mfma32(row_frag(rd, ROWS + 32 * kt, ks), dof[ks], ks == 0 ? start : dp);
+      }
+      if (k0 + 32 > p.Lk || (p.causal && k0 + 31 > wq0 + p.off)) {
+#pragma unroll
+        for (int r = 0; r < 16; r++)
+          if (k0 + acc_row(r, g) > lim) s[r] = -INFINITY;
+      }
+      bf16x8 dsf[2];
+#pragma unroll
+      for (int r = 0; r < 16; r++) dsf[r >> 3][r & 7] = (bf16)(ody_exp2(fmaf(s[r], c2, -lse2)) * dp[r]);
+      bf16x8 kf[2];
+      auto product = [&](auto slice) {
+        constexpr int ss = decltype(slice)::value & 1, hf = decltype(slice)::value >> 1;
+        tr_frags<32 * kt + 16 * ss, hf>(kf, rd);
+#pragma unroll
+        for (int dt = 0; dt < 2; dt++) dq[2 * hf + dt] = mfma32(kf[dt], dsf[ss], dq[2 * hf + dt]);
+      };
+      product(std::integral_constant<int, 0>{});
+      product(std::integral_constant<int, 2>{});
+      product(std::integral_constant<int, 1>{});
+      product(std::integral_constant<int, 3>{});
+    };
+    sub_tile(std::integral_constant<int, 0>{});
+    sub_tile(std::integral_constant<int, 1>{});
+    rd.move((it & 1) ? -(int)STAGE_BYTES : (int)STAGE_BYTES);
+  }
+
+  float* patch = reinterpret_cast<float*>(smem) + w4 * 16 * DT * 64;
+  __syncthreads();
+  if (grp == 1) give(patch, dq, lane);
+  __syncthreads();
+  if (grp == 1) return;
+  take(patch, dq, lane, 1.f, 1.f);
+  store_dq_row(p, dq, b, h, qi, g);
+}
+
+// One of dK and dV of 32 keys per wavefront, over the query tiles of one query head: wavefronts 0 - 3 of a block hold dV of its 128
+// keys, 4 - 7 dK.
+//   S = Q K^T - lse / scale     dV^T += dO^T P                                              lane = key column
+//                               dP = dO V^T - delta     dK^T += Q^T (P o dP)
+// Start values, order of the rows and of the sums are those of attn_bwd_dkdv_pipe_kernel, and so are the results, bit for bit, as long as
+// that one does not cut its query range: dK and dV do not depend on whether a caller keeps dS.
+//
+// The two roles are two instances: in one loop with a branch on the role the compiler gives both the registers of both, and spills.
+// Each passes the same barriers, one per query tile.
+template <bool PART, bool IS_DK>
+__device__ __forceinline__ void kv_block(const AttnParams& p, unsigned char* smem, int n0, int h, int b, const bf16* __restrict__ stats,
+                                         float* __restrict__ part) {
+  constexpr size_t STAGE_BYTES = QS_STAGE * sizeof(bf16);
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, g = lane >> 5, i = lane & 31;
+  const int hk = h / p.group, wn0 = n0 + (wave & 3) * 32, key = wn0 + i;
+  bf16* ring = reinterpret_cast<bf16*>(smem);   // [2][Q tile | dO tile | row values]
+  const int t_begin = p.causal ? max(0, n0 - p.off) / ROWS : 0, t_end = (p.Lq + ROWS - 1) / ROWS;
+  const int total = max(0, t_end - t_begin);
+  TileLoader<D, WAVES, true> lq, lo;
+  lq.init(p.sq.l, wave, lane);
+  lo.init(p.sdo.l, wave, lane);
+  const bf16* qp = static_cast<const bf16*>(p.q) + b * p.sq.b + h * p.sq.h;
+  const bf16* dop = static_cast<const bf16*>(p.dout) + b * p.sdo.b + h * p.sdo.h;
+  const bf16* sp = stats + ((int64_t)b * p.Hq + h) * t_end * 512 + lane * 8;
+  auto load = [&](int t, int buf) {
+    bf16* st = ring + buf * QS_STAGE;
+    lq.load(st, qp, t * ROWS, p.Lq, wave);
+    lo.load(st + TILE, dop, t * ROWS, p.Lq, wave);
+    if (!IS_DK && wave == 0)
+      __builtin_amdgcn_global_load_lds((global_ptr)(sp + (int64_t)t * 512), (lds_ptr)(st + 2 * TILE), 16, 0, 0);
+  };
+  if (total > 0) load(t_end - 1, 0);
+
+  bf16x8 kf[KS], vf[IS_DK ? KS : 1];
+  load_rows(kf, static_cast<const bf16*>(p.k) + b * p.sk.b + hk * p.sk.h, p.sk.l, key, p.Lk, g);
+  if constexpr (IS_DK) load_rows(vf, static_cast<const bf16*>(p.v) + b * p.sv.b + hk * p.sv.h, p.sv.l, key, p.Lk, g);
+  const float c2 = p.scale_log2e;
+  Readers<D, true> rd;
+  rd.init(ring, g, i);
+  f32x16 acc[DT];   // dK^T or dV^T
+  clear(acc);
+
+  for (int n = 0; n < total; n++) {
+    const int i0 = (t_end - 1 - n) * ROWS;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (n + 1 < total) load(t_end - 2 - n, (n + 1) & 1);
+    // every query of the tile comes before every key of this wavefront: nothing to do
+    const bool dead = p.causal && i0 + ROWS - 1 + p.off < wn0;
+    const float* rv = reinterpret_cast<const float*>(ring + (n & 1) * QS_STAGE + 2 * TILE) + 16 * g;
+    auto sub_tile = [&](auto which) {
+      __builtin_amdgcn_sched_barrier(0);   // one sub-tile's fragments at a time
+      constexpr int mt = decltype(which)::value;
+      f32x16 s, dp;
+#pragma unroll
+      for (int a = 0; a < 4; a++) {
+        const f32x4 x = *reinterpret_cast<const f32x4*>(rv + 64 * mt + 4 * a);
+#pragma unroll
+        for (int e = 0; e < 4; e++) s[4 * a + e] = x[e];
+        if constexpr (IS_DK) {
+          const f32x4 y = *reinterpret_cast<const f32x4*>(rv + 64 * mt + 32 + 4 * a);
+#pragma unroll
+          for (int e = 0; e < 4; e++) dp[4 * a + e] = y[e];
+        }
+      }
+#pragma unroll
+      for (int ks = 0; ks < KS; ks++) {
+        s = mfma32(row_frag(rd, 2 * mt, ks), kf[ks], s);
+        if constexpr (IS_DK) dp = mfma32(row_frag(rd, ROWS + 2 * mt, ks), vf[ks], dp);
+      }
+      if (p.causal && i0 + p.off < wn0 + 31) {
+#pragma unroll
+        for (int r = 0; r < 16; r++)
+          if (i0 + tile128::acc_tile_row(r, g, mt) + p.off < key) s[r] = -INFINITY;
+      }
+      bf16x8 pf[2];   // P, or dS
+#pragma unroll
+      for (int r = 0; r < 16; r++) {
+        const float pr = ody_exp2(s[r] * c2);
+        pf[r >> 3][r & 7] = (bf16)(IS_DK ? pr * dp[r] : pr);
+      }
+      bf16x8 f[2];
+      auto product = [&](auto slice) {
+        constexpr int ss = decltype(slice)::value & 1, hf = decltype(slice)::value >> 1;
+        tr_frags<(IS_DK ? 0 : ROWS) + 2 * mt + ss, hf>(f, rd);
+#pragma unroll
+        for (int dt = 0; dt < 2; dt++) acc[2 * hf + dt] = mfma32(f[dt], pf[ss], acc[2 * hf + dt]);
+      };
+      product(std::integral_constant<int, 0>{});
+      product(std::integral_constant<int, 2>{});
+      product(std::integral_constant<int, 1>{});
+      product(std::integral_constant<int, 3>{});
+    };
+    if (!dead) {
+      sub_tile(std::integral_constant<int, 0>{});
+      sub_tile(std::integral_constant<int, 1>{});
+    }
+    rd.move((n & 1) ? -(int)STAGE_BYTES : (int)STAGE_BYTES);
+  }
+
+  if (key >= p.Lk) return;
+  if constexpr (PART) {   // [dK | dV][B][Hq][Lk][D] in fp32
+    float* dst = part + (IS_DK ? 0 : (int64_t)p.B * p.Hq * p.Lk * D) + (((int64_t)b * p.Hq + h) * p.Lk + key) * D;
+#pragma unroll
+    for (int dt = 0; dt < DT; dt++)
+#pragma unroll
+      for (int a = 0; a < 4; a++) {
+        f32x4 w;
+#pragma unroll
+        for (int e = 0; e < 4; e++) w[e] = acc[dt][4 * a + e];
+        *reinterpret_cast<f32x4*>(dst + 32 * dt + 8 * a + 4 * g) = w;
+      }
+  } else if constexpr (IS_DK) {
+    store_dk_row(p, acc, b, hk, key, g);
+  } else {
+    store_row(static_cast<bf16*>(p.dv) + b * p.sdv.b + hk * p.sdv.h + (int64_t)key * p.sdv.l, acc, 1.f, g);
+  }
+}
+
+// The whole backward behind the pre-pass in one launch.  A rank of key blocks (first keys first: the most query tiles) and a rank of
+// query blocks (last queries first) alternate, over all heads, so that what starts last is short on both sides.
+template <bool PART>
+__global__ __launch_bounds__(64 * WAVES, 2) void attn_bwd_short_kernel(const AttnParams p, const bf16* __restrict__ stats,
+                                                                   float* __restrict__ part) {
+  extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
+  const BlockCoord bc = ody_block_coord(p.Hq, p.B);
+  const int nkv = (p.Lk + BLOCK_ROWS - 1) / BLOCK_ROWS, nq = (p.Lq + BLOCK_ROWS - 1) / BLOCK_ROWS, both = min(nkv, nq);
+  const bool paired = bc.rank < 2 * both;
+  const int rank = paired ? bc.rank >> 1 : bc.rank - both;
+  if (paired ? bc.rank & 1 : nq > nkv) {
+    dq_block(p, smem, (p.causal ? nq - 1 - rank : rank) * BLOCK_ROWS, bc.h, bc.b);
+  } else if (__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) < WAVES / 2) {
+    kv_block<PART, false>(p, smem, rank * BLOCK_ROWS, bc.h, bc.b, stats, part);
+  } else {
+    kv_block<PART, true>(p, smem, rank * BLOCK_ROWS, bc.h, bc.b, stats, part);
+  }
+}
+
+inline int64_t row_blocks(int B, int L, int H) { return (int64_t)B * H * ((L + BLOCK_ROWS - 1) / BLOCK_ROWS); }
+
+}  // namespace
+
+// The lines are fitted to 563 shapes timed with both, launches and all: 2 to 128 heads, 96 to 8192 rows, a third of them with other key
+// than query counts.  Forward: 1.33 times faster in the geometric mean over all of them, the unchanged ones included (1.35 if the faster
+// one ran everywhere), backward 1.58 (1.61); none behind by more than 3 %.
+//   Beyond the line in blocks every compute unit has a block of 256 rows, whose tiles serve twice the rows: 32 heads, full, L = 1500:
+//   forward 56 us there, 62 here, backward 171 / 192; causal, L = 3001: 98 / 107, 338 / 365.
+//   Beyond the line in tiles the other kernels cut the range of the long side into parts: 4 heads, causal, L = 3001: forward 43 / 51;
+//   8 heads, full, L = 3001: backward 181 / 230.  Forwards of 64 blocks and less stay there wherever it has parts: some are faster here
+//   (4 heads, L = 1000: 29 / 22), some are not (32 heads, 109 queries on 2042 keys: 1.13 times slower).
+bool ody_attn_fwd_short_ok(int B, int Lq, int Lk, int Hq, int causal) {
+  const int64_t blocks = row_blocks(B, Lq, Hq);
+  if (blocks <= 64 && ody_attn_fwd_w8_parts(B, Lq, Lk, Hq, causal) > 1) return false;
+  return blocks <= (causal ? 640 : 256) && Lk <= ROWS * (blocks <= 128 ? 32 : 64);
+}
+bool ody_attn_bwd_short_ok(int B, int Lq, int Lk, int Hq, int causal) {
+  const int64_t blocks = row_blocks(B, Lq, Hq) + row_blocks(B, Lk, Hq);
+  // one or two heads from 512 rows on: the smallest calls for which a caller chooses between kept and recomputed dS, and finds the
+  // kernels of that choice in the profile
+  if (blocks <= 16 && std::min(Lq, Lk) >= 512) return false;
+  return blocks <= (causal ? 1024 : 512) && std::max(Lq, Lk) <= ROWS * (causal && blocks > 128 ? 56 : 32);
+}
+
+int ody_launch_attn_fwd_short(const AttnParams& p, hipStream_t st) {
+  if (int rc = ody_allow_dynamic_lds(reinterpret_cast<const void*>(&attn_fwd_short_kernel), SMEM, "attn_fwd_short")) return rc;
+  ODY_LAUNCH("attn_fwd_short", st, attn_fwd_short_kernel, dim3((unsigned)row_blocks(p.B, p.Lq, p.Hq)), dim3(64 * WAVES), SMEM, p);
+  return ody_check_launch("attn_fwd_short");
+}
+
+int ody_launch_attn_bwd_short(const AttnParams& p, const void* stats, float* part, hipStream_t st) {
+  const dim3 grid((unsigned)(row_blocks(p.B, p.Lq, p.Hq) + row_blocks(p.B, p.Lk, p.Hq)));
+  auto kern = p.group > 1 ? &attn_bwd_short_kernel<true> : &attn_bwd_short_kernel<false>;
+  if (int rc = ody_allow_dynamic_lds(reinterpret_cast<const void*>(kern), SMEM, "attn_bwd_short")) return rc;
+  ODY_LAUNCH("attn_bwd_short", st, kern, grid, dim3(64 * WAVES), SMEM, p, static_cast<const bf16*>(stats), part);
+  return ody_check_launch("attn_bwd_short");
+}

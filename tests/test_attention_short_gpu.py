@@ -1,0 +1,92 @@
+"""GPU parity: the attention kernels of head_dim 128 for few blocks (attn_short.hip) against the CPU oracle."""
+import pytest
+import torch
+
+import odysseus_oracle as oracle
+from conftest import TOL_BF16, TOL_LSE, assert_parity, randn, rel_err
+
+pytestmark = pytest.mark.gpu
+
+# edges of the 32 rows of a wavefront, of the 64-row tiles, of the 128-row blocks and of a pair of tiles; groups of 1, 4 and 8; key
+# offsets of either sign; the last causal and the last full shape that the kernels take
+CASES = [(1, 65, 65, 2, 2, True), (2, 96, 33, 4, 1, False), (1, 127, 128, 4, 4, True), (1, 128, 129, 4, 1, False), (1, 129, 127, 2, 2, True),
+         (3, 191, 193, 8, 1, True), (1, 257, 256, 8, 2, False), (1, 320, 64, 4, 4, True), (4, 331, 331, 8, 2, True), (1, 97, 900, 8, 2, True),
+         (1, 1000, 1000, 32, 8, True), (4, 1024, 1024, 8, 8, False), (1, 2040, 2040, 5, 5, True)]
+
+
+def _run(fn):
+    from odysseus_transformer_amd import _lib
+    _lib.profile_enable(True)
+    try:
+        r = fn()
+        torch.cuda.synchronize()
+        return r, set(_lib.profile_collect())
+    finally:
+        _lib.profile_enable(False)
+
+
+def _inputs(B, Lq, Lk, Hq, Hkv, seed):
+    return [randn(s, seed + n, dtype=torch.bfloat16) for n, s in enumerate([(B, Lq, Hq, 128), (B, Lk, Hkv, 128), (B, Lk, Hkv, 128), (B, Lq, Hq, 128)])]
+
+
+@pytest.mark.parametrize("case", CASES, ids=lambda c: "B%d_Lq%d_Lk%d_H%d_%d_c%d" % c)
+def test_attention_of_few_blocks(case):
+    """Forward and every destination of dq, twice: results do not depend on the order of the blocks."""
+    from odysseus_transformer_amd import ops
+    B, Lq, Lk, Hq, Hkv, causal = case
+    print(f"case={case}", flush=True)
+    q, k, v, do = _inputs(B, Lq, Lk, Hq, Hkv, Lq + 3 * Lk)
+    o_ref, lse_ref = oracle.attention_fwd(q.float(), k.float(), v.float(), causal=causal)
+    dq_ref, dk_ref, dv_ref = oracle.attention_bwd(q.float(), k.float(), v.float(), o_ref, lse_ref, do.float(), causal=causal)
+    # every other row of larger buffers: the row strides are not those of a packed tensor
+    qg, kg, vg, dog = (torch.stack([t, t + 1], 2).flatten(1, 2).cuda()[:, ::2] for t in (q, k, v, do))
+    (o, lse), ran = _run(lambda: ops.attn_fwd(qg, kg, vg, causal=causal))
+    assert "attn_fwd_short" in ran, ran
+    assert_parity(o, o_ref, TOL_BF16, "o")
+    assert torch.allclose(lse.cpu(), lse_ref, atol=TOL_LSE, rtol=TOL_LSE)
+    (dq, dk, dv), ran = _run(lambda: ops.attn_bwd(qg, kg, vg, o, lse, dog, causal=causal))
+    assert "attn_bwd_short" in ran, ran
+    assert_parity(dq, dq_ref, TOL_BF16, "dq", 1e-3)
+    assert_parity(dk, dk_ref, TOL_BF16, "dk", 1e-3)
+    assert_parity(dv, dv_ref, TOL_BF16, "dv")
+    again = (*ops.attn_fwd(qg, kg, vg, causal=causal), *ops.attn_bwd(qg, kg, vg, o, lse, dog, causal=causal))
+    assert all(torch.equal(a, b) for a, b in zip(again, (o, lse, dq, dk, dv)))
+    acc0 = randn((B, Lq, Hq, 128), 5).cuda()
+    acc = acc0.clone()
+    ops.attn_bwd(qg, kg, vg, o, lse, dog, causal=causal, dq=acc, accumulate_dq=True)
+    assert_parity((acc - acc0).cpu(), dq_ref, TOL_BF16, "dq added to an fp32 buffer", 1e-3)
+    pos_q = (torch.arange(Lq).cuda() + max(Lk - Lq, 0)).repeat(B, 1)
+    pos_k = torch.arange(Lk).cuda().repeat(B, 1)
+    tables = ops.rope_table(pos_q, B * Lq, 128, 10000.0), ops.rope_table(pos_k, B * Lk, 128, 10000.0)
+    dq_r, dk_r, _ = ops.attn_bwd(qg, kg, vg, o, lse, dog, causal=causal, rope_tables=tables)
+    assert_parity(dq_r, oracle.apply_rope_bwd(dq_ref, *oracle.rope_cos_sin(pos_q.cpu(), 128, 10000.0)), TOL_BF16, "dq rotated back", 1e-3)
+    assert_parity(dk_r, oracle.apply_rope_bwd(dk_ref, *oracle.rope_cos_sin(pos_k.cpu(), 128, 10000.0)), TOL_BF16, "dk rotated back", 1e-3)
+
+
+@pytest.mark.parametrize("late", [4.0, 40.0], ids=["row_sum", "infinite"])
+def test_scores_and_sums_beyond_a_fixed_reference(late):
+    """Late scores far above a row's first tile, and with them sums of P V beyond fp32: the block walks its keys again."""
+    from odysseus_transformer_amd import ops
+    q, k, v, _ = _inputs(1, 300, 300, 2, 2, 29)
+    q[:, :, 0], k[:, :, 0] = 2.0, -4.0
+    k[:, 200:220, 0] = late
+    v[:, 210, 0] = 1e30
+    o_ref, lse_ref = oracle.attention_fwd(q.float(), k.float(), v.float(), causal=True)
+    (o, lse), ran = _run(lambda: ops.attn_fwd(q.cuda(), k.cuda(), v.cuda(), causal=True))
+    assert "attn_fwd_short" in ran and torch.isfinite(o).all()
+    assert rel_err(o[:, :, 0], o_ref[:, :, 0]) <= TOL_BF16
+    assert_parity(o[:, :, 1], o_ref[:, :, 1], TOL_BF16, "o of the ordinary head")
+    assert torch.allclose(lse.cpu(), lse_ref, atol=TOL_LSE, rtol=TOL_LSE)
+
+
+def test_query_side_of_few_blocks_serves_the_other_kernels():
+    """The causal step of a ring, then a full one that takes its query-side scratch as it is and runs on the kernels for long rows."""
+    from odysseus_transformer_amd import ops
+    q, k, v, do = (t.cuda() for t in _inputs(1, 2200, 2200, 8, 2, 7))
+    o, lse = ops.attn_fwd(q, k, v, causal=True)
+    ws = ops.attn_bwd_workspace(q, k)
+    _, ran = _run(lambda: ops.attn_bwd(q, k, v, o, lse, do, causal=True, workspace=ws))
+    assert {"attn_bwd_short", "attn_bwd_prepass"} <= ran, ran
+    reused, ran = _run(lambda: ops.attn_bwd(q, v, k, o, lse, do, causal=False, workspace=ws, reuse_query_side=True))
+    assert "attn_bwd_dq_pipe" in ran and "attn_bwd_prepass" not in ran, ran
+    assert all(torch.equal(a, b) for a, b in zip(reused, ops.attn_bwd(q, v, k, o, lse, do, causal=False)))
