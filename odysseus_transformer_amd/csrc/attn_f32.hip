@@ -2,7 +2,7 @@
 // pre-pass shared with the bf16 backward.
 //
 // These kernels serve the fp32 configuration, whose 1e-4 tolerance rules out bf16
-// operands.  All products run on v_mfma_f32_32x32x2_f32 (lane = 32 g + i holds
+// operands: head_dim 128, dropout, and the shortest forwards of head_dim 64, whose other calls are in attn_f32_parts.hip.  All products run on v_mfma_f32_32x32x2_f32 (lane = 32 g + i holds
 // A[row i][k = g] and B[k = g][col i]; the 32 x 32 result sits in 16 registers,
 // register r of lane (i, g) = row 8 (r / 4) + 4 g + r % 4, column i).
 //
@@ -31,46 +31,15 @@
 // Everything is deterministic: no atomics, fixed summation order.
 #include <algorithm>
 #include <cmath>
-#include "attn_params.h"
-#include "attn_tile.h"
+#include "attn_f32.h"
 
 namespace {
+
+using namespace f32tile;
 
 constexpr int F_WAVES = 4;
 constexpr int F_THREADS = 64 * F_WAVES;
 constexpr int F_ROWS = 32 * F_WAVES;  // rows owned by a workgroup
-constexpr int F_TILE = 32;            // rows of the streamed side per LDS tile
-constexpr float LN2 = 0.6931471805599453f;
-
-__device__ __forceinline__ f32x16 mfma_f32(float a, float b, f32x16 c) {
-  return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
-}
-
-// row of a 32-row tile that result register r of a lane in half g holds
-__device__ __forceinline__ int acc_row(int r, int g) { return 8 * (r >> 2) + 4 * g + (r & 3); }
-
-// One 32-row tile of a (rows, D) fp32 matrix on its way from global memory to LDS, brought by NT threads: 8 D / NT
-// 16-byte pieces per thread, rows past `nvalid` read as zero.
-template <int D, int NT>
-struct TileRegs {
-  static constexpr int N = 8 * D / NT, LD = D + 4;
-  f32x4 v[N];
-  __device__ __forceinline__ void fetch(const float* src, int64_t stride, int row0, int nvalid, int tid) {
-#pragma unroll
-    for (int c = 0; c < N; c++) {
-      const int e = tid + c * NT, r = e / (D / 4), x = e % (D / 4);
-      v[c] = (r < nvalid) ? *reinterpret_cast<const f32x4*>(src + (int64_t)(row0 + r) * stride + 4 * x)
-                          : f32x4{0.f, 0.f, 0.f, 0.f};
-    }
-  }
-  __device__ __forceinline__ void put(float* dst, int tid) const {
-#pragma unroll
-    for (int c = 0; c < N; c++) {
-      const int e = tid + c * NT, r = e / (D / 4), x = e % (D / 4);
-      *reinterpret_cast<f32x4*>(dst + r * LD + 4 * x) = v[c];
-    }
-  }
-};
 
 // Geometry of an instance: who owns which rows, who streams which tiles, through which LDS.
 template <int D, bool SPLIT>
@@ -114,83 +83,6 @@ __device__ __forceinline__ void sum_wavefronts(float* lds, const f32x16 (&acc)[D
     if (add) v += *out;
     *out = v;
   }
-}
-
-// The resident operand of a head_dim contraction: row `row` of a (rows, D) matrix in
-// k-step order (element 4 j + t = column 8 j + 4 g + t), times `mul`.
-template <int D>
-__device__ __forceinline__ void load_row_frag(float (&f)[D / 2], const float* base, int64_t stride, int row, bool ok,
-                                              int g, float mul) {
-#pragma unroll
-  for (int j = 0; j < D / 8; j++) {
-    const f32x4 v = ok ? *reinterpret_cast<const f32x4*>(base + (int64_t)row * stride + 8 * j + 4 * g)
-                       : f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int t = 0; t < 4; t++) f[4 * j + t] = v[t] * mul;
-  }
-}
-
-// acc (+)= T F^T for a 32-row LDS tile T (rows = MFMA rows) and a resident fragment F;
-// two accumulation chains, summed by the caller.
-template <int D>
-__device__ __forceinline__ void tile_times_frag(const float* tile, int i, int g, const float (&f)[D / 2], f32x16& c0,
-                                                f32x16& c1) {
-  constexpr int LD = D + 4;
-#pragma unroll
-  for (int j = 0; j < D / 8; j++) {
-    const f32x4 a = *reinterpret_cast<const f32x4*>(tile + i * LD + 8 * j + 4 * g);
-#pragma unroll
-    for (int t = 0; t < 4; t++) {
-      if (j & 1) c1 = mfma_f32(a[t], f[4 * j + t], c1);
-      else c0 = mfma_f32(a[t], f[4 * j + t], c0);
-    }
-  }
-}
-
-// Two products of that kind at once, interleaved: each is the other's independent chain.
-template <int D>
-__device__ __forceinline__ void tiles_times_frags(const float* ta, const float (&fa)[D / 2], f32x16& ca, const float* tb,
-                                                  const float (&fb)[D / 2], f32x16& cb, int i, int g) {
-  constexpr int LD = D + 4;
-#pragma unroll
-  for (int j = 0; j < D / 8; j++) {
-    const f32x4 a = *reinterpret_cast<const f32x4*>(ta + i * LD + 8 * j + 4 * g);
-    const f32x4 b = *reinterpret_cast<const f32x4*>(tb + i * LD + 8 * j + 4 * g);
-#pragma unroll
-    for (int t = 0; t < 4; t++) {
-      ca = mfma_f32(a[t], fa[4 * j + t], ca);
-      cb = mfma_f32(b[t], fb[4 * j + t], cb);
-    }
-  }
-}
-
-// acc[db] += T^T W for a 32-row LDS tile T (its 32 rows are contracted) and the weights
-// W held in result-register order; D / 32 independent chains.
-template <int D>
-__device__ __forceinline__ void tile_t_times_regs(const float* tile, int i, int g, const f32x16& w,
-                                                  f32x16 (&acc)[D / 32]) {
-  constexpr int LD = D + 4;
-#pragma unroll
-  for (int ks = 0; ks < 16; ks++) {
-    const float* row = tile + acc_row(ks, g) * LD + i;
-#pragma unroll
-    for (int db = 0; db < D / 32; db++) acc[db] = mfma_f32(row[32 * db], w[ks], acc[db]);
-  }
-}
-
-// acc[db][r] is element (row i of the owner, column 32 db + 8 (r / 4) + 4 g + r % 4):
-// four consecutive columns per register quad -> one 16-byte store each.
-template <int D>
-__device__ __forceinline__ void store_rows(float* dst, const f32x16 (&acc)[D / 32], int g, float mul, bool add) {
-#pragma unroll
-  for (int db = 0; db < D / 32; db++)
-#pragma unroll
-    for (int a = 0; a < 4; a++) {
-      f32x4* out = reinterpret_cast<f32x4*>(dst + 32 * db + 8 * a + 4 * g);
-      f32x4 v{acc[db][4 * a] * mul, acc[db][4 * a + 1] * mul, acc[db][4 * a + 2] * mul, acc[db][4 * a + 3] * mul};
-      if (add) v += *out;
-      *out = v;
-    }
 }
 
 // ---------------------------------------------------------------------------------------
@@ -608,8 +500,16 @@ int launch_one(const char* name, K kern, int rows, int heads, const AttnParams& 
 template <int D, bool DROP>
 int launch_fwd(const AttnParams& p, hipStream_t st) {
   const int heads = p.Hq * p.B;
-  if (few_rows<D>(p.Lq, heads, walk(p, false))) return launch_one<D, true>("attn_fwd_f32_split", &attn_fwd_f32_kernel<D, DROP, true>, p.Lq, heads, p, st);
-  return launch_one<D, false>("attn_fwd_f32", &attn_fwd_f32_kernel<D, DROP, false>, p.Lq, heads, p, st);
+  const bool few = few_rows<D>(p.Lq, heads, walk(p, false));
+  if constexpr (D == 64 && !DROP) {
+    // a tile for each wavefront and no more: the products are over before splitting the operands pays (8 heads, 71 tokens: 9.8 us here,
+    // 10.9 there; 300 tokens 15.6 and 14.0)
+    if (few && p.Lk <= Shape<D, true>::STEP) return launch_one<D, true>("attn_fwd_f32_split", &attn_fwd_f32_kernel<D, DROP, true>, p.Lq, heads, p, st);
+    return ody_launch_attn_fwd_f32_parts(p, st);
+  } else {
+    if (few) return launch_one<D, true>("attn_fwd_f32_split", &attn_fwd_f32_kernel<D, DROP, true>, p.Lq, heads, p, st);
+    return launch_one<D, false>("attn_fwd_f32", &attn_fwd_f32_kernel<D, DROP, false>, p.Lq, heads, p, st);
+  }
 }
 
 template <int D, bool DROP, bool SPLIT>
@@ -625,11 +525,16 @@ int launch_dkdv(const AttnParams& p, hipStream_t st) {
 
 template <int D, bool DROP>
 int launch_bwd(const AttnParams& p, hipStream_t st) {
-  const int rc = few_rows<D>(p.Lk, p.Hkv * p.B, walk(p, true)) ? launch_dkdv<D, DROP, true>(p, st) : launch_dkdv<D, DROP, false>(p, st);
-  if (rc) return rc;
-  const int heads = p.Hq * p.B;
-  if (few_rows<D>(p.Lq, heads, walk(p, false))) return launch_one<D, true>("attn_bwd_dq_f32_split", &attn_bwd_dq_f32_kernel<D, DROP, true>, p.Lq, heads, p, st);
-  return launch_one<D, false>("attn_bwd_dq_f32", &attn_bwd_dq_f32_kernel<D, DROP, false>, p.Lq, heads, p, st);
+  if constexpr (D == 64 && !DROP) {
+    if (int rc = ody_launch_attn_bwd_dkdv_f32_parts(p, st)) return rc;
+    return ody_launch_attn_bwd_dq_f32_parts(p, st);
+  } else {
+    const int rc = few_rows<D>(p.Lk, p.Hkv * p.B, walk(p, true)) ? launch_dkdv<D, DROP, true>(p, st) : launch_dkdv<D, DROP, false>(p, st);
+    if (rc) return rc;
+    const int heads = p.Hq * p.B;
+    if (few_rows<D>(p.Lq, heads, walk(p, false))) return launch_one<D, true>("attn_bwd_dq_f32_split", &attn_bwd_dq_f32_kernel<D, DROP, true>, p.Lq, heads, p, st);
+    return launch_one<D, false>("attn_bwd_dq_f32", &attn_bwd_dq_f32_kernel<D, DROP, false>, p.Lq, heads, p, st);
+  }
 }
 
 template <typename T, int D>

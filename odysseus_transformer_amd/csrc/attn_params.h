@@ -113,7 +113,11 @@ int ody_launch_attn_fwd_short(const AttnParams& p, hipStream_t st);
 int ody_launch_attn_bwd_short(const AttnParams& p, const void* stats, float* part, hipStream_t st);
 // with dropout, both head dims
 int ody_launch_attn_bwd_mfma(const AttnParams& p, int D, hipStream_t st);
-// fp32 on the fp32 matrix cores
+// fp32, head_dim 64, no dropout, on the bf16 matrix cores in three parts per value (attn_f32_parts.hip)
+int ody_launch_attn_fwd_f32_parts(const AttnParams& p, hipStream_t st);
+int ody_launch_attn_bwd_dq_f32_parts(const AttnParams& p, hipStream_t st);
+int ody_launch_attn_bwd_dkdv_f32_parts(const AttnParams& p, hipStream_t st);
+// fp32, the rest on the fp32 matrix cores
 int ody_launch_attn_fwd_f32(const AttnParams& p, int D, hipStream_t st);
 int ody_launch_attn_bwd_f32(const AttnParams& p, int D, hipStream_t st);
 int ody_launch_attn_delta(const AttnParams& p, int D, int dtype, hipStream_t st);
