@@ -29,6 +29,7 @@
 // 1614 / 1600).  A call between two events of its own shows the launch and the clock's way up as well: the second NT product
 // 1320 right after idling (torch.matmul 1300 to 1550), 1480 once the card has worked for a second (1470).
 #pragma once
+#include <type_traits>
 #include "gemm_epi.h"
 
 namespace gemm_tile {
@@ -141,12 +142,35 @@ __device__ __forceinline__ int xcd_position(int id, int n) {
   return x * whole + min(x, extra) + (id >> 3);
 }
 
-// The BM x BN results from row m0 and column n0 on (n0 / BN = tn), this wavefront's share
-template <bool A_KC, bool B_KC, int BM, int BN, bool SPLITK, int EPI>
-__device__ __forceinline__ void gemm_tile_block(const Args& p, int m0, int tn) {
+// First row and column (in tiles) of the tile at a position of the walk: down M in groups of 8 tiles, so that the tiles in flight share
+// panels of both operands
+struct TileAt { int m, n; };
+__device__ __forceinline__ TileAt tile_at(const Args& p, int pos) {
+  constexpr int GROUP = 8;
+  const int per_group = GROUP * p.tiles_n, first_m = pos / per_group * GROUP, gsz = min(p.tiles_m - first_m, GROUP);
+  return TileAt{first_m + (pos % per_group) % gsz, (pos % per_group) / gsz};
+}
+
+// The lane, to the compiler a new value each time: what follows from it inside a loop is formed there and takes no registers in between
+__device__ __forceinline__ int lane_anew() {
+  int x;
+  asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(x));
+  return x;
+}
+
+constexpr int ROUND = 256;   // blocks of a launch whose blocks take several tiles: one per compute unit
+
+// The BM x BN results from row m0 and column n0 on (n0 / BN = tn), this wavefront's share.
+//
+// ROUNDS: the block goes on to the tiles ROUND ids further, up to `tiles` of them, without a break: the last slabs of a tile load the first ones
+// of the next, and a group stores its results in its memory phase, while the other one multiplies.  A wavefront's patch for them is the part
+// of the A stage just read that its own loads fill, so that nobody waits for anybody.  K of three slabs and more.
+template <bool A_KC, bool B_KC, int BM, int BN, bool SPLITK, int EPI, bool ROUNDS = false>
+__device__ __forceinline__ void gemm_tile_block(const Args& p, int m0, int tn, int tiles = 0) {
   constexpr int WM = BM / 32, WN = BN / 64;      // 16-row blocks per wavefront: rows BM / 2, columns BN / 4
   constexpr int HALF = BM / 2, NH = WN / 2;
   static_assert(EPI == EPI_NONE || !SPLITK, "fused epilogues: one pass over K");
+  static_assert(!ROUNDS || (EPI == EPI_NONE && !SPLITK && BM == 256 && BN == 256), "several tiles a block: plain products");
   static_assert((EPI != EPI_SWIGLU_FWD && EPI != EPI_ROPE) || (A_KC && B_KC), "these epilogues belong to the NT product");
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
   bf16* As = reinterpret_cast<bf16*>(smem);      // [A_STAGES][2 halves][HALF x 64]
@@ -154,7 +178,7 @@ __device__ __forceinline__ void gemm_tile_block(const Args& p, int m0, int tn) {
 
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, c = lane & 15, q = lane >> 4;
   const int wm = wave >> 2, wn = wave & 3;
-  const int n0 = tn * BN;
+  int n0 = tn * BN;
 
   // slabs [s0, s0 + nk) of the K range
   const int slabs = (p.K + BK - 1) / BK;
@@ -168,22 +192,28 @@ __device__ __forceinline__ void gemm_tile_block(const Args& p, int m0, int tn) {
   Mover<A_KC, HALF, 4> ma;
   Mover<B_KC, BN, 8> mb;
   const int j0 = EPI == EPI_SWIGLU_FWD ? tn * (BN / 2) : 0;   // first column of h
-  if (A_KC) ma.init(wn, lane, p.lda, [&](int r) { return min(m0 + wm * HALF + r, p.M - 1) - m0; });
-  else ma.init(wn, lane, p.lda, [&](int col) { return min(m0 + wm * HALF + col, p.M - 8) - m0; });
-  if (EPI == EPI_SWIGLU_FWD)
-    mb.init(wave, lane, p.ldb, [&](int r) { return min(j0 + (r & (BN / 2 - 1)), p.ep.I - 1) + (r < BN / 2 ? 0 : p.ep.I); });
-  else if (B_KC) mb.init(wave, lane, p.ldb, [&](int r) { return min(n0 + r, p.N - 1) - n0; });
-  else mb.init(wave, lane, p.ldb, [&](int col) { return min(n0 + col, p.N - 8) - n0; });
-  const bf16* a_base = A_KC ? p.A + (int64_t)m0 * p.lda : p.A + m0;
-  const bf16* b_base = EPI == EPI_SWIGLU_FWD ? p.B : (B_KC ? p.B + (int64_t)n0 * p.ldb : p.B + n0);
+  const bf16 *a_base, *b_base;
+  auto aim_a = [&](int lane) {
+    if (A_KC) ma.init(wn, lane, p.lda, [&](int r) { return min(m0 + wm * HALF + r, p.M - 1) - m0; });
+    else ma.init(wn, lane, p.lda, [&](int col) { return min(m0 + wm * HALF + col, p.M - 8) - m0; });
+    a_base = A_KC ? p.A + (int64_t)m0 * p.lda : p.A + m0;
+  };
+  auto aim_b = [&](int lane) {
+    if (EPI == EPI_SWIGLU_FWD)
+      mb.init(wave, lane, p.ldb, [&](int r) { return min(j0 + (r & (BN / 2 - 1)), p.ep.I - 1) + (r < BN / 2 ? 0 : p.ep.I); });
+    else if (B_KC) mb.init(wave, lane, p.ldb, [&](int r) { return min(n0 + r, p.N - 1) - n0; });
+    else mb.init(wave, lane, p.ldb, [&](int col) { return min(n0 + col, p.N - 8) - n0; });
+    b_base = EPI == EPI_SWIGLU_FWD ? p.B : (B_KC ? p.B + (int64_t)n0 * p.ldb : p.B + n0);
+  };
+  aim_a(lane);
+  aim_b(lane);
   const int64_t a_slab = A_KC ? BK : BK * p.lda, b_slab = B_KC ? BK : BK * p.ldb;
-  // loads past the range repeat its last slab: in bounds, and nobody reads them
-  auto load_a = [&](int kt) {
-    const int s = s0 + min(kt, nk - 1);
-    ma.load(a_base + s * a_slab, As + (kt & 1) * BM * BK + wm * HALF * BK, wn, lane, p.K - s * BK);
+  auto load_a = [&](int kt, int stage) {
+    const int s = s0 + kt;
+    ma.load(a_base + s * a_slab, As + stage * BM * BK + wm * HALF * BK, wn, lane, p.K - s * BK);
   };
   auto load_b = [&](int kt, int slot) {
-    const int s = s0 + min(kt, nk - 1);
+    const int s = s0 + kt;
     mb.load(b_base + s * b_slab, Bs + slot * BN * BK, wave, lane, p.K - s * BK);
   };
 
@@ -202,22 +232,38 @@ __device__ __forceinline__ void gemm_tile_block(const Args& p, int m0, int tn) {
   const int b_tr = B_KC ? 0 : (8 * q + (c >> 2)) * BN + 16 * ((wn * WN) ^ group_perm<BN>(8 * q + (c >> 2))) + 4 * (c & 3);
 
   f32x4 acc[WM][WN];
+  auto clear_acc = [&] {
 #pragma unroll
-  for (int a = 0; a < WM; a++)
+    for (int a = 0; a < WM; a++)
 #pragma unroll
-    for (int b = 0; b < WN; b++) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int b = 0; b < WN; b++) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+  };
+  clear_acc();
+
+  auto store16 = [](bf16* dst, bf16x8 w) {
+    typedef unsigned raw_t __attribute__((ext_vector_type(4)));
+    __builtin_nontemporal_store(__builtin_bit_cast(raw_t, w), reinterpret_cast<raw_t*>(dst));
+  };
+  auto rounded = [](f32x4 x) {
+    bf16x4 w;
+#pragma unroll
+    for (int e = 0; e < 4; e++) w[e] = (bf16)x[e];
+    return w;
+  };
 
   if (nk > 0) {
     constexpr int NA = Mover<A_KC, HALF, 4>::NINS, NB = Mover<B_KC, BN, 8>::NINS;
     load_b(0, 0);
-    load_a(0);
-    load_b(1, 1);
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NB) : "memory");
+    load_a(0, 0);
+    load_b(min(1, nk - 1), 1);
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(ROUNDS ? 0 : NB) : "memory");
     __builtin_amdgcn_s_barrier();
     if (wm == 1) __builtin_amdgcn_s_barrier();   // the second group runs one phase behind
-    int slot = 0;
-    for (int kt = 0; kt < nk; kt++) {
-      const bf16* At = As + (kt & 1) * BM * BK + wm * HALF * BK;
+    int slot = 0, stage = 0;
+    // one slab, loading slab `na` of A and slab `nb` of B; STORED: behind a tile's stores, which stand behind all loads issued before
+    auto slab = [&](int na, int nb, auto stored) {
+      constexpr bool STORED = decltype(stored)::value;
+      const bf16* At = As + stage * BM * BK + wm * HALF * BK;
       const bf16* Bt = Bs + slot * BN * BK;
       Frags<A_KC, WM> fa;
       Frags<B_KC, WN> fb;
@@ -248,12 +294,13 @@ __device__ __forceinline__ void gemm_tile_block(const Args& p, int m0, int tn) {
           }
         }
         ODY_FENCE();
-        if (ks == 0) load_a(kt + 1);
-        else load_b(kt + 2, slot == 0 ? 2 : slot - 1);
+        if (ks == 0) load_a(na, stage ^ 1);
+        else load_b(nb, slot == 0 ? 2 : slot - 1);
         ODY_FENCE();
       }
       // this wavefront's part of B's next slab has landed (the other group may read it two barriers from here)
-      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(NA + NB) : "memory");
+      if (STORED) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      else asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(NA + NB) : "memory");
       tie(fa);
       tie(fb);
       __builtin_amdgcn_s_barrier();
@@ -271,10 +318,63 @@ __device__ __forceinline__ void gemm_tile_block(const Args& p, int m0, int tn) {
       __builtin_amdgcn_s_barrier();
       asm volatile("" ::: "memory");
       slot = slot == 2 ? 0 : slot + 1;
+      stage ^= 1;
+    };
+    // loads past the range repeat its last slab: in bounds, and nobody reads them
+    if constexpr (!ROUNDS) {
+      for (int kt = 0; kt < nk; kt++) slab(min(kt + 1, nk - 1), min(kt + 2, nk - 1), std::false_type{});
+    } else {
+      for (int id = blockIdx.x;; id += ROUND) {
+        const TileAt at = tile_at(p, xcd_position(id, tiles));
+        const bool more = id + ROUND < tiles;
+        slab(1, 2, std::true_type{});
+        for (int kt = 1; kt < nk; kt++) {
+          int na = kt + 1, nb = kt + 2;
+          if (nb >= nk) {   // the last two slabs
+            if (!more) {
+              na = nb = nk - 1;
+            } else if (na < nk) {
+              const TileAt next = tile_at(p, xcd_position(id + ROUND, tiles));
+              m0 = next.m * BM, n0 = next.n * BN;
+              aim_b(lane_anew());
+              nb = 0;
+            } else {
+              aim_a(lane_anew());
+              na = 0, nb = 1;
+            }
+          }
+          slab(na, nb, std::false_type{});
+        }
+        constexpr int COLS = 16 * WN, EP = COLS + 8, CPR = COLS / 8, RPP = 64 / CPR, OWN = Mover<A_KC, HALF, 4>::NINS * 512;
+        static_assert(16 * EP <= OWN, "16 rows fit");
+        bf16* band = As + (stage ^ 1) * BM * BK + wm * HALF * BK + wn * OWN;
+        const int lane = lane_anew(), c = lane & 15, q = lane >> 4;
+        const int mw = at.m * BM + wm * HALF, nw = at.n * BN + wn * COLS;
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the next tile's first slabs, which the stores would stand behind
+#pragma unroll
+        for (int a = 0; a < WM; a++) {
+          ODY_FENCE();
+          wavefront_sync();
+#pragma unroll
+          for (int b = 0; b < WN; b++) *reinterpret_cast<bf16x4*>(band + c * EP + 16 * b + 4 * q) = rounded(acc[a][b]);
+          wavefront_sync();
+#pragma unroll
+          for (int pass = 0; pass < 16 / RPP; pass++) {
+            const int row = pass * RPP + lane / CPR, ch = lane % CPR, m = mw + 16 * a + row, n = nw + 8 * ch;
+            const bf16x8 v = *reinterpret_cast<const bf16x8*>(band + row * EP + 8 * ch);
+            if (m < p.M && n < p.N) store16(p.C + (int64_t)m * p.ldc + n, v);
+          }
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        ODY_FENCE();
+        if (!more) break;
+        clear_acc();
+      }
     }
     if (wm == 0) __builtin_amdgcn_s_barrier();
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   }
+  if constexpr (ROUNDS) return;
   __syncthreads();   // the epilogue reuses the operand stages
 
   // ---- epilogue.  Lane 16 q + c holds row m = c and columns n = 4 q .. 4 q + 3 of each 16 x 16 block; the blocks leave through a
@@ -282,16 +382,6 @@ __device__ __forceinline__ void gemm_tile_block(const Args& p, int m0, int tn) {
   // rows, by streaming stores: this kernel does not read them again.
   constexpr int COLS = 16 * WN;
   const int mw = m0 + wm * HALF;
-  auto store16 = [](bf16* dst, bf16x8 w) {
-    typedef unsigned raw_t __attribute__((ext_vector_type(4)));
-    __builtin_nontemporal_store(__builtin_bit_cast(raw_t, w), reinterpret_cast<raw_t*>(dst));
-  };
-  auto rounded = [](f32x4 x) {
-    bf16x4 w;
-#pragma unroll
-    for (int e = 0; e < 4; e++) w[e] = (bf16)x[e];
-    return w;
-  };
   auto biased = [&](f32x4 x, int b) {
     if (EPI == EPI_NONE && !SPLITK && p.bias) {
       const bf16x4 bv = *reinterpret_cast<const bf16x4*>(p.bias + min(n0 + wn * COLS + 16 * b + 4 * q, p.N - 4));
@@ -464,13 +554,12 @@ __device__ __forceinline__ void gemm_tile_block(const Args& p, int m0, int tn) {
 }
 #undef ODY_FENCE
 
-// Block -> tile: a walk down M in groups of 8 tiles, so that the tiles in flight share panels of both operands; first the whole
-// tiles, then, PARTS blocks each, those whose halves or quarters fill a last round better (plan_bf16).  (One kernel for both: 0.3 %
+// Block -> tile: first the whole tiles, then, PARTS blocks each, those whose halves or quarters fill a last round better (plan_bf16).  (One kernel for both: 0.3 %
 // slower where halves are taken.)
-template <bool A_KC, bool B_KC, int BM, int BN, bool SPLITK, int EPI, int PARTS>
+template <bool A_KC, bool B_KC, int BM, int BN, bool SPLITK, int EPI, int PARTS, bool ROUNDS>
 __global__ __launch_bounds__(THREADS, BM * BN <= 128 * 128 ? 4 : 2) void gemm_tile_kernel(const Args p) {
   const int whole = p.tiles_m * p.tiles_n - p.cut;
-  int pos = blockIdx.x, part = 0;
+  int pos = ROUNDS && blockIdx.x >= ROUND ? blockIdx.x - ROUND + whole : blockIdx.x, part = 0;
   const bool in_part = BM == 256 && !SPLITK && pos >= whole;
   if (in_part) {
     pos = xcd_position(pos - whole, PARTS * p.cut);
@@ -479,9 +568,8 @@ __global__ __launch_bounds__(THREADS, BM * BN <= 128 * 128 ? 4 : 2) void gemm_ti
   } else {
     pos = xcd_position(pos, whole);
   }
-  constexpr int GROUP = 8;
-  const int per_group = GROUP * p.tiles_n, first_m = pos / per_group * GROUP, gsz = min(p.tiles_m - first_m, GROUP);
-  const int m0 = (first_m + (pos % per_group) % gsz) * BM, tn = (pos % per_group) / gsz;
+  const TileAt at = tile_at(p, pos);
+  const int m0 = at.m * BM, tn = at.n;
   if constexpr (BM == 256 && !SPLITK) {
     if (in_part) {
       const int mp = m0 + 128 * (part & 1);
@@ -496,25 +584,43 @@ __global__ __launch_bounds__(THREADS, BM * BN <= 128 * 128 ? 4 : 2) void gemm_ti
       return;
     }
   }
-  gemm_tile_block<A_KC, B_KC, BM, BN, SPLITK, EPI>(p, m0, tn);
+  gemm_tile_block<A_KC, B_KC, BM, BN, SPLITK, EPI, ROUNDS>(p, m0, tn, whole);
 }
 
-template <bool A_KC, bool B_KC, int BM, int BN, bool SPLITK, int EPI, int PARTS>
-int launch_parts(const char* name, Args a, int splits, hipStream_t st) {
+// Whether the blocks take several tiles each (a grid of ROUND blocks): where there are two rounds and more.  A block of one tile waits about
+// 4 us for its first slabs and its stores, which nothing hides with one block on a unit; here the matrix cores go on meanwhile.  The same
+// sums in the same order.  us before / here: 32768 x 4096 x 512 NT 139 / 118, NN 141 / 121, TN 155 / 136; 4096 x 11008 x 1000 82 / 77, 81 / 76,
+// 87 / 82; 22016 x 4096 x 4096 NT 483 / 476, NN 506 / 494; 8192^3 679 / 673, 705 / 692.  TN's memory phase is the longest of the three (all of its
+// fragments are transposing reads) and has no room for the choice of the next slab: 11008 x 4096 x 2048 151 / 148, but K = 4096 between 0.99
+// and 1.01 of the speed before and 8192^3 767 / 772, so it is left at the former form from there on.
+template <bool A_KC>
+bool takes_rounds(const Args& a) {
+  return a.tiles_m * a.tiles_n - a.cut >= 2 * ROUND && a.K > 2 * BK && (A_KC || a.K < 4096) && a.vec16 && !a.bias && !a.add;
+}
+
+template <bool A_KC, bool B_KC, int BM, int BN, bool SPLITK, int EPI, int PARTS, bool ROUNDS>
+int launch_parts(const char* name, const Args& a, int splits, hipStream_t st) {
   constexpr size_t smem = sizeof(bf16) * BK * (A_STAGES * BM + B_STAGES * BN);
   static_assert(smem >= 8 * 32 * (BN / 4 + 4) * sizeof(float), "the fp32 bands fit in the operand stages");
-  auto kern = &gemm_tile_kernel<A_KC, B_KC, BM, BN, SPLITK, EPI, PARTS>;
+  auto kern = &gemm_tile_kernel<A_KC, B_KC, BM, BN, SPLITK, EPI, PARTS, ROUNDS>;
   if (int rc = ody_allow_dynamic_lds(reinterpret_cast<const void*>(kern), smem, name)) return rc;
-  a.tiles_m = (a.M + BM - 1) / BM, a.tiles_n = (a.N + BN - 1) / BN;
-  if (EPI == EPI_SWIGLU_FWD) a.tiles_n = (a.ep.I + BN / 2 - 1) / (BN / 2);
-  ODY_LAUNCH(name, st, kern, dim3(a.tiles_m * a.tiles_n + (PARTS - 1) * a.cut, splits), dim3(THREADS), smem, a);
+  const int whole = a.tiles_m * a.tiles_n - a.cut;
+  ODY_LAUNCH(name, st, kern, dim3((ROUNDS ? ROUND : whole) + PARTS * a.cut, splits), dim3(THREADS), smem, a);
   return ody_check_launch(name);
 }
 template <bool A_KC, bool B_KC, int BM, int BN, bool SPLITK, int EPI>
-int launch(const char* name, const Args& a, int splits, hipStream_t st) {
-  if constexpr (BM == 256 && !SPLITK)
-    if (a.cut_parts == 4) return launch_parts<A_KC, B_KC, BM, BN, SPLITK, EPI, 4>(name, a, splits, st);
-  return launch_parts<A_KC, B_KC, BM, BN, SPLITK, EPI, 2>(name, a, splits, st);
+int launch(const char* name, Args a, int splits, hipStream_t st) {
+  a.tiles_m = (a.M + BM - 1) / BM, a.tiles_n = (a.N + BN - 1) / BN;
+  if (EPI == EPI_SWIGLU_FWD) a.tiles_n = (a.ep.I + BN / 2 - 1) / (BN / 2);
+  if constexpr (BM == 256 && !SPLITK) {
+    if constexpr (EPI == EPI_NONE && BN == 256)
+      if (takes_rounds<A_KC>(a)) {
+        if (a.cut_parts == 4) return launch_parts<A_KC, B_KC, BM, BN, SPLITK, EPI, 4, true>(name, a, splits, st);
+        return launch_parts<A_KC, B_KC, BM, BN, SPLITK, EPI, 2, true>(name, a, splits, st);
+      }
+    if (a.cut_parts == 4) return launch_parts<A_KC, B_KC, BM, BN, SPLITK, EPI, 4, false>(name, a, splits, st);
+  }
+  return launch_parts<A_KC, B_KC, BM, BN, SPLITK, EPI, 2, false>(name, a, splits, st);
 }
 
 }  // namespace gemm_tile

@@ -267,3 +267,24 @@ def test_tiles_of_a_nearly_empty_last_round(what, M, dev):
         ref = ref + r.float()
     assert rel_err(y, ref.cpu()) <= TOL_BF16
     assert rel_err(y[4096:], ref[4096:].cpu()) <= TOL_BF16
+
+
+@pytest.mark.parametrize("op", ["nt", "nn", "tn"])
+@pytest.mark.parametrize("M,N,K", [(4096, 8192, 64), (4096, 8192, 72), (4096, 8192, 128), (4104, 8200, 136), (4224, 8200, 192), (6152, 8184, 200),
+                                   (5384, 12296, 1000), (12296, 4872, 264)], ids=lambda v: str(v))
+def test_several_tiles_a_block(op, M, N, K, dev):
+    """512 and more tiles of 256 x 256: odd and even numbers of slabs from one on, a partial last one, rounds that are full, short, and left to
+    halves and quarters of tiles.  Same bits as with a bias of zero, where every block has one tile; rows of C some way apart."""
+    from odysseus_transformer_amd import ops
+    print(f"op={op} M={M} N={N} K={K}", flush=True)
+    dt = torch.bfloat16
+    a = randn((K, M) if op == "tn" else (M, K), 1, dtype=dt).to(dev)
+    b = randn((N, K) if op == "nt" else (K, N), 2, std=0.05, dtype=dt).to(dev)
+    code = {"nt": ops.GEMM_NT, "nn": ops.GEMM_NN, "tn": ops.GEMM_TN}[op]
+    y = ops.gemm(code, a, b)
+    assert torch.equal(y, ops.gemm(code, a, b, bias=torch.zeros(N, dtype=dt, device=dev)))
+    ref = (a.float().t() if op == "tn" else a.float()) @ (b.float().t() if op == "nt" else b.float())
+    assert rel_err(y, ref) <= TOL_BF16
+    out = torch.ones((M, N + 8), dtype=dt, device=dev)
+    ops.gemm(code, a, b, out=out[:, :N])
+    assert torch.equal(out[:, :N], y) and bool((out[:, N:] == 1).all())
