@@ -288,3 +288,30 @@ def test_several_tiles_a_block(op, M, N, K, dev):
     out = torch.ones((M, N + 8), dtype=dt, device=dev)
     ops.gemm(code, a, b, out=out[:, :N])
     assert torch.equal(out[:, :N], y) and bool((out[:, N:] == 1).all())
+
+
+@pytest.mark.parametrize("M,K", [(8192, 136), (8456, 192), (12288, 200), (12296, 1000)], ids=lambda v: str(v))
+@pytest.mark.parametrize("what", ["rope", "swiglu", "swiglu_h", "dgrad_swiglu"])
+def test_several_tiles_a_block_with_an_epilogue(what, M, K, dev):
+    """512 and more tiles of 256 x 256 with an epilogue, several of them a block for the forward of SwiGLU: same bits as calls on 4096 rows at
+    a time, whose blocks have one tile."""
+    from odysseus_transformer_amd import ops
+    print(f"what={what} M={M} K={K}", flush=True)
+    dt, N = torch.bfloat16, 4096
+    x, w = randn((M, K), 1, dtype=dt).to(dev), randn((N, K), 2, std=0.05, dtype=dt).to(dev)
+    if what == "rope":
+        table = ops.rope_table(torch.arange(M, device=dev), M, 128)
+        run = lambda r: [ops.linear_rope(x[r], w, table[r], 20, 128)]
+    elif what == "swiglu":
+        run = lambda r: ops.linear_swiglu(x[r], w)
+    elif what == "swiglu_h":
+        run = lambda r: [ops.linear_swiglu_h(x[r], w)]
+    else:
+        gate_up, down = randn((M, 2 * N), 3, dtype=dt).to(dev), w.t().contiguous()
+        run = lambda r: [ops.linear_dgrad_swiglu(x[r], down, gate_up[r])]
+    whole = run(slice(0, M))
+    for m in range(0, M - 4095, 4096):
+        for got, want in zip(whole, run(slice(m, m + 4096))):
+            assert torch.equal(got[m:m + 4096], want)
+    for got, want in zip(whole, run(slice(M - 264, M))):   # K in ranges there, perhaps
+        assert rel_err(got[M - 264:], want.float()) <= TOL_BF16
