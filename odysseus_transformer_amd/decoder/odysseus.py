@@ -375,12 +375,25 @@ class OdysseusDecoderLayer(nn.Module):
     def _folds_norms(self, hidden_states) -> bool:
         """A decoding step, or a handful of tokens that nothing records: the modules get the rows before their norm and the norm, which
         then rides in the prologue of their first product.  Only where nobody else would see those rows instead of the normalised
-        ones: no hooks, and the modules that this class made."""
+        ones, or a keyword that he does not know: modules that run what this file defines, and nothing around it."""
         attn, mlp, norms = self.self_attn, self.mlp, (self.input_layernorm, self.post_attention_layernorm)
         return (hidden_states.is_cuda and hidden_states.dtype == torch.bfloat16 and hidden_states.dim() == 3
                 and hidden_states.shape[0] * hidden_states.shape[1] <= ops.NORM_LINEAR_MAX_ROWS and not ops.watched()
-                and type(attn) is LlamaFlashAttention2TPSP and type(mlp) is LlamaMLPZeRO
-                and all(type(n) is LlamaRMSNorm and n.weight.dtype == torch.bfloat16 for n in norms) and not _has_hooks(attn, mlp, *norms))
+                and all(n.weight.dtype == torch.bfloat16 for n in norms)
+                and _runs_its_own_forward(attn, LlamaFlashAttention2TPSP) and _runs_its_own_forward(mlp, LlamaMLPZeRO)
+                and all(_runs_its_own_forward(n, LlamaRMSNorm) for n in norms))
+
+
+_OWN_FORWARD = {cls: cls.forward for cls in (LlamaFlashAttention2TPSP, LlamaMLPZeRO, LlamaRMSNorm)}
+
+
+def _runs_its_own_forward(m, cls) -> bool:
+    """Whether calling `m` is `cls`'s forward of this file and nothing else: no subclass, no forward put on the instance or the class,
+    no compiled call, no hooks of the module or of all modules."""
+    everywhere = torch.nn.modules.module
+    return (type(m) is cls and cls.forward is _OWN_FORWARD[cls] and "forward" not in m.__dict__
+            and getattr(m, "_compiled_call_impl", None) is None and not _has_hooks(m)
+            and not everywhere._global_forward_hooks and not everywhere._global_forward_pre_hooks)
 
 
 def _has_hooks(*modules) -> bool:

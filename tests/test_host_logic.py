@@ -725,3 +725,47 @@ def test_swiglu_backward_of_pitches_beyond_the_tile_kernel_has_room_for_dh(opera
     below, at = ((limit - 8, I), (limit, I)) if operand == "dy" else ((K, limit - 8), (K, limit))
     assert given(*below) == 0
     assert given(*at) >= T * I * 2
+
+
+def _layer_and_a_decoding_step():
+    from odysseus_transformer_amd.decoder.odysseus import OdysseusDecoderLayer
+    cfg = types.SimpleNamespace(hidden_size=256, num_attention_heads=2, num_key_value_heads=1, head_dim=128, intermediate_size=256,
+                                hidden_act="silu", attention_dropout=0.0, rms_norm_eps=1e-6, rope_theta=10000.0, pretraining_tp=1)
+    layer = OdysseusDecoderLayer(cfg).to(torch.bfloat16)
+    return layer, types.SimpleNamespace(is_cuda=True, dtype=torch.bfloat16, shape=(1, 1, 256), dim=lambda: 3)
+
+
+@pytest.mark.parametrize("who", ["self_attn", "mlp", "input_layernorm", "post_attention_layernorm"])
+@pytest.mark.parametrize("what", ["forward", "hook", "pre_hook", "subclass", "class_forward", "compiled"])
+def test_norms_are_folded_only_into_modules_that_run_their_own_forward(what, who, monkeypatch):
+    """Whoever replaced or watches a module's forward gets the rows and arguments that it always got."""
+    layer, x = _layer_and_a_decoding_step()
+    with torch.no_grad():
+        assert layer._folds_norms(x)
+        m = getattr(layer, who)
+        if what == "forward":
+            m.forward = lambda x, residual=None: x
+        elif what == "hook":
+            m.register_forward_hook(lambda m, a, y: None)
+        elif what == "pre_hook":
+            m.register_forward_pre_hook(lambda m, a: None)
+        elif what == "subclass":
+            m.__class__ = type("Other", (type(m),), {})
+        elif what == "class_forward":
+            monkeypatch.setattr(type(m), "forward", lambda self, x, residual=None: x)
+        else:
+            m._compiled_call_impl = lambda *a: None
+        assert not layer._folds_norms(x)
+
+
+@pytest.mark.parametrize("register", ["register_module_forward_pre_hook", "register_module_forward_hook"])
+def test_norms_are_not_folded_under_hooks_of_all_modules(register):
+    layer, x = _layer_and_a_decoding_step()
+    with torch.no_grad():
+        assert layer._folds_norms(x)
+        h = getattr(torch.nn.modules.module, register)(lambda *a: None)
+        try:
+            assert not layer._folds_norms(x)
+        finally:
+            h.remove()
+        assert layer._folds_norms(x)
