@@ -376,24 +376,27 @@ class OdysseusDecoderLayer(nn.Module):
         """A decoding step, or a handful of tokens that nothing records: the modules get the rows before their norm and the norm, which
         then rides in the prologue of their first product.  Only where nobody else would see those rows instead of the normalised
         ones, or a keyword that he does not know: modules that run what this file defines, and nothing around it."""
-        attn, mlp, norms = self.self_attn, self.mlp, (self.input_layernorm, self.post_attention_layernorm)
-        return (hidden_states.is_cuda and hidden_states.dtype == torch.bfloat16 and hidden_states.dim() == 3
-                and hidden_states.shape[0] * hidden_states.shape[1] <= ops.NORM_LINEAR_MAX_ROWS and not ops.watched()
-                and all(n.weight.dtype == torch.bfloat16 for n in norms)
-                and _runs_its_own_forward(attn, LlamaFlashAttention2TPSP) and _runs_its_own_forward(mlp, LlamaMLPZeRO)
-                and all(_runs_its_own_forward(n, LlamaRMSNorm) for n in norms))
+        if (not hidden_states.is_cuda or hidden_states.dtype != torch.bfloat16 or hidden_states.dim() != 3
+                or hidden_states.shape[0] * hidden_states.shape[1] > ops.NORM_LINEAR_MAX_ROWS or ops.watched()
+                or _EVERY_MODULE._global_forward_hooks or _EVERY_MODULE._global_forward_pre_hooks):
+            return False
+        m = self._modules
+        n1, n2 = m["input_layernorm"], m["post_attention_layernorm"]
+        return (_runs_its_own_forward(m["self_attn"], LlamaFlashAttention2TPSP) and _runs_its_own_forward(m["mlp"], LlamaMLPZeRO)
+                and _runs_its_own_forward(n1, LlamaRMSNorm) and _runs_its_own_forward(n2, LlamaRMSNorm)
+                and n1.weight.dtype == n2.weight.dtype == torch.bfloat16)
 
 
+_EVERY_MODULE = torch.nn.modules.module
 _OWN_FORWARD = {cls: cls.forward for cls in (LlamaFlashAttention2TPSP, LlamaMLPZeRO, LlamaRMSNorm)}
 
 
 def _runs_its_own_forward(m, cls) -> bool:
-    """Whether calling `m` is `cls`'s forward of this file and nothing else: no subclass, no forward put on the instance or the class,
-    no compiled call, no hooks of the module or of all modules."""
-    everywhere = torch.nn.modules.module
-    return (type(m) is cls and cls.forward is _OWN_FORWARD[cls] and "forward" not in m.__dict__
-            and getattr(m, "_compiled_call_impl", None) is None and not _has_hooks(m)
-            and not everywhere._global_forward_hooks and not everywhere._global_forward_pre_hooks)
+    """Whether calling `m` is `cls`'s forward of this file and nothing else of its own: no subclass, no forward put on the instance or
+    the class, no compiled call, no hooks."""
+    d = m.__dict__
+    return (type(m) is cls and cls.forward is _OWN_FORWARD[cls] and "forward" not in d and d.get("_compiled_call_impl") is None
+            and not d["_forward_hooks"] and not d["_forward_pre_hooks"])
 
 
 def _has_hooks(*modules) -> bool:
