@@ -65,22 +65,25 @@ def _compile(src: Path, force: bool) -> Path:
 
 
 def _build_native(force: bool) -> None:
-    if not force and not _newer(NATIVE_SRC, NATIVE_LIB, INCLUDE.glob("*.h")):
-        return
     import torch
+    built_for = OBJ / "native_built_for"   # the module is tied to one torch
+    version = str(torch.__version__)
+    if not force and built_for.exists() and built_for.read_text() == version and not _newer(NATIVE_SRC, NATIVE_LIB, INCLUDE.glob("*.h")):
+        return
     root = Path(torch.__file__).resolve().parent
     rocm = Path(_hipcc()).resolve().parent.parent
     cxx = shutil.which("g++") or shutil.which("c++")
     if cxx is None:
         raise RuntimeError("no host C++ compiler found")
     cmd = [cxx, "-O2", "-std=c++17", "-fPIC", "-shared", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
-           "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", "-I", str(INCLUDE), "-isystem", str(root / "include"), "-isystem",
+           f'-DODY_TORCH_VERSION="{version}"', "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", "-I", str(INCLUDE), "-isystem", str(root / "include"), "-isystem",
            str(root / "include" / "torch" / "csrc" / "api" / "include"), "-isystem", str(rocm / "include"), "-isystem", "/opt/rocm/include",
            "-isystem", sysconfig.get_paths()["include"], str(NATIVE_SRC), "-o", str(NATIVE_LIB), "-L", str(root / "lib"), "-lc10", "-lc10_hip",
            "-ltorch_cpu", "-ltorch_python"]
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError(f"{cxx} failed for {NATIVE_SRC.name}:\n{r.stderr}")
+    built_for.write_text(version)
 
 
 def build(force: bool = False, jobs: int = 4, verbose: bool = True) -> Path:

@@ -484,4 +484,8 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_odysseus_native", nullptr, -1, me
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__odysseus_native() { return PyModule_Create(&module); }
+PyMODINIT_FUNC PyInit__odysseus_native() {
+  PyObject* m = PyModule_Create(&module);
+  if (m && PyModule_AddStringConstant(m, "TORCH_VERSION", ODY_TORCH_VERSION) != 0) Py_CLEAR(m);
+  return m;
+}

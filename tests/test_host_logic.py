@@ -769,3 +769,38 @@ def test_norms_are_not_folded_under_hooks_of_all_modules(register):
         finally:
             h.remove()
         assert layer._folds_norms(x)
+
+
+@pytest.mark.parametrize("why", ["missing", "not a module", "another torch"])
+def test_ops_without_the_host_module(why, tmp_path, monkeypatch):
+    """The kernels' library is all that the ops need: without a module that fits, every plain form answers None (the Python of the op goes
+    on) after one warning."""
+    import warnings
+    from odysseus_transformer_amd import _lib, _native
+    if not _lib.LIB_PATH.exists() or not _native.PATH.exists():
+        pytest.skip("nothing is built")
+    path = tmp_path / "_odysseus_native.so"
+    if why == "not a module":
+        path.write_bytes(b"no ELF")
+    if why == "another torch":
+        monkeypatch.setattr(torch, "__version__", "0.0.1")
+        path = _native.PATH
+    monkeypatch.setenv("ODYSSEUS_NATIVE_LIB", str(path))
+    native = _native._Native()
+    with pytest.warns(RuntimeWarning, match="cannot be used"):
+        assert native.attn_fwd(1, 2, 3, True, 0.5) is None
+    with warnings.catch_warnings():
+        warnings.simplefilter("error")
+        assert native.attn_fwd(1, 2, 3, True, 0.5) is None and native.gemm(0, None, None) is None
+
+
+def test_host_module_in_another_place(tmp_path, monkeypatch):
+    import shutil
+    from odysseus_transformer_amd import _lib, _native
+    if not _lib.LIB_PATH.exists() or not _native.PATH.exists():
+        pytest.skip("nothing is built")
+    shutil.copy(_native.PATH, tmp_path / "_odysseus_native.so")
+    monkeypatch.setattr(_native, "PATH", tmp_path / "not there")
+    monkeypatch.setenv("ODYSSEUS_NATIVE_LIB", str(tmp_path / "_odysseus_native.so"))
+    native = _native._Native()
+    assert native.gemm(0, None, None) is None and native.TORCH_VERSION == str(torch.__version__)
