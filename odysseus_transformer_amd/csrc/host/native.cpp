@@ -374,10 +374,13 @@ PyObject* rope(Call c) {
   const int64_t n_rot = c.whole(1);
   const int B = x.size(0), L = x.size(1), D = x.size(3);
   need(n_rot >= 0 && n_rot <= x.size(2));
-  need(c.none(2) || THPVariable_CheckExact(c.args[2]));
-  if (!c.none(2)) need(THPVariable_Unpack(c.args[2]).dim() >= 1 && THPVariable_Unpack(c.args[2]).size(-1) == L);
+  if (!c.none(2)) {   // (B, L), or (L) of a batch of one
+    const at::Tensor& given = c.any(2);
+    need((given.dim() == 2 || (given.dim() == 1 && B == 1)) && given.size(-1) == L);
+  }
   const int64_t* pos = positions(c, 2, (int64_t)B * L);
   const at::Tensor& f = frequencies(c, 3, D);
+  need(f.dim() == 1);
   CALL(ody_rope, x.data_ptr(), pos, f.data_ptr<float>(), B, L, (int)n_rot, D, STRIDES(x), (float)c.real(4), (int)c.flag(5), dt(x), (void*)c.stream);
   Py_RETURN_TRUE;
 }

@@ -265,3 +265,123 @@ def test_decoding_layer_folds_its_norms_and_gives_hooks_what_they_had(dev):
     z, ran, seen = step(True)
     assert "rmsnorm_fwd" in ran and torch.equal(seen[0], ops.rmsnorm(x[:, 33:], layer.input_layernorm.weight, 1e-6))
     assert (y.float() - z.float()).norm() <= 1e-2 * z.float().norm()
+
+
+def _refused(fn):
+    try:
+        fn()
+    except Exception as e:  # noqa: BLE001  (its type is the answer)
+        return type(e)
+    return None
+
+
+def test_what_either_path_refuses(dev, monkeypatch):
+    """One definition of what an op takes: the same exception with the module and without it, for operands that no kernel may see."""
+    from odysseus_transformer_amd import ops
+    bf = torch.bfloat16
+    x, w, r = (randn(s, n, dtype=bf).to(dev) for n, s in enumerate([(16, 64), (256, 64), (16, 256)]))
+    f = randn((16, 64), 5).to(dev)
+    n = torch.ones(64, dtype=bf, device=dev)
+    rstd = torch.ones(16, device=dev)
+    table = ops.rope_table(torch.arange(16, device=dev), 16, 128)
+    q, k = randn((2, 8, 4, 128), 6, dtype=bf).to(dev), randn((2, 8, 2, 128), 7, dtype=bf).to(dev)
+    out, lse = ops.attn_fwd(q, k, k)
+    y = randn((2, 8, 4, 64), 8, dtype=bf).to(dev)
+    one = randn((1, 8, 4, 64), 9, dtype=bf).to(dev)
+    pos, inv = torch.arange(8, device=dev), torch.ones(32, device=dev)
+    calls = {
+        "norm: weight of another size": lambda: ops.rmsnorm_fwd(x, n[:32]),
+        "norm: weight of another type": lambda: ops.rmsnorm_fwd(x, n.float()),
+        "norm: strided weight": lambda: ops.rmsnorm_fwd(x[:, :32].contiguous(), n[::2]),
+        "norm: weight of two dimensions": lambda: ops.rmsnorm_fwd(x, n[None]),
+        "norm: rows of another count": lambda: ops.rmsnorm_bwd(x, n, rstd[:8], x),
+        "norm: rstd of another type": lambda: ops.rmsnorm_bwd(x, n, rstd.double(), x),
+        "norm: dy of another shape": lambda: ops.rmsnorm_bwd(x, n, rstd, x[:8]),
+        "norm: dx_add of another type": lambda: ops.rmsnorm_bwd(x, n, rstd, x, f),
+        "gemm: inner extents": lambda: ops.gemm(ops.GEMM_NT, x, r),
+        "gemm: three dimensions": lambda: ops.gemm(ops.GEMM_NT, x[None], w),
+        "gemm: column stride": lambda: ops.gemm(ops.GEMM_NN, x, w.t()),
+        "gemm: op": lambda: ops.gemm(3, x, w),
+        "gemm: odd extent": lambda: ops.gemm(ops.GEMM_NT, x[:, :60], w[:, :60]),
+        "gemm: off a 16-byte boundary": lambda: ops.gemm(ops.GEMM_NT, x[:, 1:57], w[:, 1:57]),
+        "gemm: rows closer than their length": lambda: ops.gemm(ops.GEMM_NT, x.as_strided((4, 64), (8, 1)), w),
+        "residual: shape": lambda: ops.linear_residual(x, w, r[:8]),
+        "residual: type": lambda: ops.linear_residual(x, w, r.float()),
+        "rope: table's rows": lambda: ops.linear_rope(x, w, table[:8], 1, 128),
+        "rope: table's type": lambda: ops.linear_rope(x, w, table.float(), 1, 128),
+        "rope: heads": lambda: ops.linear_rope(x, w, table, 3, 128),
+        "rope: head_dim": lambda: ops.linear_rope(x, w, table, 1, 64),
+        "rope: fp32": lambda: ops.linear_rope(f, w.float(), table, 1, 128),
+        "swiglu: odd rows of the weight": lambda: ops.linear_swiglu(x, w[:255]),
+        "swiglu: inner extents": lambda: ops.linear_swiglu(x, r),
+        "dgrad: gate_up's shape": lambda: ops.linear_dgrad_swiglu(x, w.t().contiguous(), r),
+        "attention: kv shapes": lambda: ops.attn_fwd(q, k, k[:, :7]),
+        "attention: type": lambda: ops.attn_fwd(q, k, k.float()),
+        "attention: heads": lambda: ops.attn_fwd(q, q[:, :, :3], q[:, :, :3]),
+        "attention: head_dim": lambda: ops.attn_fwd(q[..., :32], k[..., :32], k[..., :32]),
+        "attention: stride of head_dim": lambda: ops.attn_fwd(q.transpose(2, 3).contiguous().transpose(2, 3), k, k),
+        "attention: rows off 16 bytes": lambda: ops.attn_fwd(q[..., 4:68], k[..., :64], k[..., :64]),
+        "attention: scale": lambda: ops.attn_fwd(q, k, k, scale=-1.0),
+        "attention: three dimensions": lambda: ops.attn_fwd(q[0], k[0], k[0]),
+        "backward: lse's shape": lambda: ops.attn_bwd(q, k, k, out, lse[:1], out),
+        "backward: lse's type": lambda: ops.attn_bwd(q, k, k, out, lse.double(), out),
+        "backward: dout": lambda: ops.attn_bwd(q, k, k, out, lse, out[:, :4]),
+        "backward: dk": lambda: ops.attn_bwd(q, k, k, out, lse, out, dk=torch.empty_like(q)),
+        "backward: tables": lambda: ops.attn_bwd(q, k, k, out, lse, out, rope_tables=(table[:8], table)),
+        "rotation: positions of three dimensions": lambda: ops.rope_(one, 2, pos[None, None]),
+        "rotation: positions of another batch": lambda: ops.rope_(y, 2, pos.repeat(3, 1)),
+        "rotation: positions of no dimension": lambda: ops.rope_(one, 2, pos[0]),
+        "rotation: positions of another type": lambda: ops.rope_(one, 2, pos.float()[None]),
+        "rotation: all positions in a row": lambda: ops.rope_(y, 2, torch.arange(16, device=dev)),
+        "rotation: frequencies of two dimensions": lambda: ops.rope_(one, 2, pos[None], inv_freq=inv[None]),
+        "rotation: frequencies of another count": lambda: ops.rope_(one, 2, pos[None], inv_freq=inv[:16]),
+        "rotation: heads": lambda: ops.rope_(one, 5, pos[None]),
+        "rotation: odd head_dim": lambda: ops.rope_(one[..., :63], 2, pos[None]),
+        "rotation: three dimensions": lambda: ops.rope_(one[0], 2, pos[None]),
+        "table: positions": lambda: ops.rope_table(pos, 12, 128, inv_freq=torch.ones(64, device=dev)),
+        "table: frequencies": lambda: ops.rope_table(pos, 8, 128, inv_freq=inv),
+        "folded norm: positions": lambda: ops.norm_linear_rope(x[:3], n, 1e-6, w, 1, 128, pos[:2]),
+        "folded norm: weight": lambda: ops.norm_linear_swiglu_h(x[:3], n.float(), 1e-6, w),
+    }
+    for name, fn in calls.items():
+        here = _refused(fn)
+        with monkeypatch.context() as m:
+            m.setattr(ops, "native", _Off())
+            there = _refused(fn)
+        assert here is not None and here == there, (name, here, there)
+    for p in (pos, pos[None]):   # one sequence, either way to write it
+        a, b = one.clone(), one.clone()
+        ops.rope_(a, 4, p)
+        ops.rope_(b, 4, None)
+        assert torch.equal(a, b)
+
+
+def test_threads_and_autocast(dev):
+    """Calls of several threads, each on a stream of its own, and calls under autocast, which the ops themselves do not look at."""
+    import threading
+    from odysseus_transformer_amd import ops
+    q, k, v = (randn((1, 70, h, 128), h, dtype=torch.bfloat16).to(dev) for h in (4, 2, 2))
+    want = (*ops.attn_fwd(q, k, v),)
+    want += (*ops.attn_bwd(q, k, v, *want, want[0]),)
+    torch.cuda.synchronize()
+    wrong = []
+
+    def work():
+        stream = torch.cuda.Stream()
+        with torch.cuda.stream(stream):
+            for _ in range(20):
+                got = (*ops.attn_fwd(q, k, v),)
+                got += (*ops.attn_bwd(q, k, v, *got, got[0]),)
+                stream.synchronize()
+                wrong.extend(1 for a, b in zip(got, want) if not torch.equal(a, b))
+
+    threads = [threading.Thread(target=work) for _ in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not wrong
+    x, w = randn((16, 64), 1).to(dev), randn((32, 64), 2).to(dev)
+    y = ops.gemm(ops.GEMM_NT, x, w)
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        assert torch.equal(ops.gemm(ops.GEMM_NT, x, w), y) and y.dtype == torch.float32
