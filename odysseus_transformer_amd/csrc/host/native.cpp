@@ -11,7 +11,7 @@
 // definition of what an op accepts and of the error it raises.
 //
 // No state but what bind() is given once: the addresses of the library's entry points, so that this module uses the library that
-// Python loaded, and three Python objects.
+// Python loaded, and four Python objects.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
@@ -47,6 +47,7 @@ struct Library {
 PyObject* arena_holder = nullptr;   // class whose attribute `instance` is the scratch arena, or None
 PyObject* scratch_fn = nullptr;     // scratch(nbytes, name, device) of ops.py
 PyObject* raise_fn = nullptr;       // raises for (name, status)
+PyObject* no_memory = nullptr;      // torch.OutOfMemoryError
 
 struct NotPlain {};      // the caller answers None
 struct PythonError {};   // a Python exception is set
@@ -144,7 +145,11 @@ struct Scratch {
       PyObject* device = THPDevice_New_(like);
       PyObject* r = PyObject_CallFunction(scratch_fn, "nsO", (Py_ssize_t)nbytes, name, device);
       Py_XDECREF(device);
-      if (!r) throw PythonError{};
+      if (!r) {
+        if (!PyErr_ExceptionMatches(no_memory)) throw PythonError{};
+        PyErr_Clear();
+        throw NotPlain{};
+      }
       t = THPVariable_Unpack(r);
       Py_DECREF(r);
       return;
@@ -450,10 +455,10 @@ PyObject* method(PyObject*, PyObject* const* args, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
-// (addresses by name, arena holder, scratch, raise)
+// (addresses by name, arena holder, scratch, raise, torch.OutOfMemoryError)
 PyObject* bind(PyObject*, PyObject* const* args, Py_ssize_t n) {
-  if (n != 4 || !PyDict_Check(args[0])) {
-    PyErr_SetString(PyExc_TypeError, "bind(addresses, arena_holder, scratch, raise)");
+  if (n != 5 || !PyDict_Check(args[0])) {
+    PyErr_SetString(PyExc_TypeError, "bind(addresses, arena_holder, scratch, raise, no_memory)");
     return nullptr;
   }
 #define X(name)                                                                      \
@@ -468,8 +473,8 @@ PyObject* bind(PyObject*, PyObject* const* args, Py_ssize_t n) {
   }
   ODY_ENTRY_POINTS(X)
 #undef X
-  PyObject** to[3] = {&arena_holder, &scratch_fn, &raise_fn};
-  for (int i = 0; i < 3; i++) {
+  PyObject** to[4] = {&arena_holder, &scratch_fn, &raise_fn, &no_memory};
+  for (int i = 0; i < 4; i++) {
     Py_INCREF(args[1 + i]);
     Py_XSETREF(*to[i], args[1 + i]);
   }

@@ -385,3 +385,35 @@ def test_threads_and_autocast(dev):
     y = ops.gemm(ops.GEMM_NT, x, w)
     with torch.autocast("cuda", dtype=torch.bfloat16):
         assert torch.equal(ops.gemm(ops.GEMM_NT, x, w), y) and y.dtype == torch.float32
+
+
+def test_arena_without_room_for_all_of_the_scratch(dev, monkeypatch):
+    """The backward of head_dim 64 goes on with the least workspace, as without the module; the products, which have no other way, raise."""
+    from odysseus_transformer_amd import _lib, ops
+    from odysseus_transformer_amd.utils import globals as g
+    q, k, v, do = (randn((1, 300, h, 64), n, dtype=torch.bfloat16).to(dev) for n, h in enumerate((8, 2, 2, 8)))
+    out, lse = ops.attn_fwd(q, k, v)
+    want = ops.attn_bwd(q, k, v, out, lse, do, keep_ds=False)
+    sizes = 1, 300, 300, 8, 2, 64, _lib.ODY_BF16
+    least, full = _lib.load().ody_attn_bwd_workspace_least_bytes(*sizes), _lib.load().ody_attn_bwd_workspace_bytes(*sizes)
+    assert least < full
+
+    class Small(g.GlobalMemoryBuffer):
+        refused = 0
+
+        def get_tensor(self, shape, dtype, name):
+            if shape[0] > least:
+                self.refused += 1
+                raise torch.OutOfMemoryError("no room for that")
+            return super().get_tensor(shape, dtype, name)
+
+    monkeypatch.setattr(g._Arena, "instance", Small(dev))
+    here, there, _ = _both(monkeypatch, lambda: ops.attn_bwd(q, k, v, out, lse, do, keep_ds=False))
+    assert g._Arena.instance.refused >= 2
+    _same(here, there)
+    for a, b in zip(here, want):
+        assert (a.float() - b.float()).norm() <= 1e-2 * b.float().norm()
+    x, w = randn((512, 64 * 512), 4).to(dev), randn((512, 64 * 512), 5).to(dev)
+    assert _lib.load().ody_gemm_workspace_bytes(ops.GEMM_NT, 512, 512, 64 * 512, _lib.ODY_F32) > least
+    with pytest.raises(torch.OutOfMemoryError):
+        ops.gemm(ops.GEMM_NT, x, w)
