@@ -1,7 +1,7 @@
 // fp32 products, C (M, N) = op(A) . op(B) (+ bias) (+ addend), any shape and alignment, on the bf16 matrix cores.
 //
 // An fp32 value is the sum of three bf16 values (split3.h); of the nine products of two such sums the six largest are formed, which
-// leaves out less than 2^-25 of a product, half a rounding of fp32.  The largest one and the five others accumulate apart, so that
+// leaves out at most a unit roundoff of fp32, 2^-24 of a product, and 2^-27.5 in the root mean square.  The largest one and the five others accumulate apart, so that
 // the sum of the large terms is rounded once per 16 of K (the fp32 matrix instruction: every 2).  2-norm error against 64 bits, this
 // / v_mfma_f32_32x32x2_f32 before it, N(0, 1) operands: K = 512 0.8e-7 to 1.3e-7 / 2.9e-7, 2048 1.3e-7 / 2.9e-7, 4096 4.0e-7 / 11.5e-7.
 //
@@ -13,8 +13,8 @@
 // now: 2048 x 1536 x 512 37 / 29, x 2752 60 / 43, x 512 14.8 / 12, 2048 x 512 x 1376 34 / 26, 2048 x 512 x 2752 NN 61 / 46, 2752 x 512 x 2048
 // TN 66 / 54, 512 x 512 x 2048 TN 17.6 / 16.7 (sum over all twelve 454 / 361).
 //
-// An input that is not finite, or that rounds to infinity in bf16, makes 0 x infinity in a product that is none; a wavefront that finds
-// a result that is not finite forms its tiles again on the fp32 instruction, straight from memory.
+// An input that is not finite, or from 2^111.99 on, makes 0 x infinity in a product that is none, and a result from 2^96 on is infinite before
+// SPLIT_DOWN; a wavefront that finds a result that is not finite forms its tiles again on the fp32 instruction, straight from memory.
 #include <algorithm>
 #include <type_traits>
 #include "gemm_tile.h"
@@ -74,7 +74,7 @@ struct Mover {
     for (int e = 0; e < (KC ? N : 4); e++) {
       typename FloatVec<W>::type x;
 #pragma unroll
-      for (int j = 0; j < W; j++) x[j] = KC ? r[e][j] : r[j][e];
+      for (int j = 0; j < W; j++) x[j] = (KC ? r[e][j] : r[j][e]) * SPLIT_UP;
       const Split3<W> s(x);
       bf16* dst = planes + (KC ? row_of(e, t) : row_of(0, t) + e) * PITCH + k_of(0, t);
 #pragma unroll
@@ -265,6 +265,11 @@ __global__ __launch_bounds__(256 * G, waves_per_simd(WM, WN)) void gemm_f32_kern
         }
         hi[a][b] = c;
       }
+  } else {
+#pragma unroll
+    for (int a = 0; a < WM; a++)
+#pragma unroll
+      for (int b = 0; b < WN; b++) hi[a][b] *= SPLIT_DOWN;
   }
   // register r of lane (i, g) of tile (a, b): row m = 32 (wm WM + a) + i, column n = 32 (wn WN + b) + 8 (r / 4) + 4 g + r % 4
 #pragma unroll

@@ -1,11 +1,19 @@
 // fp32 values as sums of three bf16 values, and their products on the bf16 matrix cores.
 //
-// 24 bits of significand are three times 8.  The parts of x keep the exponent range of fp32 (a scale would have to be found first if
-// they were fp16), and x0 y0 + (x0 y1 + x1 y0) + (x0 y2 + x1 y1 + x2 y0) misses x y by x1 y2 + x2 y1 + x2 y2, at most 2^-25 of it.  Values
-// below 2^-110 lose bits of their last part; infinities, NaN and values that round to infinity in bf16 (above 3.39e38) need
-// a path of their own, see the users.
+// 24 bits of significand are three times 8 (the splitting and its products: G. Henry, P. T. P. Tang, A. Heinecke, "Leveraging the
+// bfloat16 Artificial Intelligence Datatype For Higher-Precision Computations", ARITH 2019).  The parts of x keep the exponent range of
+// fp32 (a scale would have to be found first if they were fp16), and x0 y0 + (x0 y1 + x1 y0) + (x0 y2 + x1 y1 + x2 y0) misses x y by
+// x1 y2 + x2 y1 + x2 y2: as |x1| <= 2^-8 |x| and |x2| <= 2^-17 |x|, at most about 2^-24 of it, one unit roundoff of fp32 (x = y just above one);
+// 2^-27.5 in the root mean square of random values.
+//
+// The last bit of a bf16 denormal is 2^-133, so the third part of an x below 2^-110 would lose bits.  Operands are split times SPLIT_UP, which
+// puts the last bit of any fp32 value there, denormals included (the matrix cores take bf16 denormals as they are), and what comes out is
+// SPLIT_DOWN times their product.  Infinities, NaN, operands from 2^111.99 on and results from 2^96 on become infinities or NaN on the way and
+// need a path of their own, see the users.
 #pragma once
 #include "ody_common.h"
+
+constexpr float SPLIT_UP = 0x1p16f, SPLIT_DOWN = 0x1p-32f;
 
 template <int N> struct FloatVec { typedef __attribute__((ext_vector_type(N))) float type; };
 template <int N> struct Bf16Vec { typedef __attribute__((ext_vector_type(N))) __bf16 type; };

@@ -86,3 +86,20 @@ def test_values_far_from_one(scale, dev):
     y = _gemm("nt", a * scale, b)
     ref = (A @ B) * scale
     assert (y.double() - ref).norm() <= _bound(512) * ref.norm()
+
+
+@pytest.mark.parametrize("ea,eb", [(-112, 0), (0, -118), (-122, 100), (-130, 20), (-145, 60), (-60, -70), (100, -60), (113, -113), (-119, 119),
+                                   (60, 50), (-148, 100)], ids=lambda v: str(v))
+@pytest.mark.parametrize("shape", [(65, 68, 36), (512, 512, 2048), (2300, 4100, 40)], ids=lambda s: "M%d_N%d_K%d" % s)
+@pytest.mark.parametrize("op", OPS)
+def test_operands_of_any_size_keep_their_bits(op, shape, ea, eb, dev):
+    """Operands of 2^ea and 2^eb, down to denormals and up to where the parts overflow, each as exact as the type holds it: the bound of
+    operands near one, and the spacing of denormals where the result is one."""
+    M, N, K = shape
+    M = (M + 3) // 4 * 4 if op == "tn" else M
+    _, _, a, b = _operands(op, M, N, K, dev)
+    a, b = (t * 2.0 ** (e // 2) * 2.0 ** (e - e // 2) for t, e in ((a, ea), (b, eb)))
+    A, B = (a.double().t() if op == "tn" else a.double()), (b.double().t() if op == "nt" else b.double())
+    ref = A @ B
+    y = _gemm(op, a, b).double()
+    assert ((y - ref).norm() - 2.0 ** -149 * math.sqrt(M * N) * math.sqrt(K)) <= _bound(K) * ref.norm()
