@@ -1,14 +1,18 @@
 // fp32 attention of head_dim 64 (forward and backward) on the bf16 matrix cores: every operand as the sum of three bf16 values (split3.h),
 // six products for one.
 //
-// The fp32 matrix instruction takes 512 cycles for what these six take in 192; what is left is the splitting (5.5 vector instructions per
+// The fp32 matrix instruction takes 512 cycles for what these six take in 192; what is left is the splitting (6.5 vector instructions per
 // element) and LDS traffic.  Streamed tiles of 32 rows are split on their way from registers to LDS, by the wavefronts that share them, and serve
 // as row operands and, through the transposing read, as transposed ones (attn_rowtile.h); P and dS are split in registers, where they are
 // the next product's operand.  Blocks of 32, 64 or 128 rows (rows_of_block): the more rows share a tile, the less splitting; the fewer, the more
 // blocks.
 //
-// Results that are not finite (an infinity or NaN in the inputs, or values above 3.39e38, whose first part is infinite) are formed again on the
-// fp32 instruction: what comes out is what it gives.
+// Operands are split times SPLIT_UP, so that the parts hold every bit of the smallest of them too, P and dS included: scores and dP take
+// SPLIT_DOWN in the fma that follows them anyway, the results lose their factor where they are stored.  In the forward Q has the factor of K too:
+// what is left out of a K below 2^-110 is 2^-134, times a Q below 2^96 nothing that a score's exponential shows.
+//
+// Results that are not finite (an infinity or NaN in the inputs, operands from 2^96 (Q in the forward) or 2^111 on, sums from 2^96 on) are formed
+// again on the fp32 instruction, and so are those of rows whose scores are all that large and negative: what comes out is what it gives.
 //
 // Before (attn_f32.hip) / here, us: 8 heads, L = 2048, causal: forward 62 / 54, dK and dV 108 / 84, dQ 80 / 62; 16 heads, L = 4096: 387 / 240, 705 / 406,
 // 508 / 315 (143 TFLOP/s forward); 219 shapes of 64 to 8192 rows, 2 to 128 heads: 1.20, 1.37 and 1.34 times in the geometric mean.
@@ -53,35 +57,49 @@ struct Geo {
 // One streamed 32 x 64 tile on its way from memory to LDS: 8 consecutive elements of a row per piece
 template <int NT>
 struct PartTile {
-  static constexpr int N = 4 * D / NT;   // pieces per thread
+  static constexpr int N = 4 * D / NT, STEP = 8 * NT / D;   // pieces per thread, rows between them
   static_assert(N * NT == 4 * D, "whole pieces");
   f32x4 v[N][2];
+  // Rows past nvalid repeat the last one: their P and dS are zero, which a value that is finite leaves so, and one that is not sends the block to
+  // the fp32 instruction.  ZERO, there: they read as zero (on every element of every tile that is an instruction for each).
+  // LEAN: one offset of the thread's own for all of its pieces, fewer registers, and a branch.  For the instance that spills (dK and dV, 8 heads,
+  // L = 2048: 89 us without, 83 with it; dQ 62.3 and 62.9, 16 heads of 4 x 484 rows 37.2 and 38.4).
+  template <bool ZERO, bool LEAN = false>
   __device__ __forceinline__ void fetch(const float* src, int64_t stride, int row0, int nvalid, int tid) {
+    const int first = tid / (D / 8), x = tid % (D / 8);
+    const int64_t own = (int64_t)first * stride + 8 * x;
 #pragma unroll
     for (int n = 0; n < N; n++) {
-      const int e = tid + n * NT, r = e / (D / 8), x = e % (D / 8);
-      const float* s = src + (int64_t)(row0 + min(r, nvalid - 1)) * stride + 8 * x;
+      const int r = first + n * STEP;
+      const float* s;
+      if constexpr (LEAN) {
+        s = src + (int64_t)(row0 + n * STEP) * stride + own;
+        if (nvalid < F_TILE) s -= (int64_t)max(r - nvalid + 1, 0) * stride;
+      } else {
+        s = src + (int64_t)(row0 + min(r, nvalid - 1)) * stride + 8 * x;
+      }
       v[n][0] = *reinterpret_cast<const f32x4*>(s), v[n][1] = *reinterpret_cast<const f32x4*>(s + 4);
-      if (r >= nvalid) v[n][0] = v[n][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+      if (ZERO && r >= nvalid) v[n][0] = v[n][1] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
   }
   __device__ __forceinline__ void scale(float mul) {
 #pragma unroll
     for (int n = 0; n < N; n++) v[n][0] *= mul, v[n][1] *= mul;
   }
+  template <bool UP = true>   // times SPLIT_UP
   __device__ __forceinline__ void put(bf16* dst, int tid) const {   // in parts, [3][32][64], chunks permuted as attn_rowtile.h wants them
 #pragma unroll
     for (int n = 0; n < N; n++) {
       const int e = tid + n * NT, r = e / (D / 8), x = e % (D / 8);
-      const Split3<8> s(__builtin_shufflevector(v[n][0], v[n][1], 0, 1, 2, 3, 4, 5, 6, 7));
+      const Split3<8> s(__builtin_shufflevector(v[n][0], v[n][1], 0, 1, 2, 3, 4, 5, 6, 7) * (UP ? SPLIT_UP : 1.f));
 #pragma unroll
       for (int p = 0; p < 3; p++) *reinterpret_cast<bf16x8*>(dst + (PLANE * p + r) * D + 8 * (x ^ rowtile::swz<D>(r))) = s.p[p];
     }
   }
-  template <bool EXACT>
+  template <bool EXACT, bool UP = true>
   __device__ __forceinline__ void put_as(float* stage, int second, int tid) const {   // as the first or the second tile of a stage
     if constexpr (EXACT) put_f32(stage + second * (F_TILE * (D + 4)), tid);
-    else put(reinterpret_cast<bf16*>(stage) + second * PARTS_ELEMS, tid);
+    else put<UP>(reinterpret_cast<bf16*>(stage) + second * PARTS_ELEMS, tid);
   }
   __device__ __forceinline__ void put_f32(float* dst, int tid) const {
 #pragma unroll
@@ -93,7 +111,7 @@ struct PartTile {
   }
 };
 
-// The parts of a wavefront's 32 rows, times `mul`: lane (g, i) holds row i, k = 16 ks + 8 g .. + 7
+// The parts of a wavefront's 32 rows, times `mul` and SPLIT_UP: lane (g, i) holds row i, k = 16 ks + 8 g .. + 7
 __device__ __forceinline__ void load_parts(bf16x8 (&f)[KS][3], const float* base, int64_t stride, int row, bool ok, int g, float mul) {
 #pragma unroll
   for (int ks = 0; ks < KS; ks++) {
@@ -102,7 +120,7 @@ __device__ __forceinline__ void load_parts(bf16x8 (&f)[KS][3], const float* base
       const f32x4* s = reinterpret_cast<const f32x4*>(base + (int64_t)row * stride + 16 * ks + 8 * g);
       x = __builtin_shufflevector(s[0], s[1], 0, 1, 2, 3, 4, 5, 6, 7);
     }
-    const Split3<8> p(x * mul);
+    const Split3<8> p(x * (mul * SPLIT_UP));
 #pragma unroll
     for (int n = 0; n < 3; n++) f[ks][n] = p.p[n];
   }
@@ -209,6 +227,10 @@ __device__ __forceinline__ bool all_finite(const f32x16 (&x)[N]) {   // 0 times 
   return (z[0] + z[1]) + (z[2] + z[3]) == 0.f;
 }
 
+// A row whose scores may have left the range that the parts' products hold, 2^96, while their differences are small: NaN, which sends
+// the block to the fp32 instruction
+__device__ __forceinline__ float in_range(float lse) { return __builtin_fabsf(lse) > 0x1p90f && lse != INFINITY ? __builtin_nanf("") : lse; }
+
 // What the wavefronts exchange at the end, over the stages: a flag each, two rows of 64 values each, the groups' accumulators
 constexpr size_t EX_VALUES = 256, EX_ACC = EX_VALUES + 2 * WAVES * 64 * sizeof(float);
 __device__ __forceinline__ float* values(unsigned char* smem, int which, int wave) { return reinterpret_cast<float*>(smem + EX_VALUES) + (which * WAVES + wave) * 64; }
@@ -247,7 +269,7 @@ __device__ __forceinline__ void put_own(bf16* dst, const float* base, int64_t st
   PartTile<256> own;   // 32 rows by four wavefronts at a time
   for (int n = at.wave >> 2; n < RW; n += 2) {
     if (row0 + 32 * n < nrows) {
-      own.fetch(base, stride, row0 + 32 * n, min(32, nrows - row0 - 32 * n), at.tid & 255);
+      own.fetch<true>(base, stride, row0 + 32 * n, min(32, nrows - row0 - 32 * n), at.tid & 255);
       own.scale(mul);
       own.put(dst + n * PARTS_ELEMS, at.tid & 255);
     }
@@ -289,18 +311,19 @@ __global__ __launch_bounds__(64 * WAVES, 2) void attn_fwd_f32_parts_kernel(const
   rd.init(reinterpret_cast<bf16*>(at.stage), g, i);
 
   f32x16 o[DT];
-  float m, l;
+  float m, l, back = 1.f / SPLIT_UP;   // l is the row sum of P times 1 / back, o that of P V times 1 / back^2
   auto walk = [&](auto exact) {
     constexpr bool EXACT = decltype(exact)::value;
+    constexpr float DOWN = EXACT ? 1.f : SPLIT_DOWN, UP = EXACT ? 1.f : SPLIT_UP;   // of scores; of P
     bf16x8 qf[KS][3];
     float q32[EXACT ? D / 2 : 1];
     if constexpr (EXACT) f32tile::load_row_frag<D>(q32, qp, p.sq.l, qi, qi < p.Lq, g, p.scale_log2e);
-    else load_parts(qf, qp, p.sq.l, qi, qi < p.Lq, g, p.scale_log2e);   // scores come out in the log2 domain
+    else load_parts(qf, qp, p.sq.l, qi, qi < p.Lq, g, p.scale_log2e * SPLIT_UP);   // scores come out in the log2 domain
     rowtile::clear(o);
     m = -INFINITY, l = 0.f;
     PartTile<G::LOADERS> kr, vr;
-    auto fetch_k = [&](int t) { kr.fetch(kp, p.sk.l, t * F_TILE, min(F_TILE, p.Lk - t * F_TILE), at.gtid); };
-    auto fetch_v = [&](int t) { vr.fetch(vp, p.sv.l, t * F_TILE, min(F_TILE, p.Lk - t * F_TILE), at.gtid); };
+    auto fetch_k = [&](int t) { kr.template fetch<EXACT>(kp, p.sk.l, t * F_TILE, min(F_TILE, p.Lk - t * F_TILE), at.gtid); };
+    auto fetch_v = [&](int t) { vr.template fetch<EXACT>(vp, p.sv.l, t * F_TILE, min(F_TILE, p.Lk - t * F_TILE), at.gtid); };
     if (!EXACT && at.grp < ntiles) fetch_k(at.grp), fetch_v(at.grp);
 #pragma unroll 1
     for (int it = 0; it < iters; it++) {
@@ -308,7 +331,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void attn_fwd_f32_parts_kernel(const
       G::sync();
       if (t < ntiles) {
         if (EXACT) fetch_k(t), fetch_v(t);
-        kr.template put_as<EXACT>(at.stage, 0, at.gtid);
+        kr.template put_as<EXACT, false>(at.stage, 0, at.gtid);
         if (!G::ONE) vr.template put_as<EXACT>(at.stage, 1, at.gtid);
       }
       G::sync();
@@ -330,7 +353,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void attn_fwd_f32_parts_kernel(const
       float mx = s[0];
 #pragma unroll
       for (int r = 1; r < 16; r++) mx = fmaxf(mx, s[r]);
-      mx = half_swap_max(mx);
+      mx = half_swap_max(mx) * DOWN;
       if (__builtin_amdgcn_ballot_w64(mx > m) != 0) {
         const float m_new = fmaxf(m, mx), alpha = m_new == -INFINITY ? 1.f : ody_exp2(m - m_new);
         m = m_new;
@@ -342,7 +365,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void attn_fwd_f32_parts_kernel(const
       float sum = 0.f;
 #pragma unroll
       for (int r = 0; r < 16; r++) {
-        s[r] = ody_exp2(s[r] - m_use);
+        s[r] = ody_exp2(fmaf(s[r], DOWN, -m_use)) * UP;
         sum += s[r];
       }
       l += sum;
@@ -358,7 +381,9 @@ __global__ __launch_bounds__(64 * WAVES, 2) void attn_fwd_f32_parts_kernel(const
   };
   auto publish = [&]() {
     __syncthreads();   // everyone is done with the stages
-    put_flag(smem, !all_finite(o) || l * 0.f != 0.f, at.wave, at.lane);
+    // (a row that sees a key of the group's first tile, and no score that is more than minus infinity)
+    const bool lost = qi < p.Lq && at.grp * F_TILE <= lim && m == -INFINITY;
+    put_flag(smem, !all_finite(o) || l * 0.f != 0.f || lost, at.wave, at.lane);
     values(smem, 0, at.wave)[at.lane] = m;
     __syncthreads();
   };
@@ -366,6 +391,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void attn_fwd_f32_parts_kernel(const
   publish();
   if (any_flag(smem)) {
     __syncthreads();
+    back = 1.f;
     walk(std::true_type{});
     publish();
   }
@@ -391,8 +417,8 @@ __global__ __launch_bounds__(64 * WAVES, 2) void attn_fwd_f32_parts_kernel(const
   }
   l = half_swap_sum(l);
   if (qi < p.Lq) {
-    f32tile::store_rows<D>(static_cast<float*>(p.out) + b * p.so.b + h * p.so.h + (int64_t)qi * p.so.l, o, g, l > 0.f ? 1.f / l : 0.f, false);
-    if (g == 0) p.lse[((int64_t)b * p.Hq + h) * p.Lq + qi] = l > 0.f ? (top + __log2f(l)) * LN2 : -INFINITY;
+    f32tile::store_rows<D>(static_cast<float*>(p.out) + b * p.so.b + h * p.so.h + (int64_t)qi * p.so.l, o, g, l > 0.f ? back / l : 0.f, false);
+    if (g == 0) p.lse[((int64_t)b * p.Hq + h) * p.Lq + qi] = l > 0.f ? (top + __log2f(l * back)) * LN2 : -INFINITY;
   }
 }
 
@@ -414,7 +440,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void attn_bwd_dq_f32_parts_kernel(co
   const float* vp = static_cast<const float*>(p.v) + b * p.sv.b + hk * p.sv.h;
 
   const int64_t ri = ((int64_t)b * p.Hq + h) * p.Lq + qi;
-  const float lse = qi < p.Lq ? p.lse[ri] : -INFINITY, lse2 = lse * ODY_LOG2E;
+  const float lse = qi < p.Lq ? p.lse[ri] : -INFINITY;
   const float delta = qi < p.Lq ? p.delta[ri] : 0.f;
   // a query with no visible key (lse = -inf) contributes nothing
   const int lim = lse == -INFINITY ? -1 : (p.causal ? min(p.Lk - 1, qi + p.off) : p.Lk - 1);
@@ -440,8 +466,11 @@ __global__ __launch_bounds__(64 * WAVES, 2) void attn_bwd_dq_f32_parts_kernel(co
     __syncthreads();
   }
   f32x16 dq[DT];
+  float back = SPLIT_DOWN;
   auto walk = [&](auto exact) {
     constexpr bool EXACT = decltype(exact)::value;
+    constexpr float DOWN = EXACT ? 1.f : SPLIT_DOWN;
+    const float ds_scale = EXACT ? p.scale : p.scale * SPLIT_UP, lse2 = (EXACT ? lse : in_range(lse)) * ODY_LOG2E;
     bf16x8 qf[KS][3], dof[G::ONE ? 1 : KS][3];
     float q32[EXACT ? D / 2 : 1], do32[EXACT ? D / 2 : 1];
     if constexpr (EXACT) {
@@ -453,8 +482,8 @@ __global__ __launch_bounds__(64 * WAVES, 2) void attn_bwd_dq_f32_parts_kernel(co
     }
     rowtile::clear(dq);
     PartTile<G::LOADERS> kr, vr;
-    auto fetch_k = [&](int t) { kr.fetch(kp, p.sk.l, t * F_TILE, min(F_TILE, p.Lk - t * F_TILE), at.gtid); };
-    auto fetch_v = [&](int t) { vr.fetch(vp, p.sv.l, t * F_TILE, min(F_TILE, p.Lk - t * F_TILE), at.gtid); };
+    auto fetch_k = [&](int t) { kr.template fetch<EXACT>(kp, p.sk.l, t * F_TILE, min(F_TILE, p.Lk - t * F_TILE), at.gtid); };
+    auto fetch_v = [&](int t) { vr.template fetch<EXACT>(vp, p.sv.l, t * F_TILE, min(F_TILE, p.Lk - t * F_TILE), at.gtid); };
     if (!EXACT && at.grp < ntiles) fetch_k(at.grp), fetch_v(at.grp);
 #pragma unroll 1
     for (int it = 0; it < iters; it++) {
@@ -492,8 +521,8 @@ __global__ __launch_bounds__(64 * WAVES, 2) void attn_bwd_dq_f32_parts_kernel(co
       }
 #pragma unroll
       for (int r = 0; r < 16; r++) {
-        const float pr = n0 + acc_row(r, g) > lim ? 0.f : ody_exp2(s[r] - lse2);
-        s[r] = pr * (dp[r] - delta) * p.scale;   // dS^T
+        const float pr = n0 + acc_row(r, g) > lim ? 0.f : ody_exp2(fmaf(s[r], DOWN, -lse2));
+        s[r] = pr * fmaf(dp[r], DOWN, -delta) * ds_scale;   // dS^T
       }
       if constexpr (EXACT) f32tile::tile_t_times_regs<D>(at.stage, i, g, s, dq);
       else tile_t_times<0, RW == 4>(rd, s, dq);   // dQ^T += K^T dS^T
@@ -509,6 +538,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void attn_bwd_dq_f32_parts_kernel(co
   publish();
   if (any_flag(smem)) {
     __syncthreads();
+    back = 1.f;
     walk(std::true_type{});
     publish();
   }
@@ -516,7 +546,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void attn_bwd_dq_f32_parts_kernel(co
 #pragma unroll 1
   for (int n = 1; n < G::GROUPS; n++) rowtile::take(acc_room<RW, DT>(smem, n, at.w), dq, at.lane, 1.f, 1.f);
   if (qi < p.Lq)
-    f32tile::store_rows<D>(static_cast<float*>(p.dq) + b * p.sdq.b + h * p.sdq.h + (int64_t)qi * p.sdq.l, dq, g, 1.f, p.accumulate_dq != 0);
+    f32tile::store_rows<D>(static_cast<float*>(p.dq) + b * p.sdq.b + h * p.sdq.h + (int64_t)qi * p.sdq.l, dq, g, back, p.accumulate_dq != 0);
 }
 
 // ---------------------------------------------------------------------------------------------------------- dK / dV
@@ -526,6 +556,7 @@ template <int RW>
 __global__ __launch_bounds__(64 * WAVES, 2) void attn_bwd_dkdv_f32_parts_kernel(const AttnParams p) {
   using G = Geo<RW>;
   constexpr bool K_IN_LDS = RW != 4;
+  constexpr int K_AT = 3 * PLANE * RW;
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
   const Place<RW> at(smem);
   const int g = at.g, i = at.i;
@@ -546,16 +577,15 @@ __global__ __launch_bounds__(64 * WAVES, 2) void attn_bwd_dkdv_f32_parts_kernel(
   rd.init(reinterpret_cast<bf16*>(at.stage), g, i);
 
   put_own<RW>(vs, vp, p.sv.l, n0, p.Lk, 1.f, at);
-  Readers<D> vrd, krd;
+  Readers<D> vrd;   // K's parts lie K_AT rows behind V's
   vrd.init(vs + at.w * PARTS_ELEMS, g, i);
-  if constexpr (K_IN_LDS) {   // K's beside them
-    put_own<RW>(vs + RW * PARTS_ELEMS, kp, p.sk.l, n0, p.Lk, p.scale_log2e, at);
-    krd.init(vs + (RW + at.w) * PARTS_ELEMS, g, i);
-  }
+  if constexpr (K_IN_LDS) put_own<RW>(vs + K_AT * D, kp, p.sk.l, n0, p.Lk, p.scale_log2e, at);
   __syncthreads();
   f32x16 dk[DT], dv[DT];
+  float back = SPLIT_DOWN;
   auto walk = [&](auto exact) {
     constexpr bool EXACT = decltype(exact)::value;
+    constexpr float DOWN = EXACT ? 1.f : SPLIT_DOWN, UP = EXACT ? 1.f : SPLIT_UP;   // of scores and dP; of P, and with it dS
     bf16x8 kf[K_IN_LDS ? 1 : KS][3];
     float k32[EXACT ? D / 2 : 1], v32[EXACT ? D / 2 : 1];
     if constexpr (EXACT) {
@@ -570,15 +600,15 @@ __global__ __launch_bounds__(64 * WAVES, 2) void attn_bwd_dkdv_f32_parts_kernel(
     float row = 0.f;   // threads 0 .. 31 of the group carry lse, 32 .. 63 delta of the next tile
     auto fetch_q = [&](int n) {
       const int h = hk * p.group + n / ntq, i0 = i_begin + n % ntq * F_TILE, valid = min(F_TILE, p.Lq - i0);
-      qr.fetch(static_cast<const float*>(p.q) + b * p.sq.b + h * p.sq.h, p.sq.l, i0, valid, at.gtid);
+      qr.template fetch<EXACT, G::ONE>(static_cast<const float*>(p.q) + b * p.sq.b + h * p.sq.h, p.sq.l, i0, valid, at.gtid);
     };
     auto fetch_do = [&](int n) {
       const int h = hk * p.group + n / ntq, i0 = i_begin + n % ntq * F_TILE, valid = min(F_TILE, p.Lq - i0);
-      dor.fetch(static_cast<const float*>(p.dout) + b * p.sdo.b + h * p.sdo.h, p.sdo.l, i0, valid, at.gtid);
+      dor.template fetch<EXACT, G::ONE>(static_cast<const float*>(p.dout) + b * p.sdo.b + h * p.sdo.h, p.sdo.l, i0, valid, at.gtid);
       if (at.w == 0) {
         const int64_t r = ((int64_t)b * p.Hq + h) * p.Lq + i0 + min(i, valid - 1);
         const float x = g ? p.delta[r] : p.lse[r];
-        row = g ? (i < valid ? x : 0.f) : (i < valid && x != -INFINITY ? x * ODY_LOG2E : INFINITY);
+        row = g ? (i < valid ? x : 0.f) : (i < valid && x != -INFINITY ? (EXACT ? x : in_range(x)) * ODY_LOG2E : INFINITY);
       }
     };
     if (!EXACT && at.grp < turns) fetch_q(at.grp), fetch_do(at.grp);
@@ -588,7 +618,8 @@ __global__ __launch_bounds__(64 * WAVES, 2) void attn_bwd_dkdv_f32_parts_kernel(
       G::sync();
       if (n < turns) {
         if (EXACT) fetch_q(n), fetch_do(n);
-        qr.template put_as<EXACT>(at.stage, 0, at.gtid);
+        if (!EXACT && G::ONE) qr.scale(SPLIT_UP);   // once for both times
+        qr.template put_as<EXACT, !G::ONE>(at.stage, 0, at.gtid);
         if (!G::ONE) dor.template put_as<EXACT>(at.stage, 1, at.gtid);
         if (at.w == 0) rows[at.lane] = row;
       }
@@ -604,7 +635,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void attn_bwd_dkdv_f32_parts_kernel(
         for (int a = 0; a < 4; a++) {
           const f32x4 lv = *reinterpret_cast<const f32x4*>(rows + 8 * a + 4 * g);
 #pragma unroll
-          for (int e = 0; e < 4; e++) s[4 * a + e] = acc_row(4 * a + e, g) < vis ? 0.f : ody_exp2(s[4 * a + e] - lv[e]);
+          for (int e = 0; e < 4; e++) s[4 * a + e] = acc_row(4 * a + e, g) < vis ? 0.f : ody_exp2(fmaf(s[4 * a + e], DOWN, -lv[e])) * UP;
         }
       };
       auto gradients = [&]() {   // dS
@@ -612,14 +643,14 @@ __global__ __launch_bounds__(64 * WAVES, 2) void attn_bwd_dkdv_f32_parts_kernel(
         for (int a = 0; a < 4; a++) {
           const f32x4 dl = *reinterpret_cast<const f32x4*>(rows + F_TILE + 8 * a + 4 * g);
 #pragma unroll
-          for (int e = 0; e < 4; e++) dp[4 * a + e] = s[4 * a + e] * (dp[4 * a + e] - dl[e]) * p.scale;
+          for (int e = 0; e < 4; e++) dp[4 * a + e] = s[4 * a + e] * fmaf(dp[4 * a + e], DOWN, -dl[e]) * p.scale;
         }
       };
       if constexpr (G::ONE) {   // Q, dO, and Q again through the one stage
         if (n >= turns) break;
         f32x16 more = {0.f};
         if constexpr (EXACT) f32tile::tile_times_frag<D>(at.stage, i, g, k32, s, more);
-        else tile_times_parts<0>(rd, [&](int ks, int m) { return row_frag(krd, PLANE * m, ks); }, s, more);
+        else tile_times_parts<0>(rd, [&](int ks, int m) { return row_frag(vrd, K_AT + PLANE * m, ks); }, s, more);
         s += more;
         exponentials();
         G::sync();
@@ -634,14 +665,14 @@ __global__ __launch_bounds__(64 * WAVES, 2) void attn_bwd_dkdv_f32_parts_kernel(
         if constexpr (EXACT) f32tile::tile_t_times_regs<D>(at.stage, i, g, s, dv);
         else tile_t_times<0, false>(rd, s, dv);
         G::sync();
-        qr.template put_as<EXACT>(at.stage, 0, at.gtid);
+        qr.template put_as<EXACT, false>(at.stage, 0, at.gtid);
         G::sync();
         if (!EXACT && next < turns) fetch_q(next);
         if constexpr (EXACT) f32tile::tile_t_times_regs<D>(at.stage, i, g, dp, dk);
         else tile_t_times<0, false>(rd, dp, dk);
       } else {
         if constexpr (EXACT) f32tile::tiles_times_frags<D>(at.stage, k32, s, at.stage + F_TILE * (D + 4), v32, dp, i, g);
-        else tiles_times_parts<0, G::SECOND>(rd, [&](int ks, int m) { return K_IN_LDS ? row_frag(krd, PLANE * m, ks) : kf[K_IN_LDS ? 0 : ks][m]; }, s, [&](int ks, int m) { return row_frag(vrd, PLANE * m, ks); }, dp);
+        else tiles_times_parts<0, G::SECOND>(rd, [&](int ks, int m) { return K_IN_LDS ? row_frag(vrd, K_AT + PLANE * m, ks) : kf[K_IN_LDS ? 0 : ks][m]; }, s, [&](int ks, int m) { return row_frag(vrd, PLANE * m, ks); }, dp);
         exponentials();
         gradients();
         if constexpr (EXACT) {
@@ -668,6 +699,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void attn_bwd_dkdv_f32_parts_kernel(
   publish();
   if (any_flag(smem)) {   // (it does not read the own rows in LDS, which the accumulators went over)
     __syncthreads();
+    back = 1.f;
     walk(std::true_type{});
     publish();
   }
@@ -679,8 +711,8 @@ __global__ __launch_bounds__(64 * WAVES, 2) void attn_bwd_dkdv_f32_parts_kernel(
     rowtile::take(room + 16 * DT * 64, dv, at.lane, 1.f, 1.f);
   }
   if (ki >= p.Lk) return;
-  f32tile::store_rows<D>(static_cast<float*>(p.dk) + b * p.sdk.b + hk * p.sdk.h + (int64_t)ki * p.sdk.l, dk, g, 1.f, false);
-  f32tile::store_rows<D>(static_cast<float*>(p.dv) + b * p.sdv.b + hk * p.sdv.h + (int64_t)ki * p.sdv.l, dv, g, 1.f, false);
+  f32tile::store_rows<D>(static_cast<float*>(p.dk) + b * p.sdk.b + hk * p.sdk.h + (int64_t)ki * p.sdk.l, dk, g, back, false);
+  f32tile::store_rows<D>(static_cast<float*>(p.dv) + b * p.sdv.b + hk * p.sdv.h + (int64_t)ki * p.sdv.l, dv, g, back, false);
 }
 
 template <int RW>

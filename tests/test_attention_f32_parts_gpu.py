@@ -1,4 +1,6 @@
 """GPU parity: fp32 attention of head_dim 64 in three bf16 parts per value (attn_f32_parts.hip) against the CPU oracle."""
+import math
+
 import pytest
 import torch
 
@@ -11,6 +13,8 @@ pytestmark = pytest.mark.gpu
 # either sign; shapes that take each kind of block
 CASES = [(1, 33, 257, 2, 2, True), (1, 65, 289, 4, 1, False), (1, 300, 300, 8, 2, True), (1, 129, 65, 4, 4, True), (1, 1, 300, 2, 1, True),
          (4, 484, 484, 16, 16, True), (2, 300, 301, 16, 4, False), (2, 1025, 1025, 16, 16, True), (1, 1500, 700, 32, 8, False), (2, 1100, 260, 16, 16, True)]
+
+SHAPES = pytest.mark.parametrize("shape", [(1, 300, 320, 2), (4, 484, 484, 16), (2, 300, 301, 16)], ids=lambda s: "B%d_Lq%d_Lk%d_H%d" % s)
 
 
 def _inputs(B, Lq, Lk, Hq, Hkv, seed):
@@ -41,7 +45,7 @@ def test_fp32_attention_in_parts(case):
     assert_parity((acc - acc0).cpu(), grads[0], TOL_F32, "dq added to a buffer")
 
 
-@pytest.mark.parametrize("shape", [(1, 300, 320, 2), (4, 484, 484, 16), (2, 300, 301, 16)], ids=lambda s: "B%d_Lq%d_Lk%d_H%d" % s)
+@SHAPES
 def test_fp32_attention_beyond_the_range_of_the_parts(shape):
     """Values that bf16 rounds to infinity, and infinities: as the fp32 instruction gives them."""
     from odysseus_transformer_amd import ops
@@ -67,3 +71,72 @@ def test_fp32_attention_beyond_the_range_of_the_parts(shape):
     p = torch.softmax(torch.matmul(q.transpose(1, 2), k.permute(0, 2, 3, 1)) / 8, -1)
     dv_ref = torch.matmul(p.transpose(2, 3), do.transpose(1, 2)).transpose(1, 2)
     assert dv_ref.isfinite().all() and torch.allclose(dv, dv_ref, rtol=TOL_F32, atol=TOL_F32)
+
+
+def _attention64(q, k, v, do, scale, causal=False):
+    """out, dq, dk, dv in 64 bits"""
+    q, k, v, do = (t.double().transpose(1, 2) for t in (q, k, v, do))
+    s = (q @ k.transpose(2, 3)) * scale
+    if causal:
+        s = s.masked_fill(~torch.ones(s.shape[-2:], dtype=torch.bool).tril(s.shape[-1] - s.shape[-2]), float("-inf"))
+    p = s.softmax(-1)
+    o = p @ v
+    ds = p * (do @ v.transpose(2, 3) - (do * o).sum(-1, keepdim=True)) * scale
+    return [t.transpose(1, 2) for t in (o, ds @ k, ds.transpose(2, 3) @ q, p.transpose(2, 3) @ do)]
+
+
+@SHAPES
+@pytest.mark.parametrize("exps,what", [((0, 0, -122, 0), "out dv"), ((0, 0, -112, 0), "dq dk"), ((0, 0, 0, -122), "out dv"), ((0, 0, 0, -112), "dq dk"),
+                                       ((-115, 90, 0, 0), "out dq dk dv"), ((90, -115, 0, 0), "out dq dk dv"), ((0, 0, 60, 50), "out dv"),
+                                       ((0, 0, 114, 0), "out dv"), ((114, -114, 0, 0), "out dq dk dv")], ids=str)
+def test_fp32_attention_of_operands_of_any_size(shape, exps, what):
+    """q, k, v and dout times 2^exps: every operand as exact as fp32 holds it, where the results and what lies between are no denormals."""
+    from odysseus_transformer_amd import ops
+    B, Lq, Lk, H = shape
+    ins = [t * 2.0 ** e for t, e in zip(_inputs(B, Lq, Lk, H, H, 3), exps)]
+    scale = 2.0 ** -(exps[0] + exps[1]) / 8
+    ref = dict(zip(("out", "dq", "dk", "dv"), _attention64(*ins, scale)))
+    q, k, v, do = (t.cuda() for t in ins)
+    o, lse = ops.attn_fwd(q, k, v, causal=False, scale=scale)
+    got = dict(zip(("out", "dq", "dk", "dv"), (o, *ops.attn_bwd(q, k, v, o, lse, do, causal=False, scale=scale))))
+    for n in what.split():
+        err = ((got[n].cpu().double() - ref[n]).norm() / ref[n].norm()).item()
+        print(n, err)
+        assert err <= 2e-6, (n, err)
+
+
+@SHAPES
+def test_fp32_attention_of_a_key_that_nobody_attends_to(shape):
+    """Probabilities near 2^-119 (a score of -76 under a log-sum-exp of 6): the gradients of such a key are as exact as the scores (half a unit of 2^-17 in 120)."""
+    from odysseus_transformer_amd import ops
+    B, Lq, Lk, H = shape
+    q, k, v, do = _inputs(B, Lq, Lk, H, H, 13)
+    q[..., 0], k[..., 0] = 8.0, 0.0
+    k[:, 5, :, 0] = -76.0
+    _, _, dk_ref, dv_ref = _attention64(q, k, v, do, 0.125)
+    assert 0 < dv_ref[:, 5].abs().max() < 2.0 ** -100
+    qg, kg, vg, dog = (t.cuda() for t in (q, k, v, do))
+    o, lse = ops.attn_fwd(qg, kg, vg, causal=False)
+    _, dk, dv = ops.attn_bwd(qg, kg, vg, o, lse, dog, causal=False)
+    for a, b in ((dk, dk_ref), (dv, dv_ref)):
+        err = ((a.cpu().double() - b)[:, 5].norm() / b[:, 5].norm()).item()
+        print(err)
+        assert err <= 1e-5
+
+
+@SHAPES
+def test_fp32_attention_of_scores_beyond_what_the_parts_hold(shape):
+    """All scores of a row near -2^100, their differences multiples of the spacing there: the largest ones share the row."""
+    from odysseus_transformer_amd import ops
+    B, Lq, Lk, H = shape
+    q, k, v, do = _inputs(B, Lq, Lk, H, H, 17)
+    q.zero_(), k.zero_()
+    q[..., 0], k[..., 0] = 2.0 ** 50, -(2.0 ** 50) * torch.randint(1, 3, k.shape[:3]).float()
+    q[:, 7:9] *= -1.0      # and rows near 2^100
+    scale = math.log(2.0)      # scores are whole numbers of the exponent's base, exact in fp32
+    qg, kg, vg, dog = (t.cuda() for t in (q, k, v, do))
+    o, lse = ops.attn_fwd(qg, kg, vg, causal=False, scale=scale)
+    ref = _attention64(q, k, v, do, scale)
+    _, _, dv = ops.attn_bwd(qg, kg, vg, o, lse, dog, causal=False, scale=scale)
+    assert (o.cpu().double() - ref[0]).norm() <= 1e-5 * ref[0].norm()
+    assert dv.isfinite().all() and o.isfinite().all()
