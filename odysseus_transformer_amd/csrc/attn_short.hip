@@ -430,6 +430,7 @@ inline int64_t row_blocks(int B, int L, int H) { return (int64_t)B * H * ((L + B
 //   Beyond the line in tiles the other kernels cut the range of the long side into parts: 4 heads, causal, L = 3001: forward 43 / 51;
 //   8 heads, full, L = 3001: backward 181 / 230.  Forwards of 64 blocks and less stay there wherever it has parts: some are faster here
 //   (4 heads, L = 1000: 29 / 22), some are not (32 heads, 109 queries on 2042 keys: 1.13 times slower).
+// One head, too, below the line: backward of 512 rows, causal, 65 us there, 29 here, of 1024 rows 101 / 45; two heads of 512 rows 66 / 29.
 bool ody_attn_fwd_short_ok(int B, int Lq, int Lk, int Hq, int causal) {
   const int64_t blocks = row_blocks(B, Lq, Hq);
   if (blocks <= 64 && ody_attn_fwd_w8_parts(B, Lq, Lk, Hq, causal) > 1) return false;
@@ -437,9 +438,6 @@ bool ody_attn_fwd_short_ok(int B, int Lq, int Lk, int Hq, int causal) {
 }
 bool ody_attn_bwd_short_ok(int B, int Lq, int Lk, int Hq, int causal) {
   const int64_t blocks = row_blocks(B, Lq, Hq) + row_blocks(B, Lk, Hq);
-  // one or two heads from 512 rows on: the smallest calls for which a caller chooses between kept and recomputed dS, and finds the
-  // kernels of that choice in the profile
-  if (blocks <= 16 && std::min(Lq, Lk) >= 512) return false;
   return blocks <= (causal ? 1024 : 512) && std::max(Lq, Lk) <= ROWS * (causal && blocks > 128 ? 56 : 32);
 }
 

@@ -90,3 +90,20 @@ def test_query_side_of_few_blocks_serves_the_other_kernels():
     reused, ran = _run(lambda: ops.attn_bwd(q, v, k, o, lse, do, causal=False, workspace=ws, reuse_query_side=True))
     assert "attn_bwd_dq_pipe" in ran and "attn_bwd_prepass" not in ran, ran
     assert all(torch.equal(a, b) for a, b in zip(reused, ops.attn_bwd(q, v, k, o, lse, do, causal=False)))
+
+
+@pytest.mark.parametrize("case", [(1, 512, 512, 1, 1, True), (1, 512, 512, 2, 2, True), (1, 1024, 768, 1, 1, False)], ids=lambda c: "Lq%d_Lk%d_H%d_c%d" % (*c[1:4], c[5]))
+def test_backward_of_one_or_two_heads(case):
+    """The fewest blocks there are: on these kernels, and dK and dV the bits of a call that keeps dS."""
+    from odysseus_transformer_amd import ops
+    B, Lq, Lk, Hq, Hkv, causal = case
+    print(f"case={case}", flush=True)
+    q, k, v, do = (t.cuda() for t in _inputs(B, Lq, Lk, Hq, Hkv, 23))
+    o, lse = ops.attn_fwd(q, k, v, causal=causal)
+    got, ran = _run(lambda: ops.attn_bwd(q, k, v, o, lse, do, causal=causal))
+    assert "attn_bwd_short" in ran, ran
+    kept, ran = _run(lambda: ops.attn_bwd(q, k, v, o, lse, do, causal=causal, keep_ds=True))
+    assert "attn_bwd_dq_kept" in ran and torch.equal(got[1], kept[1]) and torch.equal(got[2], kept[2])
+    o_ref, lse_ref = oracle.attention_fwd(*(t.cpu().float() for t in (q, k, v)), causal=causal)
+    for a, b, n in zip(got, oracle.attention_bwd(*(t.cpu().float() for t in (q, k, v)), o_ref, lse_ref, do.cpu().float(), causal=causal), ("dq", "dk", "dv")):
+        assert_parity(a, b, TOL_BF16, n, 1e-3)
