@@ -761,21 +761,21 @@ int rows_of_block(const AttnParams& p, bool own_keys, const Cost (&cost)[3]) {
 int ody_launch_attn_fwd_f32_parts(const AttnParams& p, hipStream_t st) {
   static const Cost cost[3] = {{1, 3.95, 3.2}, {1.5, 3.32, 3.3}, {3, 2.73, -1.1}};
   const int rows = rows_of_block(p, false, cost);
-  if (rows == 32) return launch<1>("attn_fwd_f32_split", &attn_fwd_f32_parts_kernel<1>, p.Lq, p.Hq * p.B, 0, p, st);
-  if (rows == 64) return launch<2>("attn_fwd_f32_split", &attn_fwd_f32_parts_kernel<2>, p.Lq, p.Hq * p.B, 0, p, st);
-  return launch<4>("attn_fwd_f32", &attn_fwd_f32_parts_kernel<4>, p.Lq, p.Hq * p.B, 0, p, st);
+  if (rows == 32) return launch<1>("attn_fwd_f32_parts32", &attn_fwd_f32_parts_kernel<1>, p.Lq, p.Hq * p.B, 0, p, st);
+  if (rows == 64) return launch<2>("attn_fwd_f32_parts64", &attn_fwd_f32_parts_kernel<2>, p.Lq, p.Hq * p.B, 0, p, st);
+  return launch<4>("attn_fwd_f32_parts128", &attn_fwd_f32_parts_kernel<4>, p.Lq, p.Hq * p.B, 0, p, st);
 }
 int ody_launch_attn_bwd_dq_f32_parts(const AttnParams& p, hipStream_t st) {
   static const Cost cost[3] = {{1, 4.78, 2.4}, {1.5, 4.2, 2.5}, {3, 3.61, -3.2}};
   const int rows = rows_of_block(p, false, cost);
-  if (rows == 32) return launch<1>("attn_bwd_dq_f32_split", &attn_bwd_dq_f32_parts_kernel<1>, p.Lq, p.Hq * p.B, Geo<1>::OWN, p, st);
-  if (rows == 64) return launch<2>("attn_bwd_dq_f32_split", &attn_bwd_dq_f32_parts_kernel<2>, p.Lq, p.Hq * p.B, 0, p, st);
-  return launch<4>("attn_bwd_dq_f32", &attn_bwd_dq_f32_parts_kernel<4>, p.Lq, p.Hq * p.B, 0, p, st);
+  if (rows == 32) return launch<1>("attn_bwd_dq_f32_parts32", &attn_bwd_dq_f32_parts_kernel<1>, p.Lq, p.Hq * p.B, Geo<1>::OWN, p, st);
+  if (rows == 64) return launch<2>("attn_bwd_dq_f32_parts64", &attn_bwd_dq_f32_parts_kernel<2>, p.Lq, p.Hq * p.B, 0, p, st);
+  return launch<4>("attn_bwd_dq_f32_parts128", &attn_bwd_dq_f32_parts_kernel<4>, p.Lq, p.Hq * p.B, 0, p, st);
 }
 int ody_launch_attn_bwd_dkdv_f32_parts(const AttnParams& p, hipStream_t st) {
   static const Cost cost[3] = {{1, 6.34, 1.4}, {2, 5.06, -0.6}, {4, 4.58, -9.1}};
   const int rows = rows_of_block(p, true, cost);
-  if (rows == 32) return launch<1>("attn_bwd_dkdv_f32_split", &attn_bwd_dkdv_f32_parts_kernel<1>, p.Lk, p.Hkv * p.B, dkdv_more<1>(), p, st);
-  if (rows == 64) return launch<2>("attn_bwd_dkdv_f32_split", &attn_bwd_dkdv_f32_parts_kernel<2>, p.Lk, p.Hkv * p.B, dkdv_more<2>(), p, st);
-  return launch<4>("attn_bwd_dkdv_f32", &attn_bwd_dkdv_f32_parts_kernel<4>, p.Lk, p.Hkv * p.B, dkdv_more<4>(), p, st);
+  if (rows == 32) return launch<1>("attn_bwd_dkdv_f32_parts32", &attn_bwd_dkdv_f32_parts_kernel<1>, p.Lk, p.Hkv * p.B, dkdv_more<1>(), p, st);
+  if (rows == 64) return launch<2>("attn_bwd_dkdv_f32_parts64", &attn_bwd_dkdv_f32_parts_kernel<2>, p.Lk, p.Hkv * p.B, dkdv_more<2>(), p, st);
+  return launch<4>("attn_bwd_dkdv_f32_parts128", &attn_bwd_dkdv_f32_parts_kernel<4>, p.Lk, p.Hkv * p.B, dkdv_more<4>(), p, st);
 }
