@@ -241,8 +241,9 @@ def test_tiles_of_a_nearly_empty_last_round(what, M, dev):
     M = (M + 7) // 8 * 8 if what == "tn" else M
     x, w = randn((M, K), 1, dtype=dt).to(dev), randn((N, K), 2, std=0.05, dtype=dt).to(dev)
     r = randn((M, N), 3, dtype=dt).to(dev)
+    table = ops.rope_table(torch.arange(M, device=dev), M, 128)
 
-    def run(x, r):
+    def run(x, r, table):
         if what == "nt":
             return ops.gemm(ops.GEMM_NT, x, w)
         if what == "nn":
@@ -250,16 +251,18 @@ def test_tiles_of_a_nearly_empty_last_round(what, M, dev):
         if what == "tn":
             return ops.gemm(ops.GEMM_TN, x.t().contiguous(), w.t().contiguous())
         if what == "rope":
-            return ops.linear_rope(x, w, ops.rope_table(torch.arange(x.shape[0], device=dev), x.shape[0], 128), 20, 128)
+            return ops.linear_rope(x, w, table, 20, 128)
         if what == "swiglu":
             return ops.linear_swiglu(x, w)[1]
         return ops.linear_residual(x, w, r)
 
-    y = run(x, r)
-    assert torch.equal(y[:4096], run(x[:4096], r[:4096]))
+    y = run(x, r, table)
+    assert torch.equal(y[:4096], run(x[:4096], r[:4096], table[:4096]))
     ref = x.float() @ w.float().t()
-    if what == "rope":
-        return   # the rows beyond the first round: one more call on them alone, with their own positions, is another table
+    if what == "rope":   # (cos, sin) of a frequency side by side in the table, columns j and j + 64 of a head in the product
+        cos, sin = table.float().view(M, 1, 64, 2).unbind(-1)
+        a, b = ref[:, :20 * 128].reshape(M, 20, 2, 64).unbind(2)
+        ref[:, :20 * 128] = torch.stack([a * cos - b * sin, b * cos + a * sin], 2).reshape(M, -1)
     if what == "swiglu":
         g, u = ref.chunk(2, -1)
         ref = torch.nn.functional.silu(g.to(dt).float()) * u.to(dt).float()
