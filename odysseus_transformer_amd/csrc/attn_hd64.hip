@@ -26,6 +26,7 @@
 // Error of the forward against 64 bits, standard normal inputs (running maximum / first tile's): 16 heads, L = 4096, causal 2.05e-3 /
 // 2.11e-3; L = 700, full 2.21e-3 / 2.31e-3.  The roundings are the same ones; bf16 is finest just below a power of two, and that is
 // where the largest P of a row lie if the reference is its maximum (an emulation in 64 bits that rounds P and out gives these figures).
+#include <cfloat>
 #include <type_traits>
 #include <utility>
 #include "attn_rowtile.h"
@@ -94,7 +95,7 @@ __global__ __launch_bounds__(256 * GROUPS, 4) void attn_fwd_hd64_kernel(const At
   auto walk = [&](auto online) {
     constexpr bool ONLINE = decltype(online)::value;
     clear(o);
-    ref = -1e30f;   // below any score until a key was seen
+    ref = -FLT_MAX;   // no score is below it; not minus infinity, from which a masked score would be NaN
 #pragma unroll
     for (int e = 0; e < 4; e++) l4[e] = 0.f;
     Readers<D> rd;

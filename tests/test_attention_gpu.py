@@ -706,3 +706,18 @@ def test_attention_fp32_takes_the_instance_that_was_faster(D, heads, Lq, Lk, cau
     for kernel in ("attn_fwd_f32", "attn_bwd_dq_f32"):
         shared, whole = ({kernel + "_split"}, {kernel}) if D == 128 else ({kernel + "_parts32", kernel + "_parts64"}, {kernel + "_parts128"})
         assert bool(shared & names) == split and bool(whole & names) != split, names
+
+
+@pytest.mark.parametrize("causal", [False, True], ids=["full", "causal"])
+@pytest.mark.parametrize("D,L,H", [(64, 300, 4), (64, 2100, 16), (128, 300, 4), (128, 700, 8), (128, 1500, 16)])
+def test_attention_of_scores_below_any_usual_one(D, L, H, causal, dev):
+    """Every score of a row the same, near -2^120: the softmax of equal scores, whatever their size."""
+    from odysseus_transformer_amd import ops
+    print(f"D={D} L={L} H={H} causal={causal}", flush=True)
+    q = torch.zeros(1, L, H, D, dtype=torch.bfloat16, device=dev)
+    k, v = q.clone(), randn((1, L, H, D), 5, dtype=torch.bfloat16).to(dev)
+    q[..., 0], k[..., 0] = 2.0 ** 60, -(2.0 ** 60)
+    o, lse = ops.attn_fwd(q, k, v, causal=causal, scale=0.5)
+    ref = v.float().cumsum(1) / torch.arange(1, L + 1, device=dev)[None, :, None, None] if causal else v.float().mean(1, keepdim=True).expand(v.shape)
+    assert (lse == -(2.0 ** 119)).all()
+    assert_parity(o, ref, TOL_BF16, "o")
