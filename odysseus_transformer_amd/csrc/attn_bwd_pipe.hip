@@ -273,7 +273,7 @@ __host__ __device__ inline int64_t ds_block_index(int nbq, int kb, int qb, bool 
 // floats (4 broadcast reads of 16 bytes per product).  The query-side pre-pass (attn_bwd_prepass_kernel) writes them:
 // per (batch, head, tile) a table [sub-tile mt][0: -lse/scale, 1: -delta][lane group g][register r] of fp32 at the
 // start of a 1 KB record, register r of group g being query acc_tile_row(r, g, mt).  Rows that must give P = 0
-// (beyond Lq, or a query that saw no key) hold -1e30.
+// (beyond Lq, or a query that saw no key) hold minus infinity.
 //
 // SPLIT = false: a block owns 256 keys of one kv head and walks all query heads of its group.
 // SPLIT = true (grouped-query attention, or too few key blocks for the chip): a block owns 256 keys for ONE query

@@ -268,11 +268,11 @@ __global__ __launch_bounds__(256 * GROUPS, GROUPS == 1 ? 3 : 2) void attn_bwd_hd
       __builtin_amdgcn_global_load_lds((global_ptr)src, (lds_ptr)(st + 2 * TILE + 2 * ROWS), 4, 0, 0);
     }
   };
-  // -1e30 for rows that must give P = 0: past the end, or a query that saw no key
+  // minus infinity for rows that must give P = 0: past the end, or a query that saw no key
   auto put_lse = [&](int buf) {
     if (w4 != 0) return;
     const bool none = l_next == INFINITY || l_next == -INFINITY;
-    reinterpret_cast<float*>(ring + buf * QS_STAGE + 2 * TILE)[lane] = none ? -1e30f : -l_next / p.scale;
+    reinterpret_cast<float*>(ring + buf * QS_STAGE + 2 * TILE)[lane] = none ? -INFINITY : -l_next / p.scale;
   };
   if (grp < total) load(grp, 0);
   put_lse(0);

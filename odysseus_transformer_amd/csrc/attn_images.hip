@@ -107,7 +107,7 @@ __global__ __launch_bounds__(256) void attn_bwd_prepass_kernel(const AttnParams 
     float x;
     if (which == 0) {
       const float l = (qi < p.Lq) ? p.lse[((int64_t)b * p.Hq + h) * p.Lq + qi] : INFINITY;
-      x = (l == INFINITY || l == -INFINITY) ? -1e30f : -l / p.scale;
+      x = (l == INFINITY || l == -INFINITY) ? -INFINITY : -l / p.scale;
     } else {
       x = (qi < p.Lq) ? -sdelta[row] : 0.f;
     }

@@ -721,3 +721,25 @@ def test_attention_of_scores_below_any_usual_one(D, L, H, causal, dev):
     ref = v.float().cumsum(1) / torch.arange(1, L + 1, device=dev)[None, :, None, None] if causal else v.float().mean(1, keepdim=True).expand(v.shape)
     assert (lse == -(2.0 ** 119)).all()
     assert_parity(o, ref, TOL_BF16, "o")
+
+
+@pytest.mark.parametrize("causal", [False, True], ids=["full", "causal"])
+@pytest.mark.parametrize("D,L,H,Hkv", [(64, 300, 4, 4), (64, 2100, 16, 4), (128, 300, 4, 1), (128, 700, 8, 8), (128, 2100, 2, 2)])
+def test_attention_bwd_of_scores_above_any_usual_one(D, L, H, Hkv, causal, dev):
+    """Every score of a row the same, near 2^120, and a last tile of queries that is not full: what fills it up has no probability.  dV is the sum of
+    dO / (visible keys)."""
+    from odysseus_transformer_amd import ops
+    print(f"D={D} L={L} H={H} {Hkv} causal={causal}", flush=True)
+    q = torch.zeros(1, L, H, D, dtype=torch.bfloat16, device=dev)
+    k, v = q[:, :, :Hkv].clone(), randn((1, L, Hkv, D), 5, dtype=torch.bfloat16).to(dev)
+    do = randn((1, L, H, D), 6, dtype=torch.bfloat16).to(dev)
+    q[..., 0] = k[..., 0] = 2.0 ** 60
+    n = torch.arange(1, L + 1, device=dev).float() if causal else torch.full((L,), float(L), device=dev)
+    o = (v.float().cumsum(1) / n[None, :, None, None] if causal else v.float().mean(1, keepdim=True).expand(v.shape)).repeat_interleave(H // Hkv, 2)
+    # the log-sum-exp of one score: the number of the others is below its last bit
+    lse = torch.full((1, H, L), 2.0 ** 119, device=dev)
+    dq, dk, dv = ops.attn_bwd(q, k, v, o.bfloat16(), lse, do, causal=causal, scale=0.5)
+    assert all(bool(t.isfinite().all()) for t in (dq, dk, dv))
+    d = do.float().view(1, L, Hkv, H // Hkv, D).sum(3)
+    ref = d.flip(1).cumsum(1).flip(1) if causal else d.sum(1, keepdim=True).expand(d.shape)   # P = 1 everywhere, as lse says
+    assert_parity(dv, ref, TOL_BF16, "dv")
