@@ -38,7 +38,7 @@ sys.path.insert(0, str(ROOT))
 
 PEAK_BF16_TFLOPS = 2500.0   # MI355X dense bf16 MFMA, published
 PEAK_HBM_GBS = 8000.0       # MI355X HBM3E, published
-PEAK_FP32_TFLOPS = 157.3    # MI355X dense fp32 MFMA, published
+PEAK_FP32_PARTS_TFLOPS = PEAK_BF16_TFLOPS / 6   # fp32 as three bf16 parts per value: six bf16 products for one
 
 # the rank shard the metric is quoted on
 L, H, HKV, D = 32768, 4, 4, 128
@@ -739,7 +739,8 @@ def power_under_load(_lib, ops, dev, attention_step):
 
 def fp32_configuration(_lib, ops, dev):
     """The fp32 parity configuration on the GPU (d=512, 8 heads x 64, i=1376, L=2048: one decoder layer forward +
-    backward), and the fp32 kernels at a size that fills the chip, against the 157.3 TFLOP/s fp32 matrix peak."""
+    backward), and the fp32 kernels at a size that fills the chip, against a sixth of the bf16 matrix peak (both run on bf16
+    parts; the fp32 instruction itself would allow 157.3 TFLOP/s)."""
     import types
     import torch
     from odysseus_transformer_amd.decoder.odysseus import OdysseusDecoderLayer
@@ -773,13 +774,13 @@ def fp32_configuration(_lib, ops, dev):
     tb = time_gpu(lambda: ops.attn_bwd(q, k, v, o, lse, do, causal=True), 3, 1)
     res["attention_L16384_8x64"] = {"fwd_ms": round(tf * 1e3, 3), "bwd_ms": round(tb * 1e3, 3),
                                     "fwd_tflops": round(f_fwd / tf / 1e12, 1), "bwd_tflops": round(f_bwd / tb / 1e12, 1),
-                                    "frac_of_fp32_peak": round((f_fwd + f_bwd) / (tf + tb) / 1e12 / PEAK_FP32_TFLOPS, 3)}
+                                    "frac_of_bf16_peak_over_6": round((f_fwd + f_bwd) / (tf + tb) / 1e12 / PEAK_FP32_PARTS_TFLOPS, 3)}
     del q, k, v, do, o, lse
     M = N = K = 4096
     a, b, c = (torch.randn((M, K), generator=g).to(dev) for _ in range(3))
     ts = [time_gpu(lambda op=op: ops.gemm(op, a, b), 3, 1) for op in (ops.GEMM_NT, ops.GEMM_NN, ops.GEMM_TN)]
     res["gemm_4096x4096x4096"] = {"tflops_nt_nn_tn": [round(2.0 * M * N * K / t / 1e12, 1) for t in ts],
-                                  "frac_of_fp32_peak": round(2.0 * M * N * K / max(ts) / 1e12 / PEAK_FP32_TFLOPS, 3)}
+                                  "frac_of_bf16_peak_over_6": round(2.0 * M * N * K / max(ts) / 1e12 / PEAK_FP32_PARTS_TFLOPS, 3)}
     return res
 
 

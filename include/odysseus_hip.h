@@ -330,7 +330,8 @@ int ody_attn_bwd_rope(const void* q, const void* k, const void* v, const void* o
 
 /* The RMSNorm in front of a product of few rows (a decoding step) inside the product, so that the normalised rows are never stored:
  * bf16, at most 4 rows that take 64 KiB together (2 M (K + 8)), K a multiple of 8, 16-byte aligned rows (ODY_ERR_UNSUPPORTED
- * otherwise: ody_rmsnorm_fwd and the product do).  Same arithmetic as the two kernels.
+ * otherwise: ody_rmsnorm_fwd and the product do).  The arithmetic of the two kernels but for the order of the norm's sum of squares: an
+ * ulp of 1 / rms, which can move a rounding of a normalised value.
  * ody_norm_linear_rope      ody_linear_rope of ody_rmsnorm_fwd(x); head_dim 128, the angles from position_ids (M) and
  *                           inv_freq (D / 2) directly, rounded as ody_rope_table rounds them (decoder/odysseus.py:180-213 behind
  *                           decoder/ring.py:67).

@@ -105,8 +105,9 @@ int ody_launch_attn_bwd_pipe(const AttnParams& p, void* workspace, hipStream_t s
 int ody_launch_attn_fwd_hd64(const AttnParams& p, hipStream_t st);
 size_t ody_attn_bwd_hd64_workspace(int B, int Lq, int Lk, int Hq, int Hkv);
 int ody_launch_attn_bwd_hd64(const AttnParams& p, void* workspace, size_t workspace_bytes, hipStream_t st);
-// head_dim 128 where those two leave compute units idle; neither workspace nor images.  The backward runs behind the pre-pass, from
-// p.delta and its start values, and leaves fp32 dK / dV of every query head in `part` if Hq != Hkv.
+// head_dim 128 where those two leave compute units idle.  Neither reads images; the forward uses no workspace (its callers still ask for that of
+// the kernel above).  The backward runs behind the pre-pass, which writes the images of Q and dO all the same, for a later call that reuses the query
+// side; it reads p.delta and the start values, and leaves fp32 dK / dV of every query head in `part` if Hq != Hkv.
 bool ody_attn_fwd_short_ok(int B, int Lq, int Lk, int Hq, int causal);
 bool ody_attn_bwd_short_ok(int B, int Lq, int Lk, int Hq, int causal);
 int ody_launch_attn_fwd_short(const AttnParams& p, hipStream_t st);

@@ -5,7 +5,8 @@
 // serial chain of tiles is half as long; the halves add up through LDS at the end.  For dK and dV the two sets share the tiles and the
 // work: one holds dV, the other dK (S is formed twice, which costs less than the registers of both: a chain of three products instead of
 // four).  Tiles come straight to LDS, two stages, and serve as row operands and, through the transposing read, as transposed ones
-// (attn_rowtile.h), at half the LDS rate but without an image, its pass and its launch.  All of the backward behind the pre-pass is one launch.
+// (attn_rowtile.h), at half the LDS rate but without images: no pass that writes those of K and V (those of Q and dO come with the pre-pass, for later
+// calls that reuse the query side).  All of the backward behind the pre-pass is one launch.
 //
 // What bounds it: latency of a chain of tiles in a block (about 2.5 us for 128 rows against 128 keys in the forward) on 1 block a unit.
 // Before / here, us, launches included: forward of 4 x 8 heads, L = 331, causal 19.8 / 12.7 (three launches / one), backward on 2 kv heads

@@ -11,7 +11,9 @@
 //
 // 4096^3, NT / TN: 1016 / 1023 -> 690 / 720 us (199 / 191 TFLOP/s).  The products of a layer of hidden 512 over 2048 tokens, us before /
 // now: 2048 x 1536 x 512 37 / 29, x 2752 60 / 43, x 512 14.8 / 12, 2048 x 512 x 1376 34 / 26, 2048 x 512 x 2752 NN 61 / 46, 2752 x 512 x 2048
-// TN 66 / 54, 512 x 512 x 2048 TN 17.6 / 16.7 (sum over all twelve 454 / 361).
+// TN 66 / 54, 512 x 512 x 2048 TN 17.6 / 16.7 (sum over all twelve 454 / 361).  Without SPLIT_UP, which is one more instruction an element
+// and keeps the bits of operands below 2^-110, and with it, both on another box: 4096^3 NT / NN / TN 783 / 774 / 807 and 786 / 778 / 814;
+// 2048 x 1536 x 512 29.9 and 30.5, 2048 x 2752 x 512 44.6 and 45.6, 512 x 1376 x 2048 TN 32.4 and 33.6 (the most).
 //
 // An input that is not finite, or from 2^111.99 on, makes 0 x infinity in a product that is none, and a result from 2^96 on is infinite before
 // SPLIT_DOWN; a wavefront that finds a result that is not finite forms its tiles again on the fp32 instruction, straight from memory.

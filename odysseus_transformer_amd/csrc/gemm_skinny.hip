@@ -16,7 +16,7 @@ namespace {
 constexpr int SK_WAVES = 8;
 
 // NORM: A is x, and the product that of its RMS-normalised rows.  Every block normalises them for itself, into LDS, with the arithmetic of
-// the RMSNorm kernel, while its first fragments of W are on their way; EPI_ROPE then takes its angles from the positions too.  Weights
+// the RMSNorm kernel (another order of the sum), while its first fragments of W are on their way; EPI_ROPE then takes its angles from the positions too.  Weights
 // cold, us without the norm / with it, one row: 6144 x 4096 with rotation 13.3 / 15.9, 22016 x 4096 SwiGLU 41.1 / 43.2, 5632 x 1024
 // 5.9 / 6.8; four rows 13.6 / 18.1, 43.4 / 47.1, 6.1 / 8.6.  The norm's own launch takes 2.6, the table's 2.0, and each its gap and 5 of host
 // work.  (The norm inside the K loop, on every fragment, took 16.2 and 46.6; a ring of fragments refilled one by one instead of a batch
