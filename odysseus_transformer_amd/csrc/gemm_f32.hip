@@ -3,7 +3,8 @@
 // An fp32 value is the sum of three bf16 values (split3.h); of the nine products of two such sums the six largest are formed, which
 // leaves out at most a unit roundoff of fp32, 2^-24 of a product, and 2^-27.5 in the root mean square.  The largest one and the five others accumulate apart, so that
 // the sum of the large terms is rounded once per 16 of K (the fp32 matrix instruction: every 2).  2-norm error against 64 bits, this
-// / v_mfma_f32_32x32x2_f32 before it, N(0, 1) operands: K = 512 0.8e-7 to 1.3e-7 / 2.9e-7, 2048 1.3e-7 / 2.9e-7, 4096 4.0e-7 / 11.5e-7.
+// / v_mfma_f32_32x32x2_f32 before it, N(0, 1) operands: K = 512 0.8e-7 to 1.3e-7 / 2.9e-7, 2048 1.3e-7 / 2.9e-7, 4096 4.0e-7 / 11.5e-7.  Operands on [1, 2), K = 4 to 4096:
+// 2.8e-8 to 6.4e-8 / 3.8e-8 to 12.7e-8; all of them 0x1.00ff8p+0, where what is left out is largest and always of one sign: 5.9e-8 both.
 //
 // Six bf16 instructions take 192 matrix cycles where the fp32 one takes 512.  Bound by the rate of the matrix cores at the power limit
 // where the product is large (4096^3: 70 % busy at 1.7 GHz), by the loads where it is small: a 64 x 64 tile moves 16 KB per 32 of K and
