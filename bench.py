@@ -199,7 +199,7 @@ def tile_cost_ladder(_lib, dev, fwd_ms):
     nqb = L // 256
     tiles = sum(min(L // 64, (qb * 256 + 255) // 64 + 1) for qb in range(nqb)) * H     # 64-key tiles x 256-query blocks
     mfmas = (tiles * 8 - nqb * H * 12) * 32        # 12 (wavefront, tile) pairs of a diagonal block lie above the diagonal
-    res["attn_fwd_w8"] = {"ns_per_turn": round(fwd_ms * 1e6 / (mfmas / (1024 * 64)), 1),
+    res["attn_fwd_pipe"] = {"ns_per_turn": round(fwd_ms * 1e6 / (mfmas / (1024 * 64)), 1),
                           "tflops_executed": round(mfmas * 32768.0 / (fwd_ms * 1e-3) / 1e12, 1)}
     return res
 
@@ -338,7 +338,7 @@ def main():
     # (with kept dS -- ops.attn_bwd's default where the scratch fits -- the dQ kernel is the one product, over
     # the dS tiles that the dK/dV kernel stored: 2 bytes per visible pair each way)
     dq_kernel = "attn_bwd_dq_kept" if "attn_bwd_dq_kept" in prof else "attn_bwd_dq_pipe"
-    algo = {"attn_fwd_w8": f_fwd, "attn_bwd_dkdv_pipe": f_bwd * 4 / 5, dq_kernel: f_bwd * 1 / 5}
+    algo = {"attn_fwd_pipe": f_fwd, "attn_bwd_dkdv_pipe": f_bwd * 4 / 5, dq_kernel: f_bwd * 1 / 5}
     missing = [n for n in algo if n not in prof]
     if missing:
         raise SystemExit(f"bench.py: the library ran no kernel named {missing}; it reported {sorted(prof)}")
@@ -378,7 +378,7 @@ def main():
               "bf16_peak_from_cus_and_clock_tflops": round(info["compute_units"] * info["clock_khz"] * 1e3 * 4096 / 1e12, 1)}
     # kernels of the forward: the V image (one of the step's two image launches; the other is the backward's K
     # image), the main kernel and its follow-up over flagged query blocks; everything else belongs to the backward
-    fwd_ms = (prof["attn_fwd_w8"][1] + prof.get("attn_fwd_mfma", (0, 0.0, 0))[1] +
+    fwd_ms = (prof["attn_fwd_pipe"][1] + prof.get("attn_fwd_mfma", (0, 0.0, 0))[1] +
               prof.get("attn_images", (0, 0.0, 0))[1] / 2) / a.steps
     bwd_ms = sum(t for n, (_, t, _) in prof.items()) / a.steps - fwd_ms
 
@@ -411,7 +411,7 @@ def main():
     out["mfma_sustained"] = mfma_sustained(_lib, dev)
     # boxes differ by ~10 % in what they sustain at the power limit; this ratio does not
     out["value_over_mfma_sustained_random"] = round(value / out["mfma_sustained"]["random_operands_tflops"], 3)
-    out["tile_cost_ladder"] = tile_cost_ladder(_lib, dev, kernels["attn_fwd_w8"]["avg_ms"])
+    out["tile_cost_ladder"] = tile_cost_ladder(_lib, dev, kernels["attn_fwd_pipe"]["avg_ms"])
     if a.power:
         out["power"] = power_under_load(_lib, ops, dev, step)
     del qkv, q, k, v, do, dqkv
@@ -428,7 +428,7 @@ def main():
     print(json.dumps(out))
 
 
-FWD_KERNELS = ("attn_fwd_w8", "attn_fwd_mfma", "lse_merge", "cast_from_f32")
+FWD_KERNELS = ("attn_fwd_pipe", "attn_fwd_mfma", "lse_merge", "cast_from_f32")
 
 
 def other_configs(_lib, ops, rn, dev):

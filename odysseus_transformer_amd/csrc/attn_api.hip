@@ -82,14 +82,14 @@ int attn_fwd_impl(const char* who, const void* q, const void* k, const void* v, 
   }
   if (dtype == ODY_BF16 && D == 128 && p.drop_thresh == 0) {
     // the least that will do: without room for the parts of a key-split call the call runs unsplit
-    const size_t need = (ody_attn_fwd_w8_workspace(B, Lq, Lk, Hq, Hkv, false) + 255) & ~(size_t)255;
+    const size_t need = (ody_attn_fwd_pipe_workspace(B, Lq, Lk, Hq, Hkv, false) + 255) & ~(size_t)255;
     ODY_REQUIRE(workspace != nullptr, ODY_ERR_NULL, "%s: workspace is NULL", who);
     ODY_REQUIRE(workspace_bytes >= need, ODY_ERR_WORKSPACE, "%s: workspace of %zu bytes, %zu needed", who,
                 workspace_bytes, need);
     ODY_REQUIRE((reinterpret_cast<uintptr_t>(workspace) & 255u) == 0, ODY_ERR_MISALIGNED,
                 "%s: workspace must be 256-byte aligned", who);
     if (ody_attn_fwd_short_ok(B, Lq, Lk, Hq, p.causal)) return ody_launch_attn_fwd_short(p, st);
-    return ody_launch_attn_fwd_w8(p, workspace, workspace_bytes, st);
+    return ody_launch_attn_fwd_pipe(p, workspace, workspace_bytes, st);
   }
   if (dtype == ODY_BF16 && p.drop_thresh == 0) return ody_launch_attn_fwd_hd64(p, st);
   if (dtype == ODY_BF16) return ody_launch_attn_fwd_mfma(p, D, st);
@@ -161,9 +161,9 @@ extern "C" int ody_attn_fwd_noalloc(const void* q, const void* k, const void* v,
     need = (ody_attn_decode_workspace(B, Lq, Lk, Hq, Hkv, D) + 255) & ~(size_t)255;
     if (need > (size_t)ODY_ATTN_FWD_NOALLOC_SCRATCH_BYTES) need = 0;
   } else if (dtype == ODY_BF16 && D == 128) {
-    need = (ody_attn_fwd_w8_workspace(B, Lq, Lk, Hq, Hkv, true) + 255) & ~(size_t)255;
+    need = (ody_attn_fwd_pipe_workspace(B, Lq, Lk, Hq, Hkv, true) + 255) & ~(size_t)255;
     if (need > (size_t)ODY_ATTN_FWD_NOALLOC_SCRATCH_BYTES)
-      need = (ody_attn_fwd_w8_workspace(B, Lq, Lk, Hq, Hkv, false) + 255) & ~(size_t)255;
+      need = (ody_attn_fwd_pipe_workspace(B, Lq, Lk, Hq, Hkv, false) + 255) & ~(size_t)255;
   }
   ODY_REQUIRE(need <= (size_t)ODY_ATTN_FWD_NOALLOC_SCRATCH_BYTES, ODY_ERR_WORKSPACE,
               "ody_attn_fwd_noalloc: this shape needs %zu bytes of scratch, the library-owned buffer holds %zu "
@@ -181,7 +181,7 @@ extern "C" size_t ody_attn_fwd_workspace_bytes(int B, int Lq, int Lk, int Hq, in
     // a caller with dropout on these sizes (other kernels, no workspace) merely holds bytes it does not use
     return (ody_attn_decode_workspace(B, Lq, Lk, Hq, Hkv, D) + 255) & ~(size_t)255;
   }
-  if (dtype == ODY_BF16 && D == 128) return (ody_attn_fwd_w8_workspace(B, Lq, Lk, Hq, Hkv, true) + 255) & ~(size_t)255;
+  if (dtype == ODY_BF16 && D == 128) return (ody_attn_fwd_pipe_workspace(B, Lq, Lk, Hq, Hkv, true) + 255) & ~(size_t)255;
   return 0;
 }
 

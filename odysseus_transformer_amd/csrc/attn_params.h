@@ -82,12 +82,12 @@ int ody_launch_attn_images(const void* src, const AttnStrides& s, int B, int L, 
 // head_dim 128 backward, everything that depends on the queries only, in one launch: p.delta, the transposed images
 // of Q and dO and the start values (1 KB per 64-query tile)
 int ody_launch_attn_bwd_prepass(const AttnParams& p, void* qimg, void* doimg, void* stats, hipStream_t st);
-// head_dim 128 only, 8 wavefronts x 32 queries per block; workspace of ody_attn_fwd_w8_workspace(...) bytes.
+// head_dim 128 only, 256 queries per block; workspace of ody_attn_fwd_pipe_workspace(...) bytes.
 // with_split: with room for the fp32 parts of a call whose fully visible key range is cut into 2 or 4 parts (few query
 // blocks against many keys); a workspace without that room makes such a call run unsplit.
-int ody_launch_attn_fwd_w8(const AttnParams& p, void* workspace, size_t workspace_bytes, hipStream_t st);
-size_t ody_attn_fwd_w8_workspace(int B, int Lq, int Lk, int Hq, int Hkv, bool with_split);
-int ody_attn_fwd_w8_parts(int B, int Lq, int Lk, int Hq, int causal);   // of every block's key range, where the workspace has the room
+int ody_launch_attn_fwd_pipe(const AttnParams& p, void* workspace, size_t workspace_bytes, hipStream_t st);
+size_t ody_attn_fwd_pipe_workspace(int B, int Lq, int Lk, int Hq, int Hkv, bool with_split);
+int ody_attn_fwd_pipe_parts(int B, int Lq, int Lk, int Hq, int causal);   // of every block's key range, where the workspace has the room
 // forward for at most 64 rows per kv head (rows = queries x query heads of its group), key ranges cut over blocks; a workspace
 // without room for the parts makes the call run on one block per kv head
 bool ody_attn_decode_ok(int Lq, int Hq, int Hkv, int D);

@@ -1,4 +1,4 @@
-// Flash attention for bf16 and head_dim 128 where the kernels for long sequences (attn_fwd_w8.hip, attn_bwd_pipe.hip) leave compute units
+// Flash attention for bf16 and head_dim 128 where the kernels for long sequences (attn_fwd_pipe.hip, attn_bwd_pipe.hip) leave compute units
 // idle or wait for latency: few blocks of 256 rows, each a few tiles long, behind passes that write transposed images.
 //
 // A block is 128 rows: 4 wavefronts of 32 rows, twice.  In the forward and for dQ the second four take every other key tile, so that the
@@ -435,7 +435,7 @@ inline int64_t row_blocks(int B, int L, int H) { return (int64_t)B * H * ((L + B
 // One head, too, below the line: backward of 512 rows, causal, 65 us there, 29 here, of 1024 rows 101 / 45; two heads of 512 rows 66 / 29.
 bool ody_attn_fwd_short_ok(int B, int Lq, int Lk, int Hq, int causal) {
   const int64_t blocks = row_blocks(B, Lq, Hq);
-  if (blocks <= 64 && ody_attn_fwd_w8_parts(B, Lq, Lk, Hq, causal) > 1) return false;
+  if (blocks <= 64 && ody_attn_fwd_pipe_parts(B, Lq, Lk, Hq, causal) > 1) return false;
   return blocks <= (causal ? 640 : 256) && Lk <= ROWS * (blocks <= 128 ? 32 : 64);
 }
 bool ody_attn_bwd_short_ok(int B, int Lq, int Lk, int Hq, int causal) {
