@@ -1,11 +1,10 @@
 // Flash-attention backward, head_dim 128, bf16, on the tile machinery of attn_tile.h: direct
 // global->LDS loads into a ring of stages, 16-byte LDS reads only (an operand that a product
 // contracts over its row index comes from the transposed images a pre-pass writes), fenced slots
-// that keep LDS operand prefetch and MFMAs interleaved, 8 wavefronts per block = two per SIMD,
-// which overlap each other's matrix and vector phases.  Two kernels, no atomics: both recompute S
+// that keep LDS operand prefetch and MFMAs interleaved.  Two kernels, no atomics: both recompute S
 // from the saved log-sum-exp, and each owns its outputs.
 //
-// dQ kernel -- query-stationary, 32 queries per wavefront, lane = query column, so lse and delta
+// dQ kernel -- query-stationary, 8 wavefronts x 32 queries, two per SIMD, lane = query column, so lse and delta
 // are per-lane scalars; a three-deep ring of {K tile, V tile, K^T image}:
 //
 //      S^T = K Q^T            A: K rows (LDS)        B: Q^T (registers)
@@ -13,7 +12,7 @@
 //      dS^T = exp2(S^T c - lse) * (dP^T - delta)
 //      dQ^T += K^T dS^T       A: K^T image (LDS)     B: dS^T = accumulator layout
 //
-// dK/dV kernel -- key-stationary, 32 keys per wavefront (described where it is defined).
+// dK/dV kernel -- key-stationary (described where it is defined).
 #include <algorithm>
 #include <type_traits>
 #include <utility>
@@ -26,6 +25,7 @@ using namespace tile128;
 
 constexpr int D = 128, KS = D / 16, DT = D / 32;
 #define FENCE() __builtin_amdgcn_sched_barrier(0)
+#define INLINE __attribute__((always_inline))
 
 // The same accumulators as one part's unscaled fp32 sum (a dQ kernel whose key range is cut into parts):
 // dq_part [part][B][Lq][Hq][D]; attn_bwd_dq_sum_kernel adds the parts and finishes dq as store_dq_row would.
@@ -237,17 +237,27 @@ __global__ __launch_bounds__(DQ_THREADS) void attn_bwd_dq_pipe_kernel(const Attn
 // ---------------------------------------------------------------------------------
 // dK / dV
 // ---------------------------------------------------------------------------------
-// Key-stationary, 8 wavefronts x 32 keys (two wavefronts per SIMD), lane = key column.  K and V
-// rows stay in registers as B operands; 64-query tiles of Q and dO stream through a two-deep
-// ring as row tiles (A operands of S and dP) and as transposed images (A operands of dV^T and
+// Key-stationary, 4 wavefronts x 64 keys, one per SIMD with its whole register file, lane = key column.  K and V
+// rows stay in registers as B operands (128), dK^T and dV^T fill the accumulation registers (256); 64-query tiles of Q and dO stream
+// through two-deep rings as row tiles (A operands of S and dP) and as transposed images (A operands of dV^T and
 // dK^T); P and dS are accumulator tiles, which is the B-operand layout of the next product.
 //
 //      S  = Q K^T - lse/scale     the accumulators start at -lse/scale, so P = exp2(S c)
 //      dP = dO V^T - delta        likewise -delta
 //      dV^T += dO^T P             dK^T += Q^T (P o dP)
-constexpr int KV_WAVES = 8, KV_BN = 32 * KV_WAVES, KV_BQ = 64, KV_THREADS = 64 * KV_WAVES;
+//
+// The work goes by units of 32 queries x 32 keys.  While the 16 products of dV and dK of one unit and the 16 of S and dP of the next go through
+// the matrix pipe, the exponentials, dS and the packing of that next unit are formed, two or three instructions under each product, so
+// that both pipes are busy by the order of the instructions.  (Both halves of the keys in one go would read every fragment once instead of twice,
+// but needs 70 registers more than there are.)  The order of the sums, and with it every bit of dK and dV, is that of the
+// kernel before, which had 8 wavefronts of 32 keys, two per SIMD, each forming a unit's parts one after the other.  Bound: power.
+// us before / here, two boxes: 4 heads, L = 32768, causal 1886 / 1640 (constant operands, where power is no bound, 1511 / 1160: the matrix pipe 58 / 75 %
+// busy), 32 heads on 8, L = 16384 3861 / 3390, 4 heads, 8192 queries on 16384 keys 471 / 410.  Of the gain 2 % is one wait for four
+// fragments in the place of four.
+constexpr int KV_WAVES = 4, KV_KT = 2, KV_BN = 32 * KV_KT * KV_WAVES, KV_BQ = 64, KV_THREADS = 64 * KV_WAVES;
 constexpr int KV_STAT_ELEMS = 64 * 8;                                    // start-value record of one tile: 1 KB, one direct load
-constexpr int KV_STAGE = 2 * TILE_ELEMS + 2 * IMG_ELEMS + KV_STAT_ELEMS;   // Q, dO tiles; Q^T, dO^T images; start values
+constexpr int KV_ROWS = 2 * TILE_ELEMS + KV_STAT_ELEMS, KV_IMAGES = 2 * IMG_ELEMS;   // Q, dO tiles and start values; Q^T, dO^T images
+static_assert(KV_WAVES == 4, "the load split and the vmcnt waits assume 4 wavefronts");
 
 // dS kept for the dQ kernel (Lq and Lk multiples of 256; causal: Lq == Lk): one 128 KB block per (256-key block kb,
 // 256-query block qb; causal: qb >= kb), laid out for the reader, which takes 64 keys x 256 queries at a time:
@@ -275,7 +285,7 @@ __host__ __device__ inline int64_t ds_block_index(int nbq, int kb, int qb, bool 
 // start of a 1 KB record, register r of group g being query acc_tile_row(r, g, mt).  Rows that must give P = 0
 // (beyond Lq, or a query that saw no key) hold minus infinity.
 //
-// SPLIT = false: a block owns 256 keys of one kv head and walks all query heads of its group.
+// SPLIT = false: a block owns 256 keys of a kv head with one query head.
 // SPLIT = true (grouped-query attention, or too few key blocks for the chip): a block owns 256 keys for ONE query
 // head and part `bc.h % qparts` of that head's query tiles, and writes fp32 partial dK / dV to `part`, which
 // attn_bwd_group_sum_kernel adds up over the group and the parts.  With few kv heads, or few keys against many
@@ -285,196 +295,321 @@ __host__ __device__ inline int64_t ds_block_index(int nbq, int kb, int qb, bool 
 // layout described at ds_block_index, and the dQ kernel below (attn_bwd_dq_kept_kernel) reads it back
 // instead of computing S, dP and dS a second time.
 template <bool SPLIT, bool KEEP_DS>
-__global__ __launch_bounds__(KV_THREADS) void attn_bwd_dkdv_pipe_kernel(const AttnParams p,
-                                                                         const bf16* __restrict__ qimg,
-                                                                         const bf16* __restrict__ doimg,
-                                                                         const bf16* __restrict__ stats,
-                                                                         float* __restrict__ part, int qparts) {
+__global__ __launch_bounds__(KV_THREADS, 1) void attn_bwd_dkdv_pipe_kernel(const AttnParams p,
+                                                                            const bf16* __restrict__ qimg,
+                                                                            const bf16* __restrict__ doimg,
+                                                                            const bf16* __restrict__ stats,
+                                                                            float* __restrict__ part, int qparts) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
-  bf16* ring = reinterpret_cast<bf16*>(smem_raw);   // [2][KV_STAGE]
+  bf16* rring = reinterpret_cast<bf16*>(smem_raw);   // [2][KV_ROWS]
+  bf16* iring = rring + 2 * KV_ROWS;                 // [2][KV_IMAGES]
 
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, g = lane >> 5,
             i = lane & 31;
   const BlockCoord bc = ody_block_coord(SPLIT ? p.Hq * qparts : p.Hkv, p.B);   // rank 0 = first key block = most query tiles
-  const int hq = SPLIT ? bc.h / qparts : 0, qpart = SPLIT ? bc.h % qparts : 0;
-  const int hk = SPLIT ? hq / p.group : bc.h, b = bc.b;
-  const int h_first = SPLIT ? hq : hk * p.group, n_heads = SPLIT ? 1 : p.group;   // query heads this block walks
-  const int n0 = bc.rank * KV_BN, wn0 = n0 + wave * 32, key = wn0 + i;
+  const int h = SPLIT ? bc.h / qparts : bc.h, qpart = SPLIT ? bc.h % qparts : 0;   // (unless SPLIT, every head has keys of its own)
+  const int hk = SPLIT ? h / p.group : h, b = bc.b;
+  const int n0 = bc.rank * KV_BN, wn0 = n0 + wave * 32 * KV_KT;
   const int q_tiles = (p.Lq + KV_BQ - 1) / KV_BQ;
-  simd_stagger(tid);
 
-  bf16x8 kf[KS], vf[KS];
+  const int t_begin = p.causal ? max(0, n0 - p.off) / KV_BQ : 0;   // first query tile that sees a key of this block
+  int total = max(0, q_tiles - t_begin), t_top = q_tiles - 1;   // this block's tiles: t_top, t_top - 1, ... (total of them)
+  if (SPLIT && qparts > 1) {
+    const int per = (total + qparts - 1) / qparts;
+    t_top -= qpart * per;
+    total = max(0, min(per, total - qpart * per));
+  }
+  // (last query tile first: the key blocks of an XCD then read the same Q / dO tiles at the same time and share them through L2)
+  // of them, those that see a key of this wavefront, and before them those that see all of its keys
+  int w_total = total, w_full = total;
+  if (p.causal) {
+    w_total = min(total, max(0, t_top + 1 - max(0, wn0 - p.off) / KV_BQ));
+    w_full = min(total, max(0, t_top + 1 - (max(0, wn0 + 32 * KV_KT - 1 - p.off) + KV_BQ - 1) / KV_BQ));
+  }
+
+  bf16x8 kf[KV_KT][KS], vf[KV_KT][KS];
   {
     const bf16* kp = static_cast<const bf16*>(p.k) + b * p.sk.b + hk * p.sk.h;
     const bf16* vp = static_cast<const bf16*>(p.v) + b * p.sv.b + hk * p.sv.h;
 #pragma unroll
-    for (int ks = 0; ks < KS; ks++) {
-      if (key < p.Lk) {
-        kf[ks] = *reinterpret_cast<const bf16x8*>(kp + (int64_t)key * p.sk.l + 16 * ks + 8 * g);
-        vf[ks] = *reinterpret_cast<const bf16x8*>(vp + (int64_t)key * p.sv.l + 16 * ks + 8 * g);
-      } else {
-        kf[ks] = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
-        vf[ks] = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
+    for (int kh = 0; kh < KV_KT; kh++) {
+      const int key = wn0 + 32 * kh + i;
+#pragma unroll
+      for (int ks = 0; ks < KS; ks++) {
+        kf[kh][ks] = vf[kh][ks] = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
+        if (key < p.Lk) {
+          kf[kh][ks] = *reinterpret_cast<const bf16x8*>(kp + (int64_t)key * p.sk.l + 16 * ks + 8 * g);
+          vf[kh][ks] = *reinterpret_cast<const bf16x8*>(vp + (int64_t)key * p.sv.l + 16 * ks + 8 * g);
+        }
       }
     }
   }
-  f32x16 dk[DT], dv[DT];
 #pragma unroll
-  for (int dt = 0; dt < DT; dt++)
+  for (int kh = 0; kh < KV_KT; kh++)
 #pragma unroll
-    for (int r = 0; r < 16; r++) dk[dt][r] = dv[dt][r] = 0.f;
-
-  const int t_begin = p.causal ? max(0, n0 - p.off) / KV_BQ : 0;   // first query tile that sees a key of this block
-  int ntq = max(0, q_tiles - t_begin), t_top = q_tiles - 1;   // this block's tiles: t_top, t_top - 1, ... (ntq of them)
-  if (SPLIT && qparts > 1) {
-    const int per = (ntq + qparts - 1) / qparts;
-    t_top -= qpart * per;
-    ntq = max(0, min(per, ntq - qpart * per));
-  }
-  const int total = ntq * n_heads;   // flattened (query head, query tile)
+    for (int ks = 0; ks < KS; ks++) asm volatile("" : "+v"(kf[kh][ks]), "+v"(vf[kh][ks]));   // arrived before the direct loads
+  f32x16 dk[KV_KT][DT], dv[KV_KT][DT];
+#pragma unroll
+  for (int kh = 0; kh < KV_KT; kh++)
+#pragma unroll
+    for (int dt = 0; dt < DT; dt++)
+#pragma unroll
+      for (int r = 0; r < 16; r++) dk[kh][dt][r] = dv[kh][dt][r] = 0.f;
   const float c2 = p.scale_log2e;
 
-  // Direct loads of one stage: uniform base pointers plus 32-bit per-lane offsets that are
-  // recomputed from the lane id every time (cheaper than keeping them in registers here).
-  auto load_stage = [&](bf16* st, int it, int j) {   // j = 0, 1: the two halves of the stage's loads
-    const int hg = it / ntq, t = t_top - (it % ntq), h = h_first + hg;
-    const bf16* qp = static_cast<const bf16*>(p.q) + b * p.sq.b + h * p.sq.h + (int64_t)t * KV_BQ * p.sq.l;
-    const bf16* dop = static_cast<const bf16*>(p.dout) + b * p.sdo.b + h * p.sdo.h + (int64_t)t * KV_BQ * p.sdo.l;
-    const int64_t tile_id = ((int64_t)b * p.Hq + h) * q_tiles + t;
-    const bf16* qi_ = qimg + tile_id * IMG_ELEMS;
-    const bf16* doi = doimg + tile_id * IMG_ELEMS;
-    const int rmax = p.Lq - 1 - t * KV_BQ;   // rows beyond the matrix re-read its last row
-    const int ln = fresh_lane();
-    if (j == 0 && wave == KV_WAVES - 1)
-      __builtin_amdgcn_global_load_lds((global_void_ptr)(stats + tile_id * KV_STAT_ELEMS + (unsigned)(ln * 8)),
-                                       (lds_void_ptr)(st + 2 * TILE_ELEMS + 2 * IMG_ELEMS), 16, 0, 0);
-    {
-      const int grp = KV_WAVES * j + wave;
-      const int row = min(4 * grp + (ln >> 4), rmax), col = 8 * (ln & 15);
-      __builtin_amdgcn_global_load_lds((global_void_ptr)(qp + (unsigned)(row * (int)p.sq.l + col)),
-                                       (lds_void_ptr)(st + grp * GROUP_ELEMS), 16, 0, 0);
-      __builtin_amdgcn_global_load_lds((global_void_ptr)(dop + (unsigned)(row * (int)p.sdo.l + col)),
-                                       (lds_void_ptr)(st + TILE_ELEMS + grp * GROUP_ELEMS), 16, 0, 0);
-      __builtin_amdgcn_global_load_lds((global_void_ptr)(qi_ + (unsigned)((grp * 64 + ln) * 8)),
-                                       (lds_void_ptr)(st + 2 * TILE_ELEMS + grp * 512), 16, 0, 0);
-      __builtin_amdgcn_global_load_lds((global_void_ptr)(doi + (unsigned)((grp * 64 + ln) * 8)),
-                                       (lds_void_ptr)(st + 2 * TILE_ELEMS + IMG_ELEMS + grp * 512), 16, 0, 0);
-    }
+  // Direct loads: of the rows of tile `lr` (from the top) and of the images of tile `li`, the last one again where there are no more.
+  // Rows past the end read zeros: they lie beyond the descriptor.
+  int lr = 0, li = 0;
+  const int qrow = 2 * (int)p.sq.l, orow = 2 * (int)p.sdo.l;   // bytes
+  const int qlane = (4 * wave + (lane >> 4)) * qrow + 16 * (lane & 15), olane = (4 * wave + (lane >> 4)) * orow + 16 * (lane & 15);
+  const int ilane = 1024 * wave + 16 * lane;
+  const int64_t tile_id = ((int64_t)b * p.Hq + h) * q_tiles + t_top;
+  const bf16* qtp = static_cast<const bf16*>(p.q) + b * p.sq.b + h * p.sq.h + (int64_t)t_top * KV_BQ * p.sq.l;
+  const bf16* otp = static_cast<const bf16*>(p.dout) + b * p.sdo.b + h * p.sdo.h + (int64_t)t_top * KV_BQ * p.sdo.l;
+  const bf16* stp = stats + tile_id * KV_STAT_ELEMS;
+  const bf16* qip = qimg + tile_id * IMG_ELEMS;
+  const bf16* oip = doimg + tile_id * IMG_ELEMS;
+  const int top_rows = min(KV_BQ, p.Lq - t_top * KV_BQ) - 1;
+  int q_bytes = top_rows * qrow + 256, o_bytes = top_rows * orow + 256;
+  auto bring = [&](const bf16* src, int bytes, bf16* dst, int off, int soff) INLINE {
+    auto rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16*>(src), (short)0, bytes, 0x00020000);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_void_ptr)dst, 16, off, soff, 0, 0);
   };
-  if (total > 0) {
-    load_stage(ring, 0, 0);
-    load_stage(ring, 0, 1);
-  }
+  // a quarter j of the rows (two instructions per wavefront), of the images; every wavefront brings the whole record of start values
+  auto load_rows = [&](int j, int which) INLINE {
+    bf16* dst = rring + (lr & 1) * KV_ROWS + (4 * j + wave) * GROUP_ELEMS;
+    if (which == 0) bring(qtp, q_bytes, dst, qlane + 16 * j * qrow, 0);
+    else bring(otp, o_bytes, dst + TILE_ELEMS, olane + 16 * j * orow, 0);
+  };
+  auto load_stats = [&]() INLINE { bring(stp, 2 * KV_STAT_ELEMS, rring + (lr & 1) * KV_ROWS + 2 * TILE_ELEMS, ilane - 1024 * wave, 0); };
+  auto load_images = [&](int j, int which) INLINE {
+    bring(which ? oip : qip, IMG_BYTES, iring + (li & 1) * KV_IMAGES + which * IMG_ELEMS + (4 * j + wave) * 512, ilane, 4096 * j);
+  };
+  auto next_rows = [&]() INLINE {
+    const int to = min(lr + 1, total - 1), step = to - lr;
+    lr = to;
+    qtp -= (int64_t)step * (KV_BQ / 2 * qrow);
+    otp -= (int64_t)step * (KV_BQ / 2 * orow);
+    stp -= step * KV_STAT_ELEMS;
+    if (step) q_bytes = (KV_BQ - 1) * qrow + 256, o_bytes = (KV_BQ - 1) * orow + 256;
+  };
+  auto next_images = [&]() INLINE {
+    const int to = min(li + 1, total - 1), step = to - li;
+    li = to;
+    qip -= step * IMG_ELEMS;
+    oip -= step * IMG_ELEMS;
+  };
 
-  // one 32-query sub-tile against this wavefront's 32 keys: 16 MFMAs for S and dP on top of their
-  // start values, the vector work, 16 MFMAs for dV^T and dK^T
-  // kept dS: chunk 4 mt + 2 ss + g of part (y, x) = (wave >> 1, t & 3) of the block, to which `tile` points at this
-  // wavefront's 32 keys.  Streaming stores: the tiles are read once, by another kernel.
-  auto sub_tile = [&](const bf16* st, int t, int mt, bool masked, bf16* ds_tile) {
-    const int ln = fresh_lane(), g = ln >> 5, i = ln & 31;
-    const int rbase = row_frag_base(g, i), ibase = image_frag_base(g, i);
-    const bf16* Qt = st;
-    const bf16* Ot = st + TILE_ELEMS;
-    const bf16* Qi = st + 2 * TILE_ELEMS;
-    const bf16* Oi = Qi + IMG_ELEMS;
-    constexpr int PF = 2;
-    bf16x8 qfr[PF], ofr[PF];
-    f32x16 s, dp;
-    {
-      const float* Sf = reinterpret_cast<const float*>(Oi + IMG_ELEMS) + mt * 64 + g * 16;
+  const int rbase = row_frag_base(g, i), ibase = image_frag_base(g, i);
+  const int key_off = p.causal ? wn0 + i - p.off : -(1 << 30);   // + 32 kh: the first query that sees this lane's keys
+  f32x16 s, dp;                          // S, then P; dP, then dS
+  bf16x8 pf[2], dsf[2], pf_next[2], dsf_next[2];
+  // a lane's 16 start values: quarter a of those of S (which = 0) or dP (1) of sub-tile mt
+  auto start_values = [&](const bf16* rows, int mt, int which, int a, f32x16& x) INLINE {
+    const f32x4 v = *reinterpret_cast<const f32x4*>(reinterpret_cast<const float*>(rows + 2 * TILE_ELEMS) + mt * 64 + which * 32 + g * 16 + 4 * a);
+#pragma unroll
+    for (int e = 0; e < 4; e++) x[4 * a + e] = v[e];
+  };
+  // the steps of element r of a unit: exponent, P, dS, and two elements together into the operands
+  auto exponent = [&](int r, int t, int mt, int kh, auto masked) INLINE {
+    float x = s[r] * c2;
+    if (decltype(masked)::value) x = t * KV_BQ + acc_tile_row(r, g, mt) < key_off + 32 * kh ? -INFINITY : x;   // queries before the key
+    s[r] = x;
+  };
+  auto weight = [&](int r) INLINE { s[r] = ody_exp2(s[r]); };
+  auto ds = [&](int r) INLINE { dp[r] *= s[r]; };
+  auto pack = [&](bf16x8 (&dst)[2], const f32x16& src, int q) INLINE {
+    dst[q >> 2][2 * q & 7] = (bf16)src[2 * q], dst[q >> 2][(2 * q & 7) + 1] = (bf16)src[2 * q + 1];
+  };
+  // s_waitcnt lgkmcnt(4), lgkmcnt(8): with the reads that are issued behind them in the order below, half of `fr` is there (one wait for four
+  // fragments: the compiler's own would be one for each)
+  constexpr int LGKM_4 = 0xc47f, LGKM_8 = 0xc87f;
+  bf16x8 fr[8];
+  auto qfrag = [&](const bf16* rows, int mt, int n) INLINE { return row_frag(rows, rbase, n, mt); };                   // k-step n
+  auto ofrag = [&](const bf16* rows, int mt, int n) INLINE { return row_frag(rows + TILE_ELEMS, rbase, n, mt); };
+  auto ifrag = [&](const bf16* im, int mt, int m) INLINE {   // m = 2 n + which: dO^T (0) or Q^T (1) image, k-step n >> 2, columns of 32 n & 3
+    return image_frag(im + ((m & 1) ? 0 : IMG_ELEMS), ibase, (m >> 1) & 3, m >> 3, mt);
+  };
+  auto rslot = [&](int it) INLINE { return rring + (it & 1) * KV_ROWS; };
+  auto islot = [&](int it) INLINE { return iring + (it & 1) * KV_IMAGES; };
+  auto barrier_rows = [&]() INLINE {     // the rows of the next tile have landed (behind them 8 loads of images); everyone is done with those before
+    asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    next_rows();
+  };
+  auto barrier_images = [&]() INLINE {   // likewise the images (behind them 9 loads of rows and start values)
+    asm volatile("s_waitcnt vmcnt(9)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    next_images();
+  };
+  auto keep = [&](bf16* ds_tile, int mt, int kh, int ss) INLINE {
+    // Kept dS: dsf[ss] is chunk 4 mt + 2 ss + g of this lane's key, 512 contiguous bytes per half wavefront.  Streaming stores: the tiles are
+    // read once, by another kernel.
+    typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+    __builtin_nontemporal_store(__builtin_bit_cast(u32x4, dsf[ss]),
+                                reinterpret_cast<u32x4*>(ds_tile + (unsigned)((4 * mt + 2 * ss + g) * DS_PIECE + (32 * kh + i) * 8)));
+  };
+
+  // The work goes by units of 32 queries (sub-tile mt of tile it) x 32 keys (half kh).  One call: S and dP of the unit after (it, MT, KH), then dV
+  // and dK of this one, 16 products each; the vector work of the unit after runs under these 32.  `fr` holds the first 8 fragments of either
+  // part and is left with those of the next.
+  auto unit = [&](int it, auto mt_, auto kh_, auto masked, bf16* ds_tile) INLINE {
+    constexpr int MT = decltype(mt_)::value, KH = decltype(kh_)::value;
+    constexpr int NKH = KH ^ 1, NMT = KH ? MT ^ 1 : MT;                  // the unit after
+    constexpr int AMT = MT ^ 1;                                          // sub-tile of the unit behind that
+    const int nt = KH && MT ? it + 1 : it, t = t_top - nt;
+    const bf16 *rows = rslot(nt), *after = MT ? rslot(it + 1) : rslot(it), *images = islot(it);
+#pragma unroll
+    for (int m = 0; m < 16; m++) {
+      if (m == 4) __builtin_amdgcn_s_waitcnt(LGKM_8);
+      else if ((m & 3) == 0) __builtin_amdgcn_s_waitcnt(LGKM_4);
+      if (m < 8) mfma32_onto(s, fr[m], kf[NKH][m]);
+      else mfma32_onto(dp, fr[m - 8], vf[NKH][m - 8]);
+      FENCE();
+      if (m < 4) start_values(rows, NMT, 1, m, dp);
+      fr[m & 7] = m < 8 ? ofrag(rows, NMT, m) : ifrag(images, MT, m - 8);
+      if (m >= 11) weight(2 * m - 22), weight(2 * m - 21);
+      if (m >= 10) exponent(2 * m - 20, t, NMT, NKH, masked), exponent(2 * m - 19, t, NMT, NKH, masked);   // (S is 3 products old)
+      if (KEEP_DS && (m == 2 || m == 5)) keep(ds_tile, MT, KH, m == 5);
+      // the rows of the tile after the next one: from the barrier in the third unit to the one in the first
+      if (MT == 1 && KH == 1 && (m & 3) == 1) load_rows(m >> 2, 0);
+      if (MT == 0 && KH == 0 && m == 3) load_stats();
+      if (MT == 0 && KH == 0 && m == 7) barrier_images();
+      // the images of the next one: from there on to the barrier in the third unit
+      if (MT == 0 && KH == 1 && (m & 3) == 1) load_images(m >> 2, 1);
+      FENCE();
+    }
+#pragma unroll
+    for (int m = 0; m < 16; m++) {
+      if (m == 12) __builtin_amdgcn_s_waitcnt(LGKM_8);
+      else if ((m & 3) == 0) __builtin_amdgcn_s_waitcnt(LGKM_4);
+      if (m & 1) dk[KH][(m >> 1) & 3] = mfma32(fr[m & 7], dsf[m >> 3], dk[KH][(m >> 1) & 3]);
+      else dv[KH][(m >> 1) & 3] = mfma32(fr[m & 7], pf[m >> 3], dv[KH][(m >> 1) & 3]);
+      FENCE();
+      fr[m & 7] = m < 8 ? ifrag(images, MT, m + 8) : qfrag(after, AMT, m - 8);
+      if (m <= 2) weight(2 * m + 10), weight(2 * m + 11);
+      if (m <= 1) exponent(2 * m + 12, t, NMT, NKH, masked), exponent(2 * m + 13, t, NMT, NKH, masked);
+      if (m >= 2 && m < 8) {   // S is done with by product 7: its start values must be there when the next part begins
+#pragma unroll
+        for (int r = 0; r < 3; r++)
+          if (3 * (m - 2) + r < 16) ds(3 * (m - 2) + r);
+      }
+      if (m >= 3 && m < 7) pack(pf_next, s, 2 * m - 6), pack(pf_next, s, 2 * m - 5);
+      if (m >= 8) pack(dsf_next, dp, m - 8);
+      if (m == 8 || m == 9) start_values(after, AMT, 0, 2 * m - 16, s), start_values(after, AMT, 0, 2 * m - 15, s);
+      if (MT == 1 && KH == 1 && (m & 3) == 1) load_rows(m >> 2, 1);
+      if (MT == 1 && KH == 0 && m == 7) barrier_rows();
+      if (MT == 0 && KH == 0 && (m & 3) == 1) load_images(m >> 2, 0);
+      FENCE();
+    }
+#pragma unroll
+    for (int ss = 0; ss < 2; ss++) pf[ss] = pf_next[ss], dsf[ss] = dsf_next[ss];
+  };
+  std::integral_constant<int, 0> c0;
+  std::integral_constant<int, 1> c1;
+  auto kept = [&](int it) INLINE -> bf16* {   // this wavefront's 64 keys of tile `it` among the kept dS
+    if (!KEEP_DS) return nullptr;
+    const int t = t_top - it, nbq = q_tiles / 4, nbk = p.Lk / KV_BN;
+    return p.ds + (((int64_t)b * p.Hq + h) * ds_blocks_per_head(nbq, nbk, p.causal) + ds_block_index(nbq, bc.rank, t >> 2, p.causal)) * DS_BLOCK_ELEMS +
+           ((wave * 4 + (t & 3)) * 8) * DS_PIECE;
+  };
+
+  if (total > 0) {
+    auto all_rows = [&]() INLINE {
+      load_stats();
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        load_rows(j, 0);
+        load_rows(j, 1);
+      }
+    };
+    auto all_images = [&]() INLINE {
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        load_images(j, 0);
+        load_images(j, 1);
+      }
+    };
+    all_rows();
+    all_images();
+    next_rows();
+    // the rows of the second tile, but for the start values: those the first unit brings, like those of any tile
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      load_rows(j, 0);
+      load_rows(j, 1);
+    }
+    asm volatile("s_waitcnt vmcnt(16)" ::: "memory");   // the first tile's rows
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    int it = 0;
+    if (w_total > 0) {
+      // S, P, dP and dS of the first unit
+      const bf16* rows = rslot(0);
 #pragma unroll
       for (int a = 0; a < 4; a++) {
-        const f32x4 v = *reinterpret_cast<const f32x4*>(Sf + 4 * a), w = *reinterpret_cast<const f32x4*>(Sf + 32 + 4 * a);
-#pragma unroll
-        for (int e = 0; e < 4; e++) s[4 * a + e] = v[e], dp[4 * a + e] = w[e];
+        start_values(rows, 0, 0, a, s);
+        start_values(rows, 0, 1, a, dp);
       }
-    }
-    qfr[0] = row_frag(Qt, rbase, 0, mt);
-    ofr[0] = row_frag(Ot, rbase, 0, mt);
-    qfr[1] = row_frag(Qt, rbase, 1, mt);
-    ofr[1] = row_frag(Ot, rbase, 1, mt);
-    FENCE();
 #pragma unroll
-    for (int ks = 0; ks < KS; ks++) {
-      s = mfma32(qfr[ks % PF], kf[ks], s);
-      dp = mfma32(ofr[ks % PF], vf[ks], dp);
-      if (ks + PF < KS) {
-        qfr[ks % PF] = row_frag(Qt, rbase, ks + PF, mt);
-        ofr[ks % PF] = row_frag(Ot, rbase, ks + PF, mt);
+      for (int n = 0; n < 8; n++) {
+        mfma32_onto(s, qfrag(rows, 0, n), kf[0][n]);
+        mfma32_onto(dp, ofrag(rows, 0, n), vf[0][n]);
       }
+      asm volatile("s_nop 15\n\ts_nop 7" : "+v"(s), "+v"(dp));
+#pragma unroll
+      for (int r = 0; r < 16; r++) {
+        exponent(r, t_top, 0, 0, std::true_type{});
+        weight(r);
+        ds(r);
+      }
+#pragma unroll
+      for (int q = 0; q < 8; q++) {
+        pack(pf, s, q);
+        pack(dsf, dp, q);
+      }
+#pragma unroll
+      for (int a = 0; a < 4; a++) start_values(rows, 0, 0, a, s);
+#pragma unroll
+      for (int n = 0; n < 8; n++) fr[n] = qfrag(rows, 0, n);
       FENCE();
-    }
-    bf16x8 oif[PF], qif[PF];
-#pragma unroll
-    for (int n = 0; n < PF; n++) {
-      oif[n] = image_frag(Oi, ibase, n & 3, n >> 2, mt);
-      qif[n] = image_frag(Qi, ibase, n & 3, n >> 2, mt);
-    }
-    if (masked) {
-      const int lim = wn0 + i - p.off - t * KV_BQ;   // tile rows below lim come before this lane's key
-#pragma unroll
-      for (int r = 0; r < 16; r++)
-        if (acc_tile_row(r, g, mt) < lim) s[r] = -INFINITY;
-    }
-    bf16x8 pf[2], dsf[2];
-#pragma unroll
-    for (int r = 0; r < 16; r++) {
-      const float pr = ody_exp2(s[r] * c2);
-      pf[r >> 3][r & 7] = (bf16)pr;
-      dsf[r >> 3][r & 7] = (bf16)(pr * dp[r]);
-    }
-    // Kept dS: dsf[ss] is chunk 4 mt + 2 ss + g of this lane's key, 512 contiguous bytes per half wavefront;
-    // ds_tile points at part (y, x) = (wave >> 1, t & 3) of the block, at this wavefront's 32 keys.  Streaming
-    // stores (the tiles are read once, by another kernel), one under each half of the MFMAs below.  (Holding them
-    // back in LDS until the next sub-tile, so that none is still on its way at the top of the next iteration, where
-    // the wait for the tile loads waits for stores as well, was measured slower.)
-    auto keep = [&](int ss) {
-      typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
-      u32x4* dst = reinterpret_cast<u32x4*>(ds_tile + (unsigned)((4 * mt + 2 * ss + g) * DS_PIECE + i * 8));
-      __builtin_nontemporal_store(__builtin_bit_cast(u32x4, dsf[ss]), dst);
-    };
-    FENCE();
-#pragma unroll
-    for (int n = 0; n < 8; n++) {
-      const int dt = n & 3, ss = n >> 2;
-      if (KEEP_DS && (n == 1 || n == 5)) keep(n >> 2);
-      dv[dt] = mfma32(oif[n % PF], pf[ss], dv[dt]);
-      dk[dt] = mfma32(qif[n % PF], dsf[ss], dk[dt]);
-      if (n + PF < 8) {
-        oif[n % PF] = image_frag(Oi, ibase, (n + PF) & 3, (n + PF) >> 2, mt);
-        qif[n % PF] = image_frag(Qi, ibase, (n + PF) & 3, (n + PF) >> 2, mt);
+      for (; it + 1 < min(w_total, w_full); it++) {
+        bf16* d = kept(it);
+        unit(it, c0, c0, std::false_type{}, d);
+        unit(it, c0, c1, std::false_type{}, d);
+        unit(it, c1, c0, std::false_type{}, d);
+        unit(it, c1, c1, std::false_type{}, d);
       }
-      FENCE();
+      for (; it < w_total; it++) {   // (behind the last tile a unit is formed that nobody uses)
+        bf16* d = kept(it);
+        unit(it, c0, c0, std::true_type{}, d);
+        unit(it, c0, c1, std::true_type{}, d);
+        unit(it, c1, c0, std::true_type{}, d);
+        unit(it, c1, c1, std::true_type{}, d);
+      }
     }
-  };
-
-  for (int it = 0; it < total; it++) {
+    // the other wavefronts' tiles: keep bringing this one's share of them
+    for (; it < total; it++) {
+      load_stats();
+      barrier_images();
+      all_images();
+      barrier_rows();
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        load_rows(j, 0);
+        load_rows(j, 1);
+      }
+    }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    const int t = t_top - (it % ntq);   // last query tile first: the key blocks of an XCD then read the same
-                                              // Q / dO tiles at the same time and share them through L2
-    const bf16* st = ring + (it & 1) * KV_STAGE;
-    // every query of the tile is before every key of this wavefront: nothing to do
-    const bool dead = p.causal && (t * KV_BQ + KV_BQ - 1 + p.off < wn0);
-    const bool masked = p.causal && (t * KV_BQ + p.off < wn0 + 31);
-    bf16* ds_tile = nullptr;
-    if (KEEP_DS) {
-      const int nbq = q_tiles / 4, nbk = p.Lk / KV_BN;
-      ds_tile = p.ds + (((int64_t)b * p.Hq + h_first + it / ntq) * ds_blocks_per_head(nbq, nbk, p.causal) +
-                        ds_block_index(nbq, bc.rank, t >> 2, p.causal)) * DS_BLOCK_ELEMS +
-                (((wave >> 1) * 4 + (t & 3)) * 8) * DS_PIECE + (wave & 1) * 32 * 8;
-    }
-#pragma unroll 1
-    for (int mt = 0; mt < 2; mt++) {
-      // the loads of the next stage go out in two halves, one before each sub-tile: issued all at
-      // once by eight wavefronts they would queue up behind each other at the memory pipeline
-      if (it + 1 < total) load_stage(ring + ((it + 1) & 1) * KV_STAGE, it + 1, mt);
-      if (!dead) sub_tile(st, t, mt, masked, ds_tile);
-    }
   }
 
-  if (SPLIT) {
-    if (key < p.Lk) {
+#pragma unroll
+  for (int kh = 0; kh < KV_KT; kh++) {
+    const int key = wn0 + 32 * kh + i;
+    if (key >= p.Lk) continue;
+    if (SPLIT) {
       // part: [dK | dV][batch][query head][part of the queries][key][D] fp32, unscaled
       float* pk = part + (((int64_t)b * p.Hq * qparts + bc.h) * p.Lk + key) * D;
       float* pv = pk + (int64_t)p.B * p.Hq * qparts * p.Lk * D;
@@ -484,23 +619,23 @@ __global__ __launch_bounds__(KV_THREADS) void attn_bwd_dkdv_pipe_kernel(const At
         for (int a = 0; a < 4; a++) {
           f32x4 wk, wv;
 #pragma unroll
-          for (int e = 0; e < 4; e++) wk[e] = dk[dt][4 * a + e], wv[e] = dv[dt][4 * a + e];
+          for (int e = 0; e < 4; e++) wk[e] = dk[kh][dt][4 * a + e], wv[e] = dv[kh][dt][4 * a + e];
           *reinterpret_cast<f32x4*>(pk + 32 * dt + 8 * a + 4 * g) = wk;
           *reinterpret_cast<f32x4*>(pv + 32 * dt + 8 * a + 4 * g) = wv;
         }
+    } else {
+      bf16* dvp = static_cast<bf16*>(p.dv) + b * p.sdv.b + hk * p.sdv.h + (int64_t)key * p.sdv.l;
+#pragma unroll
+      for (int dt = 0; dt < DT; dt++)
+#pragma unroll
+        for (int a = 0; a < 4; a++) {
+          bf16x4 wv;
+#pragma unroll
+          for (int e = 0; e < 4; e++) wv[e] = (bf16)dv[kh][dt][4 * a + e];
+          *reinterpret_cast<bf16x4*>(dvp + 32 * dt + 8 * a + 4 * g) = wv;
+        }
+      store_dk_row(p, dk[kh], b, hk, key, g);
     }
-  } else if (key < p.Lk) {
-    bf16* dvp = static_cast<bf16*>(p.dv) + b * p.sdv.b + hk * p.sdv.h + (int64_t)key * p.sdv.l;
-#pragma unroll
-    for (int dt = 0; dt < DT; dt++)
-#pragma unroll
-      for (int a = 0; a < 4; a++) {
-        bf16x4 wv;
-#pragma unroll
-        for (int e = 0; e < 4; e++) wv[e] = (bf16)dv[dt][4 * a + e];
-        *reinterpret_cast<bf16x4*>(dvp + 32 * dt + 8 * a + 4 * g) = wv;
-      }
-    store_dk_row(p, dk, b, hk, key, g);
   }
 }
 
@@ -809,7 +944,7 @@ size_t ody_attn_bwd_pipe_ds_bytes(int B, int Lq, int Lk, int Hq, int causal) {
 
 int ody_launch_attn_bwd_pipe(const AttnParams& p, void* workspace, hipStream_t st) {
   constexpr size_t smem_q = (size_t)3 * (2 * TILE_ELEMS + IMG_ELEMS) * sizeof(bf16);
-  constexpr size_t smem_kv = (size_t)2 * KV_STAGE * sizeof(bf16);
+  constexpr size_t smem_kv = (size_t)2 * (KV_ROWS + KV_IMAGES) * sizeof(bf16);
   constexpr size_t smem_qs = (size_t)DQK_LDS_ELEMS * sizeof(bf16);
   static_assert(smem_qs <= 160 * 1024, "LDS of one CU");
   for (const auto& ks : {std::pair<const void*, size_t>{reinterpret_cast<const void*>(&attn_bwd_dq_pipe_kernel), smem_q},
@@ -842,7 +977,9 @@ int ody_launch_attn_bwd_pipe(const AttnParams& p, void* workspace, hipStream_t s
   // dK and dV are the same bits whether dS is kept or not; where that is a choice (rows in multiples of 256), a cut query range keeps a call on
   // the kernels below.  It costs what the others gain: causal, 4 heads, L = 2048 118 us here, 79 there, 8 heads, L = 3584 202 and 135
   const bool same_sums = qparts == 1 || ody_attn_bwd_pipe_ds_bytes(p.B, p.Lq, p.Lk, p.Hq, p.causal) == 0;
-  if (!p.ds && same_sums && ody_attn_bwd_short_ok(p.B, p.Lq, p.Lk, p.Hq, p.causal)) {
+  // rows too far apart for the 32-bit offsets of a tile below: that kernel's are 64 bits wide
+  const bool far = std::max(std::max(p.sq.l, p.sdo.l), std::max(p.sk.l, p.sv.l)) >= TILE_MAX_STRIDE;
+  if (far || (!p.ds && same_sums && ody_attn_bwd_short_ok(p.B, p.Lq, p.Lk, p.Hq, p.causal))) {
     // the pre-pass wrote the query side whole: a later call that reuses it may run on the kernels below
     if ((rc = ody_launch_attn_bwd_short(p, stats, part, st)) || p.group == 1) return rc;
     return group_sum(1);

@@ -42,19 +42,9 @@ using namespace tile128;
 constexpr int D = 128, KS = D / 16, DT = D / 32, BN = 64;
 constexpr int FW_WAVES = 4, FW_QT = 2, FW_BM = 32 * FW_QT * FW_WAVES, FW_THREADS = 64 * FW_WAVES;
 constexpr int FW_SLOTS = 4;                        // of the K ring and of the ring of V^T images
-constexpr int64_t MAX_ROW_STRIDE = (1 << 24) - 8;  // elements: 64 rows of K within 2 GB
 static_assert(FW_WAVES == 4, "the load split and the vmcnt waits assume 4 wavefronts");
 #define FENCE() __builtin_amdgcn_sched_barrier(0)
 #define INLINE __attribute__((always_inline))
-
-// S in ordinary registers: the compiler, which takes accumulation registers for every product of a kernel of this size, would move each score
-// out of them again.  It does not know these for products: whoever reads a score first must stay 19 wait states behind.
-__device__ __forceinline__ void mfma32_first(f32x16& c, bf16x8 a, bf16x8 b) {
-  asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, 0" : "=&v"(c) : "v"(a), "v"(b));
-}
-__device__ __forceinline__ void mfma32_next(f32x16& c, bf16x8 a, bf16x8 b) {
-  asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(c) : "v"(a), "v"(b));
-}
 
 // nsplit > 1: block id = split + nsplit * (the usual id), the block takes part `split` of its tiles; part_out
 // [split][B][Lq][Hq][D] and part_lse [split][B][Hq][Lq] in fp32 take the place of p.out / p.lse.  Under a causal mask a
@@ -103,7 +93,7 @@ __global__ __launch_bounds__(FW_THREADS, 1) void attn_fwd_pipe_kernel(const Attn
   // The direct loads of a K tile and of a V^T image, in four quarters of one instruction per wavefront each: `lk` and `lv` are the tiles being
   // brought (the last one again where there are no more).  Buffer loads: behind loads of the flat kind the compiler waits for all LDS reads in
   // flight in front of each use of one.
-  if (p.sk.l >= MAX_ROW_STRIDE) {   // beyond a tile's 32-bit offsets: left to the kernel behind
+  if (p.sk.l >= TILE_MAX_STRIDE) {   // beyond a tile's 32-bit offsets: left to the kernel behind
     if (tid == 0) atomicOr(bail_flags + ((int64_t)b * p.Hq + h) * nqb + qblk, 1);
     return;
   }
@@ -202,8 +192,8 @@ __global__ __launch_bounds__(FW_THREADS, 1) void attn_fwd_pipe_kernel(const Attn
 #pragma unroll
       for (int qt = 0; qt < FW_QT; qt++) {
         if ((n & 3) == 0 && qt == 0) __builtin_amdgcn_s_waitcnt(LGKM_4);
-        if (n == 0) mfma32_first(s[kt][qt], fr[n % PF], qf[qt][n]);
-        else mfma32_next(s[kt][qt], fr[n % PF], qf[qt][n]);
+        if (n == 0) mfma32_new(s[kt][qt], fr[n % PF], qf[qt][n]);
+        else mfma32_onto(s[kt][qt], fr[n % PF], qf[qt][n]);
         FENCE();
         if (n == 2 && qt == 0) load_k(load);
         if (n == 5 && qt == 0) load_v(load);
@@ -273,8 +263,8 @@ __global__ __launch_bounds__(FW_THREADS, 1) void attn_fwd_pipe_kernel(const Attn
           const bf16x8 f = kfrag(Kt, kt, n);
 #pragma unroll
           for (int qt = 0; qt < FW_QT; qt++)
-            if (n == 0) mfma32_first(s[kt][qt], f, qf[qt][n]);
-            else mfma32_next(s[kt][qt], f, qf[qt][n]);
+            if (n == 0) mfma32_new(s[kt][qt], f, qf[qt][n]);
+            else mfma32_onto(s[kt][qt], f, qf[qt][n]);
         }
       asm volatile("s_nop 15\n\ts_nop 7" : "+v"(s[0][0]), "+v"(s[0][1]), "+v"(s[1][0]), "+v"(s[1][1]));
 #pragma unroll

@@ -28,6 +28,7 @@ constexpr int ROWS = 64;
 constexpr int GROUP_ELEMS = 520;                 // 1040 bytes
 constexpr int TILE_ELEMS = 16 * GROUP_ELEMS;     // 8320 elements = 16640 bytes
 constexpr int TILE_BYTES = TILE_ELEMS * 2;
+constexpr int64_t TILE_MAX_STRIDE = (1 << 24) - 8;   // elements between rows from which on a tile's byte offsets leave 31 bits
 
 // tile row of MFMA row rho of sub-tile kt
 __device__ __forceinline__ int tile_row(int rho, int kt) { return 4 * (rho & 15) + (rho >> 4) + 2 * kt; }
@@ -111,6 +112,19 @@ __device__ __forceinline__ bf16x8 image_frag(const bf16* img, int base, int dt, 
 }
 
 }  // namespace tile128
+
+// Products whose results stay in ordinary registers, for kernels with more than 256: there the compiler takes accumulation registers for every
+// product and moves each score out of them again.  It does not know these for products: whoever reads a result first must stay 19 wait states
+// (three products) behind the last of them.
+__device__ __forceinline__ void mfma32_new(f32x16& d, bf16x8 a, bf16x8 b) {
+  asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, 0" : "=&v"(d) : "v"(a), "v"(b));
+}
+__device__ __forceinline__ void mfma32_from(f32x16& d, bf16x8 a, bf16x8 b, const f32x16& c) {
+  asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %3" : "=&v"(d) : "v"(a), "v"(b), "v"(c));
+}
+__device__ __forceinline__ void mfma32_onto(f32x16& d, bf16x8 a, bf16x8 b) {
+  asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(d) : "v"(a), "v"(b));
+}
 
 // The lane id, recomputed on the spot.  Where every register is spoken for, values derived from
 // it are cheaper to rebuild than to keep (the alternative is a spill to scratch memory, whose
