@@ -1,16 +1,22 @@
 // Flash-attention backward, head_dim 128, bf16, on the tile machinery of attn_tile.h: direct
-// global->LDS loads into a ring of stages, 16-byte LDS reads only (an operand that a product
+// global->LDS loads into rings (buffer loads: behind those of the flat kind the compiler waits for all LDS reads in flight in front of each use
+// of one), 16-byte LDS reads only (an operand that a product
 // contracts over its row index comes from the transposed images a pre-pass writes), fenced slots
-// that keep LDS operand prefetch and MFMAs interleaved.  Two kernels, no atomics: both recompute S
+// that fix the order of MFMAs, LDS reads and vector work.  Two kernels, no atomics: both recompute S
 // from the saved log-sum-exp, and each owns its outputs.
 //
-// dQ kernel -- query-stationary, 8 wavefronts x 32 queries, two per SIMD, lane = query column, so lse and delta
-// are per-lane scalars; a three-deep ring of {K tile, V tile, K^T image}:
+// dQ kernel -- query-stationary, 4 wavefronts x 64 queries, one per SIMD, lane = query column, so lse and delta
+// are per-lane scalars; two-deep rings of {K tile, V tile} and {K^T image}:
 //
 //      S^T = K Q^T            A: K rows (LDS)        B: Q^T (registers)
 //      dP^T = V dO^T          A: V rows (LDS)        B: dO^T (registers)
-//      dS^T = exp2(S^T c - lse) * (dP^T - delta)
+//      dS^T = exp2(S^T c - lse) * (dP^T - delta)      dP^T starts at -delta
 //      dQ^T += K^T dS^T       A: K^T image (LDS)     B: dS^T = accumulator layout
+//
+// A step forms S^T and dP^T of one 32-key sub-tile and then dQ^T of the one before, 16 products each; the vector work of the former runs under
+// the last 32 of them, and every fragment read from LDS serves both halves of the queries.  Bound: power.  Against the kernel before (8 wavefronts of 32 queries,
+// two per SIMD, a tile's parts one after the other), us, one box: 4 heads, L = 32768, causal 1420 / 1227 (constant operands 1076 / 879: the matrix
+// pipe 61 / 75 % busy), 32 heads on 8, L = 16384 2910 / 2512, 4 heads, 8192 queries on 16384 keys 348 / 308.
 //
 // dK/dV kernel -- key-stationary (described where it is defined).
 #include <algorithm>
@@ -47,191 +53,311 @@ __device__ __forceinline__ void store_dq_part(float* __restrict__ dq_part, int p
 // ---------------------------------------------------------------------------------
 // dQ
 // ---------------------------------------------------------------------------------
-constexpr int DQ_QT = 1, DQ_WAVES = 8, DQ_BM = 32 * DQ_QT * DQ_WAVES, DQ_THREADS = 64 * DQ_WAVES;
-static_assert(DQ_WAVES == 8, "the load split and the vmcnt waits assume 8 wavefronts");
+constexpr int DQ_WAVES = 8, DQ_BM = 32 * DQ_WAVES, DQ_THREADS = 64 * DQ_WAVES;   // of the kernel over kept dS
+
+constexpr int DP_WAVES = 4, DP_QT = 2, DP_THREADS = 64 * DP_WAVES, DP_BN = 64;
+constexpr int DP_ROWS = 2 * TILE_ELEMS;                         // a K tile and a V tile
+static_assert(32 * DP_QT * DP_WAVES == DQ_BM, "the same blocks as the kernel over kept dS");
+static_assert(DP_WAVES == 4, "the load split and the vmcnt waits assume 4 wavefronts");
+
+// A product whose second operand lies in accumulation registers, with results in ordinary ones (see mfma32_onto)
+__device__ __forceinline__ void mfma32_from_acc(f32x16& d, bf16x8 a, bf16x8 b, const f32x16& c) {
+  asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %3" : "=&v"(d) : "v"(a), "a"(b), "v"(c));
+}
+__device__ __forceinline__ void mfma32_onto_acc(f32x16& d, bf16x8 a, bf16x8 b) {
+  asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(d) : "v"(a), "a"(b));
+}
 
 // kparts > 1 (too few query blocks for the chip): block id = part + kparts * (the usual id), the block takes part
 // `part` of its key tiles and leaves its unscaled fp32 sum in dq_part.
-__global__ __launch_bounds__(DQ_THREADS) void attn_bwd_dq_pipe_kernel(const AttnParams p,
-                                                                       const bf16* __restrict__ kimg, int kparts,
-                                                                       float* __restrict__ dq_part) {
-  constexpr int BN = 64, QT = DQ_QT;
-  constexpr int STAGE = 2 * TILE_ELEMS + IMG_ELEMS;   // K tile, V tile, K^T image
+__global__ __launch_bounds__(DP_THREADS, 1) void attn_bwd_dq_pipe_kernel(const AttnParams p,
+                                                                          const bf16* __restrict__ kimg, int kparts,
+                                                                          float* __restrict__ dq_part) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
-  bf16* ring = reinterpret_cast<bf16*>(smem_raw);     // [3][STAGE]
+  bf16* rring = reinterpret_cast<bf16*>(smem_raw);   // [2][DP_ROWS]
+  bf16* iring = rring + 2 * DP_ROWS;                 // [2][IMG_ELEMS]
 
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, g = lane >> 5,
             i = lane & 31;
-  simd_stagger(tid);
   const int kpart = blockIdx.x % kparts;
   const BlockCoord bc = ody_block_coord_of(blockIdx.x / kparts, p.Hq, p.B);
   const int nqb = gridDim.x / (p.Hq * p.B * kparts);
   const int qblk = p.causal ? (nqb - 1 - bc.rank) : bc.rank;   // heaviest blocks first
   const int h = bc.h, b = bc.b, hk = h / p.group;
-  const int q0 = qblk * DQ_BM, wq0 = q0 + wave * 32 * QT;
-
-  const bf16* qp = static_cast<const bf16*>(p.q) + b * p.sq.b + h * p.sq.h;
-  const bf16* dop = static_cast<const bf16*>(p.dout) + b * p.sdo.b + h * p.sdo.h;
-  const bf16* kp = static_cast<const bf16*>(p.k) + b * p.sk.b + hk * p.sk.h;
-  const bf16* vp = static_cast<const bf16*>(p.v) + b * p.sv.b + hk * p.sv.h;
-  const int kv_tiles = (p.Lk + BN - 1) / BN;
-  const bf16* kip = kimg + ((int64_t)b * p.Hkv + hk) * kv_tiles * IMG_ELEMS;
+  const int q0 = qblk * DQ_BM, wq0 = q0 + wave * 32 * DP_QT;
 
   const int q_hi = min(q0 + DQ_BM, p.Lq) - 1;
   int n_end = p.causal ? min(p.Lk, q_hi + p.off + 1) : p.Lk;
   if (n_end < 0) n_end = 0;
-  int ntiles = (n_end + BN - 1) / BN;
-  int n_full = p.Lk / BN;   // tiles [0, n_full) need no mask for any wavefront of the block
-  if (p.causal) n_full = min(n_full, max(0, (q0 + p.off + 1) / BN));
-  n_full = min(n_full, ntiles);
+  int ntiles = (n_end + DP_BN - 1) / DP_BN;
   int t_first = 0;   // this block's part of the tiles: [t_first, ntiles)
   if (kparts > 1) {
     const int per = (ntiles + kparts - 1) / kparts;
     t_first = min(kpart * per, ntiles);
     ntiles = min(t_first + per, ntiles);
   }
+  // end of those that this wavefront's queries see a key of, and of those that they see whole
+  int w_end = ntiles, w_full = p.Lk / DP_BN;
+  if (p.causal) {
+    w_end = min(ntiles, max(t_first, (wq0 + 32 * DP_QT - 1 + p.off + DP_BN) / DP_BN));
+    w_full = min(w_full, max(0, wq0 + p.off + 1) / DP_BN);
+  }
 
-  auto load_part = [&](bf16* st, int t, int j) {   // j = 0, 1: the two halves of a stage's loads
-    {
-      const int grp = DQ_WAVES * j + wave;
-      int row = t * BN + 4 * grp + (lane >> 4);
-      row = row < p.Lk ? row : p.Lk - 1;
-      const int col = 8 * (lane & 15);
-      __builtin_amdgcn_global_load_lds((global_void_ptr)(kp + (int64_t)row * p.sk.l + col),
-                                       (lds_void_ptr)(st + grp * GROUP_ELEMS), 16, 0, 0);
-      __builtin_amdgcn_global_load_lds((global_void_ptr)(vp + (int64_t)row * p.sv.l + col),
-                                       (lds_void_ptr)(st + TILE_ELEMS + grp * GROUP_ELEMS), 16, 0, 0);
-      __builtin_amdgcn_global_load_lds((global_void_ptr)(kip + (int64_t)t * IMG_ELEMS + (grp * 64 + lane) * 8),
-                                       (lds_void_ptr)(st + 2 * TILE_ELEMS + grp * 512), 16, 0, 0);
-    }
-  };
-  auto load_stage = [&](bf16* st, int t) {
-    load_part(st, t, 0);
-    load_part(st, t, 1);
-  };
-  if (t_first < ntiles) load_stage(ring, t_first);
-  if (t_first + 1 < ntiles) load_stage(ring + STAGE, t_first + 1);
-
-  bf16x8 qf[QT][KS], dof[QT][KS];
-  float lse2[QT], delta[QT];
-  int lim[QT];
+  bf16x8 qf[DP_QT][KS], dof[DP_QT][KS];
+  f32x16 minus_delta[DP_QT];   // what dP starts from
+  float lse2[DP_QT];
+  int lim[DP_QT];
+  {
+    const bf16* qp = static_cast<const bf16*>(p.q) + b * p.sq.b + h * p.sq.h;
+    const bf16* dop = static_cast<const bf16*>(p.dout) + b * p.sdo.b + h * p.sdo.h;
 #pragma unroll
-  for (int qt = 0; qt < QT; qt++) {
-    const int qi = wq0 + 32 * qt + i;
+    for (int qt = 0; qt < DP_QT; qt++) {
+      const int qi = wq0 + 32 * qt + i;
 #pragma unroll
-    for (int ks = 0; ks < KS; ks++) {
-      if (qi < p.Lq) {
-        qf[qt][ks] = *reinterpret_cast<const bf16x8*>(qp + (int64_t)qi * p.sq.l + 16 * ks + 8 * g);
-        dof[qt][ks] = *reinterpret_cast<const bf16x8*>(dop + (int64_t)qi * p.sdo.l + 16 * ks + 8 * g);
-      } else {
-        qf[qt][ks] = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
-        dof[qt][ks] = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
+      for (int ks = 0; ks < KS; ks++) {
+        qf[qt][ks] = dof[qt][ks] = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
+        if (qi < p.Lq) {
+          qf[qt][ks] = *reinterpret_cast<const bf16x8*>(qp + (int64_t)qi * p.sq.l + 16 * ks + 8 * g);
+          dof[qt][ks] = *reinterpret_cast<const bf16x8*>(dop + (int64_t)qi * p.sdo.l + 16 * ks + 8 * g);
+        }
       }
+      const int64_t ri = ((int64_t)b * p.Hq + h) * p.Lq + qi;
+      float l = (qi < p.Lq) ? p.lse[ri] : INFINITY;
+      if (l == -INFINITY) l = INFINITY;   // a query that saw no key: P = 0
+      lse2[qt] = l * ODY_LOG2E;
+      const float delta = (qi < p.Lq) ? p.delta[ri] : 0.f;
+#pragma unroll
+      for (int r = 0; r < 16; r++) minus_delta[qt][r] = -delta;
+      lim[qt] = p.causal ? min(p.Lk - 1, qi + p.off) : p.Lk - 1;
     }
-    const int64_t ri = ((int64_t)b * p.Hq + h) * p.Lq + qi;
-    float l = (qi < p.Lq) ? p.lse[ri] : INFINITY;
-    if (l == -INFINITY) l = INFINITY;   // a query that saw no key: P = 0
-    lse2[qt] = l * ODY_LOG2E;
-    delta[qt] = (qi < p.Lq) ? p.delta[ri] : 0.f;
-    lim[qt] = p.causal ? min(p.Lk - 1, qi + p.off) : p.Lk - 1;
+  }
+#pragma unroll
+  for (int qt = 0; qt < DP_QT; qt++) {
+    asm volatile("" : "+v"(minus_delta[qt]), "+v"(lse2[qt]));   // arrived before the direct loads
+#pragma unroll
+    for (int ks = 0; ks < KS; ks++) asm volatile("" : "+v"(qf[qt][ks]), "+a"(dof[qt][ks]));
   }
   const float c2 = p.scale_log2e;
-  const int rbase = row_frag_base(g, i), ibase = image_frag_base(g, i);
 
-  f32x16 dq[QT][DT];
+  // Direct loads: of the rows of tile `lr` and of the image of tile `li`, the last one again where there are no more.  Rows past the end read
+  // zeros: they lie beyond the descriptor.
+  int lr = min(t_first, ntiles - 1), li = lr;
+  const int krow = 2 * (int)p.sk.l, vrow = 2 * (int)p.sv.l;   // bytes
+  const int klane = (4 * wave + (lane >> 4)) * krow + 16 * (lane & 15), vlane = (4 * wave + (lane >> 4)) * vrow + 16 * (lane & 15);
+  const int ilane = 1024 * wave + 16 * lane;
+  const bf16* ktp = static_cast<const bf16*>(p.k) + b * p.sk.b + hk * p.sk.h + (int64_t)lr * DP_BN * p.sk.l;
+  const bf16* vtp = static_cast<const bf16*>(p.v) + b * p.sv.b + hk * p.sv.h + (int64_t)lr * DP_BN * p.sv.l;
+  const bf16* kip = kimg + (((int64_t)b * p.Hkv + hk) * ((p.Lk + DP_BN - 1) / DP_BN) + lr) * IMG_ELEMS;
+  int room = p.Lk - lr * DP_BN;   // rows from the tile's first one on
+  auto bring = [&](const bf16* src, int bytes, bf16* dst, int off, int soff) INLINE {
+    auto rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16*>(src), (short)0, bytes, 0x00020000);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_void_ptr)dst, 16, off, soff, 0, 0);
+  };
+  auto load_rows = [&](int j, int which) INLINE {   // a quarter j of the K tile, of the V tile
+    bf16* dst = rring + (lr & 1) * DP_ROWS + (4 * j + wave) * GROUP_ELEMS;
+    const int last = min(room, DP_BN) - 1;
+    if (which == 0) bring(ktp, last * krow + 256, dst, klane + 16 * j * krow, 0);
+    else bring(vtp, last * vrow + 256, dst + TILE_ELEMS, vlane + 16 * j * vrow, 0);
+  };
+  auto load_image = [&](int j) INLINE { bring(kip, IMG_BYTES, iring + (li & 1) * IMG_ELEMS + (4 * j + wave) * 512, ilane, 4096 * j); };
+  auto next_rows = [&]() INLINE {
+    const int to = min(lr + 1, ntiles - 1), step = to - lr;
+    lr = to;
+    ktp += (int64_t)step * (DP_BN / 2 * krow);
+    vtp += (int64_t)step * (DP_BN / 2 * vrow);
+    room -= step * DP_BN;
+  };
+  auto next_image = [&]() INLINE {
+    const int to = min(li + 1, ntiles - 1), step = to - li;
+    li = to;
+    kip += step * IMG_ELEMS;
+  };
+
+  const int rbase = row_frag_base(g, i), ibase = image_frag_base(g, i);
+  f32x16 dq[DP_QT][DT];
 #pragma unroll
-  for (int qt = 0; qt < QT; qt++)
+  for (int qt = 0; qt < DP_QT; qt++)
 #pragma unroll
     for (int dt = 0; dt < DT; dt++)
 #pragma unroll
       for (int r = 0; r < 16; r++) dq[qt][dt][r] = 0.f;
-
-  // One 64-key tile against this wavefront's 32 queries, as two 32-key sub-tiles kt = 0, 1 with their
-  // own accumulation chains: 32 MFMAs for S^T and dP^T, the vector work, 16 MFMAs for dQ^T.
-  auto tile = [&](const bf16* st, int t, bool masked) {
-    const bf16* Kt = st;
-    const bf16* Vt = st + TILE_ELEMS;
-    const bf16* Ki = st + 2 * TILE_ELEMS;
-    constexpr int PF = 2;
-    bf16x8 kfr[PF][2], vfr[PF][2];
-#pragma unroll
-    for (int n = 0; n < PF; n++)
-#pragma unroll
-      for (int kt = 0; kt < 2; kt++) {
-        kfr[n][kt] = row_frag(Kt, rbase, n, kt);
-        vfr[n][kt] = row_frag(Vt, rbase, n, kt);
-      }
-    f32x16 s[2], dp[2];
-    FENCE();
-#pragma unroll
-    for (int ks = 0; ks < KS; ks++) {
-#pragma unroll
-      for (int kt = 0; kt < 2; kt++) {
-        if (ks == 0) {
-          s[kt] = mfma32(kfr[0][kt], qf[0][0], f32x16{0});
-          dp[kt] = mfma32(vfr[0][kt], dof[0][0], f32x16{0});
-        } else {
-          s[kt] = mfma32(kfr[ks % PF][kt], qf[0][ks], s[kt]);
-          dp[kt] = mfma32(vfr[ks % PF][kt], dof[0][ks], dp[kt]);
-        }
-      }
-      if (ks + PF < KS) {
-#pragma unroll
-        for (int kt = 0; kt < 2; kt++) {
-          kfr[ks % PF][kt] = row_frag(Kt, rbase, ks + PF, kt);
-          vfr[ks % PF][kt] = row_frag(Vt, rbase, ks + PF, kt);
-        }
-      }
-      FENCE();
-    }
-    constexpr int IPF = 4;
-    bf16x8 ifr[IPF];
-#pragma unroll
-    for (int n = 0; n < IPF; n++) ifr[n] = image_frag(Ki, ibase, n & 3, 0, 0);
-    if (masked) {
-#pragma unroll
-      for (int kt = 0; kt < 2; kt++)
-#pragma unroll
-        for (int r = 0; r < 16; r++)
-          if (t * BN + acc_tile_row(r, g, kt) > lim[0]) s[kt][r] = -INFINITY;
-    }
-    bf16x8 dsf[2][2];
-#pragma unroll
-    for (int kt = 0; kt < 2; kt++)
-#pragma unroll
-      for (int r = 0; r < 16; r++) {
-        const float pr = ody_exp2(fmaf(s[kt][r], c2, -lse2[0]));
-        dsf[kt][r >> 3][r & 7] = (bf16)(pr * (dp[kt][r] - delta[0]));
-      }
-    FENCE();
-#pragma unroll
-    for (int n = 0; n < 16; n++) {
-      const int dt = n & 3, ss = (n >> 2) & 1, kt = n >> 3;
-      dq[0][dt] = mfma32(ifr[n % IPF], dsf[kt][ss], dq[0][dt]);
-      if (n + IPF < 16) {
-        const int m = n + IPF;
-        ifr[n % IPF] = image_frag(Ki, ibase, m & 3, (m >> 2) & 1, m >> 3);
-      }
-      FENCE();
-    }
+  f32x16 s[DP_QT], dp[DP_QT];            // S, then P; dP, then dS
+  bf16x8 dsf[DP_QT][2], dsf_next[DP_QT][2];
+  // the steps of element e (query half e >> 4, register e & 15) of a sub-tile
+  auto exponent = [&](int e, int t, int kt, auto masked) INLINE {
+    const int qt = e >> 4, r = e & 15;
+    float x = s[qt][r];
+    if (decltype(masked)::value) x = t * DP_BN + acc_tile_row(r, g, kt) > lim[qt] ? -INFINITY : x;
+    s[qt][r] = fmaf(x, c2, -lse2[qt]);
+  };
+  auto weight = [&](int e) INLINE { s[e >> 4][e & 15] = ody_exp2(s[e >> 4][e & 15]); };
+  auto ds = [&](int e) INLINE { dp[e >> 4][e & 15] *= s[e >> 4][e & 15]; };
+  auto pack = [&](int q) INLINE {   // elements 2 q and 2 q + 1
+    const int qt = q >> 3, r = 2 * (q & 7);
+    dsf_next[qt][r >> 3][r & 7] = (bf16)dp[qt][r], dsf_next[qt][r >> 3][(r & 7) + 1] = (bf16)dp[qt][r + 1];
+  };
+  constexpr int LGKM_4 = 0xc47f;   // s_waitcnt lgkmcnt(4): with the reads behind them in the order below, half of `fr` is there
+  bf16x8 fr[8];
+  auto kfrag = [&](const bf16* rows, int kt, int n) INLINE { return row_frag(rows, rbase, n, kt); };                 // k-step n
+  auto vfrag = [&](const bf16* rows, int kt, int n) INLINE { return row_frag(rows + TILE_ELEMS, rbase, n, kt); };
+  auto ifrag = [&](const bf16* im, int kt, int n) INLINE { return image_frag(im, ibase, n & 3, n >> 2, kt); };      // k-step n >> 2, columns 32 (n & 3)
+  auto rslot = [&](int t) INLINE { return rring + (t & 1) * DP_ROWS; };
+  auto islot = [&](int t) INLINE { return iring + (t & 1) * IMG_ELEMS; };
+  auto barrier_rows = [&]() INLINE {     // the rows of the next tile have landed (behind them 4 loads of an image); everyone is done with those before
+    asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    next_rows();
+  };
+  auto barrier_image = [&]() INLINE {    // likewise the image (behind it 8 loads of rows)
+    asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    next_image();
   };
 
-  for (int t = t_first; t < ntiles; t++) {
-    // stage t landed (the loads of stage t+1 may still be in flight), everyone done with stage t-1
-    if (t + 1 < ntiles) {
-      asm volatile("s_waitcnt vmcnt(6)" ::: "memory");
-    } else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    const bf16* st = ring + ((t - t_first) % 3) * STAGE;
-    const bool dead = p.causal && t * BN > wq0 + 32 * QT - 1 + p.off;   // every key of the tile is after this wavefront's queries
-    if (!dead) tile(st, t, t >= n_full);
-    // the loads go last: issuing them costs this wavefront time, and here it would otherwise wait at the barrier
-    if (t + 2 < ntiles) load_part(ring + ((t + 2 - t_first) % 3) * STAGE, t + 2, 0);
-    if (t + 2 < ntiles) load_part(ring + ((t + 2 - t_first) % 3) * STAGE, t + 2, 1);
+  // One step: S and dP of the sub-tile after (tile t, sub-tile KT), then dQ of this one: three parts of 16 products, with the vector work of the
+  // sub-tile after under the last two.  A fragment serves both halves of the queries; `fr` holds those of a part when it begins and is left
+  // with those of the next.
+  auto step = [&](int t, auto kt_, auto masked) INLINE {
+    constexpr int KT = decltype(kt_)::value, NKT = KT ^ 1;
+    const int nt = KT ? t + 1 : t;
+    const bf16 *rows = rslot(nt), *after = rslot(t + 1), *image = islot(t);   // after: of the sub-tile behind the next one
+#pragma unroll
+    for (int m = 0; m < 16; m++) {
+      const int n = m >> 1, qt = m & 1;
+      if ((m & 7) == 0) __builtin_amdgcn_s_waitcnt(LGKM_4);
+      if (n == 0) mfma32_new(s[qt], fr[n], qf[qt][n]);
+      else mfma32_onto(s[qt], fr[n], qf[qt][n]);
+      FENCE();
+      if (qt == 1) fr[n] = vfrag(rows, NKT, n);
+      if (KT == 1 && (m & 7) == 4) load_rows(1, m >> 3);
+      FENCE();
+    }
+    if (KT == 0) barrier_image();
+#pragma unroll
+    for (int m = 0; m < 16; m++) {
+      const int n = m >> 1, qt = m & 1;
+      if ((m & 7) == 0) __builtin_amdgcn_s_waitcnt(LGKM_4);
+      if (n == 0) mfma32_from_acc(dp[qt], fr[n], dof[qt][n], minus_delta[qt]);
+      else mfma32_onto_acc(dp[qt], fr[n], dof[qt][n]);
+      FENCE();
+      if (qt == 1) fr[n] = ifrag(image, KT, n);
+      if (m >= 3) weight(2 * m - 6), weight(2 * m - 5);
+      if (m >= 2) exponent(2 * m - 4, nt, NKT, masked), exponent(2 * m - 3, nt, NKT, masked);   // (S is 3 products old)
+      if (KT == 0 && (m & 3) == 1) load_image(m >> 2);
+      if (KT == 1 && (m & 7) == 4) load_rows(2, m >> 3);
+      FENCE();
+    }
+    if (KT == 0) barrier_rows();
+#pragma unroll
+    for (int m = 0; m < 16; m++) {
+      const int n = m >> 1, qt = m & 1;
+      if ((m & 7) == 0) __builtin_amdgcn_s_waitcnt(LGKM_4);
+      dq[qt][n & 3] = mfma32(fr[n], dsf[qt][n >> 2], dq[qt][n & 3]);
+      FENCE();
+      if (qt == 1) fr[n] = kfrag(KT ? rslot(t + 1) : after, KT, n);
+      if (m <= 2) weight(2 * m + 26), weight(2 * m + 27);
+      if (m <= 1) exponent(2 * m + 28, nt, NKT, masked), exponent(2 * m + 29, nt, NKT, masked);
+      if (m >= 2) {   // all of dS and its operands before the next part takes the registers of S
+#pragma unroll
+        for (int e = 0; e < 3; e++)
+          if (3 * (m - 2) + e < 32) ds(3 * (m - 2) + e);
+      }
+      if (m >= 4) {
+        if (m < 12) pack(m - 4);
+        else pack(2 * m - 16), pack(2 * m - 15);
+      }
+      if (KT == 0 && (m & 7) == 4) load_rows(0, m >> 3);
+      if (KT == 1 && (m & 7) == 4) load_rows(3, m >> 3);
+      FENCE();
+    }
+#pragma unroll
+    for (int qt = 0; qt < DP_QT; qt++)
+#pragma unroll
+      for (int ss = 0; ss < 2; ss++) dsf[qt][ss] = dsf_next[qt][ss];
+  };
+  std::integral_constant<int, 0> c0;
+  std::integral_constant<int, 1> c1;
+
+  if (t_first < ntiles) {
+    auto all_rows = [&]() INLINE {
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        load_rows(j, 0);
+        load_rows(j, 1);
+      }
+    };
+    auto all_image = [&]() INLINE {
+#pragma unroll
+      for (int j = 0; j < 4; j++) load_image(j);
+    };
+    all_rows();
+    all_image();
+    next_rows();
+    all_rows();
+    asm volatile("s_waitcnt vmcnt(12)" ::: "memory");   // the first tile's rows
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    int t = t_first;
+    if (t < w_end) {
+      // S, P, dP and dS of the first sub-tile
+      const bf16* rows = rslot(t);
+#pragma unroll
+      for (int n = 0; n < 8; n++) {
+        const bf16x8 fk = kfrag(rows, 0, n), fv = vfrag(rows, 0, n);
+#pragma unroll
+        for (int qt = 0; qt < DP_QT; qt++) {
+          if (n == 0) {
+            mfma32_new(s[qt], fk, qf[qt][n]);
+            mfma32_from_acc(dp[qt], fv, dof[qt][n], minus_delta[qt]);
+          } else {
+            mfma32_onto(s[qt], fk, qf[qt][n]);
+            mfma32_onto_acc(dp[qt], fv, dof[qt][n]);
+          }
+        }
+      }
+      asm volatile("s_nop 15\n\ts_nop 7" : "+v"(s[0]), "+v"(s[1]), "+v"(dp[0]), "+v"(dp[1]));
+#pragma unroll
+      for (int e = 0; e < 32; e++) {
+        exponent(e, t, 0, std::true_type{});
+        weight(e);
+        ds(e);
+      }
+#pragma unroll
+      for (int q = 0; q < 16; q++) pack(q);
+#pragma unroll
+      for (int qt = 0; qt < DP_QT; qt++)
+#pragma unroll
+        for (int ss = 0; ss < 2; ss++) dsf[qt][ss] = dsf_next[qt][ss];
+#pragma unroll
+      for (int n = 0; n < 8; n++) fr[n] = kfrag(rows, 1, n);
+      FENCE();
+      for (; t + 1 < min(w_end, w_full); t++) {
+        step(t, c0, std::false_type{});
+        step(t, c1, std::false_type{});
+      }
+      for (; t < w_end; t++) {   // (behind the last tile a sub-tile is formed that nobody uses)
+        step(t, c0, std::true_type{});
+        step(t, c1, std::true_type{});
+      }
+    }
+    // the other wavefronts' tiles: keep bringing this one's share of them
+    for (; t < ntiles; t++) {
+      barrier_image();
+      all_image();
+      barrier_rows();
+      all_rows();
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   }
 
-  if (kparts > 1) store_dq_part(dq_part, kpart, p, dq[0], b, h, wq0 + i, g);
-  else store_dq_row(p, dq[0], b, h, wq0 + i, g);
+#pragma unroll
+  for (int qt = 0; qt < DP_QT; qt++) {
+    const int qi = wq0 + 32 * qt + i;
+    if (kparts > 1) store_dq_part(dq_part, kpart, p, dq[qt], b, h, qi, g);
+    else store_dq_row(p, dq[qt], b, h, qi, g);
+  }
 }
 
 // ---------------------------------------------------------------------------------
@@ -943,7 +1069,7 @@ size_t ody_attn_bwd_pipe_ds_bytes(int B, int Lq, int Lk, int Hq, int causal) {
 }
 
 int ody_launch_attn_bwd_pipe(const AttnParams& p, void* workspace, hipStream_t st) {
-  constexpr size_t smem_q = (size_t)3 * (2 * TILE_ELEMS + IMG_ELEMS) * sizeof(bf16);
+  constexpr size_t smem_q = (size_t)2 * (DP_ROWS + IMG_ELEMS) * sizeof(bf16);
   constexpr size_t smem_kv = (size_t)2 * (KV_ROWS + KV_IMAGES) * sizeof(bf16);
   constexpr size_t smem_qs = (size_t)DQK_LDS_ELEMS * sizeof(bf16);
   static_assert(smem_qs <= 160 * 1024, "LDS of one CU");
@@ -1018,7 +1144,7 @@ int ody_launch_attn_bwd_pipe(const AttnParams& p, void* workspace, hipStream_t s
     return ody_check_launch("attn_bwd_dq_sum");
   }
   const int kparts = key_parts(p.B, p.Lq, p.Lk, p.Hq, p.causal != 0);
-  ODY_LAUNCH("attn_bwd_dq_pipe", st, attn_bwd_dq_pipe_kernel, dim3(gq.x * kparts), dim3(DQ_THREADS), smem_q, p, kimg, kparts,
+  ODY_LAUNCH("attn_bwd_dq_pipe", st, attn_bwd_dq_pipe_kernel, dim3(gq.x * kparts), dim3(DP_THREADS), smem_q, p, kimg, kparts,
              part);
   if ((rc = ody_check_launch("attn_bwd_dq_pipe")) || kparts == 1) return rc;
   const int64_t n8 = (int64_t)p.B * p.Lq * p.Hq * (D / 8);

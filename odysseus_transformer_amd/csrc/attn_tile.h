@@ -2,7 +2,7 @@
 // global->LDS loads and read with 16-byte reads, without bank conflicts and with purely
 // additive addressing.
 //
-// A direct load (global_load_lds_dwordx4) makes the 64 lanes of a wavefront write
+// A direct load (buffer_load_dwordx4 with the LDS bit) makes the 64 lanes of a wavefront write
 // 64 consecutive 16-byte slots of LDS, each lane fetching from its own global
 // address.  One such load brings a GROUP of 4 consecutive tile rows (4 x 256 B), row
 // after row; groups are 1040 bytes apart (1024 + 16 of padding).  Hence, in elements,
@@ -40,22 +40,6 @@ __device__ __forceinline__ int acc_tile_row(int r, int g, int kt) {
 }
 
 typedef __attribute__((address_space(3))) void* lds_void_ptr;
-typedef __attribute__((address_space(1))) const void* global_void_ptr;
-
-// Issues this thread's share of the direct loads of one 64 x 128 tile: 4 loads of
-// 16 bytes (256 threads).  `base` points at row 0 of the matrix for this (batch, head);
-// rows at or beyond `nrows` re-read row nrows-1 (finite filler that the caller masks).
-__device__ __forceinline__ void load_tile_async(bf16* lds_tile, const bf16* base, int64_t row_stride, int row0,
-                                                int nrows, int wave, int lane) {
-#pragma unroll
-  for (int j = 0; j < 4; j++) {
-    const int grp = 4 * j + wave;
-    int row = row0 + 4 * grp + (lane >> 4);
-    row = row < nrows ? row : nrows - 1;
-    const bf16* src = base + (int64_t)row * row_stride + 8 * (lane & 15);
-    __builtin_amdgcn_global_load_lds((global_void_ptr)src, (lds_void_ptr)(lds_tile + grp * GROUP_ELEMS), 16, 0, 0);
-  }
-}
 
 // Per-lane element offset of the row-wise operand: MFMA row i, k = 8g..8g+7 of k-step 0,
 // sub-tile 0.  Add ks*16 + kt*KT_ELEMS elements for k-step ks of sub-tile kt.
@@ -94,15 +78,6 @@ __host__ __device__ __forceinline__ int image_pos(int row) {
   return 8 * (4 * kt + 2 * ss + g) + j;
 }
 
-__device__ __forceinline__ void load_image_async(bf16* lds_img, const bf16* img, int wave, int lane) {
-#pragma unroll
-  for (int j = 0; j < 4; j++) {
-    const int off = ((4 * j + wave) * 64 + lane) * 8;
-    __builtin_amdgcn_global_load_lds((global_void_ptr)(img + off), (lds_void_ptr)(lds_img + (4 * j + wave) * 512), 16,
-                                     0, 0);
-  }
-}
-
 // Per-lane element offset of the A operand read from an image: MFMA row i <-> d = 32*dt + i.
 // Add dt*2048 + (4*kt + 2*ss)*128 elements.
 __device__ __forceinline__ int image_frag_base(int g, int i) { return (i >> 4) * 1024 + (i & 15) * 8 + g * 128; }
@@ -124,34 +99,6 @@ __device__ __forceinline__ void mfma32_from(f32x16& d, bf16x8 a, bf16x8 b, const
 }
 __device__ __forceinline__ void mfma32_onto(f32x16& d, bf16x8 a, bf16x8 b) {
   asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(d) : "v"(a), "v"(b));
-}
-
-// The lane id, recomputed on the spot.  Where every register is spoken for, values derived from
-// it are cheaper to rebuild than to keep (the alternative is a spill to scratch memory, whose
-// reload then waits behind the tile loads in flight).
-__device__ __forceinline__ int fresh_lane() {
-  int ln;
-  asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(ln));
-  return ln;
-}
-
-// Two wavefronts of a workgroup share each SIMD.  Started together and re-aligned by every
-// workgroup barrier they run in lockstep -- both in their matrix phase, then both in their
-// vector phase -- and the matrix pipe idles half of the time.  Raising the priority of the
-// first wavefront to arrive on each SIMD breaks the symmetry: it runs ahead, and the other
-// one fills the matrix pipe while the first is in its vector phase.
-// Order of arrival of this wavefront among those of its workgroup on the same SIMD (0, 1, ...).
-__device__ __forceinline__ int simd_rank(int tid) {
-  __shared__ int simd_count[4];
-  if (tid < 4) simd_count[tid] = 0;
-  __syncthreads();
-  const int simd = __builtin_amdgcn_s_getreg((1 << 11) | (4 << 6) | 4) & 3;   // HW_ID.SIMD_ID
-  int rank = 0;
-  if ((tid & 63) == 0) rank = atomicAdd(&simd_count[simd], 1);
-  return __builtin_amdgcn_readfirstlane(rank);
-}
-__device__ __forceinline__ void simd_stagger(int tid) {
-  if (simd_rank(tid) == 0) __builtin_amdgcn_s_setprio(2);
 }
 
 // Swap of the two wavefront halves through v_permlane32_swap: returns, in every lane,
