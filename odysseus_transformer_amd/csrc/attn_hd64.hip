@@ -14,6 +14,8 @@
 // takes every other tile; the sets add up through LDS at the end.  It is for calls with too few blocks to give every SIMD three
 // wavefronts.
 //
+// Where there are blocks enough, the forward takes the kernel of attn_hd64_pipe.hip (dispatch: end of this file).
+//
 // Tiles and fragments: attn_rowtile.h.
 //
 // Measured against the kernels these replace (register-staged tiles through padded LDS rows, rescaling on every tile, one block per
@@ -39,16 +41,6 @@ constexpr int D = 64, KS = D / 16, DT = D / 32, TILE = ROWS * D;   // elements o
 constexpr int BLOCK_ROWS = 128;
 typedef TileLoader<D, 4> Loader;
 
-// Blocks heaviest first, all (head, batch) pairs of a rank together (ody_block_coord), and under a causal mask every other run
-// of 256 blocks with its ranks reversed: the three or four blocks that share a compute unit then add up to about the same
-// length.  In plain order the units with the first blocks of every run got 320 tiles where the mean was 260 (forward of 16 heads,
-// L = 8192: 182 us, 158 this way).
-__device__ __forceinline__ BlockCoord block_coord(int H, int B, int causal) {
-  BlockCoord c = ody_block_coord(H, B);
-  const int ranks = gridDim.x / (H * B), run = max(1, 256 / (H * B)), n = c.rank / run;
-  if (causal && (n & 1) && (n + 1) * run <= ranks) c.rank = n * run + run - 1 - c.rank % run;
-  return c;
-}
 constexpr size_t KV_STAGE = 2 * TILE;                    // elements: two tiles
 constexpr size_t QS_STAGE = 2 * TILE + 2 * 2 * ROWS;     // Q and dO tiles, -lse / scale and -delta of their rows in fp32
 static_assert(2 * 2 * KV_STAGE * sizeof(bf16) >= 4 * 34 * 64 * sizeof(float) && 2 * 2 * QS_STAGE * sizeof(bf16) >= 4 * 64 * 64 * sizeof(float),
@@ -545,9 +537,25 @@ int launch(const char* name, K kern, int64_t blocks, int groups, size_t stage_el
   return ody_check_launch(name);
 }
 
+// The kernels of attn_hd64_pipe.hip address a tile with 32-bit byte offsets.
+inline bool near(const AttnStrides& a, const AttnStrides& b) { return a.l < tile128::TILE_MAX_STRIDE && b.l < tile128::TILE_MAX_STRIDE; }
+
+// The forward with 256-row blocks, two to a compute unit, where they fill the chip.  Before / with it, us: full, 16 heads, L = 8192, 308 / 265;
+// 4 x 32 heads, L = 1000, 48.6 / 44.3; 16 heads, L = 4096, 256 blocks, 89 / 82; 12 heads of that, 192 blocks, 75 / 81; 4 x 32 heads, L = 512,
+// 16.8 / 16.7.  Causal, where one block is many times as long as another, only with three blocks for every unit or more and, since every block
+// has a prologue, long rows: 24 heads, L = 8192, 239 / 219; 32 heads, L = 2048 x 4, 91.7 / 89.3; 16 heads, L = 8192, 512 blocks, 179 / 173 by
+// itself and 5 us behind before a backward; 16 heads, L = 2048 x 4, 512 blocks, 49.1 / 50.1; 24 heads, L = 4096, 384 blocks, 76 / 79;
+// 64 x 16 heads, L = 256, 36.2 / 37.2.  A last block that is half empty costs its share of the rows.
+inline bool fwd_pipe_ok(const AttnParams& p) {
+  const int64_t halves = (p.Lq + BLOCK_ROWS - 1) / BLOCK_ROWS, blocks = (int64_t)p.B * p.Hq * ((halves + 1) / 2);
+  if (!near(p.sk, p.sv) || ((halves & 1) && halves < 16)) return false;
+  return p.causal ? blocks >= 768 && blocks * p.Lk >= (1 << 21) : blocks >= 256 && p.Lk >= 512;
+}
+
 }  // namespace
 
 int ody_launch_attn_fwd_hd64(const AttnParams& p, hipStream_t st) {
+  if (fwd_pipe_ok(p)) return ody_launch_attn_fwd_hd64_pipe(p, st);
   const int64_t blocks = row_blocks(p.B, p.Lq, p.Hq);
   return blocks < FEW_BLOCKS ? launch("attn_fwd_hd64", &attn_fwd_hd64_kernel<2>, blocks, 2, KV_STAGE, st, p)
                              : launch("attn_fwd_hd64", &attn_fwd_hd64_kernel<1>, blocks, 1, KV_STAGE, st, p);

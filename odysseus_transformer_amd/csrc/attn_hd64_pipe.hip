@@ -1,0 +1,364 @@
+// Flash attention for bf16 and head_dim 64 where there are blocks enough for the whole chip: the arithmetic, tiles and fragments of
+// attn_hd64.hip in the order of attn_fwd_pipe.hip -- the vector work of one sub-tile under the products of another,
+// instead of left to whichever wavefront of a SIMD has some.
+#include <cfloat>
+#include <type_traits>
+#include "attn_rowtile.h"
+
+namespace {
+
+using namespace rowtile;
+
+constexpr int D = 64, KS = D / 16, DT = D / 32, TILE = ROWS * D;   // elements of a tile: 8 KB
+#define FENCE() __builtin_amdgcn_sched_barrier(0)
+#define INLINE __attribute__((always_inline))
+
+// Direct loads of one matrix's 64-row tiles, in two halves of one instruction per wavefront each (4 wavefronts).  Rows past the end read
+// zeros: they lie beyond the descriptor.
+struct Bringer {
+  int row_bytes, lane_off;
+  __device__ __forceinline__ void init(int64_t stride, int wave, int lane) {
+    const int row = 8 * wave + (lane >> 3);
+    row_bytes = 2 * (int)stride;
+    lane_off = row * row_bytes + 16 * ((lane & 7) ^ swz<D>(row));
+  }
+  // src: the tile's first row; rows: how many are left from there on; j: half
+  __device__ __forceinline__ void load(bf16* tile, const bf16* src, int rows, int j, int wave) const {
+    auto rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16*>(src), (short)0, (min(rows, ROWS) - 1) * row_bytes + 2 * D, 0x00020000);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_ptr)(tile + (4 * j + wave) * 512), 16, lane_off + 32 * j * row_bytes, 0, 0, 0);
+  }
+};
+
+// A transposed fragment (tr_frags) whose reads are still under way: 16 rows from OFF / 128 on, 32 columns by the address pair
+struct TrFrag {
+  s16x4 lo, hi;
+};
+template <int FIRST>
+__device__ __forceinline__ void read_tr(TrFrag& f, unsigned a0, unsigned a1) {
+  asm volatile("ds_read_b64_tr_b16 %0, %2 offset:%4\n\tds_read_b64_tr_b16 %1, %3 offset:%5"
+               : "=&v"(f.lo), "=&v"(f.hi)
+               : "v"(a0), "v"(a1), "n"(2 * FIRST * D), "n"(2 * (FIRST + 8) * D));
+}
+// behind the wait for them
+__device__ __forceinline__ void tie(TrFrag& f) { asm volatile("" : "+v"(f.lo), "+v"(f.hi)); }
+__device__ __forceinline__ bf16x8 value(const TrFrag& f) {
+  return concat4(__builtin_bit_cast(bf16x4, f.lo), __builtin_bit_cast(bf16x4, f.hi));
+}
+#define WAIT_LDS(n) asm volatile("s_waitcnt lgkmcnt(" #n ")" ::: "memory")
+
+// ---------------------------------------------------------------------------------------------------------- forward
+//   S^T = K Q^T      O^T += V^T P^T       lane = query column
+//
+// Bound: the vector pipe of a wavefront's SIMD (exp, bf16 conversion and sums of 64 x 64 scores beside 32 products), so each product has its
+// share of it behind, two wavefronts per SIMD, and 64 queries each, so that a fragment read from LDS serves two products.  Before (32 queries,
+// three wavefronts per SIMD, attn_hd64.hip) / now, us: 16 heads, L = 8192, causal 179 / 173, full 308 / 265 (1037 TFLOP/s); 24 heads, causal,
+// 239 / 219; 4 x 32 heads on 8, causal, 1200 / 1067.
+constexpr int FW_QT = 2, FW_BM = 32 * FW_QT * 4, FW_SLOTS = 4;
+
+__global__ __launch_bounds__(256, 2) void attn_fwd_hd64_pipe_kernel(const AttnParams p) {
+  extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
+  bf16* kring = reinterpret_cast<bf16*>(smem);   // [FW_SLOTS][TILE]
+  bf16* vring = kring + FW_SLOTS * TILE;         // [FW_SLOTS][TILE]
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, g = lane >> 5, i = lane & 31;
+  const BlockCoord bc = block_coord(p.Hq, p.B, p.causal);
+  const int nqb = gridDim.x / (p.Hq * p.B);
+  const int qblk = p.causal ? nqb - 1 - bc.rank : bc.rank;   // heaviest blocks first
+  const int h = bc.h, b = bc.b, hk = h / p.group;
+  const int q0 = qblk * FW_BM, wq0 = q0 + wave * 32 * FW_QT;
+
+  const int n_end = p.causal ? min(p.Lk, min(q0 + FW_BM, p.Lq) + p.off) : p.Lk;
+  const int ntiles = n_end > 0 ? (n_end + ROWS - 1) / ROWS : 0;
+  // end of those tiles that this wavefront's queries see a key of, and of those that they see whole
+  int w_end = ntiles, w_full = p.Lk / ROWS;
+  if (p.causal) {
+    w_end = min(ntiles, max(0, wq0 + 32 * FW_QT - 1 + p.off + ROWS) / ROWS);
+    w_full = min(w_full, max(0, wq0 + p.off + 1) / ROWS);
+  }
+
+  Bringer bk, bv;
+  bk.init(p.sk.l, wave, lane);
+  bv.init(p.sv.l, wave, lane);
+  const bf16* kp = static_cast<const bf16*>(p.k) + b * p.sk.b + hk * p.sk.h;
+  const bf16* vp = static_cast<const bf16*>(p.v) + b * p.sv.b + hk * p.sv.h;
+  int lk = 0, lv = 0;   // the tiles being brought, the last one again where there are no more
+  const bf16 *ktp = kp, *vtp = vp;
+  auto load_k = [&](int j) INLINE { bk.load(kring + (lk & (FW_SLOTS - 1)) * TILE, ktp, p.Lk - lk * ROWS, j, wave); };
+  auto load_v = [&](int j) INLINE { bv.load(vring + (lv & (FW_SLOTS - 1)) * TILE, vtp, p.Lk - lv * ROWS, j, wave); };
+  auto next_k = [&]() INLINE {
+    const int to = min(lk + 1, ntiles - 1), step = to - lk;
+    lk = to;
+    ktp += (int64_t)step * (ROWS / 2 * bk.row_bytes);
+  };
+  auto next_v = [&]() INLINE {
+    const int to = min(lv + 1, ntiles - 1), step = to - lv;
+    lv = to;
+    vtp += (int64_t)step * (ROWS / 2 * bv.row_bytes);
+  };
+
+  bf16x8 qf[FW_QT][KS];
+  int lim[FW_QT];   // last key this lane's queries see
+#pragma unroll
+  for (int qt = 0; qt < FW_QT; qt++) {
+    const int qi = wq0 + 32 * qt + i;
+    load_rows(qf[qt], static_cast<const bf16*>(p.q) + b * p.sq.b + h * p.sq.h, p.sq.l, qi, p.Lq, g);
+    lim[qt] = p.causal ? min(p.Lk - 1, qi + p.off) : p.Lk - 1;
+  }
+  const float c2 = p.scale_log2e;
+  f32x16 o[FW_QT][DT], s[2][FW_QT];
+  float ref[FW_QT], l2[FW_QT][2];   // a row's reference in log2 units; this lane's partial row sums
+  bf16x8 pb[2][FW_QT][2];
+  Readers<D> rd;
+  rd.init(kring, g, i);   // rows of K from its row[] on; columns of V from its tr[] + the rings' distance on
+  auto score = [&](int kt, int qt, int r, int t) INLINE { return t * ROWS + 32 * kt + acc_row(r, g) > lim[qt] ? -INFINITY : s[kt][qt][r]; };
+
+  // The 32 pairs of elements of P that a turn forms: 0 .. 15 of sub-tile 1 of tile t, then those of sub-tile 0 of tile t + 1; in three steps,
+  // each one product behind the one before
+  float y[2] = {0.f, 0.f}, x[2] = {0.f, 0.f};
+  auto exponents = [&](int e, int t, auto masked) INLINE {
+    const int kt = (e & 31) < 16, qt = (e >> 3) & 1, r = 2 * (e & 7), tile = e < 16 ? t : t + 1;
+#pragma unroll
+    for (int n = 0; n < 2; n++) y[n] = fmaf(decltype(masked)::value ? score(kt, qt, r + n, tile) : s[kt][qt][r + n], c2, -ref[qt]);
+  };
+  auto take = [&](int e) INLINE {   // pair e: into the row sums and among the operands
+    const int kt = (e & 31) < 16, qt = (e >> 3) & 1, r = 2 * (e & 7);
+#pragma unroll
+    for (int n = 0; n < 2; n++) l2[qt][n] += x[n], pb[kt][qt][r >> 3][(r & 7) + n] = (bf16)x[n];
+  };
+  auto weigh = [&](int e, int t, auto masked) INLINE {
+    const float x0 = ody_exp2(y[0]), x1 = ody_exp2(y[1]);
+    exponents(e + 1, t, masked);
+    take(e == 0 ? 31 : e - 1);
+    x[0] = x0, x[1] = x1;
+  };
+  typedef const bf16x8 __attribute__((address_space(3))) * frag_ptr;
+  bf16x8 kfr[KS];       // K rows: k-step n
+  TrFrag vfr[2 * DT];   // V^T: k-step n >> 1, columns 32 (n & 1)
+  auto kslot = [&](int t) INLINE { return (t & (FW_SLOTS - 1)) * TILE * 2; };
+  auto read_k = [&](int n, unsigned slot, int kt) INLINE { kfr[n] = *(frag_ptr)(uintptr_t)(rd.row[n] + slot + 2 * 32 * kt * D); };
+  auto read_v = [&](int n, unsigned slot, auto kt) INLINE {
+    constexpr int KT = decltype(kt)::value;
+    const unsigned at = slot + FW_SLOTS * TILE * 2;
+    if (n >> 1) read_tr<32 * KT + 16>(vfr[n], rd.tr[2 * (n & 1)] + at, rd.tr[2 * (n & 1) + 1] + at);
+    else read_tr<32 * KT>(vfr[n], rd.tr[2 * (n & 1)] + at, rd.tr[2 * (n & 1) + 1] + at);
+  };
+  // S of sub-tile KT of a tile, and reads of V of sub-tile KT of the one before
+  auto s_phase = [&](auto kt, unsigned vslot, int e0, int t, int load, auto masked) INLINE {
+    constexpr int KT = decltype(kt)::value;
+#pragma unroll
+    for (int m = 0; m < 8; m++) {
+      const int n = m >> 1, qt = m & 1;
+      if (m == 0) WAIT_LDS(2);   // with two reads issued behind: fragments 0 and 1 are there
+      if (m == 4) WAIT_LDS(4);
+      s[KT][qt] = mfma32(kfr[n], qf[qt][n], n == 0 ? f32x16{0} : s[KT][qt]);
+      FENCE();
+      if (qt == 1) read_v(n, vslot, kt);
+      if (m == 2) load ? load_v(load >> 1) : load_k(0);
+      weigh(e0 + m, t, masked);
+      FENCE();
+    }
+  };
+  // O += P V of sub-tile KT, and reads of K of the other sub-tile
+  auto pv_phase = [&](auto kt, unsigned kslot, int e0, int t, int load, auto masked) INLINE {
+    constexpr int KT = decltype(kt)::value;
+#pragma unroll
+    for (int m = 0; m < 8; m++) {
+      const int n = m >> 1, qt = m & 1;
+      if (m == 0) {
+        WAIT_LDS(4);
+        tie(vfr[0]), tie(vfr[1]);
+      }
+      if (m == 4) {
+        WAIT_LDS(2);
+        tie(vfr[2]), tie(vfr[3]);
+      }
+      o[qt][n & 1] = mfma32(value(vfr[n]), pb[KT][qt][n >> 1], o[qt][n & 1]);
+      FENCE();
+      if (qt == 1) read_k(n, kslot, KT ^ 1);
+      if (m == 2) load_k(load);
+      weigh(e0 + m, t, masked);
+      FENCE();
+    }
+  };
+  std::integral_constant<int, 0> c0;
+  std::integral_constant<int, 1> c1;
+  auto turn = [&](int t, auto masked) INLINE {
+    s_phase(c0, kslot(t), 0, t, 1, masked);
+    pv_phase(c0, kslot(t + 1), 8, t, 1, masked);
+    s_phase(c1, kslot(t), 16, t, 3, masked);
+    // K tile t + 2 and V tile t + 1 have landed (behind them the 4 loads of the tiles after); everyone is done with K tile t + 1 and V tile t - 1
+    asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    next_k();
+    next_v();
+    pv_phase(c1, kslot(t + 2), 24, t, 0, masked);
+  };
+
+  // The reference of a row is the largest score of its first tile (a row that sees any key sees key 0) and stays.
+  auto clear_rows = [&]() INLINE {
+#pragma unroll
+    for (int qt = 0; qt < FW_QT; qt++) {
+      clear(o[qt]);
+      ref[qt] = -FLT_MAX;   // no score is below it; not minus infinity, from which a masked score would be NaN
+      l2[qt][0] = l2[qt][1] = 0.f;
+    }
+  };
+  auto scores = [&](int t) INLINE {
+#pragma unroll
+    for (int kt = 0; kt < 2; kt++)
+#pragma unroll
+      for (int n = 0; n < KS; n++) {
+        read_k(n, kslot(t), kt);
+#pragma unroll
+        for (int qt = 0; qt < FW_QT; qt++) s[kt][qt] = mfma32(kfr[n], qf[qt][n], n == 0 ? f32x16{0} : s[kt][qt]);
+      }
+  };
+  auto largest = [&](int qt, int t) INLINE {   // in log2 units
+    float mx = -INFINITY;
+#pragma unroll
+    for (int kt = 0; kt < 2; kt++)
+#pragma unroll
+      for (int r = 0; r < 16; r++) mx = fmaxf(mx, score(kt, qt, r, t));
+    return half_swap_max(mx) * c2;
+  };
+  auto products = [&](int t) INLINE {
+    auto half = [&](auto kt) INLINE {
+#pragma unroll
+      for (int n = 0; n < 4; n++) read_v(n, kslot(t), kt);
+      WAIT_LDS(0);
+#pragma unroll
+      for (int n = 0; n < 4; n++) {
+        tie(vfr[n]);
+#pragma unroll
+        for (int qt = 0; qt < FW_QT; qt++) o[qt][n & 1] = mfma32(value(vfr[n]), pb[decltype(kt)::value][qt][n >> 1], o[qt][n & 1]);
+      }
+    };
+    half(c0);
+    half(c1);
+  };
+  clear_rows();
+  if (ntiles > 0) {
+    // K tiles 0 .. 3 and V tiles 0 .. 2, of the last ones a part: the loop brings the rest
+    load_k(0), load_k(1);
+#pragma unroll
+    for (int a = 0; a < 3; a++) {
+      next_k();
+      if (a > 0) next_v();
+      load_k(0);
+      if (a < 2) load_v(0), load_k(1), load_v(1);
+    }
+    asm volatile("s_waitcnt vmcnt(5)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    int t = 0;
+    if (w_end > 0) {
+      scores(0);
+#pragma unroll
+      for (int qt = 0; qt < FW_QT; qt++) ref[qt] = fmaxf(ref[qt], largest(qt, 0));
+#pragma unroll
+      for (int e = 16; e < 32; e++) {   // the last pair is left to be taken by the first turn
+        exponents(e, -1, std::true_type{});
+        x[0] = ody_exp2(y[0]), x[1] = ody_exp2(y[1]);
+        if (e < 31) take(e);
+      }
+      exponents(0, 0, std::true_type{});
+#pragma unroll
+      for (int n = 0; n < KS; n++) read_k(n, kslot(1), 0);
+      FENCE();
+      for (; t + 1 < min(w_end, w_full); t++) turn(t, std::false_type{});
+      for (; t + 1 < w_end; t++) turn(t, std::true_type{});
+      // the last tile: P of its second half, the products
+      take(31);
+#pragma unroll
+      for (int e = 0; e < 16; e++) {
+        exponents(e, t, std::true_type{});
+        x[0] = ody_exp2(y[0]), x[1] = ody_exp2(y[1]);
+        take(e);
+      }
+      products(t);
+    }
+    // the other wavefronts' tiles: keep bringing this one's share of them
+    for (; t + 1 < ntiles; t++) {
+      load_v(0), load_k(1), load_v(1);
+      asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+      next_k();
+      next_v();
+      load_k(0);
+    }
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();   // everyone is done with the rings
+  {
+    // a later score that outgrew its row's reference by more than fp32 holds left a row sum beyond any real one (or a NaN), or,
+    // times large values, an infinity in O: the block walks its keys once more with the maximum so far, so that P <= 1
+    int* flags = reinterpret_cast<int*>(smem);
+    bool beyond = false;
+#pragma unroll
+    for (int qt = 0; qt < FW_QT; qt++) {
+      float zero[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int dt = 0; dt < DT; dt++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) zero[r & 3] = fmaf(o[qt][dt][r], 0.f, zero[r & 3]);
+      beyond |= !((zero[0] + zero[1]) + (zero[2] + zero[3]) == 0.f) || !(half_swap_sum(l2[qt][0] + l2[qt][1]) < 0x1p100f);
+    }
+    const int mine = __builtin_amdgcn_ballot_w64(beyond) != 0;
+    if (lane == 0) flags[wave] = mine;
+    __syncthreads();
+    const int any = flags[0] | flags[1] | flags[2] | flags[3];
+    __syncthreads();
+    if (any) {
+      clear_rows();
+      for (int t = 0; t < ntiles; t++) {
+        lk = lv = t;
+        ktp = kp + (int64_t)t * ROWS * p.sk.l, vtp = vp + (int64_t)t * ROWS * p.sv.l;
+        load_k(0), load_k(1), load_v(0), load_v(1);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        if (t < w_end) {
+          scores(t);
+#pragma unroll
+          for (int qt = 0; qt < FW_QT; qt++) {
+            const float next = fmaxf(ref[qt], largest(qt, t)), alpha = ody_exp2(ref[qt] - next);
+            ref[qt] = next;
+            l2[qt][0] *= alpha, l2[qt][1] *= alpha;
+#pragma unroll
+            for (int dt = 0; dt < DT; dt++)
+#pragma unroll
+              for (int r = 0; r < 16; r++) o[qt][dt][r] *= alpha;
+          }
+#pragma unroll
+          for (int e = 0; e < 32; e++) {
+            exponents(e, e < 16 ? t : t - 1, std::true_type{});
+            x[0] = ody_exp2(y[0]), x[1] = ody_exp2(y[1]);
+            take(e);
+          }
+          products(t);
+        }
+        __syncthreads();
+      }
+    }
+  }
+
+#pragma unroll
+  for (int qt = 0; qt < FW_QT; qt++) {
+    const int qi = wq0 + 32 * qt + i;
+    const float l = half_swap_sum(l2[qt][0] + l2[qt][1]);
+    if (qi >= p.Lq) continue;
+    const float inv = l > 0.f ? 1.f / l : 0.f;
+    store_row(static_cast<bf16*>(p.out) + b * p.so.b + h * p.so.h + (int64_t)qi * p.so.l, o[qt], inv, g);
+    if (g == 0) p.lse[((int64_t)b * p.Hq + h) * p.Lq + qi] = l > 0.f ? (ref[qt] + __log2f(l)) * ODY_LN2 : -INFINITY;
+  }
+}
+
+}  // namespace
+
+int ody_launch_attn_fwd_hd64_pipe(const AttnParams& p, hipStream_t st) {
+  constexpr size_t smem = (size_t)2 * FW_SLOTS * TILE * sizeof(bf16);
+  if (int rc = ody_allow_dynamic_lds(reinterpret_cast<const void*>(&attn_fwd_hd64_pipe_kernel), smem, "attn_fwd_hd64_pipe")) return rc;
+  const int64_t blocks = (int64_t)p.B * p.Hq * ((p.Lq + FW_BM - 1) / FW_BM);
+  ODY_LAUNCH("attn_fwd_hd64_pipe", st, attn_fwd_hd64_pipe_kernel, dim3((unsigned)blocks), dim3(256), smem, p);
+  return ody_check_launch("attn_fwd_hd64_pipe");
+}

@@ -103,6 +103,7 @@ int ody_launch_attn_bwd_pipe(const AttnParams& p, void* workspace, hipStream_t s
 // head_dim 64, bf16, no dropout; the forward needs no workspace, the backward room for its row values, which take the place of
 // p.delta.  With ody_attn_bwd_hd64_workspace(...) bytes it can take the query heads of a group apart; with less it does not.
 int ody_launch_attn_fwd_hd64(const AttnParams& p, hipStream_t st);
+int ody_launch_attn_fwd_hd64_pipe(const AttnParams& p, hipStream_t st);   // with blocks enough for the whole chip
 size_t ody_attn_bwd_hd64_workspace(int B, int Lq, int Lk, int Hq, int Hkv);
 int ody_launch_attn_bwd_hd64(const AttnParams& p, void* workspace, size_t workspace_bytes, hipStream_t st);
 // head_dim 128 where those two leave compute units idle.  Neither reads images; the forward uses no workspace (its callers still ask for that of

@@ -1,0 +1,105 @@
+"""GPU parity of the head_dim-64 forward for many blocks (csrc/attn_hd64_pipe.hip) at the edges of their tiles, rings, blocks and dispatch, against
+the oracle, and of the calls that stay with the kernel for few."""
+import pytest
+import torch
+
+from conftest import TOL_BF16, TOL_LSE, assert_parity, randn
+import odysseus_oracle as oracle
+
+pytestmark = pytest.mark.gpu
+FWD = "attn_fwd_hd64_pipe"
+
+
+def _ran(f):
+    from odysseus_transformer_amd import _lib
+    _lib.profile_enable(True)
+    try:
+        _lib.profile_collect()
+        out = f()
+        torch.cuda.synchronize()
+        return out, set(_lib.profile_collect())
+    finally:
+        _lib.profile_enable(False)
+
+
+def _inputs(B, Lq, Lk, Hq, Hkv, seed):
+    shapes = ((Lq, Hq), (Lk, Hkv), (Lk, Hkv), (Lq, Hq))
+    return [randn((B, L, H, 64), seed + n, dtype=torch.bfloat16) for n, (L, H) in enumerate(shapes)]
+
+
+def _check(B, Lq, Lk, Hq, Hkv, causal, fwd, dev, seed=61, heads=None, stretch=1.0):
+    """All of a call; the oracle for the first `heads` kv heads only, which see the others' blocks as neighbours."""
+    from odysseus_transformer_amd import ops
+    print(f"{B=} {Lq=} {Lk=} {Hq=} {Hkv=} {causal=} {stretch=}", flush=True)
+    q, k, v, do = _inputs(B, Lq, Lk, Hq, Hkv, seed)
+    k = (k.float() * torch.linspace(1.0, stretch, Lk)[None, :, None, None]).bfloat16()
+    qg, kg, vg, dog = (t.to(dev) for t in (q, k, v, do))
+    (o, lse), ran = _ran(lambda: ops.attn_fwd(qg, kg, vg, causal=causal))
+    assert (FWD in ran) == fwd, ran
+    grads = ops.attn_bwd(qg, kg, vg, o, lse, dog, causal=causal)
+    n, G = heads or Hkv, Hq // Hkv
+    q, k, v, do, o, lse = q[:, :, :n * G], k[:, :, :n], v[:, :, :n], do[:, :, :n * G], o[:, :, :n * G].cpu(), lse[:, :n * G].cpu()
+    o_ref, lse_ref = oracle.attention_fwd(q.float(), k.float(), v.float(), causal=causal)
+    assert_parity(o, o_ref, TOL_BF16, "o")
+    assert torch.allclose(lse, lse_ref, atol=TOL_LSE, rtol=TOL_LSE)
+    # gradients from the o and lse that the kernels had: one-hot rows leave dS little but the rounding of out
+    refs = oracle.attention_bwd(q.float(), k.float(), v.float(), o.float(), lse, do.float(), causal=causal)
+    for got, ref, name, count in zip(grads, refs, ("dq", "dk", "dv"), (n * G, n, n)):
+        assert_parity(got[:, :, :count], ref, TOL_BF16, name, 1e-3)
+    return o
+
+
+# keys from the fewest that the forward takes on: whole and ragged last tiles, rings that wrap; queries: whole blocks, half a last one
+@pytest.mark.parametrize("stretch", [1.0, 60.0], ids=["unit", "moving_reference"])
+@pytest.mark.parametrize("Lq,Lk", [(512, 512), (505, 513), (1024, 575), (1000, 639), (2049, 641)])
+def test_full(Lq, Lk, stretch, dev):
+    H = 256 // ((Lq + 255) // 256) + 1
+    _check(1, Lq, Lk, H, H, False, True, dev, heads=3, stretch=stretch)
+
+
+# at the lines of the causal forward: 768 blocks, 1024 blocks of 2048 keys; more keys than queries, more queries than keys
+@pytest.mark.parametrize("L,Lk,Hq,Hkv", [(4096, 4096, 48, 12), (2000, 2048, 128, 128), (1991, 2111, 128, 32), (4091, 2731, 48, 48), (4099, 4096, 46, 46),
+                                         (4500, 4096, 44, 22)])
+def test_causal(L, Lk, Hq, Hkv, dev):
+    _check(1, L, Lk, Hq, Hkv, True, True, dev, heads=1)
+
+
+@pytest.mark.parametrize("Lq,Lk,H,causal", [(320, 320, 2, False), (512, 511, 128, False), (128, 512, 256, False), (640, 512, 86, False),
+                                            (2048, 2048, 127, True), (4096, 4096, 47, True)])
+def test_calls_that_stay_with_the_kernel_for_few_blocks(Lq, Lk, H, causal, dev):
+    _check(1, Lq, Lk, H, H, causal, False, dev, heads=2)
+
+
+@pytest.mark.parametrize("stride", [64, 1 << 23, (1 << 24) - 16, (1 << 24) - 8], ids=str)
+def test_rows_far_apart(stride, dev):
+    """Row strides up to the last one whose tile fits 32-bit offsets, and the first one beyond."""
+    from odysseus_transformer_amd import ops
+    near = stride < (1 << 24) - 8
+    q, k, v, do = _inputs(1, 513 * 256, 520, 1, 1, 81)
+    q, do = q[:, :131072 - 7], do[:, :131072 - 7]
+
+    def far(t):
+        out = torch.empty(stride * (t.shape[1] - 1) + 64, dtype=torch.bfloat16, device=dev).as_strided(t.shape, (0, stride, 64, 1))
+        return out.copy_(t)
+    fk = far(k)
+    (o, lse), ran = _ran(lambda: ops.attn_fwd(q.to(dev), fk, v.to(dev), causal=False))
+    assert (FWD in ran) == near, ran
+    o_ref, lse_ref = oracle.attention_fwd(q[:, -300:].float(), k.float(), v.float(), causal=False)
+    assert_parity(o[:, -300:], o_ref, TOL_BF16, "o")
+
+
+@pytest.mark.parametrize("causal", [False, True], ids=["full", "causal"])
+def test_large_values_behind_an_outgrown_reference(causal, dev):
+    """Scores 56 above a row's first tile with |v| around 2^48: the blocks walk their keys once more, and nothing may overflow on the way."""
+    from odysseus_transformer_amd import ops
+    L, H = (4096, 48) if causal else (1000, 64)
+    q, k, v, _ = _inputs(1, L, L, H, H, 91)
+    q[..., 0], k[..., 0] = 8.0, 0.0
+    k[:, -(L // 4):, :, 0] = 56.0
+    v = (v.float() * 2.0 ** 48).bfloat16()
+    (o, lse), ran = _ran(lambda: ops.attn_fwd(q.to(dev), k.to(dev), v.to(dev), causal=causal))
+    assert FWD in ran, ran
+    assert bool(o.isfinite().all())
+    o_ref, lse_ref = oracle.attention_fwd(q[:, :, :2].float(), k[:, :, :2].float(), v[:, :, :2].float(), causal=causal)
+    assert_parity(o[:, :, :2], o_ref, TOL_BF16, "o")
+    assert torch.allclose(lse[:, :2].cpu(), lse_ref, atol=TOL_LSE, rtol=TOL_LSE)
