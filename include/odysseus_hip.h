@@ -142,9 +142,9 @@ int ody_attn_fwd_noalloc(const void* q, const void* k, const void* v, void* out,
  * the bf16 head_dim-128 kernels transposed copies of K, Q and dO, plus fp32 partial dK / dV
  * or dQ where grouped-query attention, or a call with one short side, is cut into parts
  * that a second kernel adds up in a fixed order).  The bf16 head_dim-64 kernels take a workspace of
- * ody_attn_bwd_workspace_least_bytes(...) too: without room for the fp32 dK / dV of every query head
- * they walk a group's heads in turn, which gives few key blocks less to do at once.  (Elsewhere the
- * two byte counts are the same.)
+ * ody_attn_bwd_workspace_least_bytes(...) too: without room for the start values of their scores and the
+ * fp32 dK / dV of every query head they take the slower kernel, which walks a group's heads in turn.
+ * (Elsewhere the two byte counts are the same.)
  */
 enum ody_attn_bwd_flags { ODY_BWD_ACCUMULATE_DQ = 1, ODY_BWD_DQ_F32 = 2, ODY_BWD_REUSE_QUERY_SIDE = 4, ODY_BWD_KEEP_DS = 8 };
 size_t ody_attn_bwd_workspace_bytes(int B, int Lq, int Lk, int Hq, int Hkv, int D, int dtype);

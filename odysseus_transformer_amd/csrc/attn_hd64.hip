@@ -14,7 +14,7 @@
 // takes every other tile; the sets add up through LDS at the end.  It is for calls with too few blocks to give every SIMD three
 // wavefronts.
 //
-// Where there are blocks enough, the forward takes the kernel of attn_hd64_pipe.hip (dispatch: end of this file).
+// Where there are blocks enough, the forward and dK/dV take the kernels of attn_hd64_pipe.hip (dispatch: end of this file).
 //
 // Tiles and fragments: attn_rowtile.h.
 //
@@ -202,8 +202,10 @@ __global__ __launch_bounds__(256 * GROUPS, 4) void attn_fwd_hd64_kernel(const At
 }
 
 // ---------------------------------------------------------------------------------------------------------- backward
-// -delta of every query row, (B, Hq, Lq) in fp32: what dP starts from.  8 lanes per row.
-__global__ __launch_bounds__(256) void attn_bwd_hd64_rows_kernel(const AttnParams p, float* __restrict__ neg_delta) {
+// Start values in fp32: -delta of every query row, (B, Hq, Lq), and, unless null, -lse / scale, (B, Hq, Lq rounded up to whole tiles), minus infinity
+// where P must be 0: past the end, or a query that saw no key.  8 lanes per row.
+__global__ __launch_bounds__(256) void attn_bwd_hd64_rows_kernel(const AttnParams p, float* __restrict__ neg_delta,
+                                                                 float* __restrict__ neg_lse) {
   const int lane8 = threadIdx.x & 7, qi = blockIdx.x * 32 + (threadIdx.x >> 3), h = blockIdx.y, b = blockIdx.z;
   float acc = 0.f;
   if (qi < p.Lq) {
@@ -214,14 +216,21 @@ __global__ __launch_bounds__(256) void attn_bwd_hd64_rows_kernel(const AttnParam
   }
 #pragma unroll
   for (int sft = 4; sft > 0; sft >>= 1) acc += __shfl_xor(acc, sft, 64);
-  if (lane8 == 0 && qi < p.Lq) neg_delta[((int64_t)b * p.Hq + h) * p.Lq + qi] = -acc;
+  if (lane8 != 0) return;
+  const int64_t head = (int64_t)b * p.Hq + h;
+  float l = INFINITY;
+  if (qi < p.Lq) {
+    neg_delta[head * p.Lq + qi] = -acc;
+    l = p.lse[head * p.Lq + qi];
+  }
+  const int rows = (p.Lq + ROWS - 1) / ROWS * ROWS;
+  if (neg_lse && qi < rows) neg_lse[head * rows + qi] = l == INFINITY || l == -INFINITY ? -INFINITY : -l / p.scale;
 }
 
 //   S = Q K^T - lse / scale     dP = dO V^T - delta     dV^T += dO^T P     dK^T += Q^T (P o dP)      lane = key column
 //
 // S starts from -lse / scale of its rows, which the first wavefront of a group forms from lse once per tile: a register load beside
-// the tile's direct loads, written to the tile's stage after the products of the tile before it.  (Kept in memory by the kernel
-// above they would double the workspace that a caller holds, for the same time.)
+// the tile's direct loads, written to the tile's stage after the products of the tile before it.
 //
 // PART: the block takes ONE query head and leaves fp32 sums in part [dK | dV][B][Hq][Lk][D], which the kernel below adds over the
 // heads of a group; otherwise it walks all query heads of its kv head.
@@ -521,6 +530,7 @@ __global__ __launch_bounds__(256 * GROUPS, GROUPS == 1 ? 3 : 2) void attn_bwd_hd
 
 inline size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
 inline size_t delta_bytes(int B, int Lq, int Hq) { return align256((size_t)B * Hq * Lq * sizeof(float)); }
+inline size_t lse_bytes(int B, int Lq, int Hq) { return align256((size_t)B * Hq * ((Lq + ROWS - 1) / ROWS * ROWS) * sizeof(float)); }
 inline int64_t row_blocks(int B, int L, int H) { return (int64_t)B * H * ((L + BLOCK_ROWS - 1) / BLOCK_ROWS); }
 
 // Fewer blocks than this leave SIMDs with one wavefront: two groups per block.  (More groups per block for all calls, which evens
@@ -561,23 +571,31 @@ int ody_launch_attn_fwd_hd64(const AttnParams& p, hipStream_t st) {
                              : launch("attn_fwd_hd64", &attn_fwd_hd64_kernel<1>, blocks, 1, KV_STAGE, st, p);
 }
 
-// [-delta | fp32 dK / dV of every query head]
+// [-delta | -lse / scale | fp32 dK / dV of every query head]; with less room -delta alone
 size_t ody_attn_bwd_hd64_workspace(int B, int Lq, int Lk, int Hq, int Hkv) {
-  return delta_bytes(B, Lq, Hq) + (split_heads(B, Lk, Hq, Hkv) ? align256((size_t)2 * B * Hq * Lk * D * sizeof(float)) : 0);
+  return delta_bytes(B, Lq, Hq) + lse_bytes(B, Lq, Hq) + (split_heads(B, Lk, Hq, Hkv) ? align256((size_t)2 * B * Hq * Lk * D * sizeof(float)) : 0);
 }
 
 int ody_launch_attn_bwd_hd64(const AttnParams& p, void* workspace, size_t workspace_bytes, hipStream_t st) {
   float* neg_delta = static_cast<float*>(workspace);
-  float* part = reinterpret_cast<float*>(static_cast<char*>(workspace) + delta_bytes(p.B, p.Lq, p.Hq));
+  float* neg_lse = reinterpret_cast<float*>(static_cast<char*>(workspace) + delta_bytes(p.B, p.Lq, p.Hq));
+  float* part = reinterpret_cast<float*>(reinterpret_cast<char*>(neg_lse) + lse_bytes(p.B, p.Lq, p.Hq));
+  const bool lse_room = workspace_bytes >= delta_bytes(p.B, p.Lq, p.Hq) + lse_bytes(p.B, p.Lq, p.Hq);
   int rc;
-  if (!p.reuse_query_side) {
-    ODY_LAUNCH("attn_bwd_hd64_rows", st, attn_bwd_hd64_rows_kernel, dim3((p.Lq + 31) / 32, p.Hq, p.B), dim3(256), 0, p, neg_delta);
+  if (!p.reuse_query_side) {   // -lse / scale for a later call that reuses it, too, whichever kernel that one takes
+    ODY_LAUNCH("attn_bwd_hd64_rows", st, attn_bwd_hd64_rows_kernel, dim3((p.Lq + ROWS - 1) / ROWS * (ROWS / 32), p.Hq, p.B), dim3(256), 0, p, neg_delta,
+               lse_room ? neg_lse : nullptr);
     if ((rc = ody_check_launch("attn_bwd_hd64_rows"))) return rc;
   }
   const bool heads = split_heads(p.B, p.Lk, p.Hq, p.Hkv) && workspace_bytes >= ody_attn_bwd_hd64_workspace(p.B, p.Lq, p.Lk, p.Hq, p.Hkv);
   const int64_t nkv = row_blocks(p.B, p.Lk, heads ? p.Hq : p.Hkv), nq = row_blocks(p.B, p.Lq, p.Hq);
   auto dkdv = [&](auto kern, int groups) { return launch("attn_bwd_hd64_dkdv", kern, nkv, groups, QS_STAGE, st, p, neg_delta, part); };
-  if (nkv < FEW_BLOCKS) rc = heads ? dkdv(&attn_bwd_hd64_dkdv_kernel<2, true>, 2) : dkdv(&attn_bwd_hd64_dkdv_kernel<2, false>, 2);
+  // One query head per block, in the order of attn_hd64_pipe.hip.  Whole backward before / with it, us: 16 heads, L = 8192, causal 520 / 472, full
+  // 992 / 890; 8 heads of it 386 / 308; 16 heads, L = 4096, causal 206 / 164; 4 x 32 heads, L = 500, 57.1 / 52.3.  With fewer than 6 tiles of
+  // queries its prologue shows: 32 x 16 heads, L = 300, 96.2 / 97.5; 64 x 16 heads, L = 256, causal 113.7 / 116.
+  if (lse_room && (heads || p.group == 1) && p.Lq > 5 * ROWS && near(p.sq, p.sdo))
+    rc = ody_launch_attn_bwd_hd64_dkdv_pipe(p, neg_delta, neg_lse, heads ? part : nullptr, st);
+  else if (nkv < FEW_BLOCKS) rc = heads ? dkdv(&attn_bwd_hd64_dkdv_kernel<2, true>, 2) : dkdv(&attn_bwd_hd64_dkdv_kernel<2, false>, 2);
   else rc = heads ? dkdv(&attn_bwd_hd64_dkdv_kernel<1, true>, 1) : dkdv(&attn_bwd_hd64_dkdv_kernel<1, false>, 1);
   if (rc) return rc;
   if (heads) {

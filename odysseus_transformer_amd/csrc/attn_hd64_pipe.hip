@@ -1,6 +1,11 @@
 // Flash attention for bf16 and head_dim 64 where there are blocks enough for the whole chip: the arithmetic, tiles and fragments of
-// attn_hd64.hip in the order of attn_fwd_pipe.hip -- the vector work of one sub-tile under the products of another,
+// attn_hd64.hip in the order of attn_fwd_pipe.hip and attn_bwd_pipe.hip -- the vector work of one sub-tile under the products of another,
 // instead of left to whichever wavefront of a SIMD has some.
+//
+// Tried and left: dQ in this order with 64 queries per wavefront (304 registers, one wavefront per SIMD).  Whole backward with the dQ of
+// attn_hd64.hip / with it, us: 16 heads, L = 8192, causal 481 / 457, full 893 / 838, but 8 heads of it 304 / 310, 4 x 32 heads 3907 / 4016,
+// 32 heads, L = 2048 x 4, 275 / 292, L = 1000 x 4, 97 / 104: causal blocks that long and alone on their unit leave a tail.  With 32 queries the
+// fragment reads from LDS take as long as the products.
 #include <cfloat>
 #include <type_traits>
 #include "attn_rowtile.h"
@@ -353,6 +358,265 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_hd64_pipe_kernel(const AttnPa
   }
 }
 
+// ---------------------------------------------------------------------------------------------------------- backward
+//   S = Q K^T - lse / scale     dP = dO V^T - delta     dV^T += dO^T P     dK^T += Q^T (P o dP)      lane = key column
+//
+// 4 wavefronts of 32 keys, two per SIMD: 221 registers hold the sums of 32 keys, the next sub-tile's fragments and its S and dP; with 64 keys
+// they do not.  Bound: the reads from LDS and the matrix pipe alike (16 KB of fragments and 16 products per 32 x 32 sub-tile: 128 cycles of the
+// unit's LDS, of which four SIMDs want one each, and 512 of a SIMD's matrix pipe).
+// Whole backward before (the same split without the order) / now, us: 16 heads, L = 8192, causal 520 / 472, full 992 / 890; 8 heads of it,
+// causal, 386 / 308; 4 x 32 heads, L = 500, full, 57 / 52.  PART: fp32 sums of one query head to part [dK | dV][B][Hq][Lk][D]; otherwise every kv head has one.
+constexpr int KV_BN = 128, KV_SLOTS = 4;
+constexpr int KV_STAGE = 2 * TILE + 2 * 2 * ROWS;   // elements: Q and dO tiles, -lse / scale and -delta of their rows in fp32
+
+template <bool PART>
+__global__ __launch_bounds__(256, 2) void attn_bwd_hd64_dkdv_pipe_kernel(const AttnParams p, const float* __restrict__ neg_delta,
+                                                                         const float* __restrict__ neg_lse, float* __restrict__ part) {
+  extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
+  bf16* ring = reinterpret_cast<bf16*>(smem);   // [KV_SLOTS][KV_STAGE]
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, g = lane >> 5, i = lane & 31;
+  const BlockCoord bc = block_coord(p.Hq, p.B, p.causal);   // rank 0 = first key block = most query tiles
+  const int b = bc.b, h = bc.h, hk = h / p.group;
+  const int n0 = bc.rank * KV_BN, wn0 = n0 + wave * 32, key = wn0 + i;
+  const int q_tiles = (p.Lq + ROWS - 1) / ROWS, t_top = q_tiles - 1;
+  // this block's tiles, last query tile first, and of them those that see a key of this wavefront and those that see all of its keys
+  const int total = max(0, q_tiles - (p.causal ? max(0, n0 - p.off) / ROWS : 0));
+  int w_total = total, w_full = total;
+  if (p.causal) {
+    w_total = min(total, max(0, q_tiles - max(0, wn0 - p.off) / ROWS));
+    w_full = min(total, max(0, q_tiles - (max(0, wn0 + 31 - p.off) + ROWS - 1) / ROWS));
+  }
+
+  bf16x8 kf[KS], vf[KS];
+  load_rows(kf, static_cast<const bf16*>(p.k) + b * p.sk.b + hk * p.sk.h, p.sk.l, key, p.Lk, g);
+  load_rows(vf, static_cast<const bf16*>(p.v) + b * p.sv.b + hk * p.sv.h, p.sv.l, key, p.Lk, g);
+  const float c2 = p.scale_log2e;
+
+  Bringer bq, bo;
+  bq.init(p.sq.l, wave, lane);
+  bo.init(p.sdo.l, wave, lane);
+  const int64_t head = (int64_t)b * p.Hq + h;
+  int lt = 0;   // the tile being brought, the last one again where there are no more
+  const bf16* qtp = static_cast<const bf16*>(p.q) + b * p.sq.b + h * p.sq.h + (int64_t)t_top * ROWS * p.sq.l;
+  const bf16* otp = static_cast<const bf16*>(p.dout) + b * p.sdo.b + h * p.sdo.h + (int64_t)t_top * ROWS * p.sdo.l;
+  // wavefronts 0, 2 bring -lse / scale, 1, 3 -delta (zeros for rows past the end: their P is 0)
+  const float* values = wave & 1 ? neg_delta + head * p.Lq : neg_lse + head * q_tiles * ROWS;
+  const int values_bytes = 4 * (wave & 1 ? p.Lq : q_tiles * ROWS);
+  auto load = [&](int part) INLINE {   // 0, 1: halves of Q; 2, 3: of dO; 4: the values
+    bf16* st = ring + (lt & (KV_SLOTS - 1)) * KV_STAGE;
+    const int row0 = (t_top - lt) * ROWS;
+    if (part < 2) bq.load(st, qtp, p.Lq - row0, part, wave);
+    else if (part < 4) bo.load(st + TILE, otp, p.Lq - row0, part - 2, wave);
+    else {
+      auto rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(values), (short)0, values_bytes, 0x00020000);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_ptr)(st + 2 * TILE + (wave & 1) * 2 * ROWS), 4, 4 * (row0 + lane), 0, 0, 0);
+    }
+  };
+  auto next = [&]() INLINE {
+    const int to = min(lt + 1, total - 1), step = to - lt;
+    lt = to;
+    qtp -= (int64_t)step * (ROWS / 2 * bq.row_bytes);
+    otp -= (int64_t)step * (ROWS / 2 * bo.row_bytes);
+  };
+
+  f32x16 dk[DT], dv[DT], s, s_start, dp;   // S, then P; dP, then dS
+  clear(dk);
+  clear(dv);
+  bf16x8 pf[2], dsf[2], pf_next[2], dsf_next[2];
+  Readers<D> rd;
+  rd.init(ring, g, i);
+  const int key_off = p.causal ? key - p.off : -(1 << 30);   // the first query that sees this lane's key
+  typedef const bf16x8 __attribute__((address_space(3))) * frag_ptr;
+  auto slot = [&](int it) INLINE { return (unsigned)(it & (KV_SLOTS - 1)) * (KV_STAGE * 2); };
+  bf16x8 fr[2 * KS];   // Q rows, k-step n; dO rows, k-step n - 4
+  TrFrag tf[8];        // n = 2 (2 ss + dt) + which: dO^T (0) or Q^T (1)
+  auto read_row = [&](int n, unsigned st, int mt) INLINE {
+    fr[n] = *(frag_ptr)(uintptr_t)(rd.row[n & 3] + st + 2 * ((n >> 2) * ROWS + 32 * mt) * D);
+  };
+  auto read_col = [&](int n, unsigned st, auto mt_) INLINE {
+    constexpr int MT = decltype(mt_)::value;
+    const unsigned a0 = rd.tr[2 * ((n >> 1) & 1)] + st, a1 = rd.tr[2 * ((n >> 1) & 1) + 1] + st;
+    if (n < 4) {
+      if (n & 1) read_tr<32 * MT>(tf[n], a0, a1);
+      else read_tr<ROWS + 32 * MT>(tf[n], a0, a1);
+    } else {
+      if (n & 1) read_tr<32 * MT + 16>(tf[n], a0, a1);
+      else read_tr<ROWS + 32 * MT + 16>(tf[n], a0, a1);
+    }
+  };
+  // a quarter a of a lane's 16 start values: rows 8 a + 4 g .. + 3 of sub-tile mt
+  auto start_values = [&](int it, int mt, int which, int a, f32x16& x) INLINE {
+    const f32x4 v = *reinterpret_cast<const f32x4*>(reinterpret_cast<const float*>(ring + (it & (KV_SLOTS - 1)) * KV_STAGE + 2 * TILE) + which * ROWS +
+                                                    32 * mt + 8 * a + 4 * g);
+#pragma unroll
+    for (int e = 0; e < 4; e++) x[4 * a + e] = v[e];
+  };
+  auto exponent = [&](int r, int t, int mt, auto masked) INLINE {
+    float x = s[r] * c2;
+    if (decltype(masked)::value) x = t * ROWS + 32 * mt + acc_row(r, g) < key_off ? -INFINITY : x;   // queries before the key
+    s[r] = x;
+  };
+  auto weight = [&](int r) INLINE { s[r] = ody_exp2(s[r]); };
+  auto ds = [&](int r) INLINE { dp[r] *= s[r]; };
+  auto pack = [&](bf16x8 (&dst)[2], const f32x16& src, int q) INLINE {
+    dst[q >> 2][2 * q & 7] = (bf16)src[2 * q], dst[q >> 2][(2 * q & 7) + 1] = (bf16)src[2 * q + 1];
+  };
+
+  // One call: S and dP of the sub-tile after (tile it, sub-tile MT), then dV and dK of this one, 8 products each, the vector work of the former
+  // under the later ones.
+  auto unit = [&](int it, auto mt_, auto masked) INLINE {
+    constexpr int MT = decltype(mt_)::value, NMT = MT ^ 1;
+    const int nt = MT ? it + 1 : it, t = t_top - nt;   // the sub-tile after; behind that, sub-tile MT of tile it + 1
+#pragma unroll
+    for (int m = 0; m < 8; m++) {
+      if (m == 0) WAIT_LDS(4);
+      if (m == 4) WAIT_LDS(6);
+      if (m < 4) s = mfma32(fr[m], kf[m], m == 0 ? s_start : s);
+      else dp = mfma32(fr[m], vf[m - 4], dp);
+      FENCE();
+      if (m < 2) start_values(nt, NMT, 1, 2 * m, dp), start_values(nt, NMT, 1, 2 * m + 1, dp);
+      read_col(m, slot(it), mt_);
+      if (m >= 6) {
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          if (m == 7) weight(e);
+          exponent(4 * (m - 6) + e, t, NMT, masked);
+        }
+      }
+      if (MT == 1 && (m == 2 || m == 5)) load(m == 5);
+      FENCE();
+    }
+#pragma unroll
+    for (int m = 0; m < 8; m++) {
+      if (m == 0) {
+        WAIT_LDS(8);
+#pragma unroll
+        for (int n = 0; n < 4; n++) tie(tf[n]);
+      }
+      if (m == 4) {
+        WAIT_LDS(8);
+#pragma unroll
+        for (int n = 4; n < 8; n++) tie(tf[n]);
+      }
+      const int n = m >> 1;
+      if (m & 1) dk[n & 1] = mfma32(value(tf[m]), dsf[n >> 1], dk[n & 1]);
+      else dv[n & 1] = mfma32(value(tf[m]), pf[n >> 1], dv[n & 1]);
+      FENCE();
+      if (MT == 0 && m == 0) {
+        // the tile after this one has landed (behind it the 5 loads of the next); everyone is done with the one before this
+        asm volatile("s_waitcnt vmcnt(5)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        next();
+      }
+      read_row(m, slot(it + 1), MT);
+      if (m < 4) start_values(it + 1, MT, 0, m, s_start);
+      if (m <= 2) {
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          weight(4 * (m + 1) + e);
+          if (m < 2) exponent(4 * (m + 2) + e, t, NMT, masked);
+        }
+      }
+      if (m >= 2 && m < 6) {
+#pragma unroll
+        for (int e = 0; e < 4; e++) ds(4 * (m - 2) + e);
+        pack(pf_next, s, 2 * m - 4), pack(pf_next, s, 2 * m - 3);
+      }
+      if (m >= 3 && m < 7) pack(dsf_next, dp, 2 * m - 6), pack(dsf_next, dp, 2 * m - 5);
+      if (MT == 0 && m == 5) load(4);
+      if (MT == 1 && (m == 2 || m == 5)) load(2 + (m == 5));
+      FENCE();
+    }
+#pragma unroll
+    for (int ss = 0; ss < 2; ss++) pf[ss] = pf_next[ss], dsf[ss] = dsf_next[ss];
+  };
+  std::integral_constant<int, 0> c0;
+  std::integral_constant<int, 1> c1;
+
+  if (total > 0) {
+    auto all = [&]() INLINE {
+      load(4);
+#pragma unroll
+      for (int n = 0; n < 4; n++) load(n);
+    };
+    all();
+    next();
+    all();
+    next();
+    all();
+    asm volatile("s_waitcnt vmcnt(10)" ::: "memory");   // the first tile
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    int it = 0;
+    if (w_total > 0) {
+#pragma unroll
+      for (int a = 0; a < 4; a++) {
+        start_values(0, 0, 0, a, s_start);
+        start_values(0, 0, 1, a, dp);
+      }
+#pragma unroll
+      for (int n = 0; n < 8; n++) read_row(n, slot(0), 0);
+#pragma unroll
+      for (int n = 0; n < 4; n++) {
+        s = mfma32(fr[n], kf[n], n == 0 ? s_start : s);
+        dp = mfma32(fr[4 + n], vf[n], dp);
+      }
+#pragma unroll
+      for (int r = 0; r < 16; r++) {
+        exponent(r, t_top, 0, std::true_type{});
+        weight(r);
+        ds(r);
+      }
+#pragma unroll
+      for (int q = 0; q < 8; q++) {
+        pack(pf, s, q);
+        pack(dsf, dp, q);
+      }
+#pragma unroll
+      for (int a = 0; a < 4; a++) start_values(0, 1, 0, a, s_start);
+#pragma unroll
+      for (int n = 0; n < 8; n++) read_row(n, slot(0), 1);
+      FENCE();
+      for (; it + 1 < min(w_total, w_full); it++) {
+        unit(it, c0, std::false_type{});
+        unit(it, c1, std::false_type{});
+      }
+      for (; it < w_total; it++) {   // (behind the last tile a sub-tile is formed that nobody uses)
+        unit(it, c0, std::true_type{});
+        unit(it, c1, std::true_type{});
+      }
+    }
+    // the other wavefronts' tiles: keep bringing this one's share of them
+    for (; it < total; it++) {
+      asm volatile("s_waitcnt vmcnt(5)" ::: "memory");
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+      next();
+      all();
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  }
+  if (key >= p.Lk) return;
+  if (PART) {
+    float* pk = part + (head * p.Lk + key) * D;
+    float* pv = pk + (int64_t)p.B * p.Hq * p.Lk * D;
+#pragma unroll
+    for (int dt = 0; dt < DT; dt++)
+#pragma unroll
+      for (int a = 0; a < 4; a++) {
+        f32x4 wk, wv;
+#pragma unroll
+        for (int e = 0; e < 4; e++) wk[e] = dk[dt][4 * a + e], wv[e] = dv[dt][4 * a + e];
+        *reinterpret_cast<f32x4*>(pk + 32 * dt + 8 * a + 4 * g) = wk;
+        *reinterpret_cast<f32x4*>(pv + 32 * dt + 8 * a + 4 * g) = wv;
+      }
+  } else {
+    store_row(static_cast<bf16*>(p.dk) + b * p.sdk.b + hk * p.sdk.h + (int64_t)key * p.sdk.l, dk, p.scale, g);
+    store_row(static_cast<bf16*>(p.dv) + b * p.sdv.b + hk * p.sdv.h + (int64_t)key * p.sdv.l, dv, 1.f, g);
+  }
+}
+
 }  // namespace
 
 int ody_launch_attn_fwd_hd64_pipe(const AttnParams& p, hipStream_t st) {
@@ -361,4 +625,13 @@ int ody_launch_attn_fwd_hd64_pipe(const AttnParams& p, hipStream_t st) {
   const int64_t blocks = (int64_t)p.B * p.Hq * ((p.Lq + FW_BM - 1) / FW_BM);
   ODY_LAUNCH("attn_fwd_hd64_pipe", st, attn_fwd_hd64_pipe_kernel, dim3((unsigned)blocks), dim3(256), smem, p);
   return ody_check_launch("attn_fwd_hd64_pipe");
+}
+
+int ody_launch_attn_bwd_hd64_dkdv_pipe(const AttnParams& p, const float* neg_delta, const float* neg_lse, float* part, hipStream_t st) {
+  constexpr size_t smem = (size_t)KV_SLOTS * KV_STAGE * sizeof(bf16);
+  auto kern = part ? &attn_bwd_hd64_dkdv_pipe_kernel<true> : &attn_bwd_hd64_dkdv_pipe_kernel<false>;
+  if (int rc = ody_allow_dynamic_lds(reinterpret_cast<const void*>(kern), smem, "attn_bwd_hd64_dkdv_pipe")) return rc;
+  const int64_t blocks = (int64_t)p.B * p.Hq * ((p.Lk + KV_BN - 1) / KV_BN);
+  ODY_LAUNCH("attn_bwd_hd64_dkdv_pipe", st, kern, dim3((unsigned)blocks), dim3(256), smem, p, neg_delta, neg_lse, part);
+  return ody_check_launch("attn_bwd_hd64_dkdv_pipe");
 }

@@ -1,5 +1,5 @@
-"""GPU parity of the head_dim-64 forward for many blocks (csrc/attn_hd64_pipe.hip) at the edges of their tiles, rings, blocks and dispatch, against
-the oracle, and of the calls that stay with the kernel for few."""
+"""GPU parity of the head_dim-64 kernels for many blocks (csrc/attn_hd64_pipe.hip) at the edges of their tiles, rings, blocks and dispatch, against
+the oracle, and of the calls that stay with the kernels for few."""
 import pytest
 import torch
 
@@ -7,7 +7,7 @@ from conftest import TOL_BF16, TOL_LSE, assert_parity, randn
 import odysseus_oracle as oracle
 
 pytestmark = pytest.mark.gpu
-FWD = "attn_fwd_hd64_pipe"
+FWD, DKDV = "attn_fwd_hd64_pipe", "attn_bwd_hd64_dkdv_pipe"
 
 
 def _ran(f):
@@ -27,7 +27,7 @@ def _inputs(B, Lq, Lk, Hq, Hkv, seed):
     return [randn((B, L, H, 64), seed + n, dtype=torch.bfloat16) for n, (L, H) in enumerate(shapes)]
 
 
-def _check(B, Lq, Lk, Hq, Hkv, causal, fwd, dev, seed=61, heads=None, stretch=1.0):
+def _check(B, Lq, Lk, Hq, Hkv, causal, fwd, dkdv, dev, seed=61, heads=None, stretch=1.0):
     """All of a call; the oracle for the first `heads` kv heads only, which see the others' blocks as neighbours."""
     from odysseus_transformer_amd import ops
     print(f"{B=} {Lq=} {Lk=} {Hq=} {Hkv=} {causal=} {stretch=}", flush=True)
@@ -36,7 +36,8 @@ def _check(B, Lq, Lk, Hq, Hkv, causal, fwd, dev, seed=61, heads=None, stretch=1.
     qg, kg, vg, dog = (t.to(dev) for t in (q, k, v, do))
     (o, lse), ran = _ran(lambda: ops.attn_fwd(qg, kg, vg, causal=causal))
     assert (FWD in ran) == fwd, ran
-    grads = ops.attn_bwd(qg, kg, vg, o, lse, dog, causal=causal)
+    grads, ran = _ran(lambda: ops.attn_bwd(qg, kg, vg, o, lse, dog, causal=causal))
+    assert (DKDV in ran) == dkdv, ran
     n, G = heads or Hkv, Hq // Hkv
     q, k, v, do, o, lse = q[:, :, :n * G], k[:, :, :n], v[:, :, :n], do[:, :, :n * G], o[:, :, :n * G].cpu(), lse[:, :n * G].cpu()
     o_ref, lse_ref = oracle.attention_fwd(q.float(), k.float(), v.float(), causal=causal)
@@ -54,25 +55,44 @@ def _check(B, Lq, Lk, Hq, Hkv, causal, fwd, dev, seed=61, heads=None, stretch=1.
 @pytest.mark.parametrize("Lq,Lk", [(512, 512), (505, 513), (1024, 575), (1000, 639), (2049, 641)])
 def test_full(Lq, Lk, stretch, dev):
     H = 256 // ((Lq + 255) // 256) + 1
-    _check(1, Lq, Lk, H, H, False, True, dev, heads=3, stretch=stretch)
+    _check(1, Lq, Lk, H, H, False, True, True, dev, heads=3, stretch=stretch)
 
 
 # at the lines of the causal forward: 768 blocks, 1024 blocks of 2048 keys; more keys than queries, more queries than keys
 @pytest.mark.parametrize("L,Lk,Hq,Hkv", [(4096, 4096, 48, 12), (2000, 2048, 128, 128), (1991, 2111, 128, 32), (4091, 2731, 48, 48), (4099, 4096, 46, 46),
                                          (4500, 4096, 44, 22)])
 def test_causal(L, Lk, Hq, Hkv, dev):
-    _check(1, L, Lk, Hq, Hkv, True, True, dev, heads=1)
+    _check(1, L, Lk, Hq, Hkv, True, True, True, dev, heads=1)
+
+
+# 6 tiles of queries and a few keys: fewer tiles than the ring holds for the last key blocks, wavefronts without a query, ranges of one key
+@pytest.mark.parametrize("causal", [False, True], ids=["full", "causal"])
+@pytest.mark.parametrize("B,Lq,Lk,Hq,Hkv", [(1, 321, 1, 2, 2), (2, 321, 127, 3, 3), (1, 383, 129, 4, 1), (1, 385, 700, 4, 2), (1, 700, 385, 2, 2), (1, 1031, 1031, 2, 1)])
+def test_few_keys_or_queries(B, Lq, Lk, Hq, Hkv, causal, dev):
+    _check(B, Lq, Lk, Hq, Hkv, causal, False, True, dev)
 
 
 @pytest.mark.parametrize("Lq,Lk,H,causal", [(320, 320, 2, False), (512, 511, 128, False), (128, 512, 256, False), (640, 512, 86, False),
                                             (2048, 2048, 127, True), (4096, 4096, 47, True)])
-def test_calls_that_stay_with_the_kernel_for_few_blocks(Lq, Lk, H, causal, dev):
-    _check(1, Lq, Lk, H, H, causal, False, dev, heads=2)
+def test_calls_that_stay_with_the_kernels_for_few_blocks(Lq, Lk, H, causal, dev):
+    _check(1, Lq, Lk, H, H, causal, False, Lq > 320, dev, heads=2)
+
+
+def test_the_same_bits_again_and_a_reused_query_side(dev):
+    from odysseus_transformer_amd import ops
+    q, k, v, do = (t.to(dev) for t in _inputs(1, 900, 1100, 8, 4, 71))
+    o, lse = ops.attn_fwd(q, k, v, causal=False)
+    ws = ops.attn_bwd_workspace(q, k)
+    first = ops.attn_bwd(q, k, v, o, lse, do, causal=False, workspace=ws)
+    for reuse in (True, False, True):
+        again, ran = _ran(lambda: ops.attn_bwd(q, k, v, o, lse, do, causal=False, workspace=ws, reuse_query_side=reuse))
+        assert DKDV in ran and ("attn_bwd_hd64_rows" in ran) != reuse, ran
+        assert all(torch.equal(a, b) for a, b in zip(first, again))
 
 
 @pytest.mark.parametrize("stride", [64, 1 << 23, (1 << 24) - 16, (1 << 24) - 8], ids=str)
 def test_rows_far_apart(stride, dev):
-    """Row strides up to the last one whose tile fits 32-bit offsets, and the first one beyond."""
+    """Row strides up to the last one whose tile fits 32-bit offsets, and the first one beyond: keys of the forward, queries of dK / dV."""
     from odysseus_transformer_amd import ops
     near = stride < (1 << 24) - 8
     q, k, v, do = _inputs(1, 513 * 256, 520, 1, 1, 81)
@@ -86,6 +106,15 @@ def test_rows_far_apart(stride, dev):
     assert (FWD in ran) == near, ran
     o_ref, lse_ref = oracle.attention_fwd(q[:, -300:].float(), k.float(), v.float(), causal=False)
     assert_parity(o[:, -300:], o_ref, TOL_BF16, "o")
+    del fk
+    q, k, v, do = _inputs(1, 330, 200, 1, 1, 82)
+    o_ref, lse_ref = oracle.attention_fwd(q.float(), k.float(), v.float(), causal=True)
+    refs = oracle.attention_bwd(q.float(), k.float(), v.float(), o_ref, lse_ref, do.float(), causal=True)
+    grads, ran = _ran(lambda: ops.attn_bwd(far(q), k.to(dev), v.to(dev), o_ref.bfloat16().to(dev), lse_ref.to(dev), do.to(dev), causal=True,
+                                           dq=torch.empty(q.shape, dtype=torch.bfloat16, device=dev)))
+    assert (DKDV in ran) == near, ran
+    for got, ref, name in zip(grads, refs, ("dq", "dk", "dv")):
+        assert_parity(got, ref, TOL_BF16, name)
 
 
 @pytest.mark.parametrize("causal", [False, True], ids=["full", "causal"])
