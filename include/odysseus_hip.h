@@ -176,6 +176,17 @@ int ody_lse_merge(float* out_acc, float* lse_acc, const void* out_blk, const flo
                   int B, int L, int H, int D, int64_t sb_b, int64_t sb_l, int64_t sb_h,
                   int dtype, void* stream);
 
+/* The same merge over up to ODY_MERGE_PARTS partial results at once: part i is out[i] (B, rows[i], H, D) of `dtype`, contiguous,
+ * with lse[i] (B, H, rows[i]) fp32, and covers rows first[i] .. first[i] + rows[i] - 1 of the result.  result / result_lse: (B, L, H, D) of
+ * `dtype` and (B, H, L), contiguous; result NULL: the merge goes on, and the result is left in acc (B, L, H, D) / acc_lse (B, H, L) in
+ * fp32.  have_acc: acc and acc_lse hold one more partial result, of all rows.  Rows that nothing covers: 0 and -inf.  D: 8 times a
+ * power of two, at most 512.
+ */
+#define ODY_MERGE_PARTS 8
+int ody_lse_merge_parts(int parts, const void* const* out, const float* const* lse, const int* first, const int* rows,
+                        float* acc, float* acc_lse, int have_acc, void* result, float* result_lse,
+                        int B, int L, int H, int D, int dtype, void* stream);
+
 /* Rounds an fp32 array to `dtype` (n elements, both 16-byte aligned, n a multiple of 8): the last step of a
  * result that was accumulated in fp32 over the key blocks of a ring step (running out, running dq).
  */

@@ -33,6 +33,7 @@ SIGNATURES = {
     "ody_attn_bwd_ds_bytes": (_sz, [_i] * 8),
     "ody_attn_bwd": (_i, [_p] * 9 + [_i] * 6 + [_i64] * 24 + [_f, _i, _i, _i, _p, _sz, _p]),
     "ody_cast_from_f32": (_i, [_p, _p, _i64, _i, _p]),
+    "ody_lse_merge_parts": (_i, [_i] + [_p] * 6 + [_i] + [_p] * 2 + [_i] * 5 + [_p]),
     "ody_lse_merge": (_i, [_p] * 4 + [_i] * 4 + [_i64] * 3 + [_i, _p]),
     "ody_gemm_workspace_bytes": (_sz, [_i] * 5),
     "ody_gemm": (_i, [_i] + [_p] * 4 + [_i] * 3 + [_i64] * 3 + [_i, _i, _p, _sz, _p]),

@@ -523,6 +523,84 @@ __global__ __launch_bounds__(256) void lse_merge_kernel(float* __restrict__ out_
   if (sub == 0) lse_acc[li] = nw;
 }
 
+// ---------------------------------------------------------------------------
+// Several partial results at once: 8 head-dim elements per lane, D / 8 lanes per (b, l, h) row.  HBM-bound, and a part is read once, where a
+// merge per part reads and writes the fp32 running result each time: one rank of a zigzag ring of 8 (8 parts, 4 of them of 16384 rows and 4 of
+// 8192, 4 heads of 128) 32 us, before 123 in 12 merges and 105 in the fills, copies and casts around them.
+// ---------------------------------------------------------------------------
+template <typename T>
+struct MergeParts {
+  const T* out[ODY_MERGE_PARTS];
+  const float* lse[ODY_MERGE_PARTS];
+  int first[ODY_MERGE_PARTS], rows[ODY_MERGE_PARTS];   // rows 0: none
+};
+
+template <typename T>
+__global__ __launch_bounds__(256) void lse_merge_parts_kernel(const MergeParts<T> parts, float* acc, float* acc_lse, int have_acc,
+                                                              T* __restrict__ result, float* __restrict__ result_lse, int B, int L, int H, int D) {
+  constexpr int NP = ODY_MERGE_PARTS, V = 8 / Vec16B<T>::N;   // 16-byte vectors of 8 elements
+  const int lpr = D / 8;
+  const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (idx >= (int64_t)B * L * H * lpr) return;
+  const int sub = idx % lpr;
+  const int64_t row = idx / lpr;  // (b, l, h) order
+  const int h = row % H, l = (row / H) % L, b = row / ((int64_t)H * L);
+  const int64_t li = ((int64_t)b * H + h) * L + l;
+  float w[NP + 1];
+  typename Vec16B<T>::type raw[NP][V];
+  float run[8];
+  // all loads first
+#pragma unroll
+  for (int i = 0; i < NP; i++) {
+    const int at = l - parts.first[i], n = parts.rows[i];
+    w[i] = -INFINITY;
+#pragma unroll
+    for (int v = 0; v < V; v++) raw[i][v] = typename Vec16B<T>::type{};
+    if (at < 0 || at >= n) continue;
+    w[i] = parts.lse[i][((int64_t)b * H + h) * n + at];
+    const T* src = parts.out[i] + (((int64_t)b * n + at) * H + h) * D + 8 * sub;
+#pragma unroll
+    for (int v = 0; v < V; v++) raw[i][v] = *reinterpret_cast<const typename Vec16B<T>::type*>(src + v * Vec16B<T>::N);
+  }
+  w[NP] = have_acc ? acc_lse[li] : -INFINITY;
+#pragma unroll
+  for (int e = 0; e < 8; e++) run[e] = have_acc ? acc[row * D + 8 * sub + e] : 0.f;
+
+  float mx = w[0];
+#pragma unroll
+  for (int i = 1; i <= NP; i++) mx = fmaxf(mx, w[i]);
+  float lse = -INFINITY;
+  if (mx != -INFINITY) {
+    float sum = 0.f;
+#pragma unroll
+    for (int i = 0; i <= NP; i++) sum += expf(w[i] - mx);   // 0 for what is not there
+    lse = mx + logf(sum);
+  }
+#pragma unroll
+  for (int i = 0; i <= NP; i++) w[i] = lse == -INFINITY ? 0.f : expf(w[i] - lse);
+#pragma unroll
+  for (int e = 0; e < 8; e++) {
+    run[e] *= w[NP];
+#pragma unroll
+    for (int i = 0; i < NP; i++) run[e] += (float)raw[i][e / Vec16B<T>::N][e % Vec16B<T>::N] * w[i];
+  }
+  // every lane of this row sits in one wavefront and has read acc_lse above
+  if (result) {
+#pragma unroll
+    for (int v = 0; v < V; v++) {
+      typename Vec16B<T>::type o;
+#pragma unroll
+      for (int e = 0; e < Vec16B<T>::N; e++) o[e] = (T)run[v * Vec16B<T>::N + e];
+      *reinterpret_cast<typename Vec16B<T>::type*>(result + row * D + 8 * sub + v * Vec16B<T>::N) = o;
+    }
+    if (sub == 0) result_lse[li] = lse;
+  } else {
+#pragma unroll
+    for (int e = 0; e < 8; e++) acc[row * D + 8 * sub + e] = run[e];
+    if (sub == 0) acc_lse[li] = lse;
+  }
+}
+
 constexpr int64_t MOST_BLOCKS = (1 << 24) - 1;   // of 256 threads: a launch takes fewer than 2^32 threads
 
 inline unsigned blocks_for(int64_t n) { return (unsigned)((n + 255) / 256); }
@@ -727,6 +805,42 @@ extern "C" int ody_lse_merge(float* out_acc, float* lse_acc, const void* out_blk
                ODY_LAUNCH("lse_merge", st, lse_merge_kernel<float>, dim3(blocks_for(total)), dim3(256), 0, out_acc, lse_acc,
                                   (const float*)out_blk, lse_blk, B, L, H, D, sb_b, sb_l, sb_h));
   return ody_check_launch("lse_merge");
+}
+
+namespace {
+template <typename T>
+int launch_merge_parts(int parts, const void* const* out, const float* const* lse, const int* first, const int* rows, float* acc, float* acc_lse,
+                       int have_acc, void* result, float* result_lse, int B, int L, int H, int D, hipStream_t st) {
+  MergeParts<T> t{};
+  for (int i = 0; i < parts; i++)
+    t.out[i] = static_cast<const T*>(out[i]), t.lse[i] = lse[i], t.first[i] = first[i], t.rows[i] = rows[i];
+  ODY_LAUNCH("lse_merge", st, lse_merge_parts_kernel<T>, dim3(blocks_for((int64_t)B * L * H * (D / 8))), dim3(256), 0, t, acc, acc_lse, have_acc,
+             static_cast<T*>(result), result_lse, B, L, H, D);
+  return ody_check_launch("lse_merge");
+}
+}  // namespace
+
+extern "C" int ody_lse_merge_parts(int parts, const void* const* out, const float* const* lse, const int* first, const int* rows, float* acc,
+                                   float* acc_lse, int have_acc, void* result, float* result_lse, int B, int L, int H, int D, int dtype, void* stream) {
+  ODY_REQUIRE(parts >= 0 && parts <= ODY_MERGE_PARTS, ODY_ERR_BAD_SHAPE, "ody_lse_merge_parts: %d parts, 0 to %d taken", parts, ODY_MERGE_PARTS);
+  ODY_REQUIRE(B > 0 && L > 0 && H > 0 && D > 0, ODY_ERR_BAD_SHAPE, "ody_lse_merge_parts: B=%d L=%d H=%d D=%d", B, L, H, D);
+  ODY_REQUIRE(D % 8 == 0 && D <= 512 && 64 % (D / 8) == 0, ODY_ERR_UNSUPPORTED, "ody_lse_merge_parts: D=%d must be 8 times a power of two, at most 512", D);
+  ODY_REQUIRE((int64_t)B * L * H * (D / 8) <= MOST_BLOCKS * 256, ODY_ERR_BAD_SHAPE, "ody_lse_merge_parts: too many rows for one launch");
+  ODY_REQUIRE(parts == 0 || (out && lse && first && rows), ODY_ERR_NULL, "ody_lse_merge_parts: NULL pointer");
+  for (int i = 0; i < parts; i++) {
+    ODY_REQUIRE(out[i] && lse[i], ODY_ERR_NULL, "ody_lse_merge_parts: part %d is NULL", i);
+    ODY_REQUIRE(ody_aligned16(out[i]), ODY_ERR_MISALIGNED, "ody_lse_merge_parts: part %d is not 16-byte aligned", i);
+    ODY_REQUIRE(first[i] >= 0 && rows[i] > 0 && first[i] <= L - rows[i], ODY_ERR_BAD_SHAPE, "ody_lse_merge_parts: part %d covers rows %d + %d of %d", i,
+                first[i], rows[i], L);
+  }
+  ODY_REQUIRE(result ? result_lse != nullptr : acc != nullptr, ODY_ERR_NULL, "ody_lse_merge_parts: nowhere to put the result");
+  ODY_REQUIRE((!have_acc && result) || (acc && acc_lse), ODY_ERR_NULL, "ody_lse_merge_parts: acc is NULL");
+  ODY_REQUIRE(ody_aligned16(result) && ody_aligned16(acc), ODY_ERR_MISALIGNED, "ody_lse_merge_parts: alignment");
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  if (dtype == ODY_BF16)
+    return launch_merge_parts<bf16>(parts, out, lse, first, rows, acc, acc_lse, have_acc, result, result_lse, B, L, H, D, st);
+  ODY_REQUIRE(dtype == ODY_F32, ODY_ERR_UNSUPPORTED, "ody_lse_merge_parts: dtype %d unknown", dtype);
+  return launch_merge_parts<float>(parts, out, lse, first, rows, acc, acc_lse, have_acc, result, result_lse, B, L, H, D, st);
 }
 
 // ---------------------------------------------------------------------------

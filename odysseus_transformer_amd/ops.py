@@ -7,6 +7,7 @@ of, in C++; where it answers None the Python below it decides.
 """
 from __future__ import annotations
 
+import ctypes
 import math
 import os
 from typing import Optional, Tuple
@@ -411,6 +412,40 @@ def lse_merge_(out_acc, lse_acc, out_blk, lse_blk) -> None:
             raise ValueError(f"{n} must be a contiguous float32 (B, H, L) tensor")
     _lib.call("ody_lse_merge", out_acc.data_ptr(), lse_acc.data_ptr(), out_blk.data_ptr(), lse_blk.data_ptr(),
               B, L, H, D, *_blhd(out_blk, "out_blk"), _dt(out_blk), _stream())
+
+
+class _PartialResults:
+    """Partial results (out, lse) of attention over disjoint sets of keys, each for all rows of a (B, L, H, D) result or a range of
+    them, merged in one launch; beyond MOST of them, those so far go to an fp32 running pair first, which bounds the memory they hold."""
+
+    MOST = 8   # ODY_MERGE_PARTS
+
+    def __init__(self, shape, like):
+        self.shape, self.like, self.parts, self.acc = tuple(shape), like, [], None
+
+    def add(self, out, lse, first: int = 0) -> None:
+        if len(self.parts) == self.MOST:
+            self._merge(last=False)
+        self.parts.append((out.contiguous(), lse.contiguous(), first))
+
+    def _merge(self, last: bool):
+        B, L, H, D = self.shape
+        have = self.acc is not None
+        if not last and not have:
+            self.acc = [torch.empty(s, dtype=torch.float32, device=self.like.device) for s in ((B, L, H, D), (B, H, L))]
+        result = (torch.empty(self.shape, dtype=self.like.dtype, device=self.like.device),
+                  torch.empty((B, H, L), dtype=torch.float32, device=self.like.device)) if last else None
+        n = len(self.parts)
+        pointers, ints = ctypes.c_void_p * n, ctypes.c_int * n
+        _lib.call("ody_lse_merge_parts", n, pointers(*(o.data_ptr() for o, _, _ in self.parts)), pointers(*(s.data_ptr() for _, s, _ in self.parts)),
+                  ints(*(f for _, _, f in self.parts)), ints(*(o.shape[1] for o, _, _ in self.parts)),
+                  *((t.data_ptr() for t in self.acc) if self.acc else (0, 0)), int(have), *((t.data_ptr() for t in result) if last else (0, 0)),
+                  B, L, H, D, _dt(self.like), _stream())
+        self.parts = []
+        return result
+
+    def result(self):
+        return self._merge(last=True)
 
 
 # --------------------------------------------------------------------------- linears
@@ -837,7 +872,7 @@ class RingBlocksAttnFunc(torch.autograd.Function):
     """One rank's inner loop of ring attention (entered at decoder/ring.py:30-37 in the reference):
     the local queries against a sequence of K/V blocks as they would arrive over the ring.  Block
     `causal_block` is the diagonal one (causally masked); every other block is fully visible.
-    Forward merges each block's (out, lse) into an fp32 running pair; backward runs the per-block
+    Forward merges the blocks' (out, lse) in fp32; backward runs the per-block
     flash backward with the FINAL out / lse and accumulates dq over the blocks.
 
     apply(q, causal_block, softmax_scale, *k_blocks, *v_blocks) -> (out, lse)."""
@@ -846,13 +881,11 @@ class RingBlocksAttnFunc(torch.autograd.Function):
     def forward(ctx, q, causal_block, softmax_scale, *kv):
         nb = len(kv) // 2
         ks, vs = kv[:nb], kv[nb:]
-        B, L, H, D = q.shape
-        acc = torch.zeros((B, L, H, D), dtype=torch.float32, device=q.device)
-        lse = torch.full((B, H, L), float("-inf"), dtype=torch.float32, device=q.device)
+        _need_gpu(q)
+        parts = _PartialResults(q.shape, q)
         for b in range(nb):
-            ob, lb = attn_fwd(q, ks[b], vs[b], causal=(b == causal_block), scale=softmax_scale)
-            lse_merge_(acc, lse, ob, lb)
-        out = cast_from_f32(acc, q.dtype)
+            parts.add(*attn_fwd(q, ks[b], vs[b], causal=(b == causal_block), scale=softmax_scale))
+        out, lse = parts.result()
         ctx.save_for_backward(q, out, lse, *kv)
         ctx.causal_block, ctx.softmax_scale = causal_block, softmax_scale
         ctx.mark_non_differentiable(lse)
@@ -896,7 +929,7 @@ class ZigzagRingRankAttnFunc(torch.autograd.Function):
         source rank < r  all local queries x the FIRST chunk of the block, fully visible
         source rank > r  the queries of the SECOND local chunk x the whole block, fully visible
 
-    Every step's (out, lse) is merged into fp32 running pairs (one per local chunk); backward runs the per-step
+    The steps' (out, lse) are merged in fp32; backward runs the per-step
     flash backward with the final out / lse, a running fp32 dq, and returns each block's dK / dV (zero in the
     half a step did not read), which the ring would send on with the block.
 
@@ -923,21 +956,16 @@ class ZigzagRingRankAttnFunc(torch.autograd.Function):
         for t in kv:
             if t.shape[1] != L2:
                 raise ValueError(f"every block holds two chunks of {c} tokens, got {tuple(t.shape)}")
-        acc = [torch.zeros((B, c, H, D), dtype=torch.float32, device=q.device) for _ in range(2)]
-        lse = [torch.full((B, H, c), float("-inf"), dtype=torch.float32, device=q.device) for _ in range(2)]
+        parts = _PartialResults(q.shape, q)
         for s, ((q0, q1), (k0, k1), causal) in enumerate(ZigzagRingRankAttnFunc._steps(rank, world)):
-            ob, lb = attn_fwd(q[:, q0 * c:q1 * c], ks[s][:, k0 * c:k1 * c], vs[s][:, k0 * c:k1 * c], causal=causal,
-                              scale=softmax_scale)
-            for i, ch in enumerate(range(q0, q1)):
-                lb_ch = lb if q1 - q0 == 1 else lb[:, :, i * c:(i + 1) * c].contiguous()
-                lse_merge_(acc[ch], lse[ch], ob[:, i * c:(i + 1) * c], lb_ch)
-        out = torch.cat([cast_from_f32(a, q.dtype) for a in acc], dim=1)
-        lse_full = torch.cat(lse, dim=2)
-        ctx.save_for_backward(q, out, lse_full, *kv)
+            parts.add(*attn_fwd(q[:, q0 * c:q1 * c], ks[s][:, k0 * c:k1 * c], vs[s][:, k0 * c:k1 * c], causal=causal,
+                                scale=softmax_scale), first=q0 * c)
+        out, lse = parts.result()
+        ctx.save_for_backward(q, out, lse, *kv)
         ctx.rank, ctx.world, ctx.softmax_scale = rank, world, softmax_scale
-        ctx.mark_non_differentiable(lse_full)
+        ctx.mark_non_differentiable(lse)
         ctx.set_materialize_grads(False)
-        return out, lse_full
+        return out, lse
 
     @staticmethod
     def backward(ctx, dout, _dlse):

@@ -190,6 +190,40 @@ def test_ring_backward_fp32_dq_and_reused_query_side(dev):
         ops.attn_bwd(qg, kg[0], vg[0], out, lse, dog, causal=False, reuse_query_side=True)
 
 
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("parts", [0, 1, 3, 8, 9, 19])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32], ids=["bf16", "f32"])
+def test_partial_results_in_one_merge(dtype, parts, D, dev):
+    """Parts of all rows, of the first and of the last ones, parts that saw no key, and more parts than one launch takes, against the
+    sum in 64 bits.  The weights and the sum over n parts are fp32: n + 8 roundings, and one more in the result's own format."""
+    from odysseus_transformer_amd import ops
+    B, L, H = 2, 37, 3
+    like = torch.empty((B, L, H, D), dtype=dtype, device=dev)
+    merge = ops._PartialResults(like.shape, like)
+    num, den = torch.zeros((B, L, H, D), dtype=torch.float64), torch.zeros((B, L, H, 1), dtype=torch.float64)
+    size = torch.zeros((B, L, H, D), dtype=torch.float64)   # of the terms
+    for n in range(parts):
+        first, rows = [(0, L), (0, 20), (20, L - 20), (36, 1)][n % 4]
+        o, lse = randn((B, rows, H, D), 700 + n, dtype=dtype), randn((B, H, rows), 800 + n, std=3.0)
+        if n % 3 == 2:
+            o[:, ::2], lse[:, :, ::2] = 0, float("-inf")
+        merge.add(o.to(dev), lse.to(dev), first)
+        w = lse.double().exp().permute(0, 2, 1)[..., None]
+        num[:, first:first + rows] += w * o.double()
+        size[:, first:first + rows] += w * o.double().abs()
+        den[:, first:first + rows] += w
+    out, lse = merge.result()
+    torch.cuda.synchronize()
+    seen = den > 0
+    ref = torch.where(seen, num / den.clamp_min(1e-300), torch.zeros_like(num))
+    bound = (parts + 8) * 2.0 ** -24 * 4 * size / den.clamp_min(1e-300) + (2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -23) * ref.abs()
+    assert out.dtype == dtype and out.is_contiguous() and bool(((out.double().cpu() - ref).abs() <= bound).all())
+    lref = torch.where(seen, den.clamp_min(1e-300).log(), torch.full_like(den, float("-inf")))[..., 0].permute(0, 2, 1)
+    got = lse.double().cpu()
+    assert torch.equal(torch.isinf(got), torch.isinf(lref))
+    assert bool(((got - lref).abs()[~torch.isinf(lref)] <= (parts + 8) * 2.0 ** -24 * 16).all())   # |lse| < 16
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32], ids=["bf16", "f32"])
 def test_ring_blocks_autograd_function(dtype, dev):
     """ops.ring_blocks_attn (forward merge + backward over blocks under autograd) vs. the oracle's ring loop."""
