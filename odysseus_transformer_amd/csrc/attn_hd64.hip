@@ -571,9 +571,15 @@ int ody_launch_attn_fwd_hd64(const AttnParams& p, hipStream_t st) {
                              : launch("attn_fwd_hd64", &attn_fwd_hd64_kernel<1>, blocks, 1, KV_STAGE, st, p);
 }
 
-// [-delta | -lse / scale | fp32 dK / dV of every query head]; with less room -delta alone
+// [-delta | -lse / scale | fp32 dK / dV of every query head]; with less room -delta alone.  Without query heads to split, room for the second is
+// asked where the dK / dV kernel of attn_hd64_pipe.hip reads it and has a quarter of the chip's units to run on: below, callers keep the
+// workspace that they had, and the former kernel (whole backward, us, former / that one: 4 heads, L = 1000, 32 blocks, 42.7 / 40.1; 4 heads,
+// L = 500 29.0 / 27.7; above the line 8 heads, L = 1000, 64 blocks, 42.9 / 40.1, 4 heads, L = 4000 125 / 114).
 size_t ody_attn_bwd_hd64_workspace(int B, int Lq, int Lk, int Hq, int Hkv) {
-  return delta_bytes(B, Lq, Hq) + lse_bytes(B, Lq, Hq) + (split_heads(B, Lk, Hq, Hkv) ? align256((size_t)2 * B * Hq * Lk * D * sizeof(float)) : 0);
+  if (split_heads(B, Lk, Hq, Hkv))
+    return delta_bytes(B, Lq, Hq) + lse_bytes(B, Lq, Hq) + align256((size_t)2 * B * Hq * Lk * D * sizeof(float));
+  const bool pipe = Hq == Hkv && Lq > 5 * ROWS && row_blocks(B, Lk, Hq) >= 64;
+  return delta_bytes(B, Lq, Hq) + (pipe ? lse_bytes(B, Lq, Hq) : 0);
 }
 
 int ody_launch_attn_bwd_hd64(const AttnParams& p, void* workspace, size_t workspace_bytes, hipStream_t st) {
