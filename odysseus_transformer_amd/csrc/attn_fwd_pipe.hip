@@ -155,7 +155,9 @@ __global__ __launch_bounds__(FW_THREADS, 1) void attn_fwd_pipe_kernel(const Attn
 #pragma unroll
       for (int r = 0; r < 16; r++) o[qt][dt][r] = 0.f;
   float ref_c[FW_QT] = {0.f, 0.f};          // reference * scale * log2(e); 0 for a query that sees no key
-  float l2[FW_QT][2] = {{0.f, 0.f}, {0.f, 0.f}};   // this lane's partial row sums (independent chains)
+  // this lane's partial row sums in four chains, for the roundings of a sum in order grow with its length: rms error of lse against 64 bits, 4 heads,
+  // L = 32768, causal, 6.7e-7 with two chains, 5.4e-7 with four; 32768 keys, full, 8.2e-7 and 6.0e-7.  The time is the same.
+  float l4[FW_QT][4] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
 
   f32x16 s[2][FW_QT];        // [sub-tile][half of the queries]
   bf16x8 pb[2][FW_QT][2];    // P of a sub-tile
@@ -170,7 +172,7 @@ __global__ __launch_bounds__(FW_THREADS, 1) void attn_fwd_pipe_kernel(const Attn
   };
   auto take = [&](int e) INLINE {   // element e: into the row sum, and, in pairs, among the operands
     const int kt = (e & 63) < 32, qt = (e >> 4) & 1, r = e & 15;
-    l2[qt][r & 1] += x1;
+    l4[qt][r & 3] += x1;
     if (r & 1) pb[kt][qt][r >> 3][(r & 7) - 1] = (bf16)x2, pb[kt][qt][r >> 3][r & 7] = (bf16)x1;
   };
   auto weight = [&](int e, int t, auto masked) INLINE {
@@ -324,7 +326,7 @@ __global__ __launch_bounds__(FW_THREADS, 1) void attn_fwd_pipe_kernel(const Attn
 #pragma unroll
   for (int qt = 0; qt < FW_QT; qt++) {
     const int qi = wq0 + 32 * qt + i;
-    const float lt = half_swap_sum(l2[qt][0] + l2[qt][1]);
+    const float lt = half_swap_sum((l4[qt][0] + l4[qt][1]) + (l4[qt][2] + l4[qt][3]));
     float zero[4] = {0.f, 0.f, 0.f, 0.f};   // 0 times the accumulators of O: 0 unless one of them is not finite
 #pragma unroll
     for (int dt = 0; dt < DT; dt++)

@@ -110,7 +110,7 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_hd64_pipe_kernel(const AttnPa
   }
   const float c2 = p.scale_log2e;
   f32x16 o[FW_QT][DT], s[2][FW_QT];
-  float ref[FW_QT], l2[FW_QT][2];   // a row's reference in log2 units; this lane's partial row sums
+  float ref[FW_QT], l4[FW_QT][4];   // a row's reference in log2 units; this lane's partial row sums (four chains: attn_fwd_pipe.hip)
   bf16x8 pb[2][FW_QT][2];
   Readers<D> rd;
   rd.init(kring, g, i);   // rows of K from its row[] on; columns of V from its tr[] + the rings' distance on
@@ -127,7 +127,7 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_hd64_pipe_kernel(const AttnPa
   auto take = [&](int e) INLINE {   // pair e: into the row sums and among the operands
     const int kt = (e & 31) < 16, qt = (e >> 3) & 1, r = 2 * (e & 7);
 #pragma unroll
-    for (int n = 0; n < 2; n++) l2[qt][n] += x[n], pb[kt][qt][r >> 3][(r & 7) + n] = (bf16)x[n];
+    for (int n = 0; n < 2; n++) l4[qt][(r & 3) + n] += x[n], pb[kt][qt][r >> 3][(r & 7) + n] = (bf16)x[n];
   };
   auto weigh = [&](int e, int t, auto masked) INLINE {
     const float x0 = ody_exp2(y[0]), x1 = ody_exp2(y[1]);
@@ -199,13 +199,14 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_hd64_pipe_kernel(const AttnPa
     pv_phase(c1, kslot(t + 2), 24, t, 0, masked);
   };
 
+  auto row_sum = [&](int qt) INLINE { return (l4[qt][0] + l4[qt][1]) + (l4[qt][2] + l4[qt][3]); };
   // The reference of a row is the largest score of its first tile (a row that sees any key sees key 0) and stays.
   auto clear_rows = [&]() INLINE {
 #pragma unroll
     for (int qt = 0; qt < FW_QT; qt++) {
       clear(o[qt]);
       ref[qt] = -FLT_MAX;   // no score is below it; not minus infinity, from which a masked score would be NaN
-      l2[qt][0] = l2[qt][1] = 0.f;
+      l4[qt][0] = l4[qt][1] = l4[qt][2] = l4[qt][3] = 0.f;
     }
   };
   auto scores = [&](int t) INLINE {
@@ -307,7 +308,7 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_hd64_pipe_kernel(const AttnPa
       for (int dt = 0; dt < DT; dt++)
 #pragma unroll
         for (int r = 0; r < 16; r++) zero[r & 3] = fmaf(o[qt][dt][r], 0.f, zero[r & 3]);
-      beyond |= !((zero[0] + zero[1]) + (zero[2] + zero[3]) == 0.f) || !(half_swap_sum(l2[qt][0] + l2[qt][1]) < 0x1p100f);
+      beyond |= !((zero[0] + zero[1]) + (zero[2] + zero[3]) == 0.f) || !(half_swap_sum(row_sum(qt)) < 0x1p100f);
     }
     const int mine = __builtin_amdgcn_ballot_w64(beyond) != 0;
     if (lane == 0) flags[wave] = mine;
@@ -328,7 +329,8 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_hd64_pipe_kernel(const AttnPa
           for (int qt = 0; qt < FW_QT; qt++) {
             const float next = fmaxf(ref[qt], largest(qt, t)), alpha = ody_exp2(ref[qt] - next);
             ref[qt] = next;
-            l2[qt][0] *= alpha, l2[qt][1] *= alpha;
+#pragma unroll
+            for (int e = 0; e < 4; e++) l4[qt][e] *= alpha;
 #pragma unroll
             for (int dt = 0; dt < DT; dt++)
 #pragma unroll
@@ -350,7 +352,7 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_hd64_pipe_kernel(const AttnPa
 #pragma unroll
   for (int qt = 0; qt < FW_QT; qt++) {
     const int qi = wq0 + 32 * qt + i;
-    const float l = half_swap_sum(l2[qt][0] + l2[qt][1]);
+    const float l = half_swap_sum(row_sum(qt));
     if (qi >= p.Lq) continue;
     const float inv = l > 0.f ? 1.f / l : 0.f;
     store_row(static_cast<bf16*>(p.out) + b * p.so.b + h * p.so.h + (int64_t)qi * p.so.l, o[qt], inv, g);

@@ -1,5 +1,7 @@
 """GPU parity of the long-sequence forward (csrc/attn_fwd_pipe.hip) where its ring and its phases can go wrong: key ranges of one tile, of fewer
 tiles than the ring holds and of one more, ragged last tiles, wavefronts without a key, first tiles that need the mask, strided keys."""
+import math
+
 import pytest
 import torch
 
@@ -65,3 +67,22 @@ def test_keys_far_apart(stride, dev):
     near = ops.attn_fwd(q.to(dev), k.to(dev), v.to(dev), causal=False)
     assert_parity(o, near[0].float().cpu(), TOL_BF16, "o")
     assert torch.allclose(lse, near[1], atol=TOL_LSE, rtol=TOL_LSE)
+
+
+@pytest.mark.parametrize("causal", [False, True], ids=["full", "causal"])
+@pytest.mark.parametrize("D", [64, 128])
+def test_row_sums_of_many_small_weights(D, causal, dev):
+    """The first key has weight 1, every other one 2^-24.5, less than half of the last bit of 1: what is added to a sum that holds the first key is
+    lost.  A row is summed in four chains by each half of a wavefront, so that this is an eighth of the keys (0.15: with the roundings of lse,
+    below 1e-6); with two chains it is a quarter."""
+    from odysseus_transformer_amd import ops
+    L, H = (4096, 48) if causal else (256, 256)
+    Lk = max(L, 8192)
+    q, k = torch.zeros((1, L, H, D)), torch.zeros((1, Lk, 1, D))
+    q[..., 0], k[:, 1:, :, 0] = 1.0, -24.5
+    v = randn((1, Lk, 1, D), 45, dtype=torch.bfloat16)
+    (o, lse), ran = _ran(lambda: ops.attn_fwd(q.bfloat16().to(dev), k.bfloat16().to(dev), v.to(dev), causal=causal, scale=math.log(2.0)))
+    assert ("attn_fwd_pipe" if D == 128 else "attn_fwd_hd64_pipe") in ran, ran
+    seen = torch.arange(Lk - L + 1, Lk + 1) if causal else torch.full((L,), Lk)
+    small = (seen - 1).double() * 2.0 ** -24.5
+    assert bool(((lse.cpu().double() - small.log1p()).abs() <= 0.15 * small + 1e-6).all())
