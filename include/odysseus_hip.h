@@ -129,7 +129,9 @@ int ody_attn_fwd_noalloc(const void* q, const void* k, const void* v, void* out,
  *                             blocks and rounded once by the caller at the end (ody_cast_from_f32);
  *   ODY_BWD_REUSE_QUERY_SIDE  q, out, lse, dout and the workspace are those of the previous call: delta and
  *                             the other query-side scratch in the workspace are taken as they are (the ring
- *                             step calls once per key block with the same queries);
+ *                             step calls once per key block with the same queries); for bf16 and head_dim 128
+ *                             Lk and scale are those of that call too (where the scratch lies goes by Lk, and
+ *                             scale is in it);
  *   ODY_BWD_KEEP_DS           spends memory to save arithmetic (no counterpart in the reference): the dK/dV
  *                             kernel keeps dS, rounded to bf16 as it is used there, in the workspace, and dQ is
  *                             one product dS K over it instead of a second pass over S, dP and dS.  Same

@@ -202,13 +202,13 @@ __global__ __launch_bounds__(256 * GROUPS, 4) void attn_fwd_hd64_kernel(const At
 }
 
 // ---------------------------------------------------------------------------------------------------------- backward
-// Start values in fp32: -delta of every query row, (B, Hq, Lq), and, unless null, -lse / scale, (B, Hq, Lq rounded up to whole tiles), minus infinity
-// where P must be 0: past the end, or a query that saw no key.  8 lanes per row.
+// Start values in fp32, either of them null where the call does not need it: -delta of every query row, (B, Hq, Lq), and -lse / scale,
+// (B, Hq, Lq rounded up to whole tiles), minus infinity where P must be 0: past the end, or a query that saw no key.  8 lanes per row.
 __global__ __launch_bounds__(256) void attn_bwd_hd64_rows_kernel(const AttnParams p, float* __restrict__ neg_delta,
                                                                  float* __restrict__ neg_lse) {
   const int lane8 = threadIdx.x & 7, qi = blockIdx.x * 32 + (threadIdx.x >> 3), h = blockIdx.y, b = blockIdx.z;
   float acc = 0.f;
-  if (qi < p.Lq) {
+  if (neg_delta && qi < p.Lq) {
     const bf16x8 ov = *reinterpret_cast<const bf16x8*>(static_cast<const bf16*>(p.out) + b * p.so.b + h * p.so.h + (int64_t)qi * p.so.l + 8 * lane8);
     const bf16x8 dv = *reinterpret_cast<const bf16x8*>(static_cast<const bf16*>(p.dout) + b * p.sdo.b + h * p.sdo.h + (int64_t)qi * p.sdo.l + 8 * lane8);
 #pragma unroll
@@ -218,13 +218,12 @@ __global__ __launch_bounds__(256) void attn_bwd_hd64_rows_kernel(const AttnParam
   for (int sft = 4; sft > 0; sft >>= 1) acc += __shfl_xor(acc, sft, 64);
   if (lane8 != 0) return;
   const int64_t head = (int64_t)b * p.Hq + h;
-  float l = INFINITY;
-  if (qi < p.Lq) {
-    neg_delta[head * p.Lq + qi] = -acc;
-    l = p.lse[head * p.Lq + qi];
-  }
   const int rows = (p.Lq + ROWS - 1) / ROWS * ROWS;
-  if (neg_lse && qi < rows) neg_lse[head * rows + qi] = l == INFINITY || l == -INFINITY ? -INFINITY : -l / p.scale;
+  if (neg_delta && qi < p.Lq) neg_delta[head * p.Lq + qi] = -acc;
+  if (neg_lse && qi < rows) {
+    const float l = qi < p.Lq ? p.lse[head * p.Lq + qi] : INFINITY;
+    neg_lse[head * rows + qi] = l == INFINITY || l == -INFINITY ? -INFINITY : -l / p.scale;
+  }
 }
 
 //   S = Q K^T - lse / scale     dP = dO V^T - delta     dV^T += dO^T P     dK^T += Q^T (P o dP)      lane = key column
@@ -586,21 +585,26 @@ int ody_launch_attn_bwd_hd64(const AttnParams& p, void* workspace, size_t worksp
   float* neg_delta = static_cast<float*>(workspace);
   float* neg_lse = reinterpret_cast<float*>(static_cast<char*>(workspace) + delta_bytes(p.B, p.Lq, p.Hq));
   float* part = reinterpret_cast<float*>(reinterpret_cast<char*>(neg_lse) + lse_bytes(p.B, p.Lq, p.Hq));
-  const bool lse_room = workspace_bytes >= delta_bytes(p.B, p.Lq, p.Hq) + lse_bytes(p.B, p.Lq, p.Hq);
+  const bool heads = split_heads(p.B, p.Lk, p.Hq, p.Hkv) && workspace_bytes >= ody_attn_bwd_hd64_workspace(p.B, p.Lq, p.Lk, p.Hq, p.Hkv);
+  // dK / dV with one query head per block, in the order of attn_hd64_pipe.hip.  Whole backward before / with it, us: 16 heads, L = 8192, causal
+  // 520 / 472, full 992 / 890; 8 heads of it 386 / 308; 16 heads, L = 4096, causal 206 / 164; 4 x 32 heads, L = 500, 57.1 / 52.3.  With fewer than 6
+  // tiles of queries its prologue shows: 32 x 16 heads, L = 300, 96.2 / 97.5; 64 x 16 heads, L = 256, causal 113.7 / 116.
+  const bool pipe = workspace_bytes >= delta_bytes(p.B, p.Lq, p.Hq) + lse_bytes(p.B, p.Lq, p.Hq) && (heads || p.group == 1) && p.Lq > 5 * ROWS &&
+                    near(p.sq, p.sdo);
   int rc;
-  if (!p.reuse_query_side) {   // -lse / scale for a later call that reuses it, too, whichever kernel that one takes
-    ODY_LAUNCH("attn_bwd_hd64_rows", st, attn_bwd_hd64_rows_kernel, dim3((p.Lq + ROWS - 1) / ROWS * (ROWS / 32), p.Hq, p.B), dim3(256), 0, p, neg_delta,
-               lse_room ? neg_lse : nullptr);
+  // Of a reused query side -delta alone is taken as it is: whether the call before wrote -lse / scale, and with this scale, depends on the keys
+  // and the workspace that it had.
+  if (!p.reuse_query_side || pipe) {
+    const dim3 grid((p.Lq + ROWS - 1) / ROWS * (ROWS / 32), p.Hq, p.B);
+    if (p.reuse_query_side)
+      ODY_LAUNCH("attn_bwd_hd64_lse", st, attn_bwd_hd64_rows_kernel, grid, dim3(256), 0, p, nullptr, neg_lse);
+    else
+      ODY_LAUNCH("attn_bwd_hd64_rows", st, attn_bwd_hd64_rows_kernel, grid, dim3(256), 0, p, neg_delta, pipe ? neg_lse : nullptr);
     if ((rc = ody_check_launch("attn_bwd_hd64_rows"))) return rc;
   }
-  const bool heads = split_heads(p.B, p.Lk, p.Hq, p.Hkv) && workspace_bytes >= ody_attn_bwd_hd64_workspace(p.B, p.Lq, p.Lk, p.Hq, p.Hkv);
   const int64_t nkv = row_blocks(p.B, p.Lk, heads ? p.Hq : p.Hkv), nq = row_blocks(p.B, p.Lq, p.Hq);
   auto dkdv = [&](auto kern, int groups) { return launch("attn_bwd_hd64_dkdv", kern, nkv, groups, QS_STAGE, st, p, neg_delta, part); };
-  // One query head per block, in the order of attn_hd64_pipe.hip.  Whole backward before / with it, us: 16 heads, L = 8192, causal 520 / 472, full
-  // 992 / 890; 8 heads of it 386 / 308; 16 heads, L = 4096, causal 206 / 164; 4 x 32 heads, L = 500, 57.1 / 52.3.  With fewer than 6 tiles of
-  // queries its prologue shows: 32 x 16 heads, L = 300, 96.2 / 97.5; 64 x 16 heads, L = 256, causal 113.7 / 116.
-  if (lse_room && (heads || p.group == 1) && p.Lq > 5 * ROWS && near(p.sq, p.sdo))
-    rc = ody_launch_attn_bwd_hd64_dkdv_pipe(p, neg_delta, neg_lse, heads ? part : nullptr, st);
+  if (pipe) rc = ody_launch_attn_bwd_hd64_dkdv_pipe(p, neg_delta, neg_lse, heads ? part : nullptr, st);
   else if (nkv < FEW_BLOCKS) rc = heads ? dkdv(&attn_bwd_hd64_dkdv_kernel<2, true>, 2) : dkdv(&attn_bwd_hd64_dkdv_kernel<2, false>, 2);
   else rc = heads ? dkdv(&attn_bwd_hd64_dkdv_kernel<1, true>, 1) : dkdv(&attn_bwd_hd64_dkdv_kernel<1, false>, 1);
   if (rc) return rc;

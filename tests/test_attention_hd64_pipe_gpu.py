@@ -90,6 +90,23 @@ def test_the_same_bits_again_and_a_reused_query_side(dev):
         assert all(torch.equal(a, b) for a, b in zip(first, again))
 
 
+@pytest.mark.parametrize("Hkv,first", [(8, 100), (4, 1100), (8, 1100)])
+def test_a_reused_query_side_behind_other_keys(Hkv, first, dev):
+    """Every call with the workspace of its own size, from one buffer: the one before had fewer keys and took the other dK / dV kernel, or the same
+    one, which left start values of another scale."""
+    from odysseus_transformer_amd import ops
+    q, k, v, do = (t.to(dev) for t in _inputs(1, 900, 1100, 8, Hkv, 75))
+    o, lse = ops.attn_fwd(q, k, v, causal=False)
+    want = ops.attn_bwd(q, k, v, o, lse, do, causal=False)
+    whole = torch.full_like(ops.attn_bwd_workspace(q, k), 255)
+    few, fewv = k[:, :first], v[:, :first]
+    part = whole[:ops.attn_bwd_workspace_bytes(q, few)]
+    ops.attn_bwd(q, few, fewv, o, lse, do, causal=False, workspace=part, scale=0.1)
+    got, ran = _ran(lambda: ops.attn_bwd(q, k, v, o, lse, do, causal=False, workspace=whole, reuse_query_side=True))
+    assert DKDV in ran and "attn_bwd_hd64_rows" not in ran, ran
+    assert all(torch.equal(a, b) for a, b in zip(want, got))
+
+
 @pytest.mark.parametrize("stride", [64, 1 << 23, (1 << 24) - 16, (1 << 24) - 8], ids=str)
 def test_rows_far_apart(stride, dev):
     """Row strides up to the last one whose tile fits 32-bit offsets, and the first one beyond: keys of the forward, queries of dK / dV."""
