@@ -549,16 +549,24 @@ int launch(const char* name, K kern, int64_t blocks, int groups, size_t stage_el
 // The kernels of attn_hd64_pipe.hip address a tile with 32-bit byte offsets.
 inline bool near(const AttnStrides& a, const AttnStrides& b) { return a.l < tile128::TILE_MAX_STRIDE && b.l < tile128::TILE_MAX_STRIDE; }
 
-// The forward with 256-row blocks, two to a compute unit, where they fill the chip.  Before / with it, us: full, 16 heads, L = 8192, 308 / 265;
-// 4 x 32 heads, L = 1000, 48.6 / 44.3; 16 heads, L = 4096, 256 blocks, 89 / 82; 12 heads of that, 192 blocks, 75 / 81; 4 x 32 heads, L = 512,
-// 16.8 / 16.7.  Causal, where one block is many times as long as another, only with three blocks for every unit or more and, since every block
-// has a prologue, long rows: 24 heads, L = 8192, 239 / 219; 32 heads, L = 2048 x 4, 91.7 / 89.3; 16 heads, L = 8192, 512 blocks, 179 / 173 by
-// itself and 5 us behind before a backward; 16 heads, L = 2048 x 4, 512 blocks, 49.1 / 50.1; 24 heads, L = 4096, 384 blocks, 76 / 79;
-// 64 x 16 heads, L = 256, 36.2 / 37.2.  A last block that is half empty costs its share of the rows.
+// The forward with 256-row blocks.  Before / with it, us:
+//   Full.  A compute unit takes these blocks by whole rounds of 256, the former kernel's by half rounds, so that a last round at most half full goes to
+//   the former one, unless there are rounds enough, the fewer the longer the rows, for the 5 to 17 % per round to make up for it.  512 keys: 16 heads,
+//   L = 8192, 512 blocks, 26.5 / 25.3, 9 heads, 288 blocks, 19.4 / 23.4, 18 heads 32.9 / 34.5; 1000 keys, 4 x 64 heads, L = 1000, 91 / 79, 75 heads, 300 blocks,
+//   34.9 / 37.5; 4096 keys, 57 heads, L = 2100, of whose last blocks half is empty, 155 / 177.  16 heads, L = 8192, 308 / 265.  None of 605 shapes from 192
+//   blocks and 512 keys on is behind by more than 1 % this way.
+//   Causal, where one block is many times as long as another, with three blocks for every unit or more, and work enough in all of them:
+//   64 x 48 heads, L = 256, 768 blocks, 30.1 / 31.5, 128 x 64 heads of it 333 / 285; 8 x 48 heads, L = 512, 33.9 / 35.3, 32 x 64 heads 207 / 174;
+//   1 x 24 heads, L = 8192, 235 / 213, 16 heads, 512 blocks, 179 / 173 by itself and 5 us behind before a backward; 48 heads, L = 4096, 128 / 117,
+//   24 heads, 384 blocks, 76 / 79.
+// A last block that is half empty costs its share of the rows.
 inline bool fwd_pipe_ok(const AttnParams& p) {
   const int64_t halves = (p.Lq + BLOCK_ROWS - 1) / BLOCK_ROWS, blocks = (int64_t)p.B * p.Hq * ((halves + 1) / 2);
   if (!near(p.sk, p.sv) || ((halves & 1) && halves < 16)) return false;
-  return p.causal ? blocks >= 768 && blocks * p.Lk >= (1 << 21) : blocks >= 256 && p.Lk >= 512;
+  if (p.causal) return blocks >= 768 && blocks * p.Lk >= (1 << 21);
+  const int64_t former = (int64_t)p.B * p.Hq * halves, rounds = (blocks + 255) / 256, lost = 2 * rounds - (former + 255) / 256;   // half rounds
+  if (former < FEW_BLOCKS || p.Lk < (rounds == 1 ? 640 : 512)) return false;
+  return lost == 0 || (lost == 1 && rounds > (p.Lk >= 2048 ? 2 : p.Lk >= 1024 ? 4 : 7));
 }
 
 }  // namespace

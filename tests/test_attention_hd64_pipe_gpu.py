@@ -54,7 +54,7 @@ def _check(B, Lq, Lk, Hq, Hkv, causal, fwd, dkdv, dev, seed=61, heads=None, stre
 @pytest.mark.parametrize("stretch", [1.0, 60.0], ids=["unit", "moving_reference"])
 @pytest.mark.parametrize("Lq,Lk", [(512, 512), (505, 513), (1024, 575), (1000, 639), (2049, 641)])
 def test_full(Lq, Lk, stretch, dev):
-    H = 256 // ((Lq + 255) // 256) + 1
+    H = 512 // ((Lq + 255) // 256)   # two whole rounds of 256 blocks
     _check(1, Lq, Lk, H, H, False, True, True, dev, heads=3, stretch=stretch)
 
 
@@ -76,6 +76,15 @@ def test_few_keys_or_queries(B, Lq, Lk, Hq, Hkv, causal, dev):
                                             (2048, 2048, 127, True), (4096, 4096, 47, True), (1000, 1000, 7, True), (1000, 1000, 8, False)])
 def test_calls_that_stay_with_the_kernels_for_few_blocks(Lq, Lk, H, causal, dev):
     _check(1, Lq, Lk, H, H, causal, False, Lq > 320 and H * ((Lk + 127) // 128) >= 64, dev, heads=2)
+
+
+# at the lines that rounds draw: forward, a last round that is full, more or less than half full, of few rounds and of many
+@pytest.mark.parametrize("Lq,Lk,H,causal,fwd,dkdv", [(1000, 600, 75, False, False, True), (1000, 600, 98, False, True, True), (1000, 650, 64, False, True, True),
+                                                     (1000, 600, 64, False, False, True), (2100, 600, 44, False, False, True), (260, 520, 512, False, False, False),
+                                                     (512, 1024, 258, False, False, True), (512, 1024, 514, False, True, True), (1000, 550, 385, False, False, True),
+                                                     (961, 961, 65, True, False, True), (708, 708, 85, True, False, True)])
+def test_last_rounds(Lq, Lk, H, causal, fwd, dkdv, dev):
+    _check(1, Lq, Lk, H, H, causal, fwd, dkdv, dev, heads=2)
 
 
 def test_the_same_bits_again_and_a_reused_query_side(dev):
