@@ -596,9 +596,12 @@ int ody_launch_attn_bwd_hd64(const AttnParams& p, void* workspace, size_t worksp
   const bool heads = split_heads(p.B, p.Lk, p.Hq, p.Hkv) && workspace_bytes >= ody_attn_bwd_hd64_workspace(p.B, p.Lq, p.Lk, p.Hq, p.Hkv);
   // dK / dV with one query head per block, in the order of attn_hd64_pipe.hip.  Whole backward before / with it, us: 16 heads, L = 8192, causal
   // 520 / 472, full 992 / 890; 8 heads of it 386 / 308; 16 heads, L = 4096, causal 206 / 164; 4 x 32 heads, L = 500, 57.1 / 52.3.  With fewer than 6
-  // tiles of queries its prologue shows: 32 x 16 heads, L = 300, 96.2 / 97.5; 64 x 16 heads, L = 256, causal 113.7 / 116.
-  const bool pipe = workspace_bytes >= delta_bytes(p.B, p.Lq, p.Hq) + lse_bytes(p.B, p.Lq, p.Hq) && (heads || p.group == 1) && p.Lq > 5 * ROWS &&
-                    near(p.sq, p.sdo);
+  // tiles of queries its prologue shows: 32 x 16 heads, L = 300, 96.2 / 97.5; 64 x 16 heads, L = 256, causal 113.7 / 116.  A unit holds two of its
+  // blocks and three of the former kernel's, so that beyond 512 of them it wants rows long enough for the tail not to count: full, 8 x 32 heads,
+  // L = 384, 0.98, L = 512 1.02; causal, 4 x 32 heads, L = 708, 59.0 / 63.0, 8 x 32 heads, L = 321, 0.88, 4 x 32 heads, L = 1000, 1.03.
+  const int64_t blocks = row_blocks(p.B, p.Lk, p.Hq);
+  const bool pipe = workspace_bytes >= delta_bytes(p.B, p.Lq, p.Hq) + lse_bytes(p.B, p.Lq, p.Hq) && (heads || p.group == 1) &&
+                    p.Lq > ROWS * (blocks <= 512 ? 5 : p.causal ? 15 : 7) && near(p.sq, p.sdo);
   int rc;
   // Of a reused query side -delta alone is taken as it is: whether the call before wrote -lse / scale, and with this scale, depends on the keys
   // and the workspace that it had.

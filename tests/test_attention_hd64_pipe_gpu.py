@@ -78,11 +78,13 @@ def test_calls_that_stay_with_the_kernels_for_few_blocks(Lq, Lk, H, causal, dev)
     _check(1, Lq, Lk, H, H, causal, False, Lq > 320 and H * ((Lk + 127) // 128) >= 64, dev, heads=2)
 
 
-# at the lines that rounds draw: forward, a last round that is full, more or less than half full, of few rounds and of many
+# at the lines that rounds draw: forward, a last round that is full, more or less than half full, of few rounds and of many; dK / dV, 512 key blocks
+# and more of few and of many queries
 @pytest.mark.parametrize("Lq,Lk,H,causal,fwd,dkdv", [(1000, 600, 75, False, False, True), (1000, 600, 98, False, True, True), (1000, 650, 64, False, True, True),
                                                      (1000, 600, 64, False, False, True), (2100, 600, 44, False, False, True), (260, 520, 512, False, False, False),
                                                      (512, 1024, 258, False, False, True), (512, 1024, 514, False, True, True), (1000, 550, 385, False, False, True),
-                                                     (961, 961, 65, True, False, True), (708, 708, 85, True, False, True)])
+                                                     (708, 708, 128, True, False, False), (961, 961, 65, True, False, True), (708, 708, 85, True, False, True),
+                                                     (448, 600, 128, False, False, False), (449, 600, 128, False, False, True)])
 def test_last_rounds(Lq, Lk, H, causal, fwd, dkdv, dev):
     _check(1, Lq, Lk, H, H, causal, fwd, dkdv, dev, heads=2)
 
