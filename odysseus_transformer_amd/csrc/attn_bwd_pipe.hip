@@ -527,7 +527,9 @@ __global__ __launch_bounds__(KV_THREADS, 1) void attn_bwd_dkdv_pipe_kernel(const
   };
 
   const int rbase = row_frag_base(g, i), ibase = image_frag_base(g, i);
-  const int key_off = p.causal ? wn0 + i - p.off : -(1 << 30);   // + 32 kh: the first query that sees this lane's keys
+  // + 32 kh: the first query that sees this lane's keys; less what of an accumulator's row goes by the lane (acc_tile_row), so that the mask compares
+  // this one register with scalars: with a register per row the loops went to scratch memory
+  const int key_off = p.causal ? wn0 + i - p.off - 16 * g : -(1 << 30);
   f32x16 s, dp;                          // S, then P; dP, then dS
   bf16x8 pf[2], dsf[2], pf_next[2], dsf_next[2];
   // a lane's 16 start values: quarter a of those of S (which = 0) or dP (1) of sub-tile mt
@@ -539,7 +541,7 @@ __global__ __launch_bounds__(KV_THREADS, 1) void attn_bwd_dkdv_pipe_kernel(const
   // the steps of element r of a unit: exponent, P, dS, and two elements together into the operands
   auto exponent = [&](int r, int t, int mt, int kh, auto masked) INLINE {
     float x = s[r] * c2;
-    if (decltype(masked)::value) x = t * KV_BQ + acc_tile_row(r, g, mt) < key_off + 32 * kh ? -INFINITY : x;   // queries before the key
+    if (decltype(masked)::value) x = key_off > t * KV_BQ + acc_tile_row(r, 0, mt) - 32 * kh ? -INFINITY : x;   // queries before the key
     s[r] = x;
   };
   auto weight = [&](int r) INLINE { s[r] = ody_exp2(s[r]); };
@@ -558,6 +560,7 @@ __global__ __launch_bounds__(KV_THREADS, 1) void attn_bwd_dkdv_pipe_kernel(const
   };
   auto rslot = [&](int it) INLINE { return rring + (it & 1) * KV_ROWS; };
   auto islot = [&](int it) INLINE { return iring + (it & 1) * KV_IMAGES; };
+  // (Where dS is kept its stores count as well, so that these waits are for a few more loads than they name.)
   auto barrier_rows = [&]() INLINE {     // the rows of the next tile have landed (behind them 8 loads of images); everyone is done with those before
     asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
     __builtin_amdgcn_s_barrier();
