@@ -103,45 +103,12 @@ __global__ __launch_bounds__(DP_THREADS, 1) void attn_bwd_dq_pipe_kernel(const A
     w_full = min(w_full, max(0, wq0 + p.off + 1) / DP_BN);
   }
 
-  bf16x8 qf[DP_QT][KS], dof[DP_QT][KS];
-  f32x16 minus_delta[DP_QT];   // what dP starts from
-  float lse2[DP_QT];
-  int lim[DP_QT];
-  {
-    const bf16* qp = static_cast<const bf16*>(p.q) + b * p.sq.b + h * p.sq.h;
-    const bf16* dop = static_cast<const bf16*>(p.dout) + b * p.sdo.b + h * p.sdo.h;
-#pragma unroll
-    for (int qt = 0; qt < DP_QT; qt++) {
-      const int qi = wq0 + 32 * qt + i;
-#pragma unroll
-      for (int ks = 0; ks < KS; ks++) {
-        qf[qt][ks] = dof[qt][ks] = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
-        if (qi < p.Lq) {
-          qf[qt][ks] = *reinterpret_cast<const bf16x8*>(qp + (int64_t)qi * p.sq.l + 16 * ks + 8 * g);
-          dof[qt][ks] = *reinterpret_cast<const bf16x8*>(dop + (int64_t)qi * p.sdo.l + 16 * ks + 8 * g);
-        }
-      }
-      const int64_t ri = ((int64_t)b * p.Hq + h) * p.Lq + qi;
-      float l = (qi < p.Lq) ? p.lse[ri] : INFINITY;
-      if (l == -INFINITY) l = INFINITY;   // a query that saw no key: P = 0
-      lse2[qt] = l * ODY_LOG2E;
-      const float delta = (qi < p.Lq) ? p.delta[ri] : 0.f;
-#pragma unroll
-      for (int r = 0; r < 16; r++) minus_delta[qt][r] = -delta;
-      lim[qt] = p.causal ? min(p.Lk - 1, qi + p.off) : p.Lk - 1;
-    }
-  }
-#pragma unroll
-  for (int qt = 0; qt < DP_QT; qt++) {
-    asm volatile("" : "+v"(minus_delta[qt]), "+v"(lse2[qt]));   // arrived before the direct loads
-#pragma unroll
-    for (int ks = 0; ks < KS; ks++) asm volatile("" : "+v"(qf[qt][ks]), "+a"(dof[qt][ks]));
-  }
   const float c2 = p.scale_log2e;
 
   // Direct loads: of the rows of tile `lr` and of the image of tile `li`, the last one again where there are no more.  Rows past the end read
   // zeros: they lie beyond the descriptor.
-  int lr = min(t_first, ntiles - 1), li = lr;
+  const int last_tile = max(ntiles - 1, 0);   // (a block without tiles brings tile 0 and leaves it)
+  int lr = min(t_first, last_tile), li = lr;
   const int krow = 2 * (int)p.sk.l, vrow = 2 * (int)p.sv.l;   // bytes
   const int klane = (4 * wave + (lane >> 4)) * krow + 16 * (lane & 15), vlane = (4 * wave + (lane >> 4)) * vrow + 16 * (lane & 15);
   const int ilane = 1024 * wave + 16 * lane;
@@ -161,17 +128,69 @@ __global__ __launch_bounds__(DP_THREADS, 1) void attn_bwd_dq_pipe_kernel(const A
   };
   auto load_image = [&](int j) INLINE { bring(kip, IMG_BYTES, iring + (li & 1) * IMG_ELEMS + (4 * j + wave) * 512, ilane, 4096 * j); };
   auto next_rows = [&]() INLINE {
-    const int to = min(lr + 1, ntiles - 1), step = to - lr;
+    const int to = min(lr + 1, last_tile), step = to - lr;
     lr = to;
     ktp += (int64_t)step * (DP_BN / 2 * krow);
     vtp += (int64_t)step * (DP_BN / 2 * vrow);
     room -= step * DP_BN;
   };
   auto next_image = [&]() INLINE {
-    const int to = min(li + 1, ntiles - 1), step = to - li;
+    const int to = min(li + 1, last_tile), step = to - li;
     li = to;
     kip += step * IMG_ELEMS;
   };
+
+  auto all_rows = [&]() INLINE {
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      load_rows(j, 0);
+      load_rows(j, 1);
+    }
+  };
+  auto all_image = [&]() INLINE {
+#pragma unroll
+    for (int j = 0; j < 4; j++) load_image(j);
+  };
+
+  // The first tiles, and the queries' side behind the first rows: one wait for memory in front of the first products (attn_fwd_pipe.hip)
+  all_rows();
+  FENCE();
+  bf16x8 qf[DP_QT][KS], dof[DP_QT][KS];
+  f32x16 minus_delta[DP_QT];   // what dP starts from
+  float lse2[DP_QT], delta[DP_QT];
+  int lim[DP_QT];
+  {
+    const bf16* qp = static_cast<const bf16*>(p.q) + b * p.sq.b + h * p.sq.h;
+    const bf16* dop = static_cast<const bf16*>(p.dout) + b * p.sdo.b + h * p.sdo.h;
+#pragma unroll
+    for (int qt = 0; qt < DP_QT; qt++) {
+      const int qi = wq0 + 32 * qt + i, row = min(qi, p.Lq - 1);   // rows past the end: the last one, whose results are not stored
+#pragma unroll
+      for (int ks = 0; ks < KS; ks++) {
+        qf[qt][ks] = *reinterpret_cast<const bf16x8*>(qp + (int64_t)row * p.sq.l + 16 * ks + 8 * g);
+        dof[qt][ks] = *reinterpret_cast<const bf16x8*>(dop + (int64_t)row * p.sdo.l + 16 * ks + 8 * g);
+      }
+      const int64_t ri = ((int64_t)b * p.Hq + h) * p.Lq + row;
+      lse2[qt] = p.lse[ri];
+      delta[qt] = p.delta[ri];
+      lim[qt] = p.causal ? min(p.Lk - 1, qi + p.off) : p.Lk - 1;
+    }
+  }
+  FENCE();
+  all_image();
+  next_rows();
+  all_rows();
+  FENCE();
+#pragma unroll
+  for (int qt = 0; qt < DP_QT; qt++) {
+#pragma unroll
+    for (int ks = 0; ks < KS; ks++) asm volatile("" : "+v"(qf[qt][ks]), "+a"(dof[qt][ks]));
+    if (lse2[qt] == -INFINITY || wq0 + 32 * qt + i >= p.Lq) lse2[qt] = INFINITY;   // a query that saw no key: P = 0
+    lse2[qt] *= ODY_LOG2E;
+#pragma unroll
+    for (int r = 0; r < 16; r++) minus_delta[qt][r] = -delta[qt];
+    asm volatile("" : "+v"(minus_delta[qt]), "+v"(lse2[qt]));
+  }
 
   const int rbase = row_frag_base(g, i), ibase = image_frag_base(g, i);
   f32x16 dq[DP_QT][DT];
@@ -281,21 +300,6 @@ __global__ __launch_bounds__(DP_THREADS, 1) void attn_bwd_dq_pipe_kernel(const A
   std::integral_constant<int, 1> c1;
 
   if (t_first < ntiles) {
-    auto all_rows = [&]() INLINE {
-#pragma unroll
-      for (int j = 0; j < 4; j++) {
-        load_rows(j, 0);
-        load_rows(j, 1);
-      }
-    };
-    auto all_image = [&]() INLINE {
-#pragma unroll
-      for (int j = 0; j < 4; j++) load_image(j);
-    };
-    all_rows();
-    all_image();
-    next_rows();
-    all_rows();
     asm volatile("s_waitcnt vmcnt(12)" ::: "memory");   // the first tile's rows
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
@@ -349,8 +353,8 @@ __global__ __launch_bounds__(DP_THREADS, 1) void attn_bwd_dq_pipe_kernel(const A
       barrier_rows();
       all_rows();
     }
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 
 #pragma unroll
   for (int qt = 0; qt < DP_QT; qt++) {
@@ -453,27 +457,6 @@ __global__ __launch_bounds__(KV_THREADS, 1) void attn_bwd_dkdv_pipe_kernel(const
     w_full = min(total, max(0, t_top + 1 - (max(0, wn0 + 32 * KV_KT - 1 - p.off) + KV_BQ - 1) / KV_BQ));
   }
 
-  bf16x8 kf[KV_KT][KS], vf[KV_KT][KS];
-  {
-    const bf16* kp = static_cast<const bf16*>(p.k) + b * p.sk.b + hk * p.sk.h;
-    const bf16* vp = static_cast<const bf16*>(p.v) + b * p.sv.b + hk * p.sv.h;
-#pragma unroll
-    for (int kh = 0; kh < KV_KT; kh++) {
-      const int key = wn0 + 32 * kh + i;
-#pragma unroll
-      for (int ks = 0; ks < KS; ks++) {
-        kf[kh][ks] = vf[kh][ks] = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
-        if (key < p.Lk) {
-          kf[kh][ks] = *reinterpret_cast<const bf16x8*>(kp + (int64_t)key * p.sk.l + 16 * ks + 8 * g);
-          vf[kh][ks] = *reinterpret_cast<const bf16x8*>(vp + (int64_t)key * p.sv.l + 16 * ks + 8 * g);
-        }
-      }
-    }
-  }
-#pragma unroll
-  for (int kh = 0; kh < KV_KT; kh++)
-#pragma unroll
-    for (int ks = 0; ks < KS; ks++) asm volatile("" : "+v"(kf[kh][ks]), "+v"(vf[kh][ks]));   // arrived before the direct loads
   f32x16 dk[KV_KT][DT], dv[KV_KT][DT];
 #pragma unroll
   for (int kh = 0; kh < KV_KT; kh++)
@@ -485,17 +468,18 @@ __global__ __launch_bounds__(KV_THREADS, 1) void attn_bwd_dkdv_pipe_kernel(const
 
   // Direct loads: of the rows of tile `lr` (from the top) and of the images of tile `li`, the last one again where there are no more.
   // Rows past the end read zeros: they lie beyond the descriptor.
+  const int last_tile = max(total - 1, 0), t_start = max(t_top, 0);   // (a block without tiles brings one and leaves it)
   int lr = 0, li = 0;
   const int qrow = 2 * (int)p.sq.l, orow = 2 * (int)p.sdo.l;   // bytes
   const int qlane = (4 * wave + (lane >> 4)) * qrow + 16 * (lane & 15), olane = (4 * wave + (lane >> 4)) * orow + 16 * (lane & 15);
   const int ilane = 1024 * wave + 16 * lane;
-  const int64_t tile_id = ((int64_t)b * p.Hq + h) * q_tiles + t_top;
-  const bf16* qtp = static_cast<const bf16*>(p.q) + b * p.sq.b + h * p.sq.h + (int64_t)t_top * KV_BQ * p.sq.l;
-  const bf16* otp = static_cast<const bf16*>(p.dout) + b * p.sdo.b + h * p.sdo.h + (int64_t)t_top * KV_BQ * p.sdo.l;
+  const int64_t tile_id = ((int64_t)b * p.Hq + h) * q_tiles + t_start;
+  const bf16* qtp = static_cast<const bf16*>(p.q) + b * p.sq.b + h * p.sq.h + (int64_t)t_start * KV_BQ * p.sq.l;
+  const bf16* otp = static_cast<const bf16*>(p.dout) + b * p.sdo.b + h * p.sdo.h + (int64_t)t_start * KV_BQ * p.sdo.l;
   const bf16* stp = stats + tile_id * KV_STAT_ELEMS;
   const bf16* qip = qimg + tile_id * IMG_ELEMS;
   const bf16* oip = doimg + tile_id * IMG_ELEMS;
-  const int top_rows = min(KV_BQ, p.Lq - t_top * KV_BQ) - 1;
+  const int top_rows = min(KV_BQ, p.Lq - t_start * KV_BQ) - 1;
   int q_bytes = top_rows * qrow + 256, o_bytes = top_rows * orow + 256;
   auto bring = [&](const bf16* src, int bytes, bf16* dst, int off, int soff) INLINE {
     auto rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16*>(src), (short)0, bytes, 0x00020000);
@@ -512,7 +496,7 @@ __global__ __launch_bounds__(KV_THREADS, 1) void attn_bwd_dkdv_pipe_kernel(const
     bring(which ? oip : qip, IMG_BYTES, iring + (li & 1) * KV_IMAGES + which * IMG_ELEMS + (4 * j + wave) * 512, ilane, 4096 * j);
   };
   auto next_rows = [&]() INLINE {
-    const int to = min(lr + 1, total - 1), step = to - lr;
+    const int to = min(lr + 1, last_tile), step = to - lr;
     lr = to;
     qtp -= (int64_t)step * (KV_BQ / 2 * qrow);
     otp -= (int64_t)step * (KV_BQ / 2 * orow);
@@ -520,11 +504,55 @@ __global__ __launch_bounds__(KV_THREADS, 1) void attn_bwd_dkdv_pipe_kernel(const
     if (step) q_bytes = (KV_BQ - 1) * qrow + 256, o_bytes = (KV_BQ - 1) * orow + 256;
   };
   auto next_images = [&]() INLINE {
-    const int to = min(li + 1, total - 1), step = to - li;
+    const int to = min(li + 1, last_tile), step = to - li;
     li = to;
     qip -= step * IMG_ELEMS;
     oip -= step * IMG_ELEMS;
   };
+
+  auto all_rows = [&]() INLINE {
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      load_rows(j, 0);
+      load_rows(j, 1);
+    }
+  };
+  auto all_images = [&]() INLINE {
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      load_images(j, 0);
+      load_images(j, 1);
+    }
+  };
+
+  // The first tiles, and this block's keys behind the first rows: one wait for memory in front of the first products (attn_fwd_pipe.hip).  Of the
+  // second tile not the start values: those the first unit brings, like those of any tile.
+  load_stats();
+  all_rows();
+  FENCE();
+  bf16x8 kf[KV_KT][KS], vf[KV_KT][KS];
+  {
+    const bf16* kp = static_cast<const bf16*>(p.k) + b * p.sk.b + hk * p.sk.h;
+    const bf16* vp = static_cast<const bf16*>(p.v) + b * p.sv.b + hk * p.sv.h;
+#pragma unroll
+    for (int kh = 0; kh < KV_KT; kh++) {
+      const int key = min(wn0 + 32 * kh + i, p.Lk - 1);   // keys past the end: the last one, whose results are not stored
+#pragma unroll
+      for (int ks = 0; ks < KS; ks++) {
+        kf[kh][ks] = *reinterpret_cast<const bf16x8*>(kp + (int64_t)key * p.sk.l + 16 * ks + 8 * g);
+        vf[kh][ks] = *reinterpret_cast<const bf16x8*>(vp + (int64_t)key * p.sv.l + 16 * ks + 8 * g);
+      }
+    }
+  }
+  FENCE();
+  all_images();
+  next_rows();
+  all_rows();
+  FENCE();
+#pragma unroll
+  for (int kh = 0; kh < KV_KT; kh++)
+#pragma unroll
+    for (int ks = 0; ks < KS; ks++) asm volatile("" : "+v"(kf[kh][ks]), "+v"(vf[kh][ks]));
 
   const int rbase = row_frag_base(g, i), ibase = image_frag_base(g, i);
   // + 32 kh: the first query that sees this lane's keys; less what of an accumulator's row goes by the lane (acc_tile_row), so that the mask compares
@@ -646,30 +674,6 @@ __global__ __launch_bounds__(KV_THREADS, 1) void attn_bwd_dkdv_pipe_kernel(const
   };
 
   if (total > 0) {
-    auto all_rows = [&]() INLINE {
-      load_stats();
-#pragma unroll
-      for (int j = 0; j < 4; j++) {
-        load_rows(j, 0);
-        load_rows(j, 1);
-      }
-    };
-    auto all_images = [&]() INLINE {
-#pragma unroll
-      for (int j = 0; j < 4; j++) {
-        load_images(j, 0);
-        load_images(j, 1);
-      }
-    };
-    all_rows();
-    all_images();
-    next_rows();
-    // the rows of the second tile, but for the start values: those the first unit brings, like those of any tile
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-      load_rows(j, 0);
-      load_rows(j, 1);
-    }
     asm volatile("s_waitcnt vmcnt(16)" ::: "memory");   // the first tile's rows
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
@@ -725,14 +729,10 @@ __global__ __launch_bounds__(KV_THREADS, 1) void attn_bwd_dkdv_pipe_kernel(const
       barrier_images();
       all_images();
       barrier_rows();
-#pragma unroll
-      for (int j = 0; j < 4; j++) {
-        load_rows(j, 0);
-        load_rows(j, 1);
-      }
+      all_rows();
     }
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 
 #pragma unroll
   for (int kh = 0; kh < KV_KT; kh++) {

@@ -99,7 +99,8 @@ __global__ __launch_bounds__(FW_THREADS, 1) void attn_fwd_pipe_kernel(const Attn
   }
   const int krow = 2 * (int)p.sk.l;   // bytes
   const int kcol = 16 * (lane & 15), klane = (4 * wave + (lane >> 4)) * krow + kcol, vlane = 1024 * wave + 16 * lane;
-  int lk = min(t_first, ntiles - 1), lv = lk;
+  const int last = max(ntiles - 1, 0);   // (a block without tiles brings tile 0 and leaves it)
+  int lk = min(t_first, last), lv = lk;
   const bf16* lkp = kp + (int64_t)lk * BN * p.sk.l;
   const bf16* lvp = vp + (int64_t)lk * IMG_ELEMS;
   int k_room = p.Lk - 1 - lk * BN;   // rows behind the tile's first one
@@ -115,32 +116,54 @@ __global__ __launch_bounds__(FW_THREADS, 1) void attn_fwd_pipe_kernel(const Attn
                                              vlane, 4096 * j, 0, 0);
   };
   auto next_k = [&]() INLINE {
-    const int to = min(lk + 1, ntiles - 1), step = to - lk;
+    const int to = min(lk + 1, last), step = to - lk;
     lk = to;
     lkp += (unsigned)(step * (BN / 2 * krow));
     k_room -= step * BN;
     k_last = min(k_room, BN - 1) * krow + kcol;
   };
   auto next_v = [&]() INLINE {
-    const int to = min(lv + 1, ntiles - 1), step = to - lv;
+    const int to = min(lv + 1, last), step = to - lv;
     lv = to;
     lvp += step << 13;
   };
   static_assert(IMG_ELEMS == 1 << 13, "the step of next_v");
 
+  // K tiles t_first .. + 3 and V^T images .. + 2, of the last ones a quarter (the loop brings the rest), and the queries behind the first of them: one
+  // wait for memory in front of the first products, not one for the queries and another for the tiles, and no branches, with which the compiler
+  // loses count of the loads in flight.
+#pragma unroll
+  for (int j = 0; j < 4; j++) load_k(j);
+  FENCE();
   bf16x8 qf[FW_QT][KS];
 #pragma unroll
   for (int qt = 0; qt < FW_QT; qt++)
 #pragma unroll
-    for (int ks = 0; ks < KS; ks++) {
-      const int qi = wq0 + 32 * qt + i;
-      if (qi < p.Lq) qf[qt][ks] = *reinterpret_cast<const bf16x8*>(qp + (int64_t)qi * p.sq.l + 16 * ks + 8 * g);
-      else qf[qt][ks] = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
+    for (int ks = 0; ks < KS; ks++)
+      qf[qt][ks] = *reinterpret_cast<const bf16x8*>(qp + (int64_t)min(wq0 + 32 * qt + i, p.Lq - 1) * p.sq.l + 16 * ks + 8 * g);
+  FENCE();
+#pragma unroll
+  for (int a = 0; a < 3; a++) {
+    next_k();
+    if (a > 0) next_v();
+#pragma unroll
+    for (int j = 0; j < (a < 2 ? 4 : 1); j++) {
+      load_k(j);
+      load_v(j);
     }
+  }
+  FENCE();
 #pragma unroll
   for (int qt = 0; qt < FW_QT; qt++)
 #pragma unroll
     for (int ks = 0; ks < KS; ks++) asm volatile("" : "+v"(qf[qt][ks]));
+  if (wq0 + 32 * FW_QT > p.Lq) {   // rows past the end are zeros
+#pragma unroll
+    for (int qt = 0; qt < FW_QT; qt++)
+#pragma unroll
+      for (int ks = 0; ks < KS; ks++)
+        if (wq0 + 32 * qt + i >= p.Lq) qf[qt][ks] = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
+  }
   int lim[FW_QT];   // last key this lane's queries see
 #pragma unroll
   for (int qt = 0; qt < FW_QT; qt++) lim[qt] = p.causal ? min(p.Lk - 1, wq0 + 32 * qt + i + p.off) : p.Lk - 1;
@@ -238,19 +261,6 @@ __global__ __launch_bounds__(FW_THREADS, 1) void attn_fwd_pipe_kernel(const Attn
   };
 
   if (t_first < ntiles) {
-    // K tiles t_first .. + 3 and V^T images .. + 2, of the last ones a quarter: the loop brings the rest
-#pragma unroll
-    for (int j = 0; j < 4; j++) load_k(j);
-#pragma unroll
-    for (int a = 0; a < 3; a++) {
-      next_k();
-      if (a > 0) next_v();
-#pragma unroll
-      for (int j = 0; j < (a < 2 ? 4 : 1); j++) {
-        load_k(j);
-        load_v(j);
-      }
-    }
     asm volatile("s_waitcnt vmcnt(10)" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
@@ -319,8 +329,8 @@ __global__ __launch_bounds__(FW_THREADS, 1) void attn_fwd_pipe_kernel(const Attn
       load_k(0);
       load_v(0);
     }
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 
   // ---- epilogue
 #pragma unroll
