@@ -424,15 +424,18 @@ inline int64_t row_blocks(int B, int L, int H) { return (int64_t)B * H * ((L + B
 
 }  // namespace
 
-// The lines are fitted to 563 shapes timed with both, launches and all: 2 to 128 heads, 96 to 8192 rows, a third of them with other key
-// than query counts.  Forward: 1.33 times faster in the geometric mean over all of them, the unchanged ones included (1.35 if the faster
-// one ran everywhere), backward 1.58 (1.61); none behind by more than 3 %.
-//   Beyond the line in blocks every compute unit has a block of 256 rows, whose tiles serve twice the rows: 32 heads, full, L = 1500:
-//   forward 56 us there, 62 here, backward 171 / 192; causal, L = 3001: 98 / 107, 338 / 365.
-//   Beyond the line in tiles the other kernels cut the range of the long side into parts: 4 heads, causal, L = 3001: forward 43 / 51;
-//   8 heads, full, L = 3001: backward 181 / 230.  Forwards of 64 blocks and less stay there wherever it has parts: some are faster here
-//   (4 heads, L = 1000: 29 / 22), some are not (32 heads, 109 queries on 2042 keys: 1.13 times slower).
-// One head, too, below the line: backward of 512 rows, causal, 65 us there, 29 here, of 1024 rows 101 / 45; two heads of 512 rows 66 / 29.
+// The lines were fitted against kernels that the present ones for long rows replaced, and timed again with these on shapes around them, launches and
+// all (596 forward, 556 backward: 1 to 128 heads, 64 to 8192 rows, a third with other key than query counts): 1.22 and 1.30 times as fast in the
+// geometric mean as without these kernels, 2 % behind the faster one everywhere.  Here / there, us:
+//   Beyond the line in blocks every compute unit has a block of 256 rows, whose tiles serve twice the rows: 32 heads, full, L = 1500: forward
+//   65 / 55, backward 189 / 156; causal, L = 3001: 101 / 87, 340 / 287.  Short causal rows leave those blocks a few tiles each, most of them under the
+//   mask, so that for them the line of the backward is further out: 4 x 24 heads, L = 820, 131 / 147, 4 x 32 heads, L = 683, 139.6 / 142.9, and
+//   beyond, 4 x 32 heads, L = 820, 175 / 177; L = 936 211 / 200; with longer rows 2 x 32 heads, L = 1200, 150 / 144, L = 1536 207 / 191.
+//   Beyond the line in tiles the other kernels cut the range of the long side into parts: 4 heads, causal, L = 3001: forward 48 / 40; 8 heads,
+//   full, L = 3001: backward 218 / 163.  The line in blocks is too far out for some of these (6 heads, causal, L = 3500: forward 57 / 53), too
+//   near for backwards of the fewest blocks (2 heads, L = 2500: 95 / 120).  Forwards of 64 blocks and less stay there wherever it has parts: some
+//   are faster here (4 heads, L = 1000: 21 / 28), some are not (32 heads, 109 queries on 2042 keys: 36 / 32).
+// One head, too, below the line: backward of 512 rows, causal, 28 / 67, of 1024 rows 44 / 96; two heads of 512 rows 28 / 68.
 bool ody_attn_fwd_short_ok(int B, int Lq, int Lk, int Hq, int causal) {
   const int64_t blocks = row_blocks(B, Lq, Hq);
   if (blocks <= 64 && ody_attn_fwd_pipe_parts(B, Lq, Lk, Hq, causal) > 1) return false;
@@ -440,7 +443,8 @@ bool ody_attn_fwd_short_ok(int B, int Lq, int Lk, int Hq, int causal) {
 }
 bool ody_attn_bwd_short_ok(int B, int Lq, int Lk, int Hq, int causal) {
   const int64_t blocks = row_blocks(B, Lq, Hq) + row_blocks(B, Lk, Hq);
-  return blocks <= (causal ? 1024 : 512) && std::max(Lq, Lk) <= ROWS * (causal && blocks > 128 ? 56 : 32);
+  const int rows = std::max(Lq, Lk);
+  return blocks <= (causal ? (rows <= 16 * ROWS ? 1536 : 1024) : 512) && rows <= ROWS * (causal && blocks > 128 ? 56 : 32);
 }
 
 int ody_launch_attn_fwd_short(const AttnParams& p, hipStream_t st) {

@@ -107,3 +107,20 @@ def test_backward_of_one_or_two_heads(case):
     o_ref, lse_ref = oracle.attention_fwd(*(t.cpu().float() for t in (q, k, v)), causal=causal)
     for a, b, n in zip(got, oracle.attention_bwd(*(t.cpu().float() for t in (q, k, v)), o_ref, lse_ref, do.cpu().float(), causal=causal), ("dq", "dk", "dv")):
         assert_parity(a, b, TOL_BF16, n, 1e-3)
+
+
+@pytest.mark.parametrize("L,H,short", [(1024, 96, True), (1000, 96, True), (1024, 97, False), (1025, 86, False), (1536, 42, True)])
+def test_causal_backward_of_many_blocks(L, H, short):
+    """At the line in blocks, which goes by the rows: on either side of it dK and dV are the bits of a call that keeps dS."""
+    from odysseus_transformer_amd import ops
+    print(f"L={L} H={H}", flush=True)
+    q, k, v, do = (t.cuda() for t in _inputs(1, L, L, H, H, 27))
+    o, lse = ops.attn_fwd(q, k, v, causal=True)
+    got, ran = _run(lambda: ops.attn_bwd(q, k, v, o, lse, do, causal=True))
+    assert ("attn_bwd_short" in ran) == short and ("attn_bwd_dq_pipe" in ran) != short, ran
+    if L % 256 == 0:
+        kept = ops.attn_bwd(q, k, v, o, lse, do, causal=True, keep_ds=True)
+        assert torch.equal(got[1], kept[1]) and torch.equal(got[2], kept[2])
+    q, k, v, do = (t[:, :, :2].cpu().float() for t in (q, k, v, do))
+    for a, b, n in zip(got, oracle.attention_bwd(q, k, v, *oracle.attention_fwd(q, k, v, causal=True), do, causal=True), ("dq", "dk", "dv")):
+        assert_parity(a[:, :, :2], b, TOL_BF16, n, 1e-3)
