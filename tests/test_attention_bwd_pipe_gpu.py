@@ -70,3 +70,24 @@ def test_keys_far_apart(stride, dev):
     assert ("attn_bwd_short" if stride >= 1 << 24 else "attn_bwd_dq_pipe") in ran, ran
     for a, r, n in zip(got, ops.attn_bwd(q, k, v, o, lse, do, causal=False), ("dq", "dk", "dv")):
         assert_parity(a, r.float().cpu(), TOL_BF16, n)
+
+
+@pytest.mark.parametrize("keep", [False, True], ids=["recomputed", "kept"])
+@pytest.mark.parametrize("Hkv", [1, 2])
+@pytest.mark.parametrize("which", ["q", "k", "v", "do"])
+def test_any_operand_far_apart(which, Hkv, keep, dev):
+    """Every operand of these kernels, with grouped heads and where dS would be kept: beyond 32-bit offsets all go to the kernels with 64-bit ones."""
+    from odysseus_transformer_amd import ops
+    L, stride = 256, 1 << 24
+    t = {n: randn((1, L, H, 128), 95 + m, dtype=torch.bfloat16).to(dev) for m, (n, H) in enumerate((("q", 2), ("k", Hkv), ("v", Hkv), ("do", 2)))}
+    o, lse = ops.attn_fwd(t["q"], t["k"], t["v"], causal=True)
+    want = ops.attn_bwd(t["q"], t["k"], t["v"], o, lse, t["do"], causal=True, keep_ds=True)
+    H = t[which].shape[2]
+    far = torch.empty(stride * (L - 1) + 128 * H, dtype=torch.bfloat16, device=dev).as_strided((1, L, H, 128), (0, stride, 128, 1))
+    t[which] = far.copy_(t[which])
+    print(f"{which} far apart, {Hkv} kv heads, keep_ds={keep}", flush=True)
+    new = {n: torch.empty((1, L, h, 128), dtype=torch.bfloat16, device=dev) for n, h in (("dq", 2), ("dk", Hkv), ("dv", Hkv))}
+    got, ran = _ran(lambda: ops.attn_bwd(t["q"], t["k"], t["v"], o, lse, t["do"], causal=True, keep_ds=keep, **new))
+    assert "attn_bwd_short" in ran and "attn_bwd_dq_kept" not in ran, ran
+    for a, r, n in zip(got, want, ("dq", "dk", "dv")):
+        assert_parity(a, r.float().cpu(), TOL_BF16, n)
