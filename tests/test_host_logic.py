@@ -804,3 +804,33 @@ def test_host_module_in_another_place(tmp_path, monkeypatch):
     monkeypatch.setenv("ODYSSEUS_NATIVE_LIB", str(tmp_path / "_odysseus_native.so"))
     native = _native._Native()
     assert native.gemm(0, None, None) is None and native.TORCH_VERSION == str(torch.__version__)
+
+
+def test_partial_results_of_a_ring_hold_a_bounded_number_of_bytes(monkeypatch):
+    """How many parts every merge takes: all at the end, the most that a launch takes at a time, or as many as the bytes allow, one at least."""
+    from odysseus_transformer_amd import ops
+    merges = []
+    monkeypatch.setattr(ops._lib, "call", lambda name, parts, *args: merges.append(parts))
+    monkeypatch.setattr(ops, "_stream", lambda: 0)
+    like = torch.empty((1, 64, 2, 64), dtype=torch.bfloat16)
+    size = like.numel() * 2
+    for held, parts, want in ((None, 8, [8]), (None, 19, [8, 8, 3]), (3 * size, 7, [3, 3, 1]), (3 * size - 1, 4, [2, 2]), (0, 3, [1, 1, 1]), (0, 0, [0])):
+        merges.clear()
+        with monkeypatch.context() as m:
+            if held is not None:
+                m.setattr(ops._PartialResults, "HELD_BYTES", held)
+            merge = ops._PartialResults(like.shape, like)
+            for _ in range(parts):
+                merge.add(like, torch.empty((1, 2, 64)))
+                assert sum(out.numel() * 2 for out, _, _ in merge.parts) <= max(ops._PartialResults.HELD_BYTES, size)
+            out, lse = merge.result()
+        assert merges == want, (held, parts, merges)
+        assert out.shape == like.shape and lse.shape == (1, 2, 64)
+
+
+def test_merge_parts_of_the_header_and_of_the_ring():
+    from pathlib import Path
+    import re
+    from odysseus_transformer_amd import ops
+    header = (Path(__file__).resolve().parents[1] / "include" / "odysseus_hip.h").read_text()
+    assert ops._PartialResults.MOST == int(re.search(r"#define ODY_MERGE_PARTS (\d+)", header).group(1))
