@@ -275,7 +275,7 @@ __global__ __launch_bounds__(DP_THREADS, 1) void attn_bwd_dq_pipe_kernel(const A
       if ((m & 7) == 0) __builtin_amdgcn_s_waitcnt(LGKM_4);
       dq[qt][n & 3] = mfma32(fr[n], dsf[qt][n >> 2], dq[qt][n & 3]);
       FENCE();
-      if (qt == 1) fr[n] = kfrag(KT ? rslot(t + 1) : after, KT, n);
+      if (qt == 1) fr[n] = kfrag(after, KT, n);
       if (m <= 2) weight(2 * m + 26), weight(2 * m + 27);
       if (m <= 1) exponent(2 * m + 28, nt, NKT, masked), exponent(2 * m + 29, nt, NKT, masked);
       if (m >= 2) {   // all of dS and its operands before the next part takes the registers of S

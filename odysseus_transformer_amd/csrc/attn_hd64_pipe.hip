@@ -147,7 +147,7 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_hd64_pipe_kernel(const AttnPa
     else read_tr<32 * KT>(vfr[n], rd.tr[2 * (n & 1)] + at, rd.tr[2 * (n & 1) + 1] + at);
   };
   // S of sub-tile KT of a tile, and reads of V of sub-tile KT of the one before
-  auto s_phase = [&](auto kt, unsigned vslot, int e0, int t, int load, auto masked) INLINE {
+  auto s_phase = [&](auto kt, unsigned vslot, int e0, int t, int half, auto masked) INLINE {
     constexpr int KT = decltype(kt)::value;
 #pragma unroll
     for (int m = 0; m < 8; m++) {
@@ -157,13 +157,13 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_hd64_pipe_kernel(const AttnPa
       s[KT][qt] = mfma32(kfr[n], qf[qt][n], n == 0 ? f32x16{0} : s[KT][qt]);
       FENCE();
       if (qt == 1) read_v(n, vslot, kt);
-      if (m == 2) load ? load_v(load >> 1) : load_k(0);
+      if (m == 2) load_v(half);
       weigh(e0 + m, t, masked);
       FENCE();
     }
   };
   // O += P V of sub-tile KT, and reads of K of the other sub-tile
-  auto pv_phase = [&](auto kt, unsigned kslot, int e0, int t, int load, auto masked) INLINE {
+  auto pv_phase = [&](auto kt, unsigned kslot, int e0, int t, int half, auto masked) INLINE {
     constexpr int KT = decltype(kt)::value;
 #pragma unroll
     for (int m = 0; m < 8; m++) {
@@ -179,7 +179,7 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_hd64_pipe_kernel(const AttnPa
       o[qt][n & 1] = mfma32(value(vfr[n]), pb[KT][qt][n >> 1], o[qt][n & 1]);
       FENCE();
       if (qt == 1) read_k(n, kslot, KT ^ 1);
-      if (m == 2) load_k(load);
+      if (m == 2) load_k(half);
       weigh(e0 + m, t, masked);
       FENCE();
     }
@@ -187,9 +187,9 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_hd64_pipe_kernel(const AttnPa
   std::integral_constant<int, 0> c0;
   std::integral_constant<int, 1> c1;
   auto turn = [&](int t, auto masked) INLINE {
-    s_phase(c0, kslot(t), 0, t, 1, masked);
+    s_phase(c0, kslot(t), 0, t, 0, masked);
     pv_phase(c0, kslot(t + 1), 8, t, 1, masked);
-    s_phase(c1, kslot(t), 16, t, 3, masked);
+    s_phase(c1, kslot(t), 16, t, 1, masked);
     // K tile t + 2 and V tile t + 1 have landed (behind them the 4 loads of the tiles after); everyone is done with K tile t + 1 and V tile t - 1
     asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
     __builtin_amdgcn_s_barrier();

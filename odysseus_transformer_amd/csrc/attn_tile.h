@@ -94,9 +94,6 @@ __device__ __forceinline__ bf16x8 image_frag(const bf16* img, int base, int dt, 
 __device__ __forceinline__ void mfma32_new(f32x16& d, bf16x8 a, bf16x8 b) {
   asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, 0" : "=&v"(d) : "v"(a), "v"(b));
 }
-__device__ __forceinline__ void mfma32_from(f32x16& d, bf16x8 a, bf16x8 b, const f32x16& c) {
-  asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %3" : "=&v"(d) : "v"(a), "v"(b), "v"(c));
-}
 __device__ __forceinline__ void mfma32_onto(f32x16& d, bf16x8 a, bf16x8 b) {
   asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(d) : "v"(a), "v"(b));
 }
