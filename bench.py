@@ -170,9 +170,10 @@ def mfma_sustained(_lib, dev):
 
 
 def tile_cost_ladder(_lib, dev, fwd_ms):
-    """What the ingredients of an attention tile cost on top of its MFMAs, measured with a synthetic kernel that has
-    the forward kernel's shape (8 wavefronts, two per SIMD, one workgroup per CU, a barrier per 64-key turn, 32 MFMAs
-    per wavefront and turn) and adds them one at a time -- and the forward kernel itself in the same unit."""
+    """What the ingredients of an attention tile cost on top of its MFMAs, measured with a synthetic kernel of 8 wavefronts,
+    two per SIMD (one workgroup per CU, a barrier per 64-key turn, 32 MFMAs per wavefront and turn, one part after the
+    other), that adds them one at a time.  The last entry is the forward kernel in the same unit, 64 MFMAs per SIMD: not a rung
+    of that ladder, as it has one wavefront of twice the queries per SIMD and its vector work under the MFMAs."""
     import torch
     blocks, turns = 1024, 2000                   # 4 workgroups per CU in sequence; ~10 ms per rung
     sink = torch.empty(blocks * 512, dtype=torch.float32, device=dev)
@@ -195,12 +196,12 @@ def tile_cost_ladder(_lib, dev, fwd_ms):
                 best = e0.elapsed_time(e1) if best is None else min(best, e0.elapsed_time(e1))
         res[name] = {"ns_per_turn": round(best * 1e6 / (blocks / 256 * turns), 1),
                      "tflops": round(blocks * 8 * turns * 32 * 32768.0 / (best * 1e-3) / 1e12, 1)}
-    # the forward kernel: 64 MFMAs per SIMD and turn as well; turns = executed MFMAs / (1024 SIMDs * 64)
+    # the forward kernel: turns = executed MFMAs / (1024 SIMDs * 64)
     nqb = L // 256
     tiles = sum(min(L // 64, (qb * 256 + 255) // 64 + 1) for qb in range(nqb)) * H     # 64-key tiles x 256-query blocks
     mfmas = (tiles * 8 - nqb * H * 12) * 32        # 12 (wavefront, tile) pairs of a diagonal block lie above the diagonal
     res["attn_fwd_pipe"] = {"ns_per_turn": round(fwd_ms * 1e6 / (mfmas / (1024 * 64)), 1),
-                          "tflops_executed": round(mfmas * 32768.0 / (fwd_ms * 1e-3) / 1e12, 1)}
+                            "tflops_executed": round(mfmas * 32768.0 / (fwd_ms * 1e-3) / 1e12, 1)}
     return res
 
 

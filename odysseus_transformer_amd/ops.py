@@ -177,8 +177,8 @@ def attn_bwd(q, k, v, out, lse, dout, causal: bool = True, scale: Optional[float
 
     dq may be a float32 tensor although q is bfloat16: with accumulate_dq that is the running dq of a
     ring step, summed exactly over the key blocks.  reuse_query_side=True (needs the `workspace` of
-    the previous call, with the same q / out / lse / dout) skips the scratch that depends on the
-    queries only.  rope_tables=(table_q, table_k) (rope_table() of the query / key positions; bf16,
+    the previous call, with the same q / out / lse / dout and, for bfloat16 and head_dim 128, as many keys and
+    the same scale) skips the scratch that depends on the queries only.  rope_tables=(table_q, table_k) (rope_table() of the query / key positions; bf16,
     head_dim 128) makes dq and dk the gradients of the projection BEFORE its rotary embedding.
 
     keep_ds spends scratch memory to save arithmetic: the dK/dV kernel keeps dS (2 bytes per visible
