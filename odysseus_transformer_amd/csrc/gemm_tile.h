@@ -22,14 +22,23 @@
 // Rows and columns past the edge re-read the last valid ones and are not stored.  A last slab that K does not fill reads zeros:
 // those lanes get an offset beyond the buffer descriptor's range.
 //
+// A phase is 64 MFMAs, 1024 cycles, and a wavefront issues a transposing read every 17 cycles at best (a 16-byte read of twice the bytes every 20).  The 48 of a
+// slab of the TN product, with their addresses and eight loads, made its memory phase the longer one: 1300 to 1500 cycles.  So its group reads the
+// fragments of A for the second k-step under the products of the first (each an eighth of the phase ahead of its use; A's stage belongs to the
+// group, whereas a stage of B may be refilled by the other group meanwhile), and addresses move by scalars.  TN, TFLOP/s before / here in loops, random
+// operands: 22016 x 4096 x 4096 1270 / 1500, 4096 x 11008 x 4096 1270 / 1460, 32000 x 4096 x 4096 1295 / 1500, 4096 x 4096 x 16384 1415 / 1545, 8192^3 1365 /
+// 1565, 22016 x 4096 x 1000 1110 / 1250; 1024 x 2816 x 776 11.8 / 9.1 us.  Other numbers of fragments ahead (2, 4, 6, 7 for 8) are 1 to 4 % slower, 1 is 10
+// to 20 %.  NN, whose B is read alike, 1.02 to 1.06 of the speed before (to 1.10 where K is short) by the addresses alone.
+//
 // Bound: the package power limit.  With constant operands the NT instance sustains 2170 TFLOP/s (4096 x 4096 x 11008, 87 % of
-// the matrix peak), with random ones 1500.  Measured against the kernel it replaced (4 wavefronts, operands staged through
+// the matrix peak), with random ones 1500; TN 1880 (4096 x 11008 x 4096).  Measured against the kernel it replaced (4 wavefronts, operands staged through
 // registers), TFLOP/s in loops of 30 calls and more, 8192^3 / 4096 x 4096 x 11008: NT 1305 -> 1450 / 1347 -> 1520, NN 1283 ->
-// 1443 / 1343 -> 1500, TN 1266 -> 1376 / 1265 -> 1398 (another box: 1565 / 1545, 1506 / 1500, 1402 / 1400; torch.matmul there, NT,
+// 1443 / 1343 -> 1500 (another box: 1565 / 1545, 1506 / 1500; torch.matmul there, NT,
 // 1614 / 1600).  A call between two events of its own shows the launch and the clock's way up as well: the second NT product
 // 1320 right after idling (torch.matmul 1300 to 1550), 1480 once the card has worked for a second (1470).
 #pragma once
 #include <type_traits>
+#include <utility>
 #include "gemm_epi.h"
 
 namespace gemm_tile {
@@ -64,39 +73,56 @@ template <int W> __device__ __forceinline__ int group_perm(int k) {
   return ((k >> 1) & 1) | (((k >> 3) & 1) << 1);   // W = 64: two k rows per 256 bytes
 }
 
-// One operand's share of the direct loads: W rows (columns) x 64 k per stage, brought by NW wavefronts.
+// The lane, to the compiler a new value each time: what follows from it inside a loop is formed there and takes no registers in between
+__device__ __forceinline__ int lane_anew() {
+  int x;
+  asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(x));
+  return x;
+}
+
+// One operand's share of the direct loads: W rows (columns) x 64 k per stage, brought by NW wavefronts.  `aim` sets it to a tile; `load` brings
+// slab s of K, behind slab s - 1 (KC: any).
+//
+// Not KC: what changes from slab to slab is scalar, the slab's address; chunks that K does not reach are sorted out behind a branch (`cut`, in front of
+// the load), and not in every load, because the transposing reads leave the memory phase no room.
+// KC: slab address and mask anew in every load.  The other form is 1 to 2.5 % slower there (NT, us, this / other: 8192^3 683 / 702, zeros 476 / 487;
+// 4096 x 11008 x 4096, zeros, 184 / 188), although it takes fewer instructions.
 template <bool KC, int W, int NW>
 struct Mover {
   static constexpr int NINS = W / 8 / NW;           // 1 KB instructions per wavefront and stage
   static constexpr int LPR = KC ? 8 : W / 8;        // lanes (16-byte chunks) per tile row
   static constexpr int RPI = 64 / LPR;              // tile rows per instruction
-  // a [64][W] tile's permutation takes two values over a wavefront's instructions, by bit SEL of the instruction
-  static constexpr int SEL = W == 128 && NW == 4 ? 1 : 0;
-  static constexpr int NV = KC ? NINS : (W == 128 && NW == 8 ? 1 : 2);
-  unsigned v[NV];                                    // byte offset of this lane's chunk from the slab's base
-  unsigned step;                                     // bytes between the tile rows of consecutive instructions (k rows, if not KC)
+  unsigned v[NINS];                                  // byte offsets of this lane's chunks from the slab's base
+  const bf16* base;                                  // first element of the tile's slab 0, or, not KC, of the slab to be loaded next
+  int left;                                          // k values from there on
 
   // row_of(r): operand row of tile row r (KC), or first column of the tile's columns r .. r + 7 (else), clamped to the matrix
   template <typename F>
-  __device__ __forceinline__ void init(int wv, int lane, int64_t ld, F row_of) {
-    step = (unsigned)(2 * RPI * ld);
+  __device__ __forceinline__ void aim(int wv, int lane, int64_t ld, const bf16* first, int s, int K, F row_of) {
+    base = KC ? first : first + s * (BK * ld), left = KC ? K : K - s * BK;
 #pragma unroll
-    for (int i = 0; i < NV; i++) {
-      const int j = KC ? i : (SEL ? 2 * i : i), r = (wv * NINS + j) * RPI + lane / LPR, p = lane % LPR;
-      if (KC) v[i] = (unsigned)(2 * ((int64_t)row_of(r) * ld + 8 * (p ^ (r & 7))));
-      else v[i] = (unsigned)(2 * ((int64_t)r * ld + row_of(8 * (p ^ (2 * group_perm<W>(r))))));
+    for (int j = 0; j < NINS; j++) {
+      const int r = (wv * NINS + j) * RPI + lane / LPR, p = lane % LPR;
+      if (KC) v[j] = (unsigned)(2 * ((int64_t)row_of(r) * ld + 8 * (p ^ (r & 7))));
+      else v[j] = (unsigned)(2 * ((int64_t)r * ld + row_of(8 * (p ^ (2 * group_perm<W>(r))))));
     }
   }
-  // slab: first element of the operand's slab; krem: k values left from there (>= 64 except in a last, partial slab)
-  __device__ __forceinline__ void load(const bf16* slab, bf16* stage, int wv, int lane, int krem) const {
+  __device__ __forceinline__ void cut(int wv) {
+    if (KC || left >= BK) return;
+    const int k = wv * NINS * RPI + lane_anew() / LPR;
+#pragma unroll
+    for (int j = 0; j < NINS; j++)
+      if (k + j * RPI >= left) v[j] = PAST_END;
+  }
+  __device__ __forceinline__ void load(int s, bf16* stage, int wv, int lane, int64_t ld) {
+    const bf16* slab = KC ? base + (int64_t)s * BK : base;
     auto rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16*>(slab), (short)0, 0x7fffffff, 0x00020000);
 #pragma unroll
     for (int j = 0; j < NINS; j++) {
-      const int i = KC ? j : (NV == 1 ? 0 : (j >> SEL) & 1), from = KC ? j : (NV == 1 ? 0 : (SEL ? 2 * i : i));
-      const int k = KC ? 8 * ((lane & 7) ^ (lane >> 3)) : (wv * NINS + j) * RPI + lane / LPR;   // k of the chunk inside the slab
-      const unsigned off = k < krem ? v[i] : PAST_END;
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_ptr)(stage + (wv * NINS + j) * 512), 16, (int)off, (int)((j - from) * step), 0, 0);
+      const unsigned off = !KC || 8 * ((lane & 7) ^ (lane >> 3)) < left - s * BK ? v[j] : PAST_END;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_ptr)(stage + (wv * NINS + j) * 512), 16, (int)off, 0, 0, 0);
     }
+    if (!KC) base += BK * ld, left -= BK;
   }
 };
 
@@ -118,15 +144,17 @@ template <int NB>
 __device__ __forceinline__ bf16x8 frag(const Frags<false, NB>& f, int ks, int b) {
   return concat4(__builtin_bit_cast(bf16x4, f.lo[ks][b]), __builtin_bit_cast(bf16x4, f.hi[ks][b]));
 }
-// ties the fragments to a point behind the wait for them
+// ties a fragment to a point behind the wait for it
 template <int NB>
-__device__ __forceinline__ void tie(Frags<true, NB>&) {}
+__device__ __forceinline__ void tie(Frags<true, NB>&, int, int) {}
 template <int NB>
-__device__ __forceinline__ void tie(Frags<false, NB>& f) {
-#pragma unroll
-  for (int ks = 0; ks < 2; ks++)
-#pragma unroll
-    for (int b = 0; b < NB; b++) asm volatile("" : "+v"(f.lo[ks][b]), "+v"(f.hi[ks][b]));
+__device__ __forceinline__ void tie(Frags<false, NB>& f, int ks, int b) {
+  asm volatile("" : "+v"(f.lo[ks][b]), "+v"(f.hi[ks][b]));
+}
+
+template <int... N, typename F>
+__device__ __forceinline__ void each(std::integer_sequence<int, N...>, F f) {
+  (f(std::integral_constant<int, N>{}), ...);
 }
 
 template <int OFF0, int OFF1>
@@ -151,13 +179,6 @@ __device__ __forceinline__ TileAt tile_at(const Args& p, int pos) {
   return TileAt{first_m + (pos % per_group) % gsz, (pos % per_group) / gsz};
 }
 
-// The lane, to the compiler a new value each time: what follows from it inside a loop is formed there and takes no registers in between
-__device__ __forceinline__ int lane_anew() {
-  int x;
-  asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(x));
-  return x;
-}
-
 constexpr int ROUND = 256;   // blocks of a launch whose blocks take several tiles: one per compute unit
 
 // The BM x BN results from row m0 and column n0 on (n0 / BN = tn), this wavefront's share.
@@ -169,6 +190,7 @@ template <bool A_KC, bool B_KC, int BM, int BN, bool SPLITK, int EPI, bool ROUND
 __device__ __forceinline__ void gemm_tile_block(const Args& p, int m0, int tn, int tiles = 0) {
   constexpr int WM = BM / 32, WN = BN / 64;      // 16-row blocks per wavefront: rows BM / 2, columns BN / 4
   constexpr int HALF = BM / 2, NH = WN / 2;
+  constexpr int AHEAD = A_KC ? 2 * WM : WM;       // fragments of A that the memory phase reads, of two k-steps
   static_assert(EPI == EPI_NONE || !SPLITK, "fused epilogues: one pass over K");
   static_assert(!ROUNDS || ((EPI == EPI_NONE || EPI == EPI_SWIGLU_FWD) && !SPLITK && BM == 256 && BN == 256), "several tiles a block: bf16 bands");
   static_assert((EPI != EPI_SWIGLU_FWD && EPI != EPI_ROPE) || (A_KC && B_KC), "these epilogues belong to the NT product");
@@ -192,30 +214,24 @@ __device__ __forceinline__ void gemm_tile_block(const Args& p, int m0, int tn, i
   Mover<A_KC, HALF, 4> ma;
   Mover<B_KC, BN, 8> mb;
   int j0 = EPI == EPI_SWIGLU_FWD ? tn * (BN / 2) : 0;   // first column of h
-  const bf16 *a_base, *b_base;
   auto aim_a = [&](int lane) {
-    if (A_KC) ma.init(wn, lane, p.lda, [&](int r) { return min(m0 + wm * HALF + r, p.M - 1) - m0; });
-    else ma.init(wn, lane, p.lda, [&](int col) { return min(m0 + wm * HALF + col, p.M - 8) - m0; });
-    a_base = A_KC ? p.A + (int64_t)m0 * p.lda : p.A + m0;
+    if (A_KC) ma.aim(wn, lane, p.lda, p.A + (int64_t)m0 * p.lda, s0, p.K, [&](int r) { return min(m0 + wm * HALF + r, p.M - 1) - m0; });
+    else ma.aim(wn, lane, p.lda, p.A + m0, s0, p.K, [&](int col) { return min(m0 + wm * HALF + col, p.M - 8) - m0; });
   };
   auto aim_b = [&](int lane) {
     if (EPI == EPI_SWIGLU_FWD)
-      mb.init(wave, lane, p.ldb, [&](int r) { return min(j0 + (r & (BN / 2 - 1)), p.ep.I - 1) + (r < BN / 2 ? 0 : p.ep.I); });
-    else if (B_KC) mb.init(wave, lane, p.ldb, [&](int r) { return min(n0 + r, p.N - 1) - n0; });
-    else mb.init(wave, lane, p.ldb, [&](int col) { return min(n0 + col, p.N - 8) - n0; });
-    b_base = EPI == EPI_SWIGLU_FWD ? p.B : (B_KC ? p.B + (int64_t)n0 * p.ldb : p.B + n0);
+      mb.aim(wave, lane, p.ldb, p.B, s0, p.K, [&](int r) { return min(j0 + (r & (BN / 2 - 1)), p.ep.I - 1) + (r < BN / 2 ? 0 : p.ep.I); });
+    else if (B_KC) mb.aim(wave, lane, p.ldb, p.B + (int64_t)n0 * p.ldb, s0, p.K, [&](int r) { return min(n0 + r, p.N - 1) - n0; });
+    else mb.aim(wave, lane, p.ldb, p.B + n0, s0, p.K, [&](int col) { return min(n0 + col, p.N - 8) - n0; });
   };
   aim_a(lane);
   aim_b(lane);
-  const int64_t a_slab = A_KC ? BK : BK * p.lda, b_slab = B_KC ? BK : BK * p.ldb;
-  auto load_a = [&](int kt, int stage) {
-    const int s = s0 + kt;
-    ma.load(a_base + s * a_slab, As + stage * BM * BK + wm * HALF * BK, wn, lane, p.K - s * BK);
+  auto cut = [&] {
+    ma.cut(wn);
+    mb.cut(wave);
   };
-  auto load_b = [&](int kt, int slot) {
-    const int s = s0 + kt;
-    mb.load(b_base + s * b_slab, Bs + slot * BN * BK, wave, lane, p.K - s * BK);
-  };
+  auto load_a = [&](int kt, int stage) { ma.load(s0 + kt, As + stage * BM * BK + wm * HALF * BK, wn, lane, p.lda); };
+  auto load_b = [&](int kt, int slot) { mb.load(s0 + kt, Bs + slot * BN * BK, wave, lane, p.ldb); };
 
   // tile row (column) of this wavefront's n block b
   auto nblock = [&](int b) {
@@ -228,8 +244,18 @@ __device__ __forceinline__ void gemm_tile_block(const Args& p, int m0, int tn, i
   };
   const unsigned lds0 = (unsigned)(uintptr_t)(lds_ptr)smem;
   const int kc_off = c * BK + 8 * (q ^ (c & 7));                                               // + 64 * row block, ^ 32 for ks = 1
-  const int a_tr = A_KC ? 0 : (8 * q + (c >> 2)) * HALF + 16 * group_perm<HALF>(8 * q + (c >> 2)) + 4 * (c & 3);
-  const int b_tr = B_KC ? 0 : (8 * q + (c >> 2)) * BN + 16 * ((wn * WN) ^ group_perm<BN>(8 * q + (c >> 2))) + 4 * (c & 3);
+  // byte addresses of the transposing reads, without the stage
+  unsigned a_tr[A_KC ? 1 : WM], b_tr[B_KC ? 1 : WN];
+  if constexpr (!A_KC) {
+    const int at = wm * HALF * BK + (8 * q + (c >> 2)) * HALF + 16 * group_perm<HALF>(8 * q + (c >> 2)) + 4 * (c & 3);
+#pragma unroll
+    for (int a = 0; a < WM; a++) a_tr[a] = lds0 + 2 * (at ^ (16 * a));
+  }
+  if constexpr (!B_KC) {
+    const int at = A_STAGES * BM * BK + (8 * q + (c >> 2)) * BN + 16 * ((wn * WN) ^ group_perm<BN>(8 * q + (c >> 2))) + 4 * (c & 3);
+#pragma unroll
+    for (int b = 0; b < WN; b++) b_tr[b] = lds0 + 2 * (at ^ (16 * b));
+  }
 
   f32x4 acc[WM][WN];
   auto clear_acc = [&] {
@@ -355,8 +381,10 @@ __device__ __forceinline__ void gemm_tile_block(const Args& p, int m0, int tn, i
 
   if (nk > 0) {
     constexpr int NA = Mover<A_KC, HALF, 4>::NINS, NB = Mover<B_KC, BN, 8>::NINS;
+    cut();
     load_b(0, 0);
     load_a(0, 0);
+    mb.cut(wave);
     load_b(min(1, nk - 1), 1);
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(ROUNDS ? 0 : NB) : "memory");
     __builtin_amdgcn_s_barrier();
@@ -369,6 +397,14 @@ __device__ __forceinline__ void gemm_tile_block(const Args& p, int m0, int tn, i
       const bf16* Bt = Bs + slot * BN * BK;
       Frags<A_KC, WM> fa;
       Frags<B_KC, WN> fb;
+      [[maybe_unused]] auto read_a = [&](int ks, int a) __attribute__((always_inline)) {
+        if constexpr (!A_KC) {
+          const unsigned at = a_tr[a] + 2 * stage * BM * BK;
+          if (ks == 0) read_tr<0, 8 * HALF>(at, fa.lo[0][a], fa.hi[0][a]);
+          else read_tr<64 * HALF, 72 * HALF>(at, fa.lo[1][a], fa.hi[1][a]);
+        }
+      };
+      if (!(A_KC && B_KC) && min(A_KC ? BK : ma.left, B_KC ? BK : mb.left) < BK) cut();
       // ---- memory phase: this slab's fragments; A of the next slab, B of the one after (its stage was read last two phases ago)
       ODY_FENCE();
 #pragma unroll
@@ -379,7 +415,7 @@ __device__ __forceinline__ void gemm_tile_block(const Args& p, int m0, int tn, i
         } else {
 #pragma unroll
           for (int b = 0; b < WN; b++) {
-            const unsigned at = lds0 + 2 * ((int)(Bt - As) + (b_tr ^ (16 * b)));
+            const unsigned at = b_tr[b] + 2 * slot * BN * BK;
             if (ks == 0) read_tr<0, 8 * BN>(at, fb.lo[0][b], fb.hi[0][b]);
             else read_tr<64 * BN, 72 * BN>(at, fb.lo[1][b], fb.hi[1][b]);
           }
@@ -389,11 +425,8 @@ __device__ __forceinline__ void gemm_tile_block(const Args& p, int m0, int tn, i
           for (int a = 0; a < WM; a++) fa.f[ks][a] = *reinterpret_cast<const bf16x8*>(At + (kc_off ^ (32 * ks)) + 16 * a * BK);
         } else {
 #pragma unroll
-          for (int a = 0; a < WM; a++) {
-            const unsigned at = lds0 + 2 * ((int)(At - As) + (a_tr ^ (16 * a)));
-            if (ks == 0) read_tr<0, 8 * HALF>(at, fa.lo[0][a], fa.hi[0][a]);
-            else read_tr<64 * HALF, 72 * HALF>(at, fa.lo[1][a], fa.hi[1][a]);
-          }
+          for (int a = 0; a < WM; a++)
+            if (ks * WM + a < AHEAD) read_a(ks, a);
         }
         ODY_FENCE();
         if (ks == 0) load_a(na, stage ^ 1);
@@ -403,18 +436,31 @@ __device__ __forceinline__ void gemm_tile_block(const Args& p, int m0, int tn, i
       // this wavefront's part of B's next slab has landed (the other group may read it two barriers from here)
       if (STORED) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       else asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(NA + NB) : "memory");
-      tie(fa);
-      tie(fb);
+#pragma unroll
+      for (int n = 0; n < AHEAD; n++) tie(fa, n / WM, n % WM);
+#pragma unroll
+      for (int n = 0; n < 2 * WN; n++) tie(fb, n / WN, n % WN);
       __builtin_amdgcn_s_barrier();
       ODY_FENCE();
       // ---- compute phase
+      each(std::make_integer_sequence<int, 2 * WM>{}, [&](auto which) __attribute__((always_inline)) {
+        constexpr int n = decltype(which)::value, ks = n / WM, a = n % WM, BEHIND = n + AHEAD < 2 * WM ? AHEAD - 1 : 2 * WM - 1 - n;
+        if constexpr (n >= AHEAD) {
+          asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(2 * BEHIND) : "memory");   // its two reads are back; those of BEHIND fragments may not be
+          tie(fa, ks, a);
+          ODY_FENCE();
+        }
 #pragma unroll
-      for (int ks = 0; ks < 2; ks++)
-#pragma unroll
-        for (int a = 0; a < WM; a++)
-#pragma unroll
-          for (int b = 0; b < WN; b++)
-            acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(frag(fb, ks, b), frag(fa, ks, a), acc[a][b], 0, 0, 0);   // rows = n, columns = m
+        for (int b = 0; b < WN; b++) {
+          acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(frag(fb, ks, b), frag(fa, ks, a), acc[a][b], 0, 0, 0);   // rows = n, columns = m
+          if constexpr (n + AHEAD < 2 * WM)
+            if (b == 0) {
+              ODY_FENCE();
+              read_a((n + AHEAD) / WM, (n + AHEAD) % WM);
+              ODY_FENCE();
+            }
+        }
+      });
       ODY_FENCE();
       asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NB) : "memory");   // A of the next slab has landed
       __builtin_amdgcn_s_barrier();
@@ -422,7 +468,7 @@ __device__ __forceinline__ void gemm_tile_block(const Args& p, int m0, int tn, i
       slot = slot == 2 ? 0 : slot + 1;
       stage ^= 1;
     };
-    // loads past the range repeat its last slab: in bounds, and nobody reads them
+    // loads past the range repeat its last slab, or go on behind it (not KC; beyond K they fetch nothing): in bounds, and nobody reads them
     if constexpr (!ROUNDS) {
       for (int kt = 0; kt < nk; kt++) slab(min(kt + 1, nk - 1), min(kt + 2, nk - 1), std::false_type{});
     } else {
@@ -581,16 +627,11 @@ __global__ __launch_bounds__(THREADS, BM * BN <= 128 * 128 ? 4 : 2) void gemm_ti
 // Whether the blocks take several tiles each (a grid of ROUND blocks): where there are two rounds and more.  A block of one tile waits about
 // 4 us for its first slabs and its stores, which nothing hides with one block on a unit; here the matrix cores go on meanwhile.  The same
 // sums in the same order.  us before / here: 32768 x 4096 x 512 NT 139 / 118, NN 141 / 121, TN 155 / 136; 4096 x 11008 x 1000 82 / 77, 81 / 76,
-// 87 / 82; 22016 x 4096 x 4096 NT 483 / 476, NN 506 / 494; 8192^3 679 / 673, 705 / 692.  TN's memory phase is the longest of the three (all of its
-// fragments are transposing reads) and has no room for the choice of the next slab: 11008 x 4096 x 2048 151 / 148, but K = 4096 between 0.99
-// and 1.01 of the speed before and 8192^3 767 / 772, so it is left at the former form from there on.
+// 87 / 82; 22016 x 4096 x 4096 NT 483 / 476, NN 506 / 494, TN 514 / 490; 8192^3 679 / 673, 705 / 692, 714 / 696; 32000 x 4096 x 4096 TN 739 / 716.
 // Of the epilogues, SwiGLU's forward gains: gate_up of 16384 tokens (d 4096, I 11008) 2137 / 2086, of 8192 (1024, 5504) 187 / 178.  Those that
 // read memory wait in it for the stores before (loads and stores come back in order): the rotation 0.96 to 1.00 of the speed before,
 // SwiGLU's backward 0.82 to 0.97, so they keep one tile a block; an addend's fp32 patch is larger than the room there is.
-template <bool A_KC>
-bool takes_rounds(const Args& a) {
-  return a.tiles_m * a.tiles_n - a.cut >= 2 * ROUND && a.K > 2 * BK && (A_KC || a.K < 4096) && a.vec16 && !a.bias && !a.add;
-}
+inline bool takes_rounds(const Args& a) { return a.tiles_m * a.tiles_n - a.cut >= 2 * ROUND && a.K > 2 * BK && a.vec16 && !a.bias && !a.add; }
 
 template <bool A_KC, bool B_KC, int BM, int BN, bool SPLITK, int EPI, int PARTS, bool ROUNDS>
 int launch_parts(const char* name, const Args& a, int splits, hipStream_t st) {
@@ -608,7 +649,7 @@ int launch(const char* name, Args a, int splits, hipStream_t st) {
   if (EPI == EPI_SWIGLU_FWD) a.tiles_n = (a.ep.I + BN / 2 - 1) / (BN / 2);
   if constexpr (BM == 256 && !SPLITK) {
     if constexpr ((EPI == EPI_NONE || EPI == EPI_SWIGLU_FWD) && BN == 256)
-      if (takes_rounds<A_KC>(a)) {
+      if (takes_rounds(a)) {
         if (a.cut_parts == 4) return launch_parts<A_KC, B_KC, BM, BN, SPLITK, EPI, 4, true>(name, a, splits, st);
         return launch_parts<A_KC, B_KC, BM, BN, SPLITK, EPI, 2, true>(name, a, splits, st);
       }

@@ -318,3 +318,23 @@ def test_several_tiles_a_block_with_an_epilogue(what, M, K, dev):
             assert torch.equal(got[m:m + 4096], want)
     for got, want in zip(whole, run(slice(M - 264, M))):   # K in ranges there, perhaps
         assert rel_err(got[M - 264:], want.float()) <= TOL_BF16
+
+
+@pytest.mark.parametrize("op", ["nn", "tn"])
+@pytest.mark.parametrize("M,N,K", [(72, 136, 8), (256, 256, 56), (264, 512, 72), (136, 128, 120), (1000, 264, 1544), (264, 1032, 4104), (8200, 4616, 136),
+                                   (5640, 6152, 4168)], ids=lambda v: str(v))
+def test_slabs_that_k_does_not_fill(op, M, N, K, dev):
+    """Operands with rows of K inside buffers whose other rows and columns are not numbers: one slab, a whole number of them and a part, K in ranges, one tile and
+    several a block (short K and long).  What lies behind K is read as zeros and by nobody."""
+    from odysseus_transformer_amd import ops
+    print(f"op={op} M={M} N={N} K={K}", flush=True)
+
+    def inside(t):
+        big = torch.full((t.shape[0] + 136, t.shape[1] + 16), float("nan"), dtype=t.dtype, device=dev)
+        big[8:8 + t.shape[0], 8:8 + t.shape[1]] = t.to(dev)
+        return big[8:8 + t.shape[0], 8:8 + t.shape[1]]
+
+    a = inside(randn((K, M) if op == "tn" else (M, K), 51, dtype=torch.bfloat16))
+    b = inside(randn((K, N), 52, std=0.05, dtype=torch.bfloat16))
+    y = ops.gemm({"nn": ops.GEMM_NN, "tn": ops.GEMM_TN}[op], a, b)
+    assert rel_err(y, (a.float().t() if op == "tn" else a.float()) @ b.float()) <= TOL_BF16
