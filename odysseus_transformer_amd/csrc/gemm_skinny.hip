@@ -6,22 +6,38 @@
 // until the wavefronts' partial results are summed through LDS at the end.  The rows of A (all blocks read the same ones)
 // come from cache; rows beyond M repeat row M - 1 and fall away with their unused result columns.
 //
-// Measured, weights cold, M = 1 (before: 128 x 128 tiles, one block per 128 columns): 4096 x 4096 68 -> 9.4 us (3.6 TB/s),
-// 4096 x 11008 176 -> 22 us (4.1 TB/s), 22016 x 4096 76 -> 40 us (4.5 TB/s), 32000 x 4096 82 -> 54 us (4.9 TB/s; a copy of
-// 1 GiB reaches 5.2).
+// Measured, weights cold, M = 1, us (TB/s): 4096 x 4096 8.0 (4.2), 4096 x 11008 19.3 (4.7), 32000 x 4096 45.3 (5.8), with the norm in front 22016 x 4096 33.0 (5.5),
+// 6144 x 4096 13.0 (3.9), 5632 x 1024 5.2; of each about 1.7 between two launches and 1.2 until the first bytes arrive.  A unit takes some 64 KB of loads at a
+// time and no more (deeper rings of loads to LDS, 96 KB a unit, changed nothing but the time at which what is behind them is issued), so what counts is
+// that blocks are many and even: with two groups of 16 rows and 8 wavefronts a block everywhere, 22016 x 4096 ran 512 blocks in 20 us and the
+// remaining 176 in 18, together 39.0 with the norm; the others 9.0, 20.5, 50.5, 16.0 and 6.4.
+#include <type_traits>
 #include "gemm_epi.h"
 
 namespace {
 
-constexpr int SK_WAVES = 8;
+#define FENCE() __builtin_amdgcn_sched_barrier(0)
 
+// Sum over the lanes of a wavefront, by the tree of xor 1, 2, 4 .. 32 (within groups of equal values a mirrored lane is as good as an exchanged one)
+__device__ __forceinline__ float wave_sum(float x) {
+  auto dpp = [](float v, auto ctrl) { return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), decltype(ctrl)::value, 0xf, 0xf, true)); };
+  x += dpp(x, std::integral_constant<int, 0xb1>{});    // quad_perm [1, 0, 3, 2]
+  x += dpp(x, std::integral_constant<int, 0x4e>{});    // quad_perm [2, 3, 0, 1]
+  x += dpp(x, std::integral_constant<int, 0x141>{});   // row_half_mirror
+  x += dpp(x, std::integral_constant<int, 0x140>{});   // row_mirror
+  x += __shfl_xor(x, 16, 64);
+  x += __shfl_xor(x, 32, 64);
+  return x;
+}
+
+// NT groups a block, U steps of 32 k in flight per wavefront and group, and SK_WAVES wavefronts (ody_launch_gemm_skinny).
 // NORM: A is x, and the product that of its RMS-normalised rows.  Every block normalises them for itself, into LDS, with the arithmetic of
 // the RMSNorm kernel (another order of the sum), while its first fragments of W are on their way; EPI_ROPE then takes its angles from the positions too.  Weights
-// cold, us without the norm / with it, one row: 6144 x 4096 with rotation 13.3 / 15.9, 22016 x 4096 SwiGLU 41.1 / 43.2, 5632 x 1024
-// 5.9 / 6.8; four rows 13.6 / 18.1, 43.4 / 47.1, 6.1 / 8.6.  The norm's own launch takes 2.6, the table's 2.0, and each its gap and 5 of host
-// work.  (The norm inside the K loop, on every fragment, took 16.2 and 46.6; a ring of fragments refilled one by one instead of a batch
-// at a time, without the norm, 14.9 and 41.6.)
-template <int NT, int U, int EPI, bool NORM>
+// cold, us without the norm / with it, one row: 6144 x 4096 with rotation 13.4 / 13.0, 22016 x 4096 SwiGLU 34.6 / 33.0 (the rows are read from LDS there), 5632 x 1024 5.6 / 5.2.  The norm's own launch takes 2.6, the
+// table's 2.0, and each its gap and 5 of host work.  (The norm inside the K loop, on every fragment, took 0.3 and 3.4 us longer.)
+// BATCH: all loads of a batch in front of its first product.  Left to the compiler, most of a later batch went out one or two loads at a time (NORM: 39 us for 33);
+// where A's rows are many and blocks too, its order is the better one (22016 x 4096, M = 8: 41.4 / 38.4, but 6144 x 4096 13.8 / 17.4).
+template <int NT, int U, int SK_WAVES, int EPI, bool NORM, bool BATCH>
 __global__ __launch_bounds__(64 * SK_WAVES) void gemm_skinny_kernel(const bf16* __restrict__ A, const bf16* __restrict__ W,
                                                                     bf16* __restrict__ C, const bf16* __restrict__ bias, int M,
                                                                     int N, int K, int64_t lda, int64_t ldw, int64_t ldc,
@@ -30,17 +46,20 @@ __global__ __launch_bounds__(64 * SK_WAVES) void gemm_skinny_kernel(const bf16* 
   __shared__ __attribute__((aligned(16))) bf16 angles[NORM && EPI == EPI_ROPE ? ODY_SKINNY_NORM_MAX_M : 1][16][2];
   extern __shared__ __attribute__((aligned(16))) bf16 rows[];   // NORM: [M][K + 8]
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, c = lane & 15, q = lane >> 4;
+  // a group of 16 rows of W: sixteen in a row, or, PAIRED, eight and their eight partners
+  constexpr bool TWO = EPI == EPI_SWIGLU_FWD || EPI == EPI_ROPE, PAIRED = TWO && NT == 1;
   // first W row of group t of this block
   int row0[NT];
 #pragma unroll
   for (int t = 0; t < NT; t++) {
-    if (EPI == EPI_SWIGLU_FWD) row0[t] = 16 * blockIdx.x + t * ep.I;                                   // gate, up
+    if (PAIRED) row0[t] = EPI == EPI_SWIGLU_FWD ? 8 * blockIdx.x : 128 * (blockIdx.x >> 3) + 8 * (blockIdx.x & 7);
+    else if (EPI == EPI_SWIGLU_FWD) row0[t] = 16 * blockIdx.x + t * ep.I;                              // gate, up
     else if (EPI == EPI_ROPE) row0[t] = 128 * (blockIdx.x >> 2) + 16 * (blockIdx.x & 3) + 64 * t;      // j, j + 64 of a head
     else row0[t] = 16 * (NT * blockIdx.x + t);
   }
   const bf16* wp[NT];
 #pragma unroll
-  for (int t = 0; t < NT; t++) wp[t] = W + (int64_t)min(row0[t] + c, N - 1) * ldw + 8 * q;
+  for (int t = 0; t < NT; t++) wp[t] = W + (int64_t)(PAIRED ? row0[t] + (c & 7) + (c >> 3) * (EPI == EPI_ROPE ? 64 : ep.I) : min(row0[t] + c, N - 1)) * ldw + 8 * q;
   const bf16* ap = (NORM ? rows + min(c, M - 1) * (K + 8) : A + (int64_t)min(c, M - 1) * lda) + 8 * q;
 
   f32x4 acc[NT];
@@ -81,11 +100,10 @@ __global__ __launch_bounds__(64 * SK_WAVES) void gemm_skinny_kernel(const bf16* 
 #pragma unroll
         for (int e = 0; e < 8; e++) ss = fmaf((float)x[e], (float)x[e], ss);
       }
-#pragma unroll
-      for (int d = 32; d > 0; d >>= 1) ss += __shfl_xor(ss, d, 64);
+      ss = wave_sum(ss);
       if (lane == 0) sums[r * SK_WAVES + wave] = ss;
     }
-    if (EPI == EPI_ROPE && tid < 16 * M) {   // the angles of this block's columns, one per thread, rounded as the table's
+    if (EPI == EPI_ROPE && tid < 16 * M && (tid & 15) < (PAIRED ? 8 : 16)) {   // the angles of this block's columns, one per thread, rounded as the table's
       const float th = (float)ep.positions[tid >> 4] * ep.inv_freq[(row0[0] & 127) + (tid & 15)];
       angles[tid >> 4][tid & 15][0] = (bf16)cosf(th), angles[tid >> 4][tid & 15][1] = (bf16)sinf(th);
     }
@@ -115,6 +133,7 @@ __global__ __launch_bounds__(64 * SK_WAVES) void gemm_skinny_kernel(const bf16* 
       af[u] = *reinterpret_cast<const bf16x8*>(ap + (int64_t)(s + u) * 32);
     }
     fetched = false;
+    if (BATCH) FENCE();
     multiply();
   }
   if (s < s1) {   // the remainder, all of it in flight at once
@@ -134,13 +153,15 @@ __global__ __launch_bounds__(64 * SK_WAVES) void gemm_skinny_kernel(const bf16* 
   __syncthreads();
   // lane 16 q + c of the first wavefront owns row c of A and columns 4 q .. 4 q + 3 of every group of W rows
   const int row = c;
-  if (tid >= 64 || row >= M) return;
-  f32x4 v[NT];
+  if (tid >= 64 || row >= M || (PAIRED && q >= 2)) return;
+  constexpr int NV = PAIRED ? 2 : NT;   // PAIRED: the partners' columns lie 32 lanes on
+  f32x4 v[NV];
 #pragma unroll
-  for (int t = 0; t < NT; t++) {
-    v[t] = red[0][t][lane];
+  for (int t = 0; t < NV; t++) {
+    auto part = [&](int w) { return PAIRED ? red[w][0][lane + 32 * t] : red[w][t][lane]; };
+    v[t] = part(0);
 #pragma unroll
-    for (int w = 1; w < SK_WAVES; w++) v[t] += red[w][t][lane];
+    for (int w = 1; w < SK_WAVES; w++) v[t] += part(w);
   }
   auto rounded = [](f32x4 x) {
     bf16x4 w;
@@ -204,15 +225,34 @@ __global__ __launch_bounds__(64 * SK_WAVES) void gemm_skinny_kernel(const bf16* 
   }
 }
 
-template <int NT, int U, int EPI, bool NORM = false>
-int launch(const char* name, int blocks, const bf16* A, const bf16* W, bf16* C, const bf16* bias, int M, int N, int K, int64_t lda,
+template <int NT, int U, int SK_WAVES, int EPI, bool NORM = false, bool BATCH = true>
+int launch(const char* name, const bf16* A, const bf16* W, bf16* C, const bf16* bias, int M, int N, int K, int64_t lda,
            int64_t ldw, int64_t ldc, int accumulate, const GemmEpi& ep, hipStream_t st) {
   const size_t smem = NORM ? sizeof(bf16) * M * (K + 8) : 0;
-  auto kern = &gemm_skinny_kernel<NT, U, EPI, NORM>;
+  auto kern = &gemm_skinny_kernel<NT, U, SK_WAVES, EPI, NORM, BATCH>;
   if (NORM)
     if (int rc = ody_allow_dynamic_lds(reinterpret_cast<const void*>(kern), ODY_SKINNY_NORM_BYTES, name)) return rc;
-  ODY_LAUNCH(name, st, kern, dim3(blocks), dim3(64 * SK_WAVES), smem, A, W, C, bias, M, N, K, lda, ldw, ldc, accumulate, ep);
+  ODY_LAUNCH(name, st, kern, dim3(((N + 15) / 16 + NT - 1) / NT), dim3(64 * SK_WAVES), smem, A, W, C, bias, M, N, K, lda, ldw, ldc, accumulate, ep);
   return ody_check_launch(name);
+}
+
+// What a block takes.  us, weights cold, the instance chosen / the best of the others (<2, 8, 8> and <1, 8, 8> included):
+//   M <= 4: one group of 16 rows, 8 wavefronts: 4096 x 4096 8.0 / 8.9, 2048 x 5632 9.0 / 9.7, with the norm 22016 x 4096 33.0 / 33.1, 6144 x 2048 8.4 / 8.1.  From
+//   1024 groups on 4 wavefronts with twice the loads: 32000 x 4096 45.3 / 44.8 and 46.8, M = 4 49.5 / 52.7, 32000 x 2048 24.9 / 25.8; where rows are long, too,
+//   but not with one row of A: 4096 x 11008, M = 4, 19.9 / 20.9 and 21.3, M = 1 19.3 / 19.3, 4096 x 14336, M = 1, 22.1 / 22.8.
+//   M > 4: a group's fragments of A weigh as much as those of W.  Two groups share them where there are many: M = 8, 32000 x 4096 53.0 / 56.4, 22016 x 4096
+//   38.4 / 40.6; M = 16 60.2 / 65.5, 44.1 / 47.1; below 1024 groups where rows are long or many: 6144 x 4096, M = 8, 13.8 / 13.8, M = 16 15.2 / 15.9, 5632 x 1024
+//   6.4 / 6.3, but 11264 x 2048, M = 8, 14.8 / 13.3.  Otherwise one group: 4096 x 11008, M = 8, 21.0 / 22.5, 3072 x 2048 6.0 / 7.7 (8 wavefronts where blocks are
+//   fewer than units and K is short: 2048 x 2048 5.6 / 5.9, 2048 x 5632 11.4 / 11.1).
+template <int EPI>
+int launch_for(const char* name, const bf16* A, const bf16* W, bf16* C, const bf16* bias, int M, int N, int K, int64_t lda, int64_t ldw, int64_t ldc,
+               int accumulate, const GemmEpi& ep, hipStream_t st) {
+  const int groups = (N + 15) / 16;
+  if (M > 4 && groups >= 1024) return launch<2, 4, 4, EPI, false, false>(name, A, W, C, bias, M, N, K, lda, ldw, ldc, accumulate, ep, st);
+  if (M > 4 && groups >= 320 && (K > 2048 || M > 8)) return launch<2, 4, 4, EPI>(name, A, W, C, bias, M, N, K, lda, ldw, ldc, accumulate, ep, st);
+  if (M > 4 ? groups >= 256 || K > 4096 || M > 8 : groups >= 1024 || (groups >= 256 && K > 4096 && M > 1))
+    return launch<1, 8, 4, EPI>(name, A, W, C, bias, M, N, K, lda, ldw, ldc, accumulate, ep, st);
+  return launch<1, 4, 8, EPI>(name, A, W, C, bias, M, N, K, lda, ldw, ldc, accumulate, ep, st);
 }
 
 }  // namespace
@@ -229,21 +269,13 @@ bool ody_gemm_skinny_ok(int epi, int M, int N) {
 
 int ody_launch_gemm_skinny(int epi, const bf16* A, const bf16* W, bf16* C, const bf16* bias, int M, int N, int K, int64_t lda,
                            int64_t ldw, int64_t ldc, int accumulate, const GemmEpi& ep, hipStream_t st) {
-  const int groups = (N + 15) / 16;
   if (ep.norm) {
     if (epi == EPI_SWIGLU_FWD)
-      return launch<2, 8, EPI_SWIGLU_FWD, true>("gemm_skinny_norm_swiglu", groups / 2, A, W, C, bias, M, N, K, lda, ldw, ldc, accumulate, ep, st);
-    return launch<2, 8, EPI_ROPE, true>("gemm_skinny_norm_rope", groups / 2, A, W, C, bias, M, N, K, lda, ldw, ldc, accumulate, ep, st);
+      return launch<1, 4, 8, EPI_SWIGLU_FWD, true>("gemm_skinny_norm_swiglu", A, W, C, bias, M, N, K, lda, ldw, ldc, accumulate, ep, st);
+    return launch<1, 4, 8, EPI_ROPE, true>("gemm_skinny_norm_rope", A, W, C, bias, M, N, K, lda, ldw, ldc, accumulate, ep, st);
   }
-  if (epi == EPI_SWIGLU_FWD)
-    return launch<2, 8, EPI_SWIGLU_FWD>("gemm_skinny_swiglu", groups / 2, A, W, C, bias, M, N, K, lda, ldw, ldc, accumulate, ep, st);
-  if (epi == EPI_ROPE)
-    return launch<2, 8, EPI_ROPE>("gemm_skinny_rope", groups / 2, A, W, C, bias, M, N, K, lda, ldw, ldc, accumulate, ep, st);
-  const bool wide = groups >= 1024;
-  if (epi == EPI_RESIDUAL) {
-    if (wide) return launch<2, 8, EPI_RESIDUAL>("gemm_skinny_residual", (groups + 1) / 2, A, W, C, bias, M, N, K, lda, ldw, ldc, accumulate, ep, st);
-    return launch<1, 8, EPI_RESIDUAL>("gemm_skinny_residual", groups, A, W, C, bias, M, N, K, lda, ldw, ldc, accumulate, ep, st);
-  }
-  if (wide) return launch<2, 8, EPI_NONE>("gemm_skinny", (groups + 1) / 2, A, W, C, bias, M, N, K, lda, ldw, ldc, accumulate, ep, st);
-  return launch<1, 8, EPI_NONE>("gemm_skinny", groups, A, W, C, bias, M, N, K, lda, ldw, ldc, accumulate, ep, st);
+  if (epi == EPI_SWIGLU_FWD) return launch_for<EPI_SWIGLU_FWD>("gemm_skinny_swiglu", A, W, C, bias, M, N, K, lda, ldw, ldc, accumulate, ep, st);
+  if (epi == EPI_ROPE) return launch_for<EPI_ROPE>("gemm_skinny_rope", A, W, C, bias, M, N, K, lda, ldw, ldc, accumulate, ep, st);
+  if (epi == EPI_RESIDUAL) return launch_for<EPI_RESIDUAL>("gemm_skinny_residual", A, W, C, bias, M, N, K, lda, ldw, ldc, accumulate, ep, st);
+  return launch_for<EPI_NONE>("gemm_skinny", A, W, C, bias, M, N, K, lda, ldw, ldc, accumulate, ep, st);
 }

@@ -338,3 +338,34 @@ def test_slabs_that_k_does_not_fill(op, M, N, K, dev):
     b = inside(randn((K, N), 52, std=0.05, dtype=torch.bfloat16))
     y = ops.gemm({"nn": ops.GEMM_NN, "tn": ops.GEMM_TN}[op], a, b)
     assert rel_err(y, (a.float().t() if op == "tn" else a.float()) @ b.float()) <= TOL_BF16
+
+
+@pytest.mark.parametrize("M", [1, 4, 5, 8, 9, 16])
+@pytest.mark.parametrize("N,K", [(4992, 72), (5120, 2056), (5120, 2048), (16256, 136), (16384, 72)], ids=lambda v: str(v))
+@pytest.mark.parametrize("what", ["plain", "residual", "swiglu", "rope"])
+def test_few_rows_around_the_lines_between_instances(what, N, K, M, dev):
+    """312 and 320, 1016 and 1024 groups of 16 rows of W, rows of A on both sides of 4 and 8, K on both sides of 2048: one or two groups a block on 4 or 8
+    wavefronts, the pairs of an epilogue inside a group or in two."""
+    from odysseus_transformer_amd import ops
+    print(f"what={what} M={M} N={N} K={K}", flush=True)
+    dt = torch.bfloat16
+    x, w = randn((M, K), 61, dtype=dt).to(dev), randn((N, K), 62, std=0.05, dtype=dt).to(dev)
+    ref = x.float() @ w.float().t()
+    if what == "plain":
+        assert rel_err(ops.gemm(ops.GEMM_NT, x, w), ref) <= TOL_BF16
+    elif what == "residual":
+        r = randn((M, N), 63, dtype=dt).to(dev)
+        assert rel_err(ops.linear_residual(x, w, r), ref + r.float()) <= TOL_BF16
+    elif what == "swiglu":
+        g, u = ref.to(dt).float().chunk(2, -1)
+        want = torch.nn.functional.silu(g) * u
+        gate_up, h = ops.linear_swiglu(x, w)
+        assert rel_err(gate_up, ref) <= TOL_BF16 and rel_err(h, want) <= TOL_BF16
+        assert torch.equal(ops.linear_swiglu_h(x, w), h)
+    else:
+        table = ops.rope_table(torch.arange(7, 7 + M, device=dev), M, 128)
+        n_rot = N // 128 - 3
+        cos, sin = table.float().view(M, 1, 64, 2).unbind(-1)
+        a, b = ref[:, :n_rot * 128].reshape(M, n_rot, 2, 64).unbind(2)
+        ref[:, :n_rot * 128] = torch.stack([a * cos - b * sin, b * cos + a * sin], 2).reshape(M, -1)
+        assert rel_err(ops.linear_rope(x, w, table, n_rot, 128), ref) <= TOL_BF16
