@@ -42,7 +42,7 @@ def _load():
                       "`python -m odysseus_transformer_amd.build` builds it.", RuntimeWarning, stacklevel=4)
         return None
     addresses = {name: C.cast(getattr(lib, name), C.c_void_p).value for name in _lib.SIGNATURES}
-    module.bind(addresses, _Arena, ops.scratch, _raise, torch.OutOfMemoryError)
+    module.bind(addresses, _Arena, ops.scratch, _raise, torch.OutOfMemoryError, lambda: ops._never_keeps_ds(), lambda *args: ops.attn_bwd(*args))
     return module
 
 

@@ -3,7 +3,7 @@
 //
 // Bound by the interpreter: the wrappers in ops.py take 9 to 15 us per op, of which the launch is 2; a decoding step, a short sequence
 // or a small layer is a row of ops whose kernels take no longer.  A decoding step of hidden 4096 behind 8191 tokens (8 ops of 110 us of
-// kernels): 176 us a pass through Python, 110 through here; attention of 4 x 331 tokens, forward and backward: 88 us of host work, now 65.
+// kernels): 176 us a pass through Python, 110 through here; attention of 4 x 331 tokens, forward and backward: 88 us of host work, now 65 (without the graph).
 //
 // A function here answers None for whatever is not the plain form of its op: a tensor that is not a dense CUDA tensor of the current
 // device (subclasses, wrappers of function transforms, conjugate or negative views included), a shape or stride that needs a copy or an
@@ -11,7 +11,7 @@
 // definition of what an op accepts and of the error it raises.
 //
 // No state but what bind() is given once: the addresses of the library's entry points, so that this module uses the library that
-// Python loaded, and four Python objects.
+// Python loaded, and six Python objects.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
@@ -22,6 +22,7 @@
 #include <c10/hip/HIPStream.h>
 #include <c10/util/Exception.h>
 #include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <cmath>
@@ -48,6 +49,8 @@ PyObject* arena_holder = nullptr;   // class whose attribute `instance` is the s
 PyObject* scratch_fn = nullptr;     // scratch(nbytes, name, device) of ops.py
 PyObject* raise_fn = nullptr;       // raises for (name, status)
 PyObject* no_memory = nullptr;      // torch.OutOfMemoryError
+PyObject* never_keeps_ds = nullptr; // _never_keeps_ds() of ops.py
+PyObject* attn_bwd_fn = nullptr;    // attn_bwd(q, k, v, out, lse, dout, causal, scale) of ops.py
 
 struct NotPlain {};      // the caller answers None
 struct PythonError {};   // a Python exception is set
@@ -59,6 +62,10 @@ constexpr c10::DispatchKeySet special{c10::DispatchKey::Python,          c10::Di
 
 void need(bool plain) {
   if (!plain) throw NotPlain{};
+}
+
+bool plain_tensor(const at::Tensor& t) {
+  return t.defined() && t.is_cuda() && t.layout() == c10::Layout::Strided && !t.unsafeGetTensorImpl()->key_set().has_any(special) && t.numel() > 0;
 }
 
 // The arguments of one call; `like` (the first tensor) sets device and dtype.
@@ -75,7 +82,7 @@ struct Call {
     PyObject* o = args[i];
     need(THPVariable_CheckExact(o));
     const at::Tensor& t = THPVariable_Unpack(o);
-    need(t.defined() && t.is_cuda() && t.layout() == c10::Layout::Strided && !t.unsafeGetTensorImpl()->key_set().has_any(special) && t.numel() > 0);
+    need(plain_tensor(t));
     if (device < 0) {
       device = c10::hip::current_device();
       stream = c10::hip::getCurrentHIPStream(device).stream();
@@ -315,33 +322,54 @@ void check_kv(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v) {
   need(k.sizes() == v.sizes() && k.size(0) == q.size(0) && k.size(3) == q.size(3));
 }
 
-// (q, k, v, causal, scale) -> (out, lse)
-PyObject* attn_fwd(Call c) {
-  const at::Tensor &q = c.heads(0, nullptr), &k = c.heads(1, &q), &v = c.heads(2, &q);
-  check_kv(q, k, v);
-  const bool causal = c.flag(3);
-  const float scale = (float)c.real(4);
+struct OutLse { at::Tensor out, lse; };
+OutLse run_attn_fwd(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, bool causal, float scale, hipStream_t stream) {
   const int B = q.size(0), Lq = q.size(1), Hq = q.size(2), D = q.size(3), Lk = k.size(1), Hkv = k.size(2);
   at::Tensor out = make({B, Lq, Hq, D}, q), lse = make_f32({B, Hq, Lq}, q);
   Scratch ws(lib.ody_attn_fwd_workspace_bytes(B, Lq, Lk, Hq, Hkv, D, dt(q)), "attn_fwd_workspace", q);
   CALL(ody_attn_fwd, q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), lse.data_ptr<float>(), B, Lq, Lk, Hq, Hkv, D, STRIDES(q), STRIDES(k),
-       STRIDES(v), STRIDES(out), scale, (int)causal, dt(q), ws.ptr(), ws.bytes, (void*)c.stream);
-  return tuple(out, lse);
+       STRIDES(v), STRIDES(out), scale, (int)causal, dt(q), ws.ptr(), ws.bytes, (void*)stream);
+  return {out, lse};
+}
+
+// (q, k, v, causal, scale) -> (out, lse)
+PyObject* attn_fwd(Call c) {
+  const at::Tensor &q = c.heads(0, nullptr), &k = c.heads(1, &q), &v = c.heads(2, &q);
+  check_kv(q, k, v);
+  const OutLse r = run_attn_fwd(q, k, v, c.flag(3), (float)c.real(4), c.stream);
+  return tuple(r.out, r.lse);
 }
 
 // (q, k, v, out, lse, dout, causal, scale, dq or None, dk or None, dv or None, table_q or None, table_k or None) -> (dq, dk, dv)
+void run_attn_bwd(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, const at::Tensor& out, const at::Tensor& lse, const at::Tensor& dout,
+                  bool causal, float scale, at::Tensor (&g)[3], const at::Tensor* const (&table)[2], hipStream_t stream) {
+  const int B = q.size(0), Lq = q.size(1), Hq = q.size(2), D = q.size(3), Lk = k.size(1), Hkv = k.size(2);
+  Scratch ws(lib.ody_attn_bwd_workspace_bytes(B, Lq, Lk, Hq, Hkv, D, dt(q)), "attn_bwd_workspace", q);
+#define BWD_ARGS                                                                                                                   \
+  q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), lse.data_ptr<float>(), dout.data_ptr(), g[0].data_ptr(), g[1].data_ptr(), \
+      g[2].data_ptr(), B, Lq, Lk, Hq, Hkv, D, STRIDES(q), STRIDES(k), STRIDES(v), STRIDES(out), STRIDES(dout), STRIDES(g[0]),       \
+      STRIDES(g[1]), STRIDES(g[2]), scale, (int)causal, 0, dt(q), ws.ptr(), ws.bytes, (void*)stream
+  if (table[0]) CALL(ody_attn_bwd_rope, BWD_ARGS, table[0]->data_ptr(), table[1]->data_ptr());
+  else CALL(ody_attn_bwd, BWD_ARGS);
+}
+void check_bwd(const at::Tensor& q, const at::Tensor& out, const at::Tensor& lse, const at::Tensor& dout) {
+  need(out.sizes() == q.sizes() && dout.sizes() == q.sizes());
+  need(lse.scalar_type() == at::kFloat && lse.is_contiguous() && lse.dim() == 3 && lse.size(0) == q.size(0) && lse.size(1) == q.size(2) &&
+       lse.size(2) == q.size(1));
+}
+at::Tensor gradient_of(const at::Tensor& t) { return at::empty_like(t, t.options().requires_grad(false)); }
+
 PyObject* attn_bwd(Call c) {
   const at::Tensor &q = c.heads(0, nullptr), &k = c.heads(1, &q), &v = c.heads(2, &q), &out = c.heads(3, &q), &lse = c.any(4), &dout = c.heads(5, &q);
   check_kv(q, k, v);
   const bool causal = c.flag(6);
   const float scale = (float)c.real(7);
-  const int B = q.size(0), Lq = q.size(1), Hq = q.size(2), D = q.size(3), Lk = k.size(1), Hkv = k.size(2);
-  need(out.sizes() == q.sizes() && dout.sizes() == q.sizes());
-  need(lse.scalar_type() == at::kFloat && lse.is_contiguous() && lse.dim() == 3 && lse.size(0) == B && lse.size(1) == Hq && lse.size(2) == Lq);
+  const int64_t B = q.size(0), Lq = q.size(1), D = q.size(3), Lk = k.size(1);
+  check_bwd(q, out, lse, dout);
   at::Tensor g[3];
   const at::Tensor* of[3] = {&q, &k, &v};
   for (int i = 0; i < 3; i++) {
-    g[i] = c.none(8 + i) ? at::empty_like(*of[i], of[i]->options().requires_grad(false)) : c.heads(8 + i, &q);
+    g[i] = c.none(8 + i) ? gradient_of(*of[i]) : c.heads(8 + i, &q);
     need(g[i].sizes() == of[i]->sizes() && g[i].stride(3) == 1);
   }
   need(c.none(11) == c.none(12));
@@ -349,16 +377,96 @@ PyObject* attn_bwd(Call c) {
   if (!c.none(11))
     for (int i = 0; i < 2; i++) {
       table[i] = &c.matrix(11 + i, &q);
-      need(q.scalar_type() == at::kBFloat16 && table[i]->is_contiguous() && table[i]->size(0) == (int64_t)B * (i ? Lk : Lq) && table[i]->size(1) == D);
+      need(q.scalar_type() == at::kBFloat16 && table[i]->is_contiguous() && table[i]->size(0) == B * (i ? Lk : Lq) && table[i]->size(1) == D);
     }
-  Scratch ws(lib.ody_attn_bwd_workspace_bytes(B, Lq, Lk, Hq, Hkv, D, dt(q)), "attn_bwd_workspace", q);
-#define BWD_ARGS                                                                                                                   \
-  q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), lse.data_ptr<float>(), dout.data_ptr(), g[0].data_ptr(), g[1].data_ptr(), \
-      g[2].data_ptr(), B, Lq, Lk, Hq, Hkv, D, STRIDES(q), STRIDES(k), STRIDES(v), STRIDES(out), STRIDES(dout), STRIDES(g[0]),       \
-      STRIDES(g[1]), STRIDES(g[2]), scale, (int)causal, 0, dt(q), ws.ptr(), ws.bytes, (void*)c.stream
-  if (table[0]) CALL(ody_attn_bwd_rope, BWD_ARGS, table[0]->data_ptr(), table[1]->data_ptr());
-  else CALL(ody_attn_bwd, BWD_ARGS);
+  run_attn_bwd(q, k, v, out, lse, dout, causal, scale, g, table, c.stream);
   return tuple(g[0], g[1], g[2]);
+}
+
+// ------------------------------------------------------------------------------------------------ the attention routine as a node of the graph
+// What FlashAttnFunc of ops.py is, without dropout.  Forward and backward of 4 x 331 tokens, 8 heads on 2, 49 us of kernels, in a loop: 99 us of host work
+// a pass through autograd's Python function, 80 through this one, of which an empty graph and the clearing of gradients take 35.  Its backward holds the
+// interpreter, as the scratch arena and the budget of kept dS are Python's, and where the plain form of attn_bwd is not the one to be taken it calls
+// that function.  Transforms, forward mode and tracing are left to the Python function (ops.transformed).
+struct Interpreter {
+  PyGILState_STATE state = PyGILState_Ensure();
+  ~Interpreter() { PyGILState_Release(state); }
+};
+[[noreturn]] void throw_python_error() {
+  python_error e;
+  e.persist();
+  throw e;
+}
+
+struct FlashNode : torch::autograd::Function<FlashNode> {
+  using Tensors = torch::autograd::variable_list;
+
+  static Tensors forward(torch::autograd::AutogradContext* ctx, const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, bool causal, double scale,
+                         void* stream) {
+    OutLse r = run_attn_fwd(q, k, v, causal, (float)scale, (hipStream_t)stream);
+    ctx->save_for_backward({q, k, v, r.out, r.lse});
+    ctx->saved_data["causal"] = causal;
+    ctx->saved_data["scale"] = scale;
+    ctx->mark_non_differentiable({r.lse});
+    ctx->set_materialize_grads(false);
+    return {r.out, r.lse};
+  }
+
+  static Tensors backward(torch::autograd::AutogradContext* ctx, const Tensors& grads) {
+    const Tensors saved = ctx->get_saved_variables();
+    const at::Tensor &q = saved[0], &k = saved[1], &v = saved[2], &out = saved[3], &lse = saved[4];
+    at::Tensor dout = grads[0].defined() ? grads[0] : at::zeros_like(out);
+    if (dout.dim() == 4 && dout.stride(3) != 1) dout = dout.contiguous();
+    const bool causal = ctx->saved_data["causal"].toBool();
+    const double scale = ctx->saved_data["scale"].toDouble();
+    Interpreter held;
+    try {
+      if (PyObject* never = PyObject_CallNoArgs(never_keeps_ds)) {
+        const bool plain = never == Py_True;
+        Py_DECREF(never);
+        if (plain) {
+          try {
+            const c10::DeviceIndex device = c10::hip::current_device();
+            for (const at::Tensor* t : {&q, &k, &v, &out, &lse, (const at::Tensor*)&dout}) need(plain_tensor(*t) && t->get_device() == device);
+            for (const at::Tensor* t : {&k, &v, &out, (const at::Tensor*)&dout}) need(t->scalar_type() == q.scalar_type());
+            for (const at::Tensor* t : {&q, &k, &v, &out, (const at::Tensor*)&dout}) need(t->dim() == 4 && t->stride(3) == 1);
+            check_bwd(q, out, lse, dout);
+            at::Tensor g[3] = {gradient_of(q), gradient_of(k), gradient_of(v)};
+            for (const at::Tensor& t : g) need(t.stride(3) == 1);
+            const at::Tensor* const table[2] = {nullptr, nullptr};
+            run_attn_bwd(q, k, v, out, lse, dout, causal, (float)scale, g, table, c10::hip::getCurrentHIPStream(device).stream());
+            return {g[0], g[1], g[2], at::Tensor(), at::Tensor(), at::Tensor()};
+          } catch (const NotPlain&) {
+          }
+        }
+        const at::Tensor args[6] = {q, k, v, out, lse, dout};
+        PyObject* a = PyTuple_New(8);
+        if (!a) throw PythonError{};
+        for (int i = 0; i < 6; i++) PyTuple_SET_ITEM(a, i, THPVariable_Wrap(args[i]));
+        PyTuple_SET_ITEM(a, 6, PyBool_FromLong(causal));
+        PyTuple_SET_ITEM(a, 7, PyFloat_FromDouble(scale));
+        PyObject* r = PyErr_Occurred() ? nullptr : PyObject_CallObject(attn_bwd_fn, a);
+        Py_DECREF(a);
+        if (!r) throw PythonError{};
+        Tensors g;
+        for (int i = 0; i < 3; i++) g.push_back(THPVariable_Unpack(PyTuple_GET_ITEM(r, i)));
+        Py_DECREF(r);
+        g.resize(6);
+        return g;
+      }
+      throw PythonError{};
+    } catch (const PythonError&) {
+      throw_python_error();
+    }
+  }
+};
+
+// (q, k, v, causal, scale) -> (out, lse), recorded where one of them requires a gradient
+PyObject* flash(Call c) {
+  const at::Tensor &q = c.heads(0, nullptr), &k = c.heads(1, &q), &v = c.heads(2, &q);
+  check_kv(q, k, v);
+  const auto r = FlashNode::apply(q, k, v, c.flag(3), c.real(4), (void*)c.stream);
+  return tuple(r[0], r[1]);
 }
 
 const int64_t* positions(Call& c, Py_ssize_t i, int64_t rows) {
@@ -455,10 +563,10 @@ PyObject* method(PyObject*, PyObject* const* args, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
-// (addresses by name, arena holder, scratch, raise, torch.OutOfMemoryError)
+// (addresses by name, arena holder, scratch, raise, torch.OutOfMemoryError, _never_keeps_ds, attn_bwd)
 PyObject* bind(PyObject*, PyObject* const* args, Py_ssize_t n) {
-  if (n != 5 || !PyDict_Check(args[0])) {
-    PyErr_SetString(PyExc_TypeError, "bind(addresses, arena_holder, scratch, raise, no_memory)");
+  if (n != 7 || !PyDict_Check(args[0])) {
+    PyErr_SetString(PyExc_TypeError, "bind(addresses, arena_holder, scratch, raise, no_memory, never_keeps_ds, attn_bwd)");
     return nullptr;
   }
 #define X(name)                                                                      \
@@ -473,8 +581,8 @@ PyObject* bind(PyObject*, PyObject* const* args, Py_ssize_t n) {
   }
   ODY_ENTRY_POINTS(X)
 #undef X
-  PyObject** to[4] = {&arena_holder, &scratch_fn, &raise_fn, &no_memory};
-  for (int i = 0; i < 4; i++) {
+  PyObject** to[6] = {&arena_holder, &scratch_fn, &raise_fn, &no_memory, &never_keeps_ds, &attn_bwd_fn};
+  for (int i = 0; i < 6; i++) {
     Py_INCREF(args[1 + i]);
     Py_XSETREF(*to[i], args[1 + i]);
   }
@@ -485,7 +593,7 @@ PyObject* bind(PyObject*, PyObject* const* args, Py_ssize_t n) {
 PyMethodDef methods[] = {
     {"bind", (PyCFunction)(void (*)(void))bind, METH_FASTCALL, nullptr},
     METHOD(rmsnorm_fwd, 3), METHOD(rmsnorm_bwd, 5), METHOD(gemm, 3), METHOD(linear_residual, 3), METHOD(linear_rope, 5), METHOD(linear_swiglu, 2),
-    METHOD(linear_swiglu_h, 2), METHOD(linear_dgrad_swiglu, 3), METHOD(attn_fwd, 5), METHOD(attn_bwd, 13), METHOD(rope, 6), METHOD(rope_table, 5),
+    METHOD(linear_swiglu_h, 2), METHOD(linear_dgrad_swiglu, 3), METHOD(attn_fwd, 5), METHOD(attn_bwd, 13), METHOD(flash, 5), METHOD(rope, 6), METHOD(rope_table, 5),
     METHOD(norm_linear_rope, 8), METHOD(norm_linear_swiglu_h, 4),
     METHOD(current_stream, 0), {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_odysseus_native", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};

@@ -75,6 +75,12 @@ def watched() -> bool:
             or torch._C._get_tracing_state() is not None)
 
 
+def transformed() -> bool:
+    """Whether something other than reverse-mode autograd looks at a call: forward-mode differentiation, function transforms, tracing."""
+    return (torch.autograd.forward_ad._current_level >= 0 or torch._C._are_functorch_transforms_active()
+            or torch._C._get_tracing_state() is not None or torch.compiler.is_compiling())
+
+
 def scratch(nbytes: int, name: str, device) -> torch.Tensor:
     """Kernel scratch of `nbytes` bytes.  When the process-wide arena is set up for this device
     (utils.globals._set_global_memory_buffer, as the reference's train.py:62 does), the bytes come
@@ -1016,7 +1022,10 @@ def flash_attn_func(q, k, v, dropout_p: float = 0.0, softmax_scale: Optional[flo
     a host value: a captured graph replays the mask it was captured with -- pass `seed` per step there."""
     if dropout_p != 0.0 and seed is None:
         seed = int(torch.randint(0, 1 << 62, (1,)).item())
-    out, lse = run_function(FlashAttnFunc, q, k, v, softmax_scale, causal, float(dropout_p), seed)
+    recorded = None
+    if dropout_p == 0.0 and q.is_cuda and torch.is_grad_enabled() and not transformed():
+        recorded = native.flash(q, k, v, bool(causal), 1.0 / math.sqrt(q.shape[-1]) if softmax_scale is None else softmax_scale)
+    out, lse = recorded or run_function(FlashAttnFunc, q, k, v, softmax_scale, causal, float(dropout_p), seed)
     return (out, lse) if return_lse else out
 
 

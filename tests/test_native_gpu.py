@@ -417,3 +417,101 @@ def test_arena_without_room_for_all_of_the_scratch(dev, monkeypatch):
     assert _lib.load().ody_gemm_workspace_bytes(ops.GEMM_NT, 512, 512, 64 * 512, _lib.ODY_F32) > least
     with pytest.raises(torch.OutOfMemoryError):
         ops.gemm(ops.GEMM_NT, x, w)
+
+
+def _flash_inputs(dev, dtype=torch.bfloat16, L=197, hq=8, hkv=2, D=128, needs=(True, True, True)):
+    big = randn((2, L, hq + 2 * hkv, D), 71, dtype=dtype).to(dev)
+    q, k, v = (t.detach() for t in big.split([hq, hkv, hkv], dim=2))   # heads of one packed buffer: rows far apart
+    return [t.requires_grad_(n) for t, n in zip((q, k, v), needs)]
+
+
+@pytest.mark.parametrize("dtype,D", [(torch.bfloat16, 128), (torch.bfloat16, 64), (torch.float32, 64)], ids=["bf16_128", "bf16_64", "f32_64"])
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("needs", [(True, True, True), (False, True, False), (True, False, False)], ids=lambda n: "".join("nq"[x] for x in n))
+def test_attention_routine_as_a_node_of_its_own(dtype, D, causal, needs, dev, monkeypatch):
+    """The routine through the node in C++ and through FlashAttnFunc: outputs, gradients and what requires one, bit for bit; a gradient that arrives
+    with a strided head dimension, expanded, or not at all; a graph that is kept and walked twice."""
+    from odysseus_transformer_amd import ops
+
+    def run():
+        q, k, v = _flash_inputs(dev, dtype, D=D, needs=needs)
+        out, lse = ops.flash_attn_func(q, k, v, softmax_scale=0.1, causal=causal, return_lse=True)
+        assert out.requires_grad and not lse.requires_grad and out.grad_fn is not None
+        got = [out.detach(), lse]
+        inputs = [t for t, n in zip((q, k, v), needs) if n]
+        for dout in (randn(out.shape, 72, dtype=dtype).to(dev), randn((2, D, 197, 8), 73, dtype=dtype).to(dev).permute(0, 2, 3, 1),
+                     torch.ones((), dtype=dtype, device=dev).expand(out.shape)):
+            got += torch.autograd.grad(out, inputs, dout, retain_graph=True)
+        return got
+
+    here, there, taken = _both(monkeypatch, run)
+    assert taken[0] == "flash" and "attn_bwd" not in taken
+    _same(here, there)
+
+
+def test_attention_node_keeps_what_autograd_promises(dev, monkeypatch):
+    """Hooks on saved tensors, modification in place, a graph walked twice without being kept, a budget of kept dS set between forward and backward,
+    transforms and forward mode: as through FlashAttnFunc."""
+    from odysseus_transformer_amd import _lib, ops
+    q, k, v = _flash_inputs(dev)
+    packed = []
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: (packed.append(t.shape), t.cpu())[1], lambda t: t.to(dev)):
+        out = ops.flash_attn_func(q, k, v, causal=True)
+    assert "FlashNode" in out.grad_fn.name() and len(packed) == 5
+    dout = randn(out.shape, 74, dtype=torch.bfloat16).to(dev)
+    offloaded = torch.autograd.grad(out, (q, k, v), dout)
+    plain = torch.autograd.grad(ops.flash_attn_func(q, k, v, causal=True), (q, k, v), dout)
+    _same(offloaded, plain)
+
+    out = ops.flash_attn_func(q, k, v, causal=True)
+    torch.autograd.grad(out, q, dout)
+    with pytest.raises(RuntimeError, match="second time"):
+        torch.autograd.grad(out, q, dout)
+    out = ops.flash_attn_func(q, k, v, causal=True)
+    with torch.no_grad():
+        v.mul_(1.0)
+    with pytest.raises(RuntimeError, match="inplace"):
+        torch.autograd.grad(out, q, dout)
+
+    q, k, v = (t.requires_grad_(True) for t in randn((3, 1, 2048, 4, 128), 75, dtype=torch.bfloat16).to(dev))
+    dout = randn((1, 2048, 4, 128), 76, dtype=torch.bfloat16).to(dev)
+    lib = _lib.load()
+
+    def names(fn):
+        import ctypes
+        lib.ody_profile_enable(1)
+        fn()
+        torch.cuda.synchronize()
+        buf = ctypes.create_string_buffer(1 << 16)
+        lib.ody_profile_collect(buf, 1 << 16)
+        lib.ody_profile_enable(0)
+        return buf.value.decode()
+
+    out = ops.flash_attn_func(q, k, v, causal=True)
+    ops.set_keep_ds_max_bytes(1 << 30)
+    try:
+        assert "attn_bwd_dq_kept" in names(lambda: torch.autograd.grad(out, (q, k, v), dout))
+    finally:
+        ops.set_keep_ds_max_bytes(None)
+    fails = []
+    for call in (lambda: torch.func.vmap(lambda t: ops.flash_attn_func(t, t, t))(q.detach()[None]),
+                 lambda: torch.func.jvp(lambda t: ops.flash_attn_func(t, k, v), (q,), (q.detach(),))):
+        for native in (ops.native, _Off()):
+            with monkeypatch.context() as m:
+                m.setattr(ops, "native", native)
+                with pytest.raises(Exception) as e:
+                    call()
+            fails.append(type(e.value))
+    assert fails[0] is fails[1] and fails[2] is fails[3]
+
+
+def test_an_error_inside_the_attention_node_reaches_the_caller(dev, monkeypatch):
+    """The node calls attn_bwd of ops.py where its plain form is not the one to be taken; what that raises comes out of backward()."""
+    from odysseus_transformer_amd import ops
+    q, k, v = _flash_inputs(dev)
+    out = ops.flash_attn_func(q, k, v)
+    with monkeypatch.context() as m:
+        m.setattr(ops, "_never_keeps_ds", lambda: False)
+        m.setattr(ops, "attn_bwd", lambda *args: (_ for _ in ()).throw(ValueError("from inside")))
+        with pytest.raises(ValueError, match="from inside"):
+            out.backward(torch.ones_like(out))
