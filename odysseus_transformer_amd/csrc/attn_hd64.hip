@@ -14,7 +14,7 @@
 // takes every other tile; the sets add up through LDS at the end.  It is for calls with too few blocks to give every SIMD three
 // wavefronts.
 //
-// Where there are blocks enough, the forward and dK/dV take the kernels of attn_hd64_pipe.hip (dispatch: end of this file).
+// The forward and dK/dV where there are blocks enough, and most calls' dQ, take the kernels of attn_hd64_pipe.hip (dispatch: end of this file).
 //
 // Tiles and fragments: attn_rowtile.h.
 //
@@ -495,36 +495,7 @@ __global__ __launch_bounds__(256 * GROUPS, GROUPS == 1 ? 3 : 2) void attn_bwd_hd
   }
   if (grp != 0) return;
   if (qi >= p.Lq) return;
-  const int64_t at = b * p.sdq.b + h * p.sdq.h + (int64_t)qi * p.sdq.l;
-  if (p.dq_f32) {   // the running dq of a ring step: exact accumulation over the key blocks
-    float* dst = static_cast<float*>(p.dq) + at;
-#pragma unroll
-    for (int dt = 0; dt < DT; dt++)
-#pragma unroll
-      for (int a = 0; a < 4; a++) {
-        f32x4* x = reinterpret_cast<f32x4*>(dst + 32 * dt + 8 * a + 4 * g);
-        f32x4 w = {0.f, 0.f, 0.f, 0.f};
-        if (p.accumulate_dq) w = *x;
-#pragma unroll
-        for (int e = 0; e < 4; e++) w[e] += dq[dt][4 * a + e] * p.scale;
-        *x = w;
-      }
-  } else if (p.accumulate_dq) {
-    bf16* dst = static_cast<bf16*>(p.dq) + at;
-#pragma unroll
-    for (int dt = 0; dt < DT; dt++)
-#pragma unroll
-      for (int a = 0; a < 4; a++) {
-        bf16x4* x = reinterpret_cast<bf16x4*>(dst + 32 * dt + 8 * a + 4 * g);
-        const bf16x4 old = *x;
-        bf16x4 w;
-#pragma unroll
-        for (int e = 0; e < 4; e++) w[e] = (bf16)(dq[dt][4 * a + e] * p.scale + (float)old[e]);
-        *x = w;
-      }
-  } else {
-    store_row(static_cast<bf16*>(p.dq) + at, dq, p.scale, g);
-  }
+  store_dq(p, dq, b, h, qi, g);
 }
 
 inline size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
@@ -567,6 +538,15 @@ inline bool fwd_pipe_ok(const AttnParams& p) {
   const int64_t former = (int64_t)p.B * p.Hq * halves, rounds = (blocks + 255) / 256, lost = 2 * rounds - (former + 255) / 256;   // half rounds
   if (former < FEW_BLOCKS || p.Lk < (rounds == 1 ? 640 : 512)) return false;
   return lost == 0 || (lost == 1 && rounds > (p.Lk >= 2048 ? 2 : p.Lk >= 1024 ? 4 : 7));
+}
+
+// dQ in the order of attn_hd64_pipe.hip.  A unit holds two of its blocks and three of the former kernel's (one of eight wavefronts with fewer than 512).
+// Before / with it, us: 384 blocks: L = 128 15.9 / 12.4, L = 512 24.2 / 19.1, L = 4096 106 / 85; 64 to 256 blocks 1.00 to 1.09; causal, 510 blocks, L = 700
+// 26.5 / 20.6.  From 512 blocks on it wants rows long enough for a round of two blocks instead of three: L = 256, 768 blocks, 21.9 / 23.0; L = 384 24.1 / 25.2;
+// L = 512 29.3 / 29.0; L = 1000 46.3 / 44.4; causal, where a block sees half of them, L = 384, 640 blocks, 19.4 / 21.9; L = 700 25.3 / 26.5; L = 1000 30.4 / 29.3;
+// L = 2048 50.4 / 42.2.
+inline bool dq_pipe_ok(const AttnParams& p, int64_t blocks) {
+  return near(p.sk, p.sv) && (blocks < FEW_BLOCKS || p.Lk >= (p.causal ? 1000 : 512));
 }
 
 }  // namespace
@@ -624,6 +604,7 @@ int ody_launch_attn_bwd_hd64(const AttnParams& p, void* workspace, size_t worksp
     ODY_LAUNCH("attn_bwd_hd64_sum", st, attn_bwd_hd64_sum_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, p, part);
     if ((rc = ody_check_launch("attn_bwd_hd64_sum"))) return rc;
   }
+  if (dq_pipe_ok(p, nq)) return ody_launch_attn_bwd_hd64_dq_pipe(p, neg_delta, st);
   return nq < FEW_BLOCKS ? launch("attn_bwd_hd64_dq", &attn_bwd_hd64_dq_kernel<2>, nq, 2, KV_STAGE, st, p, neg_delta)
                          : launch("attn_bwd_hd64_dq", &attn_bwd_hd64_dq_kernel<1>, nq, 1, KV_STAGE, st, p, neg_delta);
 }

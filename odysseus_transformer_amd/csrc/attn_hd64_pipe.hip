@@ -2,10 +2,10 @@
 // attn_hd64.hip in the order of attn_fwd_pipe.hip and attn_bwd_pipe.hip -- the vector work of one sub-tile under the products of another,
 // instead of left to whichever wavefront of a SIMD has some.
 //
-// Tried and left: dQ in this order with 64 queries per wavefront (304 registers, one wavefront per SIMD).  Whole backward with the dQ of
-// attn_hd64.hip / with it, us: 16 heads, L = 8192, causal 481 / 457, full 893 / 838, but 8 heads of it 304 / 310, 4 x 32 heads 3907 / 4016,
-// 32 heads, L = 2048 x 4, 275 / 292, L = 1000 x 4, 97 / 104: causal blocks that long and alone on their unit leave a tail.  With 32 queries the
-// fragment reads from LDS take as long as the products.
+// Tried and left: 64 rows per wavefront in the backward, one wavefront per SIMD, so that a fragment read from LDS serves two products.  It draws less
+// power and takes more cycles.  dQ (304 registers), whole backward with the dQ of attn_hd64.hip / with it, us: 16 heads, L = 8192, causal 481 / 457,
+// full 893 / 838, but 4 x 32 heads 3907 / 4016, 32 heads, L = 2048 x 4, 275 / 292.  dK / dV (396 registers), with the one below / with it: 491 / 468,
+// 920 / 887, but 3703 / 3732, 279 / 287, 8 heads of the first 308 / 342.
 #include <cfloat>
 #include <type_traits>
 #include "attn_rowtile.h"
@@ -619,6 +619,199 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_hd64_dkdv_pipe_kernel(const A
   }
 }
 
+//   S^T = K Q^T     dP^T = V dO^T - delta     dQ^T += K^T dS^T       lane = query column
+//
+// As above, 4 wavefronts of 32 queries, two per SIMD (194 registers).  Bound: power, at 1.7 GHz, and the vector pipe (exp, products with P and dP,
+// conversions: 416 cycles beside 384 of products per 32 x 32 sub-tile; takes 590), so addresses move once a tile and not with each read.
+// dQ alone, before (the same split without the order, three wavefronts per SIMD) / now, us: 16 heads, L = 8192, causal 212 / 194, full 417 / 370; 8 heads of it,
+// causal, 157 / 114; 4 x 32 heads of it 1629 / 1490; 16 heads, L = 4096, causal 83 / 61; on constant inputs, whose clock is not held down, full 348 / 255.
+constexpr int DQ_BM = 128, DQ_SLOTS = 4, DQ_STAGE = 2 * TILE;   // K and V tiles
+
+__global__ __launch_bounds__(256, 2) void attn_bwd_hd64_dq_pipe_kernel(const AttnParams p, const float* __restrict__ neg_delta) {
+  extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
+  bf16* ring = reinterpret_cast<bf16*>(smem);   // [DQ_SLOTS][K tile | V tile]
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, g = lane >> 5, i = lane & 31;
+  const BlockCoord bc = block_coord<2>(p.Hq, p.B, p.causal);
+  const int nqb = gridDim.x / (p.Hq * p.B);
+  const int qblk = p.causal ? nqb - 1 - bc.rank : bc.rank;   // heaviest blocks first
+  const int h = bc.h, b = bc.b, hk = h / p.group;
+  const int q0 = qblk * DQ_BM, wq0 = q0 + wave * 32, qi = wq0 + i;
+  const int n_end = p.causal ? min(p.Lk, min(q0 + DQ_BM, p.Lq) + p.off) : p.Lk;
+  // this block's tiles; the sub-tiles with a key that this wavefront sees, their tiles, and those of which all of its queries see all keys
+  const int total = max(0, n_end + ROWS - 1) / ROWS;
+  int w_subs = max(0, n_end + 31) / 32, w_full = p.Lk / ROWS;
+  if (p.causal) {
+    w_subs = min(w_subs, max(0, wq0 + 32 + p.off + 31) / 32);
+    w_full = min(w_full, max(0, wq0 + 1 + p.off) / ROWS);
+  }
+  const int w_total = (w_subs + 1) / 2;
+
+  bf16x8 qf[KS], dof[KS];
+  fetch_rows(qf, static_cast<const bf16*>(p.q) + b * p.sq.b + h * p.sq.h, p.sq.l, qi, p.Lq, g);
+  fetch_rows(dof, static_cast<const bf16*>(p.dout) + b * p.sdo.b + h * p.sdo.h, p.sdo.l, qi, p.Lq, g);
+  const int64_t head = (int64_t)b * p.Hq + h;
+  float lse2 = p.lse[head * p.Lq + min(qi, p.Lq - 1)];
+  float nd = neg_delta[head * p.Lq + min(qi, p.Lq - 1)];
+  f32x16 start;   // dP starts from -delta: one add less per element
+  const int lim = p.causal ? min(p.Lk - 1, qi + p.off) : p.Lk - 1;   // last key this lane's query sees
+  const float c2 = p.scale_log2e;
+
+  Bringer bk, bv;
+  bk.init(p.sk.l, wave, lane);
+  bv.init(p.sv.l, wave, lane);
+  int lt = 0;   // the tile being brought, the last one again where there are no more
+  const bf16* ktp = static_cast<const bf16*>(p.k) + b * p.sk.b + hk * p.sk.h;
+  const bf16* vtp = static_cast<const bf16*>(p.v) + b * p.sv.b + hk * p.sv.h;
+  auto load = [&](int part) INLINE {   // 0, 1: halves of K; 2, 3: of V
+    bf16* st = ring + (lt & (DQ_SLOTS - 1)) * DQ_STAGE;
+    const int rows = p.Lk - lt * ROWS;
+    if (part < 2) bk.load(st, ktp, rows, part, wave);
+    else bv.load(st + TILE, vtp, rows, part - 2, wave);
+  };
+  auto next = [&]() INLINE {
+    const int to = min(lt + 1, total - 1), step = to - lt;
+    lt = to;
+    ktp += (int64_t)step * (ROWS / 2 * bk.row_bytes);
+    vtp += (int64_t)step * (ROWS / 2 * bv.row_bytes);
+  };
+
+  f32x16 dq[DT], s[2], dp[2];   // of either sub-tile of a tile: S, then P; dP, then dS
+  clear(dq);
+  bf16x8 dsf[2];
+  Readers<D> rd;
+  rd.init(ring, g, i);
+  typedef const bf16x8 __attribute__((address_space(3))) * frag_ptr;
+  // from tile it's place in the ring to the next one's
+  auto onward = [&](int it) INLINE { return (it + 1) & (DQ_SLOTS - 1) ? DQ_STAGE * 2 : -(DQ_SLOTS - 1) * DQ_STAGE * 2; };
+  bf16x8 fr[2 * KS];   // K rows, k-step n; V rows, k-step n - 4
+  TrFrag tf[4];        // K^T, n = 2 ss + dt
+  auto read_row = [&](int n, int kt) INLINE {
+    fr[n] = *(frag_ptr)(uintptr_t)(rd.row[n & 3] + 2 * ((n >> 2) * ROWS + 32 * kt) * D);
+  };
+  auto read_col = [&](auto n_, auto kt_) INLINE {
+    constexpr int n = decltype(n_)::value, KT = decltype(kt_)::value;
+    read_tr<32 * KT + 16 * (n >> 1)>(tf[n], rd.tr[2 * (n & 1)], rd.tr[2 * (n & 1) + 1]);
+  };
+  // The vector work of a sub-tile in 24 steps of a product's length from the first product of its S on: element e becomes P in step
+  // 5 + 13 e / 16 (S is there from step 5 on) and dS in step 10 + 10 e / 16 (dP from step 10 on); the products of dQ are steps 20 to 23.
+  auto vector = [&](int step, int t, auto kt_, auto masked) INLINE {
+    constexpr int KT = decltype(kt_)::value;
+#pragma unroll
+    for (int e = 0; e < 16; e++) {
+      if (10 + 10 * e / 16 == step) {
+        dp[KT][e] *= s[KT][e];
+        if (e & 1) dsf[e >> 3][e & 7] = (bf16)dp[KT][e], dsf[e >> 3][(e & 7) - 1] = (bf16)dp[KT][e - 1];
+      }
+      if (5 + 13 * e / 16 == step) {
+        float x = fmaf(s[KT][e], c2, -lse2);
+        if (decltype(masked)::value) x = t * ROWS + 32 * KT + acc_row(e, g) > lim ? -INFINITY : x;
+        s[KT][e] = ody_exp2(x);
+      }
+    }
+  };
+
+  // One call: S and dP of the sub-tile after (tile it, sub-tile KT), then dQ of this one; under them the vector work of both.
+  auto unit = [&](int it, auto kt_, auto masked) INLINE {
+    constexpr int KT = decltype(kt_)::value, NKT = KT ^ 1;
+    const int nt = KT ? it + 1 : it;   // the sub-tile after; behind that, sub-tile KT of tile it + 1
+    std::integral_constant<int, NKT> nkt;
+#pragma unroll
+    for (int m = 0; m < 12; m++) {
+      if (m == 8) {
+        WAIT_LDS(4);
+#pragma unroll
+        for (int n = 0; n < 4; n++) tie(tf[n]);
+      }
+      if (m < 4) s[NKT] = mfma32(fr[m], qf[m], m == 0 ? f32x16{0} : s[NKT]);
+      else if (m < 8) dp[NKT] = mfma32(fr[m], dof[m - 4], m == 4 ? start : dp[NKT]);
+      else dq[m & 1] = mfma32(value(tf[m - 8]), dsf[(m - 8) >> 1], dq[m & 1]);
+      FENCE();
+      if (m == 0) read_col(std::integral_constant<int, 0>{}, kt_);
+      if (m == 1) read_col(std::integral_constant<int, 1>{}, kt_);
+      if (m == 2) read_col(std::integral_constant<int, 2>{}, kt_);
+      if (m == 3) read_col(std::integral_constant<int, 3>{}, kt_);
+      if (KT == 0 && m == 4) {
+        // the tile after this one has landed (behind it the 4 loads of the next); everyone is done with the one before this
+        asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        next();
+      }
+      if (m >= 4) read_row(m - 4, KT);
+      if (KT == 0 && (m == 6 || m == 9)) load(m == 9);
+      if (KT == 1 && (m == 1 || m == 5)) load(2 + (m == 5));
+      vector(12 + m, it, kt_, masked);
+      vector(m, nt, nkt, masked);
+      if (KT == 1 && m == 4)
+#pragma unroll
+        for (int n = 0; n < KS; n++) rd.tr[n] += onward(it);
+      if (KT == 1 && m == 11)
+#pragma unroll
+        for (int n = 0; n < KS; n++) rd.row[n] += onward(it + 1);
+      FENCE();
+    }
+  };
+  std::integral_constant<int, 0> c0;
+  std::integral_constant<int, 1> c1;
+
+  if (total > 0) {
+    auto all = [&]() INLINE {
+#pragma unroll
+      for (int n = 0; n < 4; n++) load(n);
+    };
+    all();
+    next();
+    all();
+    next();
+    all();
+    settle_rows(qf, qi, p.Lq);   // on their way in front of the tiles
+    settle_rows(dof, qi, p.Lq);
+    asm volatile("" : "+v"(lse2), "+v"(nd));
+    lse2 = qi >= p.Lq || lse2 == -INFINITY ? INFINITY : lse2 * ODY_LOG2E;   // past the end, or a query that saw no key: P = 0
+#pragma unroll
+    for (int r = 0; r < 16; r++) start[r] = nd;
+    asm volatile("s_waitcnt vmcnt(8)" ::: "memory");   // the first tile
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    int it = 0;
+    if (w_total > 0) {
+#pragma unroll
+      for (int n = 0; n < 8; n++) read_row(n, 0);
+#pragma unroll
+      for (int n = 0; n < 4; n++) {
+        s[0] = mfma32(fr[n], qf[n], n == 0 ? f32x16{0} : s[0]);
+        dp[0] = mfma32(fr[4 + n], dof[n], n == 0 ? start : dp[0]);
+      }
+#pragma unroll
+      for (int m = 0; m < 12; m++) vector(m, 0, c0, std::true_type{});
+#pragma unroll
+      for (int n = 0; n < 8; n++) read_row(n, 1);
+#pragma unroll
+      for (int n = 0; n < KS; n++) rd.row[n] += onward(0);   // the loop reads rows one tile ahead of columns
+      FENCE();
+      for (; it + 1 < min(w_total, w_full); it++) {
+        unit(it, c0, std::false_type{});
+        unit(it, c1, std::false_type{});
+      }
+      for (; it < w_total; it++) {   // (behind the last tile a sub-tile is formed that nobody uses)
+        unit(it, c0, std::true_type{});
+        if (2 * it + 1 < w_subs) unit(it, c1, std::true_type{});
+        else load(2), load(3);
+      }
+    }
+    // the other wavefronts' tiles: keep bringing this one's share of them
+    for (; it < total; it++) {
+      asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+      next();
+      all();
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  }
+  if (qi < p.Lq) store_dq(p, dq, b, h, qi, g);
+}
+
 }  // namespace
 
 int ody_launch_attn_fwd_hd64_pipe(const AttnParams& p, hipStream_t st) {
@@ -636,4 +829,12 @@ int ody_launch_attn_bwd_hd64_dkdv_pipe(const AttnParams& p, const float* neg_del
   const int64_t blocks = (int64_t)p.B * p.Hq * ((p.Lk + KV_BN - 1) / KV_BN);
   ODY_LAUNCH("attn_bwd_hd64_dkdv_pipe", st, kern, dim3((unsigned)blocks), dim3(256), smem, p, neg_delta, neg_lse, part);
   return ody_check_launch("attn_bwd_hd64_dkdv_pipe");
+}
+
+int ody_launch_attn_bwd_hd64_dq_pipe(const AttnParams& p, const float* neg_delta, hipStream_t st) {
+  constexpr size_t smem = (size_t)DQ_SLOTS * DQ_STAGE * sizeof(bf16);
+  if (int rc = ody_allow_dynamic_lds(reinterpret_cast<const void*>(&attn_bwd_hd64_dq_pipe_kernel), smem, "attn_bwd_hd64_dq_pipe")) return rc;
+  const int64_t blocks = (int64_t)p.B * p.Hq * ((p.Lq + DQ_BM - 1) / DQ_BM);
+  ODY_LAUNCH("attn_bwd_hd64_dq_pipe", st, attn_bwd_hd64_dq_pipe_kernel, dim3((unsigned)blocks), dim3(256), smem, p, neg_delta);
+  return ody_check_launch("attn_bwd_hd64_dq_pipe");
 }

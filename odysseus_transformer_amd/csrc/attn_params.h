@@ -107,6 +107,7 @@ int ody_launch_attn_fwd_hd64_pipe(const AttnParams& p, hipStream_t st);   // wit
 // from neg_delta, (B, Hq, Lq), and neg_lse = -lse / scale, (B, Hq, Lq rounded up to 64), minus infinity where P must be 0; part: fp32
 // [dK | dV][B][Hq][Lk][64], or null where every kv head has one query head
 int ody_launch_attn_bwd_hd64_dkdv_pipe(const AttnParams& p, const float* neg_delta, const float* neg_lse, float* part, hipStream_t st);
+int ody_launch_attn_bwd_hd64_dq_pipe(const AttnParams& p, const float* neg_delta, hipStream_t st);
 size_t ody_attn_bwd_hd64_workspace(int B, int Lq, int Lk, int Hq, int Hkv);
 int ody_launch_attn_bwd_hd64(const AttnParams& p, void* workspace, size_t workspace_bytes, hipStream_t st);
 // head_dim 128 where those two leave compute units idle.  Neither reads images; the forward uses no workspace (its callers still ask for that of

@@ -26,10 +26,13 @@ typedef __attribute__((address_space(1))) const void* global_ptr;
 // of 256 blocks with its ranks reversed: the three or four blocks that share a compute unit then add up to about the same
 // length.  In plain order the units with the first blocks of every run got 320 tiles where the mean was 260 (forward of 16 heads,
 // L = 8192: 182 us, 158 this way).
+// RUNS: so many runs of 256 are on the units from the start, and only among them ranks are reversed; what follows goes to whichever unit is done first,
+// longest first (0: all may share a unit).
+template <int RUNS = 0>
 __device__ __forceinline__ BlockCoord block_coord(int H, int B, int causal) {
   BlockCoord c = ody_block_coord(H, B);
   const int ranks = gridDim.x / (H * B), run = max(1, 256 / (H * B)), n = c.rank / run;
-  if (causal && (n & 1) && (n + 1) * run <= ranks) c.rank = n * run + run - 1 - c.rank % run;
+  if (causal && (n & 1) && (RUNS == 0 || n < RUNS) && (n + 1) * run <= ranks) c.rank = n * run + run - 1 - c.rank % run;
   return c;
 }
 
@@ -124,6 +127,22 @@ __device__ __forceinline__ void load_rows(bf16x8 (&f)[KS], const bf16* base, int
 #pragma unroll
   for (int ks = 0; ks < KS; ks++) asm volatile("" : "+v"(f[ks]));
 }
+// The same in two steps, with the loads of the first tiles between them: one latency in front of the loop instead of two.  (Without a branch
+// around the loads, at whose end the compiler waits.)
+template <int KS>
+__device__ __forceinline__ void fetch_rows(bf16x8 (&f)[KS], const bf16* base, int64_t stride, int row, int nrows, int g) {
+  const bf16* src = base + (int64_t)min(row, nrows - 1) * stride + 8 * g;
+#pragma unroll
+  for (int ks = 0; ks < KS; ks++) f[ks] = *reinterpret_cast<const bf16x8*>(src + 16 * ks);
+}
+template <int KS>
+__device__ __forceinline__ void settle_rows(bf16x8 (&f)[KS], int row, int nrows) {
+#pragma unroll
+  for (int ks = 0; ks < KS; ks++) asm volatile("" : "+v"(f[ks]));
+  if (row >= nrows)
+#pragma unroll
+    for (int ks = 0; ks < KS; ks++) f[ks] = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
+}
 
 template <int DT>
 __device__ __forceinline__ void clear(f32x16 (&x)[DT]) {
@@ -161,6 +180,40 @@ __device__ __forceinline__ void store_row(bf16* dst, const f32x16 (&x)[DT], floa
       for (int e = 0; e < 4; e++) w[e] = (bf16)(x[dt][4 * a + e] * scale);
       *reinterpret_cast<bf16x4*>(dst + 32 * dt + 8 * a + 4 * g) = w;
     }
+}
+
+// dQ^T of one query of a head of 64 (attn_store.h has that of 128) -> row qi of dq: scaled, then added to an fp32 or bf16 destination, or stored
+__device__ __forceinline__ void store_dq(const AttnParams& p, const f32x16 (&dq)[2], int b, int h, int qi, int g) {
+  const int64_t at = b * p.sdq.b + h * p.sdq.h + (int64_t)qi * p.sdq.l;
+  if (p.dq_f32) {   // the running dq of a ring step: exact accumulation over the key blocks
+    float* dst = static_cast<float*>(p.dq) + at;
+#pragma unroll
+    for (int dt = 0; dt < 2; dt++)
+#pragma unroll
+      for (int a = 0; a < 4; a++) {
+        f32x4* x = reinterpret_cast<f32x4*>(dst + 32 * dt + 8 * a + 4 * g);
+        f32x4 w = {0.f, 0.f, 0.f, 0.f};
+        if (p.accumulate_dq) w = *x;
+#pragma unroll
+        for (int e = 0; e < 4; e++) w[e] += dq[dt][4 * a + e] * p.scale;
+        *x = w;
+      }
+  } else if (p.accumulate_dq) {
+    bf16* dst = static_cast<bf16*>(p.dq) + at;
+#pragma unroll
+    for (int dt = 0; dt < 2; dt++)
+#pragma unroll
+      for (int a = 0; a < 4; a++) {
+        bf16x4* x = reinterpret_cast<bf16x4*>(dst + 32 * dt + 8 * a + 4 * g);
+        const bf16x4 old = *x;
+        bf16x4 w;
+#pragma unroll
+        for (int e = 0; e < 4; e++) w[e] = (bf16)(dq[dt][4 * a + e] * p.scale + (float)old[e]);
+        *x = w;
+      }
+  } else {
+    store_row(static_cast<bf16*>(p.dq) + at, dq, p.scale, g);
+  }
 }
 
 }  // namespace rowtile

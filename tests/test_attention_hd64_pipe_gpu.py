@@ -161,3 +161,41 @@ def test_large_values_behind_an_outgrown_reference(causal, dev):
     o_ref, lse_ref = oracle.attention_fwd(q[:, :, :2].float(), k[:, :, :2].float(), v[:, :, :2].float(), causal=causal)
     assert_parity(o[:, :, :2], o_ref, TOL_BF16, "o")
     assert torch.allclose(lse[:, :2].cpu(), lse_ref, atol=TOL_LSE, rtol=TOL_LSE)
+
+
+# blocks of 128 queries on either side of the lines of the dispatch; half and whole last sub-tiles and tiles, rings that wrap, wavefronts and blocks
+# without a key, queries past the end; every form of dq
+@pytest.mark.parametrize("form", ["new", "added", "fp32"])
+@pytest.mark.parametrize("Lq,Lk,Hq,Hkv,causal,pipe", [
+    (1, 1, 2, 1, True, True), (127, 31, 2, 2, False, True), (129, 33, 4, 2, True, True), (200, 96, 3, 3, True, True), (300, 257, 2, 1, False, True),
+    (257, 100, 2, 2, True, True), (500, 130, 1, 1, True, True), (161, 700, 2, 1, True, True), (128, 511, 512, 512, False, False),
+    (128, 512, 512, 256, False, True), (121, 999, 512, 512, True, False), (256, 1000, 256, 64, True, True)])
+def test_dq(Lq, Lk, Hq, Hkv, causal, pipe, form, dev):
+    from odysseus_transformer_amd import ops
+    print(f"{Lq=} {Lk=} {Hq=} {Hkv=} {causal=} {form=}", flush=True)
+    q, k, v, do = _inputs(1, Lq, Lk, Hq, Hkv, 101)
+    qg, kg, vg, dog = (t.to(dev) for t in (q, k, v, do))
+    o, lse = ops.attn_fwd(qg, kg, vg, causal=causal)
+    start = randn((1, Lq, Hq, 64), 105, dtype=torch.bfloat16)
+    dq = {"new": None, "added": start.to(dev), "fp32": start.float().to(dev)}[form]
+    (got, _, _), ran = _ran(lambda: ops.attn_bwd(qg, kg, vg, o, lse, dog, causal=causal, dq=dq, accumulate_dq=form != "new"))
+    assert ("attn_bwd_hd64_dq_pipe" in ran) == pipe, ran
+    n, G = min(2, Hkv), Hq // Hkv
+    ref = oracle.attention_bwd(q[:, :, :n * G].float(), k[:, :, :n].float(), v[:, :, :n].float(), o[:, :, :n * G].float().cpu(),
+                               lse[:, :n * G].cpu(), do[:, :, :n * G].float(), causal=causal)[0]
+    assert_parity(got[:, :, :n * G], ref + (0 if form == "new" else start[:, :, :n * G].float()), TOL_BF16, "dq", 1e-3)
+
+
+def test_keys_behind_a_sub_tile_of_the_mask_do_not_reach_dq(dev):
+    """Masked keys 32 and more behind a wavefront's last query are not read into its products, whatever they hold."""
+    from odysseus_transformer_amd import ops
+    L = 192
+    q, k, v, do = (t.to(dev) for t in _inputs(1, L, L, 2, 2, 111))
+    o, lse = ops.attn_fwd(q, k, v, causal=True)
+    (want, _, _), ran = _ran(lambda: ops.attn_bwd(q, k, v, o, lse, do, causal=True))
+    assert "attn_bwd_hd64_dq_pipe" in ran, ran
+    for last in (32, 64, 96, 128, 160):
+        bk, bv = k.clone(), v.clone()
+        bk[:, last:], bv[:, last:] = float("nan"), float("inf")
+        got = ops.attn_bwd(q, bk, bv, o, lse, do, causal=True)[0]
+        assert torch.equal(got[:, :last], want[:, :last]), last
