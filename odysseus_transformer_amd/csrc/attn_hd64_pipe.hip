@@ -363,11 +363,14 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_hd64_pipe_kernel(const AttnPa
 // ---------------------------------------------------------------------------------------------------------- backward
 //   S = Q K^T - lse / scale     dP = dO V^T - delta     dV^T += dO^T P     dK^T += Q^T (P o dP)      lane = key column
 //
-// 4 wavefronts of 32 keys, two per SIMD: 221 registers hold the sums of 32 keys, the next sub-tile's fragments and its S and dP; with 64 keys
+// 4 wavefronts of 32 keys, two per SIMD: 216 registers hold the sums of 32 keys, the next sub-tile's fragments and its S and dP; with 64 keys
 // they do not.  Bound: the reads from LDS and the matrix pipe alike (16 KB of fragments and 16 products per 32 x 32 sub-tile: 128 cycles of the
 // unit's LDS, of which four SIMDs want one each, and 512 of a SIMD's matrix pipe).
 // Whole backward before (the same split without the order) / now, us: 16 heads, L = 8192, causal 520 / 472, full 992 / 890; 8 heads of it,
-// causal, 386 / 308; 4 x 32 heads, L = 500, full, 57 / 52.  PART: fp32 sums of one query head to part [dK | dV][B][Hq][Lk][D]; otherwise every kv head has one.
+// causal, 386 / 308; 4 x 32 heads, L = 500, full, 57 / 52.  Of it this kernel, with every run of 256 causal blocks reversed, K and V waited for in front of
+// the first tiles' loads and an address formed with each read / as it is: 268 / 255, 491 / 483, 152 / 145; 64 heads, L = 512, full, 19.0 / 17.9; 80 heads,
+// L = 1000, causal, 39.7 / 36.5.  (With two blocks a unit the last of four runs reversed starts its longest blocks last.)
+// PART: fp32 sums of one query head to part [dK | dV][B][Hq][Lk][D]; otherwise every kv head has one.
 constexpr int KV_BN = 128, KV_SLOTS = 4;
 constexpr int KV_STAGE = 2 * TILE + 2 * 2 * ROWS;   // elements: Q and dO tiles, -lse / scale and -delta of their rows in fp32
 
@@ -377,7 +380,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_hd64_dkdv_pipe_kernel(const A
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
   bf16* ring = reinterpret_cast<bf16*>(smem);   // [KV_SLOTS][KV_STAGE]
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, g = lane >> 5, i = lane & 31;
-  const BlockCoord bc = block_coord(p.Hq, p.B, p.causal);   // rank 0 = first key block = most query tiles
+  const BlockCoord bc = block_coord<2>(p.Hq, p.B, p.causal);   // rank 0 = first key block = most query tiles
   const int b = bc.b, h = bc.h, hk = h / p.group;
   const int n0 = bc.rank * KV_BN, wn0 = n0 + wave * 32, key = wn0 + i;
   const int q_tiles = (p.Lq + ROWS - 1) / ROWS, t_top = q_tiles - 1;
@@ -390,8 +393,8 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_hd64_dkdv_pipe_kernel(const A
   }
 
   bf16x8 kf[KS], vf[KS];
-  load_rows(kf, static_cast<const bf16*>(p.k) + b * p.sk.b + hk * p.sk.h, p.sk.l, key, p.Lk, g);
-  load_rows(vf, static_cast<const bf16*>(p.v) + b * p.sv.b + hk * p.sv.h, p.sv.l, key, p.Lk, g);
+  fetch_rows(kf, static_cast<const bf16*>(p.k) + b * p.sk.b + hk * p.sk.h, p.sk.l, key, p.Lk, g);
+  fetch_rows(vf, static_cast<const bf16*>(p.v) + b * p.sv.b + hk * p.sv.h, p.sv.l, key, p.Lk, g);
   const float c2 = p.scale_log2e;
 
   Bringer bq, bo;
@@ -429,15 +432,16 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_hd64_dkdv_pipe_kernel(const A
   rd.init(ring, g, i);
   const int key_off = p.causal ? key - p.off : -(1 << 30);   // the first query that sees this lane's key
   typedef const bf16x8 __attribute__((address_space(3))) * frag_ptr;
-  auto slot = [&](int it) INLINE { return (unsigned)(it & (KV_SLOTS - 1)) * (KV_STAGE * 2); };
+  // from tile it's place in the ring to the next one's
+  auto onward = [&](int it) INLINE { return (it + 1) & (KV_SLOTS - 1) ? KV_STAGE * 2 : -(KV_SLOTS - 1) * KV_STAGE * 2; };
   bf16x8 fr[2 * KS];   // Q rows, k-step n; dO rows, k-step n - 4
   TrFrag tf[8];        // n = 2 (2 ss + dt) + which: dO^T (0) or Q^T (1)
-  auto read_row = [&](int n, unsigned st, int mt) INLINE {
-    fr[n] = *(frag_ptr)(uintptr_t)(rd.row[n & 3] + st + 2 * ((n >> 2) * ROWS + 32 * mt) * D);
+  auto read_row = [&](int n, int mt) INLINE {
+    fr[n] = *(frag_ptr)(uintptr_t)(rd.row[n & 3] + 2 * ((n >> 2) * ROWS + 32 * mt) * D);
   };
-  auto read_col = [&](int n, unsigned st, auto mt_) INLINE {
+  auto read_col = [&](int n, auto mt_) INLINE {
     constexpr int MT = decltype(mt_)::value;
-    const unsigned a0 = rd.tr[2 * ((n >> 1) & 1)] + st, a1 = rd.tr[2 * ((n >> 1) & 1) + 1] + st;
+    const unsigned a0 = rd.tr[2 * ((n >> 1) & 1)], a1 = rd.tr[2 * ((n >> 1) & 1) + 1];
     if (n < 4) {
       if (n & 1) read_tr<32 * MT>(tf[n], a0, a1);
       else read_tr<ROWS + 32 * MT>(tf[n], a0, a1);
@@ -477,7 +481,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_hd64_dkdv_pipe_kernel(const A
       else dp = mfma32(fr[m], vf[m - 4], dp);
       FENCE();
       if (m < 2) start_values(nt, NMT, 1, 2 * m, dp), start_values(nt, NMT, 1, 2 * m + 1, dp);
-      read_col(m, slot(it), mt_);
+      read_col(m, mt_);
       if (m >= 6) {
 #pragma unroll
         for (int e = 0; e < 4; e++) {
@@ -511,7 +515,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_hd64_dkdv_pipe_kernel(const A
         asm volatile("" ::: "memory");
         next();
       }
-      read_row(m, slot(it + 1), MT);
+      read_row(m, MT);
       if (m < 4) start_values(it + 1, MT, 0, m, s_start);
       if (m <= 2) {
 #pragma unroll
@@ -528,6 +532,12 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_hd64_dkdv_pipe_kernel(const A
       if (m >= 3 && m < 7) pack(dsf_next, dp, 2 * m - 6), pack(dsf_next, dp, 2 * m - 5);
       if (MT == 0 && m == 5) load(4);
       if (MT == 1 && (m == 2 || m == 5)) load(2 + (m == 5));
+      if (MT == 1 && m == 6)
+#pragma unroll
+        for (int n = 0; n < KS; n++) rd.tr[n] += onward(it);
+      if (MT == 1 && m == 7)
+#pragma unroll
+        for (int n = 0; n < KS; n++) rd.row[n] += onward(it + 1);
       FENCE();
     }
 #pragma unroll
@@ -547,6 +557,8 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_hd64_dkdv_pipe_kernel(const A
     all();
     next();
     all();
+    settle_rows(kf, key, p.Lk);   // on their way in front of the tiles
+    settle_rows(vf, key, p.Lk);
     asm volatile("s_waitcnt vmcnt(10)" ::: "memory");   // the first tile
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
@@ -558,7 +570,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_hd64_dkdv_pipe_kernel(const A
         start_values(0, 0, 1, a, dp);
       }
 #pragma unroll
-      for (int n = 0; n < 8; n++) read_row(n, slot(0), 0);
+      for (int n = 0; n < 8; n++) read_row(n, 0);
 #pragma unroll
       for (int n = 0; n < 4; n++) {
         s = mfma32(fr[n], kf[n], n == 0 ? s_start : s);
@@ -578,7 +590,9 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_hd64_dkdv_pipe_kernel(const A
 #pragma unroll
       for (int a = 0; a < 4; a++) start_values(0, 1, 0, a, s_start);
 #pragma unroll
-      for (int n = 0; n < 8; n++) read_row(n, slot(0), 1);
+      for (int n = 0; n < 8; n++) read_row(n, 1);
+#pragma unroll
+      for (int n = 0; n < KS; n++) rd.row[n] += onward(0);   // the loop reads rows one tile ahead of columns
       FENCE();
       for (; it + 1 < min(w_total, w_full); it++) {
         unit(it, c0, std::false_type{});
