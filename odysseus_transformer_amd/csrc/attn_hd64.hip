@@ -531,12 +531,24 @@ inline bool near(const AttnStrides& a, const AttnStrides& b) { return a.l < tile
 //   1 x 24 heads, L = 8192, 235 / 213, 16 heads, 512 blocks, 179 / 173 by itself and 5 us behind before a backward; 48 heads, L = 4096, 128 / 117,
 //   24 heads, 384 blocks, 76 / 79.
 // A last block that is half empty costs its share of the rows.
-inline bool fwd_pipe_ok(const AttnParams& p) {
-  const int64_t halves = (p.Lq + BLOCK_ROWS - 1) / BLOCK_ROWS, blocks = (int64_t)p.B * p.Hq * ((halves + 1) / 2);
-  if (!near(p.sk, p.sv) || ((halves & 1) && halves < 16)) return false;
+//
+// And with eight wavefronts a block, where that is one block for a unit, or causal, where two blocks to a unit from the start would leave the longer one
+// alone on it, and blocks that take a unit each, longest first, do not.  Best of the other two / this one, us:
+//   Full, more than one round of the former kernel's blocks and at most one of these: 4096 keys, 144 blocks, 70 / 60, 256 blocks 85 / 73, 1000 keys,
+//   144 blocks, 26.9 / 24.0, 768 keys, 255 blocks, 27.4 / 25.4; not with 128 blocks, for which the former one has a unit each, 84 / 108 (8192 keys), and with
+//   256 blocks not below 1024 keys: 700 22.3 / 23.1, 1000 27.4 / 27.6.
+//   Causal, from 512 blocks of the former kernel to 512 of these: L = 8192, 8 heads, 126 / 112, 16 heads, 160 / 145; L = 4096, 16 heads, 68 / 62, 32 heads, 87 / 82,
+//   L = 3000, 32 heads, 58 / 53; beyond, L = 8192, 18 heads, 176 / 179, L = 3000, 40 heads, 65.9 / 66.1, L = 2048, 48 heads, 43 / 45, or with a rectangle in front of the triangle, 3000
+//   queries on 4096 keys, 27 heads, 79 / 81.
+inline int fwd_pipe_groups(const AttnParams& p) {   // 0: not with 256-row blocks
+  const int64_t halves = (p.Lq + BLOCK_ROWS - 1) / BLOCK_ROWS, blocks = (int64_t)p.B * p.Hq * ((halves + 1) / 2), former = (int64_t)p.B * p.Hq * halves;
+  if (!near(p.sk, p.sv)) return 0;
+  if (p.causal ? former >= FEW_BLOCKS && blocks <= 512 && 8 * (int64_t)p.off <= p.Lk && p.Lk >= (blocks <= 384 ? 3000 : 4096)
+               : former > 256 && blocks <= 256 && p.Lk >= (former < FEW_BLOCKS ? 768 : 1024)) return 2;
+  if ((halves & 1) && halves < 16) return 0;
   if (p.causal) return blocks >= 768 && blocks * p.Lk >= (1 << 21);
-  const int64_t former = (int64_t)p.B * p.Hq * halves, rounds = (blocks + 255) / 256, lost = 2 * rounds - (former + 255) / 256;   // half rounds
-  if (former < FEW_BLOCKS || p.Lk < (rounds == 1 ? 640 : 512)) return false;
+  const int64_t rounds = (blocks + 255) / 256, lost = 2 * rounds - (former + 255) / 256;   // half rounds
+  if (former < FEW_BLOCKS || p.Lk < (rounds == 1 ? 640 : 512)) return 0;
   return lost == 0 || (lost == 1 && rounds > (p.Lk >= 2048 ? 2 : p.Lk >= 1024 ? 4 : 7));
 }
 
@@ -552,7 +564,7 @@ inline bool dq_pipe_ok(const AttnParams& p, int64_t blocks) {
 }  // namespace
 
 int ody_launch_attn_fwd_hd64(const AttnParams& p, hipStream_t st) {
-  if (fwd_pipe_ok(p)) return ody_launch_attn_fwd_hd64_pipe(p, st);
+  if (const int groups = fwd_pipe_groups(p)) return ody_launch_attn_fwd_hd64_pipe(p, groups, st);
   const int64_t blocks = row_blocks(p.B, p.Lq, p.Hq);
   return blocks < FEW_BLOCKS ? launch("attn_fwd_hd64", &attn_fwd_hd64_kernel<2>, blocks, 2, KV_STAGE, st, p)
                              : launch("attn_fwd_hd64", &attn_fwd_hd64_kernel<1>, blocks, 1, KV_STAGE, st, p);

@@ -58,25 +58,32 @@ __device__ __forceinline__ bf16x8 value(const TrFrag& f) {
 // share of it behind, two wavefronts per SIMD, and 64 queries each, so that a fragment read from LDS serves two products.  Before (32 queries,
 // three wavefronts per SIMD, attn_hd64.hip) / now, us: 16 heads, L = 8192, causal 179 / 173, full 308 / 265 (1037 TFLOP/s); 24 heads, causal,
 // 239 / 219; 4 x 32 heads on 8, causal, 1200 / 1067.
+//
+// GROUPS = 2: a second set of 4 wavefronts over the same rows, two per SIMD in one block, takes the later half of the tiles; their references, sums
+// and O meet in LDS at the end.  For calls with fewer blocks than units can hold two of: 16 heads, L = 8192, causal 160 / 145, L = 4096, full 85 / 73.
 constexpr int FW_QT = 2, FW_BM = 32 * FW_QT * 4, FW_SLOTS = 4;
 
-__global__ __launch_bounds__(256, 2) void attn_fwd_hd64_pipe_kernel(const AttnParams p) {
+template <int GROUPS>
+__global__ __launch_bounds__(256 * GROUPS, 2) void attn_fwd_hd64_pipe_kernel(const AttnParams p) {
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
-  bf16* kring = reinterpret_cast<bf16*>(smem);   // [FW_SLOTS][TILE]
-  bf16* vring = kring + FW_SLOTS * TILE;         // [FW_SLOTS][TILE]
-  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, g = lane >> 5, i = lane & 31;
-  const BlockCoord bc = block_coord(p.Hq, p.B, p.causal);
+  const int tid = threadIdx.x, wave8 = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, g = lane >> 5, i = lane & 31;
+  const int wave = wave8 & 3, grp = GROUPS == 1 ? 0 : wave8 >> 2;
+  bf16* kring = reinterpret_cast<bf16*>(smem) + grp * 2 * FW_SLOTS * TILE;   // [FW_SLOTS][TILE]
+  bf16* vring = kring + FW_SLOTS * TILE;                                     // [FW_SLOTS][TILE]
+  const BlockCoord bc = block_coord<GROUPS == 1 ? 0 : 1>(p.Hq, p.B, p.causal);
   const int nqb = gridDim.x / (p.Hq * p.B);
   const int qblk = p.causal ? nqb - 1 - bc.rank : bc.rank;   // heaviest blocks first
   const int h = bc.h, b = bc.b, hk = h / p.group;
   const int q0 = qblk * FW_BM, wq0 = q0 + wave * 32 * FW_QT;
 
   const int n_end = p.causal ? min(p.Lk, min(q0 + FW_BM, p.Lq) + p.off) : p.Lk;
-  const int ntiles = n_end > 0 ? (n_end + ROWS - 1) / ROWS : 0;
+  const int all_tiles = n_end > 0 ? (n_end + ROWS - 1) / ROWS : 0;
+  // this group's share of them: the second one's is not the shorter, for behind the diagonal some of it is left out
+  const int t_first = GROUPS == 1 || grp == 0 ? 0 : all_tiles / 2, ntiles = GROUPS == 1 || grp == 1 ? all_tiles : all_tiles / 2;
   // end of those tiles that this wavefront's queries see a key of, and of those that they see whole
   int w_end = ntiles, w_full = p.Lk / ROWS;
   if (p.causal) {
-    w_end = min(ntiles, max(0, wq0 + 32 * FW_QT - 1 + p.off + ROWS) / ROWS);
+    w_end = min(ntiles, max(t_first, max(0, wq0 + 32 * FW_QT - 1 + p.off + ROWS) / ROWS));
     w_full = min(w_full, max(0, wq0 + p.off + 1) / ROWS);
   }
 
@@ -85,8 +92,8 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_hd64_pipe_kernel(const AttnPa
   bv.init(p.sv.l, wave, lane);
   const bf16* kp = static_cast<const bf16*>(p.k) + b * p.sk.b + hk * p.sk.h;
   const bf16* vp = static_cast<const bf16*>(p.v) + b * p.sv.b + hk * p.sv.h;
-  int lk = 0, lv = 0;   // the tiles being brought, the last one again where there are no more
-  const bf16 *ktp = kp, *vtp = vp;
+  int lk = t_first, lv = t_first;   // the tiles being brought, the last one again where there are no more
+  const bf16 *ktp = kp + (int64_t)t_first * (ROWS / 2 * bk.row_bytes), *vtp = vp + (int64_t)t_first * (ROWS / 2 * bv.row_bytes);
   auto load_k = [&](int j) INLINE { bk.load(kring + (lk & (FW_SLOTS - 1)) * TILE, ktp, p.Lk - lk * ROWS, j, wave); };
   auto load_v = [&](int j) INLINE { bv.load(vring + (lv & (FW_SLOTS - 1)) * TILE, vtp, p.Lk - lv * ROWS, j, wave); };
   auto next_k = [&]() INLINE {
@@ -243,8 +250,8 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_hd64_pipe_kernel(const AttnPa
     half(c1);
   };
   clear_rows();
-  if (ntiles > 0) {
-    // K tiles 0 .. 3 and V tiles 0 .. 2, of the last ones a part: the loop brings the rest
+  if (t_first < ntiles) {
+    // K tiles t_first .. + 3 and V tiles .. + 2, of the last ones a part: the loop brings the rest
     load_k(0), load_k(1);
 #pragma unroll
     for (int a = 0; a < 3; a++) {
@@ -256,20 +263,20 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_hd64_pipe_kernel(const AttnPa
     asm volatile("s_waitcnt vmcnt(5)" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
-    int t = 0;
-    if (w_end > 0) {
-      scores(0);
+    int t = t_first;
+    if (w_end > t_first) {
+      scores(t);
 #pragma unroll
-      for (int qt = 0; qt < FW_QT; qt++) ref[qt] = fmaxf(ref[qt], largest(qt, 0));
+      for (int qt = 0; qt < FW_QT; qt++) ref[qt] = fmaxf(ref[qt], largest(qt, t));
 #pragma unroll
       for (int e = 16; e < 32; e++) {   // the last pair is left to be taken by the first turn
-        exponents(e, -1, std::true_type{});
+        exponents(e, t - 1, std::true_type{});
         x[0] = ody_exp2(y[0]), x[1] = ody_exp2(y[1]);
         if (e < 31) take(e);
       }
-      exponents(0, 0, std::true_type{});
+      exponents(0, t, std::true_type{});
 #pragma unroll
-      for (int n = 0; n < KS; n++) read_k(n, kslot(1), 0);
+      for (int n = 0; n < KS; n++) read_k(n, kslot(t + 1), 0);
       FENCE();
       for (; t + 1 < min(w_end, w_full); t++) turn(t, std::false_type{});
       for (; t + 1 < w_end; t++) turn(t, std::true_type{});
@@ -294,6 +301,7 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_hd64_pipe_kernel(const AttnPa
       load_k(0);
     }
   }
+  if (GROUPS == 2 && grp == 0 && (all_tiles & 1)) __builtin_amdgcn_s_barrier();   // the second group's one more
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();   // everyone is done with the rings
   {
@@ -311,16 +319,21 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_hd64_pipe_kernel(const AttnPa
       beyond |= !((zero[0] + zero[1]) + (zero[2] + zero[3]) == 0.f) || !(half_swap_sum(row_sum(qt)) < 0x1p100f);
     }
     const int mine = __builtin_amdgcn_ballot_w64(beyond) != 0;
-    if (lane == 0) flags[wave] = mine;
+    if (lane == 0) flags[wave8] = mine;
     __syncthreads();
-    const int any = flags[0] | flags[1] | flags[2] | flags[3];
+    int any = 0;
+#pragma unroll
+    for (int w = 0; w < 4 * GROUPS; w++) any |= flags[w];
     __syncthreads();
     if (any) {
       clear_rows();
-      for (int t = 0; t < ntiles; t++) {
-        lk = lv = t;
-        ktp = kp + (int64_t)t * ROWS * p.sk.l, vtp = vp + (int64_t)t * ROWS * p.sv.l;
-        load_k(0), load_k(1), load_v(0), load_v(1);
+      for (int n = 0; n < (GROUPS == 1 ? all_tiles : (all_tiles + 1) / 2); n++) {
+        const int t = t_first + n;
+        if (t < ntiles) {
+          lk = lv = t;
+          ktp = kp + (int64_t)t * ROWS * p.sk.l, vtp = vp + (int64_t)t * ROWS * p.sv.l;
+          load_k(0), load_k(1), load_v(0), load_v(1);
+        }
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
         if (t < w_end) {
@@ -349,14 +362,39 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_hd64_pipe_kernel(const AttnPa
     }
   }
 
-#pragma unroll
-  for (int qt = 0; qt < FW_QT; qt++) {
+  auto store = [&](int qt, float l) INLINE {
     const int qi = wq0 + 32 * qt + i;
-    const float l = half_swap_sum(row_sum(qt));
-    if (qi >= p.Lq) continue;
+    l = half_swap_sum(l);
+    if (qi >= p.Lq) return;
     const float inv = l > 0.f ? 1.f / l : 0.f;
     store_row(static_cast<bf16*>(p.out) + b * p.so.b + h * p.so.h + (int64_t)qi * p.so.l, o[qt], inv, g);
     if (g == 0) p.lse[((int64_t)b * p.Hq + h) * p.Lq + qi] = l > 0.f ? (ref[qt] + __log2f(l)) * ODY_LN2 : -INFINITY;
+  };
+  if constexpr (GROUPS == 1) {
+#pragma unroll
+    for (int qt = 0; qt < FW_QT; qt++) store(qt, row_sum(qt));
+  } else {
+    // a group hands half of its queries' sums to the other one and finishes the other half
+    static_assert(FW_QT == 2 && 2 * 4 * (16 * DT + 2) * 64 * sizeof(float) <= 2 * 2 * FW_SLOTS * TILE * sizeof(bf16), "in the rings");
+    float* patches = reinterpret_cast<float*>(smem);
+    auto give_half = [&](int qt) INLINE {
+      float* patch = patches + (4 * qt + wave) * (16 * DT + 2) * 64;
+      give(patch, o[qt], lane);
+      patch[16 * DT * 64 + lane] = ref[qt];
+      patch[(16 * DT + 1) * 64 + lane] = row_sum(qt);
+    };
+    auto finish = [&](int qt) INLINE {
+      const float* patch = patches + (4 * qt + wave) * (16 * DT + 2) * 64;
+      const float ref1 = patch[16 * DT * 64 + lane], next = fmaxf(ref[qt], ref1), a0 = ody_exp2(ref[qt] - next), a1 = ody_exp2(ref1 - next);
+      rowtile::take(patch, o[qt], lane, a0, a1);
+      ref[qt] = next;
+      store(qt, row_sum(qt) * a0 + patch[(16 * DT + 1) * 64 + lane] * a1);
+    };
+    if (grp == 0) give_half(1);
+    else give_half(0);
+    __syncthreads();
+    if (grp == 0) finish(0);
+    else finish(1);
   }
 }
 
@@ -828,11 +866,13 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_hd64_dq_pipe_kernel(const Att
 
 }  // namespace
 
-int ody_launch_attn_fwd_hd64_pipe(const AttnParams& p, hipStream_t st) {
-  constexpr size_t smem = (size_t)2 * FW_SLOTS * TILE * sizeof(bf16);
-  if (int rc = ody_allow_dynamic_lds(reinterpret_cast<const void*>(&attn_fwd_hd64_pipe_kernel), smem, "attn_fwd_hd64_pipe")) return rc;
+int ody_launch_attn_fwd_hd64_pipe(const AttnParams& p, int groups, hipStream_t st) {
+  const size_t smem = (size_t)groups * 2 * FW_SLOTS * TILE * sizeof(bf16);
+  auto kern = groups == 2 ? &attn_fwd_hd64_pipe_kernel<2> : &attn_fwd_hd64_pipe_kernel<1>;
+  if (int rc = ody_allow_dynamic_lds(reinterpret_cast<const void*>(kern), smem, "attn_fwd_hd64_pipe")) return rc;
   const int64_t blocks = (int64_t)p.B * p.Hq * ((p.Lq + FW_BM - 1) / FW_BM);
-  ODY_LAUNCH("attn_fwd_hd64_pipe", st, attn_fwd_hd64_pipe_kernel, dim3((unsigned)blocks), dim3(256), smem, p);
+  const char* name = groups == 2 ? "attn_fwd_hd64_pipe2" : "attn_fwd_hd64_pipe";
+  ODY_LAUNCH(name, st, kern, dim3((unsigned)blocks), dim3(256 * groups), smem, p);
   return ody_check_launch("attn_fwd_hd64_pipe");
 }
 

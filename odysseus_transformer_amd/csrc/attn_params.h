@@ -103,7 +103,7 @@ int ody_launch_attn_bwd_pipe(const AttnParams& p, void* workspace, hipStream_t s
 // head_dim 64, bf16, no dropout; the forward needs no workspace, the backward room for its row values, which take the place of
 // p.delta.  With ody_attn_bwd_hd64_workspace(...) bytes it can take the query heads of a group apart; with less it does not.
 int ody_launch_attn_fwd_hd64(const AttnParams& p, hipStream_t st);
-int ody_launch_attn_fwd_hd64_pipe(const AttnParams& p, hipStream_t st);   // with blocks enough for the whole chip
+int ody_launch_attn_fwd_hd64_pipe(const AttnParams& p, int groups, hipStream_t st);   // groups of 4 wavefronts in a block of 256 rows
 // from neg_delta, (B, Hq, Lq), and neg_lse = -lse / scale, (B, Hq, Lq rounded up to 64), minus infinity where P must be 0; part: fp32
 // [dK | dV][B][Hq][Lk][64], or null where every kv head has one query head
 int ody_launch_attn_bwd_hd64_dkdv_pipe(const AttnParams& p, const float* neg_delta, const float* neg_lse, float* part, hipStream_t st);

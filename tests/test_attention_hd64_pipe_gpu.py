@@ -199,3 +199,41 @@ def test_keys_behind_a_sub_tile_of_the_mask_do_not_reach_dq(dev):
         bk[:, last:], bv[:, last:] = float("nan"), float("inf")
         got = ops.attn_bwd(q, bk, bv, o, lse, do, causal=True)[0]
         assert torch.equal(got[:, :last], want[:, :last]), last
+
+
+# forward with eight wavefronts a block: odd counts of tiles, ragged last ones, blocks of 0, 1 and 2 tiles (fewer keys than queries), queries past the end,
+# references that a later half outgrows, and the lines of its dispatch (two: 2 on it, 0 and 1 as before)
+@pytest.mark.parametrize("stretch", [1.0, 60.0], ids=["unit", "moving_reference"])
+@pytest.mark.parametrize("Lq,Lk,Hq,Hkv,causal,two", [
+    (512, 768, 65, 13, False, True), (505, 831, 127, 127, False, True), (2049, 1024, 28, 14, False, True), (512, 767, 65, 65, False, False),
+    (512, 1023, 128, 32, False, False), (256, 2048, 128, 128, False, False), (4096, 4096, 32, 8, True, True), (3000, 3000, 22, 22, True, True),
+    (6401, 4001, 14, 14, True, True), (8192, 3969, 8, 4, True, True), (4096, 4096, 33, 33, True, False), (3000, 2999, 22, 22, True, False),
+    (3000, 4096, 24, 24, True, False)])
+def test_forward_in_two_groups(Lq, Lk, Hq, Hkv, causal, two, stretch, dev):
+    from odysseus_transformer_amd import ops
+    print(f"{Lq=} {Lk=} {Hq=} {Hkv=} {causal=} {stretch=}", flush=True)
+    q, k, v, _ = _inputs(1, Lq, Lk, Hq, Hkv, 121)
+    k = (k.float() * torch.linspace(1.0, stretch, Lk)[None, :, None, None]).bfloat16()
+    (o, lse), ran = _ran(lambda: ops.attn_fwd(q.to(dev), k.to(dev), v.to(dev), causal=causal))
+    assert ("attn_fwd_hd64_pipe2" in ran) == two, ran
+    G = Hq // Hkv
+    o_ref, lse_ref = oracle.attention_fwd(q[:, :, :G].float(), k[:, :, :1].float(), v[:, :, :1].float(), causal=causal)
+    assert_parity(o[:, :, :G], o_ref, TOL_BF16, "o")
+    assert torch.allclose(lse[:, :G].cpu(), lse_ref, atol=TOL_LSE, rtol=TOL_LSE)
+
+
+@pytest.mark.parametrize("causal", [False, True], ids=["full", "causal"])
+def test_large_values_in_two_groups(causal, dev):
+    """Keys 56 above the first ones from a quarter in front of the end on, |v| around 2^48: in the second group's tiles, whose reference is among the low ones."""
+    from odysseus_transformer_amd import ops
+    L, H = (4096, 16) if causal else (1536, 40)
+    q, k, v, _ = _inputs(1, L, L, H, H, 131)
+    q[..., 0], k[..., 0] = 8.0, 0.0
+    k[:, -(L // 4):, :, 0] = 56.0
+    v = (v.float() * 2.0 ** 48).bfloat16()
+    (o, lse), ran = _ran(lambda: ops.attn_fwd(q.to(dev), k.to(dev), v.to(dev), causal=causal))
+    assert "attn_fwd_hd64_pipe2" in ran, ran
+    assert bool(o.isfinite().all())
+    o_ref, lse_ref = oracle.attention_fwd(q[:, :, :2].float(), k[:, :, :2].float(), v[:, :, :2].float(), causal=causal)
+    assert_parity(o[:, :, :2], o_ref, TOL_BF16, "o")
+    assert torch.allclose(lse[:, :2].cpu(), lse_ref, atol=TOL_LSE, rtol=TOL_LSE)
