@@ -871,8 +871,7 @@ int ody_launch_attn_fwd_hd64_pipe(const AttnParams& p, int groups, hipStream_t s
   auto kern = groups == 2 ? &attn_fwd_hd64_pipe_kernel<2> : &attn_fwd_hd64_pipe_kernel<1>;
   if (int rc = ody_allow_dynamic_lds(reinterpret_cast<const void*>(kern), smem, "attn_fwd_hd64_pipe")) return rc;
   const int64_t blocks = (int64_t)p.B * p.Hq * ((p.Lq + FW_BM - 1) / FW_BM);
-  const char* name = groups == 2 ? "attn_fwd_hd64_pipe2" : "attn_fwd_hd64_pipe";
-  ODY_LAUNCH(name, st, kern, dim3((unsigned)blocks), dim3(256 * groups), smem, p);
+  ODY_LAUNCH("attn_fwd_hd64_pipe", st, kern, dim3((unsigned)blocks), dim3(256 * groups), smem, p);
   return ody_check_launch("attn_fwd_hd64_pipe");
 }
 

@@ -202,20 +202,20 @@ def test_keys_behind_a_sub_tile_of_the_mask_do_not_reach_dq(dev):
 
 
 # forward with eight wavefronts a block: odd counts of tiles, ragged last ones, blocks of 0, 1 and 2 tiles (fewer keys than queries), queries past the end,
-# references that a later half outgrows, and the lines of its dispatch (two: 2 on it, 0 and 1 as before)
+# references that a later half outgrows, and the lines of its dispatch (pipe: the kernel with 256-row blocks, with one group of wavefronts or two)
 @pytest.mark.parametrize("stretch", [1.0, 60.0], ids=["unit", "moving_reference"])
-@pytest.mark.parametrize("Lq,Lk,Hq,Hkv,causal,two", [
+@pytest.mark.parametrize("Lq,Lk,Hq,Hkv,causal,pipe", [
     (512, 768, 65, 13, False, True), (505, 831, 127, 127, False, True), (2049, 1024, 28, 14, False, True), (512, 767, 65, 65, False, False),
-    (512, 1023, 128, 32, False, False), (256, 2048, 128, 128, False, False), (4096, 4096, 32, 8, True, True), (3000, 3000, 22, 22, True, True),
+    (512, 1023, 128, 32, False, True), (256, 2048, 128, 128, False, False), (4096, 4096, 32, 8, True, True), (3000, 3000, 22, 22, True, True),
     (6401, 4001, 14, 14, True, True), (8192, 3969, 8, 4, True, True), (4096, 4096, 33, 33, True, False), (3000, 2999, 22, 22, True, False),
     (3000, 4096, 24, 24, True, False)])
-def test_forward_in_two_groups(Lq, Lk, Hq, Hkv, causal, two, stretch, dev):
+def test_forward_in_two_groups(Lq, Lk, Hq, Hkv, causal, pipe, stretch, dev):
     from odysseus_transformer_amd import ops
     print(f"{Lq=} {Lk=} {Hq=} {Hkv=} {causal=} {stretch=}", flush=True)
     q, k, v, _ = _inputs(1, Lq, Lk, Hq, Hkv, 121)
     k = (k.float() * torch.linspace(1.0, stretch, Lk)[None, :, None, None]).bfloat16()
     (o, lse), ran = _ran(lambda: ops.attn_fwd(q.to(dev), k.to(dev), v.to(dev), causal=causal))
-    assert ("attn_fwd_hd64_pipe2" in ran) == two, ran
+    assert (FWD in ran) == pipe, ran
     G = Hq // Hkv
     o_ref, lse_ref = oracle.attention_fwd(q[:, :, :G].float(), k[:, :, :1].float(), v[:, :, :1].float(), causal=causal)
     assert_parity(o[:, :, :G], o_ref, TOL_BF16, "o")
@@ -232,7 +232,7 @@ def test_large_values_in_two_groups(causal, dev):
     k[:, -(L // 4):, :, 0] = 56.0
     v = (v.float() * 2.0 ** 48).bfloat16()
     (o, lse), ran = _ran(lambda: ops.attn_fwd(q.to(dev), k.to(dev), v.to(dev), causal=causal))
-    assert "attn_fwd_hd64_pipe2" in ran, ran
+    assert FWD in ran, ran
     assert bool(o.isfinite().all())
     o_ref, lse_ref = oracle.attention_fwd(q[:, :, :2].float(), k[:, :, :2].float(), v[:, :, :2].float(), causal=causal)
     assert_parity(o[:, :, :2], o_ref, TOL_BF16, "o")
