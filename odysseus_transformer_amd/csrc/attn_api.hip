@@ -88,7 +88,7 @@ int attn_fwd_impl(const char* who, const void* q, const void* k, const void* v, 
                 workspace_bytes, need);
     ODY_REQUIRE((reinterpret_cast<uintptr_t>(workspace) & 255u) == 0, ODY_ERR_MISALIGNED,
                 "%s: workspace must be 256-byte aligned", who);
-    if (ody_attn_fwd_short_ok(B, Lq, Lk, Hq, p.causal)) return ody_launch_attn_fwd_short(p, st);
+    if (ody_attn_fwd_short_ok(p)) return ody_launch_attn_fwd_short(p, st);
     return ody_launch_attn_fwd_pipe(p, workspace, workspace_bytes, st);
   }
   if (dtype == ODY_BF16 && p.drop_thresh == 0) return ody_launch_attn_fwd_hd64(p, st);

@@ -113,7 +113,7 @@ int ody_launch_attn_bwd_hd64(const AttnParams& p, void* workspace, size_t worksp
 // head_dim 128 where those two leave compute units idle.  Neither reads images; the forward uses no workspace (its callers still ask for that of
 // the kernel above).  The backward runs behind the pre-pass, which writes the images of Q and dO all the same, for a later call that reuses the query
 // side; it reads p.delta and the start values, and leaves fp32 dK / dV of every query head in `part` if Hq != Hkv.
-bool ody_attn_fwd_short_ok(int B, int Lq, int Lk, int Hq, int causal);
+bool ody_attn_fwd_short_ok(const AttnParams& p);
 bool ody_attn_bwd_short_ok(int B, int Lq, int Lk, int Hq, int causal);
 int ody_launch_attn_fwd_short(const AttnParams& p, hipStream_t st);
 int ody_launch_attn_bwd_short(const AttnParams& p, const void* stats, float* part, hipStream_t st);

@@ -8,9 +8,12 @@
 // (attn_rowtile.h), at half the LDS rate but without images: no pass that writes those of K and V (those of Q and dO come with the pre-pass, for later
 // calls that reuse the query side).  All of the backward behind the pre-pass is one launch.
 //
-// What bounds it: latency of a chain of tiles in a block (about 2.5 us for 128 rows against 128 keys in the forward) on 1 block a unit.
+// The forward on more than a few tiles (the ring) takes a sub-tile of 32 keys of every tile per group instead, in the order of attn_fwd_pipe.hip: products,
+// LDS reads and vector work of neighbouring sub-tiles under one another, loads four tiles ahead.
+//
+// What bounds it: latency of a chain of tiles in a block (2.2 us for 128 rows against 128 keys in the forward, 1.5 in the ring) on 1 block a unit.
 // Before / here, us, launches included: forward of 4 x 8 heads, L = 331, causal 19.8 / 12.7 (three launches / one), backward on 2 kv heads
-// 62.2 / 33.6 (five / three); 32 heads on 8, L = 1000, causal 41.5 / 24.4 and 119 / 74; 8 heads, L = 1500, full 43 / 31 and 148 / 68.
+// 62.2 / 33.6 (five / three); 32 heads on 8, L = 1000, causal 41.5 / 20.4 and 119 / 74; 8 heads, L = 1500, full 43 / 23 and 148 / 68.
 // Error against 64 bits, standard normal inputs, before / here: out 2.07e-3 / 1.96e-3 (4 x 8 heads, L = 331), 2.34e-3 / 2.31e-3 (640 rows,
 // full); dQ, dK, dV the same within the spread of one input to the next (2.5e-3, 2.5e-3, 2.3e-3).
 #include <algorithm>
@@ -31,6 +34,35 @@ constexpr size_t QS_STAGE = 2 * TILE + 512;              // Q and dO tiles, star
 constexpr size_t SMEM = GROUPS * 2 * KV_STAGE * sizeof(bf16);
 static_assert(SMEM >= 4 * (16 * DT + 2) * 64 * sizeof(float) && SMEM >= 2 * QS_STAGE * sizeof(bf16) && SMEM <= 160 * 1024, "one block per unit");
 typedef TileLoader<D, 4> GroupLoader;
+constexpr int FW_STAGE = 2 * TILE;   // elements: K and V of a tile of the forward's ring of 4
+static_assert(4 * FW_STAGE * sizeof(bf16) <= SMEM, "the ring");
+#define FENCE() __builtin_amdgcn_sched_barrier(0)
+#define INLINE __attribute__((always_inline))
+#define WAIT_LDS(n) asm volatile("s_waitcnt lgkmcnt(" #n ")" ::: "memory")
+
+// A transposed fragment (tr_frags) whose reads are still under way: 16 rows from FIRST on, 32 columns by the address pair
+struct TrFrag {
+  s16x4 lo, hi;
+};
+template <int FIRST>
+__device__ __forceinline__ void read_tr(TrFrag& f, unsigned a0, unsigned a1) {
+  asm volatile("ds_read_b64_tr_b16 %0, %2 offset:%4\n\tds_read_b64_tr_b16 %1, %3 offset:%5"
+               : "=&v"(f.lo), "=&v"(f.hi)
+               : "v"(a0), "v"(a1), "n"(2 * FIRST * D), "n"(2 * (FIRST + 8) * D));
+}
+// behind the wait for them
+__device__ __forceinline__ void tie(TrFrag& f) { asm volatile("" : "+v"(f.lo), "+v"(f.hi)); }
+__device__ __forceinline__ bf16x8 value(const TrFrag& f) {
+  return concat4(__builtin_bit_cast(bf16x4, f.lo), __builtin_bit_cast(bf16x4, f.hi));
+}
+template <typename F, int... N>
+__device__ __forceinline__ void each_of(const F& f, std::integer_sequence<int, N...>) {
+  (f(std::integral_constant<int, N>{}), ...);
+}
+template <int COUNT, typename F>
+__device__ __forceinline__ void each(const F& f) {
+  each_of(f, std::make_integer_sequence<int, COUNT>{});
+}
 
 // ---------------------------------------------------------------------------------------------------------- forward
 //   S^T = K Q^T      O^T += V^T P^T       lane = query column
@@ -161,6 +193,287 @@ __global__ __launch_bounds__(64 * WAVES, 2) void attn_fwd_short_kernel(const Att
     for (int w = 0; w < 4 * GROUPS; w++) any |= flags[w];
     __syncthreads();
     if (any) walk(std::true_type{});
+  }
+
+  float l = (l4[0] + l4[1]) + (l4[2] + l4[3]);
+#pragma unroll 1
+  for (int from = 1; from < GROUPS; from++) {
+    float* patch = reinterpret_cast<float*>(smem) + w4 * (16 * DT + 2) * 64;
+    if (grp == from) {
+      give(patch, o, lane);
+      patch[16 * DT * 64 + lane] = ref;
+      patch[(16 * DT + 1) * 64 + lane] = l;
+    }
+    __syncthreads();
+    if (grp == 0) {
+      const float ref1 = patch[16 * DT * 64 + lane], next = fmaxf(ref, ref1), a0 = ody_exp2(ref - next), a1 = ody_exp2(ref1 - next);
+      take(patch, o, lane, a0, a1);
+      l = l * a0 + patch[(16 * DT + 1) * 64 + lane] * a1;
+      ref = next;
+    }
+    __syncthreads();
+  }
+  if (grp != 0) return;
+  l = half_swap_sum(l);
+  if (qi < p.Lq) {
+    const float inv = l > 0.f ? 1.f / l : 0.f;
+    store_row(static_cast<bf16*>(p.out) + b * p.so.b + h * p.so.h + (int64_t)qi * p.so.l, o, inv, g);
+    if (g == 0) p.lse[((int64_t)b * p.Hq + h) * p.Lq + qi] = l > 0.f ? (ref + __log2f(l)) * ODY_LN2 : -INFINITY;
+  }
+}
+
+// The same on more than a few tiles: a wavefront has one sub-tile of every tile of a ring of four, and forms S of the tile after (8 products) and P V of
+// the present one (8), each product with one element of P and one or two LDS reads behind it; K rows are read half a turn ahead, V columns a quarter.
+// Bound: the vector pipe and the reads from LDS beside the products, 1600 cycles a tile of 1024 of products, and the clock.  Before (products, vector
+// work and the waits of the transposing reads one after the other, as above) / now, us, launch included: L = 1000, causal, 32 heads, 22.7 / 20.4,
+// 16 heads 22.1 / 18.8; L = 2048, 8 heads, 36.8 / 28.4; L = 4096, 8 heads, against attn_fwd_pipe.hip's, 66 / 50.  Its fixed cost is 0.5 us more (a first
+// pass through more code, two latencies in front of the loop): short rows are left to the loop above.
+__global__ __launch_bounds__(64 * WAVES, 2) void attn_fwd_short_ring_kernel(const AttnParams p) {
+  extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, g = lane >> 5, i = lane & 31;
+  const int grp = wave >> 2, w4 = wave & 3;
+  const BlockCoord bc = ody_block_coord(p.Hq, p.B);
+  const int nqb = gridDim.x / (p.Hq * p.B);
+  const int qblk = p.causal ? nqb - 1 - bc.rank : bc.rank;   // heaviest blocks first
+  const int h = bc.h, b = bc.b, hk = h / p.group;
+  const int q0 = qblk * BLOCK_ROWS, wq0 = q0 + w4 * 32, qi = wq0 + i;
+
+  int n_end = p.causal ? min(p.Lk, min(q0 + BLOCK_ROWS, p.Lq) + p.off) : p.Lk;
+  const int ntiles = n_end > 0 ? (n_end + ROWS - 1) / ROWS : 0;
+  const bf16* kp = static_cast<const bf16*>(p.k) + b * p.sk.b + hk * p.sk.h;
+  const bf16* vp = static_cast<const bf16*>(p.v) + b * p.sv.b + hk * p.sv.h;
+  const int lim = p.causal ? min(p.Lk - 1, qi + p.off) : p.Lk - 1;   // last key this lane's query sees
+  const float c2 = p.scale_log2e;
+  bf16x8 qf[KS];
+  f32x16 o[DT];
+  float ref;     // the row's reference in log2 units
+  float l4[4];   // this lane's partial row sums
+
+  // The direct loads of a tile: halves of K (0, 1) and of V (2, 3), one instruction per wavefront each.  Rows past the end read zeros, and a tile past
+  // the end nothing else: its loads are there to be counted.
+  bf16* fring = reinterpret_cast<bf16*>(smem);   // [4][K tile | V tile]
+  const int brow = 4 * wave + (lane >> 4), bcol = 16 * ((lane & 15) ^ swz<D>(brow)), krow = 2 * (int)p.sk.l, vrow = 2 * (int)p.sv.l;
+  const int koff = brow * krow + bcol, voff = brow * vrow + bcol;
+  auto load = [&](int t, int part) INLINE {
+    const int rows = min(p.Lk - t * ROWS, ROWS), row = part < 2 ? krow : vrow;
+    const bf16* src = (part < 2 ? kp : vp) + (int64_t)(t * ROWS) * (row / 2);
+    auto rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16*>(src), (short)0, t < ntiles ? (rows - 1) * row + 2 * D : 0, 0x00020000);
+    bf16* dst = fring + (t & 3) * FW_STAGE + (part < 2 ? 0 : TILE) + (8 * (part & 1) + wave) * 512;
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_ptr)dst, 16, (part < 2 ? koff : voff) + 32 * (part & 1) * row, 0, 0, 0);
+  };
+  // K of tile 0 and the queries first: what the first products wait for is not behind four tiles
+  load(0, 0), load(0, 1);
+  FENCE();
+  fetch_rows(qf, static_cast<const bf16*>(p.q) + b * p.sq.b + h * p.sq.h, p.sq.l, qi, p.Lq, g);
+  FENCE();
+#pragma unroll
+  for (int t = 0; t < 4; t++) {
+    if (t < 3) load(t + 1, 0), load(t + 1, 1);
+    load(t, 2), load(t, 3);
+  }
+  settle_rows(qf, qi, p.Lq);
+  // The reference of a row and a group is the largest score of its first two sub-tiles (a row that sees any key of the group's sees their first one) and
+  // stays.  Of the first one alone it would do, but the further below a row's maximum it is, the coarser bf16 is where the large P lie (out of 32 heads,
+  // L = 1000, 2.053e-3 from 64 bits, 2.033e-3 as in the loop above).  Sub-tile `grp` of every tile is this group's.
+  const int sub_end = min(n_end, p.causal ? wq0 + 32 + p.off : n_end) - 32 * grp, sub_full = min(p.Lk, p.causal ? wq0 + 1 + p.off : p.Lk) - 32 * grp - 32;
+  const int w_live = sub_end > 0 ? (sub_end + ROWS - 1) / ROWS : 0;   // sub-tiles with a key that this wavefront sees
+  const int w_full = sub_full >= 0 ? sub_full / ROWS + 1 : 0;         // those of which all of its queries see all keys
+  const int seen = lim - 32 * grp - 4 * g;   // last key this lane's query sees, from this lane's first one in tile 0 on
+  f32x16 s[2];                       // of even and odd tiles
+  bf16x8 pb[2][2], kfr[KS];          // P, alike; K rows: k-step n
+  TrFrag vfr[2 * DT];                // V^T: 16 keys n / DT, columns 32 (n % DT)
+  Readers<D> rd;
+  rd.init(fring, g, i);
+#pragma unroll
+  for (int n = 0; n < KS; n++) rd.row[n] += 2 * 32 * D * grp, rd.tr[n] += 2 * 32 * D * grp;
+  typedef const bf16x8 __attribute__((address_space(3))) * frag_ptr;
+  // ODD: of the two tiles that the readers' place in the ring has
+  auto read_k = [&](int n, int odd) INLINE { kfr[n] = *(frag_ptr)(uintptr_t)(rd.row[n] + odd * FW_STAGE * 2); };
+  auto read_v = [&](auto n_, auto odd_) INLINE {
+    constexpr int n = decltype(n_)::value, FIRST = decltype(odd_)::value * 2 * ROWS + ROWS + 16 * (n / DT);
+    read_tr<FIRST>(vfr[n], rd.tr[2 * (n % DT)], rd.tr[2 * (n % DT) + 1]);
+  };
+  auto score = [&](int t, int par, int e, auto masked) INLINE {
+    return decltype(masked)::value && acc_row(e, 0) > seen - t * ROWS ? -INFINITY : s[par][e];
+  };
+  // The vector work of a sub-tile in steps of a product's length from the first product of its S on: element e in step 10 + e; the products with
+  // its first 8 elements begin in step 24.
+  auto vector = [&](int step, int t, auto par_, auto masked) INLINE {
+    constexpr int P = decltype(par_)::value;
+    const int e = step - 10;
+    if (e < 0 || e >= 16) return;
+    const float x = ody_exp2(fmaf(score(t, P, e, masked), c2, -ref));
+    l4[e & 3] += x;
+    pb[P][e >> 3][e & 7] = (bf16)x;
+  };
+  std::integral_constant<int, 0> c0;
+  std::integral_constant<int, 1> c1;
+  // One call: S of the tile after t, then P V of tile t (P: t & 1), 8 products each; under them the vector work of both.
+  auto unit = [&](int t, auto par_, auto masked) INLINE {
+    constexpr int P = decltype(par_)::value;
+    std::integral_constant<int, P ^ 1> other;
+    auto slot = [&](auto m_) INLINE {
+      constexpr int m = decltype(m_)::value;
+      if (m == 8) {
+        WAIT_LDS(0);
+#pragma unroll
+        for (int n = 0; n < 2 * DT; n++) tie(vfr[n]);
+        // K of tile t + 2 and V of tile t + 1 have landed (behind them 6 loads); everyone is done with tile t
+        asm volatile("s_waitcnt vmcnt(6)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+      }
+      if (m < 8) s[P ^ 1] = mfma32(kfr[m & 7], qf[m & 7], m == 0 ? f32x16{0} : s[P ^ 1]);
+      else o[m & 3] = mfma32(value(vfr[m & 7]), pb[P][(m & 7) >> 2], o[m & 3]);
+      FENCE();
+      if constexpr (m < 4) read_v(std::integral_constant<int, 4 + (m & 3)>{}, par_);
+      if constexpr (m >= 8 && m < 12) read_k(2 * (m & 3), P), read_k(2 * (m & 3) + 1, P);
+      if constexpr (m >= 12) read_v(std::integral_constant<int, m & 3>{}, other);
+      if (m > 8 && (m & 1)) load(t + 4, (m - 9) >> 1);
+      if (P == 1 && m == 4)
+#pragma unroll
+        for (int n = 0; n < KS; n++) rd.tr[n] += t & 2 ? -4 * FW_STAGE : 4 * FW_STAGE;
+      if (P == 1 && m == 15)
+#pragma unroll
+        for (int n = 0; n < KS; n++) rd.row[n] += t & 2 ? 4 * FW_STAGE : -4 * FW_STAGE;
+      vector(16 + m, t, par_, masked);
+      vector(m, t + 1, other, masked);
+      FENCE();
+    };
+    each<16>(slot);
+  };
+  auto clear_rows = [&]() INLINE {
+    clear(o);
+    ref = -FLT_MAX;   // no score is below it; not minus infinity, from which a masked score would be NaN
+#pragma unroll
+    for (int e = 0; e < 4; e++) l4[e] = 0.f;
+  };
+  clear_rows();
+  if (ntiles > 0) {
+    asm volatile("s_waitcnt vmcnt(14)" ::: "memory");   // K of tile 0
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    int t = 0;
+    if (w_live > 0) {
+#pragma unroll
+      for (int n = 0; n < KS; n++) read_k(n, 0);
+#pragma unroll
+      for (int n = 0; n < KS; n++) s[0] = mfma32(kfr[n], qf[n], n == 0 ? f32x16{0} : s[0]);
+    }
+    asm volatile("s_waitcnt vmcnt(10)" ::: "memory");   // K of tile 1, V of tile 0
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    if (w_live > 0) {
+#pragma unroll
+      for (int n = 0; n < KS; n++) read_k(n, 1);
+      each<DT>([&](auto n) INLINE { read_v(n, c0); });
+      // (S of the second one is formed again by the loop)
+      float mx = -INFINITY;
+#pragma unroll
+      for (int e = 0; e < 16; e++) mx = fmaxf(mx, score(0, 0, e, std::true_type{}));
+      if (w_live > 1) {
+#pragma unroll
+        for (int n = 0; n < KS; n++) s[1] = mfma32(kfr[n], qf[n], n == 0 ? f32x16{0} : s[1]);
+#pragma unroll
+        for (int e = 0; e < 16; e++) mx = fmaxf(mx, score(1, 1, e, std::true_type{}));
+      }
+      ref = fmaxf(ref, half_swap_max(mx) * c2);
+#pragma unroll
+      for (int m = 0; m < 16; m++) vector(m, 0, c0, std::true_type{});
+#pragma unroll
+      for (int n = 0; n < KS; n++) rd.row[n] += 4 * FW_STAGE;   // the loop reads rows two tiles ahead of columns
+      FENCE();
+      for (; t + 1 < w_live && t + 2 < w_full; t += 2) {
+        unit(t, c0, std::false_type{});
+        unit(t + 1, c1, std::false_type{});
+      }
+      for (; t + 1 < w_live; t += 2) {   // (behind the last tile one is formed that nobody uses)
+        unit(t, c0, std::true_type{});
+        unit(t + 1, c1, std::true_type{});
+      }
+      if (t < w_live) {   // an even tile is left
+        each<DT>([&](auto n) INLINE { read_v(std::integral_constant<int, DT + decltype(n)::value>{}, c0); });
+#pragma unroll
+        for (int m = 0; m < 16; m++) vector(16 + m, t, c0, std::true_type{});
+        WAIT_LDS(0);
+#pragma unroll
+        for (int n = 0; n < 2 * DT; n++) {
+          tie(vfr[n]);
+          o[n & 3] = mfma32(value(vfr[n]), pb[0][n >> 2], o[n & 3]);
+        }
+      } else {
+        WAIT_LDS(0);   // the reads of the tile behind
+#pragma unroll
+        for (int n = 0; n < DT; n++) tie(vfr[n]);
+      }
+    }
+    // the other wavefronts' tiles: keep bringing this one's share of them
+    for (; t < ntiles; t++) {
+      asm volatile("s_waitcnt vmcnt(6)" ::: "memory");
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+#pragma unroll
+      for (int j = 0; j < 4; j++) load(t + 4, j);
+    }
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();   // everyone is done with the ring
+  {
+    // a later score that outgrew its row's reference by more than fp32 holds left a row sum beyond any real one (or a NaN), or,
+    // times large values, an infinity in O: 0 times the accumulators is 0 unless one of them is not finite
+    int* flags = reinterpret_cast<int*>(smem);
+    float zero[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int dt = 0; dt < DT; dt++)
+#pragma unroll
+      for (int r = 0; r < 16; r++) zero[r & 3] = fmaf(o[dt][r], 0.f, zero[r & 3]);
+    const bool finite = (zero[0] + zero[1]) + (zero[2] + zero[3]) == 0.f;
+    const bool beyond = __builtin_amdgcn_ballot_w64(!finite || !(half_swap_sum((l4[0] + l4[1]) + (l4[2] + l4[3])) < 0x1p100f)) != 0;
+    if (lane == 0) flags[wave] = beyond;
+    __syncthreads();
+    int any = 0;
+#pragma unroll
+    for (int w = 0; w < 4 * GROUPS; w++) any |= flags[w];
+    __syncthreads();
+    if (any) {   // once more, with the maximum so far as a row's reference, so that P <= 1 and P V overflows for no values that P = 1 would hold
+      clear_rows();
+      for (int t = 0; t < ntiles; t++) {
+#pragma unroll
+        for (int j = 0; j < 4; j++) load(t, j);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        if (t < w_live) {
+          int own = lane;
+          asm volatile("" : "+v"(own));   // so that no address of this is kept in a register meanwhile
+          Readers<D> again;
+          again.init(fring + (t & 3) * FW_STAGE + 32 * D * grp, own >> 5, own & 31);
+#pragma unroll
+          for (int n = 0; n < KS; n++) s[0] = mfma32(row_frag(again, 0, n), qf[n], n == 0 ? f32x16{0} : s[0]);
+          float mx = -INFINITY;
+#pragma unroll
+          for (int e = 0; e < 16; e++) mx = fmaxf(mx, score(t, 0, e, std::true_type{}));
+          const float next = fmaxf(ref, half_swap_max(mx) * c2), alpha = ody_exp2(ref - next);
+          ref = next;
+#pragma unroll
+          for (int e = 0; e < 4; e++) l4[e] *= alpha;
+#pragma unroll
+          for (int dt = 0; dt < DT; dt++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) o[dt][r] *= alpha;
+#pragma unroll
+          for (int m = 10; m < 26; m++) vector(m, t, c0, std::true_type{});
+          auto product = [&](auto slice) INLINE {   // 16 keys, 64 columns of the head
+            constexpr int ss = decltype(slice)::value >> 1, hf = decltype(slice)::value & 1;
+            bf16x8 vf[2];
+            tr_frags<ROWS + 16 * ss, hf>(vf, again);
+#pragma unroll
+            for (int dt = 0; dt < 2; dt++) o[2 * hf + dt] = mfma32(vf[dt], pb[0][ss], o[2 * hf + dt]);
+          };
+          each<4>(product);
+        }
+        __syncthreads();
+      }
+    }
   }
 
   float l = (l4[0] + l4[1]) + (l4[2] + l4[3]);
@@ -431,15 +744,19 @@ inline int64_t row_blocks(int B, int L, int H) { return (int64_t)B * H * ((L + B
 //   65 / 55, backward 189 / 156; causal, L = 3001: 101 / 87, 340 / 287.  Short causal rows leave those blocks a few tiles each, most of them under the
 //   mask, so that for them the line of the backward is further out: 4 x 24 heads, L = 820, 131 / 147, 4 x 32 heads, L = 683, 139.6 / 142.9, and
 //   beyond, 4 x 32 heads, L = 820, 175 / 177; L = 936 211 / 200; with longer rows 2 x 32 heads, L = 1200, 150 / 144, L = 1536 207 / 191.
-//   Beyond the line in tiles the other kernels cut the range of the long side into parts: 4 heads, causal, L = 3001: forward 48 / 40; 8 heads,
-//   full, L = 3001: backward 218 / 163.  The line in blocks is too far out for some of these (6 heads, causal, L = 3500: forward 57 / 53), too
-//   near for backwards of the fewest blocks (2 heads, L = 2500: 95 / 120).  Forwards of 64 blocks and less stay there wherever it has parts: some
-//   are faster here (4 heads, L = 1000: 21 / 28), some are not (32 heads, 109 queries on 2042 keys: 36 / 32).
+//   Beyond the line in tiles the other kernels cut the range of the long side into parts: 8 heads, full, L = 3001: backward 218 / 163.  The line is too near for
+//   backwards of the fewest blocks (2 heads, L = 2500: 95 / 120).  The forward, in the ring: 4 heads, L = 4096, 46.5 / 47.6; 2 heads, L = 6000, 64 / 52; 3 heads,
+//   L = 8192, 84 / 77, 4 heads 91 / 94; 3 heads, L = 6000, full, 67 / 80; 12 heads, L = 4096, causal, 58 / 70; 6 heads, L = 12 000, 215 / 257.  Up to 64 blocks
+//   calls of 1024 keys and more stay with the parts, 300 queries on 8000 keys 82 / 65, also where they are short enough to be faster here, 8 heads, L = 1024,
+//   19 / 32; with fewer keys they do not (8 heads, L = 1000, 18.6 / 31.6).
 // One head, too, below the line: backward of 512 rows, causal, 28 / 67, of 1024 rows 44 / 96; two heads of 512 rows 28 / 68.
-bool ody_attn_fwd_short_ok(int B, int Lq, int Lk, int Hq, int causal) {
-  const int64_t blocks = row_blocks(B, Lq, Hq);
-  if (blocks <= 64 && ody_attn_fwd_pipe_parts(B, Lq, Lk, Hq, causal) > 1) return false;
-  return blocks <= (causal ? 640 : 256) && Lk <= ROWS * (blocks <= 128 ? 32 : 64);
+bool ody_attn_fwd_short_ok(const AttnParams& p) {
+  if (std::max(p.sk.l, p.sv.l) >= tile128::TILE_MAX_STRIDE) return false;   // rows of a tile beyond 32-bit offsets
+  const int64_t blocks = row_blocks(p.B, p.Lq, p.Hq), tiles = (p.Lk + ROWS - 1) / ROWS;
+  if (blocks <= 64 && p.Lk >= 1024 && ody_attn_fwd_pipe_parts(p.B, p.Lq, p.Lk, p.Hq, p.causal) > 1) return false;
+  if (blocks <= 128) return tiles <= 32;
+  if (blocks > (p.causal ? 640 : 256)) return false;
+  return tiles <= std::min<int64_t>(192, std::max<int64_t>(64, p.causal && blocks <= 256 ? blocks / 2 : 2 * blocks / 3));
 }
 bool ody_attn_bwd_short_ok(int B, int Lq, int Lk, int Hq, int causal) {
   const int64_t blocks = row_blocks(B, Lq, Hq) + row_blocks(B, Lk, Hq);
@@ -448,8 +765,13 @@ bool ody_attn_bwd_short_ok(int B, int Lq, int Lk, int Hq, int causal) {
 }
 
 int ody_launch_attn_fwd_short(const AttnParams& p, hipStream_t st) {
-  if (int rc = ody_allow_dynamic_lds(reinterpret_cast<const void*>(&attn_fwd_short_kernel), SMEM, "attn_fwd_short")) return rc;
-  ODY_LAUNCH("attn_fwd_short", st, attn_fwd_short_kernel, dim3((unsigned)row_blocks(p.B, p.Lq, p.Hq)), dim3(64 * WAVES), SMEM, p);
+  const int64_t blocks = row_blocks(p.B, p.Lq, p.Hq);
+  // Loop / ring, us: causal, L = 448, 32 heads, 13.5 / 13.7, L = 512 15.5 / 15.0; two blocks a unit L = 1500, 32 heads, 32.9 / 33.5, L = 2048 49.4 / 46.3;
+  // full, L = 256, 96 heads, 12.2 / 12.4, L = 331, 64 heads, 13.7 / 13.0, 85 heads 17.0 / 18.1, L = 512, 64 heads, 16.4 / 16.6, L = 1000, 32 heads, 24.7 / 23.4.
+  const bool ring = p.Lk >= (p.causal ? (blocks <= 256 ? 512 : 1536) : blocks <= 208 ? 320 : 960);
+  auto kern = ring ? &attn_fwd_short_ring_kernel : &attn_fwd_short_kernel;
+  if (int rc = ody_allow_dynamic_lds(reinterpret_cast<const void*>(kern), SMEM, "attn_fwd_short")) return rc;
+  ODY_LAUNCH("attn_fwd_short", st, kern, dim3((unsigned)row_blocks(p.B, p.Lq, p.Hq)), dim3(64 * WAVES), SMEM, p);
   return ody_check_launch("attn_fwd_short");
 }
 

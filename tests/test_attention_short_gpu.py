@@ -124,3 +124,35 @@ def test_causal_backward_of_many_blocks(L, H, short):
     q, k, v, do = (t[:, :, :2].cpu().float() for t in (q, k, v, do))
     for a, b, n in zip(got, oracle.attention_bwd(q, k, v, *oracle.attention_fwd(q, k, v, causal=True), do, causal=True), ("dq", "dk", "dv")):
         assert_parity(a[:, :, :2], b, TOL_BF16, n, 1e-3)
+
+
+# the forward's ring: fewer and more tiles than it holds, odd and even counts, ragged last sub-tiles, wavefronts and groups without a key, blocks without
+# one, and calls on either side of its lines
+@pytest.mark.parametrize("case", [(1, 512, 512, 2, 1, True), (1, 511, 511, 2, 2, True), (1, 61, 513, 3, 3, True), (1, 700, 545, 2, 2, True), (2, 900, 577, 2, 1, True),
+                                  (1, 1023, 1023, 4, 4, True), (1, 130, 320, 2, 2, False), (1, 130, 319, 2, 2, False), (1, 257, 353, 2, 1, False), (1, 97, 991, 2, 2, False),
+                                  (1, 2561, 4100, 7, 7, True), (1, 2049, 1536, 17, 17, True)], ids=lambda c: "B%d_Lq%d_Lk%d_H%d_%d_c%d" % c)
+@pytest.mark.parametrize("late", [1.0, 40.0], ids=["unit", "outgrown"])
+def test_forward_ring(case, late):
+    from odysseus_transformer_amd import ops
+    B, Lq, Lk, Hq, Hkv, causal = case
+    print(f"case={case} late={late}", flush=True)
+    q, k, v, _ = _inputs(B, Lq, Lk, Hq, Hkv, 7 * Lq + Lk)
+    k[:, Lk // 2:] *= late
+    (o, lse), ran = _run(lambda: ops.attn_fwd(q.cuda(), k.cuda(), v.cuda(), causal=causal))
+    assert "attn_fwd_short" in ran, ran
+    o_ref, lse_ref = oracle.attention_fwd(q.float(), k.float(), v.float(), causal=causal)
+    assert_parity(o, o_ref, TOL_BF16, "o")
+    assert torch.allclose(lse.cpu(), lse_ref, atol=TOL_LSE, rtol=TOL_LSE)
+
+
+@pytest.mark.parametrize("stride", [(1 << 24) - 16, (1 << 24) - 8], ids=str)
+def test_rows_beyond_a_tiles_offsets_go_to_the_other_kernels(stride):
+    from odysseus_transformer_amd import ops
+    q, k, v, _ = _inputs(1, 200, 130, 1, 1, 3)
+    far = torch.empty(stride * 129 + 128, dtype=torch.bfloat16, device="cuda").as_strided((1, 130, 1, 128), (0, stride, 128, 1))
+    far.copy_(v)
+    (o, lse), ran = _run(lambda: ops.attn_fwd(q.cuda(), k.cuda(), far, causal=True))
+    assert ("attn_fwd_short" in ran) == (stride < (1 << 24) - 8), ran
+    o_ref, lse_ref = oracle.attention_fwd(q.float(), k.float(), v.float(), causal=True)
+    assert_parity(o, o_ref, TOL_BF16, "o")
+    assert torch.allclose(lse.cpu(), lse_ref, atol=TOL_LSE, rtol=TOL_LSE)
