@@ -35,20 +35,20 @@ constexpr size_t SMEM = GROUPS * 2 * KV_STAGE * sizeof(bf16);
 static_assert(SMEM >= 4 * (16 * DT + 2) * 64 * sizeof(float) && SMEM >= 2 * QS_STAGE * sizeof(bf16) && SMEM <= 160 * 1024, "one block per unit");
 typedef TileLoader<D, 4> GroupLoader;
 constexpr int FW_STAGE = 2 * TILE;   // elements: K and V of a tile of the forward's ring of 4
-static_assert(4 * FW_STAGE * sizeof(bf16) <= SMEM, "the ring");
+static_assert(4 * FW_STAGE * sizeof(bf16) <= SMEM && 4 * QS_STAGE * sizeof(bf16) >= SMEM && 4 * QS_STAGE * sizeof(bf16) <= 160 * 1024, "the rings");
 #define FENCE() __builtin_amdgcn_sched_barrier(0)
 #define INLINE __attribute__((always_inline))
 #define WAIT_LDS(n) asm volatile("s_waitcnt lgkmcnt(" #n ")" ::: "memory")
 
-// A transposed fragment (tr_frags) whose reads are still under way: 16 rows from FIRST on, 32 columns by the address pair
+// A transposed fragment (tr_frags) whose reads are still under way: 16 rows from FIRST and FIRST + STEP on, 32 columns by the address pair
 struct TrFrag {
   s16x4 lo, hi;
 };
-template <int FIRST>
+template <int FIRST, int STEP = 8>
 __device__ __forceinline__ void read_tr(TrFrag& f, unsigned a0, unsigned a1) {
   asm volatile("ds_read_b64_tr_b16 %0, %2 offset:%4\n\tds_read_b64_tr_b16 %1, %3 offset:%5"
                : "=&v"(f.lo), "=&v"(f.hi)
-               : "v"(a0), "v"(a1), "n"(2 * FIRST * D), "n"(2 * (FIRST + 8) * D));
+               : "v"(a0), "v"(a1), "n"(2 * FIRST * D), "n"(2 * (FIRST + STEP) * D));
 }
 // behind the wait for them
 __device__ __forceinline__ void tie(TrFrag& f) { asm volatile("" : "+v"(f.lo), "+v"(f.hi)); }
@@ -595,6 +595,215 @@ __device__ __forceinline__ void dq_block(const AttnParams& p, unsigned char* sme
   store_dq_row(p, dq, b, h, qi, g);
 }
 
+// The same in the order of attn_fwd_short_ring_kernel: a wavefront has one sub-tile of every tile, and forms S and dP of the tile after (16 products)
+// and dQ of the present one (8) with the vector work of the former under them.
+__device__ __forceinline__ void dq_ring_block(const AttnParams& p, unsigned char* smem, int q0, int h, int b) {
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, g = lane >> 5, i = lane & 31;
+  const int grp = wave >> 2, w4 = wave & 3, hk = h / p.group, wq0 = q0 + w4 * 32, qi = wq0 + i;
+  const int n_end = p.causal ? min(p.Lk, min(q0 + BLOCK_ROWS, p.Lq) + p.off) : p.Lk;
+  const int ntiles = n_end > 0 ? (n_end + ROWS - 1) / ROWS : 0;
+  const bf16* kp = static_cast<const bf16*>(p.k) + b * p.sk.b + hk * p.sk.h;
+  const bf16* vp = static_cast<const bf16*>(p.v) + b * p.sv.b + hk * p.sv.h;
+  const float c2 = p.scale_log2e;
+  bf16* ring = reinterpret_cast<bf16*>(smem);   // [4][K tile | V tile]
+  const int brow = 4 * wave + (lane >> 4), bcol = 16 * ((lane & 15) ^ swz<D>(brow)), krow = 2 * (int)p.sk.l, vrow = 2 * (int)p.sv.l;
+  const int koff = brow * krow + bcol, voff = brow * vrow + bcol;
+  auto load = [&](int t, int part) INLINE {   // as in attn_fwd_short_ring_kernel
+    const int rows = min(p.Lk - t * ROWS, ROWS), row = part < 2 ? krow : vrow;
+    const bf16* src = (part < 2 ? kp : vp) + (int64_t)(t * ROWS) * (row / 2);
+    auto rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16*>(src), (short)0, t < ntiles ? (rows - 1) * row + 2 * D : 0, 0x00020000);
+    bf16* dst = ring + (t & 3) * FW_STAGE + (part < 2 ? 0 : TILE) + (8 * (part & 1) + wave) * 512;
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_ptr)dst, 16, (part < 2 ? koff : voff) + 32 * (part & 1) * row, 0, 0, 0);
+  };
+  // tile 0 and the queries first: what the first products wait for is not behind four tiles
+#pragma unroll
+  for (int j = 0; j < 4; j++) load(0, j);
+  FENCE();
+  bf16x8 qf[KS], dof[KS];
+  fetch_rows(qf, static_cast<const bf16*>(p.q) + b * p.sq.b + h * p.sq.h, p.sq.l, qi, p.Lq, g);
+  fetch_rows(dof, static_cast<const bf16*>(p.dout) + b * p.sdo.b + h * p.sdo.h, p.sdo.l, qi, p.Lq, g);
+  const int64_t head = (int64_t)b * p.Hq + h;
+  float lse2 = p.lse[head * p.Lq + min(qi, p.Lq - 1)], delta = p.delta[head * p.Lq + min(qi, p.Lq - 1)];
+  FENCE();
+#pragma unroll
+  for (int t = 1; t < 4; t++)
+#pragma unroll
+    for (int j = 0; j < 4; j++) load(t, j);
+  settle_rows(qf, qi, p.Lq);
+  settle_rows(dof, qi, p.Lq);
+  asm volatile("" : "+v"(lse2), "+v"(delta));
+  lse2 = qi >= p.Lq || lse2 == -INFINITY ? INFINITY : lse2 * ODY_LOG2E;   // past the end, or a query that saw no key: P = 0
+  if (qi >= p.Lq) delta = 0.f;
+
+  const int lim = p.causal ? min(p.Lk - 1, qi + p.off) : p.Lk - 1;   // last key this lane's query sees
+  const int sub_end = min(n_end, p.causal ? wq0 + 32 + p.off : n_end) - 32 * grp, sub_full = min(p.Lk, p.causal ? wq0 + 1 + p.off : p.Lk) - 32 * grp - 32;
+  const int w_live = sub_end > 0 ? (sub_end + ROWS - 1) / ROWS : 0;   // sub-tiles with a key that this wavefront sees
+  const int w_full = sub_full >= 0 ? sub_full / ROWS + 1 : 0;         // those of which all of its queries see all keys
+  const int seen = lim - 32 * grp - 4 * g;   // last key this lane's query sees, from this lane's first one in tile 0 on
+  f32x16 s, dp, dq[DT];
+  clear(dq);
+  bf16x8 ds[2][2], fr[KS];   // dS of even and odd tiles; rows of K, then of V, k-step n
+  TrFrag tf[DT];             // K^T: columns 32 n
+  Readers<D> rd;
+  rd.init(ring, g, i);
+#pragma unroll
+  for (int n = 0; n < KS; n++) rd.row[n] += 2 * 32 * D * grp, rd.tr[n] += 2 * 32 * D * grp;
+  typedef const bf16x8 __attribute__((address_space(3))) * frag_ptr;
+  auto read_row = [&](int n, int which, int odd) INLINE { fr[n] = *(frag_ptr)(uintptr_t)(rd.row[n] + odd * FW_STAGE * 2 + which * TILE * 2); };
+  auto read_col = [&](auto n_, auto odd_) INLINE {   // 16 keys n / DT, columns 32 (n % DT)
+    constexpr int n = decltype(n_)::value, FIRST = decltype(odd_)::value * 2 * ROWS + 16 * (n / DT);
+    read_tr<FIRST>(tf[n % DT], rd.tr[2 * (n % DT)], rd.tr[2 * (n % DT) + 1]);
+  };
+  // The vector work of a sub-tile in steps of a product's length from the first product of its S on: element e becomes P in step 9 + 11 e / 16 and
+  // dS in step 18 + 6 e / 16.
+  auto vector = [&](int step, int t, auto par_, auto masked) INLINE {
+    constexpr int P = decltype(par_)::value;
+#pragma unroll
+    for (int e = 0; e < 16; e++) {
+      if (18 + 6 * e / 16 == step) {
+        dp[e] = (dp[e] - delta) * s[e];
+        if (e & 1) ds[P][e >> 3][(e & 7) - 1] = (bf16)dp[e - 1], ds[P][e >> 3][e & 7] = (bf16)dp[e];
+      }
+      if (9 + 11 * e / 16 == step) {
+        const float x = decltype(masked)::value && acc_row(e, 0) > seen - t * ROWS ? -INFINITY : s[e];
+        s[e] = ody_exp2(fmaf(x, c2, -lse2));
+      }
+    }
+  };
+  std::integral_constant<int, 0> c0;
+  std::integral_constant<int, 1> c1;
+  auto unit = [&](int t, auto par_, auto masked) INLINE {   // P: t & 1
+    constexpr int P = decltype(par_)::value;
+    std::integral_constant<int, P ^ 1> other;
+    auto slot = [&](auto m_) INLINE {
+      constexpr int m = decltype(m_)::value;
+      if (m == 12)   // they are there; later the compiler's wait for one would be a wait for the transposing reads as well
+#pragma unroll
+        for (int n = 4; n < KS; n++) asm volatile("" : "+v"(fr[n]));
+      if constexpr (m >= 16) {
+        if (m == 20) {
+          WAIT_LDS(0);
+#pragma unroll
+          for (int n = 0; n < DT; n++) tie(tf[n]);
+          // tile t + 2 has landed (behind it the 4 loads of the next); everyone is done with tile t, and with V of the one after
+          asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+          __builtin_amdgcn_s_barrier();
+          asm volatile("" ::: "memory");
+        } else if (m < 20) {
+          WAIT_LDS(6);
+          tie(tf[m & 3]);
+        }
+      }
+      if (m < 8) s = mfma32(fr[m & 7], qf[m & 7], m == 0 ? f32x16{0} : s);
+      else if (m < 16) dp = mfma32(fr[m & 7], dof[m & 7], m == 8 ? f32x16{0} : dp);
+      else dq[m & 3] = mfma32(value(tf[m & 3]), ds[P][(m & 7) >> 2], dq[m & 3]);
+      FENCE();
+      if constexpr (m < 8) read_row(m, 1, P ^ 1);
+      if constexpr (m >= 12 && m < 20) read_col(std::integral_constant<int, m - 12>{}, par_);
+      if constexpr (m >= 20) {
+        read_row(2 * (m & 3), 0, P), read_row(2 * (m & 3) + 1, 0, P);
+        load(t + 4, m & 3);
+      }
+      if (P == 0 && m == 10)
+#pragma unroll
+        for (int n = 0; n < KS; n++) rd.row[n] += t & 2 ? -4 * FW_STAGE : 4 * FW_STAGE;
+      if (P == 1 && m == 20)
+#pragma unroll
+        for (int n = 0; n < KS; n++) rd.tr[n] += t & 2 ? -4 * FW_STAGE : 4 * FW_STAGE;
+      vector(m, t + 1, other, masked);
+      FENCE();
+    };
+    each<24>(slot);
+  };
+  if (ntiles > 0) {
+    asm volatile("s_waitcnt vmcnt(12)" ::: "memory");   // tile 0
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    int t = 0;
+    if (w_live > 0) {
+#pragma unroll
+      for (int n = 0; n < KS; n++) read_row(n, 0, 0);
+#pragma unroll
+      for (int n = 0; n < KS; n++) s = mfma32(fr[n], qf[n], n == 0 ? f32x16{0} : s);
+#pragma unroll
+      for (int n = 0; n < KS; n++) read_row(n, 1, 0);
+#pragma unroll
+      for (int n = 0; n < KS; n++) dp = mfma32(fr[n], dof[n], n == 0 ? f32x16{0} : dp);
+    }
+    asm volatile("s_waitcnt vmcnt(8)" ::: "memory");   // tile 1
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    if (w_live > 0) {
+#pragma unroll
+      for (int n = 0; n < KS; n++) read_row(n, 0, 1);
+#pragma unroll
+      for (int m = 9; m < 24; m++) vector(m, 0, c0, std::true_type{});
+      FENCE();
+      for (; t + 1 < w_live && t + 2 < w_full; t += 2) {
+        unit(t, c0, std::false_type{});
+        unit(t + 1, c1, std::false_type{});
+      }
+      for (; t + 1 < w_live; t += 2) {   // (behind the last tile one is formed that nobody uses)
+        unit(t, c0, std::true_type{});
+        unit(t + 1, c1, std::true_type{});
+      }
+      if (t < w_live) {   // an even tile is left
+        auto half = [&](auto ss_) INLINE {
+          constexpr int ss = decltype(ss_)::value;
+          each<DT>([&](auto n) INLINE { read_col(std::integral_constant<int, DT * ss + decltype(n)::value>{}, c0); });
+          WAIT_LDS(0);
+#pragma unroll
+          for (int n = 0; n < DT; n++) {
+            tie(tf[n]);
+            dq[n] = mfma32(value(tf[n]), ds[0][ss], dq[n]);
+          }
+        };
+        half(c0);
+        half(c1);
+      }
+    }
+    // the other wavefronts' tiles: keep bringing this one's share of them
+    for (; t < ntiles; t++) {
+      asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+#pragma unroll
+      for (int j = 0; j < 4; j++) load(t + 4, j);
+    }
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+
+  float* patch = reinterpret_cast<float*>(smem) + w4 * 16 * DT * 64;
+  __syncthreads();
+  if (grp == 1) give(patch, dq, lane);
+  __syncthreads();
+  if (grp == 1) return;
+  take(patch, dq, lane, 1.f, 1.f);
+  store_dq_row(p, dq, b, h, qi, g);
+}
+
+// dK^T or dV^T of a key, to its row or to the fp32 parts
+template <bool PART, bool IS_DK>
+__device__ __forceinline__ void store_kv_row(const AttnParams& p, const f32x16 (&acc)[DT], int b, int h, int hk, int key, int g, float* __restrict__ part) {
+  if (key >= p.Lk) return;
+  if constexpr (PART) {   // [dK | dV][B][Hq][Lk][D] in fp32
+    float* dst = part + (IS_DK ? 0 : (int64_t)p.B * p.Hq * p.Lk * D) + (((int64_t)b * p.Hq + h) * p.Lk + key) * D;
+#pragma unroll
+    for (int dt = 0; dt < DT; dt++)
+#pragma unroll
+      for (int a = 0; a < 4; a++) {
+        f32x4 w;
+#pragma unroll
+        for (int e = 0; e < 4; e++) w[e] = acc[dt][4 * a + e];
+        *reinterpret_cast<f32x4*>(dst + 32 * dt + 8 * a + 4 * g) = w;
+      }
+  } else if constexpr (IS_DK) {
+    store_dk_row(p, acc, b, hk, key, g);
+  } else {
+    store_row(static_cast<bf16*>(p.dv) + b * p.sdv.b + hk * p.sdv.h + (int64_t)key * p.sdv.l, acc, 1.f, g);
+  }
+}
+
 // One of dK and dV of 32 keys per wavefront, over the query tiles of one query head: wavefronts 0 - 3 of a block hold dV of its 128
 // keys, 4 - 7 dK.
 //   S = Q K^T - lse / scale     dV^T += dO^T P                                              lane = key column
@@ -695,28 +904,230 @@ __device__ __forceinline__ void kv_block(const AttnParams& p, unsigned char* sme
     rd.move((n & 1) ? -(int)STAGE_BYTES : (int)STAGE_BYTES);
   }
 
-  if (key >= p.Lk) return;
-  if constexpr (PART) {   // [dK | dV][B][Hq][Lk][D] in fp32
-    float* dst = part + (IS_DK ? 0 : (int64_t)p.B * p.Hq * p.Lk * D) + (((int64_t)b * p.Hq + h) * p.Lk + key) * D;
-#pragma unroll
-    for (int dt = 0; dt < DT; dt++)
-#pragma unroll
-      for (int a = 0; a < 4; a++) {
-        f32x4 w;
-#pragma unroll
-        for (int e = 0; e < 4; e++) w[e] = acc[dt][4 * a + e];
-        *reinterpret_cast<f32x4*>(dst + 32 * dt + 8 * a + 4 * g) = w;
-      }
-  } else if constexpr (IS_DK) {
-    store_dk_row(p, acc, b, hk, key, g);
-  } else {
-    store_row(static_cast<bf16*>(p.dv) + b * p.sdv.b + hk * p.sdv.h + (int64_t)key * p.sdv.l, acc, 1.f, g);
-  }
+  store_kv_row<PART, IS_DK>(p, acc, b, h, hk, key, g, part);
 }
 
+// The same with loads three tiles ahead and the vector work of a sub-tile of 32 queries under the products of its neighbours: one call of `unit` forms
+// S (and dP) of the sub-tile after and adds this one to dV or dK.  Each role passes the same barriers, one per query tile behind those of the prologue.
+template <bool PART, bool IS_DK>
+__device__ __forceinline__ void kv_ring_block(const AttnParams& p, unsigned char* smem, int n0, int h, int b, const bf16* __restrict__ stats,
+                                              float* __restrict__ part) {
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, g = lane >> 5, i = lane & 31;
+  const int hk = h / p.group, wn0 = n0 + (wave & 3) * 32, key = wn0 + i;
+  bf16* ring = reinterpret_cast<bf16*>(smem);   // [4][Q tile | dO tile | row values]
+  const int q_tiles = (p.Lq + ROWS - 1) / ROWS, t_top = q_tiles - 1;
+  // this block's tiles, last query tile first, and of them those that see a key of this wavefront and those that see all of its keys
+  const int total = max(0, q_tiles - (p.causal ? max(0, n0 - p.off) / ROWS : 0));
+  int w_total = total, w_full = total;
+  if (p.causal) {
+    w_total = min(total, max(0, q_tiles - max(0, wn0 - p.off) / ROWS));
+    w_full = min(total, max(0, q_tiles - (max(0, wn0 + 31 - p.off) + ROWS - 1) / ROWS));
+  }
+  const bf16* qp = static_cast<const bf16*>(p.q) + b * p.sq.b + h * p.sq.h;
+  const bf16* dop = static_cast<const bf16*>(p.dout) + b * p.sdo.b + h * p.sdo.h;
+  const bf16* sp = stats + ((int64_t)b * p.Hq + h) * q_tiles * 512;
+  // Direct loads of tile n: halves of Q (0, 1) and of dO (2, 3), a quarter of the row values (4; twice).  Rows past the end read zeros, a tile past the end
+  // nothing else.
+  const int brow = 4 * wave + (lane >> 4), qrow = 2 * (int)p.sq.l, orow = 2 * (int)p.sdo.l;
+  auto load = [&](int n, int what) INLINE {
+    const int t = t_top - n;
+    bf16* st = ring + (n & 3) * QS_STAGE;
+    if (what == 4) {
+      auto rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16*>(sp + (int64_t)t * 512), (short)0, n < total ? 1024 : 0, 0x00020000);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_ptr)(st + 2 * TILE + 128 * (wave & 3)), 4, 256 * (wave & 3) + 4 * lane, 0, 0, 0);
+      return;
+    }
+    const int rows = min(p.Lq - t * ROWS, ROWS), row = what < 2 ? qrow : orow, j = what & 1;
+    const bf16* src = (what < 2 ? qp : dop) + (int64_t)(t * ROWS) * (row / 2);
+    auto rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16*>(src), (short)0, n < total ? (rows - 1) * row + 2 * D : 0, 0x00020000);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_ptr)(st + (what < 2 ? 0 : TILE) + (8 * j + wave) * 512), 16,
+                                             (brow + 32 * j) * row + 16 * ((lane & 15) ^ swz<D>((brow + 32 * j) >> 2)), 0, 0, 0);
+  };
+  auto all = [&](int n) INLINE {
+#pragma unroll
+    for (int what = 0; what < 5; what++) load(n, what);
+  };
+  all(0);
+  FENCE();
+  bf16x8 kf[KS], vf[IS_DK ? KS : 1];
+  fetch_rows(kf, static_cast<const bf16*>(p.k) + b * p.sk.b + hk * p.sk.h, p.sk.l, key, p.Lk, g);
+  if constexpr (IS_DK) fetch_rows(vf, static_cast<const bf16*>(p.v) + b * p.sv.b + hk * p.sv.h, p.sv.l, key, p.Lk, g);
+  FENCE();
+  all(1);
+  all(2);
+  settle_rows(kf, key, p.Lk);
+  if constexpr (IS_DK) settle_rows(vf, key, p.Lk);
+
+  const float c2 = p.scale_log2e;
+  const int key_off = p.causal ? key - p.off : -(1 << 30);   // the first query that sees this lane's key
+  constexpr int NS = IS_DK ? 1 : 2, NT = IS_DK ? DT : 2 * DT;
+  f32x16 s[NS], dp, acc[DT];     // S, then P, for dV of either sub-tile of a tile; dP, then dS; dK^T or dV^T
+  bf16x8 pf[2][2], fr[KS];       // P or dS of either sub-tile; rows of Q, and for dK then of dO, k-step n
+  TrFrag tf[NT];                 // dO^T or Q^T: 16 queries n / DT, columns 32 (n % DT)
+  clear(acc);
+  Readers<D, true> rd;
+  rd.init(ring, g, i);
+  // from tile n's place in the ring to the next one's
+  auto onward = [&](int n) INLINE { return (n + 1) & 3 ? (int)(QS_STAGE * 2) : -3 * (int)(QS_STAGE * 2); };
+  typedef const bf16x8 __attribute__((address_space(3))) * frag_ptr;
+  auto read_row = [&](int n, int which, int mt) INLINE { fr[n] = *(frag_ptr)(uintptr_t)(rd.row[n] + 2 * (which * TILE + 2 * mt * D)); };
+  auto read_col = [&](auto n_, auto mt_) INLINE {
+    constexpr int n = decltype(n_)::value, FIRST = (IS_DK ? 0 : ROWS) + 2 * decltype(mt_)::value + n / DT;
+    read_tr<FIRST, 32>(tf[n % NT], rd.tr[2 * (n % DT)], rd.tr[2 * (n % DT) + 1]);
+  };
+  // a quarter a of a lane's 16 start values of sub-tile mt of tile n
+  auto start = [&](int n, int mt, int which, int a, f32x16& x) INLINE {
+    const f32x4 v = *reinterpret_cast<const f32x4*>(reinterpret_cast<const float*>(ring + (n & 3) * QS_STAGE + 2 * TILE) + 16 * g + 64 * mt + 32 * which + 4 * a);
+#pragma unroll
+    for (int e = 0; e < 4; e++) x[4 * a + e] = v[e];
+  };
+  // The vector work of sub-tile mt of tile n in steps of a product's length from the first product of its S on.  dV: element e becomes P in step 9 + 12 e / 16,
+  // the products with it begin in step 24.  dK: P in step 9 + 11 e / 16, dS in step 18 + 6 e / 16, the products in step 40.
+  auto vector = [&](int step, int n, auto mt_, auto masked) INLINE {
+    constexpr int MT = decltype(mt_)::value, S = IS_DK ? 0 : MT;
+#pragma unroll
+    for (int e = 0; e < 16; e++) {
+      if (IS_DK && 18 + 6 * e / 16 == step) {
+        dp[e] = s[S][e] * dp[e];
+        if (e & 1) pf[MT][e >> 3][(e & 7) - 1] = (bf16)dp[e - 1], pf[MT][e >> 3][e & 7] = (bf16)dp[e];
+      }
+      if (9 + (IS_DK ? 11 : 12) * e / 16 == step) {
+        const float x = decltype(masked)::value && (t_top - n) * ROWS + tile128::acc_tile_row(e, g, MT) < key_off ? -INFINITY : s[S][e];
+        s[S][e] = ody_exp2(x * c2);
+        if (!IS_DK && (e & 1)) pf[MT][e >> 3][(e & 7) - 1] = (bf16)s[S][e - 1], pf[MT][e >> 3][e & 7] = (bf16)s[S][e];
+      }
+    }
+  };
+  std::integral_constant<int, 0> c0;
+  std::integral_constant<int, 1> c1;
+  // tile n + 1 has landed (behind it the 5 loads of the next); everyone is done with tile n - 1
+  auto turn = [&]() INLINE {
+    asm volatile("s_waitcnt vmcnt(5)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+  auto move = [&](unsigned (&x)[KS], int bytes) INLINE {
+#pragma unroll
+    for (int n = 0; n < KS; n++) x[n] += bytes;
+  };
+  auto unit = [&](int n, auto mt_, auto masked) INLINE {
+    constexpr int MT = decltype(mt_)::value, NMT = MT ^ 1, S = IS_DK ? 0 : NMT;
+    std::integral_constant<int, NMT> nmt;
+    const int nn = MT ? n + 1 : n;   // the sub-tile after is in tile nn; behind that, sub-tile MT of tile n + 1
+    auto slot = [&](auto m_) INLINE {
+      constexpr int m = decltype(m_)::value;
+      if constexpr (IS_DK) {
+        if (m == 12)   // they are there; later the compiler's wait for one would be a wait for the transposing reads as well
+#pragma unroll
+          for (int r = 4; r < KS; r++) asm volatile("" : "+v"(fr[r]));
+        if (m >= 16 && m < 20) {
+          WAIT_LDS(6);
+          tie(tf[m & 3]);
+        }
+        if (m == 20) {
+          WAIT_LDS(0);
+#pragma unroll
+          for (int r = 0; r < DT; r++) tie(tf[r]);
+          if (MT == 0) turn();
+        }
+        if (m < 8) s[0] = mfma32(fr[m & 7], kf[m & 7], s[0]);
+        else if (m < 16) dp = mfma32(fr[m & 7], vf[m & 7], dp);
+        else acc[m & 3] = mfma32(value(tf[m & 3]), pf[MT][(m & 7) >> 2], acc[m & 3]);
+        FENCE();
+        if (m < 4) start(nn, NMT, 1, m, dp);
+        if constexpr (m < 8) read_row(m, 1, NMT);
+        if (MT == 0 && m == 10) move(rd.row, onward(n));
+        if constexpr (m >= 12 && m < 20) read_col(std::integral_constant<int, m - 12>{}, mt_);
+        if (MT == 1 && m == 20) move(rd.tr, onward(n));
+        if constexpr (m >= 20) read_row(2 * (m & 3), 0, MT), read_row(2 * (m & 3) + 1, 0, MT);
+        if (MT == 0 && m == 21) load(n + 3, 0), load(n + 3, 1);
+        if (MT == 1 && (m == 2 || m == 10 || m == 20)) load(n + 3, m == 2 ? 2 : m == 10 ? 3 : 4);
+        vector(m, nn, nmt, masked);
+        if (m == 23)
+#pragma unroll
+          for (int a = 0; a < 4; a++) start(n + 1, MT, 0, a, s[0]);
+      } else {
+        if (m == 8) {
+          WAIT_LDS(0);
+#pragma unroll
+          for (int r = 0; r < NT; r++) tie(tf[r]);
+          if (MT == 0) turn();
+        }
+        if (m < 8) s[S] = mfma32(fr[m & 7], kf[m & 7], s[S]);
+        else acc[m & 3] = mfma32(value(tf[m & 7]), pf[MT][(m & 7) >> 2], acc[m & 3]);
+        FENCE();
+        if constexpr (m < 8) read_col(m_, mt_);
+        if (MT == 1 && m == 8) move(rd.tr, onward(n));
+        if constexpr (m >= 8) read_row(m & 7, 0, MT);
+        if (MT == 1 && m == 15) move(rd.row, onward(n + 1));
+        if (MT == 0 && (m == 10 || m == 13)) load(n + 3, m == 13);
+        if (MT == 1 && (m == 2 || m == 6 || m == 10)) load(n + 3, m == 2 ? 2 : m == 6 ? 3 : 4);
+        vector(16 + m, n, mt_, masked);
+        vector(m, nn, nmt, masked);
+        if (m >= 12) start(n + 1, MT, 0, m & 3, s[MT]);
+      }
+      FENCE();
+    };
+    each<IS_DK ? 24 : 16>(slot);
+  };
+  if (total > 0) {
+    asm volatile("s_waitcnt vmcnt(10)" ::: "memory");   // the first tile
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    int n = 0;
+    if (w_total > 0) {
+#pragma unroll
+      for (int a = 0; a < 4; a++) {
+        start(0, 0, 0, a, s[0]);
+        if constexpr (IS_DK) start(0, 0, 1, a, dp);
+        else start(0, 1, 0, a, s[1]);
+      }
+#pragma unroll
+      for (int r = 0; r < KS; r++) read_row(r, 0, 0);
+#pragma unroll
+      for (int r = 0; r < KS; r++) s[0] = mfma32(fr[r], kf[r], s[0]);
+      if constexpr (IS_DK) {
+#pragma unroll
+        for (int r = 0; r < KS; r++) read_row(r, 1, 0);
+#pragma unroll
+        for (int r = 0; r < KS; r++) dp = mfma32(fr[r], vf[r], dp);
+      }
+#pragma unroll
+      for (int r = 0; r < KS; r++) read_row(r, 0, 1);
+#pragma unroll
+      for (int m = 9; m < (IS_DK ? 24 : 16); m++) vector(m, 0, c0, std::true_type{});
+      if constexpr (IS_DK) {
+#pragma unroll
+        for (int a = 0; a < 4; a++) start(0, 1, 0, a, s[0]);
+      } else {
+        move(rd.row, onward(0));   // the loop reads rows one tile ahead of columns
+      }
+      FENCE();
+      for (; n + 1 < min(w_total, w_full); n++) {
+        unit(n, c0, std::false_type{});
+        unit(n, c1, std::false_type{});
+      }
+      for (; n < w_total; n++) {   // (behind the last tile a sub-tile is formed that nobody uses)
+        unit(n, c0, std::true_type{});
+        unit(n, c1, std::true_type{});
+      }
+    }
+    // the other wavefronts' tiles: keep bringing this one's share of them
+    for (; n < total; n++) {
+      turn();
+      all(n + 3);
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  }
+  store_kv_row<PART, IS_DK>(p, acc, b, h, hk, key, g, part);
+}
+
+// RING: where rows have tiles enough, dq_ring_block and kv_ring_block.  Bound: a block's longest role, dK, 48 products a tile and wavefront beside dV's 32 (1.75 us
+// a tile where these take 1.15; 2.2 before, in waits for transposing reads and for tiles one ahead).
+//
 // The whole backward behind the pre-pass in one launch.  A rank of key blocks (first keys first: the most query tiles) and a rank of
 // query blocks (last queries first) alternate, over all heads, so that what starts last is short on both sides.
-template <bool PART>
+template <bool PART, bool RING>
 __global__ __launch_bounds__(64 * WAVES, 2) void attn_bwd_short_kernel(const AttnParams p, const bf16* __restrict__ stats,
                                                                    float* __restrict__ part) {
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
@@ -725,11 +1136,14 @@ __global__ __launch_bounds__(64 * WAVES, 2) void attn_bwd_short_kernel(const Att
   const bool paired = bc.rank < 2 * both;
   const int rank = paired ? bc.rank >> 1 : bc.rank - both;
   if (paired ? bc.rank & 1 : nq > nkv) {
-    dq_block(p, smem, (p.causal ? nq - 1 - rank : rank) * BLOCK_ROWS, bc.h, bc.b);
+    if constexpr (RING) dq_ring_block(p, smem, (p.causal ? nq - 1 - rank : rank) * BLOCK_ROWS, bc.h, bc.b);
+    else dq_block(p, smem, (p.causal ? nq - 1 - rank : rank) * BLOCK_ROWS, bc.h, bc.b);
   } else if (__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) < WAVES / 2) {
-    kv_block<PART, false>(p, smem, rank * BLOCK_ROWS, bc.h, bc.b, stats, part);
+    if constexpr (RING) kv_ring_block<PART, false>(p, smem, rank * BLOCK_ROWS, bc.h, bc.b, stats, part);
+    else kv_block<PART, false>(p, smem, rank * BLOCK_ROWS, bc.h, bc.b, stats, part);
   } else {
-    kv_block<PART, true>(p, smem, rank * BLOCK_ROWS, bc.h, bc.b, stats, part);
+    if constexpr (RING) kv_ring_block<PART, true>(p, smem, rank * BLOCK_ROWS, bc.h, bc.b, stats, part);
+    else kv_block<PART, true>(p, smem, rank * BLOCK_ROWS, bc.h, bc.b, stats, part);
   }
 }
 
@@ -744,8 +1158,8 @@ inline int64_t row_blocks(int B, int L, int H) { return (int64_t)B * H * ((L + B
 //   65 / 55, backward 189 / 156; causal, L = 3001: 101 / 87, 340 / 287.  Short causal rows leave those blocks a few tiles each, most of them under the
 //   mask, so that for them the line of the backward is further out: 4 x 24 heads, L = 820, 131 / 147, 4 x 32 heads, L = 683, 139.6 / 142.9, and
 //   beyond, 4 x 32 heads, L = 820, 175 / 177; L = 936 211 / 200; with longer rows 2 x 32 heads, L = 1200, 150 / 144, L = 1536 207 / 191.
-//   Beyond the line in tiles the other kernels cut the range of the long side into parts: 8 heads, full, L = 3001: backward 218 / 163.  The line is too near for
-//   backwards of the fewest blocks (2 heads, L = 2500: 95 / 120).  The forward, in the ring: 4 heads, L = 4096, 46.5 / 47.6; 2 heads, L = 6000, 64 / 52; 3 heads,
+//   Beyond the line in tiles the other kernels cut the range of the long side into parts, backward, in the ring: 8 heads, full, L = 3000, 185 / 167, 2 heads,
+//   causal, L = 5000, 134 / 126; inside it 3 heads, L = 2500, causal or full, 75 / 121, 5 heads, L = 3000, full, 104 / 141.  The forward, in the ring: 4 heads, L = 4096, 46.5 / 47.6; 2 heads, L = 6000, 64 / 52; 3 heads,
 //   L = 8192, 84 / 77, 4 heads 91 / 94; 3 heads, L = 6000, full, 67 / 80; 12 heads, L = 4096, causal, 58 / 70; 6 heads, L = 12 000, 215 / 257.  Up to 64 blocks
 //   calls of 1024 keys and more stay with the parts, 300 queries on 8000 keys 82 / 65, also where they are short enough to be faster here, 8 heads, L = 1024,
 //   19 / 32; with fewer keys they do not (8 heads, L = 1000, 18.6 / 31.6).
@@ -761,7 +1175,7 @@ bool ody_attn_fwd_short_ok(const AttnParams& p) {
 bool ody_attn_bwd_short_ok(int B, int Lq, int Lk, int Hq, int causal) {
   const int64_t blocks = row_blocks(B, Lq, Hq) + row_blocks(B, Lk, Hq);
   const int rows = std::max(Lq, Lk);
-  return blocks <= (causal ? (rows <= 16 * ROWS ? 1536 : 1024) : 512) && rows <= ROWS * (causal && blocks > 128 ? 56 : 32);
+  return blocks <= (causal ? (rows <= 16 * ROWS ? 1536 : 1024) : 512) && rows <= ROWS * (causal || blocks <= 256 ? 56 : 32);
 }
 
 int ody_launch_attn_fwd_short(const AttnParams& p, hipStream_t st) {
@@ -777,8 +1191,14 @@ int ody_launch_attn_fwd_short(const AttnParams& p, hipStream_t st) {
 
 int ody_launch_attn_bwd_short(const AttnParams& p, const void* stats, float* part, hipStream_t st) {
   const dim3 grid((unsigned)(row_blocks(p.B, p.Lq, p.Hq) + row_blocks(p.B, p.Lk, p.Hq)));
-  auto kern = p.group > 1 ? &attn_bwd_short_kernel<true> : &attn_bwd_short_kernel<false>;
-  if (int rc = ody_allow_dynamic_lds(reinterpret_cast<const void*>(kern), SMEM, "attn_bwd_short")) return rc;
-  ODY_LAUNCH("attn_bwd_short", st, kern, grid, dim3(64 * WAVES), SMEM, p, static_cast<const bf16*>(stats), part);
+  // Loop / ring, the whole backward, us: causal, L = 331, 21 heads, 22.6 / 22.7, L = 600, 13 heads, 34.9 / 32.6, L = 1000, 8 heads, 45.5 / 40.1; more than one block
+  // for a unit: L = 512, 96 heads, 58 / 59, L = 700, 43 heads, 54 / 56, L = 1000, 32 heads, 62 / 60, L = 1500 106 / 101.
+  const bool near = std::max(std::max(p.sq.l, p.sdo.l), std::max(p.sk.l, p.sv.l)) < tile128::TILE_MAX_STRIDE;   // 32-bit offsets in a tile
+  const bool ring = near && std::max(p.Lq, p.Lk) >= (grid.x <= 256 ? 512 : 960);
+  auto kern = ring ? (p.group > 1 ? &attn_bwd_short_kernel<true, true> : &attn_bwd_short_kernel<false, true>)
+                   : (p.group > 1 ? &attn_bwd_short_kernel<true, false> : &attn_bwd_short_kernel<false, false>);
+  const size_t smem = ring ? 4 * QS_STAGE * sizeof(bf16) : SMEM;
+  if (int rc = ody_allow_dynamic_lds(reinterpret_cast<const void*>(kern), smem, "attn_bwd_short")) return rc;
+  ODY_LAUNCH("attn_bwd_short", st, kern, grid, dim3(64 * WAVES), smem, p, static_cast<const bf16*>(stats), part);
   return ody_check_launch("attn_bwd_short");
 }

@@ -145,6 +145,39 @@ def test_forward_ring(case, late):
     assert torch.allclose(lse.cpu(), lse_ref, atol=TOL_LSE, rtol=TOL_LSE)
 
 
+# the backward's rings likewise: either side of their line, in one direction only, few and many tiles, wavefronts without a query or a key
+@pytest.mark.parametrize("case", [(1, 511, 512, 2, 1, True), (1, 511, 511, 2, 2, True), (1, 33, 545, 3, 3, True), (1, 700, 31, 2, 2, True), (2, 900, 577, 2, 1, True),
+                                  (1, 130, 513, 2, 2, False), (1, 577, 65, 4, 1, False), (1, 1023, 1025, 4, 4, True), (1, 97, 991, 2, 2, False),
+                                  (1, 3401, 3400, 1, 1, True), (1, 1601, 3500, 3, 3, False), (1, 959, 959, 17, 17, True), (1, 961, 960, 17, 17, True)],
+                         ids=lambda c: "B%d_Lq%d_Lk%d_H%d_%d_c%d" % c)
+def test_backward_rings(case):
+    from odysseus_transformer_amd import ops
+    B, Lq, Lk, Hq, Hkv, causal = case
+    print(f"case={case}", flush=True)
+    q, k, v, do = _inputs(B, Lq, Lk, Hq, Hkv, 11 * Lq + Lk)
+    o_ref, lse_ref = oracle.attention_fwd(q.float(), k.float(), v.float(), causal=causal)
+    refs = oracle.attention_bwd(q.float(), k.float(), v.float(), o_ref, lse_ref, do.float(), causal=causal)
+    qg, kg, vg, dog = (t.cuda() for t in (q, k, v, do))
+    o, lse = ops.attn_fwd(qg, kg, vg, causal=causal)
+    grads, ran = _run(lambda: ops.attn_bwd(qg, kg, vg, o, lse, dog, causal=causal))
+    assert "attn_bwd_short" in ran, ran
+    for got, ref, name in zip(grads, refs, ("dq", "dk", "dv")):
+        assert_parity(got, ref, TOL_BF16, name, 1e-3)
+    assert all(torch.equal(a, b) for a, b in zip(grads, ops.attn_bwd(qg, kg, vg, o, lse, dog, causal=causal)))
+
+
+def test_backward_ring_has_the_sums_of_the_kernels_for_long_rows():
+    """dK and dV do not depend on whether dS is kept, which those kernels do."""
+    from odysseus_transformer_amd import ops
+    q, k, v, do = (t.cuda() for t in _inputs(1, 1024, 1024, 16, 4, 77))
+    o, lse = ops.attn_fwd(q, k, v, causal=True)
+    got, ran = _run(lambda: ops.attn_bwd(q, k, v, o, lse, do, causal=True))
+    assert "attn_bwd_short" in ran, ran
+    kept, ran = _run(lambda: ops.attn_bwd(q, k, v, o, lse, do, causal=True, keep_ds=True))
+    assert "attn_bwd_short" not in ran, ran
+    assert torch.equal(got[1], kept[1]) and torch.equal(got[2], kept[2])
+
+
 @pytest.mark.parametrize("stride", [(1 << 24) - 16, (1 << 24) - 8], ids=str)
 def test_rows_beyond_a_tiles_offsets_go_to_the_other_kernels(stride):
     from odysseus_transformer_amd import ops
