@@ -232,18 +232,28 @@ __global__ __launch_bounds__(256) void gemm_splitk_rope_kernel(const float* __re
 // tiles) 183 / 150, gate_up of 1000 tokens (344) 183 / 161, of 3001 (1032) 484 / 453, four weight gradients over 1000 tokens 394 / 371.
 // Halves / quarters: QKV of 3001 tokens 141 / 136, gate_up of 2100 (774) 333 / 325, of 3001 428 / 421, its input gradient of 5000 (320)
 // 778 / 745.
+//
+// Twelve or sixteen ranges of K, of 40 slabs each or more, where every block then has a unit of its own (the model above knows no memory, which is
+// what such products wait for) and eight ranges leave a third of the units idle (fewer than 24 quarter tiles) or read a matrix of few rows or columns
+// twice over (more than 32).  us, eight / up to sixteen ranges, NN: 130 x 1024 x 50264 85 / 54, 48 x 2048 x 50264 78 / 49, 172 x 4096 x 50264, just
+// written by another product, 140 / 102; what the lines keep out: 200 x 1536 x 33000 46 / 61, 128 x 4096 x 36864 67 / 72, 136 x 2048 x 45056 57 / 64,
+// 1024 x 1024 x 57344 118 / 119, and, with shorter ranges, 80 x 4096 x 11008 25 / 27, 128 x 4096 x 28672 57 / 73.
 struct Plan { int bm, bn, splits, cut, cut_parts; };
 
-Plan plan_bf16(int M, int N, int K, bool may_split) {
+enum { ONE_RANGE = 1, FEW_RANGES = 8, MOST_RANGES = 16 };
+
+Plan plan_bf16(int M, int N, int K, int most_ranges) {
   struct Tile { int bm, bn, per_cu; double idle_us, full_us; };
   static const Tile tiles[] = {{256, 256, 1, 0.80, 1.42}, {128, 256, 1, 0.55, 0.83}, {128, 128, 2, 0.35, 0.90}};
-  const int slabs = (K + BK - 1) / BK;
+  const int slabs = (K + BK - 1) / BK, quarters = ((M + 127) / 128) * ((N + 127) / 128);
+  const bool long_k = quarters < 24 || (quarters > 32 && (M < N ? M : N) <= 256);
   Plan best{256, 256, 1, 0, 1};
   double best_us = 1e30;
   for (const Tile& t : tiles) {
     const int64_t tiles_mn = (int64_t)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
-    for (int s = 1; s <= (may_split ? 8 : 1); s++) {
-      if (s > 1 && slabs < 4 * s) break;
+    for (int s = 1; s <= most_ranges; s += s < 8 ? 1 : 4) {
+      if (s > 1 && slabs < (s > 8 ? 40 : 4) * s) break;
+      if (s > 8 && !(long_k && tiles_mn * s <= 256)) break;
       const int64_t slots = 256 * t.per_cu, full = tiles_mn * s / slots, rest = tiles_mn * s % slots;
       double per_slab = full * t.full_us;
       if (rest) per_slab += t.idle_us + (t.full_us - t.idle_us) * rest / slots;
@@ -262,11 +272,14 @@ Plan plan_bf16(int M, int N, int K, bool may_split) {
   return best;
 }
 
-// a caller without room for the partial tiles gets the best plan that needs none
+// a caller with less room for the partial tiles gets the best plan of those with at most eight ranges, or of those with one
 Plan plan_with_workspace(int M, int N, int K, const void* workspace, size_t workspace_bytes) {
-  if (workspace == nullptr || !ody_aligned16(workspace)) return plan_bf16(M, N, K, false);
-  const Plan pl = plan_bf16(M, N, K, true);
-  return (size_t)pl.splits * M * N * sizeof(float) <= workspace_bytes ? pl : plan_bf16(M, N, K, false);
+  if (workspace != nullptr && ody_aligned16(workspace))
+    for (int most : {MOST_RANGES, FEW_RANGES}) {
+      const Plan pl = plan_bf16(M, N, K, most);
+      if ((size_t)pl.splits * M * N * sizeof(float) <= workspace_bytes) return pl;
+    }
+  return plan_bf16(M, N, K, ONE_RANGE);
 }
 
 bool vec16(const void* p, int64_t ld) { return ody_aligned16(p) && ld % 8 == 0; }
@@ -328,7 +341,7 @@ extern "C" size_t ody_gemm_workspace_bytes(int op, int M, int N, int K, int dtyp
   if (dtype == ODY_F32) return ody_gemm_f32_workspace(M, N, K);
   if (dtype != ODY_BF16) return 0;
   if (op == ODY_GEMM_NT && ody_gemm_skinny_ok(EPI_NONE, M, N)) return 0;
-  const int splits = plan_bf16(M, N, K, true).splits;
+  const int splits = plan_bf16(M, N, K, MOST_RANGES).splits;
   return splits > 1 ? (size_t)splits * M * N * sizeof(float) : 0;
 }
 
@@ -475,7 +488,7 @@ int linear_swiglu_fused(const void* x, const void* w_gate_up, void* gate_up, voi
     return !launch ? ODY_OK : ody_launch_gemm_skinny(EPI_SWIGLU_FWD, static_cast<const bf16*>(x), static_cast<const bf16*>(w_gate_up),
                                                      static_cast<bf16*>(gate_up), nullptr, T, 2 * I, K, ldx, ldw, ld_gu, 0, ep, st);
   if (I % 128 == 0 && tile_pitch_ok(ODY_GEMM_NT, ldx, ldw) && (int64_t)I * ldw < (1ll << 29))
-    return !launch ? ODY_OK : launch_tiles(ODY_GEMM_NT, EPI_SWIGLU_FWD, plan_bf16(T, 2 * I, K, false),
+    return !launch ? ODY_OK : launch_tiles(ODY_GEMM_NT, EPI_SWIGLU_FWD, plan_bf16(T, 2 * I, K, ONE_RANGE),
                                            fused_args(x, w_gate_up, gate_up, T, 2 * I, K, ldx, ldw, ld_gu, ep), st);
   return ODY_ERR_UNSUPPORTED;
 }
@@ -570,7 +583,7 @@ extern "C" int ody_linear_dgrad_swiglu(const void* dy, const void* w_down, const
   if (dtype == ODY_BF16 && I % 128 == 0 && K % 8 == 0 && tile_pitch_ok(ODY_GEMM_NN, ld_dy, ldw) && vec16(dy, ld_dy) &&
       vec16(w_down, ldw) && vec16(gate_up, ld_gu) && vec16(d_gate_up, ld_dgu)) {
     const GemmEpi ep{static_cast<const bf16*>(gate_up), nullptr, ld_gu, 0, I};
-    return launch_tiles(ODY_GEMM_NN, EPI_SWIGLU_BWD, plan_bf16(T, I, K, false),
+    return launch_tiles(ODY_GEMM_NN, EPI_SWIGLU_BWD, plan_bf16(T, I, K, ONE_RANGE),
                         fused_args(dy, w_down, d_gate_up, T, I, K, ld_dy, ldw, ld_dgu, ep), st);
   }
   const size_t need = (size_t)T * I * (dtype == ODY_BF16 ? 2 : 4);

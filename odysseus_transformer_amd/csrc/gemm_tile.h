@@ -204,11 +204,12 @@ __device__ __forceinline__ void gemm_tile_block(const Args& p, int m0, int tn, i
 
   // slabs [s0, s0 + nk) of the K range
   const int slabs = (p.K + BK - 1) / BK;
-  int s0 = 0, nk = slabs;
+  int s0 = 0, nk = slabs, k_end = p.K;
   if (SPLITK) {
     const int per = (slabs + (int)gridDim.y - 1) / (int)gridDim.y;
     s0 = blockIdx.y * per;
     nk = max(0, min(slabs - s0, per));
+    k_end = min(p.K, (s0 + nk) * BK);
   }
 
   Mover<A_KC, HALF, 4> ma;
@@ -216,13 +217,13 @@ __device__ __forceinline__ void gemm_tile_block(const Args& p, int m0, int tn, i
   int j0 = EPI == EPI_SWIGLU_FWD ? tn * (BN / 2) : 0;   // first column of h
   auto aim_a = [&](int lane) {
     if (A_KC) ma.aim(wn, lane, p.lda, p.A + (int64_t)m0 * p.lda, s0, p.K, [&](int r) { return min(m0 + wm * HALF + r, p.M - 1) - m0; });
-    else ma.aim(wn, lane, p.lda, p.A + m0, s0, p.K, [&](int col) { return min(m0 + wm * HALF + col, p.M - 8) - m0; });
+    else ma.aim(wn, lane, p.lda, p.A + m0, s0, k_end, [&](int col) { return min(m0 + wm * HALF + col, p.M - 8) - m0; });
   };
   auto aim_b = [&](int lane) {
     if (EPI == EPI_SWIGLU_FWD)
       mb.aim(wave, lane, p.ldb, p.B, s0, p.K, [&](int r) { return min(j0 + (r & (BN / 2 - 1)), p.ep.I - 1) + (r < BN / 2 ? 0 : p.ep.I); });
     else if (B_KC) mb.aim(wave, lane, p.ldb, p.B + (int64_t)n0 * p.ldb, s0, p.K, [&](int r) { return min(n0 + r, p.N - 1) - n0; });
-    else mb.aim(wave, lane, p.ldb, p.B + n0, s0, p.K, [&](int col) { return min(n0 + col, p.N - 8) - n0; });
+    else mb.aim(wave, lane, p.ldb, p.B + n0, s0, k_end, [&](int col) { return min(n0 + col, p.N - 8) - n0; });
   };
   aim_a(lane);
   aim_b(lane);
@@ -468,7 +469,7 @@ __device__ __forceinline__ void gemm_tile_block(const Args& p, int m0, int tn, i
       slot = slot == 2 ? 0 : slot + 1;
       stage ^= 1;
     };
-    // loads past the range repeat its last slab, or go on behind it (not KC; beyond K they fetch nothing): in bounds, and nobody reads them
+    // loads past the range repeat its last slab (KC) or fetch nothing: in bounds, and nobody reads them
     if constexpr (!ROUNDS) {
       for (int kt = 0; kt < nk; kt++) slab(min(kt + 1, nk - 1), min(kt + 2, nk - 1), std::false_type{});
     } else {

@@ -369,3 +369,31 @@ def test_few_rows_around_the_lines_between_instances(what, N, K, M, dev):
         a, b = ref[:, :n_rot * 128].reshape(M, n_rot, 2, 64).unbind(2)
         ref[:, :n_rot * 128] = torch.stack([a * cos - b * sin, b * cos + a * sin], 2).reshape(M, -1)
         assert rel_err(ops.linear_rope(x, w, table, n_rot, 128), ref) <= TOL_BF16
+
+
+@pytest.mark.parametrize("op", ["nt", "nn", "tn"])
+@pytest.mark.parametrize("M,N,K,ranges", [(8, 264, 40960, 16), (72, 1032, 30720, 12), (136, 1280, 41032, 16), (168, 4096, 40968, 16), (40, 392, 30656, 8),
+                                          (128, 3072, 40960, 8)], ids=lambda v: str(v))
+def test_ranges_of_a_long_k(op, M, N, K, ranges, dev):
+    """More than eight ranges of K at their lines (`ranges`: the most there may be; fewer rows than a tile, a last slab that K does not fill, a last range
+    shorter than the others), and a workspace with room for eight ranges, for one, and for none: the same product each time."""
+    from odysseus_transformer_amd import _lib, ops
+    print(f"long K {op} {M}x{N}x{K}", flush=True)
+    if op == "nt" and M <= 16:
+        pytest.skip("kernels for few rows have no ranges")
+    code, lib = {"nt": ops.GEMM_NT, "nn": ops.GEMM_NN, "tn": ops.GEMM_TN}[op], _lib.load()
+    a = randn((K, M) if op == "tn" else (M, K), 61, dtype=torch.bfloat16).to(dev)
+    b = randn((N, K) if op == "nt" else (K, N), 62, std=0.05, dtype=torch.bfloat16).to(dev)
+    ref = (a.double().t() if op == "tn" else a.double()) @ (b.double().t() if op == "nt" else b.double())
+    need = lib.ody_gemm_workspace_bytes(code, M, N, K, _lib.ODY_BF16)
+    assert need <= ranges * M * N * 4
+    assert need > 8 * M * N * 4 or ranges == 8
+    assert rel_err(ops.gemm(code, a, b), ref) <= TOL_BF16
+    for room in (need, 8 * M * N * 4, need // ranges):
+        ws = torch.full((room // 4 + 64,), float("nan"), dtype=torch.float32, device=dev)
+        y = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device=dev)
+        rc = lib.ody_gemm(code, a.data_ptr(), b.data_ptr(), y.data_ptr(), None, M, N, K, a.stride(0), b.stride(0), N, 0, _lib.ODY_BF16, ws.data_ptr(), room,
+                          torch.cuda.current_stream().cuda_stream)
+        assert rc == 0
+        assert rel_err(y, ref) <= TOL_BF16
+        assert torch.isnan(ws[room // 4:]).all()
