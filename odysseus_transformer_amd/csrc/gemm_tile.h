@@ -84,7 +84,9 @@ __device__ __forceinline__ int lane_anew() {
 // slab s of K, behind slab s - 1 (KC: any).
 //
 // Not KC: what changes from slab to slab is scalar, the slab's address; chunks that K does not reach are sorted out behind a branch (`cut`, in front of
-// the load), and not in every load, because the transposing reads leave the memory phase no room.
+// the load of a slab that K fills in part), and not in every load, because the transposing reads leave the memory phase no room.  A slab behind K's end has a
+// range of no bytes instead: with `cut` there too, products of one slab, most of whose loads are such, took 1 to 4 % longer than with a mask in every load (TN, us, mask /
+// `cut` / range: 32000 x 2048 x 64 35.2 / 36.4 / 35.0, x 24 35.7 / 36.7 / 35.1, 4096 x 4096 x 24 9.9 / 10.1 / 9.8; 1024 x 2816 x 128 5.16 / 4.98 / 4.69; K = 4096 the same).
 // KC: slab address and mask anew in every load.  The other form is 1 to 2.5 % slower there (NT, us, this / other: 8192^3 683 / 702, zeros 476 / 487;
 // 4096 x 11008 x 4096, zeros, 184 / 188), although it takes fewer instructions.
 template <bool KC, int W, int NW>
@@ -107,8 +109,9 @@ struct Mover {
       else v[j] = (unsigned)(2 * ((int64_t)r * ld + row_of(8 * (p ^ (2 * group_perm<W>(r))))));
     }
   }
+  __device__ __forceinline__ bool partial() const { return !KC && (unsigned)(left - 1) < BK - 1; }   // 0 < left < BK
   __device__ __forceinline__ void cut(int wv) {
-    if (KC || left >= BK) return;
+    if (!partial()) return;
     const int k = wv * NINS * RPI + lane_anew() / LPR;
 #pragma unroll
     for (int j = 0; j < NINS; j++)
@@ -116,7 +119,7 @@ struct Mover {
   }
   __device__ __forceinline__ void load(int s, bf16* stage, int wv, int lane, int64_t ld) {
     const bf16* slab = KC ? base + (int64_t)s * BK : base;
-    auto rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16*>(slab), (short)0, 0x7fffffff, 0x00020000);
+    auto rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16*>(slab), (short)0, KC || left > 0 ? 0x7fffffff : 0, 0x00020000);
 #pragma unroll
     for (int j = 0; j < NINS; j++) {
       const unsigned off = !KC || 8 * ((lane & 7) ^ (lane >> 3)) < left - s * BK ? v[j] : PAST_END;
@@ -405,7 +408,7 @@ __device__ __forceinline__ void gemm_tile_block(const Args& p, int m0, int tn, i
           else read_tr<64 * HALF, 72 * HALF>(at, fa.lo[1][a], fa.hi[1][a]);
         }
       };
-      if (!(A_KC && B_KC) && min(A_KC ? BK : ma.left, B_KC ? BK : mb.left) < BK) cut();
+      if (ma.partial() || mb.partial()) cut();
       // ---- memory phase: this slab's fragments; A of the next slab, B of the one after (its stage was read last two phases ago)
       ODY_FENCE();
 #pragma unroll

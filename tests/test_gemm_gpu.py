@@ -322,7 +322,7 @@ def test_several_tiles_a_block_with_an_epilogue(what, M, K, dev):
 
 @pytest.mark.parametrize("op", ["nn", "tn"])
 @pytest.mark.parametrize("M,N,K", [(72, 136, 8), (256, 256, 56), (264, 512, 72), (136, 128, 120), (1000, 264, 1544), (264, 1032, 4104), (8200, 4616, 136),
-                                   (5640, 6152, 4168)], ids=lambda v: str(v))
+                                   (5640, 6152, 4168), (264, 520, 64), (8200, 4616, 64), (136, 264, 128)], ids=lambda v: str(v))
 def test_slabs_that_k_does_not_fill(op, M, N, K, dev):
     """Operands with rows of K inside buffers whose other rows and columns are not numbers: one slab, a whole number of them and a part, K in ranges, one tile and
     several a block (short K and long).  What lies behind K is read as zeros and by nobody."""
