@@ -93,3 +93,11 @@ def randn(shape, seed, std=1.0, dtype=torch.float32):
 @pytest.fixture(scope="session")
 def dev():
     return torch.device("cuda:0")
+
+
+def device_kernels(fn):
+    """fn() and the names, template arguments and all, of the kernels that it launched: what tells the instances of one launch name apart."""
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as prof:
+        out = fn()
+        torch.cuda.synchronize()
+    return out, [e.key for e in prof.key_averages()]

@@ -2,7 +2,7 @@
 import pytest
 import torch
 
-from conftest import TOL_BF16, TOL_F32, randn, rel_err
+from conftest import TOL_BF16, TOL_F32, device_kernels, randn, rel_err
 import odysseus_oracle as oracle
 
 pytestmark = pytest.mark.gpu
@@ -340,12 +340,7 @@ def test_slabs_that_k_does_not_fill(op, M, N, K, dev):
     assert rel_err(y, (a.float().t() if op == "tn" else a.float()) @ b.float()) <= TOL_BF16
 
 
-@pytest.mark.parametrize("M", [1, 4, 5, 8, 9, 16])
-@pytest.mark.parametrize("N,K", [(4992, 72), (5120, 2056), (5120, 2048), (16256, 136), (16384, 72)], ids=lambda v: str(v))
-@pytest.mark.parametrize("what", ["plain", "residual", "swiglu", "rope"])
-def test_few_rows_around_the_lines_between_instances(what, N, K, M, dev):
-    """312 and 320, 1016 and 1024 groups of 16 rows of W, rows of A on both sides of 4 and 8, K on both sides of 2048: one or two groups a block on 4 or 8
-    wavefronts, the pairs of an epilogue inside a group or in two."""
+def _few_rows(what, N, K, M, dev):
     from odysseus_transformer_amd import ops
     print(f"what={what} M={M} N={N} K={K}", flush=True)
     dt = torch.bfloat16
@@ -371,16 +366,43 @@ def test_few_rows_around_the_lines_between_instances(what, N, K, M, dev):
         assert rel_err(ops.linear_rope(x, w, table, n_rot, 128), ref) <= TOL_BF16
 
 
-@pytest.mark.parametrize("op", ["nt", "nn", "tn"])
-@pytest.mark.parametrize("M,N,K,ranges", [(8, 264, 40960, 16), (72, 1032, 30720, 12), (136, 1280, 41032, 16), (168, 4096, 40968, 16), (40, 392, 30656, 8),
-                                          (128, 3072, 40960, 8)], ids=lambda v: str(v))
+@pytest.mark.parametrize("M", [1, 4, 5, 8, 9, 16])
+@pytest.mark.parametrize("N,K", [(4992, 72), (5120, 2056), (5120, 2048), (16256, 136), (16384, 72)], ids=lambda v: str(v))
+@pytest.mark.parametrize("what", ["plain", "residual", "swiglu", "rope"])
+def test_few_rows_around_the_lines_between_instances(what, N, K, M, dev):
+    """312 and 320, 1016 and 1024 groups of 16 rows of W, rows of A on both sides of 4 and 8, K on both sides of 2048: one or two groups a block on 4 or 8
+    wavefronts, the pairs of an epilogue inside a group or in two."""
+    _few_rows(what, N, K, M, dev)
+
+
+# groups of 16 rows of W a block, steps of K in flight, wavefronts: on both sides of every line of the choice
+@pytest.mark.parametrize("what,N,K,M,instance", [
+    ("plain", 2048, 1024, 9, "1, 8, 4"), ("plain", 2048, 1032, 9, "1, 4, 8"), ("residual", 2048, 2048, 9, "1, 4, 8"), ("plain", 2048, 2056, 9, "1, 8, 4"),
+    ("plain", 4080, 4104, 2, "1, 4, 8"), ("plain", 4096, 4104, 2, "1, 8, 4"), ("plain", 4096, 4096, 2, "1, 4, 8"), ("plain", 4096, 4104, 1, "1, 4, 8"),
+    ("residual", 4096, 4096, 5, "1, 4, 8"), ("residual", 4096, 4104, 5, "1, 8, 4"), ("plain", 4080, 4104, 5, "1, 8, 4"), ("residual", 4112, 72, 5, "1, 8, 4"),
+    ("residual", 4112, 2056, 5, "2, 4, 4"), ("plain", 4112, 72, 9, "2, 4, 4"), ("rope", 4096, 72, 4, "1, 4, 8"), ("rope", 4224, 2048, 4, "2, 8, 8"),
+    ("rope", 4224, 2048, 8, "2, 8, 8"), ("rope", 4224, 2048, 9, "2, 8, 8"), ("swiglu", 4128, 2048, 8, "2, 8, 8"), ("swiglu", 4128, 2048, 9, "2, 4, 4"),
+    ("rope", 4224, 2056, 4, "2, 8, 8"), ("swiglu", 4224, 2056, 5, "2, 4, 4"), ("rope", 7168, 2056, 1, "2, 8, 8"), ("rope", 7296, 2056, 1, "1, 4, 8"),
+    ("swiglu", 7200, 2056, 4, "1, 4, 8"), ("rope", 8192, 136, 16, "2, 8, 8"), ("rope", 8320, 136, 1, "1, 8, 4"), ("swiglu", 8192, 72, 1, "2, 8, 8"),
+    ("swiglu", 8224, 72, 3, "1, 8, 4"), ("plain", 8192, 72, 4, "1, 4, 8"), ("plain", 8208, 72, 4, "1, 8, 4"), ("plain", 8208, 2056, 16, "1, 8, 4"),
+    ("plain", 12784, 72, 9, "1, 8, 4"), ("plain", 12800, 72, 9, "2, 4, 4"), ("residual", 12800, 72, 8, "1, 8, 4"), ("residual", 12800, 2056, 8, "2, 4, 4")],
+    ids=lambda v: str(v))
+def test_few_rows_on_the_instance_of_their_sizes(what, N, K, M, instance, dev):
+    _, ran = device_kernels(lambda: _few_rows(what, N, K, M, dev))
+    ran = [name for name in ran if "gemm_skinny_kernel<" in name]
+    assert ran and all(f"gemm_skinny_kernel<{instance}, " in name for name in ran), ran
+
+
+LONG_K = [(8, 264, 40960, 16), (72, 1032, 30720, 12), (136, 1280, 41032, 16), (168, 4096, 40968, 16), (40, 392, 30656, 8), (128, 3072, 40960, 8)]
+
+
+# (NT products of 16 rows and fewer have kernels of their own, without ranges)
+@pytest.mark.parametrize("op,M,N,K,ranges", [(op, *c) for op in ("nt", "nn", "tn") for c in LONG_K if op != "nt" or c[0] > 16], ids=lambda v: str(v))
 def test_ranges_of_a_long_k(op, M, N, K, ranges, dev):
     """More than eight ranges of K at their lines (`ranges`: the most there may be; fewer rows than a tile, a last slab that K does not fill, a last range
     shorter than the others), and a workspace with room for eight ranges, for one, and for none: the same product each time."""
     from odysseus_transformer_amd import _lib, ops
     print(f"long K {op} {M}x{N}x{K}", flush=True)
-    if op == "nt" and M <= 16:
-        pytest.skip("kernels for few rows have no ranges")
     code, lib = {"nt": ops.GEMM_NT, "nn": ops.GEMM_NN, "tn": ops.GEMM_TN}[op], _lib.load()
     a = randn((K, M) if op == "tn" else (M, K), 61, dtype=torch.bfloat16).to(dev)
     b = randn((N, K) if op == "nt" else (K, N), 62, std=0.05, dtype=torch.bfloat16).to(dev)
@@ -389,7 +411,7 @@ def test_ranges_of_a_long_k(op, M, N, K, ranges, dev):
     assert need <= ranges * M * N * 4
     assert need > 8 * M * N * 4 or ranges == 8
     assert rel_err(ops.gemm(code, a, b), ref) <= TOL_BF16
-    for room in (need, 8 * M * N * 4, need // ranges):
+    for room in (need, 8 * M * N * 4, need // ranges, 0):
         ws = torch.full((room // 4 + 64,), float("nan"), dtype=torch.float32, device=dev)
         y = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device=dev)
         rc = lib.ody_gemm(code, a.data_ptr(), b.data_ptr(), y.data_ptr(), None, M, N, K, a.stride(0), b.stride(0), N, 0, _lib.ODY_BF16, ws.data_ptr(), room,
