@@ -425,6 +425,18 @@ def _flash_inputs(dev, dtype=torch.bfloat16, L=197, hq=8, hkv=2, D=128, needs=(T
     return [t.requires_grad_(n) for t, n in zip((q, k, v), needs)]
 
 
+class _NoGradient(torch.autograd.Function):
+    """Passes its input on and no gradient back."""
+
+    @staticmethod
+    def forward(ctx, x):
+        return x.clone()
+
+    @staticmethod
+    def backward(ctx, grad):
+        return None
+
+
 @pytest.mark.parametrize("dtype,D", [(torch.bfloat16, 128), (torch.bfloat16, 64), (torch.float32, 64)], ids=["bf16_128", "bf16_64", "f32_64"])
 @pytest.mark.parametrize("causal", [True, False])
 @pytest.mark.parametrize("needs", [(True, True, True), (False, True, False), (True, False, False)], ids=lambda n: "".join("nq"[x] for x in n))
@@ -442,6 +454,8 @@ def test_attention_routine_as_a_node_of_its_own(dtype, D, causal, needs, dev, mo
         for dout in (randn(out.shape, 72, dtype=dtype).to(dev), randn((2, D, 197, 8), 73, dtype=dtype).to(dev).permute(0, 2, 3, 1),
                      torch.ones((), dtype=dtype, device=dev).expand(out.shape)):
             got += torch.autograd.grad(out, inputs, dout, retain_graph=True)
+        got += torch.autograd.grad(_NoGradient.apply(out).sum(), inputs)
+        assert all(not g.any() for g in got[-len(inputs):])
         return got
 
     here, there, taken = _both(monkeypatch, run)
