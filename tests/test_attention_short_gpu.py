@@ -3,7 +3,7 @@ import pytest
 import torch
 
 import odysseus_oracle as oracle
-from conftest import TOL_BF16, TOL_LSE, assert_parity, randn, rel_err
+from conftest import TOL_BF16, TOL_LSE, assert_parity, device_kernels, randn, rel_err
 
 pytestmark = pytest.mark.gpu
 
@@ -126,31 +126,43 @@ def test_causal_backward_of_many_blocks(L, H, short):
         assert_parity(a[:, :, :2], b, TOL_BF16, n, 1e-3)
 
 
+def _instance(names, kernel):
+    """The one instance of `kernel` among the launched ones: its template arguments, "" if it has none, None if it did not run."""
+    ran = {n.split(kernel, 1)[1].split("(", 1)[0] for n in names if kernel in n}
+    assert len(ran) <= 1, names
+    return ran.pop() if ran else None
+
+
 # the forward's ring: fewer and more tiles than it holds, odd and even counts, ragged last sub-tiles, wavefronts and groups without a key, blocks without
 # one, and calls on either side of its lines
-@pytest.mark.parametrize("case", [(1, 512, 512, 2, 1, True), (1, 511, 511, 2, 2, True), (1, 61, 513, 3, 3, True), (1, 700, 545, 2, 2, True), (2, 900, 577, 2, 1, True),
-                                  (1, 1023, 1023, 4, 4, True), (1, 130, 320, 2, 2, False), (1, 130, 319, 2, 2, False), (1, 257, 353, 2, 1, False), (1, 97, 991, 2, 2, False),
-                                  (1, 2561, 4100, 7, 7, True), (1, 2049, 1536, 17, 17, True)], ids=lambda c: "B%d_Lq%d_Lk%d_H%d_%d_c%d" % c)
+@pytest.mark.parametrize("case,ring", [
+    ((1, 512, 512, 2, 1, True), True), ((1, 511, 511, 2, 2, True), False), ((1, 61, 513, 3, 3, True), True), ((1, 700, 545, 2, 2, True), True),
+    ((2, 900, 577, 2, 1, True), True), ((1, 1023, 1023, 4, 4, True), True), ((1, 130, 320, 2, 2, False), True), ((1, 130, 319, 2, 2, False), False),
+    ((1, 257, 353, 2, 1, False), True), ((1, 97, 991, 2, 2, False), True), ((1, 2561, 4100, 7, 7, True), True), ((1, 2049, 1536, 17, 17, True), True),
+    ((1, 2049, 1535, 17, 17, True), False), ((1, 1664, 320, 16, 8, False), True), ((1, 1665, 959, 15, 5, False), False), ((1, 1665, 960, 15, 15, False), True)],
+    ids=lambda c: "B%d_Lq%d_Lk%d_H%d_%d_c%d" % c if isinstance(c, tuple) else "ring" if c else "loop")
 @pytest.mark.parametrize("late", [1.0, 40.0], ids=["unit", "outgrown"])
-def test_forward_ring(case, late):
+def test_forward_ring(case, ring, late):
     from odysseus_transformer_amd import ops
     B, Lq, Lk, Hq, Hkv, causal = case
     print(f"case={case} late={late}", flush=True)
     q, k, v, _ = _inputs(B, Lq, Lk, Hq, Hkv, 7 * Lq + Lk)
     k[:, Lk // 2:] *= late
-    (o, lse), ran = _run(lambda: ops.attn_fwd(q.cuda(), k.cuda(), v.cuda(), causal=causal))
-    assert "attn_fwd_short" in ran, ran
+    (o, lse), ran = device_kernels(lambda: ops.attn_fwd(q.cuda(), k.cuda(), v.cuda(), causal=causal))
+    assert _instance(ran, "attn_fwd_short") == ("_ring_kernel" if ring else "_kernel"), ran
     o_ref, lse_ref = oracle.attention_fwd(q.float(), k.float(), v.float(), causal=causal)
     assert_parity(o, o_ref, TOL_BF16, "o")
     assert torch.allclose(lse.cpu(), lse_ref, atol=TOL_LSE, rtol=TOL_LSE)
 
 
 # the backward's rings likewise: either side of their line, in one direction only, few and many tiles, wavefronts without a query or a key
-@pytest.mark.parametrize("case", [(1, 511, 512, 2, 1, True), (1, 511, 511, 2, 2, True), (1, 33, 545, 3, 3, True), (1, 700, 31, 2, 2, True), (2, 900, 577, 2, 1, True),
-                                  (1, 130, 513, 2, 2, False), (1, 577, 65, 4, 1, False), (1, 1023, 1025, 4, 4, True), (1, 97, 991, 2, 2, False),
-                                  (1, 3401, 3400, 1, 1, True), (1, 1601, 3500, 3, 3, False), (1, 959, 959, 17, 17, True), (1, 961, 960, 17, 17, True)],
-                         ids=lambda c: "B%d_Lq%d_Lk%d_H%d_%d_c%d" % c)
-def test_backward_rings(case):
+@pytest.mark.parametrize("case,ring", [
+    ((1, 511, 512, 2, 1, True), True), ((1, 511, 511, 2, 2, True), False), ((1, 33, 545, 3, 3, True), True), ((1, 700, 31, 2, 2, True), True),
+    ((2, 900, 577, 2, 1, True), True), ((1, 130, 513, 2, 2, False), True), ((1, 577, 65, 4, 1, False), True), ((1, 1023, 1025, 4, 4, True), True),
+    ((1, 97, 991, 2, 2, False), True), ((1, 3401, 3400, 1, 1, True), True), ((1, 1601, 3500, 3, 3, False), True), ((1, 959, 959, 17, 17, True), False),
+    ((1, 961, 960, 17, 17, True), True)],
+    ids=lambda c: "B%d_Lq%d_Lk%d_H%d_%d_c%d" % c if isinstance(c, tuple) else "ring" if c else "loop")
+def test_backward_rings(case, ring):
     from odysseus_transformer_amd import ops
     B, Lq, Lk, Hq, Hkv, causal = case
     print(f"case={case}", flush=True)
@@ -159,8 +171,8 @@ def test_backward_rings(case):
     refs = oracle.attention_bwd(q.float(), k.float(), v.float(), o_ref, lse_ref, do.float(), causal=causal)
     qg, kg, vg, dog = (t.cuda() for t in (q, k, v, do))
     o, lse = ops.attn_fwd(qg, kg, vg, causal=causal)
-    grads, ran = _run(lambda: ops.attn_bwd(qg, kg, vg, o, lse, dog, causal=causal))
-    assert "attn_bwd_short" in ran, ran
+    grads, ran = device_kernels(lambda: ops.attn_bwd(qg, kg, vg, o, lse, dog, causal=causal))
+    assert _instance(ran, "attn_bwd_short_kernel") == f"<{str(Hq != Hkv).lower()}, {str(ring).lower()}>", ran
     for got, ref, name in zip(grads, refs, ("dq", "dk", "dv")):
         assert_parity(got, ref, TOL_BF16, name, 1e-3)
     assert all(torch.equal(a, b) for a, b in zip(grads, ops.attn_bwd(qg, kg, vg, o, lse, dog, causal=causal)))
@@ -189,3 +201,34 @@ def test_rows_beyond_a_tiles_offsets_go_to_the_other_kernels(stride):
     o_ref, lse_ref = oracle.attention_fwd(q.float(), k.float(), v.float(), causal=True)
     assert_parity(o, o_ref, TOL_BF16, "o")
     assert torch.allclose(lse.cpu(), lse_ref, atol=TOL_LSE, rtol=TOL_LSE)
+
+
+@pytest.mark.parametrize("stride", [(1 << 24) - 16, (1 << 24) - 8], ids=str)
+@pytest.mark.parametrize("far", ["keys", "queries"])
+def test_rings_over_rows_far_apart(far, stride):
+    """Keys and values, or queries and the gradient of the output, with the last row stride whose tile fits 32-bit offsets and the first one beyond: the
+    rings, and the kernels with 64-bit ones."""
+    from odysseus_transformer_amd import ops
+    Lq, Lk = (130, 545) if far == "keys" else (545, 130)
+    near = stride < (1 << 24) - 8
+    print(f"{far=} {stride=}", flush=True)
+    q, k, v, do = _inputs(1, Lq, Lk, 1, 1, 5)
+    o_ref, lse_ref = oracle.attention_fwd(q.float(), k.float(), v.float(), causal=False)
+    refs = oracle.attention_bwd(q.float(), k.float(), v.float(), o_ref, lse_ref, do.float(), causal=False)
+    rows = max(Lq, Lk)
+    apart = torch.empty(stride * (rows - 1) + 256, dtype=torch.bfloat16, device="cuda")
+    pair = [apart.as_strided((1, rows, 1, 128), (0, stride, 128, 1), 128 * n).copy_(t) for n, t in enumerate((k, v) if far == "keys" else (q, do))]
+    q, k, v, do = (t.cuda() for t in (q, k, v, do))
+    if far == "keys":
+        k, v = pair
+        (o, lse), ran = device_kernels(lambda: ops.attn_fwd(q, k, v, causal=False))
+        assert _instance(ran, "attn_fwd_short") == ("_ring_kernel" if near else None), ran
+        assert_parity(o, o_ref, TOL_BF16, "o")
+        assert torch.allclose(lse.cpu(), lse_ref, atol=TOL_LSE, rtol=TOL_LSE)
+    else:
+        q, do = pair
+    new = {n: torch.empty((1, L, 1, 128), dtype=torch.bfloat16, device="cuda") for n, L in (("dq", Lq), ("dk", Lk), ("dv", Lk))}
+    grads, ran = device_kernels(lambda: ops.attn_bwd(q, k, v, o_ref.bfloat16().cuda(), lse_ref.cuda(), do, causal=False, **new))
+    assert _instance(ran, "attn_bwd_short_kernel") == f"<false, {str(near).lower()}>", ran
+    for got, ref, name in zip(grads, refs, ("dq", "dk", "dv")):
+        assert_parity(got, ref, TOL_BF16, name, 1e-3)
