@@ -1104,7 +1104,7 @@ int ody_launch_attn_bwd_pipe(const AttnParams& p, void* workspace, hipStream_t s
   };
   const int qparts = query_parts(p.B, p.Lq, p.Lk, p.Hq, p.Hkv, p.causal != 0);
   // dK and dV are the same bits whether dS is kept or not; where that is a choice (rows in multiples of 256), a cut query range keeps a call on
-  // the kernels below.  It costs what the others gain: causal, 4 heads, L = 2048 109 us here, 78 there, 8 heads, L = 3584 176 and 135
+  // the kernels below.  It costs what the others gain: causal, 4 heads, L = 2048 109 us here, 65 there, 8 heads, L = 3584 178 and 124
   const bool same_sums = qparts == 1 || ody_attn_bwd_pipe_ds_bytes(p.B, p.Lq, p.Lk, p.Hq, p.causal) == 0;
   // rows too far apart for the 32-bit offsets of a tile below: that kernel's are 64 bits wide
   const bool far = std::max(std::max(p.sq.l, p.sdo.l), std::max(p.sk.l, p.sv.l)) >= TILE_MAX_STRIDE;

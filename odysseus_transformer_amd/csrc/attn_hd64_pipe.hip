@@ -673,8 +673,9 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_hd64_dkdv_pipe_kernel(const A
 
 //   S^T = K Q^T     dP^T = V dO^T - delta     dQ^T += K^T dS^T       lane = query column
 //
-// As above, 4 wavefronts of 32 queries, two per SIMD (194 registers).  Bound: power, at 1.7 GHz, and the vector pipe (exp, products with P and dP,
-// conversions: 416 cycles beside 384 of products per 32 x 32 sub-tile; takes 590), so addresses move once a tile and not with each read.
+// As above, 4 wavefronts of 32 queries, two per SIMD (194 registers).  Bound: power, and the vector pipe (exp, products with P and dP, conversions: 416 cycles
+// beside 384 of products per 32 x 32 sub-tile; takes 600), so addresses move once a tile and not with each read.  Counters, 16 heads, L = 8192, full: 1.63 GHz, matrix
+// pipe 64 % busy, vector 59 %, LDS 43 %.
 // dQ alone, before (the same split without the order, three wavefronts per SIMD) / now, us: 16 heads, L = 8192, causal 212 / 194, full 417 / 370; 8 heads of it,
 // causal, 157 / 114; 4 x 32 heads of it 1629 / 1490; 16 heads, L = 4096, causal 83 / 61; on constant inputs, whose clock is not held down, full 348 / 255.
 constexpr int DQ_BM = 128, DQ_SLOTS = 4, DQ_STAGE = 2 * TILE;   // K and V tiles

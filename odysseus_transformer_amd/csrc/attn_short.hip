@@ -12,8 +12,8 @@
 // LDS reads and vector work of neighbouring sub-tiles under one another, loads four tiles ahead.
 //
 // What bounds it: latency of a chain of tiles in a block (2.2 us for 128 rows against 128 keys in the forward, 1.5 in the ring) on 1 block a unit.
-// Before / here, us, launches included: forward of 4 x 8 heads, L = 331, causal 19.8 / 12.7 (three launches / one), backward on 2 kv heads
-// 62.2 / 33.6 (five / three); 32 heads on 8, L = 1000, causal 41.5 / 20.4 and 119 / 74; 8 heads, L = 1500, full 43 / 23 and 148 / 68.
+// On the kernels for long sequences / here, us, launches included: forward of 4 x 8 heads, L = 331, causal 19.5 / 12.2 (three launches / one), backward on 2 kv
+// heads 66 / 33.5 (five / three); 32 heads on 8, L = 1000, causal 38.3 / 20.4 and 110 / 69; 8 heads, L = 1500, full 40 / 23.8 and 129 / 58.
 // Error against 64 bits, standard normal inputs, before / here: out 2.07e-3 / 1.96e-3 (4 x 8 heads, L = 331), 2.34e-3 / 2.31e-3 (640 rows,
 // full); dQ, dK, dV the same within the spread of one input to the next (2.5e-3, 2.5e-3, 2.3e-3).
 #include <algorithm>
@@ -1151,19 +1151,21 @@ inline int64_t row_blocks(int B, int L, int H) { return (int64_t)B * H * ((L + B
 
 }  // namespace
 
-// The lines were fitted against kernels that the present ones for long rows replaced, and timed again with these on shapes around them, launches and
-// all (596 forward, 556 backward: 1 to 128 heads, 64 to 8192 rows, a third with other key than query counts): 1.22 and 1.30 times as fast in the
-// geometric mean as without these kernels, 2 % behind the faster one everywhere.  Here / there, us:
+// The lines were fitted against kernels that the present ones, on both sides, have since replaced.  As they are now, 300 calls of each direction (1 to 64 heads, 64 to
+// 8192 rows, a third with other key than query counts) against both kernels for all of them: 1.30 and 1.49 times as fast in the geometric mean as without the kernels
+// here, 2.6 and 1.9 % behind the faster one in the mean, and by more than 5 % in 29 and 25 of the 300: forwards of up to 64 blocks from 1024 keys on, which the parts
+// keep (1.1 to 1.6 times), backwards that go to the other kernels for their tiles or for their cut query range (1.05 to 1.6).  Here / there, us:
 //   Beyond the line in blocks every compute unit has a block of 256 rows, whose tiles serve twice the rows: 32 heads, full, L = 1500: forward
-//   65 / 55, backward 189 / 156; causal, L = 3001: 101 / 87, 340 / 287.  Short causal rows leave those blocks a few tiles each, most of them under the
-//   mask, so that for them the line of the backward is further out: 4 x 24 heads, L = 820, 131 / 147, 4 x 32 heads, L = 683, 139.6 / 142.9, and
-//   beyond, 4 x 32 heads, L = 820, 175 / 177; L = 936 211 / 200; with longer rows 2 x 32 heads, L = 1200, 150 / 144, L = 1536 207 / 191.
-//   Beyond the line in tiles the other kernels cut the range of the long side into parts, backward, in the ring: 8 heads, full, L = 3000, 185 / 167, 2 heads,
-//   causal, L = 5000, 134 / 126; inside it 3 heads, L = 2500, causal or full, 75 / 121, 5 heads, L = 3000, full, 104 / 141.  The forward, in the ring: 4 heads, L = 4096, 46.5 / 47.6; 2 heads, L = 6000, 64 / 52; 3 heads,
-//   L = 8192, 84 / 77, 4 heads 91 / 94; 3 heads, L = 6000, full, 67 / 80; 12 heads, L = 4096, causal, 58 / 70; 6 heads, L = 12 000, 215 / 257.  Up to 64 blocks
-//   calls of 1024 keys and more stay with the parts, 300 queries on 8000 keys 82 / 65, also where they are short enough to be faster here, 8 heads, L = 1024,
-//   19 / 32; with fewer keys they do not (8 heads, L = 1000, 18.6 / 31.6).
-// One head, too, below the line: backward of 512 rows, causal, 28 / 67, of 1024 rows 44 / 96; two heads of 512 rows 28 / 68.
+//   52 / 51, backward 167 / 152; causal, L = 3001: 92 / 86, 310 / 285.  Short causal rows leave those blocks a few tiles each, most of them under the
+//   mask, so that for them the line of the backward is further out: 4 x 24 heads, L = 820, 133 / 147, 4 x 32 heads, L = 683, 142 / 144, and
+//   beyond, 4 x 32 heads, L = 820, 182 / 183; L = 936 220 / 204; with longer rows 2 x 32 heads, L = 1200, 147 / 148, L = 1536 203 / 195.
+//   Beyond the line in tiles the other kernels cut the range of the long side into parts, backward, in the ring: 8 heads, full, L = 3000, 182 / 161, 2 heads,
+//   causal, L = 5000, 134 / 126; inside it 3 heads, L = 2500, causal 76 / 120, full 77 / 122, 5 heads, L = 3000, full, 101 / 139.  The forward, in the ring: 4 heads,
+//   L = 4096, 46 / 47; 2 heads, L = 6000, 63 / 52; 3 heads, L = 8192, 85 / 76, 4 heads 92 / 93; 3 heads, L = 6000, full, 68 / 79; 12 heads, L = 4096, causal, 59 / 79; 6 heads,
+//   L = 12 000, 216 / 252.  Up to 64 blocks calls of 1024 keys and more stay with the parts: many keys, 300 queries on 8000, 81 / 60, are the line of 32 tiles' case and not
+//   this one's, which no time puts where it is: 8 heads, L = 1024, 19 / 32, 4 heads, L = 1536, 23.7 / 34.8, L = 2048 28 / 36; with fewer keys calls come here (8 heads,
+//   L = 1000, 18.9 / 31.6).
+// One head, too, below the line: backward of 512 rows, causal, 27 / 68, of 1024 rows 39 / 96; two heads of 512 rows 27 / 68.
 bool ody_attn_fwd_short_ok(const AttnParams& p) {
   if (std::max(p.sk.l, p.sv.l) >= tile128::TILE_MAX_STRIDE) return false;   // rows of a tile beyond 32-bit offsets
   const int64_t blocks = row_blocks(p.B, p.Lq, p.Hq), tiles = (p.Lk + ROWS - 1) / ROWS;

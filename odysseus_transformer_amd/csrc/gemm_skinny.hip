@@ -33,7 +33,7 @@ __device__ __forceinline__ float wave_sum(float x) {
 // NT groups a block, U steps of 32 k in flight per wavefront and group, and SK_WAVES wavefronts (ody_launch_gemm_skinny).
 // NORM: A is x, and the product that of its RMS-normalised rows.  Every block normalises them for itself, into LDS, with the arithmetic of
 // the RMSNorm kernel (another order of the sum), while its first fragments of W are on their way; EPI_ROPE then takes its angles from the positions too.  Weights
-// cold, us without the norm / with it, one row: 6144 x 4096 with rotation 13.4 / 13.0, 22016 x 4096 SwiGLU 34.6 / 33.0 (the rows are read from LDS there), 5632 x 1024 5.6 / 5.2.  The norm's own launch takes 2.6, the
+// cold, us without the norm / with it, one row: 6144 x 4096 with rotation 12.6 / 13.0, 22016 x 4096 SwiGLU 34.6 / 33.0 (the rows are read from LDS there), 5632 x 1024 5.6 / 5.2.  The norm's own launch takes 2.6, the
 // table's 2.0, and each its gap and 5 of host work.  (The norm inside the K loop, on every fragment, took 0.3 and 3.4 us longer.)
 // BATCH: all loads of a batch in front of its first product.  Left to the compiler, most of a later batch went out one or two loads at a time (NORM: 39 us for 33);
 // where A's rows are many and blocks too, its order is the better one (22016 x 4096, M = 8: 41.4 / 38.4, but 6144 x 4096 13.8 / 17.4).
@@ -267,9 +267,10 @@ int launch_for(const char* name, const bf16* A, const bf16* W, bf16* C, const bf
 }  // namespace
 
 bool ody_gemm_skinny_ok(int epi, int M, int N) {
-  // one 16-row operand: with a second one the loads of A weigh as much as those of W, and the tile kernel, which shares both
-  // through LDS and cuts K over blocks, is ahead (weights cold, us here / there: 6144 x 4096, M = 8: 17.8 / 17.6, 16: 20.8 / 17.8,
-  // 32: 27.5 / 18.7; 4096 x 4096, M = 8: 10.7 / 14.0, 16: 12.2 / 13.9, 32: 15.5 / 14.2; 2048 x 2048, M = 16: 6.7 / 9.3)
+  // One 16-row operand, up to which this is the faster one but for the longest rows (weights cold, us, M = 8 and 16 here / M = 17 in the tile kernel, which shares
+  // both operands through LDS and cuts K over blocks: 6144 x 4096 13.7, 15.1 / 16.6; 4096 x 4096 9.4, 10.5 / 12.8; 2048 x 2048 5.6, 6.6 / 9.3; 22016 x 4096 37.9, 43.4 /
+  // 48.6; 32000 x 4096 52.3, 59.4 / 64.7; 4096 x 11008 20.8, 24.4 / 24.1).  A second operand was tried with instances slower than these, 6144 x 4096, M = 32, 27.5 / 18.7; with
+  // one the time of M = 8 grows by 8 to 18 % to M = 16, and by more for the loads of a second set of rows.
   if (M > ODY_SKINNY_MAX_M) return false;
   if (epi == EPI_SWIGLU_FWD) return N % 32 == 0;   // whole groups of 16 gate rows and of 16 up rows
   if (epi == EPI_ROPE) return N % 128 == 0;
