@@ -202,20 +202,20 @@ def test_keys_behind_a_sub_tile_of_the_mask_do_not_reach_dq(dev):
 
 
 # forward with eight wavefronts a block: odd counts of tiles, ragged last ones, blocks of 0, 1 and 2 tiles (fewer keys than queries), queries past the end,
-# references that a later half outgrows, and the lines of its dispatch (groups of four wavefronts in a block of 256 rows; 0: the kernel with 128-row blocks)
+# references that a later half outgrows, and the lines of its dispatch (pipe: the kernel with 256-row blocks, with one group of wavefronts or two)
 @pytest.mark.parametrize("stretch", [1.0, 60.0], ids=["unit", "moving_reference"])
-@pytest.mark.parametrize("Lq,Lk,Hq,Hkv,causal,groups", [
-    (512, 768, 65, 13, False, 2), (505, 831, 127, 127, False, 2), (2049, 1024, 28, 14, False, 2), (512, 767, 65, 65, False, 0),
-    (512, 1023, 128, 32, False, 1), (512, 1024, 128, 32, False, 2), (256, 2048, 128, 128, False, 0), (4096, 4096, 32, 8, True, 2), (3000, 3000, 22, 22, True, 2),
-    (6401, 4001, 14, 14, True, 2), (8192, 3969, 8, 4, True, 2), (4096, 4096, 33, 33, True, 0), (3000, 2999, 22, 22, True, 0),
-    (3000, 4096, 24, 24, True, 0)])
-def test_forward_in_two_groups(Lq, Lk, Hq, Hkv, causal, groups, stretch, dev):
+@pytest.mark.parametrize("Lq,Lk,Hq,Hkv,causal,pipe", [
+    (512, 768, 65, 13, False, True), (505, 831, 127, 127, False, True), (2049, 1024, 28, 14, False, True), (512, 767, 65, 65, False, False),
+    (512, 1023, 128, 32, False, True), (256, 2048, 128, 128, False, False), (4096, 4096, 32, 8, True, True), (3000, 3000, 22, 22, True, True),
+    (6401, 4001, 14, 14, True, True), (8192, 3969, 8, 4, True, True), (4096, 4096, 33, 33, True, False), (3000, 2999, 22, 22, True, False),
+    (3000, 4096, 24, 24, True, False)])
+def test_forward_in_two_groups(Lq, Lk, Hq, Hkv, causal, pipe, stretch, dev):
     from odysseus_transformer_amd import ops
     print(f"{Lq=} {Lk=} {Hq=} {Hkv=} {causal=} {stretch=}", flush=True)
     q, k, v, _ = _inputs(1, Lq, Lk, Hq, Hkv, 121)
     k = (k.float() * torch.linspace(1.0, stretch, Lk)[None, :, None, None]).bfloat16()
-    (o, lse), ran = device_kernels(lambda: ops.attn_fwd(q.to(dev), k.to(dev), v.to(dev), causal=causal))
-    assert [g for g in (1, 2) if any(f"attn_fwd_hd64_pipe_kernel<{g}>" in n for n in ran)] == ([groups] if groups else []), ran
+    (o, lse), ran = _ran(lambda: ops.attn_fwd(q.to(dev), k.to(dev), v.to(dev), causal=causal))
+    assert (FWD in ran) == pipe, ran
     G = Hq // Hkv
     o_ref, lse_ref = oracle.attention_fwd(q[:, :, :G].float(), k[:, :, :1].float(), v[:, :, :1].float(), causal=causal)
     assert_parity(o[:, :, :G], o_ref, TOL_BF16, "o")
@@ -237,6 +237,22 @@ def test_large_values_in_two_groups(causal, dev):
     o_ref, lse_ref = oracle.attention_fwd(q[:, :, :2].float(), k[:, :, :2].float(), v[:, :, :2].float(), causal=causal)
     assert_parity(o[:, :, :2], o_ref, TOL_BF16, "o")
     assert torch.allclose(lse[:, :2].cpu(), lse_ref, atol=TOL_LSE, rtol=TOL_LSE)
+
+
+# Which of the forwards runs, on both sides of every line (groups of four wavefronts in a block of 256 rows; 0: the kernel with 128-row blocks)
+@pytest.mark.parametrize("Lq,Lk,Hq,Hkv,causal,groups", [
+    (512, 768, 65, 13, False, 2), (512, 767, 65, 65, False, 0), (512, 1023, 128, 32, False, 1), (512, 1024, 128, 32, False, 2), (256, 2048, 128, 128, False, 0),
+    (4096, 4096, 32, 8, True, 2), (4096, 4096, 33, 33, True, 0), (3000, 3000, 22, 22, True, 2), (3000, 2999, 22, 22, True, 0), (3000, 4096, 24, 24, True, 0)])
+def test_forward_on_the_instance_of_its_sizes(Lq, Lk, Hq, Hkv, causal, groups, dev):
+    from odysseus_transformer_amd import ops
+    print(f"{Lq=} {Lk=} {Hq=} {Hkv=} {causal=}", flush=True)
+    q, k, v, _ = _inputs(1, Lq, Lk, Hq, Hkv, 151)
+    (o, lse), ran = device_kernels(lambda: ops.attn_fwd(q.to(dev), k.to(dev), v.to(dev), causal=causal))
+    assert [g for g in (1, 2) if any(f"attn_fwd_hd64_pipe_kernel<{g}>" in n for n in ran)] == ([groups] if groups else []), ran
+    G = Hq // Hkv
+    o_ref, lse_ref = oracle.attention_fwd(q[:, :, :G].float(), k[:, :, :1].float(), v[:, :, :1].float(), causal=causal)
+    assert_parity(o[:, :, :G], o_ref, TOL_BF16, "o")
+    assert torch.allclose(lse[:, :G].cpu(), lse_ref, atol=TOL_LSE, rtol=TOL_LSE)
 
 
 @pytest.mark.parametrize("stride", [(1 << 24) - 16, (1 << 24) - 8], ids=str)
