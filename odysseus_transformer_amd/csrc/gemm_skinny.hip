@@ -239,10 +239,13 @@ int launch(const char* name, const bf16* A, const bf16* W, bf16* C, const bf16* 
 // What a block takes.  us; weights cold unless "warm" (a matrix that the last-level cache holds, again and again).
 //   M <= 4: one group of 16 rows, 8 wavefronts: 4096 x 4096 8.0 (8.9 otherwise), 2048 x 5632 9.0 / 9.7, with the norm 22016 x 4096 33.0 / 33.1.  Beyond 512 groups 4
 //   wavefronts with twice the loads: 13312 x 2816, M = 4, 18.6 / 21.0, 32000 x 4096 45.3 / 44.8 and 46.8; where rows are long, too, but not with one row of A:
-//   4096 x 11008, M = 4, 19.9 / 20.9 and 21.3, M = 1 19.3 / 19.3, 4096 x 14336, M = 1, 22.1 / 22.8.
+//   4096 x 11008, M = 4, 19.9 / 20.9 and 21.3, M = 1 19.3 / 19.3, 4096 x 14336, M = 1, 22.1 / 22.8.  (Warm, two
+//   groups on 8 wavefronts would be ahead from three rows on: 32000 x 2048, M = 4, 22.9 / 21.7, 65536 x 1536 32.9 / 30.1, cold 27.3 / 28.0 and 39.7 / 42.3.)
 //   M > 4: a group's fragments of A weigh as much as those of W.  Two groups share them where such blocks fill their last round of units, to 512 groups and from 800 on:
 //   22016 x 4096, M = 8, 38.4 / 40.6, 6144 x 4096, M = 16, 15.2 / 15.9, 4608 x 3072, rotated, M = 16, 12.3 / 15.2 (one group); between the two, 1.1 to 1.5 rounds, they do not:
-//   9216 x 2816, M = 5, 18.5, one group 14.5, 12288 x 4096, M = 5, 24.6 / 20.6.  Otherwise one group: 4096 x 11008, M = 8, 21.0 / 22.5, 3072 x 2048 6.0 / 7.7; 8 wavefronts
+//   9216 x 2816, M = 5, 18.5, one group 14.5, 12288 x 4096, M = 5, 24.6 / 20.6.  Rows of 1792 to 2048 are two batches for each of 8 wavefronts, four for 4;
+//   with 5 to 12 rows of A, 8 / 4 wavefronts: 50264 x 2048, M = 5, 43.1 / 45.2, M = 12 48.2 / 49.6, 32000 x 2048, M = 5, 27.1 / 29.2, M = 12 30.3 / 29.9, 32000 x 1920, M = 5, 25.2 / 29.8,
+//   warm 16384 x 2048, M = 9, 12.6 / 13.7; beyond, 32000 x 1792, M = 5, 26.0 / 24.5, warm 32000 x 2176 24.0 / 23.0, 40960 x 2048, M = 16, 40.5 / 39.1.  Otherwise one group: 4096 x 11008, M = 8, 21.0 / 22.5, 3072 x 2048 6.0 / 7.7; 8 wavefronts
 //   where groups are no more than units and K is short: 4096 x 4096, M = 5, 8.6 / 9.1, warm 7.2 / 7.5, or two batches for either, 2048 x 2048, M = 12, 6.1 / 6.3.
 //   Pairs of rows (rotation, SwiGLU) with 257 to 512 groups: blocks of two whole groups are one for a unit, those of half and half up to two, and the second one's start shows.
 //   Two / half and half: rotated, 6144 x 2048, M = 1, 7.3 / 8.2, M = 8 8.0 / 9.6, M = 12 8.4 / 9.2, 5120 x 4096, M = 1, 12.1 / 13.3; SwiGLU, 5632 x 1024, M = 6, warm, 4.6 / 4.9
@@ -256,6 +259,8 @@ int launch_for(const char* name, const bf16* A, const bf16* W, bf16* C, const bf
   if constexpr (EPI == EPI_SWIGLU_FWD || EPI == EPI_ROPE)
     if (one_each && (K > 2048 ? M <= 4 && groups <= 448 : M <= 8 || EPI == EPI_ROPE))
       return launch<2, 8, 8, EPI, false, false>(name, A, W, C, bias, M, N, K, lda, ldw, ldc, accumulate, ep, st);
+  if (M > 4 && M <= 12 && groups >= 1024 && K > 1792 && K <= 2048)
+    return launch<2, 4, 8, EPI, false, false>(name, A, W, C, bias, M, N, K, lda, ldw, ldc, accumulate, ep, st);
   if (M > 4 && groups >= 1024) return launch<2, 4, 4, EPI, false, false>(name, A, W, C, bias, M, N, K, lda, ldw, ldc, accumulate, ep, st);
   if (M > 4 && (one_each || groups >= 800) && (K > 2048 || M > 8)) return launch<2, 4, 4, EPI>(name, A, W, C, bias, M, N, K, lda, ldw, ldc, accumulate, ep, st);
   const bool long_rows = M > 8 ? K > 2048 || K <= 1024 : K > 4096 && M > 4;

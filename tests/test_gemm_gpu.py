@@ -423,6 +423,14 @@ def test_few_rows_on_the_instance_of_their_sizes(what, N, K, M, instance, dev):
     assert ran and all(f"gemm_skinny_kernel<{instance}, " in name for name in ran), ran
 
 
+@pytest.mark.parametrize("what,N,K,M,instance", [
+    ("plain", 16384, 1792, 5, "2, 4, 4"), ("plain", 16384, 1800, 5, "2, 4, 8"), ("residual", 16392, 2048, 8, "2, 4, 8"), ("plain", 16384, 2048, 12, "2, 4, 8"), ("plain", 16384, 2048, 13, "2, 4, 4"),
+    ("plain", 16384, 2048, 4, "1, 8, 4"), ("swiglu", 16384, 2056, 8, "2, 4, 4"), ("swiglu", 16416, 2040, 6, "2, 4, 8"), ("rope", 16384, 1920, 7, "2, 4, 8"),
+    ("plain", 16352, 2048, 5, "1, 8, 4")], ids=lambda v: str(v))
+def test_few_rows_of_two_batches(what, N, K, M, instance, dev):
+    test_few_rows_on_the_instance_of_their_sizes(what, N, K, M, instance, dev)
+
+
 @pytest.mark.parametrize("op", ["nt", "nn", "tn"])
 @pytest.mark.parametrize("M,N,K", [(72, 1032, 30720), (136, 1280, 41032), (40, 392, 30656)], ids=lambda v: str(v))
 def test_a_long_k_without_a_workspace(op, M, N, K, dev):
